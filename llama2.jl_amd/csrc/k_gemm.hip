@@ -337,7 +337,7 @@ __global__ __launch_bounds__(64) void route_kernel(const float *z, int64_t ldz, 
     __shared__ int s_sel[64];
     __shared__ float s_score[64];
     const int64_t m = blockIdx.x;
-    l_route(z + m * ldz, bias, E, top, kind, s_mem, s_sel, s_score);
+    l_route<false>(z + m * ldz, bias, E, top, kind, s_mem, s_sel, s_score);
     for (int k = threadIdx.x; k < top; k += 64) {
         choice[m * top + k] = s_sel[k];
         score[m * top + k] = s_score[k];

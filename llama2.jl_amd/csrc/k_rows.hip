@@ -16,11 +16,20 @@ __device__ __forceinline__ int xs_index(int e, int plane) { return ((e >> 2) & 1
 struct RowsChunk {
     uint4 p, q;
 };
+typedef uint32_t rows_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 rows_word(const uint16_t *w) {
+#ifdef ROWS_PLAIN
+    return *(const uint4 *)w;
+#else
+    const rows_u32x4 v = __builtin_nontemporal_load((const rows_u32x4 *)w);
+    return make_uint4(v.x, v.y, v.z, v.w);
+#endif
+}
+// (no load is skipped: how many are under way has to be known when the code is compiled for a wait to leave the later ones alone)
 __device__ __forceinline__ void rows_load(RowsChunk &c, const uint16_t *w0, const uint16_t *w1, int k, int ld) {
-    if (k < ld) {
-        c.p = *(const uint4 *)(w0 + k);
-        c.q = *(const uint4 *)(w1 + k);
-    }
+    const int at = min(k, ld - 8);
+    c.p = rows_word(w0 + at);
+    c.q = rows_word(w1 + at);
 }
 __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, int plane, int k, int ld, float &acc0, float &acc1) {
     if (k >= ld) return;
@@ -44,31 +53,89 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
     acc1 = fmaf(l_bf16_hi(q.w), xb.w, acc1);
 }
 
-#define ROWS_V 4  // steps of 4 elements a thread of the staged vectors
-#define ROWS_U 4  // chunks of a row pair fetched together: 2 rows x 4 KB per wavefront
 
-// KSPLIT: the wavefronts share every pair of rows, each its part of the inputs (matrices with few rows)
-template <int PRO, int EPI, bool KSPLIT>
-__global__ __launch_bounds__(ROWS_THREADS) void rows_kernel(RowsArgs a, int rows_per_wg, int plane) {
+// how a matrix's rows are dealt out (rows_plan): workgroup b has `pairs` row pairs, and one more for b < more, one after another
+struct RowsPlan {
+    int plane;            // half of a staged vector's floats
+    int pairs, more;
+    int per_vec, per_pair;  // steps of a row pair per staged vector, in all
+};
+
+// What bounds a decode step's products is the matrix bytes, so nothing may stand between the launch and the stream of loads: the
+// vector is requested first, the wavefront's first step right behind it (loads return in order), and the prologue's barriers
+// order LDS traffic only, so that the step stays under way while the norm is formed.  (With barriers that wait for memory, as
+// __syncthreads does, 128 x 4096 rows behind a norm started streaming 6 us late.)
+//
+// U: chunks of a row pair fetched together (2 rows x U KB per wavefront), one step.  A workgroup owns a run of row pairs and its
+// wavefronts share the run's steps evenly, across the borders of pairs: with whole pairs per wavefront the rows of a 12 576 x
+// 4096 matrix came to 1.5 pairs a wavefront, that is two, on 393 of 512 places.  A pair's first wavefront leaves its sums in
+// s_res; wavefronts that go on with a pair leave theirs in s_part, added in order.  Four wavefronts per SIMD (128 registers): two
+// workgroups a CU.
+//
+// V: steps of four elements a thread in which the vector is requested; Y: with a pending update.
+template <int PRO, int EPI, int U, int V, bool Y>
+__global__ __launch_bounds__(ROWS_THREADS, 4) void rows_kernel(RowsArgs a, RowsPlan pl) {
     extern __shared__ __align__(16) float s_mem[];
-    __shared__ float s_red[ROWS_WAVES];
+    __shared__ float s_red[2][ROWS_WAVES];
     __shared__ float s_part[ROWS_WAVES][2];
+    __shared__ int s_head[ROWS_WAVES];  // the pair that s_part belongs to
     __shared__ int s_sel[ROWS_MAX_TOP];
     __shared__ float s_score[ROWS_MAX_TOP];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    float *xs = s_mem;
-    const int K = a.K, ld = a.ld;
+    const int K = a.K, ld = a.ld, plane = pl.plane;
     const int nvec = PRO == RP_DOWN ? a.top : 1;  // vectors staged, each in its own 2 * plane floats
+    float *xs = s_mem, *s_res = s_mem + nvec * 2 * plane;
 
-    // the work of this wavefront: pairs of rows, each in steps of ROWS_U chunks
-    const int64_t row_end = min((int64_t)(blockIdx.x + 1) * rows_per_wg, a.n_rows);
-    const int pair_step = KSPLIT ? 2 : 2 * ROWS_WAVES;
-    int64_t r0 = (int64_t)blockIdx.x * rows_per_wg + (KSPLIT ? 0 : 2 * wave);
-    const int kw = KSPLIT ? ((ld + 511) / 512 + ROWS_WAVES - 1) / ROWS_WAVES * 512 : 0;  // inputs of a wavefront
-    const int kstart = KSPLIT ? min(wave * kw, ld) : 0, kend = KSPLIT ? min(kstart + kw, ld) : ld;
-    constexpr int kstep = ROWS_U * 512;
-    auto row_ptrs = [&](int64_t r, int v, const uint16_t *&w0, const uint16_t *&w1) {
-        const int64_t r1 = r + 1 < row_end ? r + 1 : r;
+    // ---- the vector is requested ----------------------------------------------------------------------------------
+    // (four elements a thread and step)
+    const bool quads = K % 4 == 0 && (PRO != RP_HEADNORM || a.hv % 4 == 0);
+    const bool fast = quads && nvec * K <= 4 * V * ROWS_THREADS;
+    constexpr bool as_is = PRO == RP_PLAIN || PRO == RP_DOWN;
+    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 x[V], w[as_is ? 1 : V], g[PRO == RP_HEADNORM ? V : 1], y[Y ? V : 1], yw[Y ? V : 1];
+    if (Y && fast) {
+#pragma unroll
+        for (int u = 0; u < V; u++) {
+            const int i = 4 * (t + u * ROWS_THREADS);
+            y[u] = yw[u] = zero4;
+            if (i < K) {
+                y[u] = *(const float4 *)(a.y + i);
+                yw[u] = *(const float4 *)(a.yw + i);
+            }
+        }
+    }
+    if (fast) {
+#pragma unroll
+        for (int u = 0; u < V; u++) {
+            const int i = 4 * (t + u * ROWS_THREADS);
+            x[u] = zero4;
+            if (i < nvec * K) x[u] = *(const float4 *)(a.x + i);
+            if constexpr (!as_is) {
+                w[u] = zero4;
+                if (PRO != RP_HEADNORM && i < K) w[u] = *(const float4 *)(a.normw + i);
+            }
+            if constexpr (PRO == RP_HEADNORM) {
+                g[u] = zero4;
+                if (i < K) g[u] = *(const float4 *)(a.gate + i);
+            }
+        }
+    }
+    const int b = blockIdx.x, n_pairs = pl.pairs + (b < pl.more);
+    const int64_t p0 = (int64_t)b * pl.pairs + min(b, pl.more), row0 = 2 * p0, row_end = min(2 * (p0 + n_pairs), a.n_rows);
+    constexpr int kstep = U * 512;
+    // (of the row whose result this thread writes first)
+    float before = 0.0f;
+    if (EPI == RE_RESID && row0 + t < row_end) before = a.resid[row0 + t];
+    if (EPI == RE_EMBED && row0 + t < row_end) before = l_bf16(a.emb[(int64_t)l_step_token(a.ctl, a.prompt) * a.emb_ld + row0 + t]);
+    asm volatile("" ::: "memory");
+
+    // ---- the work of this wavefront: steps u0 .. u1 - 1 of the workgroup's pairs --------------------------------------
+    const int total = n_pairs * pl.per_pair;
+    const int u0 = (unsigned)(total * wave) / ROWS_WAVES, u1 = (unsigned)(total * (wave + 1)) / ROWS_WAVES;
+    int pair = (unsigned)min(u0, total - 1) / (unsigned)pl.per_pair, step = min(u0, total - 1) - pair * pl.per_pair;
+    int v = PRO == RP_DOWN ? (unsigned)step / (unsigned)pl.per_vec : 0, k = (step - v * pl.per_vec) * kstep;
+    auto row_ptrs = [&](int pair, int v, const uint16_t *&w0, const uint16_t *&w1) {
+        const int64_t r = row0 + 2 * pair, r1 = r + 1 < row_end ? r + 1 : r;
         if (PRO == RP_UP) {
             const unsigned n = (unsigned)a.rows_each, e0 = (unsigned)r / n, e1 = (unsigned)r1 / n;
             w0 = a.w + ((int64_t)s_sel[e0] * a.rows_each + (r - e0 * a.rows_each)) * ld;
@@ -81,60 +148,35 @@ __global__ __launch_bounds__(ROWS_THREADS) void rows_kernel(RowsArgs a, int rows
             w1 = a.w + r1 * ld;
         }
     };
-    RowsChunk cur[ROWS_U], nxt[ROWS_U];
+    RowsChunk cur[U], nxt[U];
     const uint16_t *w0 = nullptr, *w1 = nullptr;
-    auto fetch = [&](RowsChunk (&c)[ROWS_U], int k) {
+    auto fetch = [&](RowsChunk (&c)[U], int k) {
 #pragma unroll
-        for (int u = 0; u < ROWS_U; u++) rows_load(c[u], w0, w1, k + 512 * u + 8 * lane, kend);
+        for (int u = 0; u < U; u++) rows_load(c[u], w0, w1, k + 512 * u + 8 * lane, ld);
     };
-    // the first rows do not depend on the vector: they are under way while it is made
-    if (PRO != RP_UP && PRO != RP_DOWN && r0 < row_end) {
-        row_ptrs(r0, 0, w0, w1);
-        fetch(cur, kstart);
-    }
-
-    if (PRO == RP_UP || PRO == RP_DOWN) {
-        l_route(a.z, a.z_bias, a.n_experts, a.top, a.route, s_mem + (int64_t)nvec * 2 * plane, s_sel, s_score);
-        if (r0 < row_end) {
-            row_ptrs(r0, 0, w0, w1);
-            fetch(cur, kstart);
-        }
-    }
+    if (PRO == RP_UP || PRO == RP_DOWN) l_route<true>(a.z, a.z_bias, a.n_experts, a.top, a.route, s_res, s_sel, s_score);
+    row_ptrs(pair, v, w0, w1);
+    fetch(cur, k);
+    asm volatile("" ::: "memory");
+    if (lane == 0) s_head[wave] = -1;
 
     // ---- the vector -------------------------------------------------------------------------------------------
-    // (four elements a thread and step; the vectors of one prologue are fetched together, ROWS_V steps at a time)
-    const bool quads = K % 4 == 0 && (PRO != RP_HEADNORM || a.hv % 4 == 0);
     auto put4 = [&](float *dst, int q, float4 v) { *(float4 *)(dst + (q & 1) * plane + 4 * (q >> 1)) = v; };
-    if (PRO == RP_NORM || PRO == RP_UP) {
+    auto head_scale = [&](int h) {
+        float ss = 0.0f;
+        for (int p = 0; p < a.n_split; p++) ss += a.ssq[h * a.n_split + p];
+        return 1.0f / sqrtf(ss / (float)a.hv + a.eps);
+    };
+    if constexpr (PRO == RP_NORM || PRO == RP_UP) {
         float r;
-        if (quads && K <= 4 * ROWS_V * ROWS_THREADS) {
-            float4 x[ROWS_V], w[ROWS_V];
-#pragma unroll
-            for (int u = 0; u < ROWS_V; u++) {
-                const int i = 4 * (t + u * ROWS_THREADS);
-                x[u] = w[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (i < K) {
-                    x[u] = *(const float4 *)(a.x + i);
-                    w[u] = *(const float4 *)(a.normw + i);
-                }
-            }
-            if (a.y) {
-                float4 y[ROWS_V], yw[ROWS_V];
+        if (fast) {
+            if constexpr (Y) {
                 float ss = 0.0f;
 #pragma unroll
-                for (int u = 0; u < ROWS_V; u++) {
-                    const int i = 4 * (t + u * ROWS_THREADS);
-                    y[u] = yw[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (i < K) {
-                        y[u] = *(const float4 *)(a.y + i);
-                        yw[u] = *(const float4 *)(a.yw + i);
-                    }
-                }
+                for (int u = 0; u < V; u++) ss = fmaf(y[u].x, y[u].x, fmaf(y[u].y, y[u].y, fmaf(y[u].z, y[u].z, fmaf(y[u].w, y[u].w, ss))));
+                const float f = a.mult / sqrtf(l_block_sum_lds(ss, s_red[0]) / (float)K + a.eps);
 #pragma unroll
-                for (int u = 0; u < ROWS_V; u++) ss = fmaf(y[u].x, y[u].x, fmaf(y[u].y, y[u].y, fmaf(y[u].z, y[u].z, fmaf(y[u].w, y[u].w, ss))));
-                const float f = a.mult / sqrtf(l_block_sum(ss, s_red) / (float)K + a.eps);
-#pragma unroll
-                for (int u = 0; u < ROWS_V; u++) {
+                for (int u = 0; u < V; u++) {
                     const int i = 4 * (t + u * ROWS_THREADS);
                     x[u].x = fmaf(f * y[u].x, yw[u].x, x[u].x);
                     x[u].y = fmaf(f * y[u].y, yw[u].y, x[u].y);
@@ -145,26 +187,26 @@ __global__ __launch_bounds__(ROWS_THREADS) void rows_kernel(RowsArgs a, int rows
             }
             float ss = 0.0f;
 #pragma unroll
-            for (int u = 0; u < ROWS_V; u++) ss = fmaf(x[u].x, x[u].x, fmaf(x[u].y, x[u].y, fmaf(x[u].z, x[u].z, fmaf(x[u].w, x[u].w, ss))));
-            r = 1.0f / sqrtf(l_block_sum(ss, s_red) / (float)K + a.eps);
+            for (int u = 0; u < V; u++) ss = fmaf(x[u].x, x[u].x, fmaf(x[u].y, x[u].y, fmaf(x[u].z, x[u].z, fmaf(x[u].w, x[u].w, ss))));
+            r = 1.0f / sqrtf(l_block_sum_lds(ss, s_red[1]) / (float)K + a.eps);
 #pragma unroll
-            for (int u = 0; u < ROWS_V; u++) {
+            for (int u = 0; u < V; u++) {
                 const int q = t + u * ROWS_THREADS;
                 if (4 * q < ld) put4(xs, q, make_float4(r * x[u].x * w[u].x, r * x[u].y * w[u].y, r * x[u].z * w[u].z, r * x[u].w * w[u].w));
             }
         } else {
             float f = 0.0f;
-            if (a.y) {
+            if (Y) {
                 float ss = 0.0f;
                 for (int i = t; i < K; i += ROWS_THREADS) ss = fmaf(a.y[i], a.y[i], ss);
-                f = a.mult / sqrtf(l_block_sum(ss, s_red) / (float)K + a.eps);
+                f = a.mult / sqrtf(l_block_sum_lds(ss, s_red[0]) / (float)K + a.eps);
             }
             float ss = 0.0f;
             for (int i = t; i < ld; i += ROWS_THREADS) {
                 float v = 0.0f;
                 if (i < K) {
                     v = a.x[i];
-                    if (a.y) {
+                    if (Y) {
                         v = fmaf(f * a.y[i], a.yw[i], v);
                         if (blockIdx.x == 0) a.x_out[i] = v;
                     }
@@ -173,152 +215,161 @@ __global__ __launch_bounds__(ROWS_THREADS) void rows_kernel(RowsArgs a, int rows
                 if (i < K) v *= a.normw[i];
                 xs[xs_index(i, plane)] = v;
             }
-            r = 1.0f / sqrtf(l_block_sum(ss, s_red) / (float)K + a.eps);
+            r = 1.0f / sqrtf(l_block_sum_lds(ss, s_red[1]) / (float)K + a.eps);
             for (int i = t; i < ld; i += ROWS_THREADS) xs[i] *= r;
         }
-    } else if (PRO == RP_HEADNORM) {
-        auto scale = [&](int h) {
-            float ss = 0.0f;
-            for (int p = 0; p < a.n_split; p++) ss += a.ssq[h * a.n_split + p];
-            return 1.0f / sqrtf(ss / (float)a.hv + a.eps);
-        };
-        if (quads) {
-            for (int q0 = t; 4 * q0 < ld; q0 += ROWS_V * ROWS_THREADS) {
-                float4 x[ROWS_V], g[ROWS_V], w[ROWS_V];
-                float r[ROWS_V];
-#pragma unroll
-                for (int u = 0; u < ROWS_V; u++) {
-                    const int i = 4 * (q0 + u * ROWS_THREADS);
-                    x[u] = g[u] = w[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    r[u] = 0.0f;
-                    if (i < K) {
-                        const int h = i / a.hv;
-                        x[u] = *(const float4 *)(a.x + i);
-                        g[u] = *(const float4 *)(a.gate + i);
-                        w[u] = *(const float4 *)(a.normw + (i - h * a.hv));
-                        r[u] = scale(h);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < ROWS_V; u++) {
-                    const int q = q0 + u * ROWS_THREADS;
-                    if (4 * q < ld)
-                        put4(xs, q, make_float4(r[u] * x[u].x * w[u].x * g[u].x, r[u] * x[u].y * w[u].y * g[u].y,
-                                                r[u] * x[u].z * w[u].z * g[u].z, r[u] * x[u].w * w[u].w * g[u].w));
-                }
+    } else if constexpr (PRO == RP_HEADNORM) {
+        auto normed = [&](int q, float4 x, float4 g) {
+            const int i = 4 * q;
+            if (i >= ld) return;
+            float4 o = zero4;
+            if (i < K) {
+                const int h = (unsigned)i / (unsigned)a.hv;
+                const float r = head_scale(h);
+                const float4 n = *(const float4 *)(a.normw + (i - h * a.hv));
+                o = make_float4(r * x.x * n.x * g.x, r * x.y * n.y * g.y, r * x.z * n.z * g.z, r * x.w * n.w * g.w);
             }
+            put4(xs, q, o);
+        };
+        if (fast) {
+#pragma unroll
+            for (int u = 0; u < V; u++) normed(t + u * ROWS_THREADS, x[u], g[u]);
+        } else if (quads) {
+            for (int q = t; 4 * q < ld; q += ROWS_THREADS)
+                normed(q, 4 * q < K ? *(const float4 *)(a.x + 4 * q) : zero4, 4 * q < K ? *(const float4 *)(a.gate + 4 * q) : zero4);
         } else {
             for (int i = t; i < ld; i += ROWS_THREADS) {
                 float v = 0.0f;
                 if (i < K) {
                     const int h = i / a.hv;
-                    v = a.x[i] * scale(h) * a.normw[i - h * a.hv] * a.gate[i];
+                    v = a.x[i] * head_scale(h) * a.normw[i - h * a.hv] * a.gate[i];
                 }
                 xs[xs_index(i, plane)] = v;
             }
         }
-    } else {
-        for (int v = 0; v < nvec; v++) {
-            const float *src = a.x + (int64_t)v * K;
-            float *dst = xs + v * 2 * plane;
-            if (quads) {
-                for (int q0 = t; 4 * q0 < ld; q0 += ROWS_V * ROWS_THREADS) {
-                    float4 x[ROWS_V];
+    } else if (fast) {
 #pragma unroll
-                    for (int u = 0; u < ROWS_V; u++) {
-                        const int i = 4 * (q0 + u * ROWS_THREADS);
-                        x[u] = i < K ? *(const float4 *)(src + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-                    }
-#pragma unroll
-                    for (int u = 0; u < ROWS_V; u++)
-                        if (4 * (q0 + u * ROWS_THREADS) < ld) put4(dst, q0 + u * ROWS_THREADS, x[u]);
-                }
-            } else {
-                for (int i = t; i < ld; i += ROWS_THREADS) dst[xs_index(i, plane)] = i < K ? src[i] : 0.0f;
-            }
+        for (int u = 0; u < V; u++) {
+            const int i = 4 * (t + u * ROWS_THREADS);
+            if (i >= nvec * K) continue;
+            const int v = PRO == RP_DOWN ? (unsigned)i / (unsigned)K : 0;
+            put4(xs + v * 2 * plane, (i - v * K) >> 2, x[u]);
         }
+        for (int i = K + t; i < ld; i += ROWS_THREADS)
+            for (int v = 0; v < nvec; v++) xs[v * 2 * plane + xs_index(i, plane)] = 0.0f;
+    } else if (quads) {
+        for (int v = 0; v < nvec; v++)
+#pragma unroll 4
+            for (int q = t; 4 * q < ld; q += ROWS_THREADS) put4(xs + v * 2 * plane, q, 4 * q < K ? *(const float4 *)(a.x + (int64_t)v * K + 4 * q) : zero4);
+    } else {
+        for (int v = 0; v < nvec; v++)
+            for (int i = t; i < ld; i += ROWS_THREADS) xs[v * 2 * plane + xs_index(i, plane)] = i < K ? a.x[(int64_t)v * K + i] : 0.0f;
     }
-    __syncthreads();
+    l_lds_barrier();
 
     // ---- rows -------------------------------------------------------------------------------------------------
-    int v = 0, k = kstart;
+    bool began = step == 0;  // this wavefront began the pair it is at
     float acc0 = 0.0f, acc1 = 0.0f;
-    while (r0 < row_end) {
-        // where the next step is; its chunks are fetched before this step's are used
-        int64_t rn = r0;
-        int vn = v, kn = k + kstep;
-        if (kn >= kend) {
-            kn = kstart;
-            if (++vn == nvec) {
-                vn = 0;
-                rn = r0 + pair_step;
-            }
-        }
-        if (rn < row_end) {
-            if (rn != r0 || vn != v) row_ptrs(rn, vn, w0, w1);
-            fetch(nxt, kn);
-        }
+    auto multiply = [&] {
         const float *xv = xs + v * 2 * plane;
 #pragma unroll
-        for (int u = 0; u < ROWS_U; u++) rows_fma(cur[u], xv, plane, k + 512 * u + 8 * lane, kend, acc0, acc1);
-        if (rn != r0) {
-            const bool two = r0 + 1 < row_end;
-            acc0 = l_wave_sum(acc0);
-            acc1 = l_wave_sum(acc1);
-            if (KSPLIT) {
-                __syncthreads();
-                if (lane == 0) {
-                    s_part[wave][0] = acc0;
-                    s_part[wave][1] = acc1;
-                }
-                __syncthreads();
-                acc0 = acc1 = 0.0f;
-#pragma unroll
-                for (int i = 0; i < ROWS_WAVES; i++) {
-                    acc0 += s_part[i][0];
-                    acc1 += s_part[i][1];
-                }
+        for (int i = 0; i < U; i++) rows_fma(cur[i], xv, plane, k + 512 * i + 8 * lane, ld, acc0, acc1);
+    };
+    auto put = [&] {
+        acc0 = l_wave_sum(acc0);
+        acc1 = l_wave_sum(acc1);
+        if (lane == 0) {
+            float *p = began ? s_res + 2 * pair : s_part[wave];
+            p[0] = acc0;
+            p[1] = acc1;
+            if (!began) s_head[wave] = pair;
+        }
+    };
+    for (int u = u0; u + 1 < u1; u++) {
+        // where the next step is; its chunks are fetched before this step's are used
+        int pn = pair, vn = v, kn = k + kstep;
+        if (kn >= ld) {
+            kn = 0;
+            if (++vn == nvec) {
+                vn = 0;
+                pn++;
             }
-            if (EPI == RE_GLU || (EPI == RE_STORE_GLU && r0 >= a.glu_from)) {  // (whole pairs)
-                if ((!KSPLIT || wave == 0) && lane == 0) {
-                    float s_in = 1.0f, s_out = 1.0f;
-                    if (PRO == RP_UP) (a.route == LROUTE_SIGMOID_IN ? s_in : s_out) = s_score[(unsigned)r0 / (unsigned)a.rows_each];
-                    const float o = s_out * l_act(a.act, s_in * acc0) * (s_in * acc1);
-                    if (EPI == RE_GLU)
-                        a.out[r0 >> 1] = o;
-                    else
-                        a.out2[(r0 - a.glu_from) >> 1] = o;
-                }
-            } else if ((!KSPLIT || wave == 0) && lane < (two ? 2 : 1)) {
-                const int64_t r = r0 + lane;
-                const float val = lane ? acc1 : acc0;
-                float o = val;
-                if (EPI == RE_RESID) o = a.resid[r] + a.mult * val;
-                if (EPI == RE_ACT) o = l_act(a.act, val);
-                if (EPI == RE_UP) {
-                    const float f = s_score[(unsigned)r / (unsigned)a.rows_each];
-                    o = a.route == LROUTE_SIGMOID_IN ? l_act(a.act, f * val) : f * l_act(a.act, val);
-                }
-                if (EPI == RE_EMBED) o = l_act(a.act, val) * l_bf16(a.emb[(int64_t)l_step_token(a.ctl, a.prompt) * a.emb_ld + r]);
-                a.out[r] = o;
-            }
+        }
+        if (pn != pair || vn != v) row_ptrs(pn, vn, w0, w1);
+        fetch(nxt, kn);
+        multiply();
+        if (pn != pair) {
+            put();
             acc0 = acc1 = 0.0f;
+            began = true;
         }
 #pragma unroll
-        for (int u = 0; u < ROWS_U; u++) cur[u] = nxt[u];
-        r0 = rn;
+        for (int i = 0; i < U; i++) cur[i] = nxt[i];
+        pair = pn;
         v = vn;
         k = kn;
+    }
+    if (u0 < u1) {
+        multiply();
+        put();
+    }
+    l_lds_barrier();
+
+    // ---- results: a thread per row -------------------------------------------------------------------------------------
+    for (int i = t; row0 + i < row_end; i += ROWS_THREADS) {
+        const int64_t r = row0 + i;
+        const bool glu = EPI == RE_GLU || (EPI == RE_STORE_GLU && r >= a.glu_from);  // (whole pairs)
+        if (glu && (i & 1)) continue;
+        float val = s_res[i], up = glu ? s_res[i + 1] : 0.0f;
+        if (pl.per_pair > 1) {
+#pragma unroll
+            for (int h = 1; h < ROWS_WAVES; h++) {
+                const bool here = s_head[h] == i >> 1;
+                val += here ? s_part[h][i & 1] : 0.0f;
+                up += here ? s_part[h][1] : 0.0f;
+            }
+        }
+        float f = 1.0f;
+        if (PRO == RP_UP) f = s_score[(unsigned)r / (unsigned)a.rows_each];
+        const float f_in = a.route == LROUTE_SIGMOID_IN ? f : 1.0f, f_out = a.route == LROUTE_SIGMOID_IN ? 1.0f : f;
+        if (glu) {
+            const float o = f_out * l_act(a.act, f_in * val) * (f_in * up);
+            if (EPI == RE_GLU)
+                a.out[r >> 1] = o;
+            else
+                a.out2[(r - a.glu_from) >> 1] = o;
+            continue;
+        }
+        float o = val;
+        if (EPI == RE_RESID) o = (i == t ? before : a.resid[r]) + a.mult * val;
+        if (EPI == RE_ACT) o = l_act(a.act, val);
+        if (EPI == RE_UP) o = a.route == LROUTE_SIGMOID_IN ? l_act(a.act, f * val) : f * l_act(a.act, val);
+        if (EPI == RE_EMBED)
+            o = l_act(a.act, val) * (i == t ? before : l_bf16(a.emb[(int64_t)l_step_token(a.ctl, a.prompt) * a.emb_ld + r]));
+        a.out[r] = o;
     }
 }
 
 #define ROWS_MAX_DEVICES 64
+#define ROWS_MAX_PAIRS 4096  // of a workgroup: 32 KB of results
 
-template <int PRO, int EPI, bool KSPLIT>
-static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t rows_per_wg) {
-    const int plane = a.ld / 2;
+// LDS of a workgroup: the vectors, then the results of its pairs, where the choice of experts has its logits before
+static size_t rows_lds(const RowsArgs &a, int pro, int pairs) {
+    const int nvec = pro == RP_DOWN ? a.top : 1;
+    return ((size_t)nvec * a.ld + std::max(2 * pairs, pro == RP_UP || pro == RP_DOWN ? a.n_experts : 0)) * sizeof(float);
+}
+
+template <int PRO, int EPI, int U, int V, bool Y>
+static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
     const int nvec = PRO == RP_DOWN ? a.top : 1;
-    const size_t lds = ((size_t)nvec * 2 * plane + (PRO == RP_UP || PRO == RP_DOWN ? a.n_experts : 0)) * sizeof(float);
+    const int64_t pairs = (a.n_rows + 1) / 2;
+    RowsPlan pl;
+    pl.plane = a.ld / 2;
+    pl.pairs = (int)(pairs / grid);
+    pl.more = (int)(pairs % grid);
+    pl.per_vec = (a.ld + 512 * U - 1) / (512 * U);
+    pl.per_pair = nvec * pl.per_vec;
+    const size_t lds = rows_lds(a, PRO, pl.pairs + 1);
     if (lds > 152 * 1024) return hipErrorInvalidValue;
     if (lds > 48 * 1024) {
         int dev = 0;
@@ -327,25 +378,50 @@ static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t rows_per
         if (dev < 0 || dev >= ROWS_MAX_DEVICES) return hipErrorInvalidDevice;
         static bool attr_set[ROWS_MAX_DEVICES] = {};
         if (!attr_set[dev]) {
-            e = hipFuncSetAttribute((const void *)rows_kernel<PRO, EPI, KSPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
+            e = hipFuncSetAttribute((const void *)rows_kernel<PRO, EPI, U, V, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
             if (e != hipSuccess) return e;
             attr_set[dev] = true;
         }
     }
-    const unsigned grid = (unsigned)((a.n_rows + rows_per_wg - 1) / rows_per_wg);
-    hipLaunchKernelGGL((rows_kernel<PRO, EPI, KSPLIT>), dim3(grid), dim3(ROWS_THREADS), lds, s, a, (int)rows_per_wg, plane);
+    hipLaunchKernelGGL((rows_kernel<PRO, EPI, U, V, Y>), dim3((unsigned)grid), dim3(ROWS_THREADS), lds, s, a, pl);
     return hipGetLastError();
 }
 
-template <int PRO, int EPI>
+template <int PRO, int EPI, int V, bool Y>
 static hipError_t rows_split(hipStream_t s, const RowsArgs &a, int n_cu) {
     const int64_t pairs = (a.n_rows + 1) / 2;
-    // fewer pairs of rows than wavefronts on half of the CUs: a workgroup per pair
-    if (pairs < 2 * n_cu && a.ld >= 1024) return rows_launch<PRO, EPI, true>(s, a, 2);
-    // about two workgroups per CU where the rows allow it; whole pairs of rows per wavefront
-    int64_t per = (pairs + (int64_t)2 * n_cu - 1) / ((int64_t)2 * n_cu);
-    per = (per + ROWS_WAVES - 1) / ROWS_WAVES * ROWS_WAVES;  // pairs per workgroup
-    return rows_launch<PRO, EPI, false>(s, a, 2 * per);
+    const int nvec = PRO == RP_DOWN ? a.top : 1;
+    auto steps = [&](int u) { return pairs * nvec * ((a.ld + 512 * u - 1) / (512 * u)); };
+    // two workgroups per CU where LDS holds their vectors and there is a step for every wavefront
+    const int64_t most = (rows_lds(a, PRO, (int)std::min<int64_t>(ROWS_MAX_PAIRS, pairs / (2 * n_cu) + 1)) > 78 * 1024 ? 1 : 2) * (int64_t)n_cu;
+    auto grid = [&](int u) {
+        const int64_t n = std::max<int64_t>(1, std::min(std::min(most, pairs), (steps(u) + ROWS_WAVES - 1) / ROWS_WAVES));
+        return std::max(n, (pairs + ROWS_MAX_PAIRS - 2) / (ROWS_MAX_PAIRS - 1));
+    };
+    // 4 KB of a row at a time where that leaves at least half of the wavefronts' places a step (a 4096 x 4096 matrix: 7.9 us, against
+    // 8.8 in steps of 1 KB); rows of up to 1024 inputs whole (3072 x 768: 3.5 us against 4.8 in two steps).  A pending update of
+    // more than 4096 elements takes the registers of the long steps.
+    if constexpr (!(Y && V > 2))
+        if (a.ld >= 2048 && steps(4) >= most * ROWS_WAVES / 2) return rows_launch<PRO, EPI, 4, V, Y>(s, a, grid(4));
+    if (a.ld > 512 && (steps(2) >= most * ROWS_WAVES / 2 || (a.ld <= 1024 && steps(2) >= n_cu))) return rows_launch<PRO, EPI, 2, V, Y>(s, a, grid(2));
+    return rows_launch<PRO, EPI, 1, V, Y>(s, a, grid(1));
+}
+
+// the vector's registers: two steps for up to 4096 elements behind a norm, four for more; eight for one that is staged as it is
+template <int PRO, int EPI>
+static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu) {
+    if constexpr (PRO == RP_PLAIN || PRO == RP_DOWN) {
+        return rows_split<PRO, EPI, 8, false>(s, a, n_cu);
+    } else if constexpr (PRO == RP_HEADNORM) {
+        return rows_split<PRO, EPI, 4, false>(s, a, n_cu);
+    } else {
+        const bool few = a.K <= 2 * 4 * ROWS_THREADS;
+        if constexpr (PRO == RP_NORM && (EPI == RE_STORE || EPI == RE_STORE_GLU)) {
+            if (a.y) return few ? rows_split<PRO, EPI, 2, true>(s, a, n_cu) : rows_split<PRO, EPI, 4, true>(s, a, n_cu);
+        }
+        if (a.y) return hipErrorInvalidValue;
+        return few ? rows_split<PRO, EPI, 2, false>(s, a, n_cu) : rows_split<PRO, EPI, 4, false>(s, a, n_cu);
+    }
 }
 
 hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu) {
@@ -356,7 +432,7 @@ hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu) 
     if ((epi == RE_GLU && a.n_rows % 2 != 0) || (epi == RE_STORE_GLU && (a.n_rows % 2 != 0 || a.glu_from % 2 != 0 || !a.out2)))
         return hipErrorInvalidValue;
 #define GO(P, E) \
-    if (pro == P && epi == E) return rows_split<P, E>(s, a, n_cu)
+    if (pro == P && epi == E) return rows_pick<P, E>(s, a, n_cu)
     GO(RP_NORM, RE_STORE);
     GO(RP_NORM, RE_ACT);
     GO(RP_PLAIN, RE_STORE);

@@ -75,6 +75,19 @@ __device__ __forceinline__ float l_block_sum(float v, float *red) {
     return t;
 }
 
+// a barrier that orders LDS traffic only: what the wavefronts have under way to and from memory stays under way
+__device__ __forceinline__ void l_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// l_block_sum with such a barrier; `red` is not used again behind it
+__device__ __forceinline__ float l_block_sum_lds(float v, float *red) {
+    const int nw = (blockDim.x + 63) >> 6;
+    v = l_wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    l_lds_barrier();
+    float t = 0.0f;
+    for (int w = 0; w < nw; w++) t += red[w];
+    return t;
+}
+
 // activations: bf16 or fp32 elements behind one pointer
 template <int PREC>
 __device__ __forceinline__ void l_store_act(void *p, int64_t i, float v) {
@@ -121,12 +134,19 @@ __device__ __forceinline__ void l_rotate_norm(const float *src, float *dst, int 
 
 // Choice of experts by one workgroup: an expert's place among all by its logit is the number of larger ones (the lower index
 // first among equals); sel[place], score[place] for the first `top` places.  zs: LDS for E logits; sel and score are LDS or
-// global memory of the workgroup's own.
+// global memory of the workgroup's own (IN_LDS: LDS, and the barriers order nothing else).
+template <bool IN_LDS>
 __device__ __forceinline__ void l_route(const float *z, const float *bias, int E, int top, int kind, float *zs, int *sel, float *score) {
     const int t = threadIdx.x, nt = blockDim.x;
+    auto route_barrier = [] {
+        if (IN_LDS)
+            l_lds_barrier();
+        else
+            __syncthreads();
+    };
     for (int e = t; e < E; e += nt) zs[e] = z[e] + (bias ? bias[e] : 0.0f);
     for (int k = t; k < top; k += nt) sel[k] = 0, score[k] = 0.0f;  // (a place that no number takes, with NaN among them, stays defined)
-    __syncthreads();
+    route_barrier();
     for (int e = t; e < E; e += nt) {
         const float v = zs[e];
         int rank = 0;
@@ -137,13 +157,13 @@ __device__ __forceinline__ void l_route(const float *z, const float *bias, int E
             score[rank] = kind == LROUTE_SIGMOID_IN ? l_sigmoid(v) : v;
         }
     }
-    __syncthreads();
+    route_barrier();
     if (kind == LROUTE_SOFTMAX_OUT) {
         if (t < 64) {  // (top <= 64)
             const float v = t < top ? score[t] : -INFINITY, m = wave_max_f32(v);
             const float p = t < top ? expf(v - m) : 0.0f, sum = l_wave_sum(p);
             if (t < top) score[t] = p / sum;
         }
-        __syncthreads();
+        route_barrier();
     }
 }

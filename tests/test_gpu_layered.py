@@ -186,6 +186,20 @@ def test_long_decoding(pkg):
     dev.close()
 
 
+@pytest.mark.parametrize("width,ff,eff,vocab", [(1030, 513, 515, 4099), (1024, 2050, 1024, 1026), (2112, 9000, 1100, 4099),
+                                                (4160, 700, 4096, 601), (8256, 16448, 24, 515)])
+def test_widths_of_a_decode_step(pkg, width, ff, eff, vocab):
+    """A step's products at the borders of their rules: vectors of up to 4096 and 8192 elements, longer ones and ones that are no
+    multiple of four; steps of 512, 1024 and 2048 inputs; row pairs that several wavefronts share, a last row without a partner"""
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=32, vdim=32, rot=32, mlp=lc.dense(ff)),
+                   lc.delta(heads=2, kv_heads=2, dim=32, vdim=32, conv=4, ranks=(16, 16), mlp=lc.moe(5, 3, eff))], width=width, vocab=vocab, side=24)
+    t = lc.settle_routers(c, ref.random_tensors(c, 41), 2)
+    tok = lc.tokens(3, c["vocab"], 8)
+    dev = lc.language_model(pkg, c, t).device()
+    assert lc.error(_decode(dev, tok), ref.Sequence(c, t).run(tok)) <= TOL["float32"]
+    dev.close()
+
+
 def test_prompt_longer_than_one_chunk(pkg):
     """2048 positions go at a time: a longer prompt continues from the cache and state its first chunk left"""
     c = lc.config([lc.delta(heads=2, kv_heads=1, dim=16, vdim=16, conv=4, ranks=(4, 4)), lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=40, rot=16)],
