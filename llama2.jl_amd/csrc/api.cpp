@@ -239,6 +239,7 @@ static void model_free_state(l2h_model *m) {
     m->pf_lt_tried = false;
     m->pf_plain = false;
     m->sample_p = nullptr;
+    m->sample_part = nullptr;
     m->sample_out = nullptr;
     m->finalized = false;
 }
@@ -1472,10 +1473,11 @@ extern "C" int l2h_sample(l2h_model *m, float temperature, float u, int32_t *tok
     HIPCHK(ctx, hipSetDevice(ctx->device));
     if (!m->sample_p) {
         int rc;
+        if (!m->sample_part && (rc = dalloc(m, &m->sample_part, L_SAMPLE_PART_DOUBLES, false))) return rc;
+        if (!m->sample_out && (rc = dalloc(m, &m->sample_out, 1, true))) return rc;
         if ((rc = dalloc(m, &m->sample_p, m->c.vocab_size, false))) return rc;
-        if ((rc = dalloc(m, &m->sample_out, 1, true))) return rc;
     }
-    HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_out));
+    HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_part, m->sample_out));
     HIPCHK(ctx, hipMemcpyAsync(token, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
     if (probs)
         HIPCHK(ctx, hipMemcpyAsync(probs, m->sample_p, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost, ctx->stream));

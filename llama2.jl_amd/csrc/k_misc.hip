@@ -389,49 +389,97 @@ hipError_t k_f32_to_f64(hipStream_t s, const float *x, double *y, int64_t n) {
 // temperature sampling (reference src/inference.jl:363-367): logits ./= T; softmax!; wsample.
 // wsample's walk is reproduced with a host-supplied uniform number u in [0, 1): the pick is the first
 // index whose cumulative weight reaches u * sum(weights).  exp in fp64 rounded to fp32 and the sums
-// in fp64 (as everywhere in this library); one workgroup, thread t owns a contiguous slice.
+// in fp64 (as everywhere in this library).
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void sample_kernel(const float *logits, int n, float temperature, float u,
-                                                      float *p, int32_t *out) {
-    __shared__ double redd[16];
-    __shared__ float redf[16];
-    __shared__ double s_cum[1025];
-    const int tid = threadIdx.x;
-    const int per = (n + 1023) / 1024, lo = min(n, tid * per), hi = min(n, lo + per);
+// In four launches over SAMPLE_PARTS workgroups at most, each a run of the logits: one workgroup alone took 558 us for 128 256 of
+// them (125 exponentials in fp64 a thread, and 1024 running sums added by one thread), the four take 18 us, which is what four
+// dependent launches take.  part: the runs' largest values, sums of exponentials, sums of probabilities.
+#define SAMPLE_THREADS 256
+#define SAMPLE_PARTS 256
+struct SampleRun {
+    int lo, hi;
+};
+__device__ __forceinline__ SampleRun sample_run(int n, int per, int b) {
+    return SampleRun{(int)min((int64_t)n, (int64_t)b * per), (int)min((int64_t)n, (int64_t)(b + 1) * per)};
+}
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(const float *logits, int n, int per, float temperature, float *p, double *part) {
+    __shared__ float red[SAMPLE_THREADS / 64];
+    const SampleRun r = sample_run(n, per, blockIdx.x);
     float mx = -INFINITY;
-    for (int i = lo; i < hi; i++) {
+    for (int i = r.lo + threadIdx.x; i < r.hi; i += SAMPLE_THREADS) {
         const float v = logits[i] / temperature;
         p[i] = v;
         mx = fmaxf(mx, v);
     }
-    mx = block_max_f32(mx, redf);
+    mx = block_max_f32(mx, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = (double)mx;
+}
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_exp_kernel(int n, int per, int parts, float *p, double *part) {
+    __shared__ float redf[SAMPLE_THREADS / 64];
+    __shared__ double red[SAMPLE_THREADS / 64];
+    const SampleRun r = sample_run(n, per, blockIdx.x);
+    const float mx = block_max_f32((int)threadIdx.x < parts ? (float)part[threadIdx.x] : -INFINITY, redf);
     double sum = 0.0;
-    for (int i = lo; i < hi; i++) {
+    for (int i = r.lo + threadIdx.x; i < r.hi; i += SAMPLE_THREADS) {
         const float e = (float)exp((double)(p[i] - mx));
         p[i] = e;
         sum += (double)e;
     }
-    const float sf = (float)block_sum_f64(sum, redd);
-    double mine = 0.0;
-    for (int i = lo; i < hi; i++) {
+    sum = block_sum_f64(sum, red);
+    if (threadIdx.x == 0) part[SAMPLE_PARTS + blockIdx.x] = sum;
+}
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int per, int parts, float *p, double *part) {
+    __shared__ double red[SAMPLE_THREADS / 64];
+    const SampleRun r = sample_run(n, per, blockIdx.x);
+    const float sf = (float)block_sum_f64((int)threadIdx.x < parts ? part[SAMPLE_PARTS + threadIdx.x] : 0.0, red);
+    double sum = 0.0;
+    for (int i = r.lo + threadIdx.x; i < r.hi; i += SAMPLE_THREADS) {
         const float pr = p[i] / sf;
         p[i] = pr;
-        mine += (double)pr;
-    }
-    s_cum[tid + 1] = mine;
-    __syncthreads();
-    if (tid == 0) {
-        s_cum[0] = 0.0;
-        for (int k = 1; k <= 1024; k++) s_cum[k] += s_cum[k - 1];
+        sum += (double)pr;
     }
     __syncthreads();
-    const double target = (double)u * s_cum[1024];
-    // the slice in which the cumulative weight first reaches the target (the last non-empty one if
-    // rounding leaves the target just above the total)
-    const bool here = lo < hi && s_cum[tid] < target && (target <= s_cum[tid + 1] || hi == n);
-    const bool first_zero = tid == 0 && target <= 0.0;
-    if (here || first_zero) {
-        double cw = s_cum[tid];
+    sum = block_sum_f64(sum, red);
+    if (threadIdx.x == 0) part[2 * SAMPLE_PARTS + blockIdx.x] = sum;
+}
+// running sums over the workgroup's values: cum[t + 1] = v of threads 0 .. t, cum[0] = 0
+__device__ void sample_scan(double v, double *cum) {
+    const int t = threadIdx.x;
+    if (t == 0) cum[0] = 0.0;
+    cum[t + 1] = v;
+    for (int d = 1; d < SAMPLE_THREADS; d *= 2) {
+        __syncthreads();
+        const double w = t + 1 > d ? cum[t + 1 - d] : 0.0;
+        __syncthreads();
+        cum[t + 1] += w;
+    }
+    __syncthreads();
+}
+// the first index at which the running sum reaches u times the whole (the last one of its run if rounding leaves the target just
+// above the total)
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(int n, int per, int parts, float u, const float *p, const double *part, int32_t *out) {
+    __shared__ double cum[SAMPLE_THREADS + 1];
+    __shared__ int s_at, s_pick;
+    const int t = threadIdx.x;
+    sample_scan(t < parts ? part[2 * SAMPLE_PARTS + t] : 0.0, cum);
+    const double target = (double)u * cum[parts];
+    if (t == 0) s_at = s_pick = 0x7FFFFFFF;
+    __syncthreads();
+    // (runs are not empty)
+    if (t < parts && ((cum[t] < target && (target <= cum[t + 1] || t == parts - 1)) || (t == 0 && target <= 0.0)))
+        atomicMin(&s_at, t);  // (rounding may leave a running sum a last bit below the one before it)
+    __syncthreads();
+    if (s_at == 0x7FFFFFFF) return;  // (not a number among the logits)
+    const SampleRun r = sample_run(n, per, s_at);
+    const double before = cum[s_at];
+    const int each = (per + SAMPLE_THREADS - 1) / SAMPLE_THREADS, lo = min(r.hi, r.lo + t * each), hi = min(r.hi, lo + each);
+    double mine = 0.0;
+    for (int i = lo; i < hi; i++) mine += (double)p[i];
+    __syncthreads();
+    sample_scan(mine, cum);
+    const bool last = hi == r.hi && lo < hi;
+    if (lo < hi && (before + cum[t] < target || t == 0) && (target <= before + cum[t + 1] || last)) {
+        double cw = before + cum[t];
         int pick = hi - 1;
         for (int i = lo; i < hi; i++) {
             cw += (double)p[i];
@@ -440,11 +488,17 @@ __global__ __launch_bounds__(1024) void sample_kernel(const float *logits, int n
                 break;
             }
         }
-        *out = pick;
+        atomicMin(&s_pick, pick);
     }
+    __syncthreads();
+    if (t == 0) *out = s_pick;
 }
 
-hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, int32_t *out) {
-    hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(1024), 0, s, logits, n, temperature, u, p, out);
+hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, int32_t *out) {
+    const int per = std::max(1024, (int)(((int64_t)n + SAMPLE_PARTS - 1) / SAMPLE_PARTS)), parts = (int)(((int64_t)n + per - 1) / per);
+    hipLaunchKernelGGL(sample_max_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, logits, n, per, temperature, p, part);
+    hipLaunchKernelGGL(sample_exp_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, n, per, parts, p, part);
+    hipLaunchKernelGGL(sample_prob_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, n, per, parts, p, part);
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(1), dim3(SAMPLE_THREADS), 0, s, n, per, parts, u, p, part, out);
     return hipGetLastError();
 }

@@ -239,7 +239,8 @@ hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, 
 // argmax without allocations: k_noalloc_init once per device (that device current), then k_argmax_noalloc
 hipError_t k_noalloc_init(int device);
 hipError_t k_argmax_noalloc(hipStream_t s, int device, const float *x_dev, int64_t n, int32_t *out_dev);
-hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, int32_t *out);
+#define L_SAMPLE_PART_DOUBLES (3 * 256)
+hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, int32_t *out);
 hipError_t k_kv_layout(hipStream_t s, float *kc, float *vc, float *k_lin, float *v_lin, int pos0, int n, int head_size,
                        int n_kv_heads, int seq_len, bool to_cache, int kv16);
 hipError_t k_stream_read(hipStream_t s, const uint4 *p, int64_t n16, uint32_t *sink);

@@ -67,6 +67,7 @@ struct l2h_model {
     long long *timeline = nullptr, *timeline2 = nullptr;
 #endif
     float *sample_p = nullptr;  // probabilities of the last l2h_sample call
+    double *sample_part = nullptr;
     int32_t *sample_out = nullptr;
     // streaming decode kernel
     bool flow = false;

@@ -491,6 +491,27 @@ def test_temperature_sampling_on_device(pkg, rng):
         dev.sample_token(1.0, 1.0)
 
 
+@pytest.mark.parametrize("vocab", [3, 1023, 1025, 4096, 262145, 300001])
+def test_sampling_over_any_number_of_logits(pkg, vocab):
+    """The draw is split into runs of 1024 logits, or of vocab / 256 from 262 144 on: its probabilities and picks against numpy at
+    the borders, on logits of which some are far below the rest."""
+    plan, kw = CASES["f32"]
+    dev = _model(pkg, plan, **dict(kw, vocab_size=vocab, n_layers=1)).device()
+    logits, _ = dev.forward(2, 0)
+    T = 0.02
+    xs = (logits / np.float32(T)).astype(np.float32)
+    e = np.exp((xs - xs.max()).astype(np.float64)).astype(np.float32)
+    p = (e / np.float32(e.astype(np.float64).sum())).astype(np.float32)
+    cum = np.cumsum(p.astype(np.float64))
+    assert np.allclose(dev.sample_token(T, 0.25, want_probs=True)[1], p, rtol=1e-6, atol=0)
+    for u in [0.0, 1e-9, 0.99999994] + np.random.default_rng(2).random(60).astype(np.float32).tolist():
+        tok, target = dev.sample_token(T, float(u)), float(np.float32(u)) * cum[-1]
+        want = min(int(np.searchsorted(cum, target, side="left")), vocab - 1)
+        if tok != want:  # only where the target lies within rounding of a running sum (one fp32 step of a probability, a few steps off)
+            assert abs(cum[min(tok, want)] - target) <= 1e-7, (u, tok, want)
+    dev.close()
+
+
 # Prompt pass (bf16 products of float activations) against sequential decode (q8_K activations, integer products) at
 # full depth: two roundings of the same sums whose difference grows with the layers (0.02-0.05 of the largest value
 # after 2 layers, about 0.2 after 32: observed 0.195 / 0.184 / 0.149 for logits / K / V, root mean square 0.19 / 0.17 /
