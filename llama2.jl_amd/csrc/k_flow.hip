@@ -129,7 +129,7 @@ __host__ __device__ inline int flow_half(const FlowGeom &g) {
 template <bool H = true>
 __host__ __device__ inline int flow_wg_pieces(const FlowGeom &g, int wg) {
     const int n = flow_n_local(g, wg), h = flow_half<H>(g);
-    return h ? (n >> 1) * h : n * g.ppr;
+    return h ? ((n + 1) >> 1) * h : n * g.ppr;  // (an odd number of rows: the classifier's last one alone)
 }
 // the first logical row that piece j of a workgroup holds super-blocks of
 __host__ __device__ inline int flow_piece_row(const FlowGeom &g, int j) {
@@ -769,10 +769,13 @@ __device__ __forceinline__ void flow_top_up_q6(Ring &r, unsigned char *ring_base
     }
 }
 
+// PAIR: rows of 2048 inputs (or up to a quarter less) go in pairs, one piece a pair: the lower 32 lanes hold the even row's
+// super-blocks, the upper 32 the odd one's, and a piece leaves two sums
+template <bool PAIR>
 __device__ __forceinline__ void flow_loop_q6(const FlowGeom &g, Ring &r, unsigned char *ring_base, int wg) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ppr = uni(g.ppr);
-    const int cnt = uni(flow_wave_pieces<false>(g, wg, wave)), start = uni(flow_wave_start<false>(g, wg, wave));
+    const int ppr = PAIR ? 1 : uni(g.ppr);
+    const int cnt = uni(flow_wave_pieces<PAIR>(g, wg, wave)), start = uni(flow_wave_start<PAIR>(g, wg, wave));
     const int b = lane >> 2, c = lane & 3, n = c >> 1, h = c & 1;
     const XLds x = flow_x();
     RingLoop<FLOW_Q6_PIECE, FLOW_Q6_D, 5> q;
@@ -799,6 +802,12 @@ __device__ __forceinline__ void flow_loop_q6(const FlowGeom &g, Ring &r, unsigne
             q.fetched();
         }
         q.next_slot();
+        if constexpr (PAIR) {
+            const double v = row16_sum_f64_dpp(chunk_term<false>(ch, lane & 31, x, nullptr, nullptr, 0));
+            const double even = readlane_f64(v, 0) + readlane_f64(v, 16), odd = readlane_f64(v, 32) + readlane_f64(v, 48);
+            if (lane < 2) s_part[2 * (start + k) + lane] = lane ? odd : even;
+            continue;
+        }
         acc += chunk_term<false>(ch, part * 64 + lane, x, nullptr, nullptr, 0);
         const bool last = k == cnt - 1 || part == ppr - 1;
         if (last) {
@@ -1205,7 +1214,7 @@ __device__ __noinline__ void flow_finish_cls(int wg, unsigned e_cls) {
     wg = uni(wg), e_cls = uni(e_cls);
     const FlowArgs &a = c_flow;
     const int n_local = flow_n_local(a.cls, wg), tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    flow_row_values<false>(n_local, a.cls.ppr);
+    flow_row_values<false>(n_local, a.cls.ppr ? a.cls.ppr : 1);  // (rows in pairs leave one sum each)
     unsigned long long best = 0;
     if (tid < n_local) {
         const int64_t row = (int64_t)wg * a.cls.rpw + tid;
@@ -1857,7 +1866,7 @@ __device__ __noinline__ bool flow_attention_split(int layer, int pos, unsigned e
 // n_tok: steps of the token loop (reference src/inference.jl:349-386) that this launch runs, one after the other; the
 // epochs of step t start at gen0 + t * (5 * n_layers + 2).
 // HALF (with MIXED): the layer matrices' rows of dim inputs end in the middle of a piece (FlowGeom::half)
-template <int T_CLS, bool MIXED, bool HALF = false>
+template <int T_CLS, bool MIXED, bool HALF = false, bool PAIR = false>
 __global__ __launch_bounds__(1024) void flow_token_kernel(unsigned int gen0, int n_tok) {
     const FlowArgs &a = c_flow;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1921,7 +1930,7 @@ __global__ __launch_bounds__(1024) void flow_token_kernel(unsigned int gen0, int
         ring_uniform(r);  // values that came through vector loads are the same on every lane: make them scalar
         // the register pieces follow the ring's part of the stream, in the order in which they are used
         reg_ptr = uni(r.gptr + (int64_t)a.n_layers * ring_layer * FLOW_SLOT +
-                      (int64_t)flow_wave_pieces<false>(a.cls, wg, wave) * (T_CLS == L2H_TYPE_Q6_K ? FLOW_Q6_PIECE : FLOW_SLOT));
+                      (int64_t)flow_wave_pieces<PAIR>(a.cls, wg, wave) * (T_CLS == L2H_TYPE_Q6_K ? FLOW_Q6_PIECE : FLOW_SLOT));
         flow_top_up_q4(r, ring_base, lane);
     }
     FTL();
@@ -2048,7 +2057,7 @@ __global__ __launch_bounds__(1024) void flow_token_kernel(unsigned int gen0, int
         if constexpr (MIXED) r.gptr = mr.gptr;
         r.issued = r.consumed = r.drain_mark = 0;
         r.off = 0;
-        r.left = flow_wave_pieces<false>(a.cls, wg, wave);
+        r.left = flow_wave_pieces<PAIR>(a.cls, wg, wave);
         ring_uniform(r);
         if (T_CLS == L2H_TYPE_Q6_K)
             flow_top_up_q6(r, ring_base, lane);
@@ -2066,7 +2075,7 @@ __global__ __launch_bounds__(1024) void flow_token_kernel(unsigned int gen0, int
     }
     flow_drain(r);
     if (T_CLS == L2H_TYPE_Q6_K)
-        flow_loop_q6(a.cls, r, ring_base, wg);
+        flow_loop_q6<PAIR>(a.cls, r, ring_base, wg);
     else
         flow_loop_q4<false, false>(a.cls, r, ring_base, wg, rp, 0);
     flow_finish_cls(wg, e_cls);
@@ -2464,17 +2473,24 @@ __global__ __launch_bounds__(64) void flow_repack_kernel(FlowRepackArgs p) {
     } else {  // q6_K classifier
         const int64_t off = cls_at;
         uint4 *dst = (uint4 *)(p.stream + p.wave_off[wg * FLOW_NW + wave] + off + (int64_t)idx * FLOW_Q6_PIECE);
-        const int64_t blk0 = row * t.nb + part * 16;
-        const int nbv = (int)min((int64_t)16, max((int64_t)0, t.nb - (int64_t)part * 16));  // (16 unless the row is padded)
+        // super-block b of the piece: its place in the tensor; valid unless the row is padded or, in a pair, not there
         const uint4 z4 = make_uint4(0u, 0u, 0u, 0u);
-        const uint4 *ql = (const uint4 *)(t.qs + blk0 * 128), *qh = (const uint4 *)(t.qh + blk0 * 64);
-        dst[lane] = (lane >> 3) < nbv ? ql[lane] : z4;
-        dst[64 + lane] = 8 + (lane >> 3) < nbv ? ql[64 + lane] : z4;
-        dst[128 + lane] = (lane >> 2) < nbv ? qh[lane] : z4;
-        if (lane < 16) dst[192 + lane] = lane < nbv ? ((const uint4 *)(t.sc6 + blk0 * 4))[lane] : z4;
+        auto at = [&](int b, int64_t &bi) -> bool {
+            if (half) {
+                bi = (row + (b >> 3)) * t.nb + (b & 7);
+                return (b & 7) < t.nb && row + (b >> 3) < g.n_rows;
+            }
+            bi = row * t.nb + part * 16 + b;
+            return (int64_t)part * 16 + b < t.nb;
+        };
+        int64_t bi;
+        dst[lane] = at(lane >> 3, bi) ? ((const uint4 *)(t.qs + bi * 128))[lane & 7] : z4;
+        dst[64 + lane] = at(8 + (lane >> 3), bi) ? ((const uint4 *)(t.qs + bi * 128))[lane & 7] : z4;
+        dst[128 + lane] = at(lane >> 2, bi) ? ((const uint4 *)(t.qh + bi * 64))[lane & 3] : z4;
+        if (lane < 16) dst[192 + lane] = at(lane, bi) ? ((const uint4 *)(t.sc6 + bi * 4))[0] : z4;
         if (lane < 2) {
             uint16_t dd[8];
-            for (int b = 0; b < 8; b++) dd[b] = 8 * lane + b < nbv ? t.d6[blk0 + 8 * lane + b] : (uint16_t)0;
+            for (int b = 0; b < 8; b++) dd[b] = at(8 * lane + b, bi) ? t.d6[bi] : (uint16_t)0;
             dst[208 + lane] = make_uint4(dd[0] | (uint32_t)dd[1] << 16, dd[2] | (uint32_t)dd[3] << 16,
                                          dd[4] | (uint32_t)dd[5] << 16, dd[6] | (uint32_t)dd[7] << 16);
         }
@@ -2505,9 +2521,10 @@ static FlowGeom make_geom(int64_t n_rows, int64_t K, int type, int grid, bool ha
 }
 
 // Can the model run on this kernel?  q4_K layer matrices with input lengths that are multiples of
-// 2048 (whole pieces per row), a q4_K or q6_K classifier (q6_K: multiples of 4096), and sizes that
+// 2048 (whole pieces per row), a q4_K or q6_K classifier, and sizes that
 // fit the kernel's LDS areas.  On success fills the geometry fields of `a` for a grid of `grid`.
-bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why) {
+// cls_pairs: a q6_K classifier with dim_pad 2048 may run with its rows in pairs.
+bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why, bool cls_pairs) {
     auto no = [&](const char *m) {
         if (why) *why = m;
         return false;
@@ -2560,7 +2577,7 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
     if (a.dim % 256 != 0 || (int64_t)a.dim * 4 < (int64_t)a.dim_pad * 3 || a.hidden % 2048 != 0)
         return no("dim must be a multiple of 2048 (or of 256 and within a quarter below one), hidden_dim a multiple of 2048");
     if (a.dim_pad != a.dim) a.mixed = 1;
-    if (cls_type == L2H_TYPE_Q6_K && a.dim_pad % 4096 != 0) return no("a q6_K classifier needs dim to be a multiple of 4096");
+    if (cls_type == L2H_TYPE_Q6_K && a.dim_pad % 4096 != 0 && !cls_pairs) return no("a q6_K classifier needs dim to be a multiple of 4096");
     if (a.hidden > 14336 || a.dim_pad > 4096) return no("dim above 4096 or hidden_dim above 14336");
     if (a.n_heads > grid || (a.hs != 32 && a.hs != 64 && a.hs != 96 && a.hs != 128)) return no("head size must be 32, 64, 96 or 128");
     if (a.hs == 96) a.mixed = 1;
@@ -2579,6 +2596,10 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
     a.w13 = make_geom(2 * (int64_t)a.hidden, halves ? a.dim : a.dim_pad, L2H_TYPE_Q4_K, grid, halves);
     a.w2 = make_geom(a.dim, a.hidden, L2H_TYPE_Q4_K, grid);
     a.cls = make_geom(a.vocab, a.dim_pad, cls_type, grid);
+    if (cls_type == L2H_TYPE_Q6_K && a.dim_pad % 4096 != 0) {  // (the same pieces of 16 super-blocks, two rows to a piece)
+        a.cls.ppr = 0;
+        a.cls.K = 1024;
+    }
     const FlowGeom *gs[5] = {&a.qkv, &a.wo, &a.w13, &a.w2, &a.cls};
     for (const FlowGeom *g : gs)
         if (g->rpw > FLOW_MAX_ROWS || flow_wg_capacity(*g) > (g == &a.cls ? FLOW_MAX_PIECES : FLOW_MAX_PIECES / 4))
@@ -2689,9 +2710,11 @@ hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a) {
 // else.  The kernel has no grid-wide barrier and every wait in it is bounded, so residency is what makes it
 // fast, not what makes it correct: workgroups that had to wait for a CU would let the others run into their
 // wait limit, and the launch would end with the error that l2h_model_set_wait_limit describes.
-// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece
+// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs
 static const void *flow_kernel_fn(int cls_type, int form) {
     if (cls_type == L2H_TYPE_F32) return (const void *)flow_f32_kernel;
+    if (form == 4) return (const void *)flow_token_kernel<L2H_TYPE_Q6_K, false, false, true>;
+    if (form == 5) return (const void *)flow_token_kernel<L2H_TYPE_Q6_K, true, false, true>;
     if (form == 2)
         return cls_type == L2H_TYPE_Q6_K ? (const void *)flow_token_kernel<L2H_TYPE_Q6_K, true, true>
                                          : (const void *)flow_token_kernel<L2H_TYPE_Q4_K, true, true>;

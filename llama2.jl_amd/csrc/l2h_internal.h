@@ -136,6 +136,7 @@ struct FlowGeom {
     int rpw;     // rows per workgroup (even)
     int ppr;     // pieces per row; 0: rows of K = 1024 (2 i + 1) inputs end in the middle of a piece and go in pairs of
                  // K / 1024 pieces, the pair's middle piece holding the end of the even row and the start of the odd one
+                 // (a q6_K classifier of 2048 inputs: ppr 0 and K 1024, two rows to a piece of 16 super-blocks)
     int K;       // input length
 };
 struct FlowArgs {
@@ -179,7 +180,7 @@ struct FlowArgs {
 #endif
 };
 // layer_types: per layer the ggml types of wq, wk, wv, wo, w1, w2, w3 (seven numbers a layer)
-bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why);
+bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why, bool cls_pairs = false);
 int64_t k_flow_offsets(const FlowArgs &a, int cls_type, int grid, std::vector<int64_t> &off);
 // Where every typed piece goes (a.mixed): per wavefront the stream's offset, the index of its first piece in the
 // per-piece tables, where its classifier pieces start, the types of its first pieces; per piece the byte offset in
@@ -200,10 +201,10 @@ hipError_t k_flow_repack(hipStream_t s, const FlowArgs &a, unsigned char *stream
                          int layer, const DevTensor *w, int nw, int grid, int cls_type, const FlowTypedDev &typed);
 hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a);
 // one launch runs n_tok steps of the token loop; the epochs of the launch start at gen0 and take 5 * n_layers + 2 per step
-// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece (flow_form)
+// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs (flow_form)
 hipError_t k_flow_launch(hipStream_t s, unsigned int gen0, int n_tok, int cls_type, int grid, int form);
 bool k_flow_fits(int cls_type, int grid, int n_cu, int form);
-inline int flow_form(const FlowArgs &a) { return a.mixed ? (a.qkv.ppr == 0 ? 2 : 1) : 0; }
+inline int flow_form(const FlowArgs &a) { return (a.mixed ? (a.qkv.ppr == 0 ? 2 : 1) : 0) + (!a.f32 && a.cls.ppr == 0 ? 4 : 0); }
 
 // ---- launchers (kernel files) ----------------------------------------------------------------
 // Each returns hipGetLastError() of its launch.

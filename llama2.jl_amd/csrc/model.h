@@ -73,6 +73,7 @@ struct l2h_model {
     bool flow = false;
     FlowArgs flow_args{};
     int flow_grid = 0, flow_cls_type = 0;
+    bool flow_holds_state = false;  // the activations of the last step are in flow_args' words
     std::string flow_why;  // why the streaming kernel was not chosen (empty if it was, or if it was not asked for)
     unsigned int flow_gen = 1;  // epoch of the next launch's input; 0 is what cleared memory holds
     // batched prompt pass: buffers for pf_cap positions, allocated at the first l2h_prefill

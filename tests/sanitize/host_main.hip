@@ -21,7 +21,7 @@ static int fails = 0;
     } while (0)
 
 static void check_shape(int dim, int hidden, int n_layers, int n_heads, int n_kv, int vocab, int seq_len, const int *layer7,
-                        int cls_type, int kv16, bool expect_fit) {
+                        int cls_type, int kv16, bool expect_fit, bool cls_pairs = false) {
     const int grid = 256;
     FlowArgs a{};
     a.dim = dim, a.hidden = hidden, a.n_layers = n_layers, a.n_heads = n_heads, a.n_kv_heads = n_kv;
@@ -30,7 +30,7 @@ static void check_shape(int dim, int hidden, int n_layers, int n_heads, int n_kv
     for (int l = 0; l < n_layers; l++)
         for (int k = 0; k < 7; k++) types.push_back(layer7[k]);
     std::string why;
-    const bool fit = k_flow_plan(a, types.data(), (int)types.size(), cls_type, grid, &why);
+    const bool fit = k_flow_plan(a, types.data(), (int)types.size(), cls_type, grid, &why, cls_pairs);
     EXPECT(fit == expect_fit);
     if (!fit) {
         EXPECT(!why.empty());
@@ -134,6 +134,9 @@ int main() {
     check_shape(3072, 8192, 2, 32, 32, 32064, 4096, q4, 12, 1, true);     // the same with an fp16 cache
     check_shape(2048, 4096, 3, 16, 4, 1000, 160, q4, 14, 0, false);       // q6_K classifier needs 4096
     check_shape(2048, 4096, 3, 16, 4, 1000, 160, q4, 12, 0, true);
+    check_shape(2048, 8192, 3, 16, 4, 1001, 160, q4, 14, 0, true, true);  // ... unless its rows may go in pairs
+    check_shape(1792, 4096, 2, 28, 4, 999, 160, q5m, 14, 0, false, true); // (28 heads do not divide the workgroups)
+    check_shape(1536, 4096, 2, 16, 4, 999, 160, mix, 14, 0, true, true);
     check_shape(1536, 2048, 2, 16, 16, 999, 96, q4, 12, 0, true);         // a quarter below 2048: padded rows
     check_shape(3072, 8192, 2, 32, 8, 32064, 512, mix, 12, 0, true);      // halves with typed pieces and grouped heads
     check_shape(1024, 2048, 2, 16, 16, 999, 96, q4, 12, 0, false);        // half below: refused

@@ -653,3 +653,57 @@ def test_streaming_kernel_other_shapes_against_per_phase_path(pkg, shape):
         assert np.array_equal(a_logits.view(np.uint32), b_logits.view(np.uint32)), (shape, rep)
     fast.close()
     slow.close()
+
+
+PAIRED = [
+    # a q6_K classifier whose rows are half a piece: two rows to a piece; odd vocabularies, rows a quarter below a half, one row
+    # or a few per workgroup, every type of layer matrix
+    ("PLAN_Q4_K_S", 2048, 8192, 1, 16, 4, 5001, False),
+    ("PLAN_Q5_K_M", 2048, 2048, 2, 32, 32, 258, True),
+    ("PLAN_Q4_K_S", 1536, 2048, 2, 16, 4, 333, False),
+    ("PLAN_Q4_K_S", 2048, 2048, 1, 32, 8, 130001, False),
+]
+
+
+@pytest.mark.parametrize("shape", range(len(PAIRED)))
+def test_streaming_kernel_with_paired_classifier_rows(pkg, shape):
+    """Tokens, logits and the activations of the last step against the per-phase path, bit for bit; by number such a model is
+    refused, as before."""
+    from llama2_jl_amd import synth
+    from llama2_jl_amd.inference import DeviceModel
+    plan, dim, hidden, layers, heads, kv, vocab, neox = PAIRED[shape]
+    lm = _model(pkg, plan, dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=heads, n_kv_heads=kv, vocab_size=vocab,
+                seq_len=320, rope_freq_base=10000.0, rope_is_neox=neox)
+    with pytest.raises(pkg.L2HError):
+        DeviceModel(lm.config, lm.weights, path=3)
+    fast, slow = DeviceModel(lm.config, lm.weights), DeviceModel(lm.config, lm.weights, path=1)
+    assert fast.path == 3 and slow.path == 1
+    for rep, n_new in enumerate((24, 300)):
+        prompt = synth.seeded_prompt(60 + rep, 3 + 4 * rep, vocab)
+        a_ids, a_logits = fast.generate_greedy(prompt, n_new, want_logits=True)
+        b_ids, b_logits = slow.generate_greedy(prompt, n_new, want_logits=True)
+        assert np.asarray(a_ids).tolist() == np.asarray(b_ids).tolist(), (shape, rep)
+        assert np.array_equal(a_logits.view(np.uint32), b_logits.view(np.uint32)), (shape, rep)
+        for name in ("x", "xb", "q", "hb", "logits"):
+            assert np.array_equal(fast.state(name), slow.state(name)), (shape, rep, name)
+    fast.prefill(synth.seeded_prompt(9, 20, vocab))
+    slow.prefill(synth.seeded_prompt(9, 20, vocab))
+    assert np.max(np.abs(fast.state("x") - slow.state("x"))) <= 1e-3 * np.max(np.abs(slow.state("x")))
+    fast.close()
+    slow.close()
+
+
+@pytest.mark.parametrize("case", sorted(FLOW_CASES))
+def test_state_after_a_step_of_the_streaming_kernel(pkg, case):
+    """RunState buffers as the per-phase path leaves them"""
+    from llama2_jl_amd.inference import DeviceModel
+    plan, kw = FLOW_CASES[case]
+    lm = _model(pkg, plan, **kw)
+    fast, slow = DeviceModel(lm.config, lm.weights, path=3), DeviceModel(lm.config, lm.weights, path=1)
+    for pos, token in enumerate((3, 7, 1)):
+        fast.forward(token, pos)
+        slow.forward(token, pos)
+        for name in ("x", "xb", "q", "hb", "logits"):
+            assert np.array_equal(fast.state(name), slow.state(name)), (pos, name)
+    fast.close()
+    slow.close()
