@@ -1198,6 +1198,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
         a->tiles = l->tiles;
         a->n_tiles = l->n_tiles;
         a->max_tiles = max_tiles;
+        a->rows_each = slots / d.n_experts;
     }
     const int epi = d.ff_gated ? GE_GLU : GE_UP;
     up.n_rows = L.up_rows();

@@ -100,11 +100,18 @@ struct GemmArgs {
     const int32_t *n_tiles = nullptr;
     int max_tiles = 0;
     int64_t expert_stride = 0;
+    int rows_each = 0;  // rows of a matrix on average
     const int32_t *gather = nullptr;  // row of x for each row of the product
 };
 #define L_GEMM_TILE 128   // rows of a block for k_gemm ...
 #define L_IMAGE_TILE 256  // ... and for k_tiles
 hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
+// the same for few rows or positions (k_few.hip; k_gemm chooses); cols: columns the epilogue covers
+#define L_FEW_M 128      // up to so many positions
+#define L_FEW_EACH 48    // ... of an expert
+#define L_FEW_TILES 256  // or fewer 64 x 64 tiles of results than this: 509 positions x 1024 rows, 1024 inputs, fp32: 15 us against 26;
+                         // at 424 tiles (3400 rows) the two take the same
+hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations
 hipError_t k_tiles(hipStream_t s, const GemmArgs &a, int epi);

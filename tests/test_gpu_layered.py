@@ -200,6 +200,22 @@ def test_widths_of_a_decode_step(pkg, width, ff, eff, vocab):
     dev.close()
 
 
+@pytest.mark.parametrize("precision", ["float32", "bfloat16"])
+def test_short_prompts(pkg, precision):
+    """The products of few positions: 16, 32 and 64 at a time and one more, 16 and 32 rows of a matrix at a time, experts with as
+    many positions and more, inputs that do not go round eight wavefronts, row counts that are no multiple of anything"""
+    c = lc.config([lc.attention(heads=5, kv_heads=5, dim=32, vdim=32, rot=32, mlp=lc.dense(515)),
+                   lc.delta(heads=3, kv_heads=3, dim=32, vdim=32, conv=4, ranks=(70, 33), mlp=lc.moe(5, 2, 70))], width=334, vocab=8210, side=40)
+    t = lc.settle_routers(c, ref.random_tensors(c, 43), 3)
+    tok = lc.tokens(140, c["vocab"], 9)
+    want = ref.Sequence(c, t).run(tok)
+    dev = lc.language_model(pkg, c, t, precision=precision).device()
+    for n in (2, 15, 16, 17, 32, 33, 63, 64, 65, 127, 128, 129, 140):
+        at = np.arange(max(0, n - 64), n)
+        assert lc.error(dev.prefill_logits(tok[:n], at), want[at]) <= TOL[precision], n
+    dev.close()
+
+
 def test_prompt_longer_than_one_chunk(pkg):
     """2048 positions go at a time: a longer prompt continues from the cache and state its first chunk left"""
     c = lc.config([lc.delta(heads=2, kv_heads=1, dim=16, vdim=16, conv=4, ranks=(4, 4)), lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=40, rot=16)],
