@@ -352,10 +352,9 @@ hipError_t k_latent_attend(hipStream_t s, const LatentShape &w, const float *qa,
 template <int PREC>
 __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w, const float *part, const uint16_t *ukv, int ldu,
                                                                   const float *raw, int64_t ldr, void *outa, int64_t lda, int64_t cols,
-                                                                  int n_split) {
+                                                                  int n_split, int M, int pos0, const DecodeCtl *ctl) {
     extern __shared__ __align__(16) float s_mem[];
     __shared__ float s_f[L_LATENT_SPLITS];
-    __shared__ int s_used;
     const int h = blockIdx.x, e0 = blockIdx.y * LV_ROWS, m = blockIdx.z, t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int Cp = w.Cp(), st = Cp + 4, nq = Cp / 4, ng = LV_THREADS / nq;  // (Cp <= 1024)
     float *s_c = s_mem, *s_acc = s_c + ldu;
@@ -369,13 +368,22 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
         const int e = e0 + wave * RW + i;
         wr[i] = e < w.V && 8 * lane < ldu ? *(const uint4 *)(rows + (int64_t)e * ldu + 8 * lane) : make_uint4(0, 0, 0, 0);
     }
+    float gate[RW];
+#pragma unroll
+    for (int i = 0; i < RW; i++) {
+        const int e = e0 + wave * RW + i;
+        gate[i] = w.gated && e < w.V ? raw[(int64_t)m * ldr + w.off_g() + (int64_t)h * w.V + e] : 0.0f;
+    }
+    // the runs that have keys (latent_attend_kernel): at 70 positions three of 128; asking for all their sums took 7 us of HBM
+    const int n_cols = M * w.H, c0 = (m * w.H + h) & ~15, n_keys = (ctl ? ctl->pos : pos0) + min(c0 + 15, n_cols - 1) / w.H + 1;
+    const int run = ((n_keys + n_split - 1) / n_split + 31) / 32 * 32, used = min(n_split, (n_keys + run - 1) / run);
     const int cq = t % nq, cg = t / nq;
     float4 v[LV_U];
     auto fetch = [&](int i0) {
 #pragma unroll
         for (int u = 0; u < LV_U; u++) {
             const int i = i0 + cg + u * ng;
-            v[u] = cg < ng && i < n_split ? *(const float4 *)(p + (int64_t)i * st + 4 + 4 * cq) : lat_zero4();
+            v[u] = cg < ng && i < used ? *(const float4 *)(p + (int64_t)i * st + 4 + 4 * cq) : lat_zero4();
         }
     };
     fetch(0);
@@ -385,8 +393,8 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
 #pragma unroll
         for (int u = 0; u < N; u++) {
             const int i = t + 64 * u;
-            mv[u] = i < n_split ? p[(int64_t)i * st] : -INFINITY;
-            lv[u] = i < n_split ? p[(int64_t)i * st + 1] : 0.0f;
+            mv[u] = i < used ? p[(int64_t)i * st] : -INFINITY;
+            lv[u] = i < used ? p[(int64_t)i * st + 1] : 0.0f;
             mx = fmaxf(mx, mv[u]);
         }
         mx = wave_max_f32(mx);
@@ -398,25 +406,18 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
         l = l_wave_sum(l);
 #pragma unroll
         for (int u = 0; u < N; u++) s_f[t + 64 * u] = mv[u] / l;
-        int used = 0;  // runs up to the last one with keys
-#pragma unroll
-        for (int u = 0; u < N; u++) {
-            const unsigned long long b = __ballot(mv[u] != 0.0f);
-            if (b) used = 64 * u + 64 - __builtin_clzll(b);
-        }
-        if (t == 0) s_used = used;
     }
     for (int i = Cp + t; i < ldu; i += LV_THREADS) s_c[i] = 0.0f;
     __syncthreads();
     if (cg < ng) {
         float4 a = lat_zero4();
-        for (int i0 = 0; i0 < s_used; i0 += LV_U * ng) {
+        for (int i0 = 0; i0 < used; i0 += LV_U * ng) {
             if (i0) fetch(i0);
 #pragma unroll
             for (int u = 0; u < LV_U; u++) {
                 const int i = i0 + cg + u * ng;
                 const float f = i < n_split ? s_f[i] : 0.0f;
-                if (f == 0.0f) continue;  // (a run without keys, whose sums were not written)
+                if (f == 0.0f) continue;  // (a run of which the token sees no key)
                 a.x = fmaf(f, v[u].x, a.x);
                 a.y = fmaf(f, v[u].y, a.y);
                 a.z = fmaf(f, v[u].z, a.z);
@@ -458,22 +459,22 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
         const int e = e0 + wave * RW + i;
         if (lane == i && e < w.V) {
             const int64_t at = (int64_t)h * w.V + e;
-            l_store_act<PREC>(outa, m * lda + at, w.gated ? a * l_sigmoid(raw[(int64_t)m * ldr + w.off_g() + at]) : a);
+            l_store_act<PREC>(outa, m * lda + at, w.gated ? a * l_sigmoid(gate[i]) : a);
         }
     }
     if (h == w.H - 1 && blockIdx.y == 0)
         for (int64_t i = (int64_t)w.H * w.V + t; i < cols; i += LV_THREADS) l_store_act<PREC>(outa, m * lda + i, 0.0f);
 }
 hipError_t k_latent_value(hipStream_t s, const LatentShape &w, const float *part, const uint16_t *ukv, int ldu, const float *raw,
-                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec) {
+                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec, int pos0, const DecodeCtl *ctl) {
     if (M < 1 || w.C > L_LATENT_MAX_RANK || ldu % 64 != 0 || ldu < w.C || cols > lda || cols < (int64_t)w.H * w.V) return hipErrorInvalidValue;
     const int ns = latent_splits((int64_t)M * w.H), nq = w.Cp() / 4, ng = LV_THREADS / nq;
     const size_t lds = ((size_t)ldu + (size_t)ng * w.Cp()) * sizeof(float);
     const dim3 grid((unsigned)w.H, (unsigned)((w.V + LV_ROWS - 1) / LV_ROWS), (unsigned)M);
     if (prec)
-        hipLaunchKernelGGL((latent_value_kernel<1>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns);
+        hipLaunchKernelGGL((latent_value_kernel<1>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, M, pos0, ctl);
     else
-        hipLaunchKernelGGL((latent_value_kernel<0>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns);
+        hipLaunchKernelGGL((latent_value_kernel<0>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, M, pos0, ctl);
     return hipGetLastError();
 }
 
