@@ -482,7 +482,7 @@ __global__ __launch_bounds__(256) void pf_gemm_kernel(PfGemmArgs a) {
 // the 8 XCDs in turn, so workgroup w takes tile (w % 8) * per + w / 8: each XCD works through a contiguous run of tiles,
 // positions fastest, and the workgroups that share a weight tile share an L2.
 
-// the tile (row group nt, position block mt) of one workgroup; s_all: two stages of LDS
+// the tile (row group nt, position block mt) of one workgroup
 template <int EPI, int JT>
 __device__ __forceinline__ void pf_gemm_bf16_tile(const PfGemmArgs &a, unsigned nt, unsigned mt, uint4 *s_all) {
     const int64_t n0 = (int64_t)nt * 256;
@@ -976,7 +976,7 @@ hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave
             const unsigned n_mt = (unsigned)((M + 64 * jt - 1) / (64 * jt)), n_tiles = n_mt * nnt;
             const unsigned per = (n_tiles + 7) / 8;
             const dim3 grid(8 * per);
-            const size_t lds = 2 * (size_t)(32768 + 64 * jt * 128);
+            const size_t lds = (size_t)pf_tile_lds(jt);
 #define GO(E, J)                                                                                              \
     do {                                                                                                      \
         static bool attr_set[PF_MAX_DEVICES] = {}; /* the attribute is kept per device */                     \
@@ -1014,7 +1014,7 @@ hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave
             if (na <= n_nt) {
                 const unsigned t4 = na * n_mt4, t2 = (n_nt - na) * n_mt2, per4 = (t4 + 7) / 8, per2 = (t2 + 7) / 8;
                 const dim3 grid(8 * (per4 + per2));
-                const size_t lds = 2 * (size_t)(32768 + 256 * 128);
+                const size_t lds = (size_t)std::max(pf_tile_lds(4), pf_tile_lds(2));
 #define GO(E)                                                                                                       \
     do {                                                                                                            \
         static bool attr_set[PF_MAX_DEVICES] = {};                                                                  \

@@ -83,7 +83,7 @@ __global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, u
 
 template <int EPI, int JT, bool GROUPED>
 static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, unsigned n_mt) {
-    constexpr int lds = 2 * (32768 + 64 * JT * 128);
+    constexpr int lds = pf_tile_lds(GROUPED && pf_tile_lds(2) > pf_tile_lds(JT) ? 2 : JT);  // (a grouped one runs both)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;

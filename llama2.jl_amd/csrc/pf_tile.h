@@ -31,17 +31,22 @@ __host__ __device__ __forceinline__ int pf_swz(int r) { return (r >> 1) & 7; }
 // 32 JT positions.  Both operand tiles of a K step travel from global memory
 // straight into LDS (16 bytes per lane and load, a wavefront's load filling 1 KB in lane order): the weight
 // tile is a linear copy of its 32 KB image, the position tile gets the c ^ pf_swz(r) placement by the choice
-// of the address each lane reads.  Two LDS stages: the loads of step kt + 1 are in flight during the products
-// of step kt, one barrier per step.
+// of the address each lane reads.  The loads of step kt + 1 are in flight during the products of step kt, one barrier
+// per step, with two LDS stages of 64 KB; of the 48 KB stages of JT = 2 three fit, and the loads of step kt + 2 are in
+// flight too: where such tiles do not fill the chip a step takes as long as its loads (333 positions x 14 336 rows x 4096
+// inputs: 98 us with two stages, 88 with three).
 typedef uint32_t pf_u32x4 __attribute__((ext_vector_type(4)));
 
-// wtiles: the row group's tiles, K / 64 of them in a row; act: bf16 rows of K elements; s_all: two stages of LDS.  row(r) is the
+constexpr int pf_tile_stage(int jt) { return 32768 + 64 * jt * 128; }  // bytes: weight tile, then position tile
+constexpr int pf_tile_stages(int jt) { return jt == 2 ? 3 : 2; }
+constexpr int pf_tile_lds(int jt) { return pf_tile_stages(jt) * pf_tile_stage(jt); }
+
+// wtiles: the row group's tiles, K / 64 of them in a row; act: bf16 rows of K elements; s_all: pf_tile_lds(JT) bytes of LDS.  row(r) is the
 // activation row of the tile's position r; epi(acc, wn, wm, lane) takes the results: a lane holds position
 // 32 JT wm + 32 j + lane % 32 and, in register r of tile i, weight row 64 wn + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4.
 template <int JT, class Row, class Epi>
 __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const uint16_t *act, int64_t K, uint4 *s_all, Row row, Epi epi) {
-    constexpr int MT = 64 * JT;                   // positions per workgroup
-    constexpr int STAGE = 32768 + MT * 128;       // bytes: weight tile, then position tile
+    constexpr int STAGE = pf_tile_stage(JT), STAGES = pf_tile_stages(JT);
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), wn = wave & 3, wm = wave >> 2;
     const int64_t nk = K >> 6;
 
@@ -147,14 +152,18 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
     } while (0)
 
     issue(0);
+    if (STAGES == 3 && nk > 1) issue(1);
+    int stage = 0, free_stage = STAGES - 1;
     for (int64_t kt = 0; kt < nk; kt++) {
-        const int stage = (int)(kt & 1);
-        // this wavefront's loads of the stage have landed; the barrier says the same of the others' and that
-        // everyone is done reading the other stage (its last PF_WAIT retired every read), which the next loads
-        // then overwrite
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // this wavefront's loads of the stage have landed (with three stages, all but those of the next one); the barrier
+        // says the same of the others' and that everyone is done reading the stage before (its last PF_WAIT retired every
+        // read), which the next loads then overwrite
+        if (STAGES == 3 && kt + 1 < nk)
+            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
-        if (kt + 1 < nk) issue(stage ^ 1);
+        if (kt + STAGES - 1 < nk) issue(free_stage);
         const unsigned sb = lds0 + (unsigned)(stage * STAGE);
         PF_READ(F0, 0);
         PF_READ(F1, 1);
@@ -168,6 +177,8 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
         PF_PRODUCTS(F0);
         PF_WAIT(F1, true);
         PF_PRODUCTS(F1);
+        free_stage = stage;
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
 #undef PF_PRODUCTS
 #undef PF_WAIT
