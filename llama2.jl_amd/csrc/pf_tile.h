@@ -151,35 +151,77 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
         }                                                                                                         \
     } while (0)
 
-    issue(0);
-    if (STAGES == 3 && nk > 1) issue(1);
-    int stage = 0, free_stage = STAGES - 1;
-    for (int64_t kt = 0; kt < nk; kt++) {
-        // this wavefront's loads of the stage have landed (with three stages, all but those of the next one); the barrier
-        // says the same of the others' and that everyone is done reading the stage before (its last PF_WAIT retired every
-        // read), which the next loads then overwrite
-        if (STAGES == 3 && kt + 1 < nk)
-            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        if (kt + STAGES - 1 < nk) issue(free_stage);
-        const unsigned sb = lds0 + (unsigned)(stage * STAGE);
-        PF_READ(F0, 0);
-        PF_READ(F1, 1);
-        PF_WAIT(F0, false);
-        PF_PRODUCTS(F0);
-        PF_READ(F0, 2);
-        PF_WAIT(F1, false);
-        PF_PRODUCTS(F1);
-        PF_READ(F1, 3);
-        PF_WAIT(F0, false);
-        PF_PRODUCTS(F0);
-        PF_WAIT(F1, true);
-        PF_PRODUCTS(F1);
-        free_stage = stage;
-        stage = stage + 1 == STAGES ? 0 : stage + 1;
+    // A stage is entered in the middle of the products of the one before: when its last slice's operands are in registers, a
+    // wavefront waits for its loads of the next stage, meets the others at the barrier (which says that the next stage is
+    // whole and that everyone is done reading this one), sends the loads that overwrite this stage and asks for the next
+    // stage's first slice, all before the products of the last slice: the matrix cores do not wait for the barrier or for
+    // the first reads behind it.  (2048 positions x 28 672 rows x 4096 inputs in 256 x 256 and 256 x 128 tiles: 473 us with the
+    // barrier between the slices of two stages, 439 like this.)
+    constexpr int AHEAD = STAGES - 1;  // stages under way
+    // this wavefront's loads of the oldest stage under way have landed (NEWER: those of another one may be under way)
+#define PF_LANDED(NEWER)                                       \
+    do {                                                       \
+        if (NEWER)                                             \
+            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");   \
+        else                                                   \
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   \
+        __builtin_amdgcn_s_barrier();                          \
+    } while (0)
+    // (the products of F are not to move in front of what stands before this)
+#define PF_HERE(F)                                                                                                       \
+    do {                                                                                                                 \
+        if constexpr (JT == 2)                                                                                           \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]));                                           \
+        else                                                                                                             \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[JT]), "+v"(F[JT + 1]));             \
+    } while (0)
+    int stage = 0;
+    unsigned sb = lds0;
+    for (int i = 0; i < AHEAD && i < nk; i++) issue(i);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (AHEAD < nk) issue(AHEAD);
+    PF_READ(F0, 0);
+#define PF_SLICES()           \
+    do {                      \
+        PF_READ(F1, 1);       \
+        PF_WAIT(F0, false);   \
+        PF_PRODUCTS(F0);      \
+        PF_READ(F0, 2);       \
+        PF_WAIT(F1, false);   \
+        PF_PRODUCTS(F1);      \
+        PF_READ(F1, 3);       \
+        PF_WAIT(F0, false);   \
+        PF_PRODUCTS(F0);      \
+        PF_WAIT(F1, true);    \
+    } while (0)
+#define PF_NEXT_STAGE()                                        \
+    do {                                                       \
+        stage = stage + 1 == STAGES ? 0 : stage + 1;           \
+        sb = lds0 + (unsigned)(stage * STAGE);                 \
+        PF_READ(F0, 0);                                        \
+        PF_HERE(F1);                                           \
+        PF_PRODUCTS(F1);                                       \
+    } while (0)
+    // (whether a stage is left to load is not asked inside the loops: the last ones have their own)
+    int64_t kt = 1;
+    for (; kt + AHEAD < nk; kt++) {
+        PF_SLICES();
+        PF_LANDED(AHEAD == 2);
+        issue(stage);
+        PF_NEXT_STAGE();
     }
+    for (; kt < nk; kt++) {
+        PF_SLICES();
+        PF_LANDED(false);
+        PF_NEXT_STAGE();
+    }
+    PF_SLICES();
+    PF_PRODUCTS(F1);
+#undef PF_HERE
+#undef PF_LANDED
+#undef PF_NEXT_STAGE
+#undef PF_SLICES
 #undef PF_PRODUCTS
 #undef PF_WAIT
 #undef PF_READ
