@@ -352,7 +352,7 @@ hipError_t k_latent_attend(hipStream_t s, const LatentShape &w, const float *qa,
 template <int PREC>
 __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w, const float *part, const uint16_t *ukv, int ldu,
                                                                   const float *raw, int64_t ldr, void *outa, int64_t lda, int64_t cols,
-                                                                  int n_split, int M, int pos0, const DecodeCtl *ctl) {
+                                                                  int n_split, const DecodeCtl *ctl) {
     extern __shared__ __align__(16) float s_mem[];
     __shared__ float s_f[L_LATENT_SPLITS];
     const int h = blockIdx.x, e0 = blockIdx.y * LV_ROWS, m = blockIdx.z, t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -374,9 +374,13 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
         const int e = e0 + wave * RW + i;
         gate[i] = w.gated && e < w.V ? raw[(int64_t)m * ldr + w.off_g() + (int64_t)h * w.V + e] : 0.0f;
     }
-    // the runs that have keys (latent_attend_kernel): at 70 positions three of 128; asking for all their sums took 7 us of HBM
-    const int n_cols = M * w.H, c0 = (m * w.H + h) & ~15, n_keys = (ctl ? ctl->pos : pos0) + min(c0 + 15, n_cols - 1) / w.H + 1;
-    const int run = ((n_keys + n_split - 1) / n_split + 31) / 32 * 32, used = min(n_split, (n_keys + run - 1) / run);
+    // the runs that have keys (latent_attend_kernel) in a decode step: at 70 positions three of 128; asking for all their sums took
+    // 7 us of HBM.  (A prompt's tokens have few runs each, and so many workgroups that the divisions show: 81 us against 75.)
+    int used = n_split;
+    if (ctl) {
+        const int n_keys = ctl->pos + 1, run = ((n_keys + n_split - 1) / n_split + 31) / 32 * 32;
+        used = min(n_split, (n_keys + run - 1) / run);
+    }
     const int cq = t % nq, cg = t / nq;
     float4 v[LV_U];
     auto fetch = [&](int i0) {
@@ -466,15 +470,15 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
         for (int64_t i = (int64_t)w.H * w.V + t; i < cols; i += LV_THREADS) l_store_act<PREC>(outa, m * lda + i, 0.0f);
 }
 hipError_t k_latent_value(hipStream_t s, const LatentShape &w, const float *part, const uint16_t *ukv, int ldu, const float *raw,
-                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec, int pos0, const DecodeCtl *ctl) {
-    if (M < 1 || w.C > L_LATENT_MAX_RANK || ldu % 64 != 0 || ldu < w.C || cols > lda || cols < (int64_t)w.H * w.V) return hipErrorInvalidValue;
+                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec, const DecodeCtl *ctl) {
+    if (M < 1 || (ctl && M != 1) || w.C > L_LATENT_MAX_RANK || ldu % 64 != 0 || ldu < w.C || cols > lda || cols < (int64_t)w.H * w.V) return hipErrorInvalidValue;
     const int ns = latent_splits((int64_t)M * w.H), nq = w.Cp() / 4, ng = LV_THREADS / nq;
     const size_t lds = ((size_t)ldu + (size_t)ng * w.Cp()) * sizeof(float);
     const dim3 grid((unsigned)w.H, (unsigned)((w.V + LV_ROWS - 1) / LV_ROWS), (unsigned)M);
     if (prec)
-        hipLaunchKernelGGL((latent_value_kernel<1>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, M, pos0, ctl);
+        hipLaunchKernelGGL((latent_value_kernel<1>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, ctl);
     else
-        hipLaunchKernelGGL((latent_value_kernel<0>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, M, pos0, ctl);
+        hipLaunchKernelGGL((latent_value_kernel<0>), grid, dim3(LV_THREADS), lds, s, w, part, ukv, ldu, raw, ldr, outa, lda, cols, ns, ctl);
     return hipGetLastError();
 }
 

@@ -770,7 +770,7 @@ static hipError_t step_latent(l2h_model *m, const LayerDev &L, const LayerRun &r
     CK(k_latent_query(s, w, L.freq, l->lq, L.ukv.w, L.ukv.ld, l->qa, 1, 0, m->ctl, l->in, L.kvnorm, run.kc));
     CK(k_latent_attend(s, w, l->qa, run.kc, l->part, 1, 0, m->ctl));
     const int64_t cols = L.joined ? L.o_cols : w.H * w.V;
-    return k_latent_value(s, w, l->part, L.ukv.w, L.ukv.ld, l->in, 0, 1, l->mix, cols, cols, 1, 0, m->ctl);
+    return k_latent_value(s, w, l->part, L.ukv.w, L.ukv.ld, l->in, 0, 1, l->mix, cols, cols, 1, m->ctl);
 }
 
 hipError_t layered_enqueue_token(l2h_model *m) {
@@ -1155,7 +1155,7 @@ static hipError_t prompt_latent(l2h_model *m, LayerDev &L, const LayerRun &run, 
             void *out = (char *)l->ao + (int64_t)m0 * lda * l->asize();
             CK(k_latent_query(s, w, L.freq, l->qkv + m0 * ldq, L.ukv.w, L.ukv.ld, l->lat_qa, n, pos0 + m0, nullptr, nullptr, nullptr, nullptr));
             CK(k_latent_attend(s, w, l->lat_qa, run.kc, l->lat_part, n, pos0 + m0, nullptr));
-            CK(k_latent_value(s, w, l->lat_part, L.ukv.w, L.ukv.ld, l->raw + m0 * ldr, ldr, n, out, lda, L.o_cols, prec, pos0 + m0, nullptr));
+            CK(k_latent_value(s, w, l->lat_part, L.ukv.w, L.ukv.ld, l->raw + m0 * ldr, ldr, n, out, lda, L.o_cols, prec, nullptr));
         }
         return hipSuccess;
     }

@@ -242,7 +242,7 @@ hipError_t k_latent_attend(hipStream_t s, const LatentShape &w, const float *qa,
                            const DecodeCtl *ctl);
 // joins them, applies v_up and the gates raw[m][ldr]: outa[m][h V + e], columns H V .. cols - 1 zeroed
 hipError_t k_latent_value(hipStream_t s, const LatentShape &w, const float *part, const uint16_t *ukv, int ldu, const float *raw,
-                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec, int pos0, const DecodeCtl *ctl);
+                          int64_t ldr, int M, void *outa, int64_t lda, int64_t cols, int prec, const DecodeCtl *ctl);
 // for the matrix-core attention: rotated queries as bf16 [M][H hs], cached latents n rows from pos0 as activations [n][lda]
 hipError_t k_latent_heads(hipStream_t s, const LatentShape &w, const float *freq, const float *q, uint16_t *qb, int hs, int M, int pos0);
 hipError_t k_latent_rows(hipStream_t s, const LatentShape &w, const float *cache, int pos0, int n, uint16_t *outa, int64_t lda);
