@@ -109,6 +109,8 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // the same for few rows or positions (k_few.hip; k_gemm chooses); cols: columns the epilogue covers
 #define L_FEW_M 128      // up to so many positions
 #define L_FEW_EACH 48    // ... of an expert
+#define L_FEW_EACH_F32 224  // in fp32 (prompts of 200, 509, 800 positions, 16 experts of 512 x 1024, 4 each: 563, 679, 908 us in blocks of
+                            // 128, 461, 616, 867 like this; 1500, 375 an expert: 1395, 1425)
 #define L_FEW_TILES 256  // or fewer 64 x 64 tiles of results than this: 509 positions x 1024 rows, 1024 inputs, fp32: 15 us against 26;
                          // at 424 tiles (3400 rows) the two take the same
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
