@@ -241,9 +241,13 @@ hipError_t k_window_prepare(hipStream_t s, const WindowShape &w, const float *fr
 }
 
 // fp32 attention: workgroup = one head x WR_Q queries, keys in tiles of WR_K; a wavefront owns WR_Q / 4 queries, its lanes
-// the keys of a tile, then the value columns
+// the keys of a tile, then the value columns.  A CU gets about one workgroup of it, so latency bounds it: the key elements are
+// requested WR_U words at a time and the values of a tile before its scores, which are formed without a barrier (8 heads of 128,
+// 509 queries, all before them in the window: 181 us with one load after the other, 97 us like this)
 #define WR_Q 16
 #define WR_K 64
+#define WR_U 8
+typedef float wr_f32x4 __attribute__((ext_vector_type(4)));
 template <int PREC>
 __global__ __launch_bounds__(256) void window_rows_kernel(WindowShape w, const float *qf, const float *raw, int64_t ldr, const float *kc,
                                                           const float *vc, int M, int pos0, void *outa, int64_t lda) {
@@ -258,6 +262,7 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowShape w, const f
         const int q = i / Dp, e = i - q * Dp;
         s_q[i] = (q0 + q < M && e < D) ? qf[((int64_t)(q0 + q) * w.H + h) * D + e] : 0.0f;
     }
+    __syncthreads();
     float mrun[QW], lrun[QW], acc[QW][4];  // V <= 256: four columns per lane
 #pragma unroll
     for (int a = 0; a < QW; a++) {
@@ -269,24 +274,44 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowShape w, const f
     const int last = pos0 + min(q0 + WR_Q, M) - 1, first = max(0, pos0 + q0 - w.window + 1);
     for (int k0 = first; k0 <= last; k0 += WR_K) {
         const int n = min(WR_K, last + 1 - k0);
-        __syncthreads();
-        for (int i = t; i < n * V; i += 256) s_v[i] = vc[((int64_t)g * w.seq_len + k0) * V + i];
-        __syncthreads();
+        const float *vsrc = vc + ((int64_t)g * w.seq_len + k0) * V;
+        const int nq = V % 4 == 0 ? n * V / 4 : 0;  // (a row of values then begins on 16 bytes)
+        wr_f32x4 vq[WR_U];
+        if (nq) {
+#pragma unroll
+            for (int u = 0; u < WR_U; u++) vq[u] = *(const wr_f32x4 *)(vsrc + 4 * min(t + 256 * u, nq - 1));
+        }
         float sc[QW];
 #pragma unroll
         for (int a = 0; a < QW; a++) sc[a] = 0.0f;
-        if (lane < n)
-            for (int i = 0; i < D4; i++) {
-                const float4 kv = *(const float4 *)(kc + (krow + (int64_t)i * w.seq_len + k0 + lane) * 4);
+        const float *kp = kc + (krow + k0 + min(lane, n - 1)) * 4;
+        for (int i0 = 0; i0 < D4; i0 += WR_U) {
+            float4 kv[WR_U];
 #pragma unroll
-                for (int a = 0; a < QW; a++) {
-                    const float4 qv = *(const float4 *)(s_q + (wave * QW + a) * Dp + 4 * i);
-                    sc[a] = fmaf(qv.x, kv.x, sc[a]);
-                    sc[a] = fmaf(qv.y, kv.y, sc[a]);
-                    sc[a] = fmaf(qv.z, kv.z, sc[a]);
-                    sc[a] = fmaf(qv.w, kv.w, sc[a]);
+            for (int u = 0; u < WR_U; u++) kv[u] = *(const float4 *)(kp + (int64_t)min(i0 + u, D4 - 1) * w.seq_len * 4);
+#pragma unroll
+            for (int u = 0; u < WR_U; u++)
+                if (i0 + u < D4) {
+#pragma unroll
+                    for (int a = 0; a < QW; a++) {
+                        const float4 qv = *(const float4 *)(s_q + (wave * QW + a) * Dp + 4 * (i0 + u));
+                        sc[a] = fmaf(qv.x, kv[u].x, sc[a]);
+                        sc[a] = fmaf(qv.y, kv[u].y, sc[a]);
+                        sc[a] = fmaf(qv.z, kv[u].z, sc[a]);
+                        sc[a] = fmaf(qv.w, kv[u].w, sc[a]);
+                    }
                 }
-            }
+        }
+        if (k0 != first) __syncthreads();  // (everyone is through with the values of the tile before)
+        if (nq) {
+#pragma unroll
+            for (int u = 0; u < WR_U; u++)
+                if (t + 256 * u < nq) *(wr_f32x4 *)(s_v + 4 * (t + 256 * u)) = vq[u];
+            for (int i = t + 256 * WR_U; i < nq; i += 256) *(float4 *)(s_v + 4 * i) = *(const float4 *)(vsrc + 4 * i);
+        } else {
+            for (int i = t; i < n * V; i += 256) s_v[i] = vsrc[i];
+        }
+        __syncthreads();
 #pragma unroll
         for (int a = 0; a < QW; a++) {
             const int qp = pos0 + q0 + wave * QW + a, key = k0 + lane;
@@ -302,16 +327,24 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowShape w, const f
             for (int b = 0; b < 4; b++) acc[a][b] *= alpha;
         }
         __builtin_amdgcn_wave_barrier();
-        for (int i = 0; i < n; i++)
+        for (int i = 0; i < n; i += 4) {  // (a key that is not there has p = 0; its values are those of the last one)
+            const float *v0 = s_v + i * V, *v1 = s_v + min(i + 1, n - 1) * V, *v2 = s_v + min(i + 2, n - 1) * V, *v3 = s_v + min(i + 3, n - 1) * V;
 #pragma unroll
             for (int b = 0; b < 4; b++) {
                 const int c = lane + 64 * b;
                 if (c < V) {
-                    const float v = s_v[i * V + c];
+                    const float x0 = v0[c], x1 = v1[c], x2 = v2[c], x3 = v3[c];
 #pragma unroll
-                    for (int a = 0; a < QW; a++) acc[a][b] = fmaf(s_p[(wave * QW + a) * WR_K + i], v, acc[a][b]);
+                    for (int a = 0; a < QW; a++) {
+                        const float4 p = *(const float4 *)(s_p + (wave * QW + a) * WR_K + i);
+                        acc[a][b] = fmaf(p.x, x0, acc[a][b]);
+                        acc[a][b] = fmaf(p.y, x1, acc[a][b]);
+                        acc[a][b] = fmaf(p.z, x2, acc[a][b]);
+                        acc[a][b] = fmaf(p.w, x3, acc[a][b]);
+                    }
                 }
             }
+        }
     }
 #pragma unroll
     for (int a = 0; a < QW; a++) {
