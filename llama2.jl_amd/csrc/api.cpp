@@ -1330,8 +1330,12 @@ static hipError_t prefill_chunk(l2h_model *m, int M, int pos0) {
                          nullptr, 0));
         CK(k_pf_rmsnorm(s, m->pf_x, m->L(l, L2H_RMS_FFN).f32, m->pf_xn, M, dim));
         const DevTensor w13[2] = {m->L(l, L2H_W1), m->L(l, L2H_W3)};
-        CK(k_pf_gemm(s, w13, 2, 1, wb ? wb + m->pf_off_w13 : nullptr, 2 * (int64_t)c.hidden_dim, m->pf_xn, M, dim,
-                     PF_SWIGLU, nullptr, 0, 0, m->pf_hb, c.hidden_dim));
+        const int64_t n13 = 2 * (int64_t)c.hidden_dim;
+        if (lib && k_pf_few_pays(n13, M))
+            CK(k_pf_few(s, wb + m->pf_off_w13, n13, m->pf_xn, M, dim, m->pf_hb, c.hidden_dim));
+        else
+            CK(k_pf_gemm(s, w13, 2, 1, wb ? wb + m->pf_off_w13 : nullptr, n13, m->pf_xn, M, dim, PF_SWIGLU, nullptr, 0, 0,
+                         m->pf_hb, c.hidden_dim));
         const DevTensor w2 = m->L(l, L2H_W2);
         if (lib)
             CK(pf_lt_gemm(m->pf_lt, s, wb + m->pf_off_w2, m->pf_hb, m->pf_x, M, dim, c.hidden_dim, dim, true, &m->pf_lt_err));

@@ -135,6 +135,33 @@ def test_prefill_weight_copy_changes_nothing(pkg, case):
     assert not dev.prefill_library and nxt == got[0][1] and np.array_equal(logits, got[0][0])
 
 
+@pytest.mark.parametrize("dim,hidden,lengths", [
+    (64, 192, (1, 16, 17, 33, 95)),     # one step of inputs for eight wavefronts, 32 x 32 results a workgroup
+    (576, 320, (2, 31, 32, 64, 129)),   # nine steps
+    (64, 4160, (16, 17, 63, 64, 65)),   # 130 tiles of 64 x 64 results, part of the last group of 256 rows; from 65 on 260, in whole groups
+    (1088, 8192, (1, 33, 64)),          # one tile of 64 x 64 a CU
+], ids=["one_step", "nine_steps", "part_group", "tile_a_cu"])
+def test_short_prompts(pkg, dim, hidden, lengths):
+    """The w1/w3 product of short prompts beside the library's plain products sums its inputs in eight parts; with the library
+    off every product sums them in one.  Tolerances: as in test_prefill_weight_copy_changes_nothing, for the same reason."""
+    from llama2_jl_amd import synth
+    lm = _model(pkg, "PLAN_F32", dim=dim, hidden_dim=hidden, n_layers=2, n_heads=dim // 32, n_kv_heads=dim // 32, vocab_size=256,
+                seq_len=160, rope_freq_base=10000.0, rope_is_neox=False)
+    dev = lm.device()
+    for n in lengths:
+        prompt = synth.seeded_prompt(n, n, 256)
+        got = []
+        for library in (True, False):
+            dev.set_prefill_library(library)
+            dev.reset()
+            logits, _ = dev.prefill(prompt, 0)
+            assert dev.prefill_library == library
+            got.append((logits.copy(), *[a.copy() for a in dev.kv_read(1, 0, n)]))
+        e, ekv = _rel(got[0][0], got[1][0]), max(_rel(got[0][1], got[1][1]), _rel(got[0][2], got[1][2]))
+        print("\n%d x %d, %d positions: logits rel diff %.3g, K/V %.3g" % (hidden, dim, n, e, ekv), flush=True)
+        assert e <= 1.5e-2 and ekv <= 1e-2
+
+
 def test_prefill_without_the_gemm_library(pkg, monkeypatch):
     """Where hipBLASLt cannot be opened (here: L2H_HIPBLASLT names a file that does not exist) the prompt pass runs this
     library's product kernels and says so; same results, bit for bit, as with the library switched off by the caller."""
