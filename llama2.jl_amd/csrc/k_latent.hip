@@ -167,10 +167,18 @@ hipError_t k_latent_query(hipStream_t s, const LatentShape &w, const float *freq
     return hipGetLastError();
 }
 
+// keys of a run: 32 at least; in a decode step 16 while that makes no more than 64 runs (a step on 16 heads, this kernel and the
+// joining one: 57 keys 15.7 us with 32 and 14.1 with 16; 1000 keys 16.9 and 15.3; 2000 keys, 125 runs of 16: 17.7 and 18.2)
+__device__ __forceinline__ int latent_run(int n_keys, int n_split, bool step) {
+    const int least = step && n_keys <= 16 * 64 ? 16 : 32;
+    return ((n_keys + n_split - 1) / n_split + least - 1) / least * least;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
-// Scores and value sums on the cached rows: workgroup (run of keys, 16 columns), a column being a (token, head).  Keys go 32 at
-// a time.  The scores' contraction (the row's elements, 16 at a time) is shared out among the eight wavefronts and their parts
-// are added in LDS; every wavefront then has the 32 x 16 scores in registers, in the layout that is the second product's
+// Scores and value sums on the cached rows: workgroup (run of keys, 16 columns), a column being a (token, head).  Keys go 16 KH
+// at a time: 32 in a prompt, 16 in a decode step, where a few CUs pull all of the rows and a run's latency is the launch's (57 keys,
+// 16 heads of rank 512: three runs of 32 keys 10.0 us, four of 16 7.5).  The scores' contraction (the row's elements, 16 at a time) is shared out among the eight wavefronts and their parts
+// are added in LDS; every wavefront then has the 16 KH x 16 scores in registers, in the layout that is the second product's
 // operand when its contraction takes key 4 (lane / 16) + r in step r, and sums its own 64-element blocks of the latent:
 // wavefront v the blocks v, v + 8, ...
 //   v_mfma_f32_16x16x4_f32: operands hold (row or column lane % 16, k = lane / 16), the result (row 4 (lane / 16) + r, column
@@ -178,11 +186,12 @@ hipError_t k_latent_query(hipStream_t s, const LatentShape &w, const float *freq
 // ---------------------------------------------------------------------------------------------------------------
 #define LA_WAVES 8
 #define LA_J 5  // 16-element steps of the scores' contraction a wavefront fetches together: rows of up to 640 elements
-template <int NB>
+template <int NB, int KH>
 __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShape w, const float *qa, const float *cache, float *part, int n_cols,
                                                             int pos0, const DecodeCtl *ctl, int n_split) {
+    constexpr int KEYS = 16 * KH;
     extern __shared__ __align__(16) float s_q[];  // [16][ld + 4]
-    __shared__ float s_sc[2][LA_WAVES][8][64];
+    __shared__ float s_sc[2][LA_WAVES][4 * KH][64];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, col = lane & 15;
     const int ld = w.ld(), Cp = w.Cp(), qs = ld + 4, st = Cp + 4;
     const int c0 = 16 * blockIdx.y;
@@ -195,9 +204,9 @@ __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShap
     for (int u = 0; u < LA_J; u++) qr[u] = *(const float4 *)(qsrc + min(qe + QE * u, ld - 4));
     const int first = ctl ? ctl->pos : pos0;
     const int n_keys = first + min(c0 + 15, n_cols - 1) / w.H + 1;
-    const int run = ((n_keys + n_split - 1) / n_split + 31) / 32 * 32, k0 = run * (int)blockIdx.x, k1 = min(k0 + run, n_keys);
+    const int run = latent_run(n_keys, n_split, ctl), k0 = run * (int)blockIdx.x, k1 = min(k0 + run, n_keys);
     if (k0 >= k1) {
-        if (t < 16 && c0 + t < n_cols) {
+        if (!ctl && t < 16 && c0 + t < n_cols) {  // (a decode step reads no run without keys)
             float *p = part + ((int64_t)(c0 + t) * n_split + blockIdx.x) * st;
             p[0] = -INFINITY;
             p[1] = 0.0f;
@@ -206,20 +215,19 @@ __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShap
     }
     // the latents of the second product: keys kb + 4 g + r and 16 further, elements 64 (wave + 8 b) + 4 col ..; of the first:
     // keys kb + col and 16 further, elements 16 j + 4 g .., j = wave, wave + 8, ...
-    float4 ka[LA_J], kc[LA_J], va[NB][8];
+    float4 ka[KH][LA_J], va[NB][4 * KH];
     auto key = [&](int k) { return cache + (int64_t)min(k, k1 - 1) * ld; };
     auto fetch_k = [&](int kb) {
-        const float *a = key(kb + col) + 4 * g, *c = key(kb + 16 + col) + 4 * g;
 #pragma unroll
-        for (int u = 0; u < LA_J; u++) {
-            const int at = min(16 * (wave + LA_WAVES * u), ld - 16);  // (a step past the row is not used)
-            ka[u] = *(const float4 *)(a + at);
-            kc[u] = *(const float4 *)(c + at);
+        for (int i = 0; i < KH; i++) {
+            const float *a = key(kb + 16 * i + col) + 4 * g;
+#pragma unroll
+            for (int u = 0; u < LA_J; u++) ka[i][u] = *(const float4 *)(a + min(16 * (wave + LA_WAVES * u), ld - 16));  // (a step past the row is not used)
         }
     };
     auto fetch_v = [&](int kb) {
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
+        for (int r = 0; r < 4 * KH; r++) {
             const float *row = key(kb + 16 * (r >> 2) + 4 * g + (r & 3));
 #pragma unroll
             for (int b = 0; b < NB; b++) {
@@ -242,35 +250,42 @@ __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShap
         for (int i = 0; i < 4; i++) o[b][i] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
     float mrun = -INFINITY, lrun = 0.0f;
     int stage = 0;
-    for (int kb = k0; kb < k1; kb += 32, stage ^= 1) {
-        lat_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+    for (int kb = k0; kb < k1; kb += KEYS, stage ^= 1) {
+        lat_f32x4 sc[KH];
+#pragma unroll
+        for (int i = 0; i < KH; i++) sc[i] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
         const float *qp = s_q + col * qs + 4 * g;
-        auto score = [&](float4 x, float4 y, int j) {
+        auto score = [&](const float4 (&x)[KH], int j) {
             const float4 q = *(const float4 *)(qp + 16 * j);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, q.x, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(y.x, q.x, s1, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, q.y, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(y.y, q.y, s1, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, q.z, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(y.z, q.z, s1, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, q.w, s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(y.w, q.w, s1, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < KH; i++) sc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i].x, q.x, sc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < KH; i++) sc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i].y, q.y, sc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < KH; i++) sc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i].z, q.z, sc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < KH; i++) sc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i].w, q.w, sc[i], 0, 0, 0);
         };
 #pragma unroll
-        for (int u = 0; u < LA_J; u++)
-            if (16 * (wave + LA_WAVES * u) < ld) score(ka[u], kc[u], wave + LA_WAVES * u);
-        for (int j = wave + LA_WAVES * LA_J; 16 * j < ld; j += LA_WAVES)
-            score(*(const float4 *)(key(kb + col) + 4 * g + 16 * j), *(const float4 *)(key(kb + 16 + col) + 4 * g + 16 * j), j);
-        if (kb + 32 < k1) fetch_k(kb + 32);
+        for (int u = 0; u < LA_J; u++) {
+            float4 x[KH];
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            s_sc[stage][wave][r][lane] = s0[r];
-            s_sc[stage][wave][4 + r][lane] = s1[r];
+            for (int i = 0; i < KH; i++) x[i] = ka[i][u];
+            if (16 * (wave + LA_WAVES * u) < ld) score(x, wave + LA_WAVES * u);
         }
-        __syncthreads();  // (the other stage is written again only behind the next one)
-        float p[8], mx = -INFINITY;
+        for (int j = wave + LA_WAVES * LA_J; 16 * j < ld; j += LA_WAVES) {
+            float4 x[KH];
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
+            for (int i = 0; i < KH; i++) x[i] = *(const float4 *)(key(kb + 16 * i + col) + 4 * g + 16 * j);
+            score(x, j);
+        }
+        if (kb + KEYS < k1) fetch_k(kb + KEYS);
+#pragma unroll
+        for (int r = 0; r < 4 * KH; r++) s_sc[stage][wave][r][lane] = sc[r >> 2][r & 3];
+        __syncthreads();  // (the other stage is written again only behind the next one)
+        float p[4 * KH], mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4 * KH; r++) {
             float v = 0.0f;
 #pragma unroll
             for (int i = 0; i < LA_WAVES; i++) v += s_sc[stage][i][r][lane];
@@ -282,7 +297,7 @@ __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShap
         const float mnew = fmaxf(mrun, mx), alpha = mnew == -INFINITY ? 1.0f : expf(mrun - mnew);
         float sum = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
+        for (int r = 0; r < 4 * KH; r++) {
             p[r] = p[r] == -INFINITY ? 0.0f : expf(p[r] - mnew);
             sum += p[r];
         }
@@ -295,14 +310,14 @@ __global__ __launch_bounds__(64 * LA_WAVES) void latent_attend_kernel(LatentShap
 #pragma unroll
             for (int i = 0; i < 4; i++) o[b][i] *= alpha;
 #pragma unroll
-            for (int r = 0; r < 8; r++) {
+            for (int r = 0; r < 4 * KH; r++) {
                 o[b][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[b][r].x, p[r], o[b][0], 0, 0, 0);
                 o[b][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[b][r].y, p[r], o[b][1], 0, 0, 0);
                 o[b][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[b][r].z, p[r], o[b][2], 0, 0, 0);
                 o[b][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[b][r].w, p[r], o[b][3], 0, 0, 0);
             }
         }
-        if (kb + 32 < k1) fetch_v(kb + 32);
+        if (kb + KEYS < k1) fetch_v(kb + KEYS);
     }
     if (mine >= n_cols) return;
     float *dst = part + ((int64_t)mine * n_split + blockIdx.x) * st;
@@ -326,19 +341,23 @@ hipError_t k_latent_attend(hipStream_t s, const LatentShape &w, const float *qa,
     if (lds > 100 * 1024) return hipErrorInvalidValue;
     const int nb = ((w.Cp() + 63) / 64 + LA_WAVES - 1) / LA_WAVES;  // at most 2
     const dim3 grid((unsigned)ns, (unsigned)((cols + 15) / 16));
-#define GO(N)                                                                                                                          \
-    do {                                                                                                                               \
-        if (lds > 32 * 1024) {                                                                                                         \
-            const hipError_t e = hipFuncSetAttribute((const void *)latent_attend_kernel<N>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                                     100 * 1024);                                                                      \
-            if (e != hipSuccess) return e;                                                                                             \
-        }                                                                                                                              \
-        hipLaunchKernelGGL((latent_attend_kernel<N>), grid, dim3(64 * LA_WAVES), lds, s, w, qa, cache, part, cols, pos0, ctl, ns);               \
+#define GO(N, K)                                                                                                                          \
+    do {                                                                                                                                  \
+        if (lds > 32 * 1024) {                                                                                                            \
+            const hipError_t e = hipFuncSetAttribute((const void *)latent_attend_kernel<N, K>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                                     100 * 1024);                                                                         \
+            if (e != hipSuccess) return e;                                                                                                \
+        }                                                                                                                                 \
+        hipLaunchKernelGGL((latent_attend_kernel<N, K>), grid, dim3(64 * LA_WAVES), lds, s, w, qa, cache, part, cols, pos0, ctl, ns);      \
     } while (0)
-    if (nb == 1)
-        GO(1);
+    if (ctl && nb == 1)
+        GO(1, 1);
+    else if (ctl)
+        GO(2, 1);
+    else if (nb == 1)
+        GO(1, 2);
     else
-        GO(2);
+        GO(2, 2);
 #undef GO
     return hipGetLastError();
 }
@@ -378,7 +397,7 @@ __global__ __launch_bounds__(LV_THREADS) void latent_value_kernel(LatentShape w,
     // 7 us of HBM.  (A prompt's tokens have few runs each, and so many workgroups that the divisions show: 81 us against 75.)
     int used = n_split;
     if (ctl) {
-        const int n_keys = ctl->pos + 1, run = ((n_keys + n_split - 1) / n_split + 31) / 32 * 32;
+        const int n_keys = ctl->pos + 1, run = latent_run(n_keys, n_split, true);
         used = min(n_split, (n_keys + run - 1) / run);
     }
     const int cq = t % nq, cg = t / nq;

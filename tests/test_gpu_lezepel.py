@@ -206,6 +206,20 @@ def test_prompt_longer_than_one_chunk(pkg, precision):
     dev.close()
 
 
+@pytest.mark.parametrize("heads,rank", [(2, 20), (17, 600)])
+def test_decoding_where_the_runs_of_keys_grow(pkg, heads, rank):
+    """A decode step's runs of keys are of 16 up to 1024 keys and of 32 beyond; up to 32 keys there are one or two of them."""
+    c = zc.config([zc.layer(heads=heads, dim=12, rot_dim=4, vdim=16, kv_rank=rank, q_rank=24)], width=32, vocab=50)
+    t = ref.random_tensors(c, 9)
+    tok = lc.tokens(1030, 50, 3)
+    want = ref.Sequence(c, t).run(tok)
+    dev = zc.language_model(pkg, c, t, seq_len=1100).device()
+    assert lc.error(_decode(dev, tok[:35]), want[:35]) <= TOL["float32"]
+    dev.prefill_logits(tok[35:1018], [], 35)
+    assert lc.error(_decode(dev, tok[1018:], 1018), want[1018:]) <= TOL["float32"]
+    dev.close()
+
+
 def test_greedy_generation(pkg):
     c, t = zc.CASES["mixed"], zc.tensors("mixed")
     prompt = lc.tokens(11, c["vocab"], 8)
