@@ -14,7 +14,6 @@ typedef __bf16 few_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float few_f32x4 __attribute__((ext_vector_type(4)));
 
 #define FEW_WAVES 8
-#define FEW_RED 16384  // floats: 8 wavefronts x 64 positions x 32 rows
 
 // one step's operands of a lane: UK groups of 32 inputs
 template <int PREC, int RN, int JM, int UK>
