@@ -503,7 +503,12 @@ static int put_rows(l2h_model *m, uint16_t *dst, int64_t pitch, const void *host
         HIPCHK(ctx, hipMemcpy(dst, host, (size_t)(ne0 * ne1) * 2, hipMemcpyHostToDevice));
         return L2H_OK;
     }
-    if (!l->stage) HIPCHK(ctx, hipMalloc(&l->stage, (size_t)L_STAGE_BYTES));
+    if (!l->stage && hipMalloc(&l->stage, (size_t)L_STAGE_BYTES) != hipSuccess) {  // (a device that has room for the model only)
+        (void)hipGetLastError();
+        l->stage = nullptr;
+        HIPCHK(ctx, hipMemcpy2D(dst, (size_t)pitch * 2, host, (size_t)ne0 * 2, (size_t)ne0 * 2, (size_t)ne1, hipMemcpyHostToDevice));
+        return L2H_OK;
+    }
     const int64_t most = std::max<int64_t>(1, L_STAGE_BYTES / 2 / ne0);
     for (int64_t r = 0; r < ne1; r += most) {
         const int64_t n = std::min(most, ne1 - r);
@@ -601,6 +606,7 @@ int layered_finalize(l2h_model *m) {
         if ((rc = missing(l->have, r, -1))) return rc;
     if (c.side_dim && (rc = missing(l->have, L2H_SIDE_EMB, -1))) return rc;
     if (c.loop_times && (rc = missing(l->have, L2H_LOOP_STEP, -1))) return rc;
+    free_stage(l);
 #define DA(p, n, z)                       \
     if ((rc = dalloc(m, &(p), (n), (z)))) \
         return rc;
@@ -672,7 +678,6 @@ int layered_finalize(l2h_model *m) {
     DA(m->rope_cs, 2, true);
     DA(m->logits, c.vocab_size, true);
 #undef DA
-    free_stage(l);
     l->pos = 0;
     return L2H_OK;
 }
