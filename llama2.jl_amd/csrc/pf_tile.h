@@ -41,12 +41,12 @@ constexpr int pf_tile_stage(int jt) { return 32768 + 64 * jt * 128; }  // bytes:
 constexpr int pf_tile_stages(int jt) { return jt == 2 ? 3 : 2; }
 constexpr int pf_tile_lds(int jt) { return pf_tile_stages(jt) * pf_tile_stage(jt); }
 
-// wtiles: the row group's tiles, K / 64 of them in a row; act: bf16 rows of K elements; s_all: pf_tile_lds(JT) bytes of LDS.  row(r) is the
+// wtiles: the row group's tiles, K / 64 of them in a row; act: bf16 rows of K elements; s_all: STAGES * pf_tile_stage(JT) bytes of LDS.  row(r) is the
 // activation row of the tile's position r; epi(acc, wn, wm, lane) takes the results: a lane holds position
 // 32 JT wm + 32 j + lane % 32 and, in register r of tile i, weight row 64 wn + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4.
-template <int JT, class Row, class Epi>
+template <int JT, int STAGES = pf_tile_stages(JT), class Row, class Epi>
 __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const uint16_t *act, int64_t K, uint4 *s_all, Row row, Epi epi) {
-    constexpr int STAGE = pf_tile_stage(JT), STAGES = pf_tile_stages(JT);
+    constexpr int STAGE = pf_tile_stage(JT);
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), wn = wave & 3, wm = wave >> 2;
     const int64_t nk = K >> 6;
 
