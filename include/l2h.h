@@ -190,7 +190,9 @@ int l2h_prefill_logits(l2h_model *m, const int32_t *tokens, int n, int pos0, con
 /* The temperature branch of sample() (src/inference.jl:363-367) on the logits the last step left on
  * the device: logits ./= temperature, softmax!, then wsample's walk with the caller's uniform number
  * u in [0, 1) in place of the global RNG: token = first index whose cumulative probability reaches
- * u * sum(p).  probs (vocab floats, may be NULL) receives the probabilities.  temperature > 0. */
+ * u * sum(p).  probs (vocab floats, may be NULL) receives the probabilities.  temperature > 0.  Where the
+ * probabilities are not numbers (a logit that is none, or too large once divided) it fails with L2H_EINVAL and
+ * leaves *token alone. */
 int l2h_sample(l2h_model *m, float temperature, float u, int32_t *token, float *probs);
 /* Copies an activation of the last forward call: which = 0 x, 1 xb, 2 q (rotated), 5 hb,
  * 6 logits (RunState fields, src/inference.jl:72-86; k and v go straight into the cache). */

@@ -1496,10 +1496,13 @@ extern "C" int l2h_sample(l2h_model *m, float temperature, float u, int32_t *tok
         if ((rc = dalloc(m, &m->sample_p, m->c.vocab_size, false))) return rc;
     }
     HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_part, m->sample_out));
-    HIPCHK(ctx, hipMemcpyAsync(token, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
+    int32_t pick = -1;
     if (probs)
         HIPCHK(ctx, hipMemcpyAsync(probs, m->sample_p, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(&pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    if (pick < 0) return set_err(ctx, L2H_EINVAL, "nothing to draw from: the logits divided by %g are not all finite", (double)temperature);
+    *token = pick;
     return L2H_OK;
 }
 

@@ -469,7 +469,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(int n, int 
     if (t < parts && ((cum[t] < target && (target <= cum[t + 1] || t == parts - 1)) || (t == 0 && target <= 0.0)))
         atomicMin(&s_at, t);  // (rounding may leave a running sum a last bit below the one before it)
     __syncthreads();
-    if (s_at == 0x7FFFFFFF) return;  // (not a number among the logits)
+    if (s_at == 0x7FFFFFFF) {  // (the probabilities are not numbers: one of the logits was none, or was not finite once divided)
+        if (t == 0) *out = -1;
+        return;
+    }
     const SampleRun r = sample_run(n, per, s_at);
     const double before = cum[s_at];
     const int each = (per + SAMPLE_THREADS - 1) / SAMPLE_THREADS, lo = min(r.hi, r.lo + t * each), hi = min(r.hi, lo + each);

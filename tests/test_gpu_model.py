@@ -512,6 +512,21 @@ def test_sampling_over_any_number_of_logits(pkg, vocab):
     dev.close()
 
 
+@pytest.mark.parametrize("vocab", [5, 2500])
+def test_a_draw_from_what_is_not_a_number_is_an_error(pkg, vocab):
+    """A temperature at which the division overflows leaves no probabilities: an error, not the token of the draw before."""
+    plan, kw = CASES["f32"]
+    dev = _model(pkg, plan, **dict(kw, vocab_size=vocab, n_layers=1)).device()
+    dev.forward(2, 0)
+    first = dev.sample_token(0.9, 0.7)
+    with pytest.raises(pkg.L2HError, match="finite"):
+        dev.sample_token(1e-44, 0.7)
+    with pytest.raises(pkg.L2HError, match="finite"):
+        dev.sample_token(1e-44, 0.0, want_probs=True)
+    assert dev.sample_token(0.9, 0.7) == first
+    dev.close()
+
+
 # Prompt pass (bf16 products of float activations) against sequential decode (q8_K activations, integer products) at
 # full depth: two roundings of the same sums whose difference grows with the layers (0.02-0.05 of the largest value
 # after 2 layers, about 0.2 after 32: observed 0.195 / 0.184 / 0.149 for logits / K / V, root mean square 0.19 / 0.17 /
