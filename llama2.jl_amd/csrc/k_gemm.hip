@@ -164,9 +164,7 @@ static hipError_t gemm_launch(hipStream_t s, const GemmArgs &a) {
     // columns the epilogue covers: an activation-typed result is zeroed up to its row stride
     const bool acts = EPI == GE_ACT || EPI == GE_UP || EPI == GE_EMBED;
     const int64_t cols = EPI == GE_GLU ? 2 * a.acols : acts ? a.acols : a.n_rows;
-    // k_few.hip for few positions, in all or an expert's, and where 64 x 64 tiles would give fewer than one workgroup per CU
-    if (a.tiles ? a.rows_each <= (PREC ? L_FEW_EACH_F32 : L_FEW_EACH) : a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) < L_FEW_TILES)
-        return k_few(s, a, PREC, EPI, cols);
+    if (k_few_pays(a, PREC, cols)) return k_few(s, a, PREC, EPI, cols);
     if (a.tiles) {
         if (EPI != GE_STORE && EPI != GE_UP && EPI != GE_GLU) return hipErrorInvalidValue;
         constexpr int E = EPI == GE_UP || EPI == GE_GLU ? EPI : GE_STORE;

@@ -106,13 +106,31 @@ struct GemmArgs {
 #define L_GEMM_TILE 128   // rows of a block for k_gemm ...
 #define L_IMAGE_TILE 256  // ... and for k_tiles
 hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
-// the same for few rows or positions (k_few.hip; k_gemm chooses); cols: columns the epilogue covers
-#define L_FEW_M 128      // up to so many positions
-#define L_FEW_EACH 48    // ... of an expert
-#define L_FEW_EACH_F32 224  // in fp32 (prompts of 200, 509, 800 positions, 16 experts of 512 x 1024, 4 each: 563, 679, 908 us in blocks of
-                            // 128, 461, 616, 867 like this; 1500, 375 an expert: 1395, 1425)
-#define L_FEW_TILES 256  // or fewer 64 x 64 tiles of results than this: 509 positions x 1024 rows, 1024 inputs, fp32: 15 us against 26;
-                         // at 424 tiles (3400 rows) the two take the same
+// The same for few rows or positions (k_few.hip), which k_gemm hands on to where that is the faster way; cols: columns the epilogue
+// covers.  Gains: the time of k_gemm's own tiles over that of k_few, distinct matrices one after the other.
+//
+// Grouped: up to 48 positions a matrix.  Gains at 12, 32, 48 and 56, 8 to 96 matrices of 512 to 4096 inputs: 2.7 to 12, 1.5 to 9, 1.0 to 8
+// and 0.8 to 5 in fp32; in bf16 2.4 to 8, 1.7 to 8, 1.2 to 7 and 1.0 to 5.  Beyond, in fp32 (bf16 products have images there), while blocks
+// of 128 x 128 would be few for the CUs: up to 224 positions a matrix and, in all, (positions) x (blocks of 128 columns) up to 28 672.
+// Sixty products of 8 to 32 matrices with 256 to 4096 rows, 56 to 240 positions each: 1.2 to 5 at up to half of that, 0.8 to 1.3 there, 0.6 to
+// 0.9 at twice as much (16 matrices of 4096 x 2048, 192 positions each: 0.59).  Within it the blocks are the faster way only near
+// 104 to 136 positions, which just fill one (0.8 to 1.6).
+//
+// Plain: up to 128 positions in bf16 (1.5 to 13, 256 to 32 000 rows), 32 in fp32 (1.0 to 10).  Otherwise where tiles of 64 x 64 are few:
+// at most 256 in bf16 (8192 rows, 128 positions: 1.6 to 2.0), 384 in fp32 (8192 rows, 128 positions, 256 tiles: 1.06 to 1.22; 160 positions,
+// 384 tiles: 1.15 to 1.3; 448 and 500 tiles: 0.92 to 0.99).
+#define L_FEW_M 128
+#define L_FEW_M_F32 32
+#define L_FEW_EACH 48
+#define L_FEW_EACH_F32 224
+#define L_FEW_BLOCKS_F32 28672
+#define L_FEW_TILES 256
+#define L_FEW_TILES_F32 384
+inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
+    if (a.tiles)
+        return a.rows_each <= L_FEW_EACH || (prec && a.rows_each <= L_FEW_EACH_F32 && a.M * ((cols + 127) / 128) <= L_FEW_BLOCKS_F32);
+    return a.M <= (prec ? L_FEW_M_F32 : L_FEW_M) || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (prec ? L_FEW_TILES_F32 : L_FEW_TILES);
+}
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations

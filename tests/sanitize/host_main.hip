@@ -5,6 +5,7 @@
 // (hipcc with the sanitizers on the host side only).
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
+#include "../../llama2.jl_amd/csrc/layered.h"
 
 #include <stdio.h>
 
@@ -124,7 +125,28 @@ static void check_shape(int dim, int hidden, int n_layers, int n_heads, int n_kv
     }
 }
 
+// which kernel takes a product of a layered model: `each` positions for each of `experts` matrices (0: one matrix, `each` positions)
+static bool few(int prec, int experts, int64_t cols, int each) {
+    GemmTile tile{};
+    GemmArgs a;
+    a.n_rows = cols;
+    a.M = experts ? experts * each : each;
+    a.rows_each = each;
+    a.tiles = experts ? &tile : nullptr;
+    return k_few_pays(a, prec, cols);
+}
+static void check_product_rule() {
+    // sizes at which the one or the other takes at least 1.15 times as long (measured)
+    EXPECT(few(1, 8, 512, 224) && few(1, 16, 512, 224) && few(1, 32, 256, 224) && few(1, 12, 1536, 160) && few(1, 16, 2048, 96) && few(1, 32, 2048, 48));
+    EXPECT(!few(1, 16, 4096, 192) && !few(1, 32, 4096, 112) && !few(1, 24, 2048, 192) && !few(1, 16, 2048, 192) && !few(1, 12, 3072, 176));
+    EXPECT(!few(1, 8, 256, 320) && few(1, 96, 4096, 40) && !few(1, 96, 4096, 56) && few(0, 96, 4096, 48) && !few(0, 8, 512, 64));
+    EXPECT(few(1, 0, 32000, 16) && few(1, 0, 8192, 160) && few(1, 0, 9216, 128) && few(1, 0, 1024, 509) && few(0, 0, 32000, 128) && !few(0, 0, 32000, 160) && !few(1, 0, 32000, 256));
+    // ... and where the smaller kernel is up to 8 % behind
+    EXPECT(!few(1, 0, 14336, 96) && !few(1, 0, 32000, 64));
+}
+
 int main() {
+    check_product_rule();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
     check_shape(4096, 14336, 32, 32, 8, 128256, 512, q4, 14, 0, true);    // the headline model
