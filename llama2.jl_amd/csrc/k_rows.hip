@@ -2,9 +2,9 @@
 // choice), its wavefronts stream whole matrix rows, two at a time, 16 bytes per lane and load, and a fused epilogue writes
 // the results.  Activations and sums are fp32 throughout.
 #include "layered_dev.h"
+#include "rows_plan.h"
 
 #define ROWS_THREADS 512
-#define ROWS_WAVES 8
 #define ROWS_MAX_EXPERTS 1024
 #define ROWS_MAX_TOP 64
 
@@ -351,26 +351,18 @@ __global__ __launch_bounds__(ROWS_THREADS, 4) void rows_kernel(RowsArgs a, RowsP
 }
 
 #define ROWS_MAX_DEVICES 64
-#define ROWS_MAX_PAIRS 4096  // of a workgroup: 32 KB of results
-
-// LDS of a workgroup: the vectors, then the results of its pairs, where the choice of experts has its logits before
-static size_t rows_lds(const RowsArgs &a, int pro, int pairs) {
-    const int nvec = pro == RP_DOWN ? a.top : 1;
-    return ((size_t)nvec * a.ld + std::max(2 * pairs, pro == RP_UP || pro == RP_DOWN ? a.n_experts : 0)) * sizeof(float);
-}
 
 template <int PRO, int EPI, int U, int V, bool Y>
 static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
-    const int nvec = PRO == RP_DOWN ? a.top : 1;
     const int64_t pairs = (a.n_rows + 1) / 2;
     RowsPlan pl;
     pl.plane = a.ld / 2;
     pl.pairs = (int)(pairs / grid);
     pl.more = (int)(pairs % grid);
     pl.per_vec = (a.ld + 512 * U - 1) / (512 * U);
-    pl.per_pair = nvec * pl.per_vec;
+    pl.per_pair = rows_vectors(a, PRO) * pl.per_vec;
     const size_t lds = rows_lds(a, PRO, pl.pairs + 1);
-    if (lds > 152 * 1024) return hipErrorInvalidValue;
+    if (lds > ROWS_LDS) return hipErrorInvalidValue;
     if (lds > 48 * 1024) {
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
@@ -378,7 +370,7 @@ static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
         if (dev < 0 || dev >= ROWS_MAX_DEVICES) return hipErrorInvalidDevice;
         static bool attr_set[ROWS_MAX_DEVICES] = {};
         if (!attr_set[dev]) {
-            e = hipFuncSetAttribute((const void *)rows_kernel<PRO, EPI, U, V, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
+            e = hipFuncSetAttribute((const void *)rows_kernel<PRO, EPI, U, V, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, ROWS_LDS);
             if (e != hipSuccess) return e;
             attr_set[dev] = true;
         }
@@ -389,15 +381,9 @@ static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
 
 template <int PRO, int EPI, int V, bool Y>
 static hipError_t rows_split(hipStream_t s, const RowsArgs &a, int n_cu) {
-    const int64_t pairs = (a.n_rows + 1) / 2;
-    const int nvec = PRO == RP_DOWN ? a.top : 1;
-    auto steps = [&](int u) { return pairs * nvec * ((a.ld + 512 * u - 1) / (512 * u)); };
-    // two workgroups per CU where LDS holds their vectors and there is a step for every wavefront
-    const int64_t most = (rows_lds(a, PRO, (int)std::min<int64_t>(ROWS_MAX_PAIRS, pairs / (2 * n_cu) + 1)) > 78 * 1024 ? 1 : 2) * (int64_t)n_cu;
-    auto grid = [&](int u) {
-        const int64_t n = std::max<int64_t>(1, std::min(std::min(most, pairs), (steps(u) + ROWS_WAVES - 1) / ROWS_WAVES));
-        return std::max(n, (pairs + ROWS_MAX_PAIRS - 2) / (ROWS_MAX_PAIRS - 1));
-    };
+    const int64_t most = rows_most(a, PRO, n_cu);
+    auto steps = [&](int u) { return rows_steps(a, PRO, u); };
+    auto grid = [&](int u) { return rows_grid(a, PRO, n_cu, u); };
     // 4 KB of a row at a time where that leaves at least half of the wavefronts' places a step (a 4096 x 4096 matrix: 7.9 us, against
     // 8.8 in steps of 1 KB); rows of up to 1024 inputs whole (3072 x 768: 3.5 us against 4.8 in two steps).  A pending update of
     // more than 4096 elements takes the registers of the long steps.

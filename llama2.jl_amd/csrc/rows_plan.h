@@ -1,0 +1,37 @@
+// How k_rows.hip deals out a matrix: workgroups, and the LDS of one.
+#pragma once
+
+#include <algorithm>
+
+#include "layered.h"
+
+#define ROWS_WAVES 8
+#define ROWS_MAX_PAIRS 4096  // row pairs of a workgroup at most: 32 KB of results
+#define ROWS_LDS (152 * 1024)
+
+inline int rows_vectors(const RowsArgs &a, int pro) { return pro == RP_DOWN ? a.top : 1; }
+
+// LDS of a workgroup of `pairs` row pairs: the vectors, then the results, where the choice of experts has its logits before
+inline size_t rows_lds(const RowsArgs &a, int pro, int64_t pairs) {
+    return ((size_t)rows_vectors(a, pro) * a.ld + std::max<size_t>(2 * (size_t)pairs, pro == RP_UP || pro == RP_DOWN ? a.n_experts : 0)) * sizeof(float);
+}
+
+// steps of 512 u inputs (rows_kernel) in all
+inline int64_t rows_steps(const RowsArgs &a, int pro, int u) {
+    return (a.n_rows + 1) / 2 * rows_vectors(a, pro) * ((a.ld + 512 * u - 1) / (512 * u));
+}
+
+// two workgroups per CU where LDS holds their vectors and results
+inline int64_t rows_most(const RowsArgs &a, int pro, int n_cu) {
+    const int64_t pairs = (a.n_rows + 1) / 2;
+    return (rows_lds(a, pro, std::min<int64_t>(ROWS_MAX_PAIRS, pairs / (2 * n_cu) + 1)) > 78 * 1024 ? 1 : 2) * (int64_t)n_cu;
+}
+
+// workgroups: no more than that while there is a step for every wavefront and, beside the vectors, LDS for the results
+// (32 768 inputs leave room for 3072 pairs)
+inline int64_t rows_grid(const RowsArgs &a, int pro, int n_cu, int u) {
+    const int64_t pairs = (a.n_rows + 1) / 2, vectors = (int64_t)rows_vectors(a, pro) * a.ld;
+    const int64_t room = std::max<int64_t>(2, std::min<int64_t>(ROWS_MAX_PAIRS, (ROWS_LDS / 4 - vectors) / 2));
+    const int64_t n = std::max<int64_t>(1, std::min(std::min(rows_most(a, pro, n_cu), pairs), (rows_steps(a, pro, u) + ROWS_WAVES - 1) / ROWS_WAVES));
+    return std::max(n, (pairs + room - 2) / (room - 1));
+}

@@ -5,7 +5,7 @@
 // (hipcc with the sanitizers on the host side only).
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
-#include "../../llama2.jl_amd/csrc/layered.h"
+#include "../../llama2.jl_amd/csrc/rows_plan.h"
 
 #include <stdio.h>
 
@@ -145,8 +145,27 @@ static void check_product_rule() {
     EXPECT(!few(1, 0, 14336, 96) && !few(1, 0, 32000, 64));
 }
 
+// a decode product's workgroups have the LDS they need at every size that a model may have
+static void check_rows_plan() {
+    for (int n_cu : {32, 256})
+        for (int K : {1, 700, 2048, 8192, 32768, 36864})
+            for (int64_t rows : {(int64_t)1, (int64_t)255, (int64_t)32768, (int64_t)262144, (int64_t)1600000, (int64_t)20000000})
+                for (int pro : {RP_PLAIN, RP_NORM, RP_UP, RP_DOWN})
+                    for (int top : {1, 9, 64}) {
+                        RowsArgs a;
+                        a.K = K, a.ld = (K + 63) / 64 * 64, a.n_rows = rows, a.top = top, a.n_experts = 1024;
+                        if (pro == RP_DOWN && (int64_t)top * a.ld > 36864) continue;
+                        if (pro == RP_NORM && K > 32768) continue;
+                        for (int u : {1, 2, 4}) {
+                            const int64_t n = rows_grid(a, pro, n_cu, u), pairs = (rows + 1) / 2;
+                            EXPECT(n >= 1 && n <= pairs && rows_lds(a, pro, pairs / n + 1) <= ROWS_LDS);
+                        }
+                    }
+}
+
 int main() {
     check_product_rule();
+    check_rows_plan();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
     check_shape(4096, 14336, 32, 32, 8, 128256, 512, q4, 14, 0, true);    // the headline model
