@@ -4,6 +4,7 @@
 // issues their launch sequences; the token loop, the recorded graph, argmax, sampling
 // and the prompt pass's chunking are the library's own (api.cpp).
 #include <math.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include "layered.h"
@@ -48,6 +49,7 @@ struct Layered {
     uint64_t have = 0;
     int pos = 0;  // positions the state has taken in
     void *stage = nullptr;  // for uploads, until finalize
+    int64_t stage_bytes = (int64_t)64 << 20;
     // one token
     float *x_alt = nullptr, *in = nullptr, *mix = nullptr, *ssq = nullptr, *gate = nullptr, *hid = nullptr, *z = nullptr,
           *se = nullptr, *y = nullptr, *part = nullptr, *x0 = nullptr, *lq = nullptr, *qa = nullptr;
@@ -196,6 +198,7 @@ extern "C" int l2h_layered_create(l2h_ctx *ctx, const l2h_layered_config *cfg, c
     m->c.vocab_size = c.vocab_size;
     m->c.seq_len = c.seq_len;
     l->c = c;
+    if (const char *e = getenv("L2H_STAGE_BYTES")) l->stage_bytes = std::min<long long>((int64_t)64 << 20, std::max<long long>(0, atoll(e)));
     l->layer.resize((size_t)c.n_layers);
     for (int i = 0; i < c.n_layers; i++) {
         const bool again = c.loop_times > 0 && i == c.loop_start;
@@ -494,8 +497,7 @@ static int layered_slot(l2h_model *m, int role, int layer, int expert, LSlot *s)
 
 // ne1 rows of ne0 bf16 elements from the host to rows `pitch` elements apart.  A strided copy out of pageable memory goes row by row
 // (0.3 to 0.6 GB/s measured; a 7 GB model took 12 s to load), a plain one at 20 GB/s: rows that do not lie end to end are
-// uploaded as they are into a staging block and spread out on the device.
-#define L_STAGE_BYTES ((int64_t)64 << 20)
+// uploaded as they are into a staging block and spread out on the device.  L2H_STAGE_BYTES: the block's size (0: none).
 static int put_rows(l2h_model *m, uint16_t *dst, int64_t pitch, const void *host, int64_t ne0, int64_t ne1) {
     l2h_ctx *ctx = m->ctx;
     Layered *l = m->lay;
@@ -503,13 +505,15 @@ static int put_rows(l2h_model *m, uint16_t *dst, int64_t pitch, const void *host
         HIPCHK(ctx, hipMemcpy(dst, host, (size_t)(ne0 * ne1) * 2, hipMemcpyHostToDevice));
         return L2H_OK;
     }
-    if (!l->stage && hipMalloc(&l->stage, (size_t)L_STAGE_BYTES) != hipSuccess) {  // (a device that has room for the model only)
+    const int64_t most = l->stage_bytes / 2 / ne0;  // rows of a block; 0: it does not hold one
+    if (most && !l->stage && hipMalloc(&l->stage, (size_t)l->stage_bytes) != hipSuccess) {  // (a device that has room for the model only)
         (void)hipGetLastError();
         l->stage = nullptr;
+    }
+    if (!most || !l->stage) {
         HIPCHK(ctx, hipMemcpy2D(dst, (size_t)pitch * 2, host, (size_t)ne0 * 2, (size_t)ne0 * 2, (size_t)ne1, hipMemcpyHostToDevice));
         return L2H_OK;
     }
-    const int64_t most = std::max<int64_t>(1, L_STAGE_BYTES / 2 / ne0);
     for (int64_t r = 0; r < ne1; r += most) {
         const int64_t n = std::min(most, ne1 - r);
         HIPCHK(ctx, hipMemcpy(l->stage, (const uint16_t *)host + r * ne0, (size_t)(n * ne0) * 2, hipMemcpyHostToDevice));

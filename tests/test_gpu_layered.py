@@ -216,6 +216,25 @@ def test_short_prompts(pkg, precision):
     dev.close()
 
 
+@pytest.mark.parametrize("stage", ["0", "100", "4000", "70001"])
+def test_upload_through_any_staging_block(pkg, monkeypatch, stage):
+    """Matrices go up the same through a block of any size: one that holds no row of theirs or cannot be had (0), some rows, whole matrices"""
+    c = lc.config([lc.attention(heads=3, kv_heads=1, dim=20, vdim=12, rot=8, mlp=lc.dense(75)),
+                   lc.delta(heads=2, kv_heads=2, dim=16, vdim=16, conv=4, ranks=(7, 9), mlp=lc.moe(5, 2, 33))], width=90, vocab=201, side=24)
+    t = ref.random_tensors(c, 47)
+    tok = lc.tokens(9, c["vocab"], 3)
+    got = []
+    for value in (stage, None):
+        if value is None:
+            monkeypatch.delenv("L2H_STAGE_BYTES", raising=False)
+        else:
+            monkeypatch.setenv("L2H_STAGE_BYTES", value)
+        dev = lc.language_model(pkg, c, t).device()
+        got.append(_decode(dev, tok))
+        dev.close()
+    assert np.array_equal(got[0], got[1]) and np.all(np.isfinite(got[0]))
+
+
 def test_prompt_longer_than_one_chunk(pkg):
     """2048 positions go at a time: a longer prompt continues from the cache and state its first chunk left"""
     c = lc.config([lc.delta(heads=2, kv_heads=1, dim=16, vdim=16, conv=4, ranks=(4, 4)), lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=40, rot=16)],
