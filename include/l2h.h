@@ -104,7 +104,8 @@ int l2h_model_set_kv_type(l2h_model *m, int kv_type);
  * streams fetched ahead into LDS, activations exchanged as epoch-tagged words).  Path 3 takes
  *   - q4_K, q5_K or q6_K layer matrices (w1 and w3 of a layer of one type) with a q4_K or q6_K classifier:
  *     dim a multiple of 256, at most 4096, and either a multiple of 2048 or at most a quarter below one
- *     (1536..2048, 3072..4096; with a q6_K classifier and the lower range by the automatic choice only);
+ *     (1536..2048, 3072..4096; with a q6_K classifier the lower range is taken by the automatic choice and refused
+ *     where path 3 is asked for by number);
  *     hidden_dim a multiple of 2048 up to 14336; head size 32, 64, 96 or 128; fp32 or fp16 cache;
  *   - models whose matrices are all fp32: dim and hidden_dim multiples of 4, at most 4096; head size 32, 64
  *     or 128; fp32 cache;

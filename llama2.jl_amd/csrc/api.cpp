@@ -702,8 +702,8 @@ static int flow_setup(l2h_model *m) {
     const int cls_type = m->glob[L2H_OUTPUT].type;
     std::string why;
     // A q6_K classifier with dim 1536 .. 2048 has its rows in pairs.  8 layers of 2048 x 8192 (16 heads on 4) with one: a
-    // 37-token prompt and 16 tokens 6.47 ms on path 1, 4.50 ms here.  The automatic choice takes it; a caller that asks for path 3 by number is told, as ever, that
-    // the model does not fit it.
+    // 37-token prompt and 16 tokens 6.47 ms on path 1, 4.50 ms here.  The automatic choice takes it.  Asked for by number path 3 refuses
+    // such a model as it did before its rows could go in pairs (the reason says so): what callers were refused stays refused.
     if (!k_flow_plan(a, types.data(), (int)types.size(), cls_type, grid, &why, !required)) {
         m->flow_why = why;
         return required ? set_err(ctx, L2H_EINVAL, "streaming kernel not available: %s", why.c_str()) : L2H_OK;

@@ -2577,7 +2577,7 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
     if (a.dim % 256 != 0 || (int64_t)a.dim * 4 < (int64_t)a.dim_pad * 3 || a.hidden % 2048 != 0)
         return no("dim must be a multiple of 2048 (or of 256 and within a quarter below one), hidden_dim a multiple of 2048");
     if (a.dim_pad != a.dim) a.mixed = 1;
-    if (cls_type == L2H_TYPE_Q6_K && a.dim_pad % 4096 != 0 && !cls_pairs) return no("a q6_K classifier needs dim to be a multiple of 4096");
+    if (cls_type == L2H_TYPE_Q6_K && a.dim_pad % 4096 != 0 && !cls_pairs) return no("with a q6_K classifier and dim up to 2048 it runs by the automatic choice only");
     if (a.hidden > 14336 || a.dim_pad > 4096) return no("dim above 4096 or hidden_dim above 14336");
     if (a.n_heads > grid || (a.hs != 32 && a.hs != 64 && a.hs != 96 && a.hs != 128)) return no("head size must be 32, 64, 96 or 128");
     if (a.hs == 96) a.mixed = 1;

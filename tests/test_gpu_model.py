@@ -708,6 +708,24 @@ def test_streaming_kernel_with_paired_classifier_rows(pkg, shape):
     slow.close()
 
 
+def test_paired_classifier_rows_say_who_may_have_them(pkg):
+    """Asked for by number, path 3 refuses such a model for what it is, not for a size that its kernel could not run; with an fp16 cache
+    the automatic choice takes it too, with the per-phase path's results."""
+    from llama2_jl_amd import synth
+    from llama2_jl_amd.inference import DeviceModel
+    plan, dim, hidden, layers, heads, kv, vocab, neox = PAIRED[2]
+    lm = _model(pkg, plan, dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=heads, n_kv_heads=kv, vocab_size=vocab,
+                seq_len=320, rope_freq_base=10000.0, rope_is_neox=neox)
+    with pytest.raises(pkg.L2HError, match="automatic choice"):
+        DeviceModel(lm.config, lm.weights, path=3)
+    fast, slow = DeviceModel(lm.config, lm.weights, kv_fp16=True), DeviceModel(lm.config, lm.weights, path=1, kv_fp16=True)
+    assert fast.path == 3 and slow.path == 1
+    got = [d.generate_greedy(synth.seeded_prompt(64, 5, vocab), 40, want_logits=True) for d in (fast, slow)]
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    fast.close()
+    slow.close()
+
+
 @pytest.mark.parametrize("case", sorted(FLOW_CASES))
 def test_state_after_a_step_of_the_streaming_kernel(pkg, case):
     """RunState buffers as the per-phase path leaves them"""
