@@ -119,8 +119,9 @@ __host__ __device__ inline int flow_n_local(const FlowGeom &g, int wg) {
     const int hi = lo + g.rpw < g.n_rows ? lo + g.rpw : g.n_rows;
     return hi > lo ? hi - lo : 0;
 }
-// Rows that end in the middle of a piece (FlowGeom::ppr == 0) come in pairs of flow_half() pieces: rpw and n_rows are
-// even.  H = false: the caller knows that the geometry has none (kernels that are not built for them do not look).
+// Rows that end in the middle of a piece (FlowGeom::ppr == 0) come in pairs of flow_half() pieces: rpw is even, and so is
+// n_rows in the layer phases.  A classifier in pairs may have an odd number of rows: the missing row of its last pair is zero
+// super-blocks whose sum nobody reads.  H = false: the caller knows that the geometry has none (kernels that are not built for them do not look).
 template <bool H = true>
 __host__ __device__ inline int flow_half(const FlowGeom &g) {
     return H && g.ppr == 0 ? g.K >> 10 : 0;
@@ -2520,10 +2521,10 @@ static FlowGeom make_geom(int64_t n_rows, int64_t K, int type, int grid, bool ha
     return g;
 }
 
-// Can the model run on this kernel?  q4_K layer matrices with input lengths that are multiples of
-// 2048 (whole pieces per row), a q4_K or q6_K classifier, and sizes that
-// fit the kernel's LDS areas.  On success fills the geometry fields of `a` for a grid of `grid`.
-// cls_pairs: a q6_K classifier with dim_pad 2048 may run with its rows in pairs.
+// Can the model run on this kernel?  q4_K, q5_K or q6_K layer matrices whose rows are whole pieces of 2048 inputs, padded to them by a
+// third at most, or go in pairs (dim 3072); a q4_K or q6_K classifier; or fp32 matrices throughout; and sizes that fit the kernel's LDS
+// areas.  On success fills the geometry fields of `a` for a grid of `grid`.
+// cls_pairs: a q6_K classifier with dim_pad 2048, whose rows are half a piece, may run with them in pairs.
 bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why, bool cls_pairs) {
     auto no = [&](const char *m) {
         if (why) *why = m;

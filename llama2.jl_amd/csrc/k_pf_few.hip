@@ -108,10 +108,11 @@ __global__ __launch_bounds__(512, T == 1 ? 4 : 2) void pf_few_kernel(PfFewArgs a
 // unlike k_pf_gemm's, which is the same bit for bit from the quantized blocks: for passes that form other sums their own way too.
 //
 // Chosen where its tiles of 64 x 64 results are at most one a CU.  Microseconds in 256-row tiles and like this, rows x inputs: 16384 x
-// 2048: 8, 37, 64 positions 29.4, 33.5, 34.8 and 16.3, 21.3, 24.4, but beyond one tile a CU 200 positions 36.8 and 60.6; 16384 x 3072:
-// 40.4, 45.3, 47.3 and 21.6, 29.6, 34.9; 4000 x 1024: 18.9 and 6.4 (64 positions), 21.2 and 11.1 (256), 21.2 and 19.3 (500); 28672 x
-// 4096, 37 positions (448 tiles): 62.6 and 68.0.  Tiles of 32 x 32 where the positions fit one of those or where the larger ones are
-// at most half the CUs: 4000 x 1024, 96 positions: 9.2, against 10.3; 200 (252 tiles): 14.3 and 10.6; 16384 x 2048, 16: 18.2 and 19.6.
+// 2048: 8, 37, 64 positions 28.9, 33.3, 35.0 and 15.7, 20.9, 23.8, but beyond one tile a CU 128 positions 38.6 and 38.5; 16384 x 3072:
+// 39.5, 45.2, 47.6 and 21.1, 29.3, 34.5; 4096 x 1024: 64 and 256 positions 21.3, 23.0 and 6.9, 11.3; 28672 x 4096,
+// 37 positions (448 tiles): 62.8 and 69.2.  Tiles of 32 x 32 where the positions fit one of those or where the larger ones are at most half
+// the CUs: 4096 x 1024, 96 positions (128 tiles): 9.8, against 10.8; 200 (256 tiles): 14.7 and 10.5; 16384 x 2048, 16: 17.6 and 19.2.
+// (rows: twice hidden_dim, which is a multiple of 64 where there is a bf16 copy.)
 static int64_t pf_few_tiles(int64_t rows, int M, int side) { return (rows / side) * ((M + side - 1) / side); }
 bool k_pf_few_pays(int64_t rows, int M) { return pf_few_tiles(rows, M, 64) <= 256; }
 hipError_t k_pf_few(hipStream_t s, const uint16_t *wbf, int64_t rows, const uint16_t *act, int M, int64_t K, uint16_t *hb, int64_t ldb) {

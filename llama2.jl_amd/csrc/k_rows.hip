@@ -18,12 +18,8 @@ struct RowsChunk {
 };
 typedef uint32_t rows_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 rows_word(const uint16_t *w) {
-#ifdef ROWS_PLAIN
-    return *(const uint4 *)w;
-#else
     const rows_u32x4 v = __builtin_nontemporal_load((const rows_u32x4 *)w);
     return make_uint4(v.x, v.y, v.z, v.w);
-#endif
 }
 // (no load is skipped: how many are under way has to be known when the code is compiled for a wait to leave the later ones alone)
 __device__ __forceinline__ void rows_load(RowsChunk &c, const uint16_t *w0, const uint16_t *w1, int k, int ld) {
@@ -53,8 +49,7 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
     acc1 = fmaf(l_bf16_hi(q.w), xb.w, acc1);
 }
 
-
-// how a matrix's rows are dealt out (rows_plan): workgroup b has `pairs` row pairs, and one more for b < more, one after another
+// how a matrix's rows are dealt out (rows_plan.h): workgroup b has `pairs` row pairs, and one more for b < more, one after another
 struct RowsPlan {
     int plane;            // half of a staged vector's floats
     int pairs, more;
