@@ -1318,6 +1318,10 @@ __device__ __forceinline__ int flow_next_token(unsigned epoch) {
             if ((spins & 63) == 63 && __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
             __builtin_amdgcn_s_sleep(1);
         }
+        // The step before has appended cache rows, and a line of keys holds eight positions: what this compute unit's vector cache has of
+        // those lines is thrown away.  (Uncached memory is uncached in the L2s only.  Without this a model whose rows do not sweep the
+        // vector cache between two reads of a line, dim 256 and hidden 4, took old keys from the third step of a launch on.)
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if ((threadIdx.x & 63) == 0) s_tok = tok;
     }
     flow_barrier_lds();

@@ -1,0 +1,39 @@
+"""Decoding of small fp32 models by the single-launch kernel against the per-phase path, bit for bit.  Both form exact products and
+fp64 sums that are rounded once, so that another order of a sum shows only where it lies within 1e-15 of the middle between two
+floats."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(pkg, seed, dim, hidden, layers, heads, kv, vocab, neox):
+    from llama2_jl_amd import synth
+    from llama2_jl_amd.inference import DeviceModel
+    cfg = pkg.ModelConfig(dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=heads, n_kv_heads=kv, vocab_size=vocab, seq_len=320,
+                          rope_freq_base=10000.0, rope_is_neox=neox)
+    lm = synth.synthetic_model(cfg, synth.PLAN_F32, seed=seed)
+    fast, slow = DeviceModel(cfg, lm.weights, path=3), DeviceModel(cfg, lm.weights, path=1)
+    assert fast.path == 3 and slow.path == 1
+    return fast, slow
+
+
+def _same(fast, slow, prompt, n_new):
+    fast.reset()
+    slow.reset()
+    (a, la), (b, lb) = (d.generate_greedy(prompt, n_new, want_logits=True) for d in (fast, slow))
+    assert np.asarray(a).tolist() == np.asarray(b).tolist()
+    assert np.array_equal(la.view(np.uint32), lb.view(np.uint32))
+    for name in ("x", "xb", "q", "hb"):
+        assert np.array_equal(fast.state(name).view(np.uint32), slow.state(name).view(np.uint32)), name
+
+
+@pytest.mark.parametrize("n_new", [2, 7, 19])
+def test_keys_of_the_steps_before_in_one_launch(pkg, n_new):
+    """A layer so small that nothing sweeps the vector cache between a step's read of a line of keys and the next step's"""
+    from llama2_jl_amd import synth
+    fast, slow = _pair(pkg, 31, 256, 4, 2, 8, 8, 300, False)
+    assert fast.steps_per_launch == 8
+    _same(fast, slow, synth.seeded_prompt(70, 2, 300), n_new)
+    fast.close()
+    slow.close()
