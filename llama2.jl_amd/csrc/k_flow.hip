@@ -2357,6 +2357,419 @@ __global__ __launch_bounds__(1024) void flow_f32_kernel(unsigned int gen0, int n
 }
 
 // ------------------------------------------------------------------------------------------
+// small models of fp32 matrices (dim 256 or 512; f32_wave_plan): a wavefront takes a pair of rows from the input to the stores of its results
+//
+// What bounds such a model is the chain of hand-overs, not its bytes (a 512-wide layer's 12.6 MB stream in 3 us).  So
+//  * a phase has one barrier, behind the wait for its input.  Wavefronts with rows then take the input from LDS into registers, in the
+//    places of the row's own 16-byte loads, each norms it for itself, and lanes 0 and 1 finish the pair.  w2's rows, up to 4096
+//    long, go in slices of at most 512 inputs, a wavefront each, that meet in LDS behind a second barrier.
+//  * a phase's rows are requested as soon as the phase before it has its input: a compute unit's loads pass its polls by, and a
+//    request of 24 KB in front of a wait makes the wait 1 to 1.5 us longer (7.3 ms against 5.8 in the run below).
+//  * the heads' workgroups have no rows: theirs would come late behind the attention and hold up the next phase (6.5 ms).
+// 48 tokens of 8 layers of 512 x 1376 and 32 000 rows of classifier: 5.90 ms; 8.46 with flow_f32_kernel, whose workgroups stage an
+// input between two barriers, on all wavefronts, and begin loops and epilogues with divisions and scalar loads (about 1 us of loop and 0.4 to 1.2
+// of epilogue a phase against 0.6 and 0.1 to 0.6 here).  Every wavefront waiting for the whole input itself, with no barrier at
+// all: 6.9 ms (six wavefronts of a CU that read 4 KB a poll).
+// ------------------------------------------------------------------------------------------
+template <int NQ>
+struct F32Rows {
+    f32x4v w[2][NQ];
+};
+// What a request that a wavefront may leave out has left in these registers before is of no use to anybody; without saying so they
+// would be kept from one request to the next, across the attention, on the stack.
+template <int N>
+__device__ __forceinline__ void flowv_forget(f32x4v (&x)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; u++) asm volatile("" : "=v"(x[u]));
+}
+template <int NQ>
+__device__ __forceinline__ void flowv_forget(F32Rows<NQ> &r) {
+    flowv_forget(r.w[0]);
+    flowv_forget(r.w[1]);
+}
+// Said before the next rows are requested, behind a wait: the compiler counts the loads under way for itself and would wait for the new
+// rows too at the first use of the old ones, the new request being conditional (1.3 us of loop instead of 0.6).
+template <int N>
+__device__ __forceinline__ void flowv_arrived(f32x4v (&x)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; u++) asm volatile("" : "+v"(x[u]));
+}
+template <int NQ>
+__device__ __forceinline__ void flowv_arrived(F32Rows<NQ> &r) {
+    flowv_arrived(r.w[0]);
+    flowv_arrived(r.w[1]);
+}
+// 16-byte groups lane, lane + 64, ... of the n4 of a row pair (a lane beyond them repeats the last one; not used)
+template <int NQ>
+__device__ __forceinline__ void flowv_rows(F32Rows<NQ> &r, const float *w0, const float *w1, int n4, int lane) {
+    const AS1 f32x4v *p0 = (const AS1 f32x4v *)w0, *p1 = (const AS1 f32x4v *)w1;
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        const int i = min(lane + 64 * u, n4 - 1);
+        r.w[0][u] = __builtin_nontemporal_load(p0 + i);
+        r.w[1][u] = __builtin_nontemporal_load(p1 + i);
+    }
+}
+template <int NQ>
+__device__ __forceinline__ void flowv_norm_weights(f32x4v (&nw)[NQ], const float *w, int n4, int lane) {
+#pragma unroll
+    for (int u = 0; u < NQ; u++) nw[u] = ((const AS1 f32x4v *)w)[min(lane + 64 * u, n4 - 1)];
+}
+// The workgroup's first wavefronts wait for the 4 n4 bare words at src, 64 groups of four each, and put them into LDS (the last ones, which
+// have no rows: 6.2 ms, in the terms above; polls that go out while the rows are still coming).  False if a wait gave up; every wavefront calls this.
+__device__ __forceinline__ bool flowv_stage(const unsigned *src, int n4, int wave, int lane) {
+    const int i = 64 * wave + lane;
+    if (64 * wave < n4) {
+        u32x4v w = {FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY};
+        const unsigned *p = src + 4 * min(i, n4 - 1);
+        unsigned spins = 0;
+        for (;;) {
+            const bool full = w.x != FLOW_EMPTY && w.y != FLOW_EMPTY && w.z != FLOW_EMPTY && w.w != FLOW_EMPTY;
+            if (!full) POLL_BARE1(w, p);
+            const bool all = w.x != FLOW_EMPTY && w.y != FLOW_EMPTY && w.z != FLOW_EMPTY && w.w != FLOW_EMPTY;
+            if (__ballot(!all) == 0ull) break;
+            if (++spins > c_flow.spin_limit ||
+                ((spins & 63) == 0 && __hip_atomic_load(c_flow.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                s_flag = 1;
+                break;
+            }
+        }
+        if (i < n4) ((u32x4v *)s_act)[i] = w;
+    }
+    flow_barrier_lds();
+    if (s_flag) {
+        if (threadIdx.x == 0) __hip_atomic_store(c_flow.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    return true;
+}
+// groups first + lane, first + lane + 64, ... of the staged input, zero beyond n4 of them
+template <int NQ>
+__device__ __forceinline__ void flowv_input(f32x4v (&x)[NQ], int first, int n4, int lane) {
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        x[u] = ((const f32x4v *)s_act)[first + min(lane + 64 * u, n4 - 1)];
+        if (lane + 64 * u >= n4) x[u] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    }
+}
+// rmsnorm! (reference src/inference.jl:102-110) of the K elements that the wavefront holds
+template <int NQ>
+__device__ __forceinline__ void flowv_norm(f32x4v (&x)[NQ], const f32x4v (&nw)[NQ], int K) {
+    double acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < NQ; u++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc = fma((double)x[u][k], (double)x[u][k], acc);
+    float ss = (float)wave_sum_f64_dpp(acc);
+    ss /= (float)K;
+    ss += 1e-5f;
+    ss = 1.0f / sqrtf(ss);
+#pragma unroll
+    for (int u = 0; u < NQ; u++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[u][k] = nw[u][k] * (ss * x[u][k]);
+}
+// the wavefront's pair of rows against x: exact products, fp64 sums; both values on every lane
+template <int NQ>
+__device__ __forceinline__ void flowv_dot(const F32Rows<NQ> &r, const f32x4v (&x)[NQ], int n4, int lane, double &v0, double &v1) {
+    double a0 = 0.0, a1 = 0.0;
+#pragma unroll
+    for (int u = 0; u < NQ; u++)
+        if (lane + 64 * u < n4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double xk = (double)x[u][k];
+                a0 = fma((double)r.w[0][u][k], xk, a0);
+                a1 = fma((double)r.w[1][u][k], xk, a1);
+            }
+        }
+    v0 = wave_sum_f64_dpp(a0);
+    v1 = wave_sum_f64_dpp(a1);
+}
+// Functions of their own for the constants of their fp64 arithmetic: inlined into the loops over layers and steps those are
+// hoisted out of them, into registers that the attention's call then puts on the stack.
+__device__ __noinline__ float flowv_swiglu(float h1, float h3) { return swiglu_val(h1, h3); }
+__device__ __noinline__ void flowv_rope(int pos, int i) {
+    float theta = 1.0f * (float)pos;
+    for (int k = 0; k < i; k++) theta *= c_flow.theta_scale;
+    s_rope[2 * i] = (float)cos((double)theta);
+    s_rope[2 * i + 1] = (float)sin((double)theta);
+}
+
+#define FLOWV_CLS 16  // 16-byte groups of classifier rows that a lane has under way
+template <int NQ>
+__global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, int n_tok) {
+    const FlowArgs &a = c_flow;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wg = blockIdx.x, nwg = gridDim.x;
+    const int pos_first = a.ctl->pos, step_first = a.ctl->step, n_prompt = a.ctl->n_prompt, tok_first = a.ctl->last_argmax;
+    if (tid == 0) s_flag = 0;
+#ifdef L2H_TIMELINE
+    int tl_n = 0;
+#define VTL()                                                                                   \
+    do {                                                                                        \
+        if (a.timeline && tid == 0 && tl_n < 64) a.timeline[wg * 64 + tl_n++] = wall_clock64(); \
+    } while (0)
+#else
+#define VTL()
+#endif
+    // (the lane number anew in every phase: what derives from it is computed there, not kept across all of them)
+#define LANE()                   \
+    int lane = threadIdx.x & 63; \
+    asm volatile("" : "+v"(lane))
+    constexpr int dim = 256 * NQ, n4 = dim >> 2;
+    const int hs = a.hs, n_layers = a.n_layers;
+    // attention of head h runs on workgroup h * stride + h % stride (spread over the XCDs), which has no rows of the layers; rw: this
+    // workgroup's number among those that have (past the last row on the heads')
+    const int att_stride = nwg / a.n_heads;
+    const int att_h = uni(wg / att_stride), att_at = att_h % att_stride;
+    const bool is_att = uni((int)(att_h < a.n_heads && wg % att_stride == att_at)) != 0;
+    const int rw = is_att ? nwg : wg - min(att_h, a.n_heads) - (att_h < a.n_heads && wg % att_stride > att_at ? 1 : 0);
+    // this wavefront's tasks: a pair of rows of q|k|v, of wo and of w1|w3; one slice of a pair of w2's
+    const int np_qkv = flow_n_local(a.qkv, rw) >> 1, np_wo = flow_n_local(a.wo, rw) >> 1, np_w13 = flow_n_local(a.w13, rw) >> 1;
+    // (w2's on the last wavefronts: their rows are requested while the first ones work on w1|w3, whose SwiGLU, a function, waits on entry
+    // for what its wavefront has under way)
+    const int sl_log = __builtin_ctz(a.w2.ppr), task2 = FLOW_NW - 1 - wave, slice = task2 & (a.w2.ppr - 1), pair2 = task2 >> sl_log;
+    const int h4 = a.hidden >> 2, per_s = (h4 + a.w2.ppr - 1) >> sl_log, s0 = slice * per_s, n4s = min(per_s, h4 - s0);
+    const bool has_qkv = wave < np_qkv, has_wo = wave < np_wo, has_w13 = wave < np_w13, has_w2 = pair2 < np_wo;
+    const int row_wo = rw * a.wo.rpw + 2 * wave;  // (also the rows of x whose value this wavefront keeps, on lanes 0 and 1)
+    int seg, row, row1;                           // the pair of q|k|v
+    flow_row_src(0, rw * a.qkv.rpw + 2 * wave, dim, a.kv_dim, hs, a.neox, seg, row);
+    flow_row_src(0, rw * a.qkv.rpw + 2 * wave + 1, dim, a.kv_dim, hs, a.neox, seg, row1);
+    float resid = 0.0f;
+    // rows of q|k|v and of w1|w3 are requested a phase ahead, as soon as that phase has its input: a request in front of a wait delays it
+    F32Rows<NQ> r_next;
+    f32x4v nw[NQ];
+    auto request_qkv = [&](int l) {
+        flowv_forget(r_next);
+        flowv_forget(nw);
+        if (!has_qkv) return;
+        LANE();
+        const float *base = (seg == 0 ? a.f_w[0] : (seg == 1 ? a.f_w[1] : a.f_w[2])) +
+                            (int64_t)l * (seg == 0 ? a.f_stride[0] : (seg == 1 ? a.f_stride[1] : a.f_stride[2]));
+        flowv_rows(r_next, base + (int64_t)row * dim, base + (int64_t)row1 * dim, n4, lane);
+        flowv_norm_weights(nw, a.rms_att + (int64_t)l * a.norm_stride, n4, lane);
+    };
+#pragma nounroll
+  for (int t_step = 0; t_step < n_tok; t_step++) {
+    VTL();
+    const unsigned E0 = gen0 + (unsigned)t_step * (5u * (unsigned)n_layers + 2u);
+    const int pos = pos_first + t_step, step = step_first + t_step;
+    // ---- this step's RoPE angles (reference src/inference.jl:122-127) and token; one barrier covers both ----
+    if (wave == 1 && tid - 64 < (hs >> 1)) flowv_rope(pos, tid - 64);  // (the first wavefront waits for the token)
+    request_qkv(0);
+    int tok = tok_first;
+    if (t_step > 0) {
+        tok = uni(flow_next_token(E0));
+        if (tok < 0) {
+            if (tid == 0) __hip_atomic_store(a.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+    } else {
+        flow_barrier_lds();
+    }
+    if (step < n_prompt) tok = a.prompt[step];
+    if (has_wo) {
+        LANE();
+        resid = 0.0f;
+        if (lane < 2) resid = __uint_as_float(bare_of(dequant_elem(a.emb, tok, row_wo + lane)));
+    }
+#pragma nounroll
+    for (int l = 0; l < n_layers; l++) {
+        const unsigned e_x = E0 + 5u * (unsigned)l;
+        const unsigned e_q = e_x + 1, e_att = e_x + 2, e_w13 = e_x + 4;
+        // ---- rmsnorm (:244), q, k, v (:247-249), rope (:255-256), cache append (:259-260) ----
+        {
+            LANE();
+            f32x4v x[NQ];
+            if (l > 0 && !uni((int)flowv_stage(a.x_a, n4, wave, lane))) return;
+            VTL();
+            flowv_arrived(r_next);
+            flowv_arrived(nw);
+            if (is_att && pos < FLOW_ATT_SHORT) flow_touch_cache(l, att_h, pos);
+            if (has_qkv) {
+                if (l == 0) {
+#pragma unroll
+                    for (int u = 0; u < NQ; u++) {
+                        const int i = lane + 64 * u;
+                        if (a.emb.type == L2H_TYPE_F32)
+                            x[u] = *(const AS1 f32x4v *)(a.emb.f32 + (int64_t)tok * dim + 4 * i);
+                        else
+                            x[u] = f32x4v{dequant_elem(a.emb, tok, 4 * i), dequant_elem(a.emb, tok, 4 * i + 1), dequant_elem(a.emb, tok, 4 * i + 2),
+                                          dequant_elem(a.emb, tok, 4 * i + 3)};
+                    }
+                } else {
+                    flowv_input(x, 0, n4, lane);
+                }
+                flowv_norm(x, nw, dim);
+                double v0, v1;
+                flowv_dot(r_next, x, n4, lane, v0, v1);
+                VTL();
+                if (lane < 2) {
+                    const int my_row = lane ? row1 : row, half = hs >> 1;
+                    const int hs_log = 31 - __builtin_clz(hs), head = my_row >> hs_log, el = my_row & (hs - 1);
+                    const int ang = a.neox ? (el & (half - 1)) : (el >> 1);
+                    const float c = s_rope[2 * ang], s = s_rope[2 * ang + 1];
+                    const float re = (float)v0, im = (float)v1;
+                    // complex product (re + i im)(c + i s), each of the four products rounded
+                    const float turned = lane == 0 ? (re * c) - (im * s) : (re * s) + (im * c);
+                    const float out = seg == 2 ? (lane == 0 ? re : im) : turned;
+                    tag_store((seg == 0 ? a.q : (seg == 1 ? a.kcur : a.vcur)) + my_row, out, e_q);
+                    if (seg != 0)
+                        ((seg == 1 ? a.kc : a.vc) + (int64_t)l * a.cache_layer_elems)[seg == 1 ? (((int64_t)head * (hs >> 2) + (el >> 2)) * a.seq_len + pos) * 4 + (el & 3)
+                                                                                               : ((int64_t)head * a.seq_len + pos) * hs + el] = out;
+                }
+                VTL();
+            }
+        }
+        // ---- attention (:263-278) ----
+        if (is_att || pos >= FLOW_ATT_SHORT) {
+            const bool fine = pos >= FLOW_ATT_SHORT ? flow_attention_split<false>(l, pos, e_q, e_att)
+                              : hs == 128 ? flow_attention_short<128>(l, att_h, pos, e_q, e_att)
+                              : hs == 64  ? flow_attention_short<64>(l, att_h, pos, e_q, e_att)
+                                          : flow_attention_short<32>(l, att_h, pos, e_q, e_att);
+            if (!uni((int)fine)) return;
+        }
+        // ---- x += wo * xb (:281-284) ----
+        {
+            LANE();
+            F32Rows<NQ> r;
+            f32x4v x[NQ];
+            flowv_forget(r);
+            if (has_wo) {
+                const float *base = a.f_w[3] + (int64_t)l * a.f_stride[3] + (int64_t)row_wo * dim;
+                flowv_rows(r, base, base + dim, n4, lane);
+            }
+            if (!uni((int)flowv_stage(a.xo + (int64_t)(e_att & 1u) * dim, n4, wave, lane))) return;
+            VTL();
+            flowv_arrived(r);
+            flowv_forget(r_next);
+            flowv_forget(nw);
+            if (has_w13) {
+                const int64_t u = (int64_t)(rw * (a.w13.rpw >> 1) + wave);
+                flowv_rows(r_next, a.f_w[4] + (int64_t)l * a.f_stride[4] + u * dim, a.f_w[5] + (int64_t)l * a.f_stride[5] + u * dim, n4, lane);
+                flowv_norm_weights(nw, a.rms_ffn + (int64_t)l * a.norm_stride, n4, lane);
+            }
+            if (has_wo) {
+                flowv_input(x, 0, n4, lane);
+                double v0, v1;
+                flowv_dot(r, x, n4, lane, v0, v1);
+                VTL();
+                if (lane < 2) {
+                    const unsigned neww = bare_of(resid + (float)(lane ? v1 : v0));
+                    bare_store(a.x_b + row_wo + lane, neww);
+                    resid = __uint_as_float(neww);  // (the value as the other wavefronts read it)
+                    bare_store(a.x_a + row_wo + lane, FLOW_EMPTY);  // (its readers are through: see FLOW_EMPTY)
+                }
+                VTL();
+            }
+        }
+        // ---- rmsnorm (:287), w1, w3 (:291-292), SwiGLU (:295-299) ----
+        F32Rows<2> r_w2;  // (a slice is at most 512 inputs)
+        {
+            LANE();
+            f32x4v x[NQ];
+            const int64_t u = (int64_t)(rw * (a.w13.rpw >> 1) + wave);
+            if (!uni((int)flowv_stage(a.x_b, n4, wave, lane))) return;
+            VTL();
+            flowv_arrived(r_next);
+            flowv_arrived(nw);
+            flowv_forget(r_w2);
+            if (has_w2) {
+                const float *base = a.f_w[6] + (int64_t)l * a.f_stride[6] + (int64_t)(rw * a.w2.rpw + 2 * pair2) * a.hidden + 4 * s0;
+                flowv_rows(r_w2, base, base + a.hidden, n4s, lane);
+            }
+            if (has_w13) {
+                flowv_input(x, 0, n4, lane);
+                flowv_norm(x, nw, dim);
+                double v0, v1;
+                flowv_dot(r_next, x, n4, lane, v0, v1);
+                VTL();
+                const float g = flowv_swiglu((float)v0, (float)v1);
+                if (lane == 0) {
+                    bare_store(a.hbw + (int64_t)(e_w13 & 1u) * a.hidden + u, bare_of(g));
+                    bare_store(a.hbw + (int64_t)((e_w13 & 1u) ^ 1u) * a.hidden + u, FLOW_EMPTY);
+                }
+                VTL();
+            }
+        }
+        // ---- x += w2 * hb (:302-305) ----
+        {
+            LANE();
+            f32x4v x[2];
+            if (!uni((int)flowv_stage(a.hbw + (int64_t)(e_w13 & 1u) * a.hidden, h4, wave, lane))) return;
+            VTL();
+            flowv_arrived(r_w2);
+            if (l + 1 < n_layers) request_qkv(l + 1);
+            if (has_w2) {
+                flowv_input(x, s0, n4s, lane);
+                double v0, v1;
+                flowv_dot(r_w2, x, n4s, lane, v0, v1);
+                if (lane < 2) s_part[2 * task2 + lane] = lane ? v1 : v0;
+            }
+            flow_barrier_lds();
+            VTL();
+            if (has_wo && lane < 2) {
+                double v = 0.0;
+                const double *p = s_part + 2 * (wave << sl_log) + lane;
+                for (int i = 0; i < 1 << sl_log; i++) v += p[2 * i];
+                const unsigned neww = bare_of(resid + (float)v);
+                bare_store(a.x_a + row_wo + lane, neww);
+                resid = __uint_as_float(neww);
+                bare_store(a.x_b + row_wo + lane, FLOW_EMPTY);
+            }
+            VTL();
+        }
+    }
+    // ---- final rmsnorm (:309) + classifier (:312): the wavefronts that wait for x request their rows behind it, the others before ----
+    const unsigned e_cls = E0 + 5u * (unsigned)n_layers + 1;
+    {
+        LANE();
+        constexpr int RB = FLOWV_CLS / NQ;  // rows a batch
+        const int cnt = uni(flow_wave_pieces<false>(a.cls, wg, wave)), start = uni(flow_wave_start<false>(a.cls, wg, wave));
+        const float *cls_w = a.f_w[7] + ((int64_t)wg * a.cls.rpw + start) * dim;
+        f32x4v wc[RB][NQ], x[NQ], nw[NQ];
+#pragma unroll
+        for (int i = 0; i < RB; i++) flowv_forget(wc[i]);
+        auto fetch = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+#pragma unroll
+                for (int u = 0; u < NQ; u++)
+                    wc[i][u] = __builtin_nontemporal_load((const AS1 f32x4v *)(cls_w + (int64_t)max(0, min(i0 + i, cnt - 1)) * dim) + min(lane + 64 * u, n4 - 1));
+        };
+        flowv_norm_weights(nw, a.rms_final, n4, lane);
+        const bool waits = 64 * wave < n4;
+        if (!waits && cnt > 0) fetch(0);
+        if (!uni((int)flowv_stage(a.x_a, n4, wave, lane))) return;
+        if (waits && cnt > 0) fetch(0);
+        flowv_input(x, 0, n4, lane);
+        flowv_norm(x, nw, dim);
+#pragma nounroll
+        for (int i0 = 0; i0 < cnt; i0 += RB) {
+            if (i0) fetch(i0);
+#pragma unroll
+            for (int i = 0; i < RB; i++) {
+                double acc = 0.0;
+#pragma unroll
+                for (int u = 0; u < NQ; u++)
+                    if (lane + 64 * u < n4) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) acc = fma((double)wc[i][u][k], (double)x[u][k], acc);
+                    }
+                const double v = wave_sum_f64_dpp(acc);
+                if (lane == 0 && i0 + i < cnt) s_part[start + i0 + i] = v;
+            }
+        }
+    }
+    flow_finish_cls(wg, e_cls);
+    if (wg == 0) flow_pick_token(nwg, e_cls, t_step + 1 < n_tok ? e_cls + 1 : 0u);
+  }
+#undef VTL
+#undef LANE
+}
+
+// ------------------------------------------------------------------------------------------
 // building the streams (once per model)
 // ------------------------------------------------------------------------------------------
 // bytes a wavefront's stream holds for one layer, and before phase `kind` within a layer
@@ -2525,6 +2938,27 @@ static FlowGeom make_geom(int64_t n_rows, int64_t K, int type, int grid, bool ha
     return g;
 }
 
+// flow_f32_wave_kernel: the layers' rows go over the workgroups that run no head; a wavefront for every pair of rows and every slice
+// (at most 512 inputs; a power of two of them) of a pair of w2's.  Returns the 16-byte groups per lane of a row of dim inputs, or 0
+// where that does not fit and flow_f32_kernel runs.  Six layers and 32 000 rows of classifier, microseconds a token at
+// position 20 (300) with that kernel and with this one: dim 256: 121 (175), 91 (147); dim 512: 136 (187), 94 (149); dim 1024, built for
+// four groups: 193 (236), 194 (236).  Head sizes and counts that the kernels take leave no dim between those.
+static int f32_wave_plan(FlowArgs &a, int grid) {
+    if ((a.dim != 256 && a.dim != 512) || a.kv_dim % 2 != 0 || grid <= a.n_heads) return 0;
+    FlowGeom g[4] = {a.qkv, a.wo, a.w13, a.w2};
+    const int n_wg = grid - a.n_heads;
+    for (FlowGeom &p : g) {
+        p.rpw = (p.n_rows + n_wg - 1) / n_wg;
+        p.rpw += p.rpw & 1;
+        p.ppr = 1;
+    }
+    while ((a.hidden / 4 + g[3].ppr - 1) / g[3].ppr > 128) g[3].ppr *= 2;
+    if (g[0].rpw > 2 * FLOW_NW || g[2].rpw > 2 * FLOW_NW || (g[3].rpw / 2) * g[3].ppr > FLOW_NW) return 0;
+    a.qkv = g[0], a.wo = g[1], a.w13 = g[2], a.w2 = g[3];
+    a.cls.ppr = 1;
+    return a.dim / 256;
+}
+
 // Can the model run on this kernel?  q4_K, q5_K or q6_K layer matrices whose rows are whole pieces of 2048 inputs, padded to them by a
 // third at most, or go in pairs (dim 3072); a q4_K or q6_K classifier; or fp32 matrices throughout; and sizes that fit the kernel's LDS
 // areas.  On success fills the geometry fields of `a` for a grid of `grid`.
@@ -2561,6 +2995,7 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
             if ((a.dim + 2 * a.kv_dim) % 2 != 0) return no("odd row count");
             if (a.wo.rpw != a.w2.rpw || a.wo.rpw > FLOW_RESID_ROWS) return no("too many rows of x per workgroup");
             a.f32 = 1;
+            a.f32_quads = f32_wave_plan(a, grid);
             a.dim_pad = a.dim;
             return true;
         }
@@ -2717,7 +3152,10 @@ hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a) {
 // wait limit, and the launch would end with the error that l2h_model_set_wait_limit describes.
 // form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs
 static const void *flow_kernel_fn(int cls_type, int form) {
-    if (cls_type == L2H_TYPE_F32) return (const void *)flow_f32_kernel;
+    if (cls_type == L2H_TYPE_F32)
+        return form == 1   ? (const void *)flow_f32_wave_kernel<1>
+               : form == 2 ? (const void *)flow_f32_wave_kernel<2>
+                           : (const void *)flow_f32_kernel;
     if (form == 4) return (const void *)flow_token_kernel<L2H_TYPE_Q6_K, false, false, true>;
     if (form == 5) return (const void *)flow_token_kernel<L2H_TYPE_Q6_K, true, false, true>;
     if (form == 2)

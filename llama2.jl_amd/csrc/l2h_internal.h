@@ -173,6 +173,7 @@ struct FlowArgs {
     // a model of fp32 matrices (llama2.c files): no streams, the rows are read where the tensors lie.
     // f_w: wq, wk, wv, wo, w1, w3, w2 of layer 0 and the classifier; f_stride: floats from a layer's tensor to the next layer's
     int f32;
+    int f32_quads;  // with f32: 1 or 2: the kernel for small models, so many 16-byte groups of a row per lane
     const float *f_w[8];
     int64_t f_stride[8];
 #ifdef L2H_TIMELINE
@@ -204,7 +205,11 @@ hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a);
 // form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs (flow_form)
 hipError_t k_flow_launch(hipStream_t s, unsigned int gen0, int n_tok, int cls_type, int grid, int form);
 bool k_flow_fits(int cls_type, int grid, int n_cu, int form);
-inline int flow_form(const FlowArgs &a) { return (a.mixed ? (a.qkv.ppr == 0 ? 2 : 1) : 0) + (!a.f32 && a.cls.ppr == 0 ? 4 : 0); }
+// (of an fp32 model: f32_quads)
+inline int flow_form(const FlowArgs &a) {
+    if (a.f32) return a.f32_quads;
+    return (a.mixed ? (a.qkv.ppr == 0 ? 2 : 1) : 0) + (a.cls.ppr == 0 ? 4 : 0);
+}
 
 // ---- launchers (kernel files) ----------------------------------------------------------------
 // Each returns hipGetLastError() of its launch.

@@ -37,3 +37,43 @@ def test_keys_of_the_steps_before_in_one_launch(pkg, n_new):
     _same(fast, slow, synth.seeded_prompt(70, 2, 300), n_new)
     fast.close()
     slow.close()
+
+
+SHAPES = [
+    # (dim, hidden, layers, heads, kv heads, vocabulary, neox): hidden sizes around the slices of 512 that w2's rows are cut into and
+    # the longest, row counts that leave workgroups, wavefronts and the last pair of the classifier without rows, every head size
+    (256, 4, 2, 8, 8, 1, False),
+    (256, 512, 2, 4, 2, 255, True),
+    (256, 516, 1, 8, 1, 4097, False),
+    (512, 1376, 2, 8, 8, 32000, False),
+    (512, 2052, 2, 16, 4, 3, True),
+    (512, 4096, 2, 4, 4, 1000, False),
+]
+
+
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_rows_slices_and_heads(pkg, shape):
+    from llama2_jl_amd import synth
+    fast, slow = _pair(pkg, 40 + shape, *SHAPES[shape])
+    for rep, n_new in enumerate((19, 290)):  # the second run crosses into the attention of long caches
+        _same(fast, slow, synth.seeded_prompt(70 + rep, 2 + 5 * rep, SHAPES[shape][5]), n_new)
+    fast.close()
+    slow.close()
+
+
+def test_gives_up_and_recovers(pkg):
+    """a wait bound of zero, set from the host: every wavefront leaves at the next barrier, and the model decodes as before afterwards"""
+    from llama2_jl_amd import synth
+    cfg = pkg.ModelConfig(dim=512, hidden_dim=1376, n_layers=2, n_heads=8, n_kv_heads=8, vocab_size=500, seq_len=64, rope_freq_base=10000.0)
+    dev = synth.synthetic_model(cfg, synth.PLAN_F32, seed=5).device(path=3)
+    prompt = synth.seeded_prompt(11, 6, 500)
+    want = np.asarray(dev.generate_greedy(prompt, 12)).tolist()
+    dev.set_wait_limit(0)
+    dev.reset()
+    with pytest.raises(pkg.L2HError):
+        dev.generate_greedy(prompt, 12)
+    dev.set_wait_limit(1 << 20)
+    for _ in range(2):
+        dev.reset()
+        assert np.asarray(dev.generate_greedy(prompt, 12)).tolist() == want
+    dev.close()
