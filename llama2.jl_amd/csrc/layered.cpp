@@ -53,6 +53,7 @@ struct Layered {
     // one token
     float *x_alt = nullptr, *in = nullptr, *mix = nullptr, *ssq = nullptr, *gate = nullptr, *hid = nullptr, *z = nullptr,
           *se = nullptr, *y = nullptr, *part = nullptr, *x0 = nullptr, *lq = nullptr, *qa = nullptr;
+    unsigned *count = nullptr;  // k_step_latent's, zero between launches
     // prompt pass, for `cap` positions
     int cap = 0;
     int32_t *tok = nullptr, *choice = nullptr, *slot_row = nullptr, *slot_of = nullptr, *n_tiles = nullptr, *want = nullptr;
@@ -600,6 +601,7 @@ int layered_finalize(l2h_model *m) {
     const l2h_layered_config &c = l->c;
     int n_in = 1, hv = 1, hid = 1, ne = 1, ssq = 1;
     int64_t part = 1, lq = 0, qa = 0;
+    int heads = 0;
     auto missing = [&](uint64_t have, int role, int layer) -> int {
         if (have >> role & 1) return L2H_OK;
         return set_err(ctx, L2H_ESTATE, "missing tensor \"%s\"%s%s", layered_role_name(role), layer >= 0 ? " of layer " : "",
@@ -646,7 +648,8 @@ int layered_finalize(l2h_model *m) {
         if (d.mixer == L2H_MIX_ATTENTION) part = std::max(part, window_part_floats(window_shape(l, L)));
         if (d.mixer == L2H_MIX_LATENT) {
             const LatentShape w = latent_shape(l, L);
-            part = std::max(part, latent_part_floats(w, w.H));
+            part = std::max(part, std::max(latent_part_floats(w, w.H), (int64_t)w.H * L_STEP_SPLITS * (L_STEP_RANK + 4)));
+            heads = std::max(heads, w.H);
             lq = std::max(lq, (int64_t)w.H * w.hq());
             qa = std::max(qa, (int64_t)w.H * w.ld());
         }
@@ -666,6 +669,7 @@ int layered_finalize(l2h_model *m) {
     if (l->adds_again()) DA(l->x0, c.width, true);
     if (lq) {
         DA(l->lq, lq, true);
+        DA(l->count, 2 * heads, true);
         DA(l->qa, qa, true);
     }
     DA(m->x, c.width, true);
@@ -782,6 +786,120 @@ static hipError_t step_latent(l2h_model *m, const LayerDev &L, const LayerRun &r
     return k_latent_value(s, w, l->part, L.ukv.w, L.ukv.ld, l->in, 0, 1, l->mix, cols, cols, 1, m->ctl);
 }
 
+// The products of a parallel layer with latent attention and a gated feed-forward as its launches of a decode step take them
+struct LatentLayerStep {
+    RowsArgs uq, up, down, o;
+    int up_pro, down_pro;
+};
+static void set_router(RowsArgs &a, const LayerDev &L, const float *z) {
+    a.z = z;
+    a.z_bias = L.router_bias;
+    a.n_experts = L.d.n_experts;
+    a.top = L.d.top;
+    a.route = L.d.route;
+}
+static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int cu, LatentLayerStep &a) {
+    const l2h_layer &d = L.d;
+    if (!d.parallel || d.mixer != L2H_MIX_LATENT || d.ff == L2H_FF_NONE || !d.ff_gated) return false;
+    const LatentShape w = latent_shape(l, L);
+    const bool dense = d.ff == L2H_FF_DENSE;
+    a.uq = rows_of(L.uq, l->in, l->lq);
+    a.uq.normw = L.qnorm;
+    a.uq.eps = w.eps;
+    a.up = rows_of(L.up, x, l->hid);
+    a.up.normw = L.norm1;
+    a.up.eps = l->c.norm_eps;
+    a.up.act = d.ff_act;
+    a.down = rows_of(dense && L.joined ? L.o : L.down, l->hid, x);
+    a.o = rows_of(L.o, l->mix, x);
+    if (L.joined) {  // a row of the output matrix goes on as one of the feed-forward's
+        a.o.K = a.o.ld = L.o_cols;
+        a.o.stride = a.down.stride = L.o.ld;
+        a.down.w += L.o_cols;
+        a.down.K = d.ff_dim;
+        a.down.ld = L.o.ld - L.o_cols;
+    }
+    a.o.resid = a.down.resid = x;
+    a.o.mult = a.down.mult = l->c.residual_mult;
+    a.up_pro = dense ? RP_NORM : RP_UP;
+    a.down_pro = dense ? RP_PLAIN : RP_DOWN;
+    if (!dense) {
+        set_router(a.up, L, l->in + L.off_z);
+        set_router(a.down, L, l->in + L.off_z);
+        a.up.rows_each = L.up_rows();
+        a.up.n_rows = (int64_t)d.top * L.up_rows();
+        a.down.rows_each = a.down.n_rows = l->c.width;
+    }
+    return k_step_fits(w, L.ukv.ld, a.uq, a.up, a.up_pro, a.down, a.down_pro, cu);
+}
+
+// Mixer and feed-forward of a layer, a launch each; `in` reads the norm of the stream x into the mixer's projected row
+static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x) {
+    Layered *l = m->lay;
+    hipStream_t s = m->ctx->stream;
+    const int cu = m->ctx->prop.multiProcessorCount;
+    const l2h_layered_config &c = l->c;
+    const l2h_layer &d = L.d;
+    const bool early = d.parallel;  // the feed-forward reads the mixer's input
+    hipError_t e;
+    if (L.stacked()) {
+        in.glu_from = L.n_plain;
+        in.act = d.ff_act;
+        in.out2 = L.joined ? l->mix + L.o_cols : l->hid;
+        CK(k_rows(s, in, RP_NORM, RE_STORE_GLU, cu));
+    } else {
+        CK(k_rows(s, in, RP_NORM, RE_STORE, cu));
+    }
+    RowsArgs o = rows_of(L.o, l->mix, x);
+    o.resid = x;
+    o.mult = c.residual_mult;
+    int o_pro = RP_PLAIN;
+    if (d.mixer == L2H_MIX_ATTENTION) {
+        CK(k_window_step(s, window_shape(l, L), L.freq, l->in, run.kc, run.vc, m->ctl, l->part, l->mix));
+    } else if (d.mixer == L2H_MIX_LATENT) {
+        CK(step_latent(m, L, run, cu));
+    } else {
+        const DeltaWeights w = {L.conv, L.rate, L.bias, L.a2.w, L.g2.w, L.a2.ld, L.g2.ld};
+        CK(k_delta_step(s, delta_shape(l, L), w, l->in, run.ring, run.state, m->ctl, l->mix, l->ssq, l->gate));
+        o.normw = L.mixnorm;
+        o.eps = c.norm_eps;
+        o.ssq = l->ssq;
+        o.gate = l->gate;
+        o.hv = d.vdim;
+        o.n_split = delta_splits(d.vdim);
+        o_pro = RP_HEADNORM;
+    }
+    if (!early || d.ff == L2H_FF_NONE || (L.stacked() && L.joined)) CK(k_rows(s, o, o_pro, RE_RESID, cu));
+    if (d.ff != L2H_FF_NONE && !(L.stacked() && L.joined)) {
+        RowsArgs up = rows_of(L.up, x, l->hid), down = rows_of(L.down, l->hid, x);
+        up.normw = early ? L.norm1 : L.norm2;
+        up.eps = c.norm_eps;
+        up.act = d.ff_act;
+        down.resid = x;
+        down.mult = c.residual_mult;
+        if (d.ff == L2H_FF_DENSE) {
+            if (L.joined) up.out = l->mix + L.o_cols;
+            if (!L.stacked()) CK(k_rows(s, up, RP_NORM, d.ff_gated ? RE_GLU : RE_ACT, cu));
+            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
+            if (!L.joined) CK(k_rows(s, down, RP_PLAIN, RE_RESID, cu));
+        } else {
+            RowsArgs r = rows_of(L.router, x, l->z);
+            r.normw = up.normw;
+            r.eps = c.norm_eps;
+            if (!early) CK(k_rows(s, r, RP_NORM, RE_STORE, cu));
+            for (RowsArgs *a : {&up, &down}) set_router(*a, L, early ? l->in + L.off_z : l->z);
+            up.rows_each = L.up_rows();
+            up.n_rows = (int64_t)d.top * L.up_rows();
+            down.rows_each = c.width;
+            down.n_rows = c.width;
+            CK(k_rows(s, up, RP_UP, d.ff_gated ? RE_GLU : RE_UP, cu));
+            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
+            CK(k_rows(s, down, RP_DOWN, RE_RESID, cu));
+        }
+    }
+    return hipSuccess;
+}
+
 hipError_t layered_enqueue_token(l2h_model *m) {
     Layered *l = m->lay;
     hipStream_t s = m->ctx->stream;
@@ -792,7 +910,6 @@ hipError_t layered_enqueue_token(l2h_model *m) {
     CK(k_embed(s, m->glob[L2H_TOK_EMB], m->ctl, m->prompt_dev, st.x, m->rope_cs, 0, 1.0f, c.embed_scale, l->x0));
     for (const LayerRun &run : l->run) {
         LayerDev &L = l->layer[(size_t)run.layer];
-        const l2h_layer &d = L.d;
         if (run.pass >= 0) {
             if (st.yw) CK(k_norm_rows(s, st.x, c.width, 1, nullptr, c.norm_eps, l->y, st.yw, c.residual_mult, nullptr, nullptr, 0, 1));
             st.yw = nullptr;
@@ -800,67 +917,18 @@ hipError_t layered_enqueue_token(l2h_model *m) {
         }
         RowsArgs in = st.normed(L.in, L.norm1, l->in);
         float *x = st.x;
-        const bool early = d.parallel;  // the feed-forward reads the mixer's input
-        if (L.stacked()) {
-            in.glu_from = L.n_plain;
-            in.act = d.ff_act;
-            in.out2 = L.joined ? l->mix + L.o_cols : l->hid;
-            CK(k_rows(s, in, RP_NORM, RE_STORE_GLU, cu));
-        } else {
+        LatentLayerStep shared;
+        if (shares_launches(l, L, x, cu, shared)) {
+            in.n_rows = L.n_plain;
             CK(k_rows(s, in, RP_NORM, RE_STORE, cu));
-        }
-        RowsArgs o = rows_of(L.o, l->mix, x);
-        o.resid = x;
-        o.mult = c.residual_mult;
-        int o_pro = RP_PLAIN;
-        if (d.mixer == L2H_MIX_ATTENTION) {
-            CK(k_window_step(s, window_shape(l, L), L.freq, l->in, run.kc, run.vc, m->ctl, l->part, l->mix));
-        } else if (d.mixer == L2H_MIX_LATENT) {
-            CK(step_latent(m, L, run, cu));
+            const LatentShape w = latent_shape(l, L);
+            const LatentStep a = {w, L.freq, l->lq, l->qa, L.ukv.w, L.ukv.ld, l->in, L.kvnorm, run.kc, l->part, l->count, l->mix,
+                                  L.joined ? L.o_cols : w.H * w.V, m->ctl, L_STEP_SPLITS};
+            CK(k_step_pair(s, a, shared.uq, shared.up, shared.up_pro, cu));
+            CK(k_step_latent(s, a, shared.down, shared.down_pro, cu));
+            CK(k_rows(s, shared.o, RP_PLAIN, RE_RESID, cu));
         } else {
-            const DeltaWeights w = {L.conv, L.rate, L.bias, L.a2.w, L.g2.w, L.a2.ld, L.g2.ld};
-            CK(k_delta_step(s, delta_shape(l, L), w, l->in, run.ring, run.state, m->ctl, l->mix, l->ssq, l->gate));
-            o.normw = L.mixnorm;
-            o.eps = c.norm_eps;
-            o.ssq = l->ssq;
-            o.gate = l->gate;
-            o.hv = d.vdim;
-            o.n_split = delta_splits(d.vdim);
-            o_pro = RP_HEADNORM;
-        }
-        if (!early || d.ff == L2H_FF_NONE || (L.stacked() && L.joined)) CK(k_rows(s, o, o_pro, RE_RESID, cu));
-        if (d.ff != L2H_FF_NONE && !(L.stacked() && L.joined)) {
-            RowsArgs up = rows_of(L.up, x, l->hid), down = rows_of(L.down, l->hid, x);
-            up.normw = early ? L.norm1 : L.norm2;
-            up.eps = c.norm_eps;
-            up.act = d.ff_act;
-            down.resid = x;
-            down.mult = c.residual_mult;
-            if (d.ff == L2H_FF_DENSE) {
-                if (L.joined) up.out = l->mix + L.o_cols;
-                if (!L.stacked()) CK(k_rows(s, up, RP_NORM, d.ff_gated ? RE_GLU : RE_ACT, cu));
-                if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
-                if (!L.joined) CK(k_rows(s, down, RP_PLAIN, RE_RESID, cu));
-            } else {
-                RowsArgs r = rows_of(L.router, x, l->z);
-                r.normw = up.normw;
-                r.eps = c.norm_eps;
-                if (!early) CK(k_rows(s, r, RP_NORM, RE_STORE, cu));
-                for (RowsArgs *a : {&up, &down}) {
-                    a->z = early ? l->in + L.off_z : l->z;
-                    a->z_bias = L.router_bias;
-                    a->n_experts = d.n_experts;
-                    a->top = d.top;
-                    a->route = d.route;
-                }
-                up.rows_each = L.up_rows();
-                up.n_rows = (int64_t)d.top * L.up_rows();
-                down.rows_each = c.width;
-                down.n_rows = c.width;
-                CK(k_rows(s, up, RP_UP, d.ff_gated ? RE_GLU : RE_UP, cu));
-                if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
-                CK(k_rows(s, down, RP_DOWN, RE_RESID, cu));
-            }
+            CK(separate_launches(m, L, run, in, x));
         }
         if (c.side_dim) {
             RowsArgs g = rows_of(L.side_gate, x, l->se);

@@ -32,11 +32,13 @@ enum { LROUTE_SIGMOID_IN = 0, LROUTE_SOFTMAX_OUT = 1 };
 enum { RP_PLAIN = 0, RP_NORM = 1, RP_UP = 2, RP_DOWN = 3, RP_HEADNORM = 4 };
 // epilogues: RE_STORE v; RE_RESID resid + mult * v; RE_ACT act(v); RE_UP act(score * v) or score * act(v) with the expert's score;
 // RE_EMBED act(v) * the token's row of an embedding table; RE_GLU rows 2 i and 2 i + 1 give out[i] = act(v) * v', with the
-// expert's score behind RP_UP; RE_STORE_GLU stores rows below glu_from and treats the others so, into out2
-enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6 };
+// expert's score behind RP_UP; RE_STORE_GLU stores rows below glu_from and treats the others so, into out2; RE_STORE_AGENT v, past the
+// caches of the storing workgroup
+enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6, RE_STORE_AGENT = 7 };
 struct RowsArgs {
     const uint16_t *w = nullptr;
     int ld = 0, K = 0;
+    int64_t stride = 0;  // from row to row (0: ld); not for RP_UP, RP_DOWN
     int64_t n_rows = 0;
     const float *x = nullptr;
     float *out = nullptr;
@@ -266,3 +268,35 @@ hipError_t k_latent_value(hipStream_t s, const LatentShape &w, const float *part
 // for the matrix-core attention: rotated queries as bf16 [M][H hs], cached latents n rows from pos0 as activations [n][lda]
 hipError_t k_latent_heads(hipStream_t s, const LatentShape &w, const float *freq, const float *q, uint16_t *qb, int hs, int M, int pos0);
 hipError_t k_latent_rows(hipStream_t s, const LatentShape &w, const float *cache, int pos0, int n, uint16_t *outa, int64_t lda);
+
+// ---- a decode step's latent attention and feed-forward in shared launches (k_step.hip) ----------------------------
+#define L_STEP_RANK 512   // elements of the cached latent at most (a lane's eight; a thread of 512 each)
+#define L_STEP_ROT 64
+#define L_STEP_HEAD 128   // elements of a head's key, without its rotated part, and of its value
+#define L_STEP_RUN 32     // keys of a workgroup, at least ...
+#define L_STEP_SPLITS 16  // ... and workgroups of a head, at most
+// Longest sequence, of fewer than eight heads half of it (a workgroup's keys go one batch of 32 after the other).  Microseconds a token in
+// launches of their own and shared, at positions 100, 1000, 2000, 4000: 16 heads, width 2048, 4 layers (6 runs): 320 330 345 364, 254 305 324
+// 355; 32 heads, width 4096, 2 layers: 246 252 257 266, 207 236 239 255; 9 heads, width 1152, 2 layers: 96 97 101 105, 80 96 99 105; 4 heads,
+// width 512, 3 layers: 106 106 112 112, 90 103 110 122.
+#define L_STEP_KEYS 4096
+struct LatentStep {
+    LatentShape w;
+    const float *freq, *q;  // q[H hq]: the projected queries
+    float *qa;              // [H][ld]: the queries on the cached rows
+    const uint16_t *ukv;
+    int ldu;
+    const float *in, *kvnorm;  // the token's projected row
+    float *cache, *part;       // part: H splits (L_STEP_RANK + 4) floats
+    unsigned *count;           // [2 H], zero between launches
+    float *out;
+    int64_t cols;  // out up to which is zeroed behind the heads
+    const DecodeCtl *ctl;
+    int splits;
+};
+bool k_step_fits(const LatentShape &w, int ldu, const RowsArgs &uq, const RowsArgs &up, int up_pro, const RowsArgs &down, int down_pro,
+                 int n_cu);
+// uq: RP_NORM, the rows of the projected queries, then a.qa and the token's cache row from them; up: pro (RP_NORM or RP_UP), RE_GLU
+hipError_t k_step_pair(hipStream_t s, const LatentStep &a, const RowsArgs &uq, const RowsArgs &up, int pro, int n_cu);
+// down: pro (RP_PLAIN or RP_DOWN), RE_RESID
+hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &down, int pro, int n_cu);

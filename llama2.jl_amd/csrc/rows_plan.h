@@ -5,6 +5,7 @@
 
 #include "layered.h"
 
+#define ROWS_THREADS 512
 #define ROWS_WAVES 8
 #define ROWS_MAX_PAIRS 4096  // row pairs of a workgroup at most: 32 KB of results
 #define ROWS_LDS (152 * 1024)
@@ -34,4 +35,23 @@ inline int64_t rows_grid(const RowsArgs &a, int pro, int n_cu, int u) {
     const int64_t room = std::max<int64_t>(2, std::min<int64_t>(ROWS_MAX_PAIRS, (ROWS_LDS / 4 - vectors) / 2));
     const int64_t n = std::max<int64_t>(1, std::min(std::min(rows_most(a, pro, n_cu), pairs), (rows_steps(a, pro, u) + ROWS_WAVES - 1) / ROWS_WAVES));
     return std::max(n, (pairs + room - 2) / (room - 1));
+}
+
+// how a matrix's rows are dealt out: workgroup b has `pairs` row pairs, and one more for b < more, one after another
+struct RowsPlan {
+    int plane;              // half of a staged vector's floats
+    int pairs, more;
+    int per_vec, per_pair;  // steps of a row pair per staged vector, in all
+    int64_t stride;         // from row to row
+};
+inline RowsPlan rows_plan(const RowsArgs &a, int pro, int u, int64_t grid) {
+    const int64_t pairs = (a.n_rows + 1) / 2;
+    RowsPlan pl;
+    pl.plane = a.ld / 2;
+    pl.pairs = (int)(pairs / grid);
+    pl.more = (int)(pairs % grid);
+    pl.per_vec = (a.ld + 512 * u - 1) / (512 * u);
+    pl.per_pair = rows_vectors(a, pro) * pl.per_vec;
+    pl.stride = a.stride ? a.stride : a.ld;
+    return pl;
 }
