@@ -109,7 +109,9 @@ int l2h_model_set_kv_type(l2h_model *m, int kv_type);
  *     hidden_dim a multiple of 2048 up to 14336; head size 32, 64, 96 or 128; fp32 or fp16 cache;
  *   - models whose matrices are all fp32: dim and hidden_dim multiples of 4, at most 4096; head size 32, 64
  *     or 128; fp32 cache;
- *   in both cases n_heads <= 256, a head size that is a multiple of 256 / n_heads, and a cache length that fits
+ *   - by the automatic choice only, small models of q4_K, q5_K or q6_K matrices (w1 and w3 of a layer of one type): dim 512 or 1024,
+ *     hidden_dim a multiple of 256 up to 3840, at most 64 layers, head size 32 or 64, fp32 cache, up to 65 536 (dim 512) or 131 072 rows of classifier;
+ *   in all cases n_heads <= 256, a head size that is a multiple of 256 / n_heads, and a cache length that fits
  *   the attention's LDS area (with head size 128: about 2 400 positions times 256 / n_heads, e.g. 19 000
  *   for 32 heads).
  * 2 and 3 are an error at finalize if the model does not fit; l2h_model_path_reason then tells why.  All paths compute the same
@@ -118,7 +120,7 @@ int l2h_model_set_kv_type(l2h_model *m, int kv_type);
 int l2h_model_set_path(l2h_model *m, int path);
 int l2h_model_path(l2h_model *m);
 /* Steps of the token loop (src/inference.jl:349-386) that one kernel launch of l2h_generate_greedy runs: 1, or up to 8
- * on path 3 for a model in which no two heads share a cache row (n_kv_heads == n_heads; the cache then lies in uncached
+ * on path 3 for a model in which no two heads share a cache row (n_kv_heads == n_heads) and for small k-quant models (the cache then lies in uncached
  * memory).  No counterpart in the reference. */
 int l2h_model_steps_per_launch(l2h_model *m);
 /* After finalize with the automatic choice: why the streaming kernel (path 3) was not taken, e.g. "layer matrices

@@ -673,15 +673,9 @@ static int mega_setup(l2h_model *m) {
     return L2H_OK;
 }
 
-// Builds the per-wavefront weight streams and the tagged activation buffers of the streaming kernel.
-static int flow_setup(l2h_model *m) {
-    l2h_ctx *ctx = m->ctx;
+// what the streaming kernel's plans look at: sizes, and per layer the types of wq, wk, wv, wo, w1, w2, w3
+static FlowArgs flow_shape(l2h_model *m, std::vector<int> &types) {
     const l2h_config &c = m->c;
-    m->flow = false;
-    m->flow_why.clear();
-    // automatic choice: this kernel where the model fits it (it is the fastest path), else one kernel per phase
-    if (m->path_request != 3 && m->path_request != 0) return L2H_OK;
-    const bool required = m->path_request == 3;
     FlowArgs a{};
     a.dim = c.dim;
     a.hidden = c.hidden_dim;
@@ -695,16 +689,33 @@ static int flow_setup(l2h_model *m) {
     a.neox = c.rope_is_neox;
     a.theta_scale = m->theta_scale;
     a.kv16 = m->kv16;
-    std::vector<int> types;
+    types.clear();
     for (int l = 0; l < c.n_layers; l++)
         for (int r : {L2H_WQ, L2H_WK, L2H_WV, L2H_WO, L2H_W1, L2H_W2, L2H_W3}) types.push_back(m->L(l, r).type);
-    const int grid = ctx->prop.multiProcessorCount;
+    return a;
+}
+
+// Builds the per-wavefront weight streams and the tagged activation buffers of the streaming kernel.
+static int flow_setup(l2h_model *m) {
+    l2h_ctx *ctx = m->ctx;
+    const l2h_config &c = m->c;
+    m->flow = false;
+    m->flow_why.clear();
+    // automatic choice: this kernel where the model fits it (it is the fastest path), else one kernel per phase
+    if (m->path_request != 3 && m->path_request != 0) return L2H_OK;
+    const bool required = m->path_request == 3;
+    std::vector<int> types;
+    FlowArgs a = flow_shape(m, types);
+    int grid = ctx->prop.multiProcessorCount;
     const int cls_type = m->glob[L2H_OUTPUT].type;
     std::string why;
     // A q6_K classifier with dim 1536 .. 2048 has its rows in pairs.  8 layers of 2048 x 8192 (16 heads on 4) with one: a
     // 37-token prompt and 16 tokens 6.47 ms on path 1, 4.50 ms here.  The automatic choice takes it.  Asked for by number path 3 refuses
     // such a model as it did before its rows could go in pairs (the reason says so): what callers were refused stays refused.
-    if (!k_flow_plan(a, types.data(), (int)types.size(), cls_type, grid, &why, !required)) {
+    const int small_grid = k_flow_plan_small(a, types.data(), (int)types.size(), cls_type, grid, !required);
+    if (small_grid) {
+        grid = small_grid;
+    } else if (!k_flow_plan(a, types.data(), (int)types.size(), cls_type, grid, &why, !required)) {
         m->flow_why = why;
         return required ? set_err(ctx, L2H_EINVAL, "streaming kernel not available: %s", why.c_str()) : L2H_OK;
     }
@@ -726,6 +737,30 @@ static int flow_setup(l2h_model *m) {
         a.f_w[7] = m->glob[L2H_OUTPUT].f32;
         a.f_stride[7] = 0;
     }
+    if (a.kq) {
+        std::vector<FlowKqTensor> t;
+        auto put = [&](const DevTensor &d) {
+            FlowKqTensor k{};
+            const bool six = d.type == L2H_TYPE_Q6_K;
+            k.type = d.type;
+            k.qs = d.qs;
+            k.hdr = six ? (const unsigned char *)d.sc6 : (const unsigned char *)d.hdr;
+            k.qh = d.type == L2H_TYPE_Q4_K ? d.qs : d.qh;
+            k.qh_block = six ? 64 : (d.type == L2H_TYPE_Q5_K ? 32 : 0);
+            k.d = six ? (const unsigned char *)d.d6 : (const unsigned char *)d.hdr;
+            k.d_block = six ? 2 : 0;
+            t.push_back(k);
+        };
+        for (int l = 0; l < c.n_layers; l++)
+            for (int r : {L2H_WQ, L2H_WK, L2H_WV, L2H_WO, L2H_W1, L2H_W3, L2H_W2}) put(m->L(l, r));
+        put(m->glob[L2H_OUTPUT]);
+        FlowKqTensor *dev = nullptr;
+        int rc;
+        if ((rc = dalloc(m, &dev, (int64_t)t.size(), false))) return rc;
+        HIPCHK(ctx, hipMemcpy(dev, t.data(), t.size() * sizeof(t[0]), hipMemcpyHostToDevice));
+        a.kq_tensors = dev;
+    }
+    const bool streams = !a.f32 && !a.kq;
     std::vector<int64_t> off;
     int64_t total = 0;
     FlowTypedTables tt;
@@ -759,12 +794,12 @@ static int flow_setup(l2h_model *m) {
         if ((rc = dalloc(m, &wt, (int64_t)tt.wave_types.size(), false))) return rc;
         HIPCHK(ctx, hipMemcpy(wt, tt.wave_types.data(), tt.wave_types.size() * 4, hipMemcpyHostToDevice));
         a.wave_types = wt;
-    } else if (!a.f32) {
+    } else if (streams) {
         total = k_flow_offsets(a, cls_type, grid, off);
     }
     unsigned char *stream = nullptr;
     int64_t *off_dev = nullptr;
-    if (!a.f32 && !required) {  // (a model that was not asked to run here does not fail for want of memory for a second copy)
+    if (streams && !required) {  // (a model that was not asked to run here does not fail for want of memory for a second copy)
         size_t free_b = 0, total_b = 0;
         HIPCHK(ctx, hipMemGetInfo(&free_b, &total_b));
         if (free_b < (size_t)total + ((size_t)64 << 20)) {
@@ -772,12 +807,12 @@ static int flow_setup(l2h_model *m) {
             return L2H_OK;
         }
     }
-    if (!a.f32) {
+    if (streams) {
         if ((rc = dalloc(m, &stream, total, false))) return rc;
         if ((rc = dalloc(m, &off_dev, (int64_t)off.size(), false))) return rc;
         HIPCHK(ctx, hipMemcpy(off_dev, off.data(), off.size() * 8, hipMemcpyHostToDevice));
     }
-    for (int l = 0; l < c.n_layers && !a.f32; l++) {
+    for (int l = 0; l < c.n_layers && streams; l++) {
         const DevTensor qkv[3] = {m->L(l, L2H_WQ), m->L(l, L2H_WK), m->L(l, L2H_WV)};
         const DevTensor wo[1] = {m->L(l, L2H_WO)};
         const DevTensor w13[2] = {m->L(l, L2H_W1), m->L(l, L2H_W3)};
@@ -787,7 +822,7 @@ static int flow_setup(l2h_model *m) {
         HIPCHK(ctx, k_flow_repack(ctx->stream, a, stream, off_dev, 2, l, w13, 2, grid, cls_type, typed));
         HIPCHK(ctx, k_flow_repack(ctx->stream, a, stream, off_dev, 3, l, w2, 1, grid, cls_type, typed));
     }
-    if (!a.f32) HIPCHK(ctx, k_flow_repack(ctx->stream, a, stream, off_dev, 4, 0, &m->glob[L2H_OUTPUT], 1, grid, cls_type, typed));
+    if (streams) HIPCHK(ctx, k_flow_repack(ctx->stream, a, stream, off_dev, 4, 0, &m->glob[L2H_OUTPUT], 1, grid, cls_type, typed));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     a.stream = stream;
     a.wave_off = off_dev;
@@ -997,10 +1032,15 @@ extern "C" int l2h_model_finalize(l2h_model *m) {
     // (and stale lines in the reader's), which only the end of a kernel puts right.  Where no two heads share a cache
     // row (n_kv_heads == n_heads: nothing is read twice, the L2 holds nothing worth keeping) the cache therefore lives
     // in uncached memory, and such a model decodes several steps per launch; with shared rows it stays in ordinary memory
-    // and every step is a launch.
+    // and every step is a launch.  A small k-quant model (kq) has it uncached also with shared rows: what lies between two launches is a seventh of
+    // its step (40 tokens of 4 layers of 512 x 1024 with 8 heads on 2: 3.34 ms against 3.65; 32 at 3900 positions 3.79 against 4.04).
     {
         const char *env = getenv("L2H_KV_UNCACHED");
-        m->kv_uncached = env ? atoi(env) != 0 : (c.n_heads == c.n_kv_heads && (m->path_request == 0 || m->path_request == 3));
+        std::vector<int> types;
+        FlowArgs shape = flow_shape(m, types);
+        if (m->path_request == 0)
+            k_flow_plan_small(shape, types.data(), (int)types.size(), m->glob[L2H_OUTPUT].type, ctx->prop.multiProcessorCount, true);
+        m->kv_uncached = env ? atoi(env) != 0 : (shape.kq || (c.n_heads == c.n_kv_heads && (m->path_request == 0 || m->path_request == 3)));
         const int64_t n = m->cache_layer_elems * c.n_layers / (m->kv16 ? 2 : 1) + 1;
         if (m->kv_uncached) {
             for (float **p : {&m->kc, &m->vc}) {

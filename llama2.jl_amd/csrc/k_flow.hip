@@ -2417,7 +2417,12 @@ __device__ __forceinline__ void flowv_norm_weights(f32x4v (&nw)[NQ], const float
 }
 // The workgroup's first wavefronts wait for the 4 n4 bare words at src, 64 groups of four each, and put them into LDS (the last ones, which
 // have no rows: 6.2 ms, in the terms above; polls that go out while the rows are still coming).  False if a wait gave up; every wavefront calls this.
-__device__ __forceinline__ bool flowv_stage(const unsigned *src, int n4, int wave, int lane) {
+// `at`: the 16-byte group of s_act where the input lies.  Consecutive inputs lie in different places: a wavefront may still be reading one
+// when others have the first words of the next (nothing but the workgroup's barriers orders them).
+#define FLOWV_X 1664   // x, behind the partial sums and row values
+#define FLOWV_XO 1792  // the attention's output
+#define FLOWV_HB 0     // the SwiGLU output
+__device__ __forceinline__ bool flowv_stage(int at, const unsigned *src, int n4, int wave, int lane) {
     const int i = 64 * wave + lane;
     if (64 * wave < n4) {
         u32x4v w = {FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY};
@@ -2434,7 +2439,7 @@ __device__ __forceinline__ bool flowv_stage(const unsigned *src, int n4, int wav
                 break;
             }
         }
-        if (i < n4) ((u32x4v *)s_act)[i] = w;
+        if (i < n4) ((u32x4v *)s_act)[at + i] = w;
     }
     flow_barrier_lds();
     if (s_flag) {
@@ -2520,22 +2525,28 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
     constexpr int dim = 256 * NQ, n4 = dim >> 2;
     const int hs = a.hs, n_layers = a.n_layers;
     // attention of head h runs on workgroup h * stride + h % stride (spread over the XCDs), which has no rows of the layers; rw: this
-    // workgroup's number among those that have (past the last row on the heads')
+    // workgroup's number among those that have
     const int att_stride = nwg / a.n_heads;
     const int att_h = uni(wg / att_stride), att_at = att_h % att_stride;
     const bool is_att = uni((int)(att_h < a.n_heads && wg % att_stride == att_at)) != 0;
-    const int rw = is_att ? nwg : wg - min(att_h, a.n_heads) - (att_h < a.n_heads && wg % att_stride > att_at ? 1 : 0);
-    // this wavefront's tasks: a pair of rows of q|k|v, of wo and of w1|w3; one slice of a pair of w2's
-    const int np_qkv = flow_n_local(a.qkv, rw) >> 1, np_wo = flow_n_local(a.wo, rw) >> 1, np_w13 = flow_n_local(a.w13, rw) >> 1;
+    const int rw = is_att ? 0 : wg - min(att_h, a.n_heads) - (att_h < a.n_heads && wg % att_stride > att_at ? 1 : 0);
+    // This wavefront's tasks: a pair of rows of q|k|v, of wo and of w1|w3; one slice of a pair of w2's.  The pairs go evenly over the workgroups
+    // without a head, and every one has some in every phase (f32_wave_plan): a phase's end then means that nobody still waits for
+    // an input of two phases ago, whose words are marked empty again.
+    const int n_wg = nwg - a.n_heads;
+    auto first = [&](const FlowGeom &g, int w) { return uni((int)((int64_t)w * (g.n_rows >> 1) / n_wg)); };
+    const int p_qkv = first(a.qkv, rw), p_wo = first(a.wo, rw), p_w13 = first(a.w13, rw);
+    const int np_qkv = is_att ? 0 : first(a.qkv, rw + 1) - p_qkv, np_wo = is_att ? 0 : first(a.wo, rw + 1) - p_wo,
+              np_w13 = is_att ? 0 : first(a.w13, rw + 1) - p_w13;
     // (w2's on the last wavefronts: their rows are requested while the first ones work on w1|w3, whose SwiGLU, a function, waits on entry
     // for what its wavefront has under way)
     const int sl_log = __builtin_ctz(a.w2.ppr), task2 = FLOW_NW - 1 - wave, slice = task2 & (a.w2.ppr - 1), pair2 = task2 >> sl_log;
     const int h4 = a.hidden >> 2, per_s = (h4 + a.w2.ppr - 1) >> sl_log, s0 = slice * per_s, n4s = min(per_s, h4 - s0);
     const bool has_qkv = wave < np_qkv, has_wo = wave < np_wo, has_w13 = wave < np_w13, has_w2 = pair2 < np_wo;
-    const int row_wo = rw * a.wo.rpw + 2 * wave;  // (also the rows of x whose value this wavefront keeps, on lanes 0 and 1)
+    const int row_wo = 2 * (p_wo + wave);  // (also the rows of x whose value this wavefront keeps, on lanes 0 and 1)
     int seg, row, row1;                           // the pair of q|k|v
-    flow_row_src(0, rw * a.qkv.rpw + 2 * wave, dim, a.kv_dim, hs, a.neox, seg, row);
-    flow_row_src(0, rw * a.qkv.rpw + 2 * wave + 1, dim, a.kv_dim, hs, a.neox, seg, row1);
+    flow_row_src(0, 2 * (p_qkv + wave), dim, a.kv_dim, hs, a.neox, seg, row);
+    flow_row_src(0, 2 * (p_qkv + wave) + 1, dim, a.kv_dim, hs, a.neox, seg, row1);
     float resid = 0.0f;
     // rows of q|k|v and of w1|w3 are requested a phase ahead, as soon as that phase has its input: a request in front of a wait delays it
     F32Rows<NQ> r_next;
@@ -2582,7 +2593,7 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
         {
             LANE();
             f32x4v x[NQ];
-            if (l > 0 && !uni((int)flowv_stage(a.x_a, n4, wave, lane))) return;
+            if (l > 0 && !is_att && !uni((int)flowv_stage(FLOWV_X, a.x_a, n4, wave, lane))) return;
             VTL();
             flowv_arrived(r_next);
             flowv_arrived(nw);
@@ -2599,7 +2610,7 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
                                           dequant_elem(a.emb, tok, 4 * i + 3)};
                     }
                 } else {
-                    flowv_input(x, 0, n4, lane);
+                    flowv_input(x, FLOWV_X, n4, lane);
                 }
                 flowv_norm(x, nw, dim);
                 double v0, v1;
@@ -2630,6 +2641,7 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
                                           : flow_attention_short<32>(l, att_h, pos, e_q, e_att);
             if (!uni((int)fine)) return;
         }
+        if (is_att) continue;  // (the heads' workgroups meet the others in q, k and v)
         // ---- x += wo * xb (:281-284) ----
         {
             LANE();
@@ -2640,18 +2652,18 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
                 const float *base = a.f_w[3] + (int64_t)l * a.f_stride[3] + (int64_t)row_wo * dim;
                 flowv_rows(r, base, base + dim, n4, lane);
             }
-            if (!uni((int)flowv_stage(a.xo + (int64_t)(e_att & 1u) * dim, n4, wave, lane))) return;
+            if (!uni((int)flowv_stage(FLOWV_XO, a.xo + (int64_t)(e_att & 1u) * dim, n4, wave, lane))) return;
             VTL();
             flowv_arrived(r);
             flowv_forget(r_next);
             flowv_forget(nw);
             if (has_w13) {
-                const int64_t u = (int64_t)(rw * (a.w13.rpw >> 1) + wave);
+                const int64_t u = p_w13 + wave;
                 flowv_rows(r_next, a.f_w[4] + (int64_t)l * a.f_stride[4] + u * dim, a.f_w[5] + (int64_t)l * a.f_stride[5] + u * dim, n4, lane);
                 flowv_norm_weights(nw, a.rms_ffn + (int64_t)l * a.norm_stride, n4, lane);
             }
             if (has_wo) {
-                flowv_input(x, 0, n4, lane);
+                flowv_input(x, FLOWV_XO, n4, lane);
                 double v0, v1;
                 flowv_dot(r, x, n4, lane, v0, v1);
                 VTL();
@@ -2669,18 +2681,18 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
         {
             LANE();
             f32x4v x[NQ];
-            const int64_t u = (int64_t)(rw * (a.w13.rpw >> 1) + wave);
-            if (!uni((int)flowv_stage(a.x_b, n4, wave, lane))) return;
+            const int64_t u = p_w13 + wave;
+            if (!uni((int)flowv_stage(FLOWV_X, a.x_b, n4, wave, lane))) return;
             VTL();
             flowv_arrived(r_next);
             flowv_arrived(nw);
             flowv_forget(r_w2);
             if (has_w2) {
-                const float *base = a.f_w[6] + (int64_t)l * a.f_stride[6] + (int64_t)(rw * a.w2.rpw + 2 * pair2) * a.hidden + 4 * s0;
+                const float *base = a.f_w[6] + (int64_t)l * a.f_stride[6] + (int64_t)(2 * (p_wo + pair2)) * a.hidden + 4 * s0;
                 flowv_rows(r_w2, base, base + a.hidden, n4s, lane);
             }
             if (has_w13) {
-                flowv_input(x, 0, n4, lane);
+                flowv_input(x, FLOWV_X, n4, lane);
                 flowv_norm(x, nw, dim);
                 double v0, v1;
                 flowv_dot(r_next, x, n4, lane, v0, v1);
@@ -2697,12 +2709,12 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
         {
             LANE();
             f32x4v x[2];
-            if (!uni((int)flowv_stage(a.hbw + (int64_t)(e_w13 & 1u) * a.hidden, h4, wave, lane))) return;
+            if (!uni((int)flowv_stage(FLOWV_HB, a.hbw + (int64_t)(e_w13 & 1u) * a.hidden, h4, wave, lane))) return;
             VTL();
             flowv_arrived(r_w2);
             if (l + 1 < n_layers) request_qkv(l + 1);
             if (has_w2) {
-                flowv_input(x, s0, n4s, lane);
+                flowv_input(x, FLOWV_HB + s0, n4s, lane);
                 double v0, v1;
                 flowv_dot(r_w2, x, n4s, lane, v0, v1);
                 if (lane < 2) s_part[2 * task2 + lane] = lane ? v1 : v0;
@@ -2723,6 +2735,10 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
     }
     // ---- final rmsnorm (:309) + classifier (:312): the wavefronts that wait for x request their rows behind it, the others before ----
     const unsigned e_cls = E0 + 5u * (unsigned)n_layers + 1;
+    if (is_att) {  // (x's words are the last layer's input until its SwiGLU output is there)
+        LANE();
+        if (!uni((int)flowv_stage(FLOWV_HB, a.hbw + (int64_t)((e_cls - 2) & 1u) * a.hidden, h4, wave, lane))) return;
+    }
     {
         LANE();
         constexpr int RB = FLOWV_CLS / NQ;  // rows a batch
@@ -2741,9 +2757,9 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
         flowv_norm_weights(nw, a.rms_final, n4, lane);
         const bool waits = 64 * wave < n4;
         if (!waits && cnt > 0) fetch(0);
-        if (!uni((int)flowv_stage(a.x_a, n4, wave, lane))) return;
+        if (!uni((int)flowv_stage(FLOWV_X, a.x_a, n4, wave, lane))) return;
         if (waits && cnt > 0) fetch(0);
-        flowv_input(x, 0, n4, lane);
+        flowv_input(x, FLOWV_X, n4, lane);
         flowv_norm(x, nw, dim);
 #pragma nounroll
         for (int i0 = 0; i0 < cnt; i0 += RB) {
@@ -2766,6 +2782,440 @@ __global__ __launch_bounds__(1024) void flow_f32_wave_kernel(unsigned int gen0, 
     if (wg == 0) flow_pick_token(nwg, e_cls, t_step + 1 < n_tok ? e_cls + 1 : 0u);
   }
 #undef VTL
+#undef LANE
+}
+
+// ------------------------------------------------------------------------------------------
+// small models of k-quant matrices (dim 512 or 1024; kq_wave_plan): the same kernel shape for rows of super-blocks
+//
+// A wavefront takes 64 / (8 NB) rows of dim = 256 NB inputs, a lane 32 weights of one super-block, where the tensors lie (no streams: such a model's
+// rows stay in the L2s from one token to the next).  Input: wavefront b < NB waits for the whole vector, norms it for itself and
+// quantises block b; the attention and SwiGLU outputs, which are only quantised, are waited for a block a wavefront.  One barrier a phase.
+// The input lies in two areas in turn: a wavefront that falls behind reads one while the next phase's input is put into the other.
+// Six tokens of 4 layers of 512 x 1024, 2048 rows of classifier: 0.807 ms as 24 launches a token of 4 to 7 us each, 0.480 here (69 us a token, about 14
+// a layer); with the embedding, the classifier and the addresses kept in the loop's registers 0.570, their spills being read back from memory in
+// front of every hand-over; with a launch a step and the cache in ordinary memory 0.640 (against that 0.570).
+// ------------------------------------------------------------------------------------------
+#define FLOWQ_AREA 5120  // up to 4096 quants, their 256 sums and 16 scales
+struct KqPiece {
+    u32x4v w, hdr, qh;
+    uint32_t d;
+};
+__shared__ FlowKqTensor s_kq[7 * FLOWQ_LAYERS + 1];
+
+__device__ __forceinline__ void flowv_forget(KqPiece &r) { asm volatile("" : "=v"(r.w), "=v"(r.hdr), "=v"(r.qh), "=v"(r.d)); }
+__device__ __forceinline__ void flowv_arrived(KqPiece &r) { asm volatile("" : "+v"(r.w), "+v"(r.hdr), "+v"(r.qh), "+v"(r.d)); }
+__device__ __forceinline__ FlowKqTensor flowq_tensor(int i) {
+    FlowKqTensor t = s_kq[i];
+    t.qs = uni(t.qs), t.hdr = uni(t.hdr), t.qh = uni(t.qh), t.d = uni(t.d);
+    t.type = uni(t.type), t.qh_block = uni(t.qh_block), t.d_block = uni(t.d_block);
+    return t;
+}
+// What lane c8 of super-block blk's eight takes.  Loads that a type does not have read one of its first blocks instead: no branch.
+__device__ __forceinline__ void flowq_request(KqPiece &r, const FlowKqTensor &t, unsigned blk, int c8) {
+    // (bytes into one matrix: 32 bits, kq_wave_plan)
+    const unsigned six = t.type == L2H_TYPE_Q6_K ? 32 * (c8 >> 2) : 0;
+    r.w = *(const AS1 u32x4v *)(t.qs + (blk * 128 + 16 * c8));
+    r.hdr = *(const AS1 u32x4v *)(t.hdr + blk * 16);
+    r.qh = *(const AS1 u32x4v *)(t.qh + (blk * t.qh_block + six + 16 * (c8 & 1)));
+    r.d = *(const AS1 uint16_t *)(t.d + blk * t.d_block);
+}
+// the lane's 32 weights against block b of the input in `area`
+__device__ __forceinline__ double flowq_term(const KqPiece &r, int type, int area, int b, int c8) {
+    const unsigned char *x = (const unsigned char *)s_act + area * FLOWQ_AREA;
+    const int16_t *bs = (const int16_t *)(x + 4096) + 16 * b;
+    const float yd = ((const float *)(x + 4608))[b];
+    const int pair = c8 >> 1, h = c8 & 1;
+    const uint4 w = make_uint4(r.w.x, r.w.y, r.w.z, r.w.w), hdr = make_uint4(r.hdr.x, r.hdr.y, r.hdr.z, r.hdr.w),
+                qh = make_uint4(r.qh.x, r.qh.y, r.qh.z, r.qh.w);
+    if (type == L2H_TYPE_Q6_K) {
+        const int w32 = pair & 1, n = c8 >> 2;
+        const uint4 *xp = (const uint4 *)(x + 256 * b + 128 * n + 32 * w32 + 16 * h);
+        const int16_t *bp = bs + 8 * n + 2 * w32 + h;
+        return flow_q6_term(w, qh, flow_q6_scales(hdr, c8), r.d, w32, xp[0], xp[4], bp[0], bp[4], yd);
+    }
+    const uint4 *xp = (const uint4 *)(x + 256 * b + 64 * pair + 16 * h);
+    const int16_t *bp = bs + 4 * pair + h;
+    int sc_a, sc_b, m_a, m_b;
+    kq_scales_pair(hdr, pair, sc_a, sc_b, m_a, m_b);
+    if (type == L2H_TYPE_Q5_K) return flow_q5_term(w, qh, hdr.x, sc_a, sc_b, m_a, m_b, 2 * pair, xp[0], xp[2], bp[0], bp[2], yd);
+    return flow_q4_term(w, hdr.x, sc_a, sc_b, m_a, m_b, xp[0], xp[2], bp[0], bp[2], yd);
+}
+__device__ __forceinline__ void flowq_put(int area, int b, const float (&v)[4], int lane) {
+    unsigned char *x = (unsigned char *)s_act + area * FLOWQ_AREA;
+    uint32_t packed;
+    int bsum;
+    float d;
+    q8k_quantize_wave(v, packed, bsum, d);
+    ((uint32_t *)x)[64 * b + lane] = packed;
+    if ((lane & 3) == 0) ((int16_t *)(x + 4096))[16 * b + (lane >> 2)] = (int16_t)bsum;
+    if (lane == 0) ((float *)(x + 4608))[b] = d;
+}
+__device__ __forceinline__ bool flowq_gave_up(unsigned &spins) {
+    if (++spins > c_flow.spin_limit || ((spins & 63) == 0 && __hip_atomic_load(c_flow.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+        s_flag = 1;
+        return true;
+    }
+    return false;
+}
+#define FLOWQ_FULL(V_) (V_.x != FLOW_EMPTY && V_.y != FLOW_EMPTY && V_.z != FLOW_EMPTY && V_.w != FLOW_EMPTY)
+// every wavefront of the workgroup passes here behind the staging of an input; false if a wait gave up
+__device__ __forceinline__ bool flowq_met() {
+    flow_barrier_lds();
+    if (s_flag) {
+        if (threadIdx.x == 0) __hip_atomic_store(c_flow.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    return true;
+}
+// a vector of 256 nb bare words that is only quantised
+__device__ __forceinline__ bool flowq_stage(int area, const unsigned *src, int nb, int wave, int lane) {
+    if (wave < nb) {
+        u32x4v w = {FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY};
+        const unsigned *p = src + 256 * wave + 4 * lane;
+        unsigned spins = 0;
+        for (;;) {
+            if (!FLOWQ_FULL(w)) POLL_BARE1(w, p);
+            const bool full = FLOWQ_FULL(w);
+            if (__ballot(!full) == 0ull || flowq_gave_up(spins)) break;
+        }
+        const float v[4] = {__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
+        flowq_put(area, wave, v, lane);
+    }
+    return flowq_met();
+}
+// rmsnorm! (reference src/inference.jl:102-110) of the dim-long vector in x, block `wave` of it quantised; nw: the norm weights of that block
+template <int NB>
+__device__ __forceinline__ void flowq_norm_put(int area, const f32x4v (&x)[NB], const f32x4v nw, int wave, int lane) {
+    double acc = 0.0;
+    f32x4v own = x[0];
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc = fma((double)x[u][k], (double)x[u][k], acc);
+        if (u == wave) own = x[u];
+    }
+    float ss = (float)wave_sum_f64_dpp(acc);
+    ss /= (float)(256 * NB);
+    ss += 1e-5f;
+    ss = 1.0f / sqrtf(ss);
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = nw[k] * (ss * own[k]);
+    flowq_put(area, wave, v, lane);
+}
+template <int NB>
+__device__ __forceinline__ bool flowq_stage_norm(int area, const unsigned *src, const f32x4v nw, int wave, int lane) {
+    if (wave < NB) {
+        const u32x4v none = {FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY, FLOW_EMPTY};
+        u32x4v w[NB];
+        const unsigned *p = src + 4 * lane;
+        unsigned spins = 0;
+#pragma unroll
+        for (int u = 0; u < NB; u++) w[u] = none;
+        for (;;) {
+            bool full = true;
+#pragma unroll
+            for (int u = 0; u < NB; u++) full = full && FLOWQ_FULL(w[u]);
+            if (!full) {
+                if constexpr (NB == 2)
+                    POLL_BARE2(w[0], w[1], p, p + 256);
+                else
+                    POLL_BARE4(w[0], w[1], w[2], w[3], p, p + 256, p + 512, p + 768);
+            }
+            full = true;
+#pragma unroll
+            for (int u = 0; u < NB; u++) full = full && FLOWQ_FULL(w[u]);
+            if (__ballot(!full) == 0ull || flowq_gave_up(spins)) break;
+        }
+        f32x4v x[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) x[u] = f32x4v{__uint_as_float(w[u].x), __uint_as_float(w[u].y), __uint_as_float(w[u].z), __uint_as_float(w[u].w)};
+        flowq_norm_put<NB>(area, x, nw, wave, lane);
+    }
+    return flowq_met();
+}
+// the wavefront's rows' values, from a term per lane: lane r < 8 / NB returns row r's, the others a copy of one of them
+template <int NB>
+__device__ __forceinline__ double flowq_rows(double term, int lane) {
+    const double s = row16_sum_f64_dpp(term);
+    const double g0 = readlane_f64(s, 0), g1 = readlane_f64(s, 16), g2 = readlane_f64(s, 32), g3 = readlane_f64(s, 48);
+    if constexpr (NB == 2) return (lane & 2) ? ((lane & 1) ? g3 : g2) : ((lane & 1) ? g1 : g0);
+    return (lane & 1) ? g2 + g3 : g0 + g1;
+}
+
+// Functions of their own, as flowv_swiglu: what the loops over layers do not need stays out of their registers.
+__device__ __noinline__ float flowq_emb_elem(int tok, int i) { return __uint_as_float(bare_of(dequant_elem(c_flow.emb, tok, i))); }
+template <int NB>
+__device__ __noinline__ void flowq_stage_emb(int tok) {  // (into the first area: a step's first input)
+    tok = uni(tok);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const f32x4v nw = *(const AS1 f32x4v *)(c_flow.rms_att + 256 * wave + 4 * lane);
+    f32x4v x[NB];
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[u][k] = __uint_as_float(bare_of(dequant_elem(c_flow.emb, tok, 256 * u + 4 * lane + k)));
+    flowq_norm_put<NB>(0, x, nw, wave, lane);
+}
+
+#define FLOWQ_CLS 4  // pieces of classifier rows that a lane has under way
+template <int NB>
+__device__ __noinline__ bool flowq_classify(int area) {
+    area = uni(area);
+    const FlowArgs &a = c_flow;
+    constexpr int R = 8 / NB;
+    const int wg = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_local = flow_n_local(a.cls, wg), n_p = (n_local + R - 1) / R;
+    const int i = lane / (8 * NB), b = (lane >> 3) & (NB - 1);
+    const FlowKqTensor t = flowq_tensor(7 * a.n_layers);
+    KqPiece rc[FLOWQ_CLS];
+#pragma unroll
+    for (int k = 0; k < FLOWQ_CLS; k++) flowv_forget(rc[k]);
+    auto fetch = [&](int p0) {  // pieces p0 + 16 k of the workgroup's n_p
+#pragma unroll
+        for (int k = 0; k < FLOWQ_CLS; k++)
+            flowq_request(rc[k], t, (wg * a.cls.rpw + min(R * (p0 + FLOW_NW * k) + i, n_local - 1)) * NB + b, lane & 7);
+    };
+    const bool waits = wave < NB;
+    f32x4v nw = {0.f, 0.f, 0.f, 0.f};
+    if (waits) nw = *(const AS1 f32x4v *)(a.rms_final + 256 * wave + 4 * lane);
+    if (!waits && wave < n_p) fetch(wave);
+    if (!uni((int)flowq_stage_norm<NB>(area, a.x_a, nw, wave, lane))) return false;
+    if (waits && wave < n_p) fetch(wave);
+#pragma nounroll
+    for (int p0 = wave; p0 < n_p; p0 += FLOW_NW * FLOWQ_CLS) {
+        if (p0 != wave) fetch(p0);
+#pragma unroll
+        for (int k = 0; k < FLOWQ_CLS; k++) {
+            const double v = flowq_rows<NB>(flowq_term(rc[k], t.type, area, b, lane & 7), lane);
+            const int lr = R * (p0 + FLOW_NW * k) + lane;
+            if (lane < R && lr < n_local) s_part[lr] = v;
+        }
+    }
+    return true;
+}
+
+template <int NB>
+__global__ __launch_bounds__(1024) void flow_kq_wave_kernel(unsigned int gen0, int n_tok) {
+    static_assert(NB == 2 || NB == 4, "an even number of rows to a wavefront, a row over whole groups of 16 lanes");
+    const FlowArgs &a = c_flow;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wg = blockIdx.x, nwg = gridDim.x;
+    const int pos_first = a.ctl->pos, step_first = a.ctl->step, n_prompt = a.ctl->n_prompt, tok_first = a.ctl->last_argmax;
+    if (tid == 0) s_flag = 0;
+    // (the lane number anew in every phase: what derives from it is computed there, not kept across all of them)
+#define LANE()                   \
+    int lane = threadIdx.x & 63; \
+    asm volatile("" : "+v"(lane))
+    constexpr int dim = 256 * NB, R = 8 / NB;  // rows of dim inputs to a wavefront
+    const int hs = a.hs, n_layers = a.n_layers, hidden = a.hidden;
+    {  // where the matrices lie
+        const uint32_t *from = (const uint32_t *)a.kq_tensors;
+        for (int i = tid; i < (7 * n_layers + 1) * (int)(sizeof(FlowKqTensor) / 4); i += 1024) ((uint32_t *)s_kq)[i] = from[i];
+    }
+    // attention of head h runs on workgroup h * stride + h % stride (spread over the XCDs), which has no rows of the layers; rw: this
+    // workgroup's number among those that have
+    const int att_stride = nwg / a.n_heads;
+    const int att_h = uni(wg / att_stride), att_at = att_h % att_stride;
+    const bool is_att = uni((int)(att_h < a.n_heads && wg % att_stride == att_at)) != 0;
+    const int rw = is_att ? 0 : wg - min(att_h, a.n_heads) - (att_h < a.n_heads && wg % att_stride > att_at ? 1 : 0);
+    // Pieces of R rows, a wavefront each, evenly over those workgroups: every one has rows in every phase (kq_wave_plan), so that a phase's end means
+    // that nobody still waits for an input of two phases ago.
+    const int n_wg = nwg - a.n_heads;
+    auto first = [&](const FlowGeom &g, int w) { return uni((int)((int64_t)w * (g.n_rows / R) / n_wg)); };
+    const int p_qkv = first(a.qkv, rw) + wave, p_wo = first(a.wo, rw), p_w13 = first(a.w13, rw) + wave;
+    const int n_wo = is_att ? 0 : first(a.wo, rw + 1) - p_wo;
+    const bool has_qkv = !is_att && p_qkv < first(a.qkv, rw + 1), has_wo = wave < n_wo, has_w13 = !is_att && p_w13 < first(a.w13, rw + 1);
+    // w2: slices of at most eight super-blocks, a wavefront for each slice of r2 rows, p2 places for super-blocks to a row; on the last
+    // wavefronts: their rows are requested while the first ones work on w1|w3, whose SwiGLU, a function, waits on entry for what its wavefront has under way
+    const int nb2 = hidden >> 8, ppr = a.w2.ppr, per_s = (nb2 + ppr - 1) / ppr, p2_log = per_s <= 2 ? 1 : (per_s <= 4 ? 2 : 3), r2 = 8 >> p2_log;
+    const int task2 = FLOW_NW - 1 - wave, slice = task2 % ppr, group2 = task2 / ppr;
+    const bool has_w2 = group2 * r2 < R * n_wo;
+    const int row_wo = R * (p_wo + wave);  // (also the rows of x whose value this wavefront keeps, on lanes 0 .. R - 1)
+    // q|k|v: one matrix for all of a wavefront's rows; the lane's row in the product and in the epilogue
+    int seg, row_mul, row_out;
+    {
+        const int L0 = R * p_qkv, lane = tid & 63;
+        flow_row_src(0, L0 + lane / (8 * NB), dim, a.kv_dim, hs, a.neox, seg, row_mul);
+        flow_row_src(0, L0 + (lane & (R - 1)), dim, a.kv_dim, hs, a.neox, seg, row_out);
+        seg = uni(seg);
+    }
+    float resid = 0.0f;
+    KqPiece r_next;
+    f32x4v nw = {0.f, 0.f, 0.f, 0.f};
+    // rows of q|k|v and of w1|w3 are requested a phase ahead, as soon as that phase has its input: a request in front of a wait delays it
+    auto request_qkv = [&](int l) {
+        flowv_forget(r_next);
+        LANE();
+        if (wave < NB) nw = *(const AS1 f32x4v *)(a.rms_att + (int64_t)l * a.norm_stride + 256 * wave + 4 * lane);
+        int row = row_mul;
+        asm volatile("" : "+v"(row));
+        if (has_qkv) flowq_request(r_next, flowq_tensor(7 * l + seg), row * NB + ((lane >> 3) & (NB - 1)), lane & 7);
+    };
+    __syncthreads();
+#pragma nounroll
+  for (int t_step = 0; t_step < n_tok; t_step++) {
+    const unsigned E0 = gen0 + (unsigned)t_step * (5u * (unsigned)n_layers + 2u);
+    const int pos = pos_first + t_step, step = step_first + t_step;
+    // ---- this step's RoPE angles (reference src/inference.jl:122-127) and token; one barrier covers both ----
+    if (wave == 1 && tid - 64 < (hs >> 1)) flowv_rope(pos, tid - 64);  // (the first wavefront waits for the token)
+    request_qkv(0);
+    int tok = tok_first;
+    if (t_step > 0) {
+        tok = uni(flow_next_token(E0));
+        if (tok < 0) {
+            if (tid == 0) __hip_atomic_store(a.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+    } else {
+        flow_barrier_lds();
+    }
+    if (step < n_prompt) tok = a.prompt[step];
+    if (has_wo) {
+        LANE();
+        resid = 0.0f;
+        if (lane < R) resid = flowq_emb_elem(tok, row_wo + lane);
+    }
+    int area = 0;
+#pragma nounroll
+    for (int l = 0; l < n_layers; l++) {
+        const unsigned e_x = E0 + 5u * (unsigned)l;
+        const unsigned e_q = e_x + 1, e_att = e_x + 2, e_w13 = e_x + 4;
+        // ---- rmsnorm (:244), q, k, v (:247-249), rope (:255-256), cache append (:259-260) ----
+        {
+            LANE();
+            if (is_att) {
+                // (the heads' workgroups meet the others in q, k and v)
+            } else if (l > 0) {
+                if (!uni((int)flowq_stage_norm<NB>(area, a.x_a, nw, wave, lane))) return;
+            } else {
+                if (wave < NB) flowq_stage_emb<NB>(tok);
+                if (!uni((int)flowq_met())) return;
+            }
+            flowv_arrived(r_next);
+            if (is_att && pos < FLOW_ATT_SHORT) flow_touch_cache(l, att_h, pos);
+            if (has_qkv) {
+                const int type = uni(s_kq[7 * l + seg].type);
+                const double v = flowq_rows<NB>(flowq_term(r_next, type, area, (lane >> 3) & (NB - 1), lane & 7), lane);
+                const float mine = (float)v, other = flow_pair_value(mine);
+                if (lane < R) {
+                    const int half = hs >> 1, hs_log = 31 - __builtin_clz(hs), head = row_out >> hs_log, el = row_out & (hs - 1);
+                    const int ang = a.neox ? (el & (half - 1)) : (el >> 1);
+                    const float c = s_rope[2 * ang], s = s_rope[2 * ang + 1];
+                    // complex product (re + i im)(c + i s), each of the four products rounded
+                    const float turned = (lane & 1) == 0 ? (mine * c) - (other * s) : (other * s) + (mine * c);
+                    const float out = seg == 2 ? mine : turned;
+                    tag_store((seg == 0 ? a.q : (seg == 1 ? a.kcur : a.vcur)) + row_out, out, e_q);
+                    if (seg != 0)
+                        ((seg == 1 ? a.kc : a.vc) + (int64_t)l * a.cache_layer_elems)[seg == 1 ? (((int64_t)head * (hs >> 2) + (el >> 2)) * a.seq_len + pos) * 4 + (el & 3)
+                                                                                               : ((int64_t)head * a.seq_len + pos) * hs + el] = out;
+                }
+            }
+            area ^= 1;
+        }
+        // ---- attention (:263-278) ----
+        if (is_att || pos >= FLOW_ATT_SHORT) {
+            const bool fine = pos >= FLOW_ATT_SHORT ? flow_attention_split<false>(l, pos, e_q, e_att)
+                              : hs == 64 ? flow_attention_short<64>(l, att_h, pos, e_q, e_att)
+                                         : flow_attention_short<32>(l, att_h, pos, e_q, e_att);
+            if (!uni((int)fine)) return;
+        }
+        if (is_att) continue;
+        // ---- x += wo * xb (:281-284) ----
+        {
+            LANE();
+            KqPiece r;
+            flowv_forget(r);
+            if (has_wo) flowq_request(r, flowq_tensor(7 * l + 3), (row_wo + lane / (8 * NB)) * NB + ((lane >> 3) & (NB - 1)), lane & 7);
+            if (!uni((int)flowq_stage(area, a.xo + (int64_t)(e_att & 1u) * dim, NB, wave, lane))) return;
+            flowv_arrived(r);
+            flowv_forget(r_next);
+            if (wave < NB) nw = *(const AS1 f32x4v *)(a.rms_ffn + (int64_t)l * a.norm_stride + 256 * wave + 4 * lane);
+            if (has_w13) {
+                const int i = lane / (8 * NB);  // (w1's rows and w3's alternate)
+                FlowKqTensor t = flowq_tensor(7 * l + 4);
+                const FlowKqTensor t3 = flowq_tensor(7 * l + 5);
+                if (i & 1) t.qs = t3.qs, t.hdr = t3.hdr, t.qh = t3.qh, t.d = t3.d;
+                flowq_request(r_next, t, ((R * p_w13 + i) >> 1) * NB + ((lane >> 3) & (NB - 1)), lane & 7);
+            }
+            if (has_wo) {
+                const int type = uni(s_kq[7 * l + 3].type);
+                const double v = flowq_rows<NB>(flowq_term(r, type, area, (lane >> 3) & (NB - 1), lane & 7), lane);
+                if (lane < R) {
+                    const unsigned neww = bare_of(resid + (float)v);
+                    bare_store(a.x_b + row_wo + lane, neww);
+                    resid = __uint_as_float(neww);  // (the value as the other wavefronts read it)
+                    bare_store(a.x_a + row_wo + lane, FLOW_EMPTY);  // (its readers are through: see FLOW_EMPTY)
+                }
+            }
+            area ^= 1;
+        }
+        // ---- rmsnorm (:287), w1, w3 (:291-292), SwiGLU (:295-299) ----
+        KqPiece r_w2;
+        {
+            LANE();
+            if (!uni((int)flowq_stage_norm<NB>(area, a.x_b, nw, wave, lane))) return;
+            flowv_arrived(r_next);
+            flowv_forget(r_w2);
+            if (has_w2) {  // (a place without a super-block repeats the slice's first one; not used)
+                const int b = (lane >> 3) & ((1 << p2_log) - 1), blk = slice * per_s + (b < per_s && slice * per_s + b < nb2 ? b : 0);
+                const int row = min(R * p_wo + group2 * r2 + (lane >> (3 + p2_log)), dim - 1);
+                flowq_request(r_w2, flowq_tensor(7 * l + 6), row * nb2 + blk, lane & 7);
+            }
+            if (has_w13) {
+                const int type = uni(s_kq[7 * l + 4].type);
+                const double v = flowq_rows<NB>(flowq_term(r_next, type, area, (lane >> 3) & (NB - 1), lane & 7), lane);
+                const float mine = (float)v, other = flow_pair_value(mine);
+                const float g = flowv_swiglu(mine, other);
+                if (lane < R && (lane & 1) == 0) {
+                    const int u = (R * p_w13 + lane) >> 1;
+                    bare_store(a.hbw + (int64_t)(e_w13 & 1u) * hidden + u, bare_of(g));
+                    bare_store(a.hbw + (int64_t)((e_w13 & 1u) ^ 1u) * hidden + u, FLOW_EMPTY);
+                }
+            }
+            area ^= 1;
+        }
+        // ---- x += w2 * hb (:302-305) ----
+        {
+            LANE();
+            if (!uni((int)flowq_stage(area, a.hbw + (int64_t)(e_w13 & 1u) * hidden, nb2, wave, lane))) return;
+            flowv_arrived(r_w2);
+            if (l + 1 < n_layers) request_qkv(l + 1);
+            if (has_w2) {
+                const int type = uni(s_kq[7 * l + 6].type);
+                const int b = (lane >> 3) & ((1 << p2_log) - 1), blk = slice * per_s + b;
+                const bool there = b < per_s && blk < nb2;
+                double term = flowq_term(r_w2, type, area, there ? blk : 0, lane & 7);
+                term = row16_sum_f64_dpp(there ? term : 0.0);
+                if ((lane & 15) == 0) s_part[4 * task2 + (lane >> 4)] = term;
+            }
+            flow_barrier_lds();
+            if (has_wo && lane < R) {
+                const int lr = R * wave + lane, n16 = 1 << (p2_log - 1);  // (groups of 16 lanes to a row)
+                const double *p = s_part + 4 * (lr / r2) * ppr + (lr & (r2 - 1)) * n16;
+                double v = 0.0;
+                for (int s = 0; s < ppr; s++)
+                    for (int i = 0; i < n16; i++) v += p[4 * s + i];
+                const unsigned neww = bare_of(resid + (float)v);
+                bare_store(a.x_a + row_wo + lane, neww);
+                resid = __uint_as_float(neww);
+                bare_store(a.x_b + row_wo + lane, FLOW_EMPTY);
+            }
+            area ^= 1;
+        }
+    }
+    // ---- final rmsnorm (:309) + classifier (:312): the wavefronts that wait for x request their rows behind it, the others before ----
+    const unsigned e_cls = E0 + 5u * (unsigned)n_layers + 1;
+    if (is_att) {  // (x's words are the last layer's input until its SwiGLU output is there)
+        LANE();
+        if (!uni((int)flowq_stage(area, a.hbw + (int64_t)((e_cls - 2) & 1u) * hidden, hidden >> 8, wave, lane))) return;
+        area ^= 1;
+    }
+    if (!uni((int)flowq_classify<NB>(area))) return;
+    flow_finish_cls(wg, e_cls);
+    if (wg == 0) flow_pick_token(nwg, e_cls, t_step + 1 < n_tok ? e_cls + 1 : 0u);
+  }
 #undef LANE
 }
 
@@ -2938,25 +3388,88 @@ static FlowGeom make_geom(int64_t n_rows, int64_t K, int type, int grid, bool ha
     return g;
 }
 
-// flow_f32_wave_kernel: the layers' rows go over the workgroups that run no head; a wavefront for every pair of rows and every slice
+// What the two kernels for small models ask of the heads: sizes that flow_attention_short is built for, workgroups beside the heads', and
+// that flow_attention_split fits.
+static bool small_heads_fit(const FlowArgs &a, int grid) {
+    if ((a.hs != 32 && a.hs != 64 && a.hs != 128) || grid <= a.n_heads) return false;
+    const int G = grid / a.n_heads;
+    if (a.hs % G != 0 || G > 64) return false;
+    const size_t run = (size_t)((((a.seq_len + G - 1) / G) + 63) & ~63);
+    return (size_t)a.hs * 8 + (size_t)std::max(FLOW_NW * a.hs, 1024) * 8 + run * 4 + (size_t)a.hs * 8 + 64 * 8 <= FLOW_ACT_BYTES;
+}
+
+// flow_f32_wave_kernel: the layers' rows go over the workgroups that run no head, some of every phase on each; a wavefront for every pair of rows and every slice
 // (at most 512 inputs; a power of two of them) of a pair of w2's.  Returns the 16-byte groups per lane of a row of dim inputs, or 0
 // where that does not fit and flow_f32_kernel runs.  Six layers and 32 000 rows of classifier, microseconds a token at
 // position 20 (300) with that kernel and with this one: dim 256: 121 (175), 91 (147); dim 512: 136 (187), 94 (149); dim 1024, built for
 // four groups: 193 (236), 194 (236).  Head sizes and counts that the kernels take leave no dim between those.
 static int f32_wave_plan(FlowArgs &a, int grid) {
-    if ((a.dim != 256 && a.dim != 512) || a.kv_dim % 2 != 0 || grid <= a.n_heads) return 0;
-    FlowGeom g[4] = {a.qkv, a.wo, a.w13, a.w2};
+    if ((a.dim != 256 && a.dim != 512) || a.hidden % 4 != 0 || a.hidden > 4096 || a.kv16 || !small_heads_fit(a, grid)) return 0;
     const int n_wg = grid - a.n_heads;
-    for (FlowGeom &p : g) {
-        p.rpw = (p.n_rows + n_wg - 1) / n_wg;
-        p.rpw += p.rpw & 1;
-        p.ppr = 1;
+    const int64_t n_rows[5] = {a.dim + 2 * a.kv_dim, a.dim, 2 * (int64_t)a.hidden, a.dim, a.vocab};
+    FlowGeom g[5];
+    for (int i = 0; i < 5; i++) {
+        g[i] = make_geom(n_rows[i], a.dim, L2H_TYPE_Q4_K, i < 4 ? n_wg : grid);
+        g[i].ppr = 1;
+        if (i == 4) break;
+        if (n_rows[i] % 2 != 0 || n_rows[i] / 2 < n_wg) return 0;
+        g[i].rpw = (int)((n_rows[i] / 2 + n_wg - 1) / n_wg) * 2;
     }
     while ((a.hidden / 4 + g[3].ppr - 1) / g[3].ppr > 128) g[3].ppr *= 2;
-    if (g[0].rpw > 2 * FLOW_NW || g[2].rpw > 2 * FLOW_NW || (g[3].rpw / 2) * g[3].ppr > FLOW_NW) return 0;
-    a.qkv = g[0], a.wo = g[1], a.w13 = g[2], a.w2 = g[3];
-    a.cls.ppr = 1;
+    if (g[0].rpw > 2 * FLOW_NW || g[2].rpw > 2 * FLOW_NW || (g[3].rpw / 2) * g[3].ppr > FLOW_NW || g[4].rpw > FLOW_MAX_ROWS) return 0;
+    a.qkv = g[0], a.wo = g[1], a.w13 = g[2], a.w2 = g[3], a.cls = g[4];
+    a.dim_pad = a.dim;
     return a.dim / 256;
+}
+
+// flow_kq_wave_kernel: rows of 512 or 1024 inputs, 8 / NB of them to a wavefront, over the workgroups that run no head; w2's rows in
+// slices of at most eight super-blocks.  Returns the super-blocks to a row of dim inputs, or 0 where the model does not fit.
+// Microseconds a token on path 1 and here, 32 000 rows of classifier, six layers, at position 20 (300, 1900): 512 x 1280 with 8 heads on 2: 225 (233, 246),
+// 100 (141, 144); 1024 x 2816 with 16 heads on 4: 241 (249, 264), 159 (199, 203), with 16 on 16 and q5_K_M: 234 (241, 259), 159 (206,
+// 214).  Dim 256, half a group of 16 lanes to a row, and rows of other lengths, whose places in a wavefront are no power of two, are not
+// built.  Heads of 128 stay on path 1, as l2h_model_path has told the callers of such models.
+static int kq_wave_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid) {
+    auto quant = [](int t) { return t == L2H_TYPE_Q4_K || t == L2H_TYPE_Q5_K || t == L2H_TYPE_Q6_K; };
+    if ((a.dim != 512 && a.dim != 1024) || a.hidden % 256 != 0 || a.hidden > 4096 || a.n_layers > FLOWQ_LAYERS || a.hs > 64 || a.kv16 || !quant(cls_type))
+        return 0;
+    for (int i = 0; i < n_layer_types; i++)
+        if (!quant(layer_types[i])) return 0;
+    for (int l = 0; l * 7 + 6 < n_layer_types; l++)  // (a wavefront's rows of w1 and w3 go through one piece of code)
+        if (layer_types[l * 7 + 4] != layer_types[l * 7 + 6]) return 0;
+    if (!small_heads_fit(a, grid)) return 0;
+    const int n_wg = grid - a.n_heads, R = 2048 / a.dim;
+    const int64_t n_rows[4] = {a.dim + 2 * a.kv_dim, a.dim, 2 * (int64_t)a.hidden, a.dim};
+    FlowGeom g[4];
+    for (int i = 0; i < 4; i++) {
+        const int64_t np = n_rows[i] / R;
+        if (np < n_wg) return 0;
+        g[i] = make_geom(n_rows[i], a.dim, L2H_TYPE_Q4_K, n_wg);
+        g[i].rpw = (int)((np + n_wg - 1) / n_wg) * R;
+        g[i].ppr = 1;
+    }
+    const int nb2 = a.hidden / 256, ppr = (nb2 + 7) / 8, per_s = (nb2 + ppr - 1) / ppr, r2 = 8 >> (per_s <= 2 ? 1 : (per_s <= 4 ? 2 : 3));
+    g[3].ppr = ppr;
+    FlowGeom cls = make_geom(a.vocab, a.dim, L2H_TYPE_Q4_K, grid);
+    cls.ppr = 1;
+    if (g[0].rpw > R * FLOW_NW || g[1].rpw > R * FLOW_NW || g[2].rpw > R * FLOW_NW || (g[3].rpw + r2 - 1) / r2 * ppr > FLOW_NW || cls.rpw > FLOW_MAX_ROWS)
+        return 0;
+    a.qkv = g[0], a.wo = g[1], a.w13 = g[2], a.w2 = g[3], a.cls = cls;
+    a.dim_pad = a.dim;
+    return a.dim / 256;
+}
+
+// On all compute units, or on a half or a quarter of them where a phase has too few pieces for more.
+int k_flow_plan_small(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int n_cu, bool automatic) {
+    a.mixed = a.f32 = a.f32_quads = a.kq = 0;
+    bool all_f32 = cls_type == L2H_TYPE_F32;
+    for (int i = 0; i < n_layer_types; i++) all_f32 = all_f32 && layer_types[i] == L2H_TYPE_F32;
+    if (all_f32 && !small_heads_fit(a, n_cu)) return 0;  // (refused by k_flow_plan too)
+    for (int grid = n_cu; grid >= 64 && grid >= n_cu / 4; grid /= 2) {
+        if (all_f32 && (a.f32_quads = f32_wave_plan(a, grid)) != 0) a.f32 = 1;
+        if (!all_f32 && automatic) a.kq = kq_wave_plan(a, layer_types, n_layer_types, cls_type, grid);
+        if (a.f32 || a.kq) return grid;
+    }
+    return 0;
 }
 
 // Can the model run on this kernel?  q4_K, q5_K or q6_K layer matrices whose rows are whole pieces of 2048 inputs, padded to them by a
@@ -2970,6 +3483,7 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
     };
     a.mixed = 0;
     a.f32 = 0;
+    a.kq = 0;
     {
         bool all_f32 = cls_type == L2H_TYPE_F32;
         for (int i = 0; i < n_layer_types; i++) all_f32 = all_f32 && layer_types[i] == L2H_TYPE_F32;
@@ -2995,7 +3509,7 @@ bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls
             if ((a.dim + 2 * a.kv_dim) % 2 != 0) return no("odd row count");
             if (a.wo.rpw != a.w2.rpw || a.wo.rpw > FLOW_RESID_ROWS) return no("too many rows of x per workgroup");
             a.f32 = 1;
-            a.f32_quads = f32_wave_plan(a, grid);
+            a.f32_quads = 0;
             a.dim_pad = a.dim;
             return true;
         }
@@ -3150,8 +3664,9 @@ hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a) {
 // else.  The kernel has no grid-wide barrier and every wait in it is bounded, so residency is what makes it
 // fast, not what makes it correct: workgroups that had to wait for a CU would let the others run into their
 // wait limit, and the launch would end with the error that l2h_model_set_wait_limit describes.
-// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs
+// form: see flow_form
 static const void *flow_kernel_fn(int cls_type, int form) {
+    if (form >= 16) return form == 18 ? (const void *)flow_kq_wave_kernel<2> : (const void *)flow_kq_wave_kernel<4>;
     if (cls_type == L2H_TYPE_F32)
         return form == 1   ? (const void *)flow_f32_wave_kernel<1>
                : form == 2 ? (const void *)flow_f32_wave_kernel<2>

@@ -139,6 +139,13 @@ struct FlowGeom {
                  // (a q6_K classifier of 2048 inputs: ppr 0 and K 1024, two rows to a piece of 16 super-blocks)
     int K;       // input length
 };
+// Where a matrix of a small k-quant model lies, as flow_kq_wave_kernel reads it: pointers into the DevTensor, for q6_K hdr = sc6 and
+// d = d6; what a type does not have points at bytes of another kind and a step of zero per super-block
+#define FLOWQ_LAYERS 64
+struct FlowKqTensor {
+    const unsigned char *qs, *hdr, *qh, *d;
+    int type, qh_block, d_block, pad;
+};
 struct FlowArgs {
     const unsigned char *stream;  // per-wavefront weight streams
     const int64_t *wave_off;      // [grid * 16] byte offset of each wavefront's stream
@@ -176,12 +183,18 @@ struct FlowArgs {
     int f32_quads;  // with f32: 1 or 2: the kernel for small models, so many 16-byte groups of a row per lane
     const float *f_w[8];
     int64_t f_stride[8];
+    // a small model of k-quant matrices: 2 or 4 super-blocks to a row of dim inputs (0: not one); no streams either.
+    // kq_tensors: wq, wk, wv, wo, w1, w3, w2 of every layer, then the classifier
+    int kq;
+    const FlowKqTensor *kq_tensors;
 #ifdef L2H_TIMELINE
     long long *timeline;  // profiling build only: [workgroup][64] wall-clock stamps of the first phases
 #endif
 };
 // layer_types: per layer the ggml types of wq, wk, wv, wo, w1, w2, w3 (seven numbers a layer)
 bool k_flow_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid, std::string *why, bool cls_pairs = false);
+// the same for the kernels of small models (f32_quads, kq; k-quants by the automatic choice only): workgroups of the launch, at most n_cu; 0: not such a model
+int k_flow_plan_small(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int n_cu, bool automatic);
 int64_t k_flow_offsets(const FlowArgs &a, int cls_type, int grid, std::vector<int64_t> &off);
 // Where every typed piece goes (a.mixed): per wavefront the stream's offset, the index of its first piece in the
 // per-piece tables, where its classifier pieces start, the types of its first pieces; per piece the byte offset in
@@ -202,11 +215,13 @@ hipError_t k_flow_repack(hipStream_t s, const FlowArgs &a, unsigned char *stream
                          int layer, const DevTensor *w, int nw, int grid, int cls_type, const FlowTypedDev &typed);
 hipError_t k_flow_bind(hipStream_t s, const FlowArgs &a);
 // one launch runs n_tok steps of the token loop; the epochs of the launch start at gen0 and take 5 * n_layers + 2 per step
-// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs (flow_form)
+// form: 0 q4_K pieces, 1 typed pieces, 2 typed pieces and rows that end inside a piece; + 4: the classifier's rows in pairs; 16 + kq: a small
+// k-quant model (flow_form)
 hipError_t k_flow_launch(hipStream_t s, unsigned int gen0, int n_tok, int cls_type, int grid, int form);
 bool k_flow_fits(int cls_type, int grid, int n_cu, int form);
 // (of an fp32 model: f32_quads)
 inline int flow_form(const FlowArgs &a) {
+    if (a.kq) return 16 + a.kq;
     if (a.f32) return a.f32_quads;
     return (a.mixed ? (a.qkv.ppr == 0 ? 2 : 1) : 0) + (a.cls.ppr == 0 ? 4 : 0);
 }
