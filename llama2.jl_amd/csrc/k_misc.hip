@@ -249,26 +249,61 @@ __global__ __launch_bounds__(256) void argmax_stage1_kernel(const float *x, int6
     if (threadIdx.x == 0) partial[blockIdx.x] = best;
 }
 
+// the control block goes on to the next step, whose token is the largest key's
+__device__ __forceinline__ void argmax_advance(unsigned long long best, DecodeCtl *ctl, int32_t *out_tokens, int max_out) {
+    const int idx = (int)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull));
+    ctl->last_argmax = idx;
+    if (ctl->step >= ctl->n_prompt - 1 && ctl->n_out < max_out) {
+        out_tokens[ctl->n_out] = idx;
+        ctl->n_out += 1;
+    }
+    ctl->step += 1;
+    ctl->pos += 1;
+}
+
 __global__ __launch_bounds__(256) void argmax_stage2_kernel(const unsigned long long *partial, int nparts,
                                                             DecodeCtl *ctl, int32_t *out_tokens, int max_out) {
     __shared__ unsigned long long red[4];
     unsigned long long best = 0;
     for (int i = threadIdx.x; i < nparts; i += blockDim.x) best = partial[i] > best ? partial[i] : best;
     best = block_max_u64(best, red);
-    if (threadIdx.x == 0) {
-        const int idx = (int)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull));
-        ctl->last_argmax = idx;
-        if (ctl->step >= ctl->n_prompt - 1 && ctl->n_out < max_out) {
-            out_tokens[ctl->n_out] = idx;
-            ctl->n_out += 1;
+    if (threadIdx.x == 0) argmax_advance(best, ctl, out_tokens, max_out);
+}
+
+// Both stages by one workgroup, all of a thread's elements under way at once: 32 000 logits in 5.8 us, against 4.6 + 4.1 in two
+// launches.  Bound by what one CU draws from the L2s; beyond 32 768 elements a thread's would no longer fit its registers.
+#define ARGMAX_ONE_N 32768
+__global__ __launch_bounds__(1024) void argmax_one_kernel(const float *x, int n, DecodeCtl *ctl, int32_t *out_tokens, int max_out) {
+    __shared__ unsigned long long red[16];
+    constexpr int Q = ARGMAX_ONE_N / 4096;
+    const int t = threadIdx.x;
+    float4 v[Q];
+#pragma unroll
+    for (int u = 0; u < Q; u++) v[u] = *(const float4 *)(x + max(0, min(4 * (t + 1024 * u), (n & ~3) - 4)));
+    const int tail = (n & ~3) + t;
+    unsigned long long best = tail < n ? argmax_key(x[tail], (uint32_t)tail) : 0ull;
+#pragma unroll
+    for (int u = 0; u < Q; u++) {
+        const int i = 4 * (t + 1024 * u);
+        if (i + 3 < n) {
+            const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned long long key = argmax_key(e[k], (uint32_t)(i + k));
+                best = key > best ? key : best;
+            }
         }
-        ctl->step += 1;
-        ctl->pos += 1;
     }
+    best = block_max_u64(best, red);
+    if (t == 0) argmax_advance(best, ctl, out_tokens, max_out);
 }
 
 hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, DecodeCtl *ctl, int32_t *out_tokens,
                     int max_out) {
+    if (n >= 4 && n <= ARGMAX_ONE_N && (uintptr_t)x % 16 == 0) {
+        hipLaunchKernelGGL(argmax_one_kernel, dim3(1), dim3(1024), 0, s, x, (int)n, ctl, out_tokens, max_out);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(argmax_stage1_kernel, dim3(L2H_ARGMAX_BLOCKS), dim3(256), 0, s, x, n,
                        (unsigned long long *)partial);
     hipError_t e = hipGetLastError();

@@ -834,7 +834,8 @@ static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int c
 }
 
 // Mixer and feed-forward of a layer, a launch each; `in` reads the norm of the stream x into the mixer's projected row
-static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x) {
+// (`plus`, `plus2`: what the next layer's pass of a loop adds to the stream, in the launch that completes it)
+static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x, const float *plus, const float *plus2) {
     Layered *l = m->lay;
     hipStream_t s = m->ctx->stream;
     const int cu = m->ctx->prop.multiProcessorCount;
@@ -869,6 +870,8 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
         o.n_split = delta_splits(d.vdim);
         o_pro = RP_HEADNORM;
     }
+    const bool o_last = d.ff == L2H_FF_NONE || (d.ff == L2H_FF_DENSE && L.joined);
+    if (o_last) o.plus = plus, o.plus2 = plus2;
     if (!early || d.ff == L2H_FF_NONE || (L.stacked() && L.joined)) CK(k_rows(s, o, o_pro, RE_RESID, cu));
     if (d.ff != L2H_FF_NONE && !(L.stacked() && L.joined)) {
         RowsArgs up = rows_of(L.up, x, l->hid), down = rows_of(L.down, l->hid, x);
@@ -877,6 +880,8 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
         up.act = d.ff_act;
         down.resid = x;
         down.mult = c.residual_mult;
+        down.plus = plus;
+        down.plus2 = plus2;
         if (d.ff == L2H_FF_DENSE) {
             if (L.joined) up.out = l->mix + L.o_cols;
             if (!L.stacked()) CK(k_rows(s, up, RP_NORM, d.ff_gated ? RE_GLU : RE_ACT, cu));
@@ -908,13 +913,21 @@ hipError_t layered_enqueue_token(l2h_model *m) {
     hipError_t e;
     Stream st(m);
     CK(k_embed(s, m->glob[L2H_TOK_EMB], m->ctl, m->prompt_dev, st.x, m->rope_cs, 0, 1.0f, c.embed_scale, l->x0));
-    for (const LayerRun &run : l->run) {
+    // What a pass of a loop begins with, x += [x0] + step, is added by the launch that completes the stream before it (a launch of its own: 4.5 us of
+    // a 280 us token twice) unless that is the embedding's or a pending update comes in between.
+    bool added = false;
+    for (size_t r = 0; r < l->run.size(); r++) {
+        const LayerRun &run = l->run[r];
+        const LayerRun *next = r + 1 < l->run.size() ? &l->run[r + 1] : nullptr;
         LayerDev &L = l->layer[(size_t)run.layer];
-        if (run.pass >= 0) {
+        if (run.pass >= 0 && !added) {
             if (st.yw) CK(k_norm_rows(s, st.x, c.width, 1, nullptr, c.norm_eps, l->y, st.yw, c.residual_mult, nullptr, nullptr, 0, 1));
             st.yw = nullptr;
             CK(k_stream_add(s, st.x, run.pass ? l->x0 : nullptr, l->loop_step + (int64_t)run.pass * c.width, 1, c.width));
         }
+        added = next && next->pass >= 0 && !c.side_dim;
+        const float *step = added ? l->loop_step + (int64_t)next->pass * c.width : nullptr, *again = added && next->pass ? l->x0 : nullptr;
+        const float *plus = again ? again : step, *plus2 = again ? step : nullptr;
         RowsArgs in = st.normed(L.in, L.norm1, l->in);
         float *x = st.x;
         LatentLayerStep shared;
@@ -926,9 +939,11 @@ hipError_t layered_enqueue_token(l2h_model *m) {
                                   L.joined ? L.o_cols : w.H * w.V, m->ctl, L_STEP_SPLITS};
             CK(k_step_pair(s, a, shared.uq, shared.up, shared.up_pro, cu));
             CK(k_step_latent(s, a, shared.down, shared.down_pro, cu));
+            shared.o.plus = plus;
+            shared.o.plus2 = plus2;
             CK(k_rows(s, shared.o, RP_PLAIN, RE_RESID, cu));
         } else {
-            CK(separate_launches(m, L, run, in, x));
+            CK(separate_launches(m, L, run, in, x, plus, plus2));
         }
         if (c.side_dim) {
             RowsArgs g = rows_of(L.side_gate, x, l->se);

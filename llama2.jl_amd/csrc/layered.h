@@ -47,6 +47,7 @@ struct RowsArgs {
     const float *y = nullptr, *yw = nullptr;
     float *x_out = nullptr;
     const float *resid = nullptr;
+    const float *plus = nullptr, *plus2 = nullptr;  // RE_RESID: vectors added to the sum, one after the other
     int act = 0;
     int64_t glu_from = 0;
     float *out2 = nullptr;

@@ -120,7 +120,12 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     constexpr int kstep = U * 512;
     // (of the row whose result this thread writes first)
     float before = 0.0f;
-    if (EPI == RE_RESID && row0 + t < row_end) before = a.resid[row0 + t];
+    float plus = 0.0f, plus2 = 0.0f;
+    if (EPI == RE_RESID && row0 + t < row_end) {
+        before = a.resid[row0 + t];
+        if (a.plus) plus = a.plus[row0 + t];
+        if (a.plus2) plus2 = a.plus2[row0 + t];
+    }
     if (EPI == RE_EMBED && row0 + t < row_end) before = l_bf16(a.emb[(int64_t)l_step_token(a.ctl, a.prompt) * a.emb_ld + row0 + t]);
     asm volatile("" ::: "memory");
 
@@ -336,7 +341,11 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
             continue;
         }
         float o = val;
-        if (EPI == RE_RESID) o = (i == t ? before : a.resid[r]) + a.mult * val;
+        if (EPI == RE_RESID) {
+            o = (i == t ? before : a.resid[r]) + a.mult * val;
+            if (a.plus) o += i == t ? plus : a.plus[r];
+            if (a.plus2) o += i == t ? plus2 : a.plus2[r];
+        }
         if (EPI == RE_ACT) o = l_act(a.act, val);
         if (EPI == RE_UP) o = a.route == LROUTE_SIGMOID_IN ? l_act(a.act, f * val) : f * l_act(a.act, val);
         if (EPI == RE_EMBED)

@@ -279,3 +279,16 @@ def test_error_paths(pkg, ctx, rng):
     with pytest.raises(pkg.L2HError) as ei:
         lm.device()
     assert ei.value.code == _lib.EINVAL
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4095, 4099, 31999, 32768, 32769])
+def test_argmax_at_the_edges_of_one_workgroup(ctx, rng, n):
+    """the first maximum, where a group of four or a workgroup's share ends, and an equal one behind it"""
+    import ctypes
+    from llama2_jl_amd import _lib
+    for at in sorted({0, n // 2, max(0, (n & ~3) - 1), n - 1}):
+        x = rng.standard_normal(n).astype(np.float32)
+        x[at] = x[n - 1] = 7.5
+        out = ctypes.c_int32(-1)
+        ctx.check(_lib.lib().l2h_argmax(ctx.handle, _lib.ptr(x), n, ctypes.byref(out)))
+        assert out.value == int(np.argmax(x))
