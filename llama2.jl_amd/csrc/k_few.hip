@@ -113,7 +113,8 @@ __device__ __forceinline__ void few_item(const GemmArgs &a, const uint16_t *W, i
         few_f32x4 v = *(few_f32x4 *)(s_red + 4 * (p * NQ + (q ^ (p & (NQ - 1)))));
 #pragma unroll
         for (int w = 1; w < FEW_WAVES; w++) v += *(few_f32x4 *)(s_red + 4 * ((w * TM + p) * NQ + (q ^ (p & (NQ - 1)))));
-        if (m0 + p < mcount) gemm_store4<PREC, EPI>(a, mb + m0 + p, n0 + 4 * q, v.x, v.y, v.z, v.w);
+        if (m0 + p < mcount)
+            gemm_store4<PREC, EPI>(a, mb + m0 + p, n0 + 4 * q, gemm_row<EPI>(a, mb + m0 + p), gemm_col<EPI>(a, n0 + 4 * q), v.x, v.y, v.z, v.w);
     }
 }
 

@@ -5,6 +5,8 @@
 
 typedef __bf16 l_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float l_f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t l_u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t l_u32x4 __attribute__((ext_vector_type(4)));
 
 // Placement of the 16-byte chunks of a 128-byte tile row: 16 consecutive rows' chunks of one index fall into different slots
 // of the 256-byte bank row.
@@ -61,24 +63,25 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
         else
             xrow16[i] = (const uint16_t *)a.x + row * a.ldx + 8 * c8;
     }
-    uint4 wreg[WL], xreg[XL];
+    // (vectors of the compiler's own: as uint4, a struct, the sixteen words went through scratch memory in every step)
+    l_u32x4 wreg[WL], xreg[XL];
     auto gload = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < WL; i++) {
             if (PREC) {
-                const uint2 v = *(const uint2 *)(wrow[i] + k0);
-                wreg[i] = make_uint4(v.x, v.y, 0, 0);
+                const l_u32x2 v = *(const l_u32x2 *)(wrow[i] + k0);
+                wreg[i] = l_u32x4{v.x, v.y, 0, 0};
             } else {
-                wreg[i] = *(const uint4 *)(wrow[i] + k0);
+                wreg[i] = *(const l_u32x4 *)(wrow[i] + k0);
             }
         }
 #pragma unroll
-        for (int i = 0; i < XL; i++) xreg[i] = PREC ? *(const uint4 *)(xrow32[i] + k0) : *(const uint4 *)(xrow16[i] + k0);
+        for (int i = 0; i < XL; i++) xreg[i] = PREC ? *(const l_u32x4 *)(xrow32[i] + k0) : *(const l_u32x4 *)(xrow16[i] + k0);
     };
     gload(0);
     for (int k0 = 0; k0 < a.ld; k0 += KSTEP) {
         if constexpr (PREC == 0) {
-            uint4 *s_w = (uint4 *)s_raw, *s_x = s_w + TN * 8;
+            l_u32x4 *s_w = (l_u32x4 *)s_raw, *s_x = s_w + TN * 8;
 #pragma unroll
             for (int i = 0; i < WL; i++) {
                 const int r = (t >> 3) + 32 * i;
@@ -146,6 +149,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
         }
         __syncthreads();
     }
+    auto col_of = [&](int i, int rq) { return n0 + (TN / 2) * wn + 32 * i + 8 * rq + 4 * (lane >> 5); };
+    float f[JM];
+    GemmCol col[IN][4];
+#pragma unroll
+    for (int j = 0; j < JM; j++) f[j] = gemm_row<EPI>(a, mb + min(m0 + (TM / 2) * wm + 32 * j + (lane & 31), mcount - 1));
+#pragma unroll
+    for (int i = 0; i < IN; i++)
+#pragma unroll
+        for (int rq = 0; rq < 4; rq++) col[i][rq] = gemm_col<EPI>(a, col_of(i, rq));
 #pragma unroll
     for (int j = 0; j < JM; j++) {
         const int m = m0 + (TM / 2) * wm + 32 * j + (lane & 31);
@@ -154,8 +166,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
         for (int i = 0; i < IN; i++)
 #pragma unroll
             for (int rq = 0; rq < 4; rq++)
-                gemm_store4<PREC, EPI>(a, mb + m, n0 + (TN / 2) * wn + 32 * i + 8 * rq + 4 * (lane >> 5), acc[i][j][4 * rq],
-                                       acc[i][j][4 * rq + 1], acc[i][j][4 * rq + 2], acc[i][j][4 * rq + 3]);
+                gemm_store4<PREC, EPI>(a, mb + m, col_of(i, rq), f[j], col[i][rq], acc[i][j][4 * rq], acc[i][j][4 * rq + 1], acc[i][j][4 * rq + 2],
+                                       acc[i][j][4 * rq + 3]);
     }
 }
 

@@ -3,18 +3,40 @@
 
 #include "layered_dev.h"
 
+// What an epilogue reads of row m and of columns L .. L + 3.  A lane reads all of it before its first store: the compiler cannot move such
+// a load past a store, and a wait for it there is one for the stores before it (GEMM_ROW_FIGURES).
+template <int EPI>
+__device__ __forceinline__ float gemm_row(const GemmArgs &a, int64_t m) {
+    return (EPI == GE_UP || EPI == GE_GLU) && a.row_scale ? a.row_scale[m] : 1.0f;
+}
+struct GemmCol {
+    float rate[4], bias[4];
+};
+template <int EPI>
+__device__ __forceinline__ GemmCol gemm_col(const GemmArgs &a, int64_t L) {
+    GemmCol c = {};
+    if (EPI != GE_DECAY) return c;
+    // (matrices have fewer than 2^31 rows: 32-bit division)
+    const unsigned last = (unsigned)a.n_rows - 1, h0 = min((unsigned)L, last) / (unsigned)a.hd;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const unsigned r = min((unsigned)(L + e), last);
+        c.bias[e] = a.bias[r];
+        c.rate[e] = a.rate[a.hd % 4 == 0 ? h0 : r / (unsigned)a.hd];
+    }
+    return c;
+}
+
 // results (m, L .. L + 3) of a product
 template <int PREC, int EPI>
-__device__ __forceinline__ void gemm_store4(const GemmArgs &a, int64_t m, int64_t L, float v0, float v1, float v2, float v3) {
+__device__ __forceinline__ void gemm_store4(const GemmArgs &a, int64_t m, int64_t L, float f, const GemmCol &col, float v0, float v1, float v2, float v3) {
     float v[4] = {v0, v1, v2, v3};
     if (EPI == GE_STORE || EPI == GE_RESID || EPI == GE_DECAY || EPI == GE_SIGMOID) {
         if (L >= a.n_rows) return;
         float *o = a.outf + m * a.ldo + L;
-        // (matrices have fewer than 2^31 rows: 32-bit division)
-        const unsigned h0 = EPI == GE_DECAY ? (unsigned)L / (unsigned)a.hd : 0u;
         auto value = [&](int e, float old) {
             if (EPI == GE_RESID) return fmaf(a.mult, v[e], old);
-            if (EPI == GE_DECAY) return -a.rate[a.hd % 4 == 0 ? h0 : (unsigned)(L + e) / (unsigned)a.hd] * l_softplus(v[e] + a.bias[L + e]);
+            if (EPI == GE_DECAY) return -col.rate[e] * l_softplus(v[e] + col.bias[e]);
             if (EPI == GE_SIGMOID) return l_sigmoid(v[e]);
             return v[e];
         };
@@ -34,7 +56,7 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs &a, int64_t m, int64_
         const int64_t i = L >> 1;
         if (i >= a.acols) return;
         float o[2] = {0.0f, 0.0f};
-        const float f = a.row_scale ? a.row_scale[m] : 1.0f, fi = a.scale_in ? f : 1.0f, fo = a.scale_in ? 1.0f : f;
+        const float fi = a.scale_in ? f : 1.0f, fo = a.scale_in ? 1.0f : f;
 #pragma unroll
         for (int e = 0; e < 2; e++)
             if (L + 2 * e < a.n_rows) o[e] = fo * l_act_rounded<PREC>(a.act, fi * v[2 * e]) * (fi * v[2 * e + 1]);
@@ -51,7 +73,7 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs &a, int64_t m, int64_
                 continue;
             }
             if (EPI == GE_UP)
-                v[e] = a.scale_in ? l_act_rounded<PREC>(a.act, a.row_scale[m] * v[e]) : a.row_scale[m] * l_act_rounded<PREC>(a.act, v[e]);
+                v[e] = a.scale_in ? l_act_rounded<PREC>(a.act, f * v[e]) : f * l_act_rounded<PREC>(a.act, v[e]);
             else if (EPI == GE_EMBED)
                 v[e] = l_act_rounded<PREC>(a.act, v[e]) * l_bf16(a.emb[(int64_t)a.tokens[m] * a.emb_ld + L + e]);
             else
