@@ -17,7 +17,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
     constexpr int IN = TN / 64, JM = TM / 64;          // 32 x 32 tiles per wavefront (2 x 2 wavefronts)
     constexpr int KSTEP = PREC ? 32 : 64;
     constexpr int FROW = 33;                            // floats per LDS row of the fp32 form
-    __shared__ __align__(16) unsigned char s_raw[(TN + TM) * (PREC ? FROW * 4 : 128)];
+    constexpr int OPERANDS = (TN + TM) * (PREC ? FROW * 4 : 128), RESULTS = 4 * 4 * gemm_epilogue_floats(IN, JM);
+    __shared__ __align__(16) unsigned char s_raw[OPERANDS > RESULTS ? OPERANDS : RESULTS];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wn = wave & 1, wm = wave >> 1;
     const uint16_t *W = a.w;
     int64_t mb = 0;
@@ -149,26 +150,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
         }
         __syncthreads();
     }
-    auto col_of = [&](int i, int rq) { return n0 + (TN / 2) * wn + 32 * i + 8 * rq + 4 * (lane >> 5); };
-    float f[JM];
-    GemmCol col[IN][4];
-#pragma unroll
-    for (int j = 0; j < JM; j++) f[j] = gemm_row<EPI>(a, mb + min(m0 + (TM / 2) * wm + 32 * j + (lane & 31), mcount - 1));
-#pragma unroll
-    for (int i = 0; i < IN; i++)
-#pragma unroll
-        for (int rq = 0; rq < 4; rq++) col[i][rq] = gemm_col<EPI>(a, col_of(i, rq));
-#pragma unroll
-    for (int j = 0; j < JM; j++) {
-        const int m = m0 + (TM / 2) * wm + 32 * j + (lane & 31);
-        if (m >= mcount) continue;
-#pragma unroll
-        for (int i = 0; i < IN; i++)
-#pragma unroll
-            for (int rq = 0; rq < 4; rq++)
-                gemm_store4<PREC, EPI>(a, mb + m, col_of(i, rq), f[j], col[i][rq], acc[i][j][4 * rq], acc[i][j][4 * rq + 1], acc[i][j][4 * rq + 2],
-                                       acc[i][j][4 * rq + 3]);
-    }
+    // (the last barrier of the loop is behind every read of the operands)
+    gemm_epilogue<PREC, EPI, IN, JM>(a, acc, (float *)s_raw + wave * gemm_epilogue_floats(IN, JM), mb, m0 + (TM / 2) * wm, mcount, n0 + (TN / 2) * wn, lane);
 }
 
 template <int PREC, int EPI>

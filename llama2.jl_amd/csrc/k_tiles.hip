@@ -35,20 +35,10 @@ __device__ __forceinline__ void tiles_item(const GemmArgs &a, const uint16_t *w,
             return a.gather ? (int64_t)a.gather[row] : row;
         },
         [&](f32x16(&acc)[2][JT], int wn, int wm, int lane) {
-            float f[JT];
-#pragma unroll
-            for (int j = 0; j < JT; j++) f[j] = gemm_row<EPI>(a, mb + min(m0 + 32 * JT * wm + 32 * j + (lane & 31), mcount - 1));
-#pragma unroll
-            for (int j = 0; j < JT; j++) {
-                const int m = m0 + 32 * JT * wm + 32 * j + (lane & 31);
-                if (m >= mcount) continue;
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int rq = 0; rq < 4; rq++)
-                        gemm_store4<0, EPI>(a, mb + m, n0 + 64 * wn + 32 * i + 8 * rq + 4 * (lane >> 5), f[j], GemmCol{}, acc[i][j][4 * rq],
-                                            acc[i][j][4 * rq + 1], acc[i][j][4 * rq + 2], acc[i][j][4 * rq + 3]);
-            }
+            static_assert(8 * 4 * gemm_epilogue_floats(2, JT) <= STAGES * pf_tile_stage(JT), "the results' place");
+            __syncthreads();  // (the operands have all been read)
+            float *s = (float *)s_all + (wn + 4 * wm) * gemm_epilogue_floats(2, JT);
+            gemm_epilogue<0, EPI, 2, JT>(a, acc, s, mb, m0 + 32 * JT * wm, mcount, n0 + 64 * wn, lane);
         });
 }
 
