@@ -123,8 +123,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, gemm_f32x16 (&a
         asm volatile("" ::: "memory");
 #pragma nounroll
         for (int p = lane / QL; p < 32; p += STEP) {
+            const float f = s_f[32 * j + p];
+            asm volatile("" ::: "memory");  // (the quad's read is the last one under way: a wait for it is a wait for everything)
             const float4 v = *(const float4 *)(s + p * LD + 4 * (lane & (QL - 1)));
-            if (m + 32 * j + p < mcount) gemm_store4<PREC, EPI>(a, mb + m + 32 * j + p, L, s_f[32 * j + p], col, v.x, v.y, v.z, v.w);
+            if (m + 32 * j + p < mcount) gemm_store4<PREC, EPI>(a, mb + m + 32 * j + p, L, f, col, v.x, v.y, v.z, v.w);
         }
         asm volatile("" ::: "memory");
     }
