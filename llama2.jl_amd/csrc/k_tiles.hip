@@ -76,10 +76,11 @@ __global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, u
         nt = item / n_mt;
         m0 = (int)(item % n_mt) * 64 * JT;
     }
-    // (a block of a grouped product that has at most 128 rows takes half the positions, in two stages as the others: with three of them,
-    // 144 KB for every workgroup, a prompt of 2048 positions through 4 layers with 32 experts took 2567 us against 2520)
+    // (A block of a grouped product that has at most 128 rows takes half the positions, in three stages: its steps last as long as their loads.
+    // 16 experts of about 84 rows, 2048 x 4096 and 4096 x 2048: 99 and 66 us in two stages, 84 and 58 in three; 32 of about 256, half
+    // of them with a few rows more, 392 and 211 against 378 and 202.)
     if (GROUPED && JT == 4 && mcount <= 128)
-        tiles_item<EPI, 2, 2>(a, w, nt, mb, m0, mcount, s_all);
+        tiles_item<EPI, 2, pf_tile_stages(2)>(a, w, nt, mb, m0, mcount, s_all);
     else
         tiles_item<EPI, JT, pf_tile_stages(JT)>(a, w, nt, mb, m0, mcount, s_all);
 }
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, u
 
 template <int EPI, int JT, bool GROUPED>
 static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, unsigned n_mt) {
-    constexpr int lds = !GROUPED && pf_tile_lds(2) > pf_tile_lds(JT) ? pf_tile_lds(2) : pf_tile_lds(JT);
+    constexpr int lds = pf_tile_lds(2) > pf_tile_lds(JT) ? pf_tile_lds(2) : pf_tile_lds(JT);  // (halves and small blocks among them)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
