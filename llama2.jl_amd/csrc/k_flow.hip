@@ -2366,7 +2366,7 @@ __global__ __launch_bounds__(1024) void flow_f32_kernel(unsigned int gen0, int n
 //  * a phase's rows are requested as soon as the phase before it has its input: a compute unit's loads pass its polls by, and a
 //    request of 24 KB in front of a wait makes the wait 1 to 1.5 us longer (7.3 ms against 5.8 in the run below).
 //  * the heads' workgroups have no rows: theirs would come late behind the attention and hold up the next phase (6.5 ms).
-// 48 tokens of 8 layers of 512 x 1376 and 32 000 rows of classifier: 5.90 ms; 8.46 with flow_f32_kernel, whose workgroups stage an
+// 48 tokens of 8 layers of 512 x 1376 and 32 000 rows of classifier: 5.92 ms; 8.46 with flow_f32_kernel, whose workgroups stage an
 // input between two barriers, on all wavefronts, and begin loops and epilogues with divisions and scalar loads (about 1 us of loop and 0.4 to 1.2
 // of epilogue a phase against 0.6 and 0.1 to 0.6 here).  Every wavefront waiting for the whole input itself, with no barrier at
 // all: 6.9 ms (six wavefronts of a CU that read 4 KB a poll).
@@ -3401,7 +3401,8 @@ static bool small_heads_fit(const FlowArgs &a, int grid) {
 // flow_f32_wave_kernel: the layers' rows go over the workgroups that run no head, some of every phase on each; a wavefront for every pair of rows and every slice
 // (at most 512 inputs; a power of two of them) of a pair of w2's.  Returns the 16-byte groups per lane of a row of dim inputs, or 0
 // where that does not fit and flow_f32_kernel runs.  Six layers and 32 000 rows of classifier, microseconds a token at
-// position 20 (300) with that kernel and with this one: dim 256: 121 (175), 91 (147); dim 512: 136 (187), 94 (149); dim 1024, built for
+// position 20 (300) with that kernel and with this one: dim 256: 121 (175), 84 (130, on half of the
+// compute units; on all of them, most without rows of wo, 91 (147)); dim 512: 136 (187), 95 (151); dim 1024, built for
 // four groups: 193 (236), 194 (236).  Head sizes and counts that the kernels take leave no dim between those.
 static int f32_wave_plan(FlowArgs &a, int grid) {
     if ((a.dim != 256 && a.dim != 512) || a.hidden % 4 != 0 || a.hidden > 4096 || a.kv16 || !small_heads_fit(a, grid)) return 0;
