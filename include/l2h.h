@@ -152,6 +152,12 @@ int l2h_model_set_prefill_copy(l2h_model *m, int on);
  * reference (matmul! on a matrix of activations is BLAS there too: src/matmul.jl:3-11 for dense matrices). */
 int l2h_model_set_prefill_library(l2h_model *m, int on);
 int l2h_model_prefill_library(l2h_model *m);
+/* For checks: which of this library's kernels the model's sizes and options have chosen, after finalize (-1 for another `what`).
+ *   L2H_CHOSEN_TILE_IMAGES  matrices of a layered model whose prompt products run from tile images (made by the first
+ *                           prompt pass of more than 128 positions); 0 otherwise
+ * No counterpart in the reference. */
+enum { L2H_CHOSEN_TILE_IMAGES = 0 };
+int l2h_model_chosen(l2h_model *m, int what);
 /* RunState(config) (src/inference.jl:88-100): checks every tensor is present, allocates
  * activations and the zeroed KV cache, records the per-token launch sequence. */
 int l2h_model_finalize(l2h_model *m);

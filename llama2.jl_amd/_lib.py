@@ -58,6 +58,7 @@ SIGNATURES = {
     "l2h_model_prefill_library": (_I, [_P]),
     "l2h_model_path": (_I, [_P]),
     "l2h_model_steps_per_launch": (_I, [_P]),
+    "l2h_model_chosen": (_I, [_P, _I]),
     "l2h_model_finalize": (_I, [_P]),
     "l2h_state_reset": (_I, [_P]),
     "l2h_kv_write": (_I, [_P, _I, _I, _I, _P, _P]),

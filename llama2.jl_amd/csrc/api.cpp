@@ -373,6 +373,12 @@ extern "C" const char *l2h_model_path_reason(l2h_model *m) {
 extern "C" int l2h_model_steps_per_launch(l2h_model *m) { return (m && m->finalized && m->flow) ? m->flow_steps_per_launch : 1; }
 extern "C" int l2h_model_path(l2h_model *m) { return (m && m->finalized) ? (m->flow ? 3 : (m->mega ? 2 : 1)) : 0; }
 
+extern "C" int l2h_model_chosen(l2h_model *m, int what) {
+    if (!m || !m->finalized) return -1;
+    if (what == L2H_CHOSEN_TILE_IMAGES) return m->lay ? layered_images(m) : 0;
+    return -1;
+}
+
 extern "C" int l2h_model_get_tensor(l2h_model *m, int role, int layer, void *host, int64_t host_bytes) {
     if (!m || !host) return set_err(m ? m->ctx : nullptr, L2H_EINVAL, "l2h_model_get_tensor: NULL argument");
     LLAMA_ONLY(m);

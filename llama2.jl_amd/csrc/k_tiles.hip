@@ -2,6 +2,7 @@
 // grouped form for mixtures of experts.
 #include "layered_gemm.h"
 #include "pf_tile.h"
+#include "tiles_plan.h"
 
 // One thread copies a 16-byte chunk of an image: n_mats matrices of `rows` rows, each padded to whole tiles of 256 rows.
 __global__ __launch_bounds__(256) void tile_image_kernel(const uint16_t *w, int ld, int64_t rows, int64_t n_chunks, uint16_t *dst) {
@@ -44,24 +45,25 @@ __device__ __forceinline__ void tiles_item(const GemmArgs &a, const uint16_t *w,
 
 // Items (row group of 256, block of 64 JT positions) are dealt to the 8 XCDs as contiguous runs: positions fastest in a single
 // product, so that workgroups on one weight tile share an L2; row groups fastest in a grouped one, where a block of positions
-// is used with one expert's matrix only.
-// whole (single products of JT = 4): so many items, whole rounds of the CUs, come first; the others go as two halves of 128 positions
-// each: 896 tiles of 28 672 x 4096 over 2048 positions 465 us in four rounds of 256, the last half empty, 431 as three rounds and 256 halves.
-// Only where the halves are one round, up to 128 tiles: two rounds of halves take as long as one of whole tiles.
+// is used with one expert's matrix only.  Of a single product of JT = 4 the last items may go as halves (tiles_plan).
 template <int EPI, int JT, bool GROUPED>
-__global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, unsigned n_mt, unsigned whole) {
+__global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, unsigned n_mt, TilesPlan plan) {
     extern __shared__ uint4 s_all[];
-    if (!GROUPED && JT == 4 && blockIdx.x >= whole) {
-        const unsigned b = blockIdx.x - whole, n_halves = 2 * (n_nt * n_mt - whole), per = (n_halves + 7) / 8, half = (b & 7u) * per + (b >> 3);
-        const unsigned item = whole + half / 2;
-        const int m0 = (int)(item % n_mt) * 256 + 128 * (int)(half & 1u);
-        if ((b >> 3) >= per || half >= n_halves || m0 >= a.M) return;
-        tiles_item<EPI, 2, pf_tile_stages(2)>(a, a.w, item / n_mt, 0, m0, a.M, s_all);
-        return;
+    unsigned item;
+    if (!GROUPED && JT == 4) {
+        const TilesWork work = tiles_work(plan, blockIdx.x);
+        if (!work.any) return;
+        if (work.half >= 0) {
+            const int m0 = (int)(work.item % n_mt) * 256 + 128 * work.half;
+            if (m0 < a.M) tiles_item<EPI, 2, pf_tile_stages(2)>(a, a.w, work.item / n_mt, 0, m0, a.M, s_all);
+            return;
+        }
+        item = work.item;
+    } else {
+        const unsigned n_items = GROUPED ? (unsigned)a.n_tiles[0] * n_nt : plan.n;
+        item = tiles_deal(n_items, blockIdx.x);
+        if (item >= n_items) return;
     }
-    const unsigned n_items = GROUPED ? (unsigned)a.n_tiles[0] * n_nt : JT == 4 ? whole : n_nt * n_mt;
-    const unsigned per = (n_items + 7) / 8, k = blockIdx.x >> 3, item = (blockIdx.x & 7u) * per + k;
-    if (k >= per || item >= n_items) return;
     unsigned nt;
     int64_t mb = 0;
     int m0 = 0, mcount = a.M;
@@ -100,14 +102,8 @@ static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, 
         if (e != hipSuccess) return e;
         attr_set[dev] = true;
     }
-    const unsigned most = GROUPED ? (unsigned)a.max_tiles * n_nt : n_nt * n_mt;
-    unsigned grid = 8 * ((most + 7) / 8), whole = most;
-    const unsigned rest = most % 256;
-    if (!GROUPED && JT == 4 && most > 256 && rest > 0 && rest <= 128) {
-        whole = most - rest;
-        grid = whole + 8 * ((2 * rest + 7) / 8);
-    }
-    hipLaunchKernelGGL((tiles_kernel<EPI, JT, GROUPED>), dim3(grid), dim3(512), lds, s, a, n_nt, n_mt, whole);
+    const TilesPlan plan = tiles_plan(GROUPED ? (unsigned)a.max_tiles * n_nt : n_nt * n_mt, !GROUPED && JT == 4);
+    hipLaunchKernelGGL((tiles_kernel<EPI, JT, GROUPED>), dim3(tiles_grid(plan)), dim3(512), lds, s, a, n_nt, n_mt, plan);
     return hipGetLastError();
 }
 

@@ -1006,6 +1006,12 @@ static int prompt_images(l2h_model *m) {
     return L2H_OK;
 }
 
+int layered_images(l2h_model *m) {
+    int n = 0;
+    for (const LayerDev &L : m->lay->layer) n += (L.up.image != nullptr) + (L.down.image != nullptr);
+    return n;
+}
+
 int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
     Layered *l = m->lay;
     const l2h_layered_config &c = l->c;

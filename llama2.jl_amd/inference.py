@@ -150,6 +150,12 @@ class DeviceModel:
         """True if the last prefill ran those products through hipBLASLt (l2h_model_prefill_library)."""
         return bool(_lib.lib().l2h_model_prefill_library(self.handle))
 
+    _CHOSEN = ("tile_images",)
+
+    def chosen(self, what):
+        """Which kernels the model's sizes have chosen (l2h_model_chosen), for checks."""
+        return _lib.lib().l2h_model_chosen(self.handle, self._CHOSEN.index(what))
+
     def forward(self, token, pos, want_logits=True):
         """transformer!(token, pos, ...) (src/inference.jl:222-315): returns (logits, argmax)."""
         logits = np.empty(self.config.vocab_size, np.float32) if want_logits else None

@@ -6,6 +6,7 @@
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
 #include "../../llama2.jl_amd/csrc/rows_plan.h"
+#include "../../llama2.jl_amd/csrc/tiles_plan.h"
 
 #include <stdio.h>
 
@@ -163,7 +164,43 @@ static void check_rows_plan() {
                     }
 }
 
+// every tile of a prompt's product is taken exactly once, as a whole or as both of its halves
+static void check_tiles_plan() {
+    int split = 0;
+    for (unsigned n = 1; n <= 2048; n++)
+        for (int halves = 0; halves < 2; halves++) {
+            const TilesPlan p = tiles_plan(n, halves != 0);
+            std::vector<int> taken(n, 0);  // in halves
+            const unsigned grid = tiles_grid(p);
+            for (unsigned b = 0; b < grid; b++) {
+                const TilesWork w = tiles_work(p, b);
+                if (!w.any) continue;
+                EXPECT(w.item < n && w.half >= -1 && w.half <= 1);
+                if (w.item >= n) continue;
+                EXPECT((taken[w.item] & (w.half < 0 ? 3 : 1 << w.half)) == 0);
+                taken[w.item] |= w.half < 0 ? 3 : 1 << w.half;
+            }
+            bool all = true;
+            for (unsigned i = 0; i < n; i++) all = all && taken[i] == 3;
+            if (!all) printf("%u tiles\n", n);
+            EXPECT(all);
+            if (halves) split += p.whole < n;
+        }
+    EXPECT(split == 7 * 128);
+    // a grouped product's grid is made for the most tiles there can be, and dealt out by how many there are
+    for (unsigned most = 1; most <= 300; most++)
+        for (unsigned n = 1; n <= most; n++) {
+            std::vector<int> taken(n, 0);
+            for (unsigned b = 0; b < tiles_workgroups(most); b++) {
+                const unsigned i = tiles_deal(n, b);
+                if (i < n) taken[i]++;
+            }
+            for (int t : taken) EXPECT(t == 1);
+        }
+}
+
 int main() {
+    check_tiles_plan();
     check_product_rule();
     check_rows_plan();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
