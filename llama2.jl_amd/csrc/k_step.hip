@@ -311,7 +311,7 @@ __device__ __forceinline__ void step_latent_body(const LatentStep &a, int b, Ste
         const float sum = step_sum16(v, lane);
         if ((lane & 12) == 0 && e < w.V) a.out[(int64_t)h * w.V + e] = w.gated ? sum * l_sigmoid(gate) : sum;
     }
-    if (b == 0)
+    if (h == 0)  // (of a head's workgroups only the one that joins its runs comes here)
         for (int64_t i = (int64_t)w.H * w.V + t; i < a.cols; i += ROWS_THREADS) a.out[i] = 0.0f;
 }
 

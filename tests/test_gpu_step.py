@@ -52,3 +52,29 @@ def test_borders(pkg, shape):
         got = dev.forward(int(tok[p]), p)[0]
         assert lc.error(got, want[p]) <= TOL, (shape, p)
     dev.close()
+
+
+def test_padding_behind_the_heads(pkg):
+    """A narrow layer behind which a wide one leaves its values in the same buffer, at positions where a head has several runs of keys: what the wide one
+    left from a sequence of numbers that are none must not reach the next sequence's output product."""
+    c = _case([zc.dense(70)], heads=3, dim=20, rot_dim=6, vdim=13, kv_rank=100, q_rank=36)
+    wide = _case([zc.dense(70)], heads=5, dim=20, rot_dim=6, vdim=40, kv_rank=100, q_rank=36)
+    c["layers"] += wide["layers"]
+    t = {k: np.array(v) for k, v in ref.random_tensors(c, 5).items()}
+    t["embed"][7, 3] = np.inf
+    n = 160
+    tok = lc.tokens(n, c["vocab"])
+    tok[tok == 7] = 8
+    s, want = ref.Sequence(c, t), []
+    for a in tok:
+        want.append(s.step(int(a)))
+    dev = zc.language_model(pkg, c, t, seq_len=n).device()
+    for at in (40, 70, 100, 130, 150):
+        dev.reset()
+        with np.errstate(invalid="ignore"):
+            assert not np.isfinite(dev.forward(7, 0)[0]).all()
+        dev.reset()
+        dev.prefill_logits(tok[:at], [], 0)
+        got = np.array([dev.forward(int(tok[p]), p)[0] for p in range(at, at + 4)])
+        assert lc.error(got, want[at:at + 4]) <= TOL, at
+    dev.close()
