@@ -11,7 +11,8 @@
  *     last failure on a context is l2h_last_error(ctx) (thread-unsafe, like the handles);
  *   - token ids and positions are 0-based here (Julia callers subtract 1);
  *   - host pointers passed in are borrowed for the duration of the call only;
- *   - handles are opaque and owned by the library; one host thread per context;
+ *   - handles are opaque and owned by the library; one host thread per context; threads with contexts of their own may
+ *     call at the same time (on launch paths 2 and 3 decode calls on one device then run one after the other);
  *   - weights are uploaded once by l2h_model_set_tensor and stay resident in HBM in the
  *     library's own layout; the KV cache and all activations live in HBM.
  */

@@ -182,8 +182,40 @@ extern "C" int l2h_device_info(l2h_ctx *ctx, char *name, int name_cap, int32_t *
 // ------------------------------------------------------------------------------------------
 // model
 // ------------------------------------------------------------------------------------------
-static l2h_model *g_bound_model = nullptr;  // whose phase arguments the persistent kernel's constant memory holds
-static l2h_model *g_flow_bound = nullptr;   // whose arguments the streaming kernel's constant memory holds
+// Launch paths 2 and 3: a kernel's arguments lie in its device's constant memory, and its workgroups wait for each other, so that two launches at once,
+// each with a part of its workgroups resident, would wait until one gives up.  From the first launch of a call to the end of its last the device is
+// therefore that call's alone; calls of other contexts (one host thread each) take turns.  The launches of path 1 and of prompt passes end by
+// themselves and take none.
+struct DeviceTurns {
+    std::mutex lock;
+    // under the lock: whose phase arguments the persistent kernel's constant memory holds, whose arguments the streaming kernel's
+    l2h_model *mega_bound = nullptr, *flow_bound = nullptr;
+    void forget(const l2h_model *m) {
+        std::lock_guard<std::mutex> hold(lock);
+        if (mega_bound == m) mega_bound = nullptr;
+        if (flow_bound == m) flow_bound = nullptr;
+    }
+};
+static DeviceTurns &device_turns(const l2h_model *m) {
+    static DeviceTurns turns[64];  // (devices that share an entry take turns too)
+    return turns[m->ctx->device & 63];
+}
+class DeviceTurn {
+  public:
+    explicit DeviceTurn(const l2h_model *m) : stream(m->ctx->stream) {
+        if (m->flow || m->mega) hold = std::unique_lock<std::mutex>(device_turns(m).lock);
+    }
+    ~DeviceTurn() {
+        if (hold.owns_lock()) (void)hipStreamSynchronize(stream);  // (a call that failed half-way)
+    }
+    void drained() {
+        if (hold.owns_lock()) hold.unlock();
+    }
+
+  private:
+    hipStream_t stream;
+    std::unique_lock<std::mutex> hold;
+};
 
 static int q8_alloc(l2h_ctx *ctx, int64_t n, Q8Dev *q, std::vector<void *> *track) {
     void *p = nullptr;
@@ -246,9 +278,8 @@ static void model_free_state(l2h_model *m) {
 
 extern "C" void l2h_model_destroy(l2h_model *m) {
     if (!m) return;
-    if (g_bound_model == m) g_bound_model = nullptr;
-    if (g_flow_bound == m) g_flow_bound = nullptr;
     (void)hipStreamSynchronize(m->ctx->stream);
+    device_turns(m).forget(m);
     model_free_state(m);
     for (auto &t : m->glob) dev_tensor_free(&t);
     for (auto &t : m->layer) dev_tensor_free(&t);
@@ -327,7 +358,7 @@ extern "C" int l2h_model_set_wait_limit(l2h_model *m, unsigned int spins) {
     LLAMA_ONLY(m);
     if (!m->flow) return set_err(m->ctx, L2H_ESTATE, "the wait limit applies to launch path 3 after finalize");
     m->flow_args.spin_limit = spins;
-    if (g_flow_bound == m) g_flow_bound = nullptr;  // the kernel's copy of the arguments is refreshed at the next launch
+    device_turns(m).forget(m);  // the kernel's copy of the arguments is refreshed at the next launch
     return L2H_OK;
 }
 
@@ -892,11 +923,14 @@ static int flow_setup(l2h_model *m) {
 
 // The streaming kernel runs up to this many steps of the token loop per launch (the next step's token passes from
 // workgroup 0 to the others inside the kernel): what lies between two launches, about 10 us, is paid once per that many tokens.
+// (The caller holds the device's turn.)
 static hipError_t flow_launch_tokens(l2h_model *m, int n_tok) {
-    if (g_flow_bound != m) {
+    l2h_model *&bound = device_turns(m).flow_bound;
+    if (bound != m) {
         hipError_t eb = k_flow_bind(m->ctx->stream, m->flow_args);
+        bound = nullptr;
         if (eb != hipSuccess) return eb;
-        g_flow_bound = m;
+        bound = m;
     }
     hipError_t e = k_flow_launch(m->ctx->stream, m->flow_gen, n_tok, m->flow_cls_type, m->flow_grid, flow_form(m->flow_args));
     if (e == hipSuccess) m->flow_gen += (unsigned)n_tok * (5u * (unsigned)m->c.n_layers + 2u);
@@ -905,10 +939,12 @@ static hipError_t flow_launch_tokens(l2h_model *m, int n_tok) {
 }
 
 static hipError_t mega_launch_token(l2h_model *m) {
-    if (g_bound_model != m) {
+    l2h_model *&bound = device_turns(m).mega_bound;
+    if (bound != m) {
         hipError_t e = k_mega_bind(m->ctx->stream, m->mega_ph);
+        bound = nullptr;
         if (e != hipSuccess) return e;
-        g_bound_model = m;
+        bound = m;
     }
     MegaArgs g = mega_args(m);
     hipError_t e = k_mega_launch(m->ctx->stream, g, m->mega_types[0], m->mega_types[1], m->mega_types[2],
@@ -1115,7 +1151,7 @@ static int mega_check(l2h_model *m) {
                 m->flow = false;
                 m->flow_why = "a wait of the streaming kernel ran into its limit (are its workgroups resident at once?); "
                               "the model now runs one kernel per phase";
-                if (g_flow_bound == m) g_flow_bound = nullptr;
+                device_turns(m).forget(m);
                 return set_err(m->ctx, L2H_EHIP, "streaming decode kernel: a wait for activations timed out; the model "
                                                  "runs on launch path 1 from now on");
             }
@@ -1208,6 +1244,7 @@ static int generate_impl(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     HIPCHK(ctx, hipMemcpyAsync(m->ctl, &h, sizeof h, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     if (m->lay && total > 0) layered_advance(m, pos0 + total);
+    DeviceTurn turn(m);
     if (decode_ms) {
         hipEvent_t e0 = nullptr, e1 = nullptr;
         HIPCHK(ctx, hipEventCreate(&e0));
@@ -1232,6 +1269,7 @@ static int generate_impl(l2h_model *m, const int32_t *prompt, int n_prompt, int 
         HIPCHK(ctx, hipMemcpyAsync(last_logits, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost,
                                    ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    turn.drained();
     return mega_check(m);
 }
 
