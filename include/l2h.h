@@ -156,8 +156,9 @@ int l2h_model_prefill_library(l2h_model *m);
 /* For checks: which of this library's kernels the model's sizes and options have chosen, after finalize (-1 for another `what`).
  *   L2H_CHOSEN_TILE_IMAGES  matrices of a layered model whose prompt products run from tile images (made by the first
  *                           prompt pass of more than 128 positions); 0 otherwise
+ *   L2H_CHOSEN_UNCACHED_CACHE  1 if the KV cache lies in uncached memory (several steps of the token loop per launch), else 0
  * No counterpart in the reference. */
-enum { L2H_CHOSEN_TILE_IMAGES = 0 };
+enum { L2H_CHOSEN_TILE_IMAGES = 0, L2H_CHOSEN_UNCACHED_CACHE = 1 };
 int l2h_model_chosen(l2h_model *m, int what);
 /* RunState(config) (src/inference.jl:88-100): checks every tensor is present, allocates
  * activations and the zeroed KV cache, records the per-token launch sequence. */

@@ -407,6 +407,7 @@ extern "C" int l2h_model_path(l2h_model *m) { return (m && m->finalized) ? (m->f
 extern "C" int l2h_model_chosen(l2h_model *m, int what) {
     if (!m || !m->finalized) return -1;
     if (what == L2H_CHOSEN_TILE_IMAGES) return m->lay ? layered_images(m) : 0;
+    if (what == L2H_CHOSEN_UNCACHED_CACHE) return m->kv_uncached ? 1 : 0;
     return -1;
 }
 
@@ -732,6 +733,8 @@ static FlowArgs flow_shape(l2h_model *m, std::vector<int> &types) {
     return a;
 }
 
+static int64_t cache_floats(const l2h_model *m) { return m->cache_layer_elems * m->c.n_layers / (m->kv16 ? 2 : 1) + 1; }  // (of keys, or of values; an fp16 cache takes half the floats)
+
 // Builds the per-wavefront weight streams and the tagged activation buffers of the streaming kernel.
 static int flow_setup(l2h_model *m) {
     l2h_ctx *ctx = m->ctx;
@@ -839,7 +842,8 @@ static int flow_setup(l2h_model *m) {
     if (streams && !required) {  // (a model that was not asked to run here does not fail for want of memory for a second copy)
         size_t free_b = 0, total_b = 0;
         HIPCHK(ctx, hipMemGetInfo(&free_b, &total_b));
-        if (free_b < (size_t)total + ((size_t)64 << 20)) {
+        // (with the cache, which comes later)
+        if (free_b < (size_t)total + 2 * 4 * (size_t)cache_floats(m) + ((size_t)64 << 20)) {
             m->flow_why = "not enough device memory for its weight streams";
             return L2H_OK;
         }
@@ -892,8 +896,6 @@ static int flow_setup(l2h_model *m) {
     TA(a.abort_flag, 1);
     TA(a.tokw, 8 * 16);  // (eight copies, a 128-byte line each: FLOW_TOK_COPIES in k_flow.hip)
 #undef TA
-    a.kc = m->kc;
-    a.vc = m->vc;
     a.logits = m->logits;
     a.rms_att = m->L(0, L2H_RMS_ATT).f32;
     a.rms_ffn = m->L(0, L2H_RMS_FFN).f32;
@@ -910,9 +912,6 @@ static int flow_setup(l2h_model *m) {
     if ((rc = dalloc(m, &m->timeline, (int64_t)grid * 64 + 1024, true))) return rc;
     a.timeline = m->timeline;
 #endif
-    // several steps per launch where the cache is coherent between the steps (L2H_FLOW_STEPS: 1..64, for measurements)
-    m->flow_steps_per_launch = m->kv_uncached ? 8 : 1;
-    if (const char *e = getenv("L2H_FLOW_STEPS")) m->flow_steps_per_launch = std::min(64, std::max(1, atoi(e)));
     m->flow_args = a;
     m->flow_grid = grid;
     m->flow_cls_type = cls_type;
@@ -1022,6 +1021,64 @@ static int loop_buffers(l2h_model *m) {
     return L2H_OK;
 }
 
+// The cache, once the launch path is known.
+// A launch of the streaming kernel that runs several steps of the token loop reads, in a later step, cache rows that
+// another XCD's workgroups appended in an earlier one: rows in ordinary memory would still sit in the writer's L2
+// (and stale lines in the reader's), which only the end of a kernel puts right.  Where no two heads share a cache
+// row (n_kv_heads == n_heads: nothing is read twice, the L2 holds nothing worth keeping) the cache of a model on that kernel therefore lives
+// in uncached memory, and such a model decodes several steps per launch; with shared rows it stays in ordinary memory
+// and every step is a launch.  A small k-quant model (kq) has it uncached also with shared rows: what lies between two launches is a seventh of
+// its step (a token of 4 layers of 512 x 1024 with 8 heads on 2 at position 20 / 1900 / 30 000: 69 / 99 / 156 us against 77 / 106 / 164 us; its prompt of 2048
+// positions 501 us against 493, shorter prompts and scores the same).
+static int cache_setup(l2h_model *m) {
+    l2h_ctx *ctx = m->ctx;
+    const l2h_config &c = m->c;
+    const char *env = getenv("L2H_KV_UNCACHED");
+    m->kv_uncached = env ? atoi(env) != 0 : m->flow && (m->flow_args.kq || c.n_heads == c.n_kv_heads);
+    const int64_t n = cache_floats(m);
+    for (float **p : {&m->kc, &m->vc}) {
+        if (m->kv_uncached) {
+            void *v = nullptr;
+            HIPCHK(ctx, uncached_alloc(ctx->device, (size_t)n * 4, &v));
+            m->uc_allocs.push_back(v);
+            HIPCHK(ctx, hipMemset(v, 0, (size_t)n * 4));
+            *p = (float *)v;
+        } else {
+            const int rc = dalloc(m, p, n, true);
+            if (rc) return rc;
+        }
+    }
+    HIPCHK(ctx, hipDeviceSynchronize());
+    m->flow_args.kc = m->kc;
+    m->flow_args.vc = m->vc;
+    // several steps per launch where the cache is coherent between the steps (L2H_FLOW_STEPS: 1..64, for measurements)
+    m->flow_steps_per_launch = m->kv_uncached ? 8 : 1;
+    if (const char *e = getenv("L2H_FLOW_STEPS")) m->flow_steps_per_launch = std::min(64, std::max(1, atoi(e)));
+    return L2H_OK;
+}
+
+// A model that leaves the streaming kernel for path 1 takes its cache along into ordinary memory (path 1 with the cache uncached, 8 heads on 2, position
+// 1900: 167 us a token against 163); without room for it the cache stays where it is.
+static int cache_to_ordinary(l2h_model *m) {
+    if (!m->kv_uncached) return L2H_OK;
+    const int64_t n = cache_floats(m);
+    float *k = nullptr, *v = nullptr;
+    if (hipMalloc((void **)&k, (size_t)n * 4) != hipSuccess || hipMalloc((void **)&v, (size_t)n * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        if (k) (void)hipFree(k);
+        return L2H_OK;
+    }
+    m->allocs.push_back(k);
+    m->allocs.push_back(v);
+    HIPCHK(m->ctx, hipMemcpyAsync(k, m->kc, (size_t)n * 4, hipMemcpyDeviceToDevice, m->ctx->stream));
+    HIPCHK(m->ctx, hipMemcpyAsync(v, m->vc, (size_t)n * 4, hipMemcpyDeviceToDevice, m->ctx->stream));
+    HIPCHK(m->ctx, hipStreamSynchronize(m->ctx->stream));
+    m->kc = k;
+    m->vc = v;
+    m->kv_uncached = false;
+    return L2H_OK;
+}
+
 extern "C" int l2h_model_finalize(l2h_model *m) {
     if (!m) return L2H_EINVAL;
     l2h_ctx *ctx = m->ctx;
@@ -1068,40 +1125,12 @@ extern "C" int l2h_model_finalize(l2h_model *m) {
             return set_err(ctx, L2H_EINVAL, "an fp16 KV cache needs a head size that is a multiple of 32, at most 128");
         if (m->path_request == 2) return set_err(ctx, L2H_EINVAL, "an fp16 KV cache does not run on launch path 2");
     }
-    // (an fp16 cache takes half the floats)
-    // A launch of the streaming kernel that runs several steps of the token loop reads, in a later step, cache rows that
-    // another XCD's workgroups appended in an earlier one: rows in ordinary memory would still sit in the writer's L2
-    // (and stale lines in the reader's), which only the end of a kernel puts right.  Where no two heads share a cache
-    // row (n_kv_heads == n_heads: nothing is read twice, the L2 holds nothing worth keeping) the cache therefore lives
-    // in uncached memory, and such a model decodes several steps per launch; with shared rows it stays in ordinary memory
-    // and every step is a launch.  A small k-quant model (kq) has it uncached also with shared rows: what lies between two launches is a seventh of
-    // its step (40 tokens of 4 layers of 512 x 1024 with 8 heads on 2: 3.34 ms against 3.65; 32 at 3900 positions 3.79 against 4.04).
-    {
-        const char *env = getenv("L2H_KV_UNCACHED");
-        std::vector<int> types;
-        FlowArgs shape = flow_shape(m, types);
-        if (m->path_request == 0)
-            k_flow_plan_small(shape, types.data(), (int)types.size(), m->glob[L2H_OUTPUT].type, ctx->prop.multiProcessorCount, true);
-        m->kv_uncached = env ? atoi(env) != 0 : (shape.kq || (c.n_heads == c.n_kv_heads && (m->path_request == 0 || m->path_request == 3)));
-        const int64_t n = m->cache_layer_elems * c.n_layers / (m->kv16 ? 2 : 1) + 1;
-        if (m->kv_uncached) {
-            for (float **p : {&m->kc, &m->vc}) {
-                void *v = nullptr;
-                HIPCHK(ctx, uncached_alloc(ctx->device, (size_t)n * 4, &v));
-                m->uc_allocs.push_back(v);
-                HIPCHK(ctx, hipMemset(v, 0, (size_t)n * 4));
-                *p = (float *)v;
-            }
-        } else {
-            DA(m->kc, n, true);
-            DA(m->vc, n, true);
-        }
-    }
 #undef DA
     if ((rc = loop_buffers(m))) return rc;
     HIPCHK(ctx, hipDeviceSynchronize());
+    if ((rc = flow_setup(m))) return rc;  // (decides what memory the cache lies in)
+    if ((rc = cache_setup(m))) return rc;
     if ((rc = mega_setup(m))) return rc;
-    if ((rc = flow_setup(m))) return rc;
 
     if (!m->mega && !m->flow && (rc = record_token(m))) return rc;
     m->finalized = true;
@@ -1146,7 +1175,8 @@ static int mega_check(l2h_model *m) {
         // workgroups are not all resident at once (another process on the GPU) would give up at every token.  A
         // caller that asked for path 3 keeps it.
         if (m->path_request == 0) {
-            const int rc = record_token(m);
+            int rc = cache_to_ordinary(m);
+            if (rc == L2H_OK) rc = record_token(m);
             if (rc == L2H_OK) {
                 m->flow = false;
                 m->flow_why = "a wait of the streaming kernel ran into its limit (are its workgroups resident at once?); "

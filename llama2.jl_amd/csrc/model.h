@@ -53,7 +53,7 @@ struct l2h_model {
     hipGraphExec_t exec = nullptr;
     // persistent decode kernel
     int kv16 = 0;          // 1: the KV cache holds fp16 elements (l2h_model_set_kv_type)
-    bool kv_uncached = false;       // the KV cache lives in uncached memory (see l2h_model_finalize)
+    bool kv_uncached = false;       // the KV cache lives in uncached memory (see cache_setup)
     int flow_steps_per_launch = 1;  // steps of the token loop per launch of the streaming kernel
     int path_request = 0;  // 0 auto, 1 one kernel per phase, 2 persistent kernel, 3 streaming kernel (2, 3: required)
     bool mega = false;

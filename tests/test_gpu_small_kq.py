@@ -76,3 +76,29 @@ def test_gives_up_and_recovers(pkg):
         dev.reset()
         assert np.asarray(dev.generate_greedy(prompt, 12)).tolist() == want
     dev.close()
+
+
+def test_memory_of_the_cache_follows_the_path(pkg):
+    """uncached for several steps a launch; a model that leaves the kernel takes its cache's rows along, one that never ran it has an ordinary cache"""
+    from llama2_jl_amd import synth
+    fast, slow = _pair(pkg, 9, synth.PLAN_Q4_K_S, 512, 1024, 2, 8, 2, 500, False)
+    assert fast.chosen("uncached_cache") == 1 and slow.chosen("uncached_cache") == 0
+    prompt = synth.seeded_prompt(11, 6, 500)
+    for d in (fast, slow):
+        ids = np.asarray(d.generate_greedy(prompt, 40))
+    fast.set_wait_limit(0)
+    with pytest.raises(pkg.L2HError):
+        fast.forward(int(ids[-1]), 45)
+    assert fast.chosen("uncached_cache") == 0
+    for l in range(2):
+        for a, b in zip(fast.kv_read(l, 0, 45), slow.kv_read(l, 0, 45)):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    (a, la), (b, lb) = (d.generate_greedy([int(ids[-1])], 30, pos0=45, want_logits=True) for d in (fast, slow))
+    assert a.tolist() == b.tolist() and np.array_equal(la.view(np.uint32), lb.view(np.uint32))
+    fast.close()
+    slow.close()
+    # heads of 80, each with keys of its own: path 1
+    cfg = pkg.ModelConfig(dim=1280, hidden_dim=1024, n_layers=1, n_heads=16, n_kv_heads=16, vocab_size=500, seq_len=64, rope_freq_base=10000.0)
+    dev = synth.synthetic_model(cfg, synth.PLAN_Q4_K_S, seed=5).device()
+    assert dev.path == 1 and dev.chosen("uncached_cache") == 0
+    dev.close()
