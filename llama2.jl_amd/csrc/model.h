@@ -71,6 +71,8 @@ struct l2h_model {
     int32_t *sample_out = nullptr;
     // streaming decode kernel
     bool flow = false;
+    bool wait_limit_set = false;  // l2h_model_set_wait_limit: the caller is told where a wait gave up
+    bool run_again = false;       // a call's launch gave up, and the call is to run on path 1
     FlowArgs flow_args{};
     int flow_grid = 0, flow_cls_type = 0;
     bool flow_holds_state = false;  // the activations of the last step are in flow_args' words

@@ -102,3 +102,20 @@ def test_memory_of_the_cache_follows_the_path(pkg):
     dev = synth.synthetic_model(cfg, synth.PLAN_Q4_K_S, seed=5).device()
     assert dev.path == 1 and dev.chosen("uncached_cache") == 0
     dev.close()
+
+
+def test_a_call_that_cannot_run_here_runs_on_path_1(pkg, monkeypatch):
+    """the library's own bound, forced to zero from the host: the call that finds it met gives path 1's results, from the rows that the cache held"""
+    from llama2_jl_amd import _lib, synth
+    monkeypatch.setenv("L2H_FLOW_SPINS", "0")
+    fast, slow = _pair(pkg, 13, synth.PLAN_Q4_K_S, 512, 1024, 2, 8, 2, 500, False)
+    tok = synth.seeded_prompt(3, 37, 500)
+    got = []
+    for d in (fast, slow):
+        d.prefill(tok)
+        ids, logits = d.generate_greedy(tok[:5], 20, pos0=37, want_logits=True)
+        got.append((ids.tolist(), logits.tobytes(), d.forward(int(ids[-1]), 61)[0].tobytes()))
+    assert got[0] == got[1]
+    assert _lib.lib().l2h_model_path(fast.handle) == 1 and "one kernel per phase" in _lib.lib().l2h_model_path_reason(fast.handle).decode()
+    fast.close()
+    slow.close()
