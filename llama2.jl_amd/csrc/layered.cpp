@@ -1180,7 +1180,7 @@ static hipError_t to_acts(l2h_model *m, GemmArgs a, int epi, void *out, int64_t 
     a.acols = cols;
     if (w && image_takes(*w, a.M)) {
         a.w = w->image;
-        return k_tiles(m->ctx->stream, a, epi);
+        return k_tiles(m->ctx->stream, a, epi, m->ctx->prop.multiProcessorCount);
     }
     return k_gemm(m->ctx->stream, a, m->lay->c.precision, epi);
 }
@@ -1310,7 +1310,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     if (image) {
         up.w = L.up.image;
         up.expert_stride = L.up.image_stride;
-        CK(k_tiles(s, up, epi));
+        CK(k_tiles(s, up, epi, m->ctx->prop.multiProcessorCount));
     } else {
         CK(k_gemm(s, up, prec, epi));
     }
@@ -1321,7 +1321,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     if (image) {
         down.w = L.down.image;
         down.expert_stride = L.down.image_stride;
-        CK(k_tiles(s, down, GE_STORE));
+        CK(k_tiles(s, down, GE_STORE, m->ctx->prop.multiProcessorCount));
     } else {
         CK(k_gemm(s, down, prec, GE_STORE));
     }

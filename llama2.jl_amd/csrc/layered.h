@@ -137,7 +137,7 @@ inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations
-hipError_t k_tiles(hipStream_t s, const GemmArgs &a, int epi);
+hipError_t k_tiles(hipStream_t s, const GemmArgs &a, int epi, int n_cu);
 int64_t k_tile_image_elems(int64_t rows, int ld);
 hipError_t k_tile_image(hipStream_t s, const uint16_t *w, int ld, int64_t rows, int64_t n_mats, uint16_t *dst);
 // outa[m][n] = act(v[m][n]) * embedding element, for products that the library has stored as fp32

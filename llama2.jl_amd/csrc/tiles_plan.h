@@ -31,10 +31,10 @@ __host__ __device__ inline TilesWork tiles_work(const TilesPlan &p, unsigned b) 
     return {i < n, p.whole + i / 2, (int)(i & 1u)};
 }
 
-// 896 tiles of 28 672 x 4096 over 2048 positions take 465 us in four rounds of the compute units, the last half empty, 431 as three rounds and
-// 256 halves.  Only where the halves are one round, up to 128 tiles: two rounds of halves take as long as one of whole tiles.
-inline TilesPlan tiles_plan(unsigned n, bool halves) {
-    const unsigned rest = n % 256;
-    const unsigned whole = halves && n > 256 && rest > 0 && rest <= 128 ? n - rest : n;
+// 896 tiles of 28 672 x 4096 over 2048 positions take 465 us in four rounds of 256 compute units, the last half empty, 431 as three rounds and
+// 256 halves.  Only where the halves are one round: two rounds of halves take as long as one of whole tiles.
+inline TilesPlan tiles_plan(unsigned n, bool halves, int n_cu) {
+    const unsigned rest = n % (unsigned)n_cu;
+    const unsigned whole = halves && n > rest && rest > 0 && 2 * rest <= (unsigned)n_cu ? n - rest : n;
     return {n, whole, tiles_workgroups(whole)};
 }

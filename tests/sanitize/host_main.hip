@@ -166,27 +166,31 @@ static void check_rows_plan() {
 
 // every tile of a prompt's product is taken exactly once, as a whole or as both of its halves
 static void check_tiles_plan() {
-    int split = 0;
-    for (unsigned n = 1; n <= 2048; n++)
-        for (int halves = 0; halves < 2; halves++) {
-            const TilesPlan p = tiles_plan(n, halves != 0);
-            std::vector<int> taken(n, 0);  // in halves
-            const unsigned grid = tiles_grid(p);
-            for (unsigned b = 0; b < grid; b++) {
-                const TilesWork w = tiles_work(p, b);
-                if (!w.any) continue;
-                EXPECT(w.item < n && w.half >= -1 && w.half <= 1);
-                if (w.item >= n) continue;
-                EXPECT((taken[w.item] & (w.half < 0 ? 3 : 1 << w.half)) == 0);
-                taken[w.item] |= w.half < 0 ? 3 : 1 << w.half;
+    for (int n_cu : {32, 64, 250, 256}) {
+        int split = 0;
+        for (unsigned n = 1; n <= 2048; n++)
+            for (int halves = 0; halves < 2; halves++) {
+                const TilesPlan p = tiles_plan(n, halves != 0, n_cu);
+                std::vector<int> taken(n, 0);  // in halves
+                const unsigned grid = tiles_grid(p);
+                for (unsigned b = 0; b < grid; b++) {
+                    const TilesWork w = tiles_work(p, b);
+                    if (!w.any) continue;
+                    EXPECT(w.item < n && w.half >= -1 && w.half <= 1);
+                    if (w.item >= n) continue;
+                    EXPECT((taken[w.item] & (w.half < 0 ? 3 : 1 << w.half)) == 0);
+                    taken[w.item] |= w.half < 0 ? 3 : 1 << w.half;
+                }
+                bool all = true;
+                for (unsigned i = 0; i < n; i++) all = all && taken[i] == 3;
+                if (!all) printf("%u tiles\n", n);
+                EXPECT(all);
+                // whole rounds, and no more than one round of halves behind them
+                EXPECT(p.whole == n || (halves && p.whole % (unsigned)n_cu == 0 && 2 * (n - p.whole) <= (unsigned)n_cu));
+                split += p.whole < n;
             }
-            bool all = true;
-            for (unsigned i = 0; i < n; i++) all = all && taken[i] == 3;
-            if (!all) printf("%u tiles\n", n);
-            EXPECT(all);
-            if (halves) split += p.whole < n;
-        }
-    EXPECT(split == 7 * 128);
+        EXPECT(n_cu != 256 || split == 7 * 128);
+    }
     // a grouped product's grid is made for the most tiles there can be, and dealt out by how many there are
     for (unsigned most = 1; most <= 300; most++)
         for (unsigned n = 1; n <= most; n++) {
