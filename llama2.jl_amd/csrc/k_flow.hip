@@ -3459,13 +3459,17 @@ static int kq_wave_plan(FlowArgs &a, const int *layer_types, int n_layer_types, 
     return a.dim / 256;
 }
 
-// On all compute units, or on a half or a quarter of them where a phase has too few pieces for more.
+// On all compute units, or on a half or a quarter of them where a phase has too few pieces for more.  On a quarter a long cache's attention takes longer than
+// the hand-overs save: 512 x 64 (fp32), six layers, 8 heads, a token at position 8000 / 16 000 / 30 000 with flow_f32_kernel on all of them 216 / 240 / 295
+// us, on a quarter 211 / 275 / 384; 512 x 200 on a half 185 / 219 / 281 against 225 / 250 / 304.
+#define FLOW_QUARTER_SEQ 8192
 int k_flow_plan_small(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int n_cu, bool automatic) {
     a.mixed = a.f32 = a.f32_quads = a.kq = 0;
     bool all_f32 = cls_type == L2H_TYPE_F32;
     for (int i = 0; i < n_layer_types; i++) all_f32 = all_f32 && layer_types[i] == L2H_TYPE_F32;
     if (all_f32 && !small_heads_fit(a, n_cu)) return 0;  // (refused by k_flow_plan too)
     for (int grid = n_cu; grid >= 64 && grid >= n_cu / 4; grid /= 2) {
+        if (grid < n_cu / 2 && a.seq_len > FLOW_QUARTER_SEQ) break;
         if (all_f32 && (a.f32_quads = f32_wave_plan(a, grid)) != 0) a.f32 = 1;
         if (!all_f32 && automatic) a.kq = kq_wave_plan(a, layer_types, n_layer_types, cls_type, grid);
         if (a.f32 || a.kq) return grid;

@@ -126,6 +126,21 @@ static void check_shape(int dim, int hidden, int n_layers, int n_heads, int n_kv
     }
 }
 
+// workgroups of the kernels for small models: 0 where the model does not go there
+static int small(int type, int dim, int hidden, int heads, int kv, int vocab, int seq_len = 320, bool automatic = true) {
+    FlowArgs a{};
+    a.dim = dim, a.hidden = hidden, a.n_layers = 2, a.n_heads = heads, a.n_kv_heads = kv;
+    a.hs = dim / heads, a.kv_dim = a.hs * kv, a.seq_len = seq_len, a.vocab = vocab;
+    const std::vector<int> types(14, type);
+    return k_flow_plan_small(a, types.data(), 14, type, 256, automatic);
+}
+static void check_small_plan() {
+    // a long cache's attention wants at least half of the compute units
+    EXPECT(small(0, 512, 64, 8, 8, 32000, 8192) == 64 && small(0, 512, 64, 8, 8, 32000, 8193) == 0);
+    EXPECT(small(0, 512, 200, 8, 8, 32000, 8192) == 128 && small(0, 512, 200, 8, 8, 32000, 32768) == 128 && small(0, 512, 1376, 8, 8, 32000, 32768) == 256);
+    EXPECT(small(0, 256, 64, 8, 8, 32000, 320) == 64 && small(0, 256, 64, 8, 8, 32000, 32768) == 0 && small(0, 256, 688, 8, 8, 32000, 32768) == 128);
+}
+
 // which kernel takes a product of a layered model: `each` positions for each of `experts` matrices (0: one matrix, `each` positions)
 static bool few(int prec, int experts, int64_t cols, int each) {
     GemmTile tile{};
@@ -205,6 +220,7 @@ static void check_tiles_plan() {
 
 int main() {
     check_tiles_plan();
+    check_small_plan();
     check_product_rule();
     check_rows_plan();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
