@@ -111,7 +111,7 @@ int l2h_model_set_kv_type(l2h_model *m, int kv_type);
  *   - models whose matrices are all fp32: dim and hidden_dim multiples of 4, at most 4096; head size 32, 64
  *     or 128; fp32 cache;
  *   - by the automatic choice only, small models of q4_K, q5_K or q6_K matrices (w1 and w3 of a layer of one type): dim 512 or 1024,
- *     hidden_dim a multiple of 256 up to 3840, at most 64 layers, head size 32 or 64, fp32 cache, up to 65 536 (dim 512) or 131 072 rows of classifier;
+ *     hidden_dim a multiple of 256 up to 3840 (3584 with heads of 32), at most 64 layers, head size 32 or 64, fp32 cache, up to 65 536 (dim 512) or 131 072 rows of classifier;
  *   in all cases n_heads <= 256, a head size that is a multiple of 256 / n_heads, and a cache length that fits
  *   the attention's LDS area (with head size 128: about 2 400 positions times 256 / n_heads, e.g. 19 000
  *   for 32 heads).
@@ -157,8 +157,10 @@ int l2h_model_prefill_library(l2h_model *m);
  *   L2H_CHOSEN_TILE_IMAGES  matrices of a layered model whose prompt products run from tile images (made by the first
  *                           prompt pass of more than 128 positions); 0 otherwise
  *   L2H_CHOSEN_UNCACHED_CACHE  1 if the KV cache lies in uncached memory (several steps of the token loop per launch), else 0
+ *   L2H_CHOSEN_SMALL_KERNEL    1 if path 3 runs one of the kernels for small models, else 0
+ *   L2H_CHOSEN_SHARED_STEPS    layers of a layered model whose attention and feed-forward share launches in a decode step
  * No counterpart in the reference. */
-enum { L2H_CHOSEN_TILE_IMAGES = 0, L2H_CHOSEN_UNCACHED_CACHE = 1 };
+enum { L2H_CHOSEN_TILE_IMAGES = 0, L2H_CHOSEN_UNCACHED_CACHE = 1, L2H_CHOSEN_SMALL_KERNEL = 2, L2H_CHOSEN_SHARED_STEPS = 3 };
 int l2h_model_chosen(l2h_model *m, int what);
 /* RunState(config) (src/inference.jl:88-100): checks every tensor is present, allocates
  * activations and the zeroed KV cache, records the per-token launch sequence. */

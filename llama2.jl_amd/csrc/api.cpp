@@ -409,6 +409,8 @@ extern "C" int l2h_model_chosen(l2h_model *m, int what) {
     if (!m || !m->finalized) return -1;
     if (what == L2H_CHOSEN_TILE_IMAGES) return m->lay ? layered_images(m) : 0;
     if (what == L2H_CHOSEN_UNCACHED_CACHE) return m->kv_uncached ? 1 : 0;
+    if (what == L2H_CHOSEN_SMALL_KERNEL) return m->flow && (m->flow_args.kq || (m->flow_args.f32 && m->flow_args.f32_quads)) ? 1 : 0;
+    if (what == L2H_CHOSEN_SHARED_STEPS) return m->lay ? layered_shared_steps(m) : 0;
     return -1;
 }
 

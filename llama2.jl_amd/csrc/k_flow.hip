@@ -2361,7 +2361,7 @@ __global__ __launch_bounds__(1024) void flow_f32_kernel(unsigned int gen0, int n
 //
 // What bounds such a model is the chain of hand-overs, not its bytes (a 512-wide layer's 12.6 MB stream in 3 us).  So
 //  * a phase has one barrier, behind the wait for its input.  Wavefronts with rows then take the input from LDS into registers, in the
-//    places of the row's own 16-byte loads, each norms it for itself, and lanes 0 and 1 finish the pair.  w2's rows, up to 4096
+//    places of the row's own 16-byte loads, each norms it for itself, and lanes 0 and 1 finish the pair.  w2's rows, up to 4032
 //    long, go in slices of at most 512 inputs, a wavefront each, that meet in LDS behind a second barrier.
 //  * a phase's rows are requested as soon as the phase before it has its input: a compute unit's loads pass its polls by, and a
 //    request of 24 KB in front of a wait makes the wait 1 to 1.5 us longer (7.3 ms against 5.8 in the run below).
@@ -3428,7 +3428,7 @@ static int f32_wave_plan(FlowArgs &a, int grid) {
 // Microseconds a token on path 1 and here, 32 000 rows of classifier, six layers, at position 20 (300, 1900): 512 x 1280 with 8 heads on 2: 225 (233, 246),
 // 100 (141, 144); 1024 x 2816 with 16 heads on 4: 241 (249, 264), 159 (199, 203), with 16 on 16 and q5_K_M: 234 (241, 259), 159 (206,
 // 214).  Dim 256, half a group of 16 lanes to a row, and rows of other lengths, whose places in a wavefront are no power of two, are not
-// built.  Heads of 128 stay on path 1, as l2h_model_path has told the callers of such models.
+// built, nor is the attention of heads of 128: such models stay on path 1.
 static int kq_wave_plan(FlowArgs &a, const int *layer_types, int n_layer_types, int cls_type, int grid) {
     auto quant = [](int t) { return t == L2H_TYPE_Q4_K || t == L2H_TYPE_Q5_K || t == L2H_TYPE_Q6_K; };
     if ((a.dim != 512 && a.dim != 1024) || a.hidden % 256 != 0 || a.hidden > 4096 || a.n_layers > FLOWQ_LAYERS || a.hs > 64 || a.kv16 || !quant(cls_type))

@@ -833,6 +833,13 @@ static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int c
     return k_step_fits(w, L.ukv.ld, a.uq, a.up, a.up_pro, a.down, a.down_pro, cu);
 }
 
+int layered_shared_steps(l2h_model *m) {
+    int n = 0;
+    LatentLayerStep a;
+    for (const LayerDev &L : m->lay->layer) n += shares_launches(m->lay, L, m->x, m->ctx->prop.multiProcessorCount, a);
+    return n;
+}
+
 // Mixer and feed-forward of a layer, a launch each; `in` reads the norm of the stream x into the mixer's projected row
 // (`plus`, `plus2`: what the next layer's pass of a loop adds to the stream, in the launch that completes it)
 static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x, const float *plus, const float *plus2) {

@@ -150,7 +150,7 @@ class DeviceModel:
         """True if the last prefill ran those products through hipBLASLt (l2h_model_prefill_library)."""
         return bool(_lib.lib().l2h_model_prefill_library(self.handle))
 
-    _CHOSEN = ("tile_images", "uncached_cache")
+    _CHOSEN = ("tile_images", "uncached_cache", "small_kernel", "shared_steps")
 
     def chosen(self, what):
         """Which kernels the model's sizes have chosen (l2h_model_chosen), for checks."""

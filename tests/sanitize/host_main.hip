@@ -135,6 +135,17 @@ static int small(int type, int dim, int hidden, int heads, int kv, int vocab, in
     return k_flow_plan_small(a, types.data(), 14, type, 256, automatic);
 }
 static void check_small_plan() {
+    // fp32, dim 256 or 512: hidden sizes at which a phase has pairs of rows for every workgroup, and wavefronts for every pair
+    EXPECT(!small(0, 512, 44, 16, 16, 500) && small(0, 512, 48, 16, 16, 500) == 64 && small(0, 512, 3840, 16, 4, 500) == 256 && !small(0, 512, 3844, 16, 4, 500));
+    EXPECT(small(0, 512, 244, 8, 8, 500) == 128 && small(0, 512, 248, 8, 8, 500) == 256 && small(0, 512, 3968, 8, 2, 500) == 256 && !small(0, 512, 3972, 8, 2, 500));
+    EXPECT(!small(0, 512, 56, 4, 4, 500) && small(0, 512, 60, 4, 4, 500) == 64 && small(0, 512, 4032, 4, 1, 500) == 256 && !small(0, 512, 4036, 4, 4, 500));
+    EXPECT(!small(0, 256, 52, 8, 8, 500) && small(0, 256, 56, 8, 8, 500) == 64 && small(0, 256, 1920, 8, 1, 500) == 128 && !small(0, 256, 1924, 8, 1, 500));
+    EXPECT(small(0, 256, 1984, 4, 4, 500) == 128 && !small(0, 256, 1988, 4, 4, 500) && !small(0, 256, 688, 2, 2, 500) && !small(0, 1024, 2048, 16, 16, 500));
+    // k-quants, dim 512 or 1024, heads of 32 or 64
+    EXPECT(small(12, 512, 256, 8, 8, 65536) == 128 && !small(12, 512, 256, 8, 8, 65537) && small(12, 512, 3840, 8, 8, 500) == 128 && !small(12, 512, 4096, 8, 8, 500));
+    EXPECT(small(13, 512, 3584, 16, 4, 500) == 128 && !small(13, 512, 3840, 16, 4, 500) && small(14, 1024, 3584, 32, 8, 500) == 256 && !small(14, 1024, 3840, 32, 8, 500));
+    EXPECT(small(12, 1024, 3840, 16, 4, 131072) == 256 && !small(12, 1024, 3840, 16, 4, 131073) && !small(12, 1024, 4096, 16, 4, 500));
+    EXPECT(!small(12, 1024, 1024, 8, 8, 500) && !small(12, 256, 512, 8, 8, 500) && !small(12, 512, 1024, 8, 2, 500, 320, false));
     // a long cache's attention wants at least half of the compute units
     EXPECT(small(0, 512, 64, 8, 8, 32000, 8192) == 64 && small(0, 512, 64, 8, 8, 32000, 8193) == 0);
     EXPECT(small(0, 512, 200, 8, 8, 32000, 8192) == 128 && small(0, 512, 200, 8, 8, 32000, 32768) == 128 && small(0, 512, 1376, 8, 8, 32000, 32768) == 256);

@@ -28,35 +28,50 @@ def _same(fast, slow, prompt, n_new):
         assert np.array_equal(fast.state(name).view(np.uint32), slow.state(name).view(np.uint32)), name
 
 
+# the smallest of each kernel: (hidden, whether the kernel for small models takes it)
+@pytest.mark.parametrize("hidden,small", [(4, 0), (56, 1), (120, 1)])
 @pytest.mark.parametrize("n_new", [2, 7, 19])
-def test_keys_of_the_steps_before_in_one_launch(pkg, n_new):
+def test_keys_of_the_steps_before_in_one_launch(pkg, n_new, hidden, small):
     """A layer so small that nothing sweeps the vector cache between a step's read of a line of keys and the next step's"""
     from llama2_jl_amd import synth
-    fast, slow = _pair(pkg, 31, 256, 4, 2, 8, 8, 300, False)
-    assert fast.steps_per_launch == 8
+    fast, slow = _pair(pkg, 31, 256, hidden, 2, 8, 8, 300, False)
+    assert fast.steps_per_launch == 8 and fast.chosen("small_kernel") == small
     _same(fast, slow, synth.seeded_prompt(70, 2, 300), n_new)
     fast.close()
     slow.close()
 
 
 SHAPES = [
-    # (dim, hidden, layers, heads, kv heads, vocabulary, neox): hidden sizes around the slices of 512 that w2's rows are cut into and
-    # the longest, row counts that leave workgroups, wavefronts and the last pair of the classifier without rows, every head size
-    (256, 4, 2, 8, 8, 1, False),
-    (256, 512, 2, 4, 2, 255, True),
-    (256, 516, 1, 8, 1, 4097, False),
-    (512, 1376, 2, 8, 8, 32000, False),
-    (512, 2052, 2, 16, 4, 3, True),
-    (512, 4096, 2, 4, 4, 1000, False),
+    # (small, dim, hidden, layers, heads, kv heads, vocabulary, neox): hidden sizes around the slices of 512 that w2's rows are cut into, the shortest and the
+    # longest of each head size that the kernel for small models takes (small = 1) and some just beyond, where the general fp32 kernel runs; row counts
+    # that leave workgroups, wavefronts and the last pair of the classifier without rows
+    (0, 256, 4, 2, 8, 8, 1, False),
+    (1, 256, 512, 2, 4, 2, 255, True),
+    (1, 256, 516, 1, 8, 1, 4097, False),
+    (1, 256, 56, 2, 8, 8, 33, True),
+    (1, 256, 1920, 2, 8, 2, 1000, False),
+    (1, 256, 1984, 2, 4, 4, 1000, True),
+    (0, 256, 1988, 2, 4, 4, 1000, True),
+    (1, 512, 1376, 2, 8, 8, 32000, False),
+    (1, 512, 2052, 2, 16, 4, 3, True),
+    (1, 512, 48, 2, 16, 16, 500, False),
+    (1, 512, 3840, 1, 16, 4, 1000, True),
+    (1, 512, 3968, 1, 8, 2, 1000, False),
+    (1, 512, 60, 2, 4, 4, 500, True),
+    (1, 512, 252, 2, 4, 1, 1, False),
+    (1, 512, 4032, 2, 4, 4, 1000, False),
+    (0, 512, 4096, 2, 4, 4, 1000, False),
 ]
 
 
 @pytest.mark.parametrize("shape", range(len(SHAPES)))
 def test_rows_slices_and_heads(pkg, shape):
     from llama2_jl_amd import synth
-    fast, slow = _pair(pkg, 40 + shape, *SHAPES[shape])
+    small, *sizes = SHAPES[shape]
+    fast, slow = _pair(pkg, 40 + shape, *sizes)
+    assert fast.chosen("small_kernel") == small and slow.chosen("small_kernel") == 0
     for rep, n_new in enumerate((19, 290)):  # the second run crosses into the attention of long caches
-        _same(fast, slow, synth.seeded_prompt(70 + rep, 2 + 5 * rep, SHAPES[shape][5]), n_new)
+        _same(fast, slow, synth.seeded_prompt(70 + rep, 2 + 5 * rep, sizes[5]), n_new)
     fast.close()
     slow.close()
 

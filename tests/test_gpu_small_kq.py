@@ -15,7 +15,7 @@ def _pair(pkg, seed, plan, dim, hidden, layers, heads, kv, vocab, neox):
                           rope_freq_base=10000.0, rope_is_neox=neox)
     lm = synth.synthetic_model(cfg, plan, seed=seed)
     fast, slow = DeviceModel(cfg, lm.weights), DeviceModel(cfg, lm.weights, path=1)
-    assert fast.path == 3 and slow.path == 1 and fast.steps_per_launch == 8
+    assert fast.path == 3 and slow.path == 1 and fast.steps_per_launch == 8 and fast.chosen("small_kernel") == 1
     return fast, slow
 
 
@@ -40,6 +40,9 @@ SHAPES = [
     ("PLAN_Q4_K_S", 1024, 2816, 2, 16, 4, 1000, False),
     ("PLAN_Q5_K_M", 1024, 3840, 2, 16, 16, 32003, True),
     ("PLAN_Q5_K_M", 1024, 256, 2, 32, 8, 300, False),
+    # the longest with heads of 32
+    ("PLAN_Q4_K_S", 512, 3584, 2, 16, 4, 300, False),
+    ("PLAN_Q5_K_M", 1024, 3584, 2, 32, 32, 300, True),
 ]
 
 
@@ -59,6 +62,25 @@ def test_asked_for_by_number_it_is_refused_as_before(pkg):
     cfg = pkg.ModelConfig(dim=512, hidden_dim=1024, n_layers=1, n_heads=8, n_kv_heads=2, vocab_size=500, seq_len=64, rope_freq_base=10000.0)
     with pytest.raises(pkg.L2HError):
         synth.synthetic_model(cfg, synth.PLAN_Q4_K_S, seed=5).device(path=3)
+
+
+@pytest.mark.parametrize("dim,hidden,heads", [(512, 3840, 16), (1024, 3840, 32), (512, 4096, 8), (1024, 1024, 8), (256, 512, 8)])
+def test_just_beyond_it_runs_on_path_1(pkg, dim, hidden, heads):
+    from llama2_jl_amd import synth
+    cfg = pkg.ModelConfig(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=heads, n_kv_heads=heads, vocab_size=300, seq_len=64, rope_freq_base=10000.0)
+    dev = synth.synthetic_model(cfg, synth.PLAN_Q4_K_S, seed=5).device()
+    assert dev.path == 1 and dev.chosen("small_kernel") == 0 and dev.path_reason
+    dev.close()
+
+
+@pytest.mark.parametrize("n_new", [2, 7, 19])
+def test_keys_of_the_steps_before_in_one_launch(pkg, n_new):
+    """as for the fp32 kernel: a layer whose rows sweep little of the vector cache between a step's read of a line of keys and the next step's"""
+    from llama2_jl_amd import synth
+    fast, slow = _pair(pkg, 31, synth.PLAN_Q4_K_S, 512, 256, 2, 16, 16, 300, False)
+    _same(fast, slow, synth.seeded_prompt(70, 2, 300), n_new)
+    fast.close()
+    slow.close()
 
 
 def test_gives_up_and_recovers(pkg):

@@ -38,6 +38,7 @@ def test_borders(pkg, shape):
         want.append(s.step(int(a)))
     want = np.array(want)
     dev = zc.language_model(pkg, c, t, seq_len=n).device()
+    assert dev.chosen("shared_steps") == (0 if shape in ("rank_beyond", "odd_query") else len(c["layers"]))
     borders = (0, 30, 62, 126, 158, 510)
     for b in borders:
         if b >= n:
@@ -69,6 +70,7 @@ def test_padding_behind_the_heads(pkg):
     for a in tok:
         want.append(s.step(int(a)))
     dev = zc.language_model(pkg, c, t, seq_len=n).device()
+    assert dev.chosen("shared_steps") == 2
     for at in (40, 70, 100, 130, 150):
         dev.reset()
         with np.errstate(invalid="ignore"):
