@@ -63,18 +63,10 @@ __device__ __forceinline__ float l_wave_sum(float v) {
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, WAVE);
     return v;
 }
-// the same by moves within the rows of 16 lanes and four reads across them; the sum is a scalar
+// v plus its value in another lane of the same sixteen
 template <int CTRL>
 __device__ __forceinline__ float l_dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float l_wave_sum_dpp(float v) {
-    v = l_dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
-    v = l_dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
-    v = l_dpp_add<0x141>(v);  // row_half_mirror
-    v = l_dpp_add<0x140>(v);  // row_mirror
-    auto at = [&](int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); };
-    return (at(0) + at(16)) + (at(32) + at(48));
 }
 // sum over the workgroup; `red` holds one float per wavefront; every thread gets the total
 __device__ __forceinline__ float l_block_sum(float v, float *red) {
