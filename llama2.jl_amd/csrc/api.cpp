@@ -967,7 +967,7 @@ static hipError_t enqueue_token(l2h_model *m) {
     } while (0)
     if (m->lay) {
         CK(layered_enqueue_token(m));
-        return k_argmax(s, m->logits, c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out);
+        return k_argmax(s, m->logits, c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, true);
     }
     // token embedding (:236) and this position's RoPE table
     CK(k_embed(s, m->glob[L2H_TOK_EMB], m->ctl, m->prompt_dev, m->x, m->rope_cs, m->hs, m->theta_scale));
@@ -986,7 +986,7 @@ static hipError_t enqueue_token(l2h_model *m) {
         CK(launch_w2(m, l));
     }
     CK(launch_output(m));
-    CK(k_argmax(s, m->logits, c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out));  // :360
+    CK(k_argmax(s, m->logits, c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, true));  // :360
 #undef CK
     return hipSuccess;
 }
@@ -1571,7 +1571,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
     HIPCHK(ctx, hipMemcpyAsync(m->ctl, &h, sizeof h, hipMemcpyHostToDevice, ctx->stream));
     hipError_t e = m->lay ? layered_output(m) : launch_output(m);
     if (e == hipSuccess)
-        e = k_argmax(ctx->stream, m->logits, m->c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out);
+        e = k_argmax(ctx->stream, m->logits, m->c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, false);
     if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "classifier launch failed: %s", hipGetErrorString(e));
     if (next_token)
         HIPCHK(ctx, hipMemcpyAsync(next_token, m->out_tokens, 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -1986,7 +1986,7 @@ extern "C" int l2h_argmax(l2h_ctx *ctx, const float *x, int64_t n, int32_t *out)
     h.n_prompt = 1;
     HIPCHK(ctx, hipMemcpy(dctl.p, &h, sizeof h, hipMemcpyHostToDevice));
     HIPCHK(ctx, hipMemcpy(dx.p, x, (size_t)n * 4, hipMemcpyHostToDevice));
-    HIPCHK(ctx, k_argmax(ctx->stream, dx.as<float>(), n, dp.as<int64_t>(), (DecodeCtl *)dctl.p, dout.as<int32_t>(), 1));
+    HIPCHK(ctx, k_argmax(ctx->stream, dx.as<float>(), n, dp.as<int64_t>(), (DecodeCtl *)dctl.p, dout.as<int32_t>(), 1, false));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     HIPCHK(ctx, hipMemcpy(out, dout.p, 4, hipMemcpyDeviceToHost));
     return L2H_OK;

@@ -272,6 +272,9 @@ __global__ __launch_bounds__(256) void argmax_stage2_kernel(const unsigned long 
 
 // Both stages by one workgroup, all of a thread's elements under way at once: 32 000 logits in 5.8 us, against 4.6 + 4.1 in two
 // launches.  Bound by what one CU draws from the L2s; beyond 32 768 elements a thread's would no longer fit its registers.
+// At the end of a prompt pass, launch by launch: 4 us less (1244 -> 1239 us, 33 positions of 4096 wide layers).  In a recorded step, whose launches
+// follow each other closely and whose next one waits for this, 0.8 to 1.4 us more (a token of Vudelix, width 768, 4 layers: 170.6 us with two launches,
+// 171.7 with one; 2176, 2 layers: 140.5, 141.7): steps take two.
 #define ARGMAX_ONE_N 32768
 __global__ __launch_bounds__(1024) void argmax_one_kernel(const float *x, int n, DecodeCtl *ctl, int32_t *out_tokens, int max_out) {
     __shared__ unsigned long long red[16];
@@ -299,8 +302,8 @@ __global__ __launch_bounds__(1024) void argmax_one_kernel(const float *x, int n,
 }
 
 hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, DecodeCtl *ctl, int32_t *out_tokens,
-                    int max_out) {
-    if (n >= 4 && n <= ARGMAX_ONE_N && (uintptr_t)x % 16 == 0) {
+                    int max_out, bool step) {
+    if (!step && n >= 4 && n <= ARGMAX_ONE_N && (uintptr_t)x % 16 == 0) {
         hipLaunchKernelGGL(argmax_one_kernel, dim3(1), dim3(1024), 0, s, x, (int)n, ctl, out_tokens, max_out);
         return hipGetLastError();
     }

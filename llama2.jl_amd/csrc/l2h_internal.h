@@ -255,8 +255,9 @@ hipError_t k_attention(hipStream_t s, const double *qd, const float *kc, const f
 hipError_t k_attention_fused(hipStream_t s, const float *q, float *xb, const float *kc, const float *vc,
                              const DecodeCtl *ctl, int head_size, int n_heads, int n_kv_heads, int seq_len);
 hipError_t k_softmax(hipStream_t s, float *x, int64_t n);
+// step: of the token loop (launch sequences that are recorded)
 hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, DecodeCtl *ctl, int32_t *out_tokens,
-                    int max_out);
+                    int max_out, bool step);
 // argmax without allocations: k_noalloc_init once per device (that device current), then k_argmax_noalloc
 hipError_t k_noalloc_init(int device);
 hipError_t k_argmax_noalloc(hipStream_t s, int device, const float *x_dev, int64_t n, int32_t *out_dev);
