@@ -6,17 +6,26 @@
 template <int PRO, int EPI, int U, int V, bool Y>
 __global__ __launch_bounds__(ROWS_THREADS, 4) void rows_kernel(RowsArgs a, RowsPlan pl) {
     extern __shared__ __align__(16) float s_mem[];
-    __shared__ RowsShared sh;
-    rows_body<PRO, EPI, U, V, Y>(a, pl, blockIdx.x, s_mem, sh);
+    rows_body<PRO, EPI, U, V, Y>(a, pl, blockIdx.x, s_mem);
+}
+template <int PRO, int EPI, int U, int V, bool Y>
+__global__ __launch_bounds__(ROWS_THREADS, 4) void rows_more_kernel(RowsArgs a, RowsPlan pl, RowsMore m) {
+    extern __shared__ __align__(16) float s_mem[];
+    rows_body<PRO, EPI, U, V, Y>(a, pl, blockIdx.x, s_mem, m);
 }
 
 #define ROWS_MAX_DEVICES 64
 
 template <int PRO, int EPI, int U, int V, bool Y>
-static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
+static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid, const RowsMore &m) {
     const RowsPlan pl = rows_plan(a, PRO, U, grid);
     const size_t lds = rows_lds(a, PRO, pl.pairs + 1);
     if (lds > ROWS_LDS) return hipErrorInvalidValue;
+    const void *fn;
+    if constexpr (EPI == RE_RESID_MORE)
+        fn = (const void *)rows_more_kernel<PRO, EPI, U, V, Y>;
+    else
+        fn = (const void *)rows_kernel<PRO, EPI, U, V, Y>;
     if (lds > 48 * 1024) {
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
@@ -24,17 +33,20 @@ static hipError_t rows_launch(hipStream_t s, const RowsArgs &a, int64_t grid) {
         if (dev < 0 || dev >= ROWS_MAX_DEVICES) return hipErrorInvalidDevice;
         static bool attr_set[ROWS_MAX_DEVICES] = {};
         if (!attr_set[dev]) {
-            e = hipFuncSetAttribute((const void *)rows_kernel<PRO, EPI, U, V, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, ROWS_LDS);
+            e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, ROWS_LDS);
             if (e != hipSuccess) return e;
             attr_set[dev] = true;
         }
     }
-    hipLaunchKernelGGL((rows_kernel<PRO, EPI, U, V, Y>), dim3((unsigned)grid), dim3(ROWS_THREADS), lds, s, a, pl);
+    if constexpr (EPI == RE_RESID_MORE)
+        hipLaunchKernelGGL((rows_more_kernel<PRO, EPI, U, V, Y>), dim3((unsigned)grid), dim3(ROWS_THREADS), lds, s, a, pl, m);
+    else
+        hipLaunchKernelGGL((rows_kernel<PRO, EPI, U, V, Y>), dim3((unsigned)grid), dim3(ROWS_THREADS), lds, s, a, pl);
     return hipGetLastError();
 }
 
 template <int PRO, int EPI, int V, bool Y>
-static hipError_t rows_split(hipStream_t s, const RowsArgs &a, int n_cu) {
+static hipError_t rows_split(hipStream_t s, const RowsArgs &a, int n_cu, const RowsMore &m) {
     const int64_t most = rows_most(a, PRO, n_cu);
     auto steps = [&](int u) { return rows_steps(a, PRO, u); };
     auto grid = [&](int u) { return rows_grid(a, PRO, n_cu, u); };
@@ -42,37 +54,43 @@ static hipError_t rows_split(hipStream_t s, const RowsArgs &a, int n_cu) {
     // 8.8 in steps of 1 KB); rows of up to 1024 inputs whole (3072 x 768: 3.5 us against 4.8 in two steps).  A pending update of
     // more than 4096 elements takes the registers of the long steps.
     if constexpr (!(Y && V > 2))
-        if (a.ld >= 2048 && steps(4) >= most * ROWS_WAVES / 2) return rows_launch<PRO, EPI, 4, V, Y>(s, a, grid(4));
-    if (a.ld > 512 && (steps(2) >= most * ROWS_WAVES / 2 || (a.ld <= 1024 && steps(2) >= n_cu))) return rows_launch<PRO, EPI, 2, V, Y>(s, a, grid(2));
-    return rows_launch<PRO, EPI, 1, V, Y>(s, a, grid(1));
+        if (a.ld >= 2048 && steps(4) >= most * ROWS_WAVES / 2) return rows_launch<PRO, EPI, 4, V, Y>(s, a, grid(4), m);
+    if (a.ld > 512 && (steps(2) >= most * ROWS_WAVES / 2 || (a.ld <= 1024 && steps(2) >= n_cu))) return rows_launch<PRO, EPI, 2, V, Y>(s, a, grid(2), m);
+    return rows_launch<PRO, EPI, 1, V, Y>(s, a, grid(1), m);
 }
 
 // the vector's registers: two steps for up to 4096 elements behind a norm, four for more; eight for one that is staged as it is
 template <int PRO, int EPI>
-static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu) {
+static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu, const RowsMore &m) {
     if constexpr (PRO == RP_PLAIN || PRO == RP_DOWN) {
-        return rows_split<PRO, EPI, 8, false>(s, a, n_cu);
+        return rows_split<PRO, EPI, 8, false>(s, a, n_cu, m);
     } else if constexpr (PRO == RP_HEADNORM) {
-        return rows_split<PRO, EPI, 4, false>(s, a, n_cu);
+        return rows_split<PRO, EPI, 4, false>(s, a, n_cu, m);
     } else {
         const bool few = a.K <= 2 * 4 * ROWS_THREADS;
         if constexpr (PRO == RP_NORM && (EPI == RE_STORE || EPI == RE_STORE_GLU)) {
-            if (a.y) return few ? rows_split<PRO, EPI, 2, true>(s, a, n_cu) : rows_split<PRO, EPI, 4, true>(s, a, n_cu);
+            if (a.y) return few ? rows_split<PRO, EPI, 2, true>(s, a, n_cu, m) : rows_split<PRO, EPI, 4, true>(s, a, n_cu, m);
         }
         if (a.y) return hipErrorInvalidValue;
-        return few ? rows_split<PRO, EPI, 2, false>(s, a, n_cu) : rows_split<PRO, EPI, 4, false>(s, a, n_cu);
+        return few ? rows_split<PRO, EPI, 2, false>(s, a, n_cu, m) : rows_split<PRO, EPI, 4, false>(s, a, n_cu, m);
     }
 }
 
-hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu) {
+hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, const RowsMore &more) {
     if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.ld % 64 != 0 || a.K > a.ld || a.K < 1) return hipErrorInvalidValue;
     if ((pro == RP_UP || pro == RP_DOWN) &&
         (!a.z || a.n_experts < 1 || a.n_experts > ROWS_MAX_EXPERTS || a.top < 1 || a.top > ROWS_MAX_TOP || a.top > a.n_experts))
         return hipErrorInvalidValue;
     if ((epi == RE_GLU && a.n_rows % 2 != 0) || (epi == RE_STORE_GLU && (a.n_rows % 2 != 0 || a.glu_from % 2 != 0 || !a.out2)))
         return hipErrorInvalidValue;
+    RowsMore m = more;
+    if (m.stride || m.plus || m.plus2) {
+        if (epi != RE_RESID || (m.stride && pro == RP_DOWN)) return hipErrorInvalidValue;
+        epi = RE_RESID_MORE;
+    }
+    if (!m.stride) m.stride = a.ld;
 #define GO(P, E) \
-    if (pro == P && epi == E) return rows_pick<P, E>(s, a, n_cu)
+    if (pro == P && epi == E) return rows_pick<P, E>(s, a, n_cu, m)
     GO(RP_NORM, RE_STORE);
     GO(RP_NORM, RE_ACT);
     GO(RP_PLAIN, RE_STORE);
@@ -83,6 +101,9 @@ hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu) 
     GO(RP_NORM, RE_STORE_GLU);
     GO(RP_UP, RE_GLU);
     GO(RP_DOWN, RE_RESID);
+    GO(RP_PLAIN, RE_RESID_MORE);
+    GO(RP_DOWN, RE_RESID_MORE);
+    GO(RP_HEADNORM, RE_RESID_MORE);
     GO(RP_HEADNORM, RE_RESID);
 #undef GO
     return hipErrorInvalidValue;

@@ -317,28 +317,26 @@ __device__ __forceinline__ void step_latent_body(const LatentStep &a, int b, Ste
 
 // workgroups below n_first: the attention; the others: rows
 template <int PRO, int U>
-__global__ __launch_bounds__(ROWS_THREADS, 4) void step_latent_kernel(LatentStep a, RowsArgs r, RowsPlan pl, int n_first) {
+__global__ __launch_bounds__(ROWS_THREADS, 4) void step_latent_kernel(LatentStep a, RowsArgs r, RowsPlan pl, RowsMore m, int n_first) {
     extern __shared__ __align__(16) float s_mem[];
     if ((int)blockIdx.x < n_first) {
         step_latent_body(a, blockIdx.x, *(StepLds *)s_mem);
         return;
     }
-    __shared__ RowsShared sh;
-    rows_body<PRO, RE_RESID, U, 8, false>(r, pl, (int)blockIdx.x - n_first, s_mem, sh);
+    rows_body<PRO, RE_RESID_MORE, U, 8, false>(r, pl, (int)blockIdx.x - n_first, s_mem, m);
 }
 // workgroups below n_first: the queries, `each` workgroups a head, of which the last takes the head's query on; the others: rows
 template <int PRO, int U>
 __global__ __launch_bounds__(ROWS_THREADS, 4) void step_pair_kernel(LatentStep a, RowsArgs q, RowsPlan plq, int each, RowsArgs r, RowsPlan pl, int n_first) {
     extern __shared__ __align__(16) float s_mem[];
-    __shared__ RowsShared sh;
     const int b = blockIdx.x;
     if (b >= n_first) {
-        rows_body<PRO, RE_GLU, U, 2, false>(r, pl, b - n_first, s_mem, sh);
+        rows_body<PRO, RE_GLU, U, 2, false>(r, pl, b - n_first, s_mem);
         return;
     }
     // (a head's workgroups are those of its number among eight, as in the next launch: workgroups go to the XCDs in turn)
     const int h = b % a.w.H, j = b / a.w.H;
-    rows_body<RP_NORM, RE_STORE_AGENT, 2, 2, false>(q, plq, h * each + j, s_mem, sh);
+    rows_body<RP_NORM, RE_STORE_AGENT, 2, 2, false>(q, plq, h * each + j, s_mem);
     StepLds &s = *(StepLds *)s_mem;
     const bool last = step_last(a.count + a.w.H + h, (unsigned)each, &s.last);
     if (!last || each == 1) step_warm(a, h, each == 1 ? 0 : j, each);
@@ -394,16 +392,18 @@ hipError_t k_step_pair(hipStream_t s, const LatentStep &a, const RowsArgs &uq, c
     return hipErrorInvalidValue;
 }
 
-hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &down, int pro, int n_cu) {
+hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &down, int64_t stride, int pro, int n_cu) {
     const int u = step_u(down), n_first = a.w.H * a.splits;
     if (a.splits < 1 || a.splits > L_STEP_SPLITS) return hipErrorInvalidValue;
     const int64_t n = step_grid(down, pro, n_cu, u, std::min(a.w.H, n_cu / 2));
     const RowsPlan pl = rows_plan(down, pro, u, n);
+    RowsMore m;
+    m.stride = stride ? stride : down.ld;
     const size_t lds = std::max(sizeof(StepLds), rows_lds(down, pro, pl.pairs + 1));
     if (lds > 64 * 1024) return hipErrorInvalidValue;
 #define GO(P, U_)                                                                                                                        \
     if (pro == P && u == U_) {                                                                                                           \
-        hipLaunchKernelGGL((step_latent_kernel<P, U_>), dim3((unsigned)(n_first + n)), dim3(ROWS_THREADS), lds, s, a, down, pl, n_first); \
+        hipLaunchKernelGGL((step_latent_kernel<P, U_>), dim3((unsigned)(n_first + n)), dim3(ROWS_THREADS), lds, s, a, down, pl, m, n_first); \
         return hipGetLastError();                                                                                                        \
     }
     GO(RP_PLAIN, 4)

@@ -790,6 +790,7 @@ static hipError_t step_latent(l2h_model *m, const LayerDev &L, const LayerRun &r
 struct LatentLayerStep {
     RowsArgs uq, up, down, o;
     int up_pro, down_pro;
+    int64_t stride = 0;  // from row to row of `down` and `o` (0: their ld)
 };
 static void set_router(RowsArgs &a, const LayerDev &L, const float *z) {
     a.z = z;
@@ -814,7 +815,7 @@ static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int c
     a.o = rows_of(L.o, l->mix, x);
     if (L.joined) {  // a row of the output matrix goes on as one of the feed-forward's
         a.o.K = a.o.ld = L.o_cols;
-        a.o.stride = a.down.stride = L.o.ld;
+        a.stride = L.o.ld;
         a.down.w += L.o_cols;
         a.down.K = d.ff_dim;
         a.down.ld = L.o.ld - L.o_cols;
@@ -841,8 +842,8 @@ int layered_shared_steps(l2h_model *m) {
 }
 
 // Mixer and feed-forward of a layer, a launch each; `in` reads the norm of the stream x into the mixer's projected row
-// (`plus`, `plus2`: what the next layer's pass of a loop adds to the stream, in the launch that completes it)
-static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x, const float *plus, const float *plus2) {
+// (`plus`: what the next layer's pass of a loop adds to the stream, in the launch that completes it)
+static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &run, RowsArgs in, float *x, const RowsMore &plus) {
     Layered *l = m->lay;
     hipStream_t s = m->ctx->stream;
     const int cu = m->ctx->prop.multiProcessorCount;
@@ -878,8 +879,8 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
         o_pro = RP_HEADNORM;
     }
     const bool o_last = d.ff == L2H_FF_NONE || (d.ff == L2H_FF_DENSE && L.joined);
-    if (o_last) o.plus = plus, o.plus2 = plus2;
-    if (!early || d.ff == L2H_FF_NONE || (L.stacked() && L.joined)) CK(k_rows(s, o, o_pro, RE_RESID, cu));
+    const RowsMore o_plus = o_last ? plus : RowsMore();
+    if (!early || d.ff == L2H_FF_NONE || (L.stacked() && L.joined)) CK(k_rows(s, o, o_pro, RE_RESID, cu, o_plus));
     if (d.ff != L2H_FF_NONE && !(L.stacked() && L.joined)) {
         RowsArgs up = rows_of(L.up, x, l->hid), down = rows_of(L.down, l->hid, x);
         up.normw = early ? L.norm1 : L.norm2;
@@ -887,13 +888,11 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
         up.act = d.ff_act;
         down.resid = x;
         down.mult = c.residual_mult;
-        down.plus = plus;
-        down.plus2 = plus2;
         if (d.ff == L2H_FF_DENSE) {
             if (L.joined) up.out = l->mix + L.o_cols;
             if (!L.stacked()) CK(k_rows(s, up, RP_NORM, d.ff_gated ? RE_GLU : RE_ACT, cu));
-            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
-            if (!L.joined) CK(k_rows(s, down, RP_PLAIN, RE_RESID, cu));
+            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu, o_plus));
+            if (!L.joined) CK(k_rows(s, down, RP_PLAIN, RE_RESID, cu, plus));
         } else {
             RowsArgs r = rows_of(L.router, x, l->z);
             r.normw = up.normw;
@@ -905,8 +904,8 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
             down.rows_each = c.width;
             down.n_rows = c.width;
             CK(k_rows(s, up, RP_UP, d.ff_gated ? RE_GLU : RE_UP, cu));
-            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu));
-            CK(k_rows(s, down, RP_DOWN, RE_RESID, cu));
+            if (early) CK(k_rows(s, o, o_pro, RE_RESID, cu, o_plus));
+            CK(k_rows(s, down, RP_DOWN, RE_RESID, cu, plus));
         }
     }
     return hipSuccess;
@@ -934,7 +933,9 @@ hipError_t layered_enqueue_token(l2h_model *m) {
         }
         added = next && next->pass >= 0 && !c.side_dim;
         const float *step = added ? l->loop_step + (int64_t)next->pass * c.width : nullptr, *again = added && next->pass ? l->x0 : nullptr;
-        const float *plus = again ? again : step, *plus2 = again ? step : nullptr;
+        RowsMore plus;
+        plus.plus = again ? again : step;
+        plus.plus2 = again ? step : nullptr;
         RowsArgs in = st.normed(L.in, L.norm1, l->in);
         float *x = st.x;
         LatentLayerStep shared;
@@ -945,12 +946,11 @@ hipError_t layered_enqueue_token(l2h_model *m) {
             const LatentStep a = {w, L.freq, l->lq, l->qa, L.ukv.w, L.ukv.ld, l->in, L.kvnorm, run.kc, l->part, l->count, l->mix,
                                   L.joined ? L.o_cols : w.H * w.V, m->ctl, L_STEP_SPLITS};
             CK(k_step_pair(s, a, shared.uq, shared.up, shared.up_pro, cu));
-            CK(k_step_latent(s, a, shared.down, shared.down_pro, cu));
-            shared.o.plus = plus;
-            shared.o.plus2 = plus2;
-            CK(k_rows(s, shared.o, RP_PLAIN, RE_RESID, cu));
+            CK(k_step_latent(s, a, shared.down, shared.stride, shared.down_pro, cu));
+            plus.stride = shared.stride;
+            CK(k_rows(s, shared.o, RP_PLAIN, RE_RESID, cu, plus));
         } else {
-            CK(separate_launches(m, L, run, in, x, plus, plus2));
+            CK(separate_launches(m, L, run, in, x, plus));
         }
         if (c.side_dim) {
             RowsArgs g = rows_of(L.side_gate, x, l->se);

@@ -33,12 +33,11 @@ enum { RP_PLAIN = 0, RP_NORM = 1, RP_UP = 2, RP_DOWN = 3, RP_HEADNORM = 4 };
 // epilogues: RE_STORE v; RE_RESID resid + mult * v; RE_ACT act(v); RE_UP act(score * v) or score * act(v) with the expert's score;
 // RE_EMBED act(v) * the token's row of an embedding table; RE_GLU rows 2 i and 2 i + 1 give out[i] = act(v) * v', with the
 // expert's score behind RP_UP; RE_STORE_GLU stores rows below glu_from and treats the others so, into out2; RE_STORE_AGENT v, past the
-// caches of the storing workgroup
-enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6, RE_STORE_AGENT = 7 };
+// caches of the storing workgroup; RE_RESID_MORE as RE_RESID, with a RowsMore (k_rows takes it where one of its fields is set)
+enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6, RE_STORE_AGENT = 7, RE_RESID_MORE = 8 };
 struct RowsArgs {
     const uint16_t *w = nullptr;
     int ld = 0, K = 0;
-    int64_t stride = 0;  // from row to row (0: ld); not for RP_UP, RP_DOWN
     int64_t n_rows = 0;
     const float *x = nullptr;
     float *out = nullptr;
@@ -47,7 +46,6 @@ struct RowsArgs {
     const float *y = nullptr, *yw = nullptr;
     float *x_out = nullptr;
     const float *resid = nullptr;
-    const float *plus = nullptr, *plus2 = nullptr;  // RE_RESID: vectors added to the sum, one after the other
     int act = 0;
     int64_t glu_from = 0;
     float *out2 = nullptr;
@@ -61,7 +59,13 @@ struct RowsArgs {
     const DecodeCtl *ctl = nullptr;
     const int32_t *prompt = nullptr;
 };
-hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu);
+// What few products of a residual have.  Apart, for the sake of the others: with these fields and their branches in every launch a token of Vudelix took 1 % longer
+// (width 768, 4 layers: 170.6 us against 169.2).
+struct RowsMore {
+    int64_t stride = 0;                             // from row to row (0: ld); not for RP_DOWN
+    const float *plus = nullptr, *plus2 = nullptr;  // vectors added to the sum, one after the other
+};
+hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, const RowsMore &more = RowsMore());
 
 // ---- many tokens: C[m][n] = sum_k X[m][k] W[n][k] (k_gemm.hip) ---------------------------------------------------
 // activations are bf16 (prec 0) or fp32 (prec 1: fp32 products on the matrix cores); ldx a multiple of 64, zero from K on
@@ -299,5 +303,5 @@ bool k_step_fits(const LatentShape &w, int ldu, const RowsArgs &uq, const RowsAr
                  int n_cu);
 // uq: RP_NORM, the rows of the projected queries, then a.qa and the token's cache row from them; up: pro (RP_NORM or RP_UP), RE_GLU
 hipError_t k_step_pair(hipStream_t s, const LatentStep &a, const RowsArgs &uq, const RowsArgs &up, int pro, int n_cu);
-// down: pro (RP_PLAIN or RP_DOWN), RE_RESID
-hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &down, int pro, int n_cu);
+// down: pro (RP_PLAIN or RP_DOWN), RE_RESID; stride: from row to row of it (0: its ld)
+hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &down, int64_t stride, int pro, int n_cu);

@@ -62,20 +62,13 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
 //
 // V: steps of four elements a thread in which the vector is requested; Y: with a pending update.  b: the workgroup's number among the
 // product's; s_mem: rows_lds() bytes.
-struct RowsShared {
-    float red[2][ROWS_WAVES];
-    float part[ROWS_WAVES][2];
-    int head[ROWS_WAVES];  // the pair that `part` belongs to
-    int sel[ROWS_MAX_TOP];
-    float score[ROWS_MAX_TOP];
-};
 template <int PRO, int EPI, int U, int V, bool Y>
-__device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl, int b, float *s_mem, RowsShared &sh) {
-    auto &s_red = sh.red;
-    auto &s_part = sh.part;
-    auto &s_head = sh.head;
-    auto &s_sel = sh.sel;
-    auto &s_score = sh.score;
+__device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl, int b, float *s_mem, const RowsMore &m = RowsMore()) {
+    __shared__ float s_red[2][ROWS_WAVES];
+    __shared__ float s_part[ROWS_WAVES][2];
+    __shared__ int s_head[ROWS_WAVES];  // the pair that s_part belongs to
+    __shared__ int s_sel[ROWS_MAX_TOP];
+    __shared__ float s_score[ROWS_MAX_TOP];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int K = a.K, ld = a.ld, plane = pl.plane;
     const int nvec = PRO == RP_DOWN ? a.top : 1;  // vectors staged, each in its own 2 * plane floats
@@ -85,6 +78,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     // (four elements a thread and step)
     const bool quads = K % 4 == 0 && (PRO != RP_HEADNORM || a.hv % 4 == 0);
     const bool fast = quads && nvec * K <= 4 * V * ROWS_THREADS;
+    constexpr bool more = EPI == RE_RESID_MORE, resid = EPI == RE_RESID || more;
     constexpr bool as_is = PRO == RP_PLAIN || PRO == RP_DOWN;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 x[V], w[as_is ? 1 : V], g[PRO == RP_HEADNORM ? V : 1], y[Y ? V : 1], yw[Y ? V : 1];
@@ -121,10 +115,10 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     // (of the row whose result this thread writes first)
     float before = 0.0f;
     float plus = 0.0f, plus2 = 0.0f;
-    if (EPI == RE_RESID && row0 + t < row_end) {
-        before = a.resid[row0 + t];
-        if (a.plus) plus = a.plus[row0 + t];
-        if (a.plus2) plus2 = a.plus2[row0 + t];
+    if (resid && row0 + t < row_end) before = a.resid[row0 + t];
+    if (more && row0 + t < row_end) {
+        if (m.plus) plus = m.plus[row0 + t];
+        if (m.plus2) plus2 = m.plus2[row0 + t];
     }
     if (EPI == RE_EMBED && row0 + t < row_end) before = l_bf16(a.emb[(int64_t)l_step_token(a.ctl, a.prompt) * a.emb_ld + row0 + t]);
     asm volatile("" ::: "memory");
@@ -144,8 +138,9 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
             w0 = a.w + ((int64_t)s_sel[v] * a.rows_each + r) * ld;
             w1 = a.w + ((int64_t)s_sel[v] * a.rows_each + r1) * ld;
         } else {
-            w0 = a.w + r * pl.stride;
-            w1 = a.w + r1 * pl.stride;
+            const int64_t stride = more ? m.stride : ld;
+            w0 = a.w + r * stride;
+            w1 = a.w + r1 * stride;
         }
     };
     RowsChunk cur[U], nxt[U];
@@ -341,10 +336,10 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
             continue;
         }
         float o = val;
-        if (EPI == RE_RESID) {
-            o = (i == t ? before : a.resid[r]) + a.mult * val;
-            if (a.plus) o += i == t ? plus : a.plus[r];
-            if (a.plus2) o += i == t ? plus2 : a.plus2[r];
+        if (resid) o = (i == t ? before : a.resid[r]) + a.mult * val;
+        if (more) {
+            if (m.plus) o += i == t ? plus : m.plus[r];
+            if (m.plus2) o += i == t ? plus2 : m.plus2[r];
         }
         if (EPI == RE_ACT) o = l_act(a.act, val);
         if (EPI == RE_UP) o = a.route == LROUTE_SIGMOID_IN ? l_act(a.act, f * val) : f * l_act(a.act, val);

@@ -42,7 +42,6 @@ struct RowsPlan {
     int plane;              // half of a staged vector's floats
     int pairs, more;
     int per_vec, per_pair;  // steps of a row pair per staged vector, in all
-    int64_t stride;         // from row to row
 };
 inline RowsPlan rows_plan(const RowsArgs &a, int pro, int u, int64_t grid) {
     const int64_t pairs = (a.n_rows + 1) / 2;
@@ -52,6 +51,5 @@ inline RowsPlan rows_plan(const RowsArgs &a, int pro, int u, int64_t grid) {
     pl.more = (int)(pairs % grid);
     pl.per_vec = (a.ld + 512 * u - 1) / (512 * u);
     pl.per_pair = rows_vectors(a, pro) * pl.per_vec;
-    pl.stride = a.stride ? a.stride : a.ld;
     return pl;
 }
