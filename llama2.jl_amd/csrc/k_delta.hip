@@ -10,19 +10,25 @@
 // ---------------------------------------------------------------------------------------------------------------
 #define CONV_AHEAD 4  // taps whose inputs are fetched together
 
+// What a channel's convolution reads: its projection, the taps' weights and the ring's slots.  No load is skipped (a slot or weight that is not
+// used is read all the same, and replaced by zero in the sum).
+struct DeltaConv {
+    float cur, w[CONV_AHEAD], x[CONV_AHEAD];  // (x[0] is not read: it is cur)
+};
+__device__ __forceinline__ void delta_conv_weights(DeltaConv &v, const float *conv, const float *in, int C, int taps, int ch) {
+    v.cur = in[ch];
+#pragma unroll
+    for (int j = 0; j < CONV_AHEAD; j++) v.w[j] = conv[(int64_t)max(taps - 1 - j, 0) * C + ch];
+}
+__device__ __forceinline__ void delta_conv_ring(DeltaConv &v, const float *ring, int C, int taps, int ch, int now) {
+#pragma unroll
+    for (int j = 1; j < CONV_AHEAD; j++) v.x[j] = ring[(int64_t)(j < taps ? (now - j < 0 ? now - j + taps : now - j) : 0) * C + ch];
+}
 // the channel's convolution at `pos`: cur is its projection, ring slot `now` = pos % taps will hold it
-__device__ __forceinline__ float delta_conv(const float *conv, const float *ring, int C, int taps, float cur, int ch, int pos, int now) {
-    float w[CONV_AHEAD], x[CONV_AHEAD];
+__device__ __forceinline__ float delta_conv(const DeltaConv &c, const float *conv, const float *ring, int C, int taps, int ch, int pos) {
+    float v = c.w[0] * c.cur;
 #pragma unroll
-    for (int j = 0; j < CONV_AHEAD; j++) {
-        const bool use = j < taps && j <= pos;
-        const int slot = now - j < 0 ? now - j + taps : now - j;
-        w[j] = use ? conv[(int64_t)(taps - 1 - j) * C + ch] : 0.0f;
-        x[j] = j == 0 ? cur : use ? ring[(int64_t)slot * C + ch] : 0.0f;
-    }
-    float v = 0.0f;
-#pragma unroll
-    for (int j = 0; j < CONV_AHEAD; j++) v = fmaf(w[j], x[j], v);
+    for (int j = 1; j < CONV_AHEAD; j++) v = j < taps && j <= pos ? fmaf(c.w[j], c.x[j], v) : v;
     for (int j = CONV_AHEAD; j < taps && j <= pos; j++)
         v = fmaf(conv[(int64_t)(taps - 1 - j) * C + ch], ring[(int64_t)((pos - j) % taps) * C + ch], v);
     return l_silu(v);
@@ -46,80 +52,101 @@ __device__ __forceinline__ float delta_sum8(float acc) {
     return acc;
 }
 
+// sum over the wavefront, in every lane: the rows of sixteen lanes without LDS
+__device__ __forceinline__ float delta_wave_sum(float v) {
+    v = l_dpp_add<0x121>(l_dpp_add<0x122>(l_dpp_add<0x124>(l_dpp_add<0x128>(v))));  // row_ror: 8, 4, 2, 1
+    v += __shfl_xor(v, 16, WAVE);
+    return v + __shfl_xor(v, 32, WAVE);
+}
+
+// What bounds this is latency: 56 KB a workgroup (a fifth of a microsecond's worth of HBM for all of them) behind a chain of three sums.  So everything is
+// requested at once, in the order in which it is used, no load skipped by lanes (which makes the compiler wait for all of them), and
+// the barriers order LDS traffic only, so that the state is still on its way while the convolutions and decays are formed.  q and k stay as the
+// convolutions leave them; what makes them unit vectors is a factor on the sums.  32 heads of 128 x 128,
+// 128 workgroups: 8.1 us; with conditional loads, full barriers and rows dealt out one by one (48 LDS reads a thread where these are 12) 11.3.
 // NR: rows of S per thread (D <= 8 NR)
 template <int NR>
 __global__ __launch_bounds__(256) void delta_step_kernel(DeltaShape d, DeltaWeights w, const float *in, float *ring, float *state,
                                                          const DecodeCtl *ctl, float *o, float *ssq, float *gate, int n_split) {
     extern __shared__ __align__(16) float s_mem[];
     float *s_q = s_mem, *s_k = s_q + 8 * NR, *s_g = s_k + 8 * NR, *s_fa = s_g + 8 * NR, *s_fg = s_fa + w.lda2;
-    __shared__ float s_v[L_DELTA_COLS], s_red[2][8][L_DELTA_COLS], s_kq;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    __shared__ float s_v[L_DELTA_COLS], s_red[2][8][L_DELTA_COLS], s_unit[3];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int sp = blockIdx.x, h = blockIdx.y, kvh = h / (d.H / d.G), pos = ctl->pos;
-    const int D = d.D, V = d.V, c0 = sp * L_DELTA_COLS, GD = d.G * D;
+    const int D = d.D, V = d.V, c0 = sp * L_DELTA_COLS, GD = d.G * D, C = d.channels();
     const int col = t & 31, rg = t >> 5, c = c0 + col;
     const bool live = c < V;
-    float *S = state + (int64_t)h * D * V;
-    float s[NR];
+    // ---- requests: convolutions, factors, state ----
+    // channels t + 256 ii of the 2 D of q and k, then the workgroup's columns of v (the last one again beyond them)
+    constexpr int NC = (16 * NR + L_DELTA_COLS + 255) / 256;
+    const int n_ch = 2 * D + min(L_DELTA_COLS, V - c0);
+    DeltaConv cv[NC];
+    int ch[NC];
 #pragma unroll
-    for (int i = 0; i < NR; i++) {
-        const int r = rg + 8 * i;
-        s[i] = (live && r < D && pos > 0) ? S[(int64_t)r * V + c] : 0.0f;
+    for (int ii = 0; ii < NC; ii++) {
+        const int i = min(t + 256 * ii, n_ch - 1), e = i >= 2 * D ? i - 2 * D : i >= D ? i - D : i;
+        ch[ii] = i >= 2 * D ? 2 * GD + h * V + c0 + e : (i >= D ? GD : 0) + kvh * D + e;
+        if (256 * ii + 64 * wave < n_ch) delta_conv_weights(cv[ii], w.conv, in, C, d.taps, ch[ii]);
     }
-    // the first 128 inputs of the low-rank factors' rows are fetched ahead
+    // (the low-rank factors' inputs; longer ones in a loop below)
+    float xa = 0.0f, xg = 0.0f;
+    if (64 * wave < w.lda2) xa = in[d.off_a() + min(t, d.ra - 1)];
+    if (64 * wave < w.ldg2) xg = in[d.off_g() + min(t, d.rg - 1)];
+    const int now = pos % d.taps;
+#pragma unroll
+    for (int ii = 0; ii < NC; ii++)
+        if (256 * ii + 64 * wave < n_ch) delta_conv_ring(cv[ii], ring, C, d.taps, ch[ii], now);
+    // the first 128 inputs of the factors' rows
     const int l8 = t & 7, r8 = t >> 3;
     uint4 fa[NR / 4][2], fg[2];
     float bias[NR / 4];
     const float rate = w.rate[h], beta = l_sigmoid(in[d.off_b() + h]);
 #pragma unroll
-    for (int i = 0; i < NR / 4; i++) bias[i] = r8 + 32 * i < D ? w.bias[h * D + r8 + 32 * i] : 0.0f;
+    for (int i = 0; i < NR / 4; i++) {
+        const int64_t r = (int64_t)h * D + min(r8 + 32 * i, D - 1);
+        bias[i] = w.bias[r];
 #pragma unroll
-    for (int i = 0; i < NR / 4; i++)
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const int r = r8 + 32 * i, kk = 8 * l8 + 64 * e;
-            fa[i][e] = make_uint4(0, 0, 0, 0);
-            if (r < D && kk < w.lda2) fa[i][e] = *(const uint4 *)(w.a2 + ((int64_t)h * D + r) * w.lda2 + kk);
-        }
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const int kk = 8 * l8 + 64 * e;
-        fg[e] = make_uint4(0, 0, 0, 0);
-        if (c0 + r8 < V && kk < w.ldg2) fg[e] = *(const uint4 *)(w.g2 + ((int64_t)h * V + c0 + r8) * w.ldg2 + kk);
+        for (int e = 0; e < 2; e++) fa[i][e] = *(const uint4 *)(w.a2 + r * w.lda2 + min(8 * l8 + 64 * e, w.lda2 - 8));
     }
-    // short convolutions; the token's own projections go into the ring (its slot is not read by this token)
-    const int C = d.channels(), now = pos % d.taps;
+    const uint16_t *row_g = w.g2 + ((int64_t)h * V + min(c0 + r8, V - 1)) * w.ldg2;
+#pragma unroll
+    for (int e = 0; e < 2; e++) fg[e] = *(const uint4 *)(row_g + min(8 * l8 + 64 * e, w.ldg2 - 8));
+    float *S = state + (int64_t)h * D * V;
+    float s[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) s[i] = S[(int64_t)min(NR * rg + i, D - 1) * V + min(c, V - 1)];
+    asm volatile("" ::: "memory");
+    // ---- short convolutions; the token's own projections go into the ring (its slot is not read by this token) ----
     float *slot = ring + (int64_t)now * C;
 #pragma unroll
-    for (int ii = 0; ii < (16 * NR + L_DELTA_COLS + 255) / 256; ii++) {
+    for (int ii = 0; ii < NC; ii++) {
         const int i = t + 256 * ii;
-        if (i >= 2 * D + L_DELTA_COLS) break;
-        const bool isv = i >= 2 * D, isk = !isv && i >= D;
-        const int e = isv ? i - 2 * D : isk ? i - D : i;
-        if (isv && c0 + e >= V) {
-            s_v[e] = 0.0f;
-            continue;
+        if (256 * ii + 64 * wave >= n_ch) break;
+        const float y = delta_conv(cv[ii], w.conv, ring, C, d.taps, ch[ii], pos);
+        if (i < n_ch) {
+            if (i >= 2 * D)
+                s_v[i - 2 * D] = y;
+            else if (i >= D)
+                s_k[i - D] = y;
+            else
+                s_q[i] = y;
+            if (i >= 2 * D || (sp == 0 && h % (d.H / d.G) == 0)) slot[ch[ii]] = cv[ii].cur;
         }
-        const int ch = isv ? 2 * GD + h * V + c0 + e : (isk ? GD : 0) + kvh * D + e;
-        const float cur = in[ch], y = delta_conv(w.conv, ring, C, d.taps, cur, ch, pos, now);
-        if (isv)
-            s_v[e] = y;
-        else if (isk)
-            s_k[e] = y;
-        else
-            s_q[e] = y;
-        if (isv || (sp == 0 && h % (d.H / d.G) == 0)) slot[ch] = cur;
     }
-    for (int i = t; i < w.lda2; i += 256) s_fa[i] = i < d.ra ? in[d.off_a() + i] : 0.0f;
-    for (int i = t; i < w.ldg2; i += 256) s_fg[i] = i < d.rg ? in[d.off_g() + i] : 0.0f;
-    __syncthreads();
-    // unit vectors (one wavefront each), then k . q
-    if (wave < 2) {
-        float *x = wave ? s_k : s_q;
+    if (t < w.lda2) s_fa[t] = t < d.ra ? xa : 0.0f;
+    if (t < w.ldg2) s_fg[t] = t < d.rg ? xg : 0.0f;
+    for (int i = t + 256; i < w.lda2; i += 256) s_fa[i] = i < d.ra ? in[d.off_a() + i] : 0.0f;
+    for (int i = t + 256; i < w.ldg2; i += 256) s_fg[i] = i < d.rg ? in[d.off_g() + i] : 0.0f;
+    l_lds_barrier();
+    // ---- what makes unit vectors of q and k, and k . q: a wavefront each ----
+    if (wave < 3) {
+        const float *x = wave == 0 ? s_q : s_k, *y = wave == 1 ? s_k : s_q;
         float ss = 0.0f;
-        for (int e = lane; e < D; e += 64) ss = fmaf(x[e], x[e], ss);
-        float r = 1.0f / sqrtf(l_wave_sum(ss) + 1e-6f);
-        if (wave == 0) r *= 1.0f / sqrtf((float)D);
-        for (int e = lane; e < D; e += 64) x[e] *= r;
+        for (int e = lane; e < D; e += 64) ss = fmaf(x[e], y[e], ss);
+        ss = delta_wave_sum(ss);
+        if (wave < 2) ss = 1.0f / sqrtf(ss + 1e-6f);
+        if (wave == 0) ss *= 1.0f / sqrtf((float)D);
+        if (lane == 0) s_unit[wave] = ss;
     }
     // decays of all key channels, gates of this workgroup's columns
 #pragma unroll
@@ -136,46 +163,45 @@ __global__ __launch_bounds__(256) void delta_step_kernel(DeltaShape d, DeltaWeig
         if (l8 == 0) s_g[r] = expf(-rate * l_softplus(z));
     }
     if (c0 + r8 < V) {
-        const uint16_t *row = w.g2 + ((int64_t)h * V + c0 + r8) * w.ldg2;
         float z = 0.0f;
 #pragma unroll
         for (int e = 0; e < 2; e++)
             if (8 * l8 + 64 * e < w.ldg2) z = delta_fma8(fg[e], s_fg + 8 * l8 + 64 * e, z);
-        for (int kk = 8 * l8 + 128; kk < w.ldg2; kk += 64) z = delta_fma8(*(const uint4 *)(row + kk), s_fg + kk, z);
+        for (int kk = 8 * l8 + 128; kk < w.ldg2; kk += 64) z = delta_fma8(*(const uint4 *)(row_g + kk), s_fg + kk, z);
         z = delta_sum8(z);
         if (l8 == 0) gate[h * V + c0 + r8] = l_sigmoid(z);
     }
-    __syncthreads();
-    if (wave == 0) {
-        float kq = 0.0f;
-        for (int e = lane; e < D; e += 64) kq = fmaf(s_k[e], s_q[e], kq);
-        kq = l_wave_sum(kq);
-        if (lane == 0) s_kq = kq;
-    }
-    float dk = 0.0f, dq = 0.0f;
+    l_lds_barrier();
+    const float uq = s_unit[0], uk = s_unit[1], kq = s_unit[2] * uq * uk;
+    float dk = 0.0f, dq = 0.0f, k[NR];
 #pragma unroll
-    for (int i = 0; i < NR; i++) {
-        const int r = rg + 8 * i;
-        if (r < D) {
-            s[i] *= s_g[r];
-            dk = fmaf(s[i], s_k[r], dk);
-            dq = fmaf(s[i], s_q[r], dq);
+    for (int i = 0; i < NR; i += 4) {
+        const int r = NR * rg + i;
+        const float4 g4 = *(const float4 *)(s_g + r), k4 = *(const float4 *)(s_k + r), q4 = *(const float4 *)(s_q + r);
+        const float g[4] = {g4.x, g4.y, g4.z, g4.w}, q[4] = {q4.x, q4.y, q4.z, q4.w};
+        k[i] = k4.x, k[i + 1] = k4.y, k[i + 2] = k4.z, k[i + 3] = k4.w;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const bool has = pos > 0 && r + j < D;  // (beyond D the words of LDS are anything)
+            s[i + j] = has ? s[i + j] * g[j] : 0.0f;
+            dk = has ? fmaf(s[i + j], k[i + j], dk) : dk;
+            dq = has ? fmaf(s[i + j], q[j], dq) : dq;
         }
     }
     s_red[0][rg][col] = dk;
     s_red[1][rg][col] = dq;
-    __syncthreads();
+    l_lds_barrier();
     dk = dq = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         dk += s_red[0][i][col];
         dq += s_red[1][i][col];
     }
-    const float u = beta * (s_v[col] - dk), ov = fmaf(s_kq, u, dq);
+    const float u = live ? beta * (s_v[col] - uk * dk) : 0.0f, ov = fmaf(kq, u, uq * dq), uu = uk * u;
 #pragma unroll
     for (int i = 0; i < NR; i++) {
-        const int r = rg + 8 * i;
-        if (live && r < D) S[(int64_t)r * V + c] = fmaf(s_k[r], u, s[i]);
+        const int r = NR * rg + i;
+        if (live && r < D) S[(int64_t)r * V + c] = fmaf(k[i], uu, s[i]);
     }
     if (rg == 0) {  // (the low half of wavefront 0)
         float ss = live ? ov * ov : 0.0f;
