@@ -965,10 +965,7 @@ static hipError_t enqueue_token(l2h_model *m) {
         e = (call);                    \
         if (e != hipSuccess) return e; \
     } while (0)
-    if (m->lay) {
-        CK(layered_enqueue_token(m));
-        return k_argmax(s, m->logits, c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, true);
-    }
+    if (m->lay) return layered_enqueue_token(m);
     // token embedding (:236) and this position's RoPE table
     CK(k_embed(s, m->glob[L2H_TOK_EMB], m->ctl, m->prompt_dev, m->x, m->rope_cs, m->hs, m->theta_scale));
     for (int l = 0; l < c.n_layers; l++) {
@@ -1016,7 +1013,7 @@ static int loop_buffers(l2h_model *m) {
 #define DA(p, n, z)                       \
     if ((rc = dalloc(m, &(p), (n), (z)))) \
         return rc;
-    DA(m->ctl, 1, true);
+    DA(m->ctl, 2, true);  // (the second: a layered model's steps hand the first on through it)
     DA(m->prompt_dev, m->c.seq_len, true);
     m->max_out = m->c.seq_len;
     DA(m->out_tokens, m->max_out, true);
@@ -1162,6 +1159,13 @@ static int run_steps(l2h_model *m, int n) {
     return L2H_OK;
 }
 
+// what is left to do behind the last of `n` steps
+static int last_token(l2h_model *m, int n) {
+    if (!m->lay || n < 1) return L2H_OK;
+    HIPCHK(m->ctx, layered_pick_token(m));
+    return L2H_OK;
+}
+
 // after the stream has drained: did a workgroup of the persistent kernel give up at a barrier?
 static int mega_check(l2h_model *m) {
     if (m->flow) {
@@ -1274,8 +1278,9 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     h.n_prompt = n_prompt;
     h.last_argmax = 0;
     h.n_out = 0;
+    const DecodeCtl both[2] = {h, h};
     HIPCHK(ctx, hipMemcpyAsync(m->prompt_dev, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(m->ctl, &h, sizeof h, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(m->ctl, both, sizeof both, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     if (m->lay && total > 0) layered_advance(m, pos0 + total);
     DeviceTurn turn(m);
@@ -1287,6 +1292,7 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
         if (he == hipSuccess) rc = run_steps(m, total - n_new);
         if (he == hipSuccess && rc == L2H_OK) he = hipEventRecord(e0, ctx->stream);
         if (he == hipSuccess && rc == L2H_OK) rc = run_steps(m, n_new);
+        if (he == hipSuccess && rc == L2H_OK) rc = last_token(m, total);
         if (he == hipSuccess && rc == L2H_OK) he = hipEventRecord(e1, ctx->stream);
         if (he == hipSuccess && rc == L2H_OK) he = hipEventSynchronize(e1);
         if (he == hipSuccess && rc == L2H_OK) he = hipEventElapsedTime(decode_ms, e0, e1);
@@ -1295,7 +1301,7 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
         if (rc) return rc;
         if (he != hipSuccess) return set_err(ctx, L2H_EHIP, "timing the decode steps failed: %s", hipGetErrorString(he));
     } else {
-        if ((rc = run_steps(m, total))) return rc;
+        if ((rc = run_steps(m, total)) || (rc = last_token(m, total))) return rc;
     }
     if (n_new > 0)
         HIPCHK(ctx, hipMemcpyAsync(out, m->out_tokens, (size_t)n_new * 4, hipMemcpyDeviceToHost, ctx->stream));

@@ -115,3 +115,11 @@ __device__ __forceinline__ float dequant_elem(const DevTensor &t, int64_t row, i
     const float d = half_bits_to_float(t.d6[blk]);
     return d * (float)(sc * q);
 }
+
+// keys of an argmax: order by value, then by lower index
+__device__ __forceinline__ unsigned long long argmax_key(float v, uint32_t idx) {
+    uint32_t b = __float_as_uint(v);
+    b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    if (v == 0.0f) b = 0x80000000u;  // -0.0 and +0.0 compare equal
+    return ((unsigned long long)b << 32) | (unsigned long long)(0xFFFFFFFFu - idx);
+}

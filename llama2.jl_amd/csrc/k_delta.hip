@@ -59,7 +59,7 @@ __device__ __forceinline__ float delta_wave_sum(float v) {
     return v + __shfl_xor(v, 32, WAVE);
 }
 
-// What bounds this is latency: 56 KB a workgroup (a fifth of a microsecond's worth of HBM for all of them) behind a chain of three sums.  So everything is
+// What bounds this is latency: 56 KB a workgroup (1.2 us of HBM in all) in front of a chain of three sums.  So everything is
 // requested at once, in the order in which it is used, no load skipped by lanes (which makes the compiler wait for all of them), and
 // the barriers order LDS traffic only, so that the state is still on its way while the convolutions and decays are formed.  q and k stay as the
 // convolutions leave them; what makes them unit vectors is a factor on the sums.  32 heads of 128 x 128,

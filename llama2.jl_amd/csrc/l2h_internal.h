@@ -60,7 +60,8 @@ struct DecodeCtl {
     int32_t n_prompt;   // prompt length of the generate call
     int32_t last_argmax;
     int32_t n_out;      // number of generated ids written so far
-    int32_t pad[2];
+    int32_t picks;      // in the copy that a layered model's step leaves: its keys are there, the token is to be picked
+    int32_t pad;
 };
 
 // One matvec launch covers up to 3 weight matrices of one type that consume the same input
@@ -258,6 +259,9 @@ hipError_t k_softmax(hipStream_t s, float *x, int64_t n);
 // step: of the token loop (launch sequences that are recorded)
 hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, DecodeCtl *ctl, int32_t *out_tokens,
                     int max_out, bool step);
+hipError_t k_argmax_keys(hipStream_t s, const unsigned long long *keys, int n, DecodeCtl *ctl, int32_t *out_tokens, int max_out);
+hipError_t k_step_begin(hipStream_t s, const DevTensor &emb, const DecodeCtl *prev, DecodeCtl *ctl, const unsigned long long *keys, int n_keys,
+                        const int32_t *prompt, int32_t *out_tokens, int max_out, float *x, float scale, float *x_copy);
 // argmax without allocations: k_noalloc_init once per device (that device current), then k_argmax_noalloc
 hipError_t k_noalloc_init(int device);
 hipError_t k_argmax_noalloc(hipStream_t s, int device, const float *x_dev, int64_t n, int32_t *out_dev);

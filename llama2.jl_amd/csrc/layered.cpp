@@ -54,6 +54,8 @@ struct Layered {
     float *x_alt = nullptr, *in = nullptr, *mix = nullptr, *ssq = nullptr, *gate = nullptr, *hid = nullptr, *z = nullptr,
           *se = nullptr, *y = nullptr, *part = nullptr, *x0 = nullptr, *lq = nullptr, *qa = nullptr;
     unsigned *count = nullptr;  // k_step_latent's, zero between launches
+    unsigned long long *keys = nullptr;  // the classifier's, a key for each of its workgroups
+    int n_keys = 0;
     // prompt pass, for `cap` positions
     int cap = 0;
     int32_t *tok = nullptr, *choice = nullptr, *slot_row = nullptr, *slot_of = nullptr, *n_tiles = nullptr, *want = nullptr;
@@ -595,6 +597,8 @@ static float **run_state(LayerRun &r, int k) {
     return p[k];
 }
 
+static RowsArgs rows_of(const LMat &w, const float *x, float *out);
+
 int layered_finalize(l2h_model *m) {
     l2h_ctx *ctx = m->ctx;
     Layered *l = m->lay;
@@ -682,6 +686,10 @@ int layered_finalize(l2h_model *m) {
     DA(l->z, ne, true);
     DA(l->se, std::max(1, c.side_dim), true);
     DA(l->y, c.width, true);
+    RowsArgs head = rows_of(l->head, m->x, m->logits);
+    head.y = c.side_dim ? l->y : nullptr;  // (what the last layer leaves pending)
+    l->n_keys = k_rows_workgroups(head, RP_NORM, ctx->prop.multiProcessorCount);
+    DA(l->keys, l->n_keys, true);
     DA(l->part, part, true);
     DA(m->rope_cs, 2, true);
     DA(m->logits, c.vocab_size, true);
@@ -918,7 +926,7 @@ hipError_t layered_enqueue_token(l2h_model *m) {
     const l2h_layered_config &c = l->c;
     hipError_t e;
     Stream st(m);
-    CK(k_embed(s, m->glob[L2H_TOK_EMB], m->ctl, m->prompt_dev, st.x, m->rope_cs, 0, 1.0f, c.embed_scale, l->x0));
+    CK(k_step_begin(s, m->glob[L2H_TOK_EMB], m->ctl + 1, m->ctl, l->keys, l->n_keys, m->prompt_dev, m->out_tokens, m->max_out, st.x, c.embed_scale, l->x0));
     // What a pass of a loop begins with, x += [x0] + step, is added by the launch that completes the stream before it (a launch of its own: 4.5 us of
     // a 280 us token twice) unless that is the embedding's or a pending update comes in between.
     bool added = false;
@@ -964,8 +972,16 @@ hipError_t layered_enqueue_token(l2h_model *m) {
             st.yw = L.side_norm;
         }
     }
-    CK(k_rows(s, st.normed(l->head, l->final_norm, m->logits), RP_NORM, RE_STORE, cu));
-    return hipSuccess;
+    RowsKeys keys;
+    keys.keys = l->keys;
+    keys.ctl = m->ctl;
+    keys.next = m->ctl + 1;
+    return k_rows_keys(s, st.normed(l->head, l->final_norm, m->logits), cu, keys);
+}
+
+// behind the last step of a call: its token
+hipError_t layered_pick_token(l2h_model *m) {
+    return k_argmax_keys(m->ctx->stream, m->lay->keys, m->lay->n_keys, m->ctl, m->out_tokens, m->max_out);
 }
 
 // ------------------------------------------------------------------------------------------

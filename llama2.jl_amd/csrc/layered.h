@@ -33,8 +33,9 @@ enum { RP_PLAIN = 0, RP_NORM = 1, RP_UP = 2, RP_DOWN = 3, RP_HEADNORM = 4 };
 // epilogues: RE_STORE v; RE_RESID resid + mult * v; RE_ACT act(v); RE_UP act(score * v) or score * act(v) with the expert's score;
 // RE_EMBED act(v) * the token's row of an embedding table; RE_GLU rows 2 i and 2 i + 1 give out[i] = act(v) * v', with the
 // expert's score behind RP_UP; RE_STORE_GLU stores rows below glu_from and treats the others so, into out2; RE_STORE_AGENT v, past the
-// caches of the storing workgroup; RE_RESID_MORE as RE_RESID, with a RowsMore (k_rows takes it where one of its fields is set)
-enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6, RE_STORE_AGENT = 7, RE_RESID_MORE = 8 };
+// caches of the storing workgroup; RE_RESID_MORE as RE_RESID, with a RowsMore (k_rows takes it where one of its fields is set); RE_STORE_KEY v, and a
+// workgroup's largest (k_rows_keys)
+enum { RE_STORE = 0, RE_RESID = 1, RE_ACT = 2, RE_UP = 3, RE_EMBED = 4, RE_GLU = 5, RE_STORE_GLU = 6, RE_STORE_AGENT = 7, RE_RESID_MORE = 8, RE_STORE_KEY = 9 };
 struct RowsArgs {
     const uint16_t *w = nullptr;
     int ld = 0, K = 0;
@@ -66,6 +67,15 @@ struct RowsMore {
     const float *plus = nullptr, *plus2 = nullptr;  // vectors added to the sum, one after the other
 };
 hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, const RowsMore &more = RowsMore());
+// A step's classifier: as RP_NORM, RE_STORE; each of its k_rows_workgroups() workgroups also leaves the key (argmax_key) of its first largest row, and the
+// first of them `ctl` in `next`, marked: what the next step's k_step_begin picks the token from.
+struct RowsKeys {
+    unsigned long long *keys = nullptr;
+    const DecodeCtl *ctl = nullptr;
+    DecodeCtl *next = nullptr;
+};
+int k_rows_workgroups(const RowsArgs &a, int pro, int n_cu);
+hipError_t k_rows_keys(hipStream_t s, const RowsArgs &a, int n_cu, const RowsKeys &keys);
 
 // ---- many tokens: C[m][n] = sum_k X[m][k] W[n][k] (k_gemm.hip) ---------------------------------------------------
 // activations are bf16 (prec 0) or fp32 (prec 1: fp32 products on the matrix cores); ldx a multiple of 64, zero from K on

@@ -68,6 +68,23 @@ template <int CTRL>
 __device__ __forceinline__ float l_dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
+template <int CTRL>
+__device__ __forceinline__ unsigned long long l_dpp_max(unsigned long long v) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, 0xF, 0xF, true);
+    const unsigned long long o = (unsigned long long)hi << 32 | lo;
+    return o > v ? o : v;
+}
+// the largest of the wavefront's, in every lane
+__device__ __forceinline__ unsigned long long l_wave_max(unsigned long long v) {
+    v = l_dpp_max<0x121>(l_dpp_max<0x122>(l_dpp_max<0x124>(l_dpp_max<0x128>(v))));  // row_ror: 8, 4, 2, 1
+#pragma unroll
+    for (int m = 16; m <= 32; m <<= 1) {
+        const unsigned long long o = __shfl_xor(v, m, WAVE);
+        v = o > v ? o : v;
+    }
+    return v;
+}
 // sum over the workgroup; `red` holds one float per wavefront; every thread gets the total
 __device__ __forceinline__ float l_block_sum(float v, float *red) {
     const int nw = (blockDim.x + 63) >> 6;

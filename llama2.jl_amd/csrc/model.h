@@ -121,7 +121,8 @@ int layered_finalize(l2h_model *m);             // checks the tensors, allocates
 int layered_reset(l2h_model *m);
 int layered_check_pos(l2h_model *m, int pos0);  // may a call start at pos0?
 void layered_advance(l2h_model *m, int pos);    // the state now holds positions 0 .. pos - 1
-hipError_t layered_enqueue_token(l2h_model *m);  // embedding to logits
+hipError_t layered_enqueue_token(l2h_model *m);  // the token that the step before left to be picked, embedding to logits
+hipError_t layered_pick_token(l2h_model *m);     // behind the last step of a call
 hipError_t layered_output(l2h_model *m);         // m->x -> m->logits
 int layered_prefill_buffers(l2h_model *m, int cap, int n_want);
 int layered_capacity(l2h_model *m);

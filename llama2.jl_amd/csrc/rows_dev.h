@@ -63,7 +63,8 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
 // V: steps of four elements a thread in which the vector is requested; Y: with a pending update.  b: the workgroup's number among the
 // product's; s_mem: rows_lds() bytes.
 template <int PRO, int EPI, int U, int V, bool Y>
-__device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl, int b, float *s_mem, const RowsMore &m = RowsMore()) {
+__device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl, int b, float *s_mem, const RowsMore &m = RowsMore(),
+                                          const RowsKeys &keys = RowsKeys()) {
     __shared__ float s_red[2][ROWS_WAVES];
     __shared__ float s_part[ROWS_WAVES][2];
     __shared__ int s_head[ROWS_WAVES];  // the pair that s_part belongs to
@@ -80,6 +81,8 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     const bool fast = quads && nvec * K <= 4 * V * ROWS_THREADS;
     constexpr bool more = EPI == RE_RESID_MORE, resid = EPI == RE_RESID || more;
     constexpr bool as_is = PRO == RP_PLAIN || PRO == RP_DOWN;
+    DecodeCtl ctl;
+    if (EPI == RE_STORE_KEY && b == 0) ctl = *keys.ctl;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 x[V], w[as_is ? 1 : V], g[PRO == RP_HEADNORM ? V : 1], y[Y ? V : 1], yw[Y ? V : 1];
     if (Y && fast) {
@@ -311,6 +314,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     l_lds_barrier();
 
     // ---- results: a thread per row -------------------------------------------------------------------------------------
+    unsigned long long best = 0;
     for (int i = t; row0 + i < row_end; i += ROWS_THREADS) {
         const int64_t r = row0 + i;
         const bool glu = EPI == RE_GLU || (EPI == RE_STORE_GLU && r >= a.glu_from);  // (whole pairs)
@@ -349,5 +353,26 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
             __hip_atomic_store(a.out + r, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else
             a.out[r] = o;
+        if (EPI == RE_STORE_KEY) {
+            const unsigned long long key = argmax_key(o, (uint32_t)r);
+            best = key > best ? key : best;
+        }
+    }
+    if constexpr (EPI == RE_STORE_KEY) {
+        __shared__ unsigned long long s_best[ROWS_WAVES];
+        best = l_wave_max(best);
+        if (row_end - row0 > 64) {  // (up to 64 rows are the first wavefront's)
+            if (lane == 0) s_best[wave] = best;
+            l_lds_barrier();
+#pragma unroll
+            for (int i = 0; i < ROWS_WAVES; i++) best = s_best[i] > best ? s_best[i] : best;
+        }
+        if (t == 0) {
+            keys.keys[b] = best;
+            if (b == 0) {
+                ctl.picks = 1;
+                *keys.next = ctl;
+            }
+        }
     }
 }
