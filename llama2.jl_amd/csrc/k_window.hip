@@ -240,141 +240,177 @@ hipError_t k_window_prepare(hipStream_t s, const WindowShape &w, const float *fr
     return hipGetLastError();
 }
 
-// fp32 attention: workgroup = one head x WR_Q queries, keys in tiles of WR_K; a wavefront owns WR_Q / 4 queries, its lanes
-// the keys of a tile, then the value columns.  A CU gets about one workgroup of it, so latency bounds it: the key elements are
-// requested WR_U words at a time and the values of a tile before its scores, which are formed without a barrier (8 heads of 128,
-// 509 queries, all before them in the window: 181 us with one load after the other, 97 us like this)
-#define WR_Q 16
-#define WR_K 64
-#define WR_U 8
+// fp32 attention on the fp32 matrix cores: workgroup = one head x 16 queries, its wavefronts take the tiles of 16 keys in turn, each with a softmax of
+// its own; they join at the end.  v_mfma_f32_16x16x4_f32: lane l has A[l % 16][l / 16], B[l / 16][l % 16] and, of the result, rows
+// 4 (l / 16) + r in register r, column l % 16.  Scores are keys x queries, so that a lane has four keys of one query, which is the next product's B
+// operand as it stands; that product is value columns x queries, row i of its tile j being column 4 i + j of a group of 64: a lane's
+// operand for four tiles is one word of 16 bytes of a key's values, and its results are 16 neighbouring columns of one query.
+// What bounds it is the matrix cores' 2 x 32 cycles for every four elements of a head, on the CU whose queries see the most keys, and the loads
+// ahead of them: a tile's values are requested before its scores are formed and the next tile's keys behind them.  8 heads of 128, 509 queries, all before
+// them in the window: 26 us; with a key a lane and the products on the vector units 94.
+// N: groups of 64 elements of a head (key and value elements up to 64 N); NW: wavefronts
 typedef float wr_f32x4 __attribute__((ext_vector_type(4)));
-template <int PREC>
-__global__ __launch_bounds__(256) void window_rows_kernel(WindowShape w, const float *qf, const float *raw, int64_t ldr, const float *kc,
-                                                          const float *vc, int M, int pos0, void *outa, int64_t lda) {
-    extern __shared__ __align__(16) float s_mem[];
-    constexpr int QW = WR_Q / 4;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int h = blockIdx.y, q0 = blockIdx.x * WR_Q, D = w.D, Dp = w.Dp(), V = w.V, D4 = Dp / 4;
-    const int g = h / (w.H / w.G);
-    float *s_q = s_mem, *s_v = s_q + WR_Q * Dp, *s_p = s_v + WR_K * V;
-    const int64_t krow = (int64_t)g * D4 * w.seq_len;
-    for (int i = t; i < WR_Q * Dp; i += 256) {
-        const int q = i / Dp, e = i - q * Dp;
-        s_q[i] = (q0 + q < M && e < D) ? qf[((int64_t)(q0 + q) * w.H + h) * D + e] : 0.0f;
+#define WR_Q 16
+template <int PREC, int N, int NW>
+__global__ __launch_bounds__(64 * NW) void window_rows_kernel(WindowShape w, const float *qf, const float *raw, int64_t ldr, const float *kc,
+                                                              const float *vc, int M, int pos0, void *outa, int64_t lda) {
+    constexpr int DT = 4 * N;
+    __shared__ __align__(16) wr_f32x4 s_o[NW / 2][4 * N][64];
+    __shared__ float s_m[NW / 2][64], s_l[NW / 2][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
+    // (the blocks that see the most keys first)
+    const int h = blockIdx.y, q0 = (int)(gridDim.x - 1 - blockIdx.x) * WR_Q, D = w.D, V = w.V, D4 = w.Dp() / 4, g = h / (w.H / w.G);
+    const int last = pos0 + min(q0 + WR_Q, M) - 1, first = max(0, pos0 + q0 - w.window + 1), qp = pos0 + q0 + col;
+    const float *kbase = kc + (int64_t)g * D4 * w.seq_len * 4, *vbase = vc + (int64_t)g * w.seq_len * V;
+    wr_f32x4 q[DT], k[DT], v[4][N], acc[N][4];
+    auto fetch_keys = [&](int k0) {  // (a key that is not there repeats the last one; elements beyond the head, the head's last ones)
+        const float *p = kbase + (int64_t)min(k0 + col, last) * 4;
+#pragma unroll
+        for (int i = 0; i < DT; i++) k[i] = *(const wr_f32x4 *)(p + (int64_t)min(4 * i + quad, D4 - 1) * w.seq_len * 4);
+    };
+    const bool v4 = V % 4 == 0;
+    auto fetch_values = [&](int k0) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float *p = vbase + (int64_t)min(k0 + 4 * quad + r, last) * V;
+#pragma unroll
+            for (int n = 0; n < N; n++) {
+                const int c = 64 * n + 4 * col;
+                if (v4)
+                    v[r][n] = *(const wr_f32x4 *)(p + min(c, V - 4));
+                else
+                    v[r][n] = wr_f32x4{p[min(c, V - 1)], p[min(c + 1, V - 1)], p[min(c + 2, V - 1)], p[min(c + 3, V - 1)]};
+            }
+        }
+    };
+    int k0 = first + 16 * wave;
+    if (k0 <= last) fetch_keys(k0);
+    {
+        const float *p = qf + ((int64_t)min(q0 + col, M - 1) * w.H + h) * D;
+#pragma unroll
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int e = 16 * i + 4 * quad + r;
+                const float x = p[min(e, D - 1)];
+                q[i][r] = e < D ? x : 0.0f;
+            }
     }
-    __syncthreads();
-    float mrun[QW], lrun[QW], acc[QW][4];  // V <= 256: four columns per lane
+    float mrun = -INFINITY, lrun = 0.0f;  // of query `col`: the same in the four lanes that have it
 #pragma unroll
-    for (int a = 0; a < QW; a++) {
-        mrun[a] = -INFINITY;
-        lrun[a] = 0.0f;
+    for (int n = 0; n < N; n++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = 0.0f;
-    }
-    const int last = pos0 + min(q0 + WR_Q, M) - 1, first = max(0, pos0 + q0 - w.window + 1);
-    for (int k0 = first; k0 <= last; k0 += WR_K) {
-        const int n = min(WR_K, last + 1 - k0);
-        const float *vsrc = vc + ((int64_t)g * w.seq_len + k0) * V;
-        const int nq = V % 4 == 0 ? n * V / 4 : 0;  // (a row of values then begins on 16 bytes)
-        wr_f32x4 vq[WR_U];
-        if (nq) {
+        for (int j = 0; j < 4; j++) acc[n][j] = wr_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (; k0 <= last; k0 += 16 * NW) {
+        fetch_values(k0);
+        wr_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
-            for (int u = 0; u < WR_U; u++) vq[u] = *(const wr_f32x4 *)(vsrc + 4 * min(t + 256 * u, nq - 1));
+        for (int i = 0; i < DT; i++) {
+            if (4 * i >= D4) break;
+            const bool has = 4 * i + quad < D4;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float kr = has ? k[i][r] : 0.0f;
+                if (i & 1)
+                    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr, q[i][r], s1, 0, 0, 0);
+                else
+                    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr, q[i][r], s0, 0, 0, 0);
+            }
         }
-        float sc[QW];
+        if (k0 + 16 * NW <= last) fetch_keys(k0 + 16 * NW);
+        float x[4], mx = mrun;
 #pragma unroll
-        for (int a = 0; a < QW; a++) sc[a] = 0.0f;
-        const float *kp = kc + (krow + k0 + min(lane, n - 1)) * 4;
-        for (int i0 = 0; i0 < D4; i0 += WR_U) {
-            float4 kv[WR_U];
-#pragma unroll
-            for (int u = 0; u < WR_U; u++) kv[u] = *(const float4 *)(kp + (int64_t)min(i0 + u, D4 - 1) * w.seq_len * 4);
-#pragma unroll
-            for (int u = 0; u < WR_U; u++)
-                if (i0 + u < D4) {
-#pragma unroll
-                    for (int a = 0; a < QW; a++) {
-                        const float4 qv = *(const float4 *)(s_q + (wave * QW + a) * Dp + 4 * (i0 + u));
-                        sc[a] = fmaf(qv.x, kv[u].x, sc[a]);
-                        sc[a] = fmaf(qv.y, kv[u].y, sc[a]);
-                        sc[a] = fmaf(qv.z, kv[u].z, sc[a]);
-                        sc[a] = fmaf(qv.w, kv[u].w, sc[a]);
-                    }
-                }
+        for (int r = 0; r < 4; r++) {
+            const int key = k0 + 4 * quad + r;
+            x[r] = key <= qp && qp - key < w.window && key <= last ? (s0[r] + s1[r]) * w.scale : -INFINITY;
+            mx = fmaxf(mx, x[r]);
         }
-        if (k0 != first) __syncthreads();  // (everyone is through with the values of the tile before)
-        if (nq) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        const float alpha = mx == -INFINITY ? 1.0f : expf(mrun - mx);
+        float sum = 0.0f;
 #pragma unroll
-            for (int u = 0; u < WR_U; u++)
-                if (t + 256 * u < nq) *(wr_f32x4 *)(s_v + 4 * (t + 256 * u)) = vq[u];
-            for (int i = t + 256 * WR_U; i < nq; i += 256) *(float4 *)(s_v + 4 * i) = *(const float4 *)(vsrc + 4 * i);
-        } else {
-            for (int i = t; i < n * V; i += 256) s_v[i] = vsrc[i];
+        for (int r = 0; r < 4; r++) {
+            x[r] = x[r] == -INFINITY ? 0.0f : expf(x[r] - mx);
+            sum += x[r];
         }
-        __syncthreads();
+        mrun = mx;
+        lrun = lrun * alpha + sum;  // (this lane's keys; joined at the end)
 #pragma unroll
-        for (int a = 0; a < QW; a++) {
-            const int qp = pos0 + q0 + wave * QW + a, key = k0 + lane;
-            const bool see = lane < n && key <= qp && qp - key < w.window;
-            const float v = see ? sc[a] * w.scale : -INFINITY;
-            const float mnew = fmaxf(mrun[a], wave_max_f32(v));
-            const float alpha = mnew == -INFINITY ? 1.0f : expf(mrun[a] - mnew);
-            const float p = see ? expf(v - mnew) : 0.0f;
-            s_p[(wave * QW + a) * WR_K + lane] = p;
-            lrun[a] = lrun[a] * alpha + l_wave_sum(p);
-            mrun[a] = mnew;
+        for (int n = 0; n < N; n++) {
+            if (64 * n >= V) break;
 #pragma unroll
-            for (int b = 0; b < 4; b++) acc[a][b] *= alpha;
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int i = 0; i < n; i += 4) {  // (a key that is not there has p = 0; its values are those of the last one)
-            const float *v0 = s_v + i * V, *v1 = s_v + min(i + 1, n - 1) * V, *v2 = s_v + min(i + 2, n - 1) * V, *v3 = s_v + min(i + 3, n - 1) * V;
+            for (int j = 0; j < 4; j++) {
+                acc[n][j] *= alpha;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int c = lane + 64 * b;
-                if (c < V) {
-                    const float x0 = v0[c], x1 = v1[c], x2 = v2[c], x3 = v3[c];
-#pragma unroll
-                    for (int a = 0; a < QW; a++) {
-                        const float4 p = *(const float4 *)(s_p + (wave * QW + a) * WR_K + i);
-                        acc[a][b] = fmaf(p.x, x0, acc[a][b]);
-                        acc[a][b] = fmaf(p.y, x1, acc[a][b]);
-                        acc[a][b] = fmaf(p.z, x2, acc[a][b]);
-                        acc[a][b] = fmaf(p.w, x3, acc[a][b]);
-                    }
-                }
+                for (int r = 0; r < 4; r++) acc[n][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[r][n][j], x[r], acc[n][j], 0, 0, 0);
             }
         }
     }
+    lrun += __shfl_xor(lrun, 16, WAVE);
+    lrun += __shfl_xor(lrun, 32, WAVE);
+    // ---- the wavefronts' sums joined, half of them onto the other half ----
 #pragma unroll
-    for (int a = 0; a < QW; a++) {
-        const int m = q0 + wave * QW + a;
-        if (m >= M) continue;
-        float f = 1.0f / lrun[a];
-        if (w.gated) f *= l_sigmoid(raw[(int64_t)m * ldr + w.off_g() + h]);
+    for (int half = NW / 2; half >= 1; half >>= 1) {
+        if (wave >= half && wave < 2 * half) {
+            s_m[wave - half][lane] = mrun;
+            s_l[wave - half][lane] = lrun;
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int c = lane + 64 * b;
-            if (c < V) l_store_act<PREC>(outa, m * lda + h * V + c, acc[a][b] * f);
+            for (int n = 0; n < N; n++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) s_o[wave - half][4 * n + j][lane] = acc[n][j];
         }
-        if (h == w.H - 1)
-            for (int64_t j = (int64_t)w.H * V + lane; j < lda; j += 64) l_store_act<PREC>(outa, m * lda + j, 0.0f);
+        __syncthreads();
+        if (wave < half) {
+            const float mo = s_m[wave][lane], mx = fmaxf(mrun, mo);
+            const float fa = mrun == -INFINITY ? 0.0f : expf(mrun - mx), fb = mo == -INFINITY ? 0.0f : expf(mo - mx);
+            mrun = mx;
+            lrun = lrun * fa + s_l[wave][lane] * fb;
+#pragma unroll
+            for (int n = 0; n < N; n++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[n][j] = acc[n][j] * fa + s_o[wave][4 * n + j][lane] * fb;
+        }
+        __syncthreads();
     }
+    const int m = q0 + col;
+    if (wave > 0 || m >= M) return;
+    float f = 1.0f / lrun;
+    if (w.gated) f *= l_sigmoid(raw[(int64_t)m * ldr + w.off_g() + h]);
+#pragma unroll
+    for (int n = 0; n < N; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int c = 64 * n + 16 * quad + 4 * r + j;
+                if (c < V) l_store_act<PREC>(outa, m * lda + h * V + c, acc[n][j][r] * f);
+            }
+    if (h == w.H - 1)
+        for (int64_t j = (int64_t)w.H * V + quad; j < lda; j += 4) l_store_act<PREC>(outa, m * lda + j, 0.0f);
 }
 hipError_t k_window_rows(hipStream_t s, const WindowShape &w, const float *qf, const float *raw, int64_t ldr, const float *kc,
                          const float *vc, int M, int pos0, void *outa, int64_t lda, int prec) {
-    if (w.V > 256 || pos0 < 0 || pos0 + M > w.seq_len) return hipErrorInvalidValue;
-    const size_t lds = (size_t)(WR_Q * w.Dp() + WR_K * w.V + WR_Q * WR_K) * sizeof(float);
-    if (lds > 120 * 1024) return hipErrorInvalidValue;
+    if (w.V > 256 || w.D > 256 || pos0 < 0 || M < 1 || pos0 + M > w.seq_len) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((M + WR_Q - 1) / WR_Q), (unsigned)w.H);
-    const void *f = prec ? (const void *)window_rows_kernel<1> : (const void *)window_rows_kernel<0>;
-    if (lds > 48 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
+    const int n = (std::max(w.Dp(), w.V) + 63) / 64;
+#define GO(P, N, NW) hipLaunchKernelGGL((window_rows_kernel<P, N, NW>), grid, dim3(64 * NW), 0, s, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda)
+    if (n == 1) {
+        if (prec)
+            GO(1, 1, 8);
+        else
+            GO(0, 1, 8);
+    } else if (n == 2) {
+        if (prec)
+            GO(1, 2, 8);
+        else
+            GO(0, 2, 8);
+    } else {
+        if (prec)
+            GO(1, 4, 4);
+        else
+            GO(0, 4, 4);
     }
-    if (prec)
-        hipLaunchKernelGGL((window_rows_kernel<1>), grid, dim3(256), lds, s, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda);
-    else
-        hipLaunchKernelGGL((window_rows_kernel<0>), grid, dim3(256), lds, s, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda);
+#undef GO
     return hipGetLastError();
 }
