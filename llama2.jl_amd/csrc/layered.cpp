@@ -1225,12 +1225,9 @@ static hipError_t prompt_delta(l2h_model *m, LayerDev &L, const LayerRun &run, i
     a.hd = d.D;
     CK(k_gemm(s, a, prec, GE_DECAY));
     CK(product(m, gemm_of(L.g2, l->fg, M), GE_SIGMOID, l->gt, hv, 1.0f));
-    if (M >= L_DELTA_WALK_MIN)
-        CK(k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->ob));
-    else
-        CK(k_delta_scan(s, d, l->qkv, l->kq, l->beta, l->lg, run.state, M, pos0, l->ob));
-    CK(k_head_norm_rows(s, l->ob, l->gt, L.mixnorm, M, d.H, d.V, d.eps, l->ao, L.o.ld, prec));
-    return hipSuccess;
+    if (M >= L_DELTA_WALK_MIN) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
+    CK(k_delta_scan(s, d, l->qkv, l->kq, l->beta, l->lg, run.state, M, pos0, l->ob));
+    return k_head_norm_rows(s, l->ob, l->gt, L.mixnorm, M, d.H, d.V, d.eps, l->ao, L.o.ld, prec);
 }
 
 static hipError_t prompt_attention(l2h_model *m, LayerDev &L, const LayerRun &run, int M, int pos0) {

@@ -198,17 +198,17 @@ struct DeltaWeights {
 hipError_t k_delta_step(hipStream_t s, const DeltaShape &d, const DeltaWeights &w, const float *in, float *ring, float *state,
                         const DecodeCtl *ctl, float *o, float *ssq, float *gate);
 // convolution, silu, unit vectors, beta: raw[M][ldr] -> qkv[M][channels], kq[M][G] (= k . q), beta[M][H], and the two low-rank
-// factors as activations; qkv and the scan's o have room for a multiple of 16 rows
+// factors as activations
 hipError_t k_delta_prepare(hipStream_t s, const DeltaShape &d, const float *conv, const float *raw, int64_t ldr, const float *ring,
                            int M, int pos0, float *qkv, float *kq, float *beta, void *fa, int64_t lfa, void *fg, int64_t lfg,
                            int prec);
 // the recurrence over M tokens, logarithms of the decays in lg[M][H D]; o[M][H V]; then the ring takes the last tokens
 hipError_t k_delta_scan(hipStream_t s, const DeltaShape &d, const float *qkv, const float *kq, const float *beta, const float *lg,
                         float *state, int M, int pos0, float *o);
-// the same in chunks of 16 tokens on the matrix cores; rec: delta_walk_floats(d, M) floats of scratch
+// the same in chunks of 32 tokens on the matrix cores, with k_head_norm_rows behind it; rec: delta_walk_floats(d, M) floats of scratch
 int64_t delta_walk_floats(const DeltaShape &d, int M);
 hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M,
-                        int pos0, float *rec, float *o);
+                        int pos0, float *rec, const float *gate, const float *normw, void *outa, int64_t lda, int prec);
 #define L_DELTA_WALK_MIN 24  // tokens from which the chunked form is used
 hipError_t k_delta_ring(hipStream_t s, const DeltaShape &d, const float *raw, int64_t ldr, float *ring, int M, int pos0);
 // outa[m][h V + j] = o * rms over the head * normw[j] * gate
