@@ -52,6 +52,22 @@ __device__ __forceinline__ float delta_sum8(float acc) {
     return acc;
 }
 
+// one of 16 sums over the 16 lanes of a row: lane l gets that of v[l].  Every step halves the sums: lanes l and 15 - l, l and 7 - l, l and l ^ 2, l and l ^ 1
+template <int CTRL>
+__device__ __forceinline__ float delta_swap_add(bool upper, float lo, float hi) {
+    return (upper ? hi : lo) + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(upper ? lo : hi), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float delta_sum16(const float (&v)[16], int l) {
+    float a[8], b[4], c[2];
+#pragma unroll
+    for (int i = 0; i < 8; i++) a[i] = delta_swap_add<0x140>(l & 8, v[i], v[i + 8]);  // row_mirror
+#pragma unroll
+    for (int i = 0; i < 4; i++) b[i] = delta_swap_add<0x141>(l & 4, a[i], a[i + 4]);  // row_half_mirror
+#pragma unroll
+    for (int i = 0; i < 2; i++) c[i] = delta_swap_add<0x4E>(l & 2, b[i], b[i + 2]);
+    return delta_swap_add<0xB1>(l & 1, c[0], c[1]);
+}
+
 // sum over the wavefront, in every lane: the rows of sixteen lanes without LDS
 __device__ __forceinline__ float delta_wave_sum(float v) {
     v = l_dpp_add<0x121>(l_dpp_add<0x122>(l_dpp_add<0x124>(l_dpp_add<0x128>(v))));  // row_ror: 8, 4, 2, 1
@@ -231,40 +247,52 @@ hipError_t k_delta_step(hipStream_t s, const DeltaShape &d, const DeltaWeights &
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// many tokens: convolutions and unit vectors.  A wavefront takes one unit (a key head's q and k, or a value head, or the
-// rest of the row) over PREP_T consecutive tokens.
+// many tokens: convolutions and unit vectors.  A wavefront takes one unit (a key head's q and k, or 64 columns of a value head, or the
+// rest of the row) over PREP_T consecutive tokens.  What bounds it is bytes, read and written once (the rows before a block of tokens from the L2), as
+// long as every unit has all its rows under way together and a wavefront's sums do not go through LDS one by one: 16 heads of 128, 2048 tokens, 100 MB
+// 32 us, against 38.
 // ---------------------------------------------------------------------------------------------------------------
 #define PREP_T 8
 
-// CONV_AHEAD - 1 + PREP_T inputs of a channel (tokens m0 - CONV_AHEAD + 1 .. m0 + PREP_T - 1) are fetched together, then the
-// convolution and silu of its PREP_T tokens; taps beyond CONV_AHEAD are added one by one
+// Offsets of the CONV_AHEAD - 1 + PREP_T rows that a block of tokens reads, from row m0 - CONV_AHEAD + 1 on; rows beyond M repeat the last one.
+struct PrepRows {
+    int64_t at[CONV_AHEAD - 1 + PREP_T];
+};
 __device__ __forceinline__ float delta_raw_at(const float *raw, int64_t ldr, const float *ring, int C, int taps, int ch, int m, int pos0) {
     if (m >= 0) return raw[(int64_t)m * ldr + ch];
     const int p = pos0 + m;
     return p >= 0 ? ring[(int64_t)(p % taps) * C + ch] : 0.0f;
 }
-__device__ __forceinline__ void delta_conv_rows(const float *conv, const float *raw, int64_t ldr, const float *ring, int C, int taps, int ch,
-                                                int m0, int M, int pos0, float (&y)[PREP_T]) {
+// A channel's inputs of a block of tokens, requested together
+struct PrepIn {
     float x[CONV_AHEAD - 1 + PREP_T], w[CONV_AHEAD];
-    const float *col = raw + ch;
+};
+__device__ __forceinline__ void delta_conv_request(PrepIn &v, const PrepRows &rows, const float *conv, const float *raw, int64_t ldr, const float *ring, int C,
+                                                   int taps, int ch, int m0, int M, int pos0) {
     if (m0 >= CONV_AHEAD - 1) {
+        const float *col = raw + (int64_t)(m0 - CONV_AHEAD + 1) * ldr + ch;
+        asm volatile("" : "+v"(col));  // (one address a lane: as a base a row, the compiler kept 335 scalars on the stack)
 #pragma unroll
-        for (int i = 0; i < CONV_AHEAD - 1 + PREP_T; i++) x[i] = col[(int64_t)min(m0 - CONV_AHEAD + 1 + i, M - 1) * ldr];
+        for (int i = 0; i < CONV_AHEAD - 1 + PREP_T; i++) v.x[i] = *(const __attribute__((address_space(1))) float *)(col + rows.at[i]);
     } else {
 #pragma unroll
         for (int i = 0; i < CONV_AHEAD - 1 + PREP_T; i++) {
             const int m = m0 - CONV_AHEAD + 1 + i;
             // (an input further back than the taps reach has left the ring: its weight is 0)
-            x[i] = (m >= 0 || -m < taps) ? delta_raw_at(raw, ldr, ring, C, taps, ch, min(m, M - 1), pos0) : 0.0f;
+            v.x[i] = (m >= 0 || -m < taps) ? delta_raw_at(raw, ldr, ring, C, taps, ch, min(m, M - 1), pos0) : 0.0f;
         }
     }
 #pragma unroll
-    for (int j = 0; j < CONV_AHEAD; j++) w[j] = j < taps ? conv[(int64_t)(taps - 1 - j) * C + ch] : 0.0f;
+    for (int j = 0; j < CONV_AHEAD; j++) v.w[j] = conv[(int64_t)max(taps - 1 - j, 0) * C + ch];
+}
+// the convolution and silu of a block's tokens; taps beyond CONV_AHEAD are added one by one
+__device__ __forceinline__ void delta_conv_rows(const PrepIn &in, const float *conv, const float *raw, int64_t ldr, const float *ring, int C, int taps, int ch,
+                                                int m0, int M, int pos0, float (&y)[PREP_T]) {
 #pragma unroll
     for (int i = 0; i < PREP_T; i++) {
         float v = 0.0f;
 #pragma unroll
-        for (int j = 0; j < CONV_AHEAD; j++) v = fmaf(w[j], x[i + CONV_AHEAD - 1 - j], v);
+        for (int j = 0; j < CONV_AHEAD; j++) v = j < taps ? fmaf(in.w[j], in.x[i + CONV_AHEAD - 1 - j], v) : v;
         y[i] = v;
     }
     for (int j = CONV_AHEAD; j < taps; j++) {
@@ -275,70 +303,118 @@ __device__ __forceinline__ void delta_conv_rows(const float *conv, const float *
 #pragma unroll
     for (int i = 0; i < PREP_T; i++) y[i] = l_silu(y[i]);
 }
+// sums over the wavefront of 16 values: lane l gets that of v[l % 16]
+__device__ __forceinline__ float delta_wave_sum16(const float (&v)[16], int lane) {
+    float s = delta_sum16(v, lane & 15);
+    s += __shfl_xor(s, 16, WAVE);
+    return s + __shfl_xor(s, 32, WAVE);
+}
 
 // NE: key channels per lane (D <= 64 NE)
 template <int PREC, int NE>
 __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaShape d, const float *conv, const float *raw, int64_t ldr,
                                                             const float *ring, int M, int pos0, float *qkv, float *kq, float *beta,
                                                             void *fa, int64_t lfa, void *fg, int64_t lfg) {
-    const int lane = threadIdx.x & 63;
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), n_units = d.G + d.H + 1;
-    const int m0 = blockIdx.y * PREP_T, m1 = min(m0 + PREP_T, M);
-    if (unit >= n_units) return;
+    const int lane = threadIdx.x & 63, nv = (d.V + 63) / 64;
+    const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = blockIdx.y * PREP_T, n = min(PREP_T, M - m0);
     const int C = d.channels(), GD = d.G * d.D, taps = d.taps;
-    if (unit == d.G + d.H) {  // beta and the low-rank factors
-        for (int m = m0; m < m1; m++) {
-            const float *r = raw + (int64_t)m * ldr;
-            for (int h = lane; h < d.H; h += 64) beta[(int64_t)m * d.H + h] = l_sigmoid(r[d.off_b() + h]);
-            for (int i = lane; i < lfa; i += 64) l_store_act<PREC>(fa, (int64_t)m * lfa + i, i < d.ra ? r[d.off_a() + i] : 0.0f);
-            for (int i = lane; i < lfg; i += 64) l_store_act<PREC>(fg, (int64_t)m * lfg + i, i < d.rg ? r[d.off_g() + i] : 0.0f);
+    PrepRows rows;
+#pragma unroll
+    for (int i = 0; i < CONV_AHEAD - 1 + PREP_T; i++) rows.at[i] = min(i, M - 1 - (m0 - CONV_AHEAD + 1)) * ldr;
+    if (unit > d.G + d.H * nv) return;
+    if (unit == d.G + d.H * nv) {  // beta and the low-rank factors: a column of all tokens at a time
+        const float *r = raw + (int64_t)m0 * ldr;
+        auto column = [&](int c, float (&x)[PREP_T]) {
+#pragma unroll
+            for (int i = 0; i < PREP_T; i++) x[i] = r[(int64_t)min(i, n - 1) * ldr + c];
+        };
+        float x[PREP_T];
+        for (int h = lane; h < d.H; h += 64) {
+            column(d.off_b() + h, x);
+#pragma unroll
+            for (int i = 0; i < PREP_T; i++)
+                if (i < n) beta[(int64_t)(m0 + i) * d.H + h] = l_sigmoid(x[i]);
+        }
+        for (int64_t j = lane; j < lfa + lfg; j += 64) {
+            const bool isa = j < lfa;
+            const int k = (int)(isa ? j : j - lfa), rank = isa ? d.ra : d.rg;
+            column((isa ? d.off_a() : d.off_g()) + min(k, rank - 1), x);
+#pragma unroll
+            for (int i = 0; i < PREP_T; i++)
+                if (i < n) l_store_act<PREC>(isa ? fa : fg, (int64_t)(m0 + i) * (isa ? lfa : lfg) + k, k < rank ? x[i] : 0.0f);
         }
         return;
     }
-    if (unit >= d.G) {  // a value head
-        const int ch0 = 2 * GD + (unit - d.G) * d.V;
-        for (int e = lane; e < d.V; e += 64) {
-            float y[PREP_T];
-            delta_conv_rows(conv, raw, ldr, ring, C, taps, ch0 + e, m0, M, pos0, y);
+    if (unit >= d.G) {  // columns of a value head
+        const int h = (unit - d.G) / nv, e = (unit - d.G - h * nv) * 64 + lane, ch = 2 * GD + h * d.V + min(e, d.V - 1);
+        PrepIn in;
+        float y[PREP_T];
+        delta_conv_request(in, rows, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0);
+        delta_conv_rows(in, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0, y);
+        if (e < d.V)
 #pragma unroll
             for (int i = 0; i < PREP_T; i++)
-                if (m0 + i < M) qkv[(int64_t)(m0 + i) * C + ch0 + e] = y[i];
-        }
+                if (i < n) qkv[(int64_t)(m0 + i) * C + ch] = y[i];
         return;
     }
     // a key head's q and k
     float q[NE][PREP_T], k[NE][PREP_T];
-#pragma unroll
-    for (int i = 0; i < NE; i++) {
-        const int e = lane + 64 * i, ch = unit * d.D + min(e, d.D - 1);
-        delta_conv_rows(conv, raw, ldr, ring, C, taps, ch, m0, M, pos0, q[i]);
-        delta_conv_rows(conv, raw, ldr, ring, C, taps, GD + ch, m0, M, pos0, k[i]);
-        if (e >= d.D)
-#pragma unroll
-            for (int j = 0; j < PREP_T; j++) q[i][j] = k[i][j] = 0.0f;
-    }
-    const float qs = 1.0f / sqrtf((float)d.D);
-#pragma unroll
-    for (int j = 0; j < PREP_T; j++) {
-        float qq = 0.0f, kk = 0.0f, qk = 0.0f;
+    {
+        PrepIn iq[NE], ik[NE];
 #pragma unroll
         for (int i = 0; i < NE; i++) {
-            qq = fmaf(q[i][j], q[i][j], qq);
-            kk = fmaf(k[i][j], k[i][j], kk);
-            qk = fmaf(q[i][j], k[i][j], qk);
+            const int ch = unit * d.D + min(lane + 64 * i, d.D - 1);
+            delta_conv_request(iq[i], rows, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0);
+            delta_conv_request(ik[i], rows, conv, raw, ldr, ring, C, taps, GD + ch, m0, M, pos0);
         }
-        const float rq = qs / sqrtf(l_wave_sum(qq) + 1e-6f), rk = 1.0f / sqrtf(l_wave_sum(kk) + 1e-6f);
-        qk = l_wave_sum(qk);
-        const int m = m0 + j;
-        if (m >= M) break;
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            const int e = lane + 64 * i, ch = unit * d.D + min(e, d.D - 1);
+            delta_conv_rows(iq[i], conv, raw, ldr, ring, C, taps, ch, m0, M, pos0, q[i]);
+            delta_conv_rows(ik[i], conv, raw, ldr, ring, C, taps, GD + ch, m0, M, pos0, k[i]);
+            if (e >= d.D)
+#pragma unroll
+                for (int j = 0; j < PREP_T; j++) q[i][j] = k[i][j] = 0.0f;
+        }
+    }
+    // lane l: what makes a unit vector of token l % 8's q, or of its k (l % 16 >= 8)
+    float v[2 * PREP_T], f;
+#pragma unroll
+    for (int j = 0; j < PREP_T; j++) {
+        v[j] = v[PREP_T + j] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            v[j] = fmaf(q[i][j], q[i][j], v[j]);
+            v[PREP_T + j] = fmaf(k[i][j], k[i][j], v[PREP_T + j]);
+        }
+    }
+    f = 1.0f / sqrtf(delta_wave_sum16(v, lane) + 1e-6f);
+    if ((lane & 15) < PREP_T) f *= 1.0f / sqrtf((float)d.D);
+    float qk = 0.0f;
+    if (kq) {
+#pragma unroll
+        for (int j = 0; j < PREP_T; j++) {
+            v[j] = v[PREP_T + j] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NE; i++) v[j] = fmaf(q[i][j], k[i][j], v[j]);
+        }
+        qk = delta_wave_sum16(v, lane);
+    }
+#pragma unroll
+    for (int j = 0; j < PREP_T; j++) {
+        if (j >= n) break;
+        const float rq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), j)),
+                    rk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), PREP_T + j));
+        float *row = qkv + (int64_t)(m0 + j) * C + unit * d.D;
 #pragma unroll
         for (int i = 0; i < NE; i++) {
             const int e = lane + 64 * i;
             if (e >= d.D) continue;
-            qkv[(int64_t)m * C + unit * d.D + e] = q[i][j] * rq;
-            qkv[(int64_t)m * C + GD + unit * d.D + e] = k[i][j] * rk;
+            row[e] = q[i][j] * rq;
+            row[GD + e] = k[i][j] * rk;
         }
-        if (lane == 0) kq[(int64_t)m * d.G + unit] = qk * rq * rk;
+        if (kq && lane == j) kq[(int64_t)(m0 + j) * d.G + unit] = qk * rq * rk;
     }
 }
 
@@ -346,7 +422,7 @@ hipError_t k_delta_prepare(hipStream_t s, const DeltaShape &d, const float *conv
                            int M, int pos0, float *qkv, float *kq, float *beta, void *fa, int64_t lfa, void *fg, int64_t lfg,
                            int prec) {
     if (d.D > 256 || M < 1) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((d.G + d.H + 1 + 3) / 4), (unsigned)((M + PREP_T - 1) / PREP_T));
+    const dim3 grid((unsigned)((d.G + d.H * ((d.V + 63) / 64) + 1 + 3) / 4), (unsigned)((M + PREP_T - 1) / PREP_T));
 #define GO(N)                                                                                                                            \
     do {                                                                                                                                 \
         if (prec)                                                                                                                        \
@@ -549,22 +625,6 @@ __device__ __forceinline__ d_f32x4 delta_mm(const d_f32x4 a, const d_f32x4 b, d_
 #pragma unroll
     for (int r = 0; r < 4; r++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
     return c;
-}
-
-// one of 16 sums over the 16 lanes of a row: lane l gets that of v[l].  Every step halves the sums: lanes l and 15 - l, l and 7 - l, l and l ^ 2, l and l ^ 1
-template <int CTRL>
-__device__ __forceinline__ float delta_swap_add(bool upper, float lo, float hi) {
-    return (upper ? hi : lo) + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(upper ? lo : hi), CTRL, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float delta_sum16(const float (&v)[16], int l) {
-    float a[8], b[4], c[2];
-#pragma unroll
-    for (int i = 0; i < 8; i++) a[i] = delta_swap_add<0x140>(l & 8, v[i], v[i + 8]);  // row_mirror
-#pragma unroll
-    for (int i = 0; i < 4; i++) b[i] = delta_swap_add<0x141>(l & 4, a[i], a[i + 4]);  // row_half_mirror
-#pragma unroll
-    for (int i = 0; i < 2; i++) c[i] = delta_swap_add<0x4E>(l & 2, b[i], b[i + 2]);
-    return delta_swap_add<0xB1>(l & 1, c[0], c[1]);
 }
 
 template <int NW>

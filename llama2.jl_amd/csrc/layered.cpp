@@ -1215,7 +1215,8 @@ static hipError_t prompt_delta(l2h_model *m, LayerDev &L, const LayerRun &run, i
     const DeltaShape d = delta_shape(l, L);
     const int64_t ldr = L.n_plain, hd = d.H * d.D, hv = d.H * d.V;
     hipError_t e;
-    CK(k_delta_prepare(s, d, L.conv, l->raw, ldr, run.ring, M, pos0, l->qkv, l->kq, l->beta, l->fa, L.a2.ld, l->fg, L.g2.ld, prec));
+    const bool walk = M >= L_DELTA_WALK_MIN;
+    CK(k_delta_prepare(s, d, L.conv, l->raw, ldr, run.ring, M, pos0, l->qkv, walk ? nullptr : l->kq, l->beta, l->fa, L.a2.ld, l->fg, L.g2.ld, prec));
     CK(k_delta_ring(s, d, l->raw, ldr, run.ring, M, pos0));
     GemmArgs a = gemm_of(L.a2, l->fa, M);
     a.outf = l->lg;
@@ -1225,7 +1226,7 @@ static hipError_t prompt_delta(l2h_model *m, LayerDev &L, const LayerRun &run, i
     a.hd = d.D;
     CK(k_gemm(s, a, prec, GE_DECAY));
     CK(product(m, gemm_of(L.g2, l->fg, M), GE_SIGMOID, l->gt, hv, 1.0f));
-    if (M >= L_DELTA_WALK_MIN) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
+    if (walk) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
     CK(k_delta_scan(s, d, l->qkv, l->kq, l->beta, l->lg, run.state, M, pos0, l->ob));
     return k_head_norm_rows(s, l->ob, l->gt, L.mixnorm, M, d.H, d.V, d.eps, l->ao, L.o.ld, prec);
 }

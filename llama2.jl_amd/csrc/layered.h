@@ -197,7 +197,7 @@ struct DeltaWeights {
 // ring: [taps][channels], slot t % taps holds token t's projected channels; state: [H][D][V]
 hipError_t k_delta_step(hipStream_t s, const DeltaShape &d, const DeltaWeights &w, const float *in, float *ring, float *state,
                         const DecodeCtl *ctl, float *o, float *ssq, float *gate);
-// convolution, silu, unit vectors, beta: raw[M][ldr] -> qkv[M][channels], kq[M][G] (= k . q), beta[M][H], and the two low-rank
+// convolution, silu, unit vectors, beta: raw[M][ldr] -> qkv[M][channels], kq[M][G] (= k . q; or nullptr), beta[M][H], and the two low-rank
 // factors as activations
 hipError_t k_delta_prepare(hipStream_t s, const DeltaShape &d, const float *conv, const float *raw, int64_t ldr, const float *ring,
                            int M, int pos0, float *qkv, float *kq, float *beta, void *fa, int64_t lfa, void *fg, int64_t lfg,
