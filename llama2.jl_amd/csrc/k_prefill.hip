@@ -12,14 +12,30 @@
 // ------------------------------------------------------------------------------------------
 // small per-position kernels
 // ------------------------------------------------------------------------------------------
-// X[m][:] = dequantized embedding row of tokens[m]  (src/inference.jl:236)
+// X[m][:] = dequantized embedding row of tokens[m]  (src/inference.jl:236).  Four elements a thread: 2048 rows of 2048 bf16 elements 10 us,
+// one a thread 16.
 __global__ __launch_bounds__(256) void pf_embed_kernel(DevTensor emb, const int32_t *tokens, float *X, int M, float scale, float *X_copy) {
     const int m = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
     if (m >= M || i >= emb.ne0) return;
-    const float v = scale * dequant_elem(emb, tokens[m], i);
-    X[(int64_t)m * emb.ne0 + i] = v;
-    if (X_copy) X_copy[(int64_t)m * emb.ne0 + i] = v;
+    const int64_t tok = tokens[m], at = (int64_t)m * emb.ne0 + i;
+    if (emb.ne0 % 4 != 0) {
+        for (int k = 0; k < min((int64_t)4, emb.ne0 - i); k++) {
+            X[at + k] = scale * dequant_elem(emb, tok, i + k);
+            if (X_copy) X_copy[at + k] = X[at + k];
+        }
+        return;
+    }
+    float4 v;
+    if (emb.type == L2H_TYPE_BF16) {
+        const uint2 w = *(const uint2 *)((const uint16_t *)emb.qs + tok * emb.ne0 + i);
+        v = make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xFFFF0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xFFFF0000u));
+    } else {
+        v = make_float4(dequant_elem(emb, tok, i), dequant_elem(emb, tok, i + 1), dequant_elem(emb, tok, i + 2), dequant_elem(emb, tok, i + 3));
+    }
+    v = make_float4(scale * v.x, scale * v.y, scale * v.z, scale * v.w);
+    *(float4 *)(X + at) = v;
+    if (X_copy) *(float4 *)(X_copy + at) = v;
 }
 
 // cos/sin of the RoPE angles of positions pos0..pos0+M-1: theta_i = fp32(pos) advanced by i fp32
@@ -886,7 +902,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 // launchers
 // ------------------------------------------------------------------------------------------
 hipError_t k_pf_embed(hipStream_t s, const DevTensor &emb, const int32_t *tokens, float *X, int M, float scale, float *X_copy) {
-    hipLaunchKernelGGL(pf_embed_kernel, dim3((unsigned)((emb.ne0 + 255) / 256), (unsigned)M), dim3(256), 0, s, emb,
+    hipLaunchKernelGGL(pf_embed_kernel, dim3((unsigned)((emb.ne0 + 1023) / 1024), (unsigned)M), dim3(256), 0, s, emb,
                        tokens, X, M, scale, X_copy);
     return hipGetLastError();
 }
