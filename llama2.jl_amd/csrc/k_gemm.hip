@@ -349,35 +349,69 @@ hipError_t k_route(hipStream_t s, const float *z, int64_t ldz, const float *bias
 }
 
 // one workgroup: counts, offsets, slots and the list of tiles.  The order of an expert's slots is whatever the LDS counters
-// give; every slot is computed on its own, so no result depends on it.
+// give; every slot is computed on its own, so no result depends on it.  What bounds it is latency, so a thread's first GROUP_Q choices are
+// requested together, a choice is counted once (its place among its expert's is what the counter was) and the offsets are a scan: 2048 tokens with four of
+// 32 experts each 8.6 us, against 15.
+#define GROUP_Q 8
 __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                                                      float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows) {
     extern __shared__ __align__(16) int s_int[];
+    __shared__ int s_wave[2][16];
     int *cnt = s_int, *off = s_int + E;
-    const int n = M * top;
-    for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
+    const int n = M * top, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int c[GROUP_Q], rank[GROUP_Q];
+    float f[GROUP_Q];
+#pragma unroll
+    for (int u = 0; u < GROUP_Q; u++) {
+        const int i = min(t + 1024 * u, n - 1);
+        c[u] = choice[i];
+        f[u] = score[i];
+    }
+    for (int e = t; e < E; e += 1024) cnt[e] = 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 1024) atomicAdd(&cnt[choice[i]], 1);
+#pragma unroll
+    for (int u = 0; u < GROUP_Q; u++)
+        if (t + 1024 * u < n) rank[u] = atomicAdd(&cnt[c[u]], 1);
+    for (int i = t + 1024 * GROUP_Q; i < n; i += 1024) slot_of[i] = atomicAdd(&cnt[choice[i]], 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int o = 0, nt = 0;
-        for (int e = 0; e < E; e++) {
-            off[e] = o;
-            for (int r = 0; r < cnt[e]; r += tile_rows) tiles[nt++] = GemmTile{e, o + r, min(tile_rows, cnt[e] - r)};
-            o += cnt[e];
-        }
-        n_tiles[0] = nt;
+    // rows and tiles of the experts before e (E <= 1024: a thread for each)
+    const int rows = t < E ? cnt[t] : 0, nt = (rows + tile_rows - 1) / tile_rows;
+    int sr = rows, st = nt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int r = __shfl_up(sr, d, WAVE), k = __shfl_up(st, d, WAVE);
+        sr += lane >= d ? r : 0;
+        st += lane >= d ? k : 0;
+    }
+    if (lane == 63) {
+        s_wave[0][wave] = sr;
+        s_wave[1][wave] = st;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 1024) {
-        const int slot = atomicAdd(&off[choice[i]], 1);
+    for (int w = 0; w < wave; w++) {
+        sr += s_wave[0][w];
+        st += s_wave[1][w];
+    }
+    if (t < E) {
+        off[t] = sr - rows;
+        for (int k = 0; k < nt; k++) tiles[st - nt + k] = GemmTile{t, sr - rows + k * tile_rows, min(tile_rows, rows - k * tile_rows)};
+    }
+    if (t == 1023) n_tiles[0] = st;
+    __syncthreads();
+    auto put = [&](int i, int expert, float scale, int place) {
+        const int slot = off[expert] + place;
         slot_row[slot] = i / top;
-        slot_scale[slot] = score[i];
+        slot_scale[slot] = scale;
         slot_of[i] = slot;
-    }
+    };
+#pragma unroll
+    for (int u = 0; u < GROUP_Q; u++)
+        if (t + 1024 * u < n) put(t + 1024 * u, c[u], f[u], rank[u]);
+    for (int i = t + 1024 * GROUP_Q; i < n; i += 1024) put(i, choice[i], score[i], slot_of[i]);
 }
 hipError_t k_group(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                    float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows) {
+    if (E < 1 || E > 1024 || M < 1 || top < 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 2 * E * sizeof(int), s, choice, score, M, E, top, slot_row, slot_scale, slot_of,
                        tiles, n_tiles, tile_rows);
     return hipGetLastError();
