@@ -124,6 +124,27 @@ static int dev_tensor_download(l2h_ctx *ctx, const DevTensor *t, void *host) {
 // ------------------------------------------------------------------------------------------
 // context
 // ------------------------------------------------------------------------------------------
+void *PinnedArena::take(size_t bytes) {
+    const size_t n = (bytes + UNIT - 1) / UNIT;
+    std::lock_guard<std::mutex> hold(lock);
+    for (size_t i = 0; mem && i + n <= UNITS; i++) {
+        size_t k = 0;
+        while (k < n && !used[i + k]) k++;
+        if (k < n) continue;
+        std::fill(used + i, used + i + n, true);
+        return mem + i * UNIT;
+    }
+    return nullptr;
+}
+bool PinnedArena::give(void *p, size_t bytes) {
+    std::lock_guard<std::mutex> hold(lock);
+    const char *c = (const char *)p;
+    if (!mem || c < mem || c >= mem + UNIT * UNITS) return false;
+    const size_t i = (size_t)(c - mem) / UNIT, n = (bytes + UNIT - 1) / UNIT;
+    std::fill(used + i, used + i + n, false);
+    return true;
+}
+
 extern "C" int l2h_ctx_create(int device, l2h_ctx **out) {
     if (!out) return set_err(nullptr, L2H_EINVAL, "l2h_ctx_create: out is NULL");
     *out = nullptr;
@@ -150,6 +171,10 @@ extern "C" int l2h_ctx_create(int device, l2h_ctx **out) {
         delete ctx;
         return L2H_ENODEV;
     }
+    if (hipHostMalloc((void **)&ctx->pinned.mem, PinnedArena::UNIT * PinnedArena::UNITS, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->pinned.mem = nullptr;
+    }
     *out = ctx;
     return L2H_OK;
 }
@@ -160,6 +185,7 @@ extern "C" void l2h_ctx_destroy(l2h_ctx *ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipStreamDestroy(ctx->stream);
     }
+    if (ctx->pinned.mem) (void)hipHostFree(ctx->pinned.mem);
     delete ctx;
 }
 
@@ -217,6 +243,20 @@ class DeviceTurn {
     std::unique_lock<std::mutex> hold;
 };
 
+// A call that returns before its copies out of the model's box have been waited for waits for them
+class BoxGuard {
+  public:
+    explicit BoxGuard(const l2h_model *m) : stream(m->ctx->stream) {}
+    ~BoxGuard() {
+        if (!waited) (void)hipStreamSynchronize(stream);
+    }
+    void drained() { waited = true; }
+
+  private:
+    hipStream_t stream;
+    bool waited = false;
+};
+
 static int q8_alloc(l2h_ctx *ctx, int64_t n, Q8Dev *q, std::vector<void *> *track) {
     void *p = nullptr;
     const int64_t o_bs = align256(n), o_d = o_bs + align256(n / 8 + 16);
@@ -263,6 +303,13 @@ static void model_free_state(l2h_model *m) {
     m->allocs.clear();
     for (void *p : m->uc_allocs) uncached_release(p);
     m->uc_allocs.clear();
+    if (m->box.mem && !m->ctx->pinned.give(m->box.mem, m->box.bytes)) {
+        if (m->box.pinned)
+            (void)hipHostFree(m->box.mem);
+        else
+            free(m->box.mem);
+    }
+    m->box = HostBox();
     m->pf_cap = 0;
     m->pf_wbf = nullptr;
     m->pf_copy_tried = false;
@@ -1013,10 +1060,27 @@ static int loop_buffers(l2h_model *m) {
 #define DA(p, n, z)                       \
     if ((rc = dalloc(m, &(p), (n), (z)))) \
         return rc;
-    DA(m->ctl, 2, true);  // (the second: a layered model's steps hand the first on through it)
-    DA(m->prompt_dev, m->c.seq_len, true);
+    // the control blocks (the second: a layered model's steps hand the first on through it) and the prompt behind them
+    static_assert(sizeof(DecodeCtl) % 16 == 0, "the prompt follows the control blocks");
+    const int64_t n = m->c.seq_len;
+    DA(m->ctl, 2 + (n * 4 + (int64_t)sizeof(DecodeCtl) - 1) / (int64_t)sizeof(DecodeCtl), true);
+    m->prompt_dev = (int32_t *)(m->ctl + 2);
     m->max_out = m->c.seq_len;
     DA(m->out_tokens, m->max_out, true);
+    HostBox &b = m->box;
+    b.bytes = 2 * sizeof(DecodeCtl) + 2 * (size_t)n * 4 + 64;
+    b.mem = m->ctx->pinned.take(b.bytes);
+    if (!b.mem && !(b.pinned = hipHostMalloc(&b.mem, b.bytes, hipHostMallocDefault) == hipSuccess)) {
+        (void)hipGetLastError();  // (then copies wait, as they do from any memory of a program)
+        b.mem = malloc(b.bytes);
+        if (!b.mem) return set_err(m->ctx, L2H_EHIP, "out of host memory");
+    }
+    memset(b.mem, 0, b.bytes);
+    b.ctl = (DecodeCtl *)b.mem;
+    b.prompt = (int32_t *)(b.ctl + 2);
+    b.out = b.prompt + n;
+    b.pick = b.out + n;
+    b.gave_up = (unsigned *)b.pick + 1;
     DA(m->argmax_partial, std::max(L2H_ARGMAX_BLOCKS, m->ctx->prop.multiProcessorCount), true);
 #undef DA
     return L2H_OK;
@@ -1167,11 +1231,15 @@ static int last_token(l2h_model *m, int n) {
 }
 
 // after the stream has drained: did a workgroup of the persistent kernel give up at a barrier?
+// (mega_ask is requested behind the launches, mega_check reads the answer once the stream has drained)
+static int mega_ask(l2h_model *m) {
+    const void *flag = m->flow ? (const void *)m->flow_args.abort_flag : m->mega ? (const void *)&m->bar->abort : nullptr;
+    if (flag) HIPCHK(m->ctx, hipMemcpyAsync(m->box.gave_up, flag, 4, hipMemcpyDeviceToHost, m->ctx->stream));
+    return L2H_OK;
+}
 static int mega_check(l2h_model *m) {
     if (m->flow) {
-        unsigned int ab = 0;
-        HIPCHK(m->ctx, hipMemcpy(&ab, m->flow_args.abort_flag, 4, hipMemcpyDeviceToHost));
-        if (!ab) return L2H_OK;
+        if (!*m->box.gave_up) return L2H_OK;
         m->flow_holds_state = false;
         HIPCHK(m->ctx, hipMemset(m->flow_args.abort_flag, 0, 4));
         // all words "not written"
@@ -1198,9 +1266,7 @@ static int mega_check(l2h_model *m) {
         return set_err(m->ctx, L2H_EHIP, "streaming decode kernel: a wait for activations timed out");
     }
     if (!m->mega) return L2H_OK;
-    unsigned int ab = 0;
-    HIPCHK(m->ctx, hipMemcpy(&ab, &m->bar->abort, 4, hipMemcpyDeviceToHost));
-    if (!ab) return L2H_OK;
+    if (!*m->box.gave_up) return L2H_OK;
     HIPCHK(m->ctx, hipMemset(m->bar, 0, sizeof(GridBar)));
     m->bar_gen = 0;
     return set_err(m->ctx, L2H_EHIP, "persistent decode kernel: a grid barrier timed out (workgroups not co-resident?)");
@@ -1278,10 +1344,10 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     h.n_prompt = n_prompt;
     h.last_argmax = 0;
     h.n_out = 0;
-    const DecodeCtl both[2] = {h, h};
-    HIPCHK(ctx, hipMemcpyAsync(m->prompt_dev, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(m->ctl, both, sizeof both, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    BoxGuard guard(m);
+    m->box.ctl[0] = m->box.ctl[1] = h;
+    memcpy(m->box.prompt, prompt, (size_t)n_prompt * 4);
+    HIPCHK(ctx, hipMemcpyAsync(m->ctl, m->box.ctl, 2 * sizeof h + (size_t)n_prompt * 4, hipMemcpyHostToDevice, ctx->stream));
     if (m->lay && total > 0) layered_advance(m, pos0 + total);
     DeviceTurn turn(m);
     if (decode_ms) {
@@ -1303,13 +1369,15 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     } else {
         if ((rc = run_steps(m, total)) || (rc = last_token(m, total))) return rc;
     }
-    if (n_new > 0)
-        HIPCHK(ctx, hipMemcpyAsync(out, m->out_tokens, (size_t)n_new * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (n_new > 0) HIPCHK(ctx, hipMemcpyAsync(m->box.out, m->out_tokens, (size_t)n_new * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if ((rc = mega_ask(m))) return rc;
     if (last_logits)
         HIPCHK(ctx, hipMemcpyAsync(last_logits, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost,
                                    ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    guard.drained();
     turn.drained();
+    if (n_new > 0) memcpy(out, m->box.out, (size_t)n_new * 4);
     return mega_check(m);
 }
 
@@ -1513,6 +1581,8 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
         if ((rc = prefill_buffers(m, std::min(n, L2H_PREFILL_CHUNK)))) return rc;
         if (m->pf_copy_mode && (rc = prefill_weights(m))) return rc;
     }
+    BoxGuard guard(m);
+    memcpy(m->box.prompt, tokens, (size_t)n * 4);
     int M = 0, w0 = 0;
     std::vector<int32_t> rows;
     for (int c0 = 0; c0 < n; c0 += M) {
@@ -1523,7 +1593,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
         float *wl = want_logits ? want_logits + (int64_t)w0 * m->c.vocab_size : nullptr;
         w0 += (int)rows.size();
         if (m->lay) {
-            HIPCHK(ctx, hipMemcpyAsync(layered_token_buffer(m), tokens + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
+            HIPCHK(ctx, hipMemcpyAsync(layered_token_buffer(m), m->box.prompt + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
             const hipError_t e = layered_prefill_chunk(m, M, pos0 + c0);
             if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "prompt pass launch failed: %s", hipGetErrorString(e));
             layered_advance(m, pos0 + c0 + M);
@@ -1549,7 +1619,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
                 if ((rc = prefill_expand(m, false))) return rc;
             }
         }
-        HIPCHK(ctx, hipMemcpyAsync(m->pf_tok, tokens + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(ctx, hipMemcpyAsync(m->pf_tok, m->box.prompt + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
         hipError_t e = prefill_chunk(m, M, pos0 + c0);
         if (e != hipSuccess)
             return set_err(ctx, L2H_EHIP, "prompt pass launch failed: %s%s%s", hipGetErrorString(e),
@@ -1563,6 +1633,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
     }
     if (!last_logits && !next_token) {
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        guard.drained();
         return L2H_OK;
     }
     // last position: its hidden state becomes the decode state; classifier and argmax as in a decode step
@@ -1574,17 +1645,19 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
     h.token = tokens[n - 1];
     h.pos = pos0 + n - 1;
     h.n_prompt = 1;
-    HIPCHK(ctx, hipMemcpyAsync(m->ctl, &h, sizeof h, hipMemcpyHostToDevice, ctx->stream));
+    m->box.ctl[0] = h;
+    HIPCHK(ctx, hipMemcpyAsync(m->ctl, m->box.ctl, sizeof h, hipMemcpyHostToDevice, ctx->stream));
     hipError_t e = m->lay ? layered_output(m) : launch_output(m);
     if (e == hipSuccess)
         e = k_argmax(ctx->stream, m->logits, m->c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, false);
     if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "classifier launch failed: %s", hipGetErrorString(e));
-    if (next_token)
-        HIPCHK(ctx, hipMemcpyAsync(next_token, m->out_tokens, 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (next_token) HIPCHK(ctx, hipMemcpyAsync(m->box.out, m->out_tokens, 4, hipMemcpyDeviceToHost, ctx->stream));
     if (last_logits)
         HIPCHK(ctx, hipMemcpyAsync(last_logits, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost,
                                    ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    guard.drained();
+    if (next_token) *next_token = m->box.out[0];
     return L2H_OK;
 }
 
@@ -1630,11 +1703,11 @@ extern "C" int l2h_sample(l2h_model *m, float temperature, float u, int32_t *tok
         if ((rc = dalloc(m, &m->sample_p, m->c.vocab_size, false))) return rc;
     }
     HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_part, m->sample_out));
-    int32_t pick = -1;
     if (probs)
         HIPCHK(ctx, hipMemcpyAsync(probs, m->sample_p, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(&pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(m->box.pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    const int32_t pick = *m->box.pick;
     if (pick < 0) return set_err(ctx, L2H_EINVAL, "nothing to draw from: the logits divided by %g are not all finite", (double)temperature);
     *token = pick;
     return L2H_OK;
