@@ -1,23 +1,20 @@
-// Many tokens through a bf16 matrix, C[m][n] = sum_k X[m][k] W[n][k], on the matrix cores: bf16 activations
-// (v_mfma_f32_32x32x16_bf16) or fp32 ones (v_mfma_f32_32x32x2_f32: fp32 operands and sums), with fused epilogues and a grouped
+// Many tokens through a bf16 matrix, C[m][n] = sum_k X[m][k] W[n][k], on the matrix cores: bf16 activations, or fp32
+// ones in three bf16 parts (v_mfma_f32_32x32x16_bf16, fp32 sums), with fused epilogues and a grouped
 // form for mixtures of experts; and the row-wise kernels around the products.
 #include "layered_gemm.h"
 
 typedef __bf16 l_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float l_f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t l_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t l_u32x4 __attribute__((ext_vector_type(4)));
 
 // Placement of the 16-byte chunks of a 128-byte tile row: 16 consecutive rows' chunks of one index fall into different slots
 // of the 256-byte bank row.
 __device__ __forceinline__ int gemm_swz(int r) { return (r >> 1) & 7; }
 
-template <int PREC, int EPI, int TN, int TM, bool GROUPED>
+template <int EPI, int TN, int TM, bool GROUPED>
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
-    constexpr int IN = TN / 64, JM = TM / 64;          // 32 x 32 tiles per wavefront (2 x 2 wavefronts)
-    constexpr int KSTEP = PREC ? 32 : 64;
-    constexpr int FROW = 33;                            // floats per LDS row of the fp32 form
-    constexpr int OPERANDS = (TN + TM) * (PREC ? FROW * 4 : 128), RESULTS = 4 * 4 * gemm_epilogue_floats(IN, JM);
+    constexpr int IN = TN / 64, JM = TM / 64;  // 32 x 32 tiles per wavefront (2 x 2 wavefronts)
+    constexpr int KSTEP = 64, OPERANDS = (TN + TM) * 128, RESULTS = 4 * 4 * gemm_epilogue_floats(IN, JM);
     __shared__ __align__(16) unsigned char s_raw[OPERANDS > RESULTS ? OPERANDS : RESULTS];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wn = wave & 1, wm = wave >> 1;
     const uint16_t *W = a.w;
@@ -41,17 +38,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-    // rows this thread copies: row t / 8 + 32 i of each tile, elements 8 (t % 8) .. (bf16) or 4 (t % 8) .. (fp32) of a step
+    // rows this thread copies: row t / 8 + 32 i of each tile, elements 8 (t % 8) .. of a step
     constexpr int WL = TN / 32, XL = TM / 32;
     const int c8 = t & 7;
-    const uint16_t *wrow[WL];
-    const uint16_t *xrow16[XL];
-    const float *xrow32[XL];
+    const uint16_t *wrow[WL], *xrow[XL];
 #pragma unroll
     for (int i = 0; i < WL; i++) {
         int64_t r = n0 + (t >> 3) + 32 * i;
         if (r >= a.n_rows) r = a.n_rows - 1;
-        wrow[i] = W + r * a.ld + (PREC ? 4 : 8) * c8;
+        wrow[i] = W + r * a.ld + 8 * c8;
     }
 #pragma unroll
     for (int i = 0; i < XL; i++) {
@@ -59,99 +54,278 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs a) {
         if (m >= mcount) m = mcount - 1;  // (repeats the last row; not stored)
         int64_t row = mb + m;
         if (a.gather) row = a.gather[row];
-        if (PREC)
-            xrow32[i] = (const float *)a.x + row * a.ldx + 4 * c8;
-        else
-            xrow16[i] = (const uint16_t *)a.x + row * a.ldx + 8 * c8;
+        xrow[i] = (const uint16_t *)a.x + row * a.ldx + 8 * c8;
     }
     // (vectors of the compiler's own: as uint4, a struct, the sixteen words went through scratch memory in every step)
     l_u32x4 wreg[WL], xreg[XL];
     auto gload = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < WL; i++) {
-            if (PREC) {
-                const l_u32x2 v = *(const l_u32x2 *)(wrow[i] + k0);
-                wreg[i] = l_u32x4{v.x, v.y, 0, 0};
-            } else {
-                wreg[i] = *(const l_u32x4 *)(wrow[i] + k0);
-            }
-        }
+        for (int i = 0; i < WL; i++) wreg[i] = *(const l_u32x4 *)(wrow[i] + k0);
 #pragma unroll
-        for (int i = 0; i < XL; i++) xreg[i] = PREC ? *(const l_u32x4 *)(xrow32[i] + k0) : *(const l_u32x4 *)(xrow16[i] + k0);
+        for (int i = 0; i < XL; i++) xreg[i] = *(const l_u32x4 *)(xrow[i] + k0);
     };
     gload(0);
     for (int k0 = 0; k0 < a.ld; k0 += KSTEP) {
-        if constexpr (PREC == 0) {
-            l_u32x4 *s_w = (l_u32x4 *)s_raw, *s_x = s_w + TN * 8;
+        l_u32x4 *s_w = (l_u32x4 *)s_raw, *s_x = s_w + TN * 8;
 #pragma unroll
-            for (int i = 0; i < WL; i++) {
-                const int r = (t >> 3) + 32 * i;
-                s_w[r * 8 + (c8 ^ gemm_swz(r))] = wreg[i];
+        for (int i = 0; i < WL; i++) {
+            const int r = (t >> 3) + 32 * i;
+            s_w[r * 8 + (c8 ^ gemm_swz(r))] = wreg[i];
+        }
+#pragma unroll
+        for (int i = 0; i < XL; i++) {
+            const int r = (t >> 3) + 32 * i;
+            s_x[r * 8 + (c8 ^ gemm_swz(r))] = xreg[i];
+        }
+        __syncthreads();
+        if (k0 + KSTEP < a.ld) gload(k0 + KSTEP);
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int c = 2 * kk + (lane >> 5);
+            l_bf16x8 A[IN], B[JM];
+#pragma unroll
+            for (int i = 0; i < IN; i++) {
+                const int r = (TN / 2) * wn + 32 * i + (lane & 31);
+                A[i] = __builtin_bit_cast(l_bf16x8, s_w[r * 8 + (c ^ gemm_swz(r))]);
             }
 #pragma unroll
-            for (int i = 0; i < XL; i++) {
-                const int r = (t >> 3) + 32 * i;
-                s_x[r * 8 + (c8 ^ gemm_swz(r))] = xreg[i];
-            }
-            __syncthreads();
-            if (k0 + KSTEP < a.ld) gload(k0 + KSTEP);
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                const int c = 2 * kk + (lane >> 5);
-                l_bf16x8 A[IN], B[JM];
-#pragma unroll
-                for (int i = 0; i < IN; i++) {
-                    const int r = (TN / 2) * wn + 32 * i + (lane & 31);
-                    A[i] = __builtin_bit_cast(l_bf16x8, s_w[r * 8 + (c ^ gemm_swz(r))]);
-                }
-#pragma unroll
-                for (int j = 0; j < JM; j++) {
-                    const int r = (TM / 2) * wm + 32 * j + (lane & 31);
-                    B[j] = __builtin_bit_cast(l_bf16x8, s_x[r * 8 + (c ^ gemm_swz(r))]);
-                }
-#pragma unroll
-                for (int i = 0; i < IN; i++)
-#pragma unroll
-                    for (int j = 0; j < JM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i], B[j], acc[i][j], 0, 0, 0);
-            }
-        } else {
-            float *s_w = (float *)s_raw, *s_x = s_w + TN * FROW;
-#pragma unroll
-            for (int i = 0; i < WL; i++) {
-                float *p = s_w + ((t >> 3) + 32 * i) * FROW + 4 * c8;
-                p[0] = l_bf16_lo(wreg[i].x);
-                p[1] = l_bf16_hi(wreg[i].x);
-                p[2] = l_bf16_lo(wreg[i].y);
-                p[3] = l_bf16_hi(wreg[i].y);
+            for (int j = 0; j < JM; j++) {
+                const int r = (TM / 2) * wm + 32 * j + (lane & 31);
+                B[j] = __builtin_bit_cast(l_bf16x8, s_x[r * 8 + (c ^ gemm_swz(r))]);
             }
 #pragma unroll
-            for (int i = 0; i < XL; i++) {
-                float *p = s_x + ((t >> 3) + 32 * i) * FROW + 4 * c8;
-                p[0] = __uint_as_float(xreg[i].x);
-                p[1] = __uint_as_float(xreg[i].y);
-                p[2] = __uint_as_float(xreg[i].z);
-                p[3] = __uint_as_float(xreg[i].w);
-            }
-            __syncthreads();
-            if (k0 + KSTEP < a.ld) gload(k0 + KSTEP);
-#pragma unroll 4
-            for (int kk = 0; kk < KSTEP; kk += 2) {
-                const int c = kk + (lane >> 5);
-                float A[IN], B[JM];
+            for (int i = 0; i < IN; i++)
 #pragma unroll
-                for (int i = 0; i < IN; i++) A[i] = s_w[((TN / 2) * wn + 32 * i + (lane & 31)) * FROW + c];
-#pragma unroll
-                for (int j = 0; j < JM; j++) B[j] = s_x[((TM / 2) * wm + 32 * j + (lane & 31)) * FROW + c];
-#pragma unroll
-                for (int i = 0; i < IN; i++)
-#pragma unroll
-                    for (int j = 0; j < JM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[i], B[j], acc[i][j], 0, 0, 0);
-            }
+                for (int j = 0; j < JM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i], B[j], acc[i][j], 0, 0, 0);
         }
         __syncthreads();
     }
     // (the last barrier of the loop is behind every read of the operands)
-    gemm_epilogue<PREC, EPI, IN, JM>(a, acc, (float *)s_raw + wave * gemm_epilogue_floats(IN, JM), mb, m0 + (TM / 2) * wm, mcount, n0 + (TN / 2) * wn, lane);
+    gemm_epilogue<0, EPI, IN, JM>(a, acc, (float *)s_raw + wave * gemm_epilogue_floats(IN, JM), mb, m0 + (TM / 2) * wm, mcount, n0 + (TN / 2) * wn, lane);
+}
+
+// eight fp32 values as three bf16 ones each, their sum exactly: the upper eight bits of the 24, the next eight, the last
+struct GemmParts {
+    l_bf16x8 part[3];
+};
+__device__ __forceinline__ GemmParts gemm_split(float4 a, float4 b) {
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t w[3][8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        w[0][e] = __float_as_uint(x[e]);
+        const float r = x[e] - __uint_as_float(w[0][e] & 0xFFFF0000u);
+        w[1][e] = __float_as_uint(r);
+        w[2][e] = __float_as_uint(r - __uint_as_float(w[1][e] & 0xFFFF0000u));
+    }
+    GemmParts g;
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        l_u32x4 u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) u[q] = __builtin_amdgcn_perm(w[p][2 * q + 1], w[p][2 * q], 0x07060302u);  // (the upper halves of both)
+        g.part[p] = __builtin_bit_cast(l_bf16x8, u);
+    }
+    return g;
+}
+
+// fp32 activations, on the bf16 matrix cores, whose rate is sixteen times that of the fp32 ones: weights are bf16, and an activation is the sum of
+// three bf16 values (gemm_split), so a product is three of theirs, each exact in the fp32 sums.  Against 64 bits the results are nearer than the
+// fp32 instructions' (v_mfma_f32_32x32x2_f32), whose sum takes two products at a time: relative rms error at 256, 1024 and 4096 normal inputs 9.0e-8,
+// 1.25e-7 and 1.4e-7, theirs 2.9e-7, 5.8e-7 and 1.2e-6; all positive 5.2e-8, 5.5e-8 and 5.0e-8, theirs 2.5e-7, 4.9e-7 and 9.8e-7.  For that, sums leave the
+// matrix cores every FOLD steps: their additions truncate, and 4096 positive inputs in one sum of theirs were 3.2e-6 low.
+//
+// Tiles of 64 x 64 results; a step's operands go through LDS, whole rows of 64 inputs, and each of four wavefronts multiplies a quarter of the step's
+// inputs for the whole tile: no operand is read from LDS or split twice.  What bounds a CU is the sum of a step's parts, 48 KB through LDS, 96
+// vector instructions to split with and 12 of the matrix cores a wavefront, 0.4 us with two workgroups on the CU.  KS: as many groups of four
+// wavefronts in a workgroup, each with a share of the steps: for grids that leave a CU one workgroup.  The fp32 instructions and this, us: 509 positions,
+// 4096 x 1024: 41, 20.5; 1024 x 4096: 42, 34.5; 1608 x 1024: 25, 12.6; 2048 positions, 4096 x 1024: 139, 71; 16 matrices of 2048 x 2048, 64 and 192
+// positions each: 132, 43 and 380, 134.  (Activations stored in parts: 6 bytes an element where 4 do, 19 and 39 us for the first two, but products of
+// few positions were 1.2 to 1.3 times slower.  Two steps of loads under way: the same.)
+template <int EPI, bool GROUPED, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, unsigned n_nt) {
+    constexpr int T = 64, KSTEP = 64, BUFFER = T * KSTEP * 6, FOLD = 8;
+    extern __shared__ __align__(16) unsigned char s_raw[];  // [KS][2][BUFFER], then the wavefronts' sums
+    const int t = threadIdx.x & 255, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const uint16_t *W = a.w;
+    int64_t mb = 0;
+    int mcount = a.M;
+    int64_t n0 = (int64_t)blockIdx.y * T;
+    int m0 = blockIdx.x * T;
+    if (GROUPED) {
+        // (blockIdx.y: which half of a block.  Items (block, columns) go to the XCDs as contiguous runs, and workgroups without one come last: with those
+        // between the others, as the columns of a grid of max_tiles, they fell on the same few CUs, and 8 matrices of 2048 x 2048 took 66 us instead of 31)
+        const unsigned n_items = (unsigned)a.n_tiles[0] * n_nt, per = (n_items + 7) / 8, k = blockIdx.x >> 3, item = (blockIdx.x & 7u) * per + k;
+        if (k >= per || item >= n_items) return;
+        const GemmTile gt = a.tiles[item / n_nt];
+        W += gt.expert * a.expert_stride;
+        mb = gt.row0;
+        mcount = gt.n;
+        n0 = (int64_t)(item % n_nt) * T;
+        m0 = T * blockIdx.y;
+        if (m0 >= mcount) return;
+    }
+    // what this thread copies of a step: elements 8 (t % 8) .. of rows t / 8 + 32 i of W, elements 4 (t % 16) .. of rows t / 16 + 16 i of X
+    const int steps = a.ld / KSTEP, share = (steps + KS - 1) / KS, first = share * part;
+    const uint16_t *wrow[2];
+    const float *xrow[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        int64_t r = n0 + (t >> 3) + 32 * i;
+        if (r >= a.n_rows) r = a.n_rows - 1;
+        wrow[i] = W + r * a.ld + 8 * (t & 7);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        int m = m0 + (t >> 4) + 16 * i;
+        if (m >= mcount) m = mcount - 1;  // (repeats the last row; not stored)
+        int64_t row = mb + m;
+        if (a.gather) row = a.gather[row];
+        xrow[i] = (const float *)a.x + row * a.ldx + 4 * (t & 15);
+    }
+    struct Step {
+        l_u32x4 w[2], x[4];
+    };
+    auto gload = [&](Step &f, int step) {
+        const int k0 = KSTEP * min(first + step, steps - 1);
+#pragma unroll
+        for (int i = 0; i < 2; i++) f.w[i] = *(const l_u32x4 *)(wrow[i] + k0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) f.x[i] = *(const l_u32x4 *)(xrow[i] + k0);
+        __builtin_amdgcn_sched_barrier(0);  // (requests stay in the order of the steps: a step's wait leaves the next one's under way)
+    };
+    l_f32x16 acc[2][2], total[2][2];
+    auto clear = [&](l_f32x16(&v)[2][2]) {
+#pragma unroll
+        for (int o = 0; o < 4; o++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) v[o >> 1][o & 1][r] = 0.0f;
+    };
+    auto run = [&](Step &f, int step, int buffer) {
+        l_u32x4 *s_w = (l_u32x4 *)(s_raw + (2 * part + buffer) * BUFFER), *s_x = s_w + T * 8;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = (t >> 3) + 32 * i;
+            s_w[r * 8 + ((t & 7) ^ gemm_swz(r))] = f.w[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = (t >> 4) + 16 * i;
+            s_x[r * 16 + ((t & 15) ^ (r & 15))] = f.x[i];
+        }
+        l_lds_barrier();
+        gload(f, step + 1);
+        if (KS > 1 && first + step >= steps) return;
+        // (a wavefront takes a quarter of the step's inputs)
+        const int c = 2 * wave + (lane >> 5);
+        l_bf16x8 A[2];
+        GemmParts B[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = 32 * i + (lane & 31);
+            A[i] = __builtin_bit_cast(l_bf16x8, s_w[r * 8 + (c ^ gemm_swz(r))]);
+            B[i] = gemm_split(__builtin_bit_cast(float4, s_x[r * 16 + ((2 * c) ^ (r & 15))]), __builtin_bit_cast(float4, s_x[r * 16 + ((2 * c + 1) ^ (r & 15))]));
+        }
+#pragma unroll
+        for (int p = 2; p >= 0; p--)  // (the small parts first)
+#pragma unroll
+            for (int o = 0; o < 4; o++)
+                acc[o >> 1][o & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[o >> 1], B[o & 1].part[p], acc[o >> 1][o & 1], 0, 0, 0);
+    };
+    Step f;
+    gload(f, 0);
+    clear(total);
+    clear(acc);
+    auto fold = [&] {
+#pragma unroll
+        for (int o = 0; o < 4; o++) total[o >> 1][o & 1] += acc[o >> 1][o & 1];
+        clear(acc);
+    };
+    const int pairs = share & ~1;
+    for (int u0 = 0; u0 < pairs; u0 += FOLD) {
+        const int u1 = min(u0 + FOLD, pairs);
+        for (int u = u0; u < u1; u += 2) {
+            run(f, u, 0);
+            run(f, u + 1, 1);
+        }
+        fold();
+    }
+    if (share & 1) {
+        run(f, pairs, 0);
+        fold();
+    }
+    // the four wavefronts' sums of a 32 x 32 tile each
+    l_lds_barrier();
+    float4 *sums = (float4 *)s_raw;
+#pragma unroll
+    for (int o = 0; o < 4; o++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const l_f32x16 &v = total[o >> 1][o & 1];
+            sums[((o * 4 * KS + 4 * part + wave) * 4 + q) * 64 + lane] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        }
+    l_lds_barrier();
+    if (part) return;
+    l_f32x16 mine[1][1];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        float4 v = sums[(wave * 4 * KS * 4 + q) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4 * KS; w++) {
+            const float4 z = sums[((wave * 4 * KS + w) * 4 + q) * 64 + lane];
+            v = make_float4(v.x + z.x, v.y + z.y, v.z + z.z, v.w + z.w);
+        }
+        mine[0][0][4 * q] = v.x, mine[0][0][4 * q + 1] = v.y, mine[0][0][4 * q + 2] = v.z, mine[0][0][4 * q + 3] = v.w;
+    }
+    // (a wavefront's own quarter of s_raw: no other one reads it any more)
+    static_assert(4 * gemm_epilogue_floats(1, 1) <= 16384 * KS, "the epilogue's floats lie among a wavefront's own sums");
+    float *own = (float *)s_raw + 4096 * KS * wave;
+    m0 += 32 * (wave & 1), n0 += 32 * (wave >> 1);
+    // An infinite activation's parts are itself and NaNs, and an infinite weight times a part that is zero is one: such results are
+    // computed again, as plain sums.
+    bool nan = false;
+#pragma unroll
+    for (int r = 0; r < 16; r++) nan |= mine[0][0][r] != mine[0][0][r];
+    if (__any(nan)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) own[64 * r + lane] = mine[0][0][r];
+        const int m = m0 + (lane & 31);
+        const float *x = (const float *)a.x + (a.gather ? (int64_t)a.gather[mb + min(m, mcount - 1)] : mb + min(m, mcount - 1)) * a.ldx;
+#pragma nounroll
+        for (int r = 0; r < 16; r++) {
+            const int64_t n = n0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            float v = own[64 * r + lane];
+            if (v != v && m < mcount && n < a.n_rows) {
+                v = 0.0f;
+                const uint16_t *w = W + n * a.ld;
+                for (int k = 0; k < a.ld && v == v; k++) v = fmaf(l_bf16(w[k]), x[k], v);
+                own[64 * r + lane] = v;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) mine[0][0][r] = own[64 * r + lane];
+    }
+    gemm_epilogue<1, EPI, 1, 1>(a, mine, own, mb, m0, mcount, n0, lane);
+}
+
+template <int EPI, bool GROUPED, int KS>
+static hipError_t gemm_parts_go(hipStream_t s, const GemmArgs &a, unsigned n_nt) {
+    constexpr unsigned lds = KS * 65536u;
+    if (KS > 1) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_parts_kernel<EPI, GROUPED, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid = GROUPED ? dim3(8 * (((unsigned)a.max_tiles * n_nt + 7) / 8), L_GEMM_TILE / 64) : dim3((unsigned)((a.M + 63) / 64), n_nt);
+    hipLaunchKernelGGL((gemm_parts_kernel<EPI, GROUPED, KS>), grid, dim3(256 * KS), lds, s, a, n_nt);
+    return hipGetLastError();
+}
+template <int EPI, bool GROUPED>
+static hipError_t gemm_parts_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
+    const unsigned n_nt = (unsigned)((cols + 63) / 64);
+    // (one workgroup a CU: two groups, from 512 inputs on.  us with one and two: 1024 x 4096, 509 positions (128 tiles) 48, 34.5; x 1024: 15, 12.3;
+    // x 256: 6.7, 6.7; 3392 x 1024 (424 tiles): 20, 23.  A matrix's last block of a grouped product is half full on average)
+    const int64_t halves = GROUPED ? (a.M + 63) / 64 + a.M / (2 * max(a.rows_each, 1)) : (a.M + 63) / 64;
+    return a.ld >= 512 && halves * n_nt <= 256 ? gemm_parts_go<EPI, GROUPED, 2>(s, a, n_nt) : gemm_parts_go<EPI, GROUPED, 1>(s, a, n_nt);
 }
 
 template <int PREC, int EPI>
@@ -163,24 +337,21 @@ static hipError_t gemm_launch(hipStream_t s, const GemmArgs &a) {
     if (a.tiles) {
         if (EPI != GE_STORE && EPI != GE_UP && EPI != GE_GLU) return hipErrorInvalidValue;
         constexpr int E = EPI == GE_UP || EPI == GE_GLU ? EPI : GE_STORE;
-        if (cols > 64) {
-            hipLaunchKernelGGL((gemm_kernel<PREC, E, 128, L_GEMM_TILE, true>), dim3((unsigned)a.max_tiles, (unsigned)((cols + 127) / 128)),
-                               dim3(256), 0, s, a);
-        } else {
-            hipLaunchKernelGGL((gemm_kernel<PREC, E, 64, L_GEMM_TILE, true>), dim3((unsigned)a.max_tiles, (unsigned)((cols + 63) / 64)),
-                               dim3(256), 0, s, a);
-        }
+        if (PREC) return gemm_parts_launch<E, true>(s, a, cols);
+        if (cols > 64)
+            hipLaunchKernelGGL((gemm_kernel<E, 128, L_GEMM_TILE, true>), dim3((unsigned)a.max_tiles, (unsigned)((cols + 127) / 128)), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((gemm_kernel<E, 64, L_GEMM_TILE, true>), dim3((unsigned)a.max_tiles, (unsigned)((cols + 63) / 64)), dim3(256), 0, s, a);
         return hipGetLastError();
     }
+    if (PREC) return gemm_parts_launch<EPI, false>(s, a, cols);
     // (up to two steps of 64 inputs, a tile is its loads' latency and its epilogue: four small ones a CU wait for each other less.  2048 positions x 2048
     // rows of 128 inputs, softplus or sigmoid behind them: 11 and 10 us, in tiles of 128 x 128 16 and 14)
     const int64_t big = ((cols + 127) / 128) * ((a.M + 127) / 128);
-    if (big >= 256 && (PREC || a.ld > 128))
-        hipLaunchKernelGGL((gemm_kernel<PREC, EPI, 128, 128, false>), dim3((unsigned)((a.M + 127) / 128), (unsigned)((cols + 127) / 128)),
-                           dim3(256), 0, s, a);
+    if (big >= 256 && a.ld > 128)
+        hipLaunchKernelGGL((gemm_kernel<EPI, 128, 128, false>), dim3((unsigned)((a.M + 127) / 128), (unsigned)((cols + 127) / 128)), dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL((gemm_kernel<PREC, EPI, 64, 64, false>), dim3((unsigned)((a.M + 63) / 64), (unsigned)((cols + 63) / 64)),
-                           dim3(256), 0, s, a);
+        hipLaunchKernelGGL((gemm_kernel<EPI, 64, 64, false>), dim3((unsigned)((a.M + 63) / 64), (unsigned)((cols + 63) / 64)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

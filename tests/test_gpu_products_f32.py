@@ -1,0 +1,61 @@
+"""fp32 products of a prompt on the bf16 matrix cores (activations in three exact parts): odd numbers of positions, rows and inputs, one and two groups of
+wavefronts a tile, blocks of an expert's rows, and infinite weights, against the oracle."""
+import numpy as np
+import pytest
+
+import layered_cases as lc
+from oracle import layered_np as ref
+
+pytestmark = pytest.mark.gpu
+
+# fp32 sums of up to 1000 products, relative to the rms of the logits: as the other fp32 runs of layered models
+TOL = 2e-5
+
+
+def check(pkg, c, t, n):
+    tok = lc.tokens(n, c["vocab"])
+    s = ref.Sequence(c, t)
+    want = np.array([s.step(int(a)) for a in tok])
+    dev = lc.language_model(pkg, c, t, seq_len=n, precision="float32").device()
+    got = dev.prefill_logits(tok, np.arange(n), 0)
+    dev.close()
+    return got, want
+
+
+# (width: inputs of the logits, vocabulary, positions): more results each than small products have; 60 and 449 inputs are one step and eight, 1000 sixteen in two
+# groups, 577 ten in two groups, 520 x 9001 more tiles than CUs
+@pytest.mark.parametrize("width,vocab,n", [(60, 5431, 97), (449, 4099, 65), (577, 2049, 129), (1000, 4100, 64), (520, 9001, 130)])
+def test_logits(pkg, width, vocab, n):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16)], width=width, vocab=vocab)
+    t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 3).items()}
+    got, want = check(pkg, c, t, n)
+    assert lc.error(got, want) <= TOL
+
+
+# (experts, chosen, elements, width, positions): about 60, 65 and 150 positions an expert
+@pytest.mark.parametrize("experts,top,ff,width,n", [(9, 3, 530, 72, 181), (4, 2, 1030, 600, 130), (3, 3, 333, 515, 150)])
+def test_experts(pkg, experts, top, ff, width, n):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16, mlp=lc.moe(experts, top, ff))], width=width, vocab=50)
+    t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 4).items()}
+    t = lc.settle_routers(c, t, 4)
+    got, want = check(pkg, c, t, n)
+    assert lc.error(got, want) <= TOL
+
+
+def test_infinite_weights(pkg):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16)], width=100, vocab=5500)
+    t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 5).items()}
+    got, want = check(pkg, c, t, 100)
+    assert lc.error(got, want) <= TOL
+    head = [k for k in t if t[k].shape == (5500, 100)]
+    assert head
+    # a row of the logits' matrix alone: the model's tokens are smaller numbers than it
+    tok = lc.tokens(100, c["vocab"])
+    row = next(r for r in range(5499, 0, -1) if r not in tok)
+    for k in head:
+        t[k] = t[k].copy()
+        t[k][row, 37] = np.inf
+    inf, _ = check(pkg, c, t, 100)
+    assert np.isinf(inf[:, row]).all() and (inf[:, row] > 0).any() and (inf[:, row] < 0).any()
+    rest = np.arange(5500) != row
+    assert np.array_equal(inf[:, rest], got[:, rest])
