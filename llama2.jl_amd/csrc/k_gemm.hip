@@ -135,23 +135,23 @@ __device__ __forceinline__ GemmParts gemm_split(float4 a, float4 b) {
 // 1.25e-7 and 1.4e-7, theirs 2.9e-7, 5.8e-7 and 1.2e-6; all positive 5.2e-8, 5.5e-8 and 5.0e-8, theirs 2.5e-7, 4.9e-7 and 9.8e-7.  For that, sums leave the
 // matrix cores every FOLD steps: their additions truncate, and 4096 positive inputs in one sum of theirs were 3.2e-6 low.
 //
-// Tiles of 64 x 64 results; a step's operands go through LDS, whole rows of 64 inputs, and each of four wavefronts multiplies a quarter of the step's
+// Tiles of 64 rows and TM positions; a step's operands go through LDS, whole rows of 64 inputs, and each of four wavefronts multiplies a quarter of the step's
 // inputs for the whole tile: no operand is read from LDS or split twice.  What bounds a CU is the sum of a step's parts, 48 KB through LDS, 96
-// vector instructions to split with and 12 of the matrix cores a wavefront, 0.4 us with two workgroups on the CU.  KS: as many groups of four
+// vector instructions to split with and 12 of the matrix cores a wavefront, 0.4 us at 64 positions with two workgroups on the CU.  KS: as many groups of four
 // wavefronts in a workgroup, each with a share of the steps: for grids that leave a CU one workgroup.  The fp32 instructions and this, us: 509 positions,
-// 4096 x 1024: 41, 20.5; 1024 x 4096: 42, 34.5; 1608 x 1024: 25, 12.6; 2048 positions, 4096 x 1024: 139, 71; 16 matrices of 2048 x 2048, 64 and 192
+// 4096 x 1024: 41, 20.5; 1024 x 4096: 42, 25; 1608 x 1024: 25, 12.6; 2048 positions, 4096 x 1024: 139, 71; 16 matrices of 2048 x 2048, 64 and 192
 // positions each: 132, 43 and 380, 134.  (Activations stored in parts: 6 bytes an element where 4 do, 19 and 39 us for the first two, but products of
 // few positions were 1.2 to 1.3 times slower.  Two steps of loads under way: the same.)
-template <int EPI, bool GROUPED, int KS>
+template <int EPI, bool GROUPED, int KS, int TM>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, unsigned n_nt) {
-    constexpr int T = 64, KSTEP = 64, BUFFER = T * KSTEP * 6, FOLD = 8;
+    constexpr int T = 64, KSTEP = 64, BUFFER = (2 * T + 4 * TM) * KSTEP, FOLD = 8, JM = TM / 32, XL = TM / 16;
     extern __shared__ __align__(16) unsigned char s_raw[];  // [KS][2][BUFFER], then the wavefronts' sums
     const int t = threadIdx.x & 255, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const uint16_t *W = a.w;
     int64_t mb = 0;
     int mcount = a.M;
     int64_t n0 = (int64_t)blockIdx.y * T;
-    int m0 = blockIdx.x * T;
+    int m0 = blockIdx.x * TM;
     if (GROUPED) {
         // (blockIdx.y: which half of a block.  Items (block, columns) go to the XCDs as contiguous runs, and workgroups without one come last: with those
         // between the others, as the columns of a grid of max_tiles, they fell on the same few CUs, and 8 matrices of 2048 x 2048 took 66 us instead of 31)
@@ -162,13 +162,13 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
         mb = gt.row0;
         mcount = gt.n;
         n0 = (int64_t)(item % n_nt) * T;
-        m0 = T * blockIdx.y;
+        m0 = TM * blockIdx.y;
         if (m0 >= mcount) return;
     }
     // what this thread copies of a step: elements 8 (t % 8) .. of rows t / 8 + 32 i of W, elements 4 (t % 16) .. of rows t / 16 + 16 i of X
     const int steps = a.ld / KSTEP, share = (steps + KS - 1) / KS, first = share * part;
     const uint16_t *wrow[2];
-    const float *xrow[4];
+    const float *xrow[XL];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         int64_t r = n0 + (t >> 3) + 32 * i;
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
         wrow[i] = W + r * a.ld + 8 * (t & 7);
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < XL; i++) {
         int m = m0 + (t >> 4) + 16 * i;
         if (m >= mcount) m = mcount - 1;  // (repeats the last row; not stored)
         int64_t row = mb + m;
@@ -184,22 +184,22 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
         xrow[i] = (const float *)a.x + row * a.ldx + 4 * (t & 15);
     }
     struct Step {
-        l_u32x4 w[2], x[4];
+        l_u32x4 w[2], x[XL];
     };
     auto gload = [&](Step &f, int step) {
         const int k0 = KSTEP * min(first + step, steps - 1);
 #pragma unroll
         for (int i = 0; i < 2; i++) f.w[i] = *(const l_u32x4 *)(wrow[i] + k0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) f.x[i] = *(const l_u32x4 *)(xrow[i] + k0);
+        for (int i = 0; i < XL; i++) f.x[i] = *(const l_u32x4 *)(xrow[i] + k0);
         __builtin_amdgcn_sched_barrier(0);  // (requests stay in the order of the steps: a step's wait leaves the next one's under way)
     };
-    l_f32x16 acc[2][2], total[2][2];
-    auto clear = [&](l_f32x16(&v)[2][2]) {
+    l_f32x16 acc[2][JM], total[2][JM];
+    auto clear = [&](l_f32x16(&v)[2][JM]) {
 #pragma unroll
-        for (int o = 0; o < 4; o++)
+        for (int o = 0; o < 2 * JM; o++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) v[o >> 1][o & 1][r] = 0.0f;
+            for (int r = 0; r < 16; r++) v[o / JM][o % JM][r] = 0.0f;
     };
     auto run = [&](Step &f, int step, int buffer) {
         l_u32x4 *s_w = (l_u32x4 *)(s_raw + (2 * part + buffer) * BUFFER), *s_x = s_w + T * 8;
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
             s_w[r * 8 + ((t & 7) ^ gemm_swz(r))] = f.w[i];
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < XL; i++) {
             const int r = (t >> 4) + 16 * i;
             s_x[r * 16 + ((t & 15) ^ (r & 15))] = f.x[i];
         }
@@ -219,18 +219,18 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
         // (a wavefront takes a quarter of the step's inputs)
         const int c = 2 * wave + (lane >> 5);
         l_bf16x8 A[2];
-        GemmParts B[2];
+        GemmParts B[JM];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int r = 32 * i + (lane & 31);
             A[i] = __builtin_bit_cast(l_bf16x8, s_w[r * 8 + (c ^ gemm_swz(r))]);
-            B[i] = gemm_split(__builtin_bit_cast(float4, s_x[r * 16 + ((2 * c) ^ (r & 15))]), __builtin_bit_cast(float4, s_x[r * 16 + ((2 * c + 1) ^ (r & 15))]));
+            if (i < JM) B[i] = gemm_split(__builtin_bit_cast(float4, s_x[r * 16 + ((2 * c) ^ (r & 15))]), __builtin_bit_cast(float4, s_x[r * 16 + ((2 * c + 1) ^ (r & 15))]));
         }
 #pragma unroll
         for (int p = 2; p >= 0; p--)  // (the small parts first)
 #pragma unroll
-            for (int o = 0; o < 4; o++)
-                acc[o >> 1][o & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[o >> 1], B[o & 1].part[p], acc[o >> 1][o & 1], 0, 0, 0);
+            for (int o = 0; o < 2 * JM; o++)
+                acc[o / JM][o % JM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[o / JM], B[o % JM].part[p], acc[o / JM][o % JM], 0, 0, 0);
     };
     Step f;
     gload(f, 0);
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
     clear(acc);
     auto fold = [&] {
 #pragma unroll
-        for (int o = 0; o < 4; o++) total[o >> 1][o & 1] += acc[o >> 1][o & 1];
+        for (int o = 0; o < 2 * JM; o++) total[o / JM][o % JM] += acc[o / JM][o % JM];
         clear(acc);
     };
     const int pairs = share & ~1;
@@ -258,14 +258,14 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
     l_lds_barrier();
     float4 *sums = (float4 *)s_raw;
 #pragma unroll
-    for (int o = 0; o < 4; o++)
+    for (int o = 0; o < 2 * JM; o++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const l_f32x16 &v = total[o >> 1][o & 1];
+            const l_f32x16 &v = total[o / JM][o % JM];
             sums[((o * 4 * KS + 4 * part + wave) * 4 + q) * 64 + lane] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
         }
     l_lds_barrier();
-    if (part) return;
+    if (part || wave >= 2 * JM) return;
     l_f32x16 mine[1][1];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
     // (a wavefront's own quarter of s_raw: no other one reads it any more)
     static_assert(4 * gemm_epilogue_floats(1, 1) <= 16384 * KS, "the epilogue's floats lie among a wavefront's own sums");
     float *own = (float *)s_raw + 4096 * KS * wave;
-    m0 += 32 * (wave & 1), n0 += 32 * (wave >> 1);
+    m0 += 32 * (wave % JM), n0 += 32 * (wave / JM);
     // An infinite activation's parts are itself and NaNs, and an infinite weight times a part that is zero is one: such results are
     // computed again, as plain sums.
     bool nan = false;
@@ -308,24 +308,29 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
     gemm_epilogue<1, EPI, 1, 1>(a, mine, own, mb, m0, mcount, n0, lane);
 }
 
-template <int EPI, bool GROUPED, int KS>
+template <int EPI, bool GROUPED, int KS, int TM>
 static hipError_t gemm_parts_go(hipStream_t s, const GemmArgs &a, unsigned n_nt) {
-    constexpr unsigned lds = KS * 65536u;
-    if (KS > 1) {
-        const hipError_t e = hipFuncSetAttribute((const void *)gemm_parts_kernel<EPI, GROUPED, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    constexpr unsigned lds = KS * TM * 1024u;  // (the sums; the operands take three quarters of it, or all)
+    static_assert(2 * (128 + 4 * TM) * 64 <= TM * 1024, "two steps' operands lie in it");
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_parts_kernel<EPI, GROUPED, KS, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    const dim3 grid = GROUPED ? dim3(8 * (((unsigned)a.max_tiles * n_nt + 7) / 8), L_GEMM_TILE / 64) : dim3((unsigned)((a.M + 63) / 64), n_nt);
-    hipLaunchKernelGGL((gemm_parts_kernel<EPI, GROUPED, KS>), grid, dim3(256 * KS), lds, s, a, n_nt);
+    const dim3 grid = GROUPED ? dim3(8 * (((unsigned)a.max_tiles * n_nt + 7) / 8), L_GEMM_TILE / TM) : dim3((unsigned)((a.M + TM - 1) / TM), n_nt);
+    hipLaunchKernelGGL((gemm_parts_kernel<EPI, GROUPED, KS, TM>), grid, dim3(256 * KS), lds, s, a, n_nt);
     return hipGetLastError();
 }
 template <int EPI, bool GROUPED>
 static hipError_t gemm_parts_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
     const unsigned n_nt = (unsigned)((cols + 63) / 64);
-    // (one workgroup a CU: two groups, from 512 inputs on.  us with one and two: 1024 x 4096, 509 positions (128 tiles) 48, 34.5; x 1024: 15, 12.3;
-    // x 256: 6.7, 6.7; 3392 x 1024 (424 tiles): 20, 23.  A matrix's last block of a grouped product is half full on average)
-    const int64_t halves = GROUPED ? (a.M + 63) / 64 + a.M / (2 * max(a.rows_each, 1)) : (a.M + 63) / 64;
-    return a.ld >= 512 && halves * n_nt <= 256 ? gemm_parts_go<EPI, GROUPED, 2>(s, a, n_nt) : gemm_parts_go<EPI, GROUPED, 1>(s, a, n_nt);
+    // Where tiles of 64 x 64 leave a CU one workgroup: two groups of wavefronts, and where they leave half the CUs none, 32 positions a tile.  us with one
+    // group, two, two and 32 positions: 509 positions, 1024 x 1024 (128 tiles) 15.2, 12.2, 9.3; x 4096: 48, 34.5, 25; x 256: 6.7, 6.8, 5.3; 2048 x 1024 (256):
+    // 15.9, 12.9, 12.2; x 256: 7.3, 7.3, 6.7; 100 positions, 8192 x 1024 (256) 15.8, 12.9, 14.0; 509, 3392 x 1024 (424) 20, 23, 21.  (A matrix's last block of
+    // a grouped product is half full on average.)
+    const int64_t halves = GROUPED ? (a.M + 63) / 64 + a.M / (2 * max(a.rows_each, 1)) : (a.M + 63) / 64, tiles = halves * n_nt;
+    if constexpr (!GROUPED)
+        if (tiles <= 128 || (a.ld < 512 && tiles <= 256)) return gemm_parts_go<EPI, false, 2, 32>(s, a, n_nt);
+    return a.ld >= 512 && tiles <= 256 ? gemm_parts_go<EPI, GROUPED, 2, 64>(s, a, n_nt) : gemm_parts_go<EPI, GROUPED, 1, 64>(s, a, n_nt);
 }
 
 template <int PREC, int EPI>

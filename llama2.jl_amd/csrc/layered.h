@@ -130,17 +130,18 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // and 1.0 to 5.  Plain: up to 128 positions (1.5 to 13, 256 to 32 000 rows), otherwise where tiles of 64 x 64 are at most 256 (8192 rows, 128
 // positions: 1.6 to 2.0).
 //
-// fp32, whose tiles of 64 x 64 run on the bf16 matrix cores: up to 2^18 results in all, 2^19 of at most 256 inputs, and up to 8 positions.  512 to 4096 inputs, both ways:
-// 2^17 results (2048 rows, 64 positions; 256 x 509) 5.2 to 21 and 7.9 to 32 us, 2^18 (4096 x 64; 2048 x 128; 512 x 509) 7.6 to 39 and 8.0 to 40,
-// 2^19 (4096 x 128; 1024 x 509) 9.3 to 42 and 8.5 to 39, of 256 inputs 6.4 and 6.7.  8, 16 and 64 matrices: 512 rows, 32 positions each, 2^17 to 2^18 in all, 5.6 to 22 and
-// 8.4 to 21; 2048 rows, 32 each, 2^19 to 2^20, 13 to 76 and 9.4 to 40.  128 256 rows of 2048 inputs, 1 position: 118 and 139; 9: 135 and 142.
+// fp32, whose tiles run on the bf16 matrix cores: up to 8 positions, and up to 2^17 results in all, 2^18 of up to 16 positions or of several matrices.
+// 256 to 4096 inputs, both ways, us: 2^17 results (2048 rows, 64 positions; 256 x 509) 4.1 to 20 and 4.7 to 23, 2^18 (4096 x 64; 2048 x 128; 512 x 509)
+// 5.2 to 39 and 4.9 to 30.  16 000 rows, 9 and 16 positions: 11 to 39 and 13 to 41; 13 to 48 and 13 to 41.  128 256 rows of 2048 inputs, 1 position:
+// 118 and 139; 9: 135 and 142.  8 and 16 matrices of 512 rows, 2^17 results in all: 5.6 to 15 and 8.3 to 20; 2^18: 7.6 to 22 and 8.4 to 21; 2048 rows,
+// 32 positions each, 2^19 to 2^20: 13 to 76 and 9.6 to 40.
 #define L_FEW_M 128
 #define L_FEW_EACH 48
 #define L_FEW_TILES 256
 #define L_FEW_M_F32 8
-#define L_FEW_RESULTS_F32 262144
+#define L_FEW_RESULTS_F32 131072
 inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
-    if (prec) return a.M <= L_FEW_M_F32 || a.M * cols <= (a.ld <= 256 ? 2 : 1) * L_FEW_RESULTS_F32;
+    if (prec) return a.M <= L_FEW_M_F32 || a.M * cols <= (a.tiles || a.M <= 16 ? 2 : 1) * L_FEW_RESULTS_F32;
     if (a.tiles) return a.rows_each <= L_FEW_EACH;
     return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= L_FEW_TILES;
 }

@@ -22,9 +22,9 @@ def check(pkg, c, t, n):
     return got, want
 
 
-# (width: inputs of the logits, vocabulary, positions): more results each than small products have; 60 and 449 inputs are one step and eight, 1000 sixteen in two
-# groups, 577 ten in two groups, 520 x 9001 more tiles than CUs
-@pytest.mark.parametrize("width,vocab,n", [(60, 5431, 97), (449, 4099, 65), (577, 2049, 129), (1000, 4100, 64), (520, 9001, 130)])
+# (width: inputs of the logits, vocabulary, positions): more results each than small products have.  60 inputs are one step, 449 eight, 577 ten, 1000
+# sixteen, a group's share being half of them; tiles of 32 and 64 positions, the last with one, two groups and (9001) one
+@pytest.mark.parametrize("width,vocab,n", [(60, 2731, 97), (60, 12345, 65), (449, 4099, 65), (577, 2049, 129), (1000, 8200, 64), (1000, 4110, 161), (520, 9001, 129)])
 def test_logits(pkg, width, vocab, n):
     c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16)], width=width, vocab=vocab)
     t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 3).items()}
