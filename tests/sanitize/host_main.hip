@@ -171,6 +171,21 @@ static void check_product_rule() {
     // ... and where the smaller kernel is up to 8 % behind
     EXPECT(!few(1, 0, 14336, 96) && !few(1, 0, 32000, 64));
 }
+// ... and whether the fp32 tiles on the bf16 matrix cores come first, at sizes where the other takes at least 1.1 times as long (measured)
+static bool parts(int experts, int64_t cols, int each) {
+    GemmTile tile{};
+    GemmArgs a;
+    a.n_rows = cols;
+    a.M = experts ? experts * each : each;
+    a.rows_each = each;
+    a.tiles = experts ? &tile : nullptr;
+    return k_parts_pays(a, cols);
+}
+static void check_parts_rule() {
+    EXPECT(parts(0, 1024, 509) && parts(0, 4096, 64) && parts(0, 512, 509) && parts(0, 32000, 24) && parts(0, 32000, 2048));
+    EXPECT(!parts(0, 256, 509) && !parts(0, 2048, 64) && !parts(0, 4096, 17) && !parts(0, 8192, 16) && !parts(0, 128256, 1) && !parts(0, 16, 2048));
+    EXPECT(parts(16, 1024, 64) && parts(16, 2048, 32) && parts(64, 512, 48) && !parts(8, 512, 32) && !parts(16, 512, 16) && !parts(8, 1024, 1));
+}
 
 // a decode product's workgroups have the LDS they need at every size that a model may have
 static void check_rows_plan() {
@@ -233,6 +248,7 @@ int main() {
     check_tiles_plan();
     check_small_plan();
     check_product_rule();
+    check_parts_rule();
     check_rows_plan();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
