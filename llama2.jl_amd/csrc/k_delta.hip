@@ -3,6 +3,7 @@
 //   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q = (decayed S)^T q + (k . q) u
 // so both products of a token are taken of the decayed state, before its own write.
 // The value columns of S are independent of one another: workgroups split them.
+#include "delta_plan.h"
 #include "layered_dev.h"
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -598,24 +599,7 @@ hipError_t k_delta_scan(hipStream_t s, const DeltaShape &d, const float *qkv, co
 // indexes taken as k = 4 (l / 16) + r, a result is the next product's B operand as it stands, and an A operand's four steps are
 // one 16-byte word of lane l: (row l % 16; columns 4 (l / 16) .. + 3).
 // ---------------------------------------------------------------------------------------------------------------
-#define WK_T 32  // tokens of a chunk
 typedef float d_f32x4 __attribute__((ext_vector_type(4)));
-
-// the record of one (chunk, head), NT tiles of 16 key channels (a multiple of 4) and NC of 16 value columns, in words of [64 lanes][4]:
-// kt, qt [2 tiles of tokens][NT]; kh [NT][2]; B [3: first, second, second x first tile]; U (before the walk, T V) [NC][2]; S0 [NC][NT]; then
-// exp(G_31) [16 NT]
-struct DeltaRec {
-    int NT, NC;
-    __host__ __device__ DeltaRec(int nt, int V) : NT(nt), NC((V + 15) / 16) {}
-    __host__ __device__ int kt(int tile, int i) const { return 256 * (tile * NT + i); }
-    __host__ __device__ int qt(int tile, int i) const { return 256 * ((2 + tile) * NT + i); }
-    __host__ __device__ int kh(int i, int tile) const { return 256 * (4 * NT + 2 * i + tile); }
-    __host__ __device__ int b(int i) const { return 256 * (6 * NT + i); }
-    __host__ __device__ int u(int c, int tile) const { return 256 * (6 * NT + 3 + 2 * c + tile); }
-    __host__ __device__ int s0(int c, int i) const { return 256 * (6 * NT + 3 + 2 * NC + c * NT + i); }
-    __host__ __device__ int gc() const { return 256 * (6 * NT + 3 + 2 * NC + NC * NT); }
-    __host__ __device__ int floats() const { return gc() + 16 * NT; }
-};
 
 #define WK_LD(DP_) ((DP_) + 4)  // LDS row of DP_ channels
 #define WK_S 20                 // LDS row of 16 tokens
@@ -1049,7 +1033,6 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaShape d, const floa
             for (int64_t j = (int64_t)HV + lane; j < lda; j += 64) l_store_act<PREC>(outa, (int64_t)(m0 + i) * lda + j, 0.0f);
 }
 
-int64_t delta_walk_floats(const DeltaShape &d, int M) { return (int64_t)((M + WK_T - 1) / WK_T) * d.H * DeltaRec((d.D + 63) / 64 * 4, d.V).floats(); }
 template <int NW>
 static hipError_t delta_walk_launch(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0,
                                     float *rec, const float *gate, const float *normw, void *outa, int64_t lda, int prec) {
@@ -1068,15 +1051,276 @@ static hipError_t delta_walk_launch(hipStream_t s, const DeltaShape &d, const fl
         hipLaunchKernelGGL((delta_out_kernel<0, NW>), g1, dim3(256), 0, s, d, rec, gate, normw, M, outa, lda);
     return hipGetLastError();
 }
-hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M,
-                        int pos0, float *rec, const float *gate, const float *normw, void *outa, int64_t lda, int prec) {
-    if (d.D > 256 || d.V > 256 || M < 1) return hipErrorInvalidValue;
-    switch ((d.D + 63) / 64) {
-    case 1: return delta_walk_launch<1>(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
-    case 2: return delta_walk_launch<2>(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
-    case 3: return delta_walk_launch<3>(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
-    default: return delta_walk_launch<4>(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
+// ---------------------------------------------------------------------------------------------------------------
+// the same in chunks of 16 tokens, where delta_plan.h says so: the walk makes the outputs too,
+//   U = T (V - (k exp(G)) S0),   O = (q exp(G)) S0 + B U,   S = diag(exp(G_15)) S0 + (k exp(G_15 - G))^T U
+// and no state goes to memory but the last.  delta_chunk16_kernel makes the scaled rows, T and B, and the head norm is a launch of its own.
+//
+// the record of one (chunk, head), NT tiles of 16 key channels (a multiple of 4): kt, qt, kh: [NT][64][4]; T, B: [64][4]; exp(G_15): [16 NT]
+// ---------------------------------------------------------------------------------------------------------------
+#define CH_T DELTA_CHUNK16
+
+template <int NW>
+__global__ __launch_bounds__(256) void delta_chunk16_kernel(DeltaShape d, const float *qkv, const float *beta, const float *lg, int M,
+                                                          float *rec) {
+    constexpr int NT = 4 * NW, DP = 16 * NT;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // s_g: the decays, then their logarithms' sums
+    __shared__ __align__(16) float s_q[CH_T * DP], s_k[CH_T * DP], s_g[CH_T * DP];
+    __shared__ float s_A[CH_T][CH_T + 1], s_B[CH_T][CH_T + 1], s_T[CH_T][CH_T + 1], s_b[CH_T];
+    const int ch = blockIdx.x, h = blockIdx.y, kvh = h / (d.H / d.G), m0 = ch * CH_T, n = min(CH_T, M - m0);
+    const int D = d.D, C = d.channels(), GD = d.G * D;
+    // a thread has one column of 16 / (256 / columns) rows at a time: column e, rows r0, r0 + RS, ...
+    constexpr int CB = DP < 256 ? DP : 256, RS = 256 / CB, NR = CH_T / RS;  // (DP: 64, 128, 192 or 256)
+    const int e0 = t % CB, r0 = t / CB;
+    float l[NR];
+    if (r0 < RS) {
+        float q[NR], k[NR];
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const int tt = r0 + RS * i;
+            q[i] = k[i] = l[i] = 0.0f;
+            if (tt < n && e0 < D) {
+                const float *row = qkv + (int64_t)(m0 + tt) * C + kvh * D + e0;
+                q[i] = row[0];
+                k[i] = row[GD];
+                l[i] = lg[((int64_t)(m0 + tt) * d.H + h) * D + e0];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const int at = (r0 + RS * i) * DP + e0;
+            s_q[at] = q[i];
+            s_k[at] = k[i];
+            s_g[at] = expf(l[i]);
+        }
     }
+    if (t < CH_T) s_b[t] = t < n ? beta[(int64_t)(m0 + t) * d.H + h] : 0.0f;
+    __syncthreads();
+    // A and B: a group of 16 lanes has row j of the pairs (j, i > j), each lane every 16th channel; r = k_j times the decays of
+    // the tokens after j
+    {
+        const int j = 4 * wave + (lane >> 4), sl = lane & 15;
+        float a[CH_T], b[CH_T];
+#pragma unroll
+        for (int i = 0; i < CH_T; i++) a[i] = b[i] = 0.0f;
+        for (int e = sl; e < D; e += 16) {
+            float r = s_k[j * DP + e];
+#pragma unroll
+            for (int i = 0; i < CH_T; i++) {
+                if (i > j) r *= s_g[i * DP + e];
+                const float u = i >= j ? r : 0.0f;
+                a[i] = fmaf(s_k[i * DP + e], u, a[i]);
+                b[i] = fmaf(s_q[i * DP + e], u, b[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < CH_T; i++) {
+            a[i] = row16_sum(a[i]);
+            b[i] = row16_sum(b[i]);
+            if (sl == i) {
+                s_A[i][j] = i > j ? a[i] : 0.0f;
+                s_B[i][j] = b[i];
+            }
+        }
+    }
+    __syncthreads();
+    // T by forward substitution, a lane per column
+    if (t < CH_T) {
+        float x[CH_T];
+#pragma unroll
+        for (int i = 0; i < CH_T; i++) {
+            float v = i == t ? 1.0f : 0.0f;
+#pragma unroll
+            for (int j = 0; j < i; j++) v = fmaf(-s_A[i][j], x[j], v);
+            x[i] = s_b[i] * v;
+            s_T[i][t] = x[i];
+        }
+    }
+    // sums of the logarithms, in place of the decays (whose readers are done)
+    if (r0 < RS)
+#pragma unroll
+        for (int i = 0; i < NR; i++) s_g[(r0 + RS * i) * DP + e0] = l[i];
+    __syncthreads();
+    for (int e = t; e < DP; e += 256) {
+        float g = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CH_T; i++) {
+            g += s_g[i * DP + e];
+            s_g[i * DP + e] = g;
+        }
+    }
+    __syncthreads();
+    float *out = rec + ((int64_t)ch * d.H + h) * delta_rec16_floats(NT);
+    for (int idx = t; idx < NT * 64; idx += 256) {
+        const int tile = idx >> 6, l = idx & 63, row = l & 15, q4 = 4 * (l >> 4);
+        float4 kt, qt, kh;
+        {
+            const int o = row * DP + 16 * tile + q4;
+            const float4 k = *(const float4 *)(s_k + o), q = *(const float4 *)(s_q + o), G = *(const float4 *)(s_g + o);
+            const float4 x = make_float4(expf(G.x), expf(G.y), expf(G.z), expf(G.w));
+            kt = make_float4(k.x * x.x, k.y * x.y, k.z * x.z, k.w * x.w);
+            qt = make_float4(q.x * x.x, q.y * x.y, q.z * x.z, q.w * x.w);
+        }
+        {  // row: the channel, columns: tokens
+            const int e = 16 * tile + row;
+            const float Gc = s_g[15 * DP + e];
+            kh = make_float4(s_k[q4 * DP + e] * expf(Gc - s_g[q4 * DP + e]), s_k[(q4 + 1) * DP + e] * expf(Gc - s_g[(q4 + 1) * DP + e]),
+                             s_k[(q4 + 2) * DP + e] * expf(Gc - s_g[(q4 + 2) * DP + e]),
+                             s_k[(q4 + 3) * DP + e] * expf(Gc - s_g[(q4 + 3) * DP + e]));
+        }
+        *(float4 *)(out + 4 * idx) = kt;
+        *(float4 *)(out + 256 * NT + 4 * idx) = qt;
+        *(float4 *)(out + 512 * NT + 4 * idx) = kh;
+    }
+    if (t < 128) {
+        const float(*m)[CH_T + 1] = wave ? s_B : s_T;
+        const int row = lane & 15, q4 = 4 * (lane >> 4);
+        *(float4 *)(out + 768 * NT + 256 * wave + 4 * lane) = make_float4(m[row][q4], m[row][q4 + 1], m[row][q4 + 2], m[row][q4 + 3]);
+    }
+    for (int e = t; e < DP; e += 256) out[768 * NT + 512 + e] = e < D ? expf(s_g[15 * DP + e]) : 0.0f;
+}
+
+// one chunk's operands of a wavefront with NW tiles of key channels
+template <int NW>
+struct DeltaOps16 {
+    d_f32x4 kt[NW], qt[NW], kh[NW], gc[NW], T;
+    float B, v[4];
+};
+
+// (records, rows of v and rows of o exist for whole chunks: what a sequence's last chunk has beyond it counts as zero)
+template <int NW>
+__global__ __launch_bounds__(256) void delta_walk16_kernel(DeltaShape d, const float *rec, const float *qkv, float *state, int M, int pos0,
+                                                         float *o, unsigned n_cb, unsigned n_items, unsigned per) {
+    __shared__ __align__(16) d_f32x4 s_w[2][4][64];
+    __shared__ float s_o[2][4][4][64];
+    constexpr int NT = 4 * NW;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, q4 = 4 * (lane >> 4);
+    // the workgroups of a head read the same records: they are dealt to one of the 8 XCDs (workgroups go to them in turn)
+    const unsigned item = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if (item >= n_items) return;
+    const int h = (int)(item / n_cb), c = (int)(item % n_cb) * 16 + col, D = d.D, V = d.V, C = d.channels(), HV = d.H * V;
+    const bool live = c < V;
+    float *S = state + (int64_t)h * D * V;
+    d_f32x4 s[NW];
+#pragma unroll
+    for (int i = 0; i < NW; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int e = 16 * (wave * NW + i) + q4 + r;
+            s[i][r] = (live && e < D && pos0 > 0) ? S[(int64_t)e * V + c] : 0.0f;
+        }
+    const int n_ch = (M + CH_T - 1) / CH_T;
+    // wavefront-uniform bases and this lane's fixed offsets from them
+    const float *rec_h = rec + (int64_t)h * delta_rec16_floats(NT) + 256 * (wave * NW);
+    const int64_t rec_step = (int64_t)d.H * delta_rec16_floats(NT);
+    const float *v_h = qkv + 2 * d.G * D + h * V;
+    float *o_h = o + (int64_t)wave * HV + h * V;
+    const unsigned l4 = 4u * lane, ov = (unsigned)(q4 * HV + c);
+    unsigned vv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) vv[r] = (unsigned)((q4 + r) * C + (live ? c : 0));
+    auto fetch = [&](DeltaOps16<NW> &x, int ch) {
+        const float *p = rec_h + ch * rec_step;
+#pragma unroll
+        for (int i = 0; i < NW; i++) {
+            x.kt[i] = *(const d_f32x4 *)(p + 256 * i + l4);
+            x.qt[i] = *(const d_f32x4 *)(p + 256 * (NT + i) + l4);
+            x.kh[i] = *(const d_f32x4 *)(p + 256 * (2 * NT + i) + l4);
+        }
+        p -= 256 * (wave * NW);
+#pragma unroll
+        for (int i = 0; i < NW; i++) x.gc[i] = *(const d_f32x4 *)(p + 768 * NT + 512 + 16 * (wave * NW + i) + q4);
+        x.T = *(const d_f32x4 *)(p + 768 * NT + l4);
+        x.B = (p + wave)[768 * NT + 256 + l4];
+        const float *v = v_h + (int64_t)ch * CH_T * C;
+#pragma unroll
+        for (int r = 0; r < 4; r++) x.v[r] = v[vv[r]];
+    };
+    // the output row 4 (lane / 16) + wave of a chunk, from the four wavefronts' parts
+    auto put = [&](int ch) {
+        const int b = ch & 1;
+        const float y = s_o[b][wave][0][lane] + s_o[b][wave][1][lane] + s_o[b][wave][2][lane] + s_o[b][wave][3][lane];
+        if (live) (o_h + (int64_t)ch * CH_T * HV)[ov] = y;
+    };
+    auto walk = [&](DeltaOps16<NW> &x, int ch) {
+        const int b = ch & 1;
+        d_f32x4 w = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NW; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) w = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kt[i][r], s[i][r], w, 0, 0, 0);
+        s_w[b][wave][lane] = w;
+#pragma unroll
+        for (int i = 0; i < NW; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qt[i][r], s[i][r], y, 0, 0, 0);
+        // LDS writes done, then the barrier (which also says that the parts of the previous chunk's output are all there);
+        // the operands under way from memory are not waited for
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        w = s_w[b][0][lane] + s_w[b][1][lane] + s_w[b][2][lane] + s_w[b][3][lane];
+        d_f32x4 u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; r++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.T[r], (ch * CH_T + q4 + r < M ? x.v[r] : 0.0f) - w[r], u, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NW; i++) {
+            s[i] *= x.gc[i];
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kh[i][r], u[r], s[i], 0, 0, 0);
+        }
+        // B U: this wavefront's quarter of the contracted tokens
+        const float uw = wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3];
+        y = __builtin_amdgcn_mfma_f32_16x16x4f32(x.B, uw, y, 0, 0, 0);
+        if (ch) put(ch - 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++) s_o[b][r][wave][lane] = y[r];
+    };
+    // the operands of three chunks are held or under way
+    DeltaOps16<NW> x0, x1, x2;
+    fetch(x0, 0);
+    fetch(x1, min(1, n_ch - 1));
+    fetch(x2, min(2, n_ch - 1));
+    for (int ch = 0; ch < n_ch; ch += 3) {  // (n_ch is the same for every wavefront: so is every barrier)
+        walk(x0, ch);
+        fetch(x0, min(ch + 3, n_ch - 1));
+        if (ch + 1 >= n_ch) break;
+        walk(x1, ch + 1);
+        fetch(x1, min(ch + 4, n_ch - 1));
+        if (ch + 2 >= n_ch) break;
+        walk(x2, ch + 2);
+        fetch(x2, min(ch + 5, n_ch - 1));
+    }
+    __syncthreads();
+    put(n_ch - 1);
+#pragma unroll
+    for (int i = 0; i < NW; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int e = 16 * (wave * NW + i) + q4 + r;
+            if (live && e < D) S[(int64_t)e * V + c] = s[i][r];
+        }
+}
+
+template <int NW>
+static hipError_t delta_walk16_launch(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0,
+                                      float *rec, float *o) {
+    const dim3 g1((unsigned)((M + CH_T - 1) / CH_T), (unsigned)d.H);
+    const unsigned n_cb = (unsigned)((d.V + 15) / 16), n_items = n_cb * (unsigned)d.H, per = (n_items + 7) / 8;
+    hipLaunchKernelGGL((delta_chunk16_kernel<NW>), g1, dim3(256), 0, s, d, qkv, beta, lg, M, rec);
+    hipLaunchKernelGGL((delta_walk16_kernel<NW>), dim3(8 * per), dim3(256), 0, s, d, rec, qkv, state, M, pos0, o, n_cb, n_items, per);
+    return hipGetLastError();
+}
+
+hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0, float *rec,
+                        float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec) {
+    if (d.D > 256 || d.V > 256 || M < 1) return hipErrorInvalidValue;
+    if (!delta_wide_chunks(d, M)) {
+        const auto launch = d.D > 192 ? delta_walk16_launch<4> : d.D > 128 ? delta_walk16_launch<3> : d.D > 64 ? delta_walk16_launch<2> : delta_walk16_launch<1>;
+        const hipError_t e = launch(s, d, qkv, beta, lg, state, M, pos0, rec, o);
+        return e != hipSuccess ? e : k_head_norm_rows(s, o, gate, normw, M, d.H, d.V, d.eps, outa, lda, prec);
+    }
+    const auto launch = d.D > 192 ? delta_walk_launch<4> : d.D > 128 ? delta_walk_launch<3> : d.D > 64 ? delta_walk_launch<2> : delta_walk_launch<1>;
+    return launch(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
 }
 
 // one wavefront per (token, head)

@@ -7,6 +7,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include "delta_plan.h"
 #include "layered.h"
 #include "model.h"
 
@@ -1226,7 +1227,7 @@ static hipError_t prompt_delta(l2h_model *m, LayerDev &L, const LayerRun &run, i
     a.hd = d.D;
     CK(k_gemm(s, a, prec, GE_DECAY));
     CK(product(m, gemm_of(L.g2, l->fg, M), GE_SIGMOID, l->gt, hv, 1.0f));
-    if (walk) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
+    if (walk) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->ob, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
     CK(k_delta_scan(s, d, l->qkv, l->kq, l->beta, l->lg, run.state, M, pos0, l->ob));
     return k_head_norm_rows(s, l->ob, l->gt, L.mixnorm, M, d.H, d.V, d.eps, l->ao, L.o.ld, prec);
 }

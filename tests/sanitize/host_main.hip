@@ -5,6 +5,7 @@
 // (hipcc with the sanitizers on the host side only).
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
+#include "../../llama2.jl_amd/csrc/delta_plan.h"
 #include "../../llama2.jl_amd/csrc/rows_plan.h"
 #include "../../llama2.jl_amd/csrc/tiles_plan.h"
 
@@ -205,6 +206,25 @@ static void check_rows_plan() {
                     }
 }
 
+// the delta rule's scratch holds the records of every prompt of up to its length, in chunks of 32 or 16
+static void check_delta_plan() {
+    for (int D : {1, 64, 65, 128, 192, 256})
+        for (int V : {1, 16, 100, 128, 129, 256})
+            for (int H : {1, 8, 16, 32, 33, 100, 768})
+                for (int cap : {256, 512, 768, 2048}) {
+                    if (H * V > 32768) continue;
+                    const DeltaShape d{H, 1, D, V, 4, 8, 8, 1e-5f};
+                    for (int M = L_DELTA_WALK_MIN; M <= cap; M++)
+                        EXPECT((delta_wide_chunks(d, M) ? (M + 31) / 32 * delta_chunk_floats(d) : delta_rec16_floats(d, M)) <= delta_walk_floats(d, cap));
+                }
+    // sizes at which the one or the other takes at least 1.05 times as long (measured)
+    auto wide = [](int H, int D, int V, int M) { return delta_wide_chunks(DeltaShape{H, 1, D, V, 4, 8, 8, 1e-5f}, M); };
+    EXPECT(wide(16, 64, 64, 2048) && wide(128, 64, 64, 2048) && wide(32, 128, 64, 2048) && wide(16, 128, 128, 2048) && wide(16, 256, 64, 2048) && wide(4, 256, 256, 2048) &&
+           wide(8, 256, 256, 2048) && wide(16, 128, 256, 2048));
+    EXPECT(!wide(128, 128, 128, 2048) && !wide(48, 192, 192, 2048) && !wide(16, 192, 192, 700) && !wide(64, 256, 256, 2048) && !wide(64, 128, 256, 2048) &&
+           !wide(96, 64, 256, 2048) && !wide(32, 64, 256, 300) && !wide(8, 256, 256, 64) && !wide(32, 256, 128, 300));
+}
+
 // every tile of a prompt's product is taken exactly once, as a whole or as both of its halves
 static void check_tiles_plan() {
     for (int n_cu : {32, 64, 250, 256}) {
@@ -250,6 +270,7 @@ int main() {
     check_product_rule();
     check_parts_rule();
     check_rows_plan();
+    check_delta_plan();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
     check_shape(4096, 14336, 32, 32, 8, 128256, 512, q4, 14, 0, true);    // the headline model
