@@ -51,8 +51,41 @@ inline int delta_most16(const DeltaShape &d, int M) {
     return delta_wide_chunks(d, L_DELTA_WALK_MIN) ? 0 : std::min(M, DELTA_WIDE_M - 1);
 }
 
-// scratch for prompts of up to M tokens
-inline int64_t delta_walk_floats(const DeltaShape &d, int M) {
-    const int64_t wide = delta_wide_chunks(d, M) ? (M + WK_T - 1) / WK_T * delta_chunk_floats(d) : 0;
-    return std::max(wide, delta_rec16_floats(d, delta_most16(d, M)));
+// Chunks of 32 a pass, passes of about the same length.  A record holds a state, so that those of a whole prompt are 1.9 times (heads of 128 x 128) what chunks of 16
+// and their outputs take: 138 MB for 2048 positions of 16 heads.  With 160 MiB that is one pass; 32 heads have two, which is as fast as one (3.37 and 3.41 ms through
+// three layers of width 4096: the records then stay in the memory-side cache).  Smaller passes cost: 16 heads 1.65 ms in one, 1.67 in two, 1.77 in three, 1.90 in five.
+#define DELTA_RECORDS ((int64_t)40 << 20)  // floats
+#define DELTA_LEAST_CHUNKS 8               // ... or as many chunks
+inline int delta_pass_chunks(const DeltaShape &d, int M, int64_t floats) {
+    const int n = (M + WK_T - 1) / WK_T;
+    const int64_t most = floats / delta_chunk_floats(d), passes = most < 1 ? 0 : (n + most - 1) / most;
+    return passes ? (int)((n + passes - 1) / passes) : 0;
 }
+// scratch for prompts of up to M tokens, and what there has to be of it
+struct DeltaScratch {
+    int64_t floats, least;
+};
+inline DeltaScratch delta_walk_scratch(const DeltaShape &d, int M) {
+    DeltaScratch s{0, 0};
+    const int64_t chunk = delta_chunk_floats(d);
+    if (delta_wide_chunks(d, M)) {
+        s.floats = std::min<int64_t>((M + WK_T - 1) / WK_T, std::max<int64_t>(DELTA_LEAST_CHUNKS, DELTA_RECORDS / chunk)) * chunk;
+        s.least = chunk;
+    }
+    const int most16 = delta_most16(d, M);
+    s.least = std::max(s.least, delta_rec16_floats(d, most16));
+    s.floats = std::max(s.floats, s.least);
+    return s;
+}
+// What there is of it then, `have` before: memory of s.floats or, where that is not to be had, of less, down to what there has to be (0: not even that).
+// get(n) says whether it got n floats.
+template <class F>
+inline int64_t delta_scratch_get(const DeltaScratch &s, int64_t have, F get) {
+    for (int64_t n = s.floats; n > have; n = std::max(s.least, n / 2)) {
+        if (get(n)) return n;
+        if (n <= s.least) break;
+    }
+    return have >= s.least ? have : 0;
+}
+// rows of outputs that the walk in chunks of 16 or the scan leaves for the head norm, for prompts of up to M tokens
+inline int delta_out_rows(const DeltaShape &d, int M) { return (std::max(delta_most16(d, M), std::min(M, L_DELTA_WALK_MIN - 1)) + 15) / 16 * 16; }

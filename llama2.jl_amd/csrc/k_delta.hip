@@ -1312,15 +1312,24 @@ static hipError_t delta_walk16_launch(hipStream_t s, const DeltaShape &d, const 
 }
 
 hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0, float *rec,
-                        float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec) {
+                        int64_t rec_floats, float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec) {
     if (d.D > 256 || d.V > 256 || M < 1) return hipErrorInvalidValue;
     if (!delta_wide_chunks(d, M)) {
+        if (rec_floats < delta_rec16_floats(d, M)) return hipErrorInvalidValue;
         const auto launch = d.D > 192 ? delta_walk16_launch<4> : d.D > 128 ? delta_walk16_launch<3> : d.D > 64 ? delta_walk16_launch<2> : delta_walk16_launch<1>;
         const hipError_t e = launch(s, d, qkv, beta, lg, state, M, pos0, rec, o);
         return e != hipSuccess ? e : k_head_norm_rows(s, o, gate, normw, M, d.H, d.V, d.eps, outa, lda, prec);
     }
+    // passes over as many chunks as have their records in memory together; a pass goes on from the state as the positions of a later call do
+    const int n = WK_T * delta_pass_chunks(d, M, rec_floats);
+    if (n < 1) return hipErrorInvalidValue;
     const auto launch = d.D > 192 ? delta_walk_launch<4> : d.D > 128 ? delta_walk_launch<3> : d.D > 64 ? delta_walk_launch<2> : delta_walk_launch<1>;
-    return launch(s, d, qkv, beta, lg, state, M, pos0, rec, gate, normw, outa, lda, prec);
+    for (int64_t m = 0; m < M; m += n) {
+        const hipError_t e = launch(s, d, qkv + m * d.channels(), beta + m * d.H, lg + m * d.H * d.D, state, std::min(n, M - (int)m), pos0 + (int)m, rec,
+                                    gate + m * d.H * d.V, normw, prec ? (void *)((float *)outa + m * lda) : (void *)((uint16_t *)outa + m * lda), lda, prec);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // one wavefront per (token, head)

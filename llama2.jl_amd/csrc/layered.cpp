@@ -59,6 +59,7 @@ struct Layered {
     int n_keys = 0;
     // prompt pass, for `cap` positions
     int cap = 0;
+    int64_t rec_floats = 0;
     int32_t *tok = nullptr, *choice = nullptr, *slot_row = nullptr, *slot_of = nullptr, *n_tiles = nullptr, *want = nullptr;
     GemmTile *tiles = nullptr;
     float *X = nullptr, *raw = nullptr, *qkv = nullptr, *kq = nullptr, *beta = nullptr, *lg = nullptr, *gt = nullptr, *ob = nullptr,
@@ -1062,10 +1063,11 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
     }
     if (l->cap >= cap) return L2H_OK;
     int64_t n_in = 1, ch = 1, g = 1, h = 1, hd = 1, hv = 1, lhv = 64, lra = 64, lrg = 64, hid = 64, ne = 1, slots = 1, up_slots = 1, tiles = 1;
-    int64_t kvt = 0, rec = 0, qb = 0, xc = 0, kvx = 0, cq = 0, lat_qa = 0, lat_part = 0;
+    int64_t kvt = 0, out_rows = 0, qb = 0, xc = 0, kvx = 0, cq = 0, lat_qa = 0, lat_part = 0;
     // tokens of a block of latent attention: few where longer prompts go another way
     const int lat_block = std::min(cap, L_LATENT_BLOCK), kvx_cap = std::min((c.seq_len + 255) / 256 * 256, 2048);
     bool moe = false;
+    DeltaScratch rec{0, 0};
     for (LayerDev &L : l->layer) {
         const l2h_layer &d = L.d;
         n_in = std::max<int64_t>(n_in, L.n_plain);
@@ -1098,7 +1100,10 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
             h = std::max<int64_t>(h, d.n_heads);
             hd = std::max<int64_t>(hd, d.n_heads * d.dim);
             lra = std::max<int64_t>(lra, L.a2.ld);
-            rec = std::max(rec, delta_walk_floats(delta_shape(l, L), cap));
+            const DeltaScratch r = delta_walk_scratch(delta_shape(l, L), cap);
+            rec.floats = std::max(rec.floats, r.floats);
+            rec.least = std::max(rec.least, r.least);
+            out_rows = std::max<int64_t>(out_rows, delta_out_rows(delta_shape(l, L), cap));
             lrg = std::max<int64_t>(lrg, L.g2.ld);
         }
         if (d.ff == L2H_FF_DENSE && !L.joined) hid = std::max<int64_t>(hid, L.down.ld);
@@ -1111,7 +1116,6 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
         }
     }
     if (kvt) DA(l->kvt, kvt);
-    if (rec) DA(l->rec, rec);
     if (cq) {
         DB(l->cq, cap * cq);
         DA(l->lat_qa, lat_qa);
@@ -1128,11 +1132,11 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
     DA(l->X, (int64_t)cap * c.width);
     DA(l->raw, cap * std::max<int64_t>(n_in, c.side_dim));
     DA(l->qkv, cap * ch);
-    DA(l->kq, cap * g);
+    DA(l->kq, std::min(cap, L_DELTA_WALK_MIN) * g);
     DA(l->beta, cap * h);
     DA(l->lg, cap * hd);
     DA(l->gt, cap * hv);
-    DA(l->ob, cap * hv);
+    DA(l->ob, out_rows * hv);
     DB(l->xn, (int64_t)cap * l->ldw());
     DB(l->fa, cap * lra);
     DB(l->fg, cap * lrg);
@@ -1152,6 +1156,16 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
     if (c.side_dim) {
         DB(l->sb, (int64_t)cap * pad64(c.side_dim));
         DA(l->Y, (int64_t)cap * c.width);
+    }
+    // (last: what is short of memory then is the delta rule's records, of which fewer do)
+    if (rec.floats) {
+        const int64_t n = delta_scratch_get(rec, l->rec_floats, [&](int64_t k) {
+            const bool got = dalloc(m, &l->rec, k, false) == L2H_OK;
+            if (!got) (void)hipGetLastError();
+            return got;
+        });
+        if (!n) return L2H_EHIP;  // (dalloc has said why)
+        l->rec_floats = n;
     }
 #undef DB
 #undef DA
@@ -1227,7 +1241,7 @@ static hipError_t prompt_delta(l2h_model *m, LayerDev &L, const LayerRun &run, i
     a.hd = d.D;
     CK(k_gemm(s, a, prec, GE_DECAY));
     CK(product(m, gemm_of(L.g2, l->fg, M), GE_SIGMOID, l->gt, hv, 1.0f));
-    if (walk) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->ob, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
+    if (walk) return k_delta_walk(s, d, l->qkv, l->beta, l->lg, run.state, M, pos0, l->rec, l->rec_floats, l->ob, l->gt, L.mixnorm, l->ao, L.o.ld, prec);
     CK(k_delta_scan(s, d, l->qkv, l->kq, l->beta, l->lg, run.state, M, pos0, l->ob));
     return k_head_norm_rows(s, l->ob, l->gt, L.mixnorm, M, d.H, d.V, d.eps, l->ao, L.o.ld, prec);
 }

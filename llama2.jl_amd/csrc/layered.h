@@ -216,9 +216,9 @@ hipError_t k_delta_prepare(hipStream_t s, const DeltaShape &d, const float *conv
 // the recurrence over M tokens, logarithms of the decays in lg[M][H D]; o[M][H V]; then the ring takes the last tokens
 hipError_t k_delta_scan(hipStream_t s, const DeltaShape &d, const float *qkv, const float *kq, const float *beta, const float *lg,
                         float *state, int M, int pos0, float *o);
-// the same in chunks on the matrix cores, with k_head_norm_rows behind it; scratch: rec as delta_plan.h says, o[M][H V], M rounded up to 16
+// the same in chunks on the matrix cores, with k_head_norm_rows behind it; scratch: rec and the rows of o as delta_plan.h says
 hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0, float *rec,
-                        float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec);
+                        int64_t rec_floats, float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec);
 #define L_DELTA_WALK_MIN 24  // tokens from which the chunked form is used
 hipError_t k_delta_ring(hipStream_t s, const DeltaShape &d, const float *raw, int64_t ldr, float *ring, int M, int pos0);
 // outa[m][h V + j] = o * rms over the head * normw[j] * gate

@@ -206,7 +206,8 @@ static void check_rows_plan() {
                     }
 }
 
-// the delta rule's scratch holds the records of every prompt of up to its length, in chunks of 32 or 16
+// the delta rule's scratch holds what every prompt of up to its length takes of it, and is not more than the outputs and records of chunks of 16 tokens
+// by what the rule says; with less memory, fewer chunks a pass
 static void check_delta_plan() {
     for (int D : {1, 64, 65, 128, 192, 256})
         for (int V : {1, 16, 100, 128, 129, 256})
@@ -214,9 +215,37 @@ static void check_delta_plan() {
                 for (int cap : {256, 512, 768, 2048}) {
                     if (H * V > 32768) continue;
                     const DeltaShape d{H, 1, D, V, 4, 8, 8, 1e-5f};
-                    for (int M = L_DELTA_WALK_MIN; M <= cap; M++)
-                        EXPECT((delta_wide_chunks(d, M) ? (M + 31) / 32 * delta_chunk_floats(d) : delta_rec16_floats(d, M)) <= delta_walk_floats(d, cap));
+                    const DeltaScratch s = delta_walk_scratch(d, cap);
+                    const int64_t chunk = delta_chunk_floats(d);
+                    EXPECT(s.least >= 1 && s.least <= s.floats && s.least <= std::max(chunk, delta_rec16_floats(d, cap)));
+                    EXPECT(s.floats <= std::max(delta_rec16_floats(d, cap), std::max((int64_t)40 << 20, 8 * chunk)));
+                    for (int64_t floats : {s.floats, s.least})
+                        for (int M = L_DELTA_WALK_MIN; M <= cap; M++) {
+                            if (!delta_wide_chunks(d, M)) {
+                                EXPECT(delta_rec16_floats(d, M) <= floats && (M + 15) / 16 * 16 <= delta_out_rows(d, cap));
+                                continue;
+                            }
+                            const int n = delta_pass_chunks(d, M, floats);
+                            EXPECT(n >= 1 && n * chunk <= floats);
+                        }
+                    EXPECT(delta_out_rows(d, cap) >= L_DELTA_WALK_MIN - 1 && delta_out_rows(d, cap) <= cap);
                 }
+    // the most there is, 128 heads of 256 x 256, takes what chunks of 16 do; 16 of 128 x 128 are one pass, 48 three
+    const DeltaShape many{128, 1, 256, 256, 4, 8, 8, 1e-5f}, few{16, 16, 128, 128, 4, 8, 8, 1e-5f}, more{48, 48, 128, 128, 4, 8, 8, 1e-5f};
+    EXPECT(delta_walk_scratch(many, 2048).floats == delta_rec16_floats(many, 2048) && !delta_wide_chunks(many, 2048));
+    EXPECT(delta_pass_chunks(few, 2048, delta_walk_scratch(few, 2048).floats) == 64 && delta_wide_chunks(few, 48));
+    EXPECT(delta_pass_chunks(more, 2048, delta_walk_scratch(more, 2048).floats) == 22 && delta_wide_chunks(more, 48));
+    for (int64_t room = 0; room <= 100; room++)
+        for (int64_t have : {0, 3, 10, 50, 64, 80}) {
+            int asked = 0;
+            const int64_t n = delta_scratch_get(DeltaScratch{64, 5}, have, [&](int64_t k) {
+                EXPECT(k > have && k >= 5 && k <= 64);
+                asked++;
+                return k <= room;
+            });
+            EXPECT(n == 0 ? have < 5 && room < 5 : n >= 5 && (n == have || (n <= room && 2 * n >= std::min<int64_t>(room, 64))));
+            EXPECT(have < 64 || !asked);
+        }
     // sizes at which the one or the other takes at least 1.05 times as long (measured)
     auto wide = [](int H, int D, int V, int M) { return delta_wide_chunks(DeltaShape{H, 1, D, V, 4, 8, 8, 1e-5f}, M); };
     EXPECT(wide(16, 64, 64, 2048) && wide(128, 64, 64, 2048) && wide(32, 128, 64, 2048) && wide(16, 128, 128, 2048) && wide(16, 256, 64, 2048) && wide(4, 256, 256, 2048) &&
