@@ -219,7 +219,9 @@ hipError_t k_delta_scan(hipStream_t s, const DeltaShape &d, const float *qkv, co
 // the same in chunks on the matrix cores, with k_head_norm_rows behind it; scratch: rec and the rows of o as delta_plan.h says
 hipError_t k_delta_walk(hipStream_t s, const DeltaShape &d, const float *qkv, const float *beta, const float *lg, float *state, int M, int pos0, float *rec,
                         int64_t rec_floats, float *o, const float *gate, const float *normw, void *outa, int64_t lda, int prec);
-#define L_DELTA_WALK_MIN 24  // tokens from which the chunked form is used
+// Tokens from which the chunked form is used.  Prompts of 24, 40, 48 and 64 through three layers, us, the scan and chunks: 16 heads of 128 x 128 464 and 488, 540 and 549, 553
+// and 549, 587 and 560; 16 of 64 x 64 345 and 362, 370 and 369, 379 and 373, 394 and 375; 8 of 256 x 256 433 and 465, 479 and 487, 493 and 494, 529 and 499.
+#define L_DELTA_WALK_MIN 48
 hipError_t k_delta_ring(hipStream_t s, const DeltaShape &d, const float *raw, int64_t ldr, float *ring, int M, int pos0);
 // outa[m][h V + j] = o * rms over the head * normw[j] * gate
 hipError_t k_head_norm_rows(hipStream_t s, const float *o, const float *gate, const float *normw, int M, int H, int V, float eps,

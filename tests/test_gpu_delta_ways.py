@@ -1,5 +1,5 @@
 """The delta rule's prompt pass in chunks of 16 (delta_plan.h), for many heads and for wide values, and in chunks of 32 with wide values from 512 tokens on: from an
-empty state and going on from one; and in several passes over the chunks."""
+empty state and going on from one; in several passes over the chunks; and up to 47 tokens one by one."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ TOL = {"float32": 2e-5, "bfloat16": 3e-2}  # as the other runs of layered models
 # (heads, key heads, dim, vdim, lengths one after the other); 768 heads have eight chunks a pass: 256 tokens
 @pytest.mark.parametrize("precision", sorted(TOL))
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,cuts", [(64, 2, 100, 100, (47, 48, 49, 80)), (4, 2, 48, 130, (63, 64, 511, 512, 600)), (100, 1, 65, 129, (48, 61)),
-                                                          (768, 1, 8, 8, (48, 256, 257, 545))])
+                                                          (768, 1, 8, 8, (48, 256, 257, 545)), (3, 3, 128, 128, (46, 47, 48, 49))])
 def test_chunks(pkg, heads, kv_heads, dim, vdim, cuts, precision):
     c = lc.config([lc.delta(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, conv=4, ranks=(8, 12))], width=72, vocab=60)
     t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 4).items()}
