@@ -124,26 +124,13 @@ static int dev_tensor_download(l2h_ctx *ctx, const DevTensor *t, void *host) {
 // ------------------------------------------------------------------------------------------
 // context
 // ------------------------------------------------------------------------------------------
-void *PinnedArena::take(size_t bytes) {
-    const size_t n = (bytes + UNIT - 1) / UNIT;
-    std::lock_guard<std::mutex> hold(lock);
-    for (size_t i = 0; mem && i + n <= UNITS; i++) {
-        size_t k = 0;
-        while (k < n && !used[i + k]) k++;
-        if (k < n) continue;
-        std::fill(used + i, used + i + n, true);
-        return mem + i * UNIT;
-    }
+static void *host_pin(size_t bytes) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return p;
+    (void)hipGetLastError();
     return nullptr;
 }
-bool PinnedArena::give(void *p, size_t bytes) {
-    std::lock_guard<std::mutex> hold(lock);
-    const char *c = (const char *)p;
-    if (!mem || c < mem || c >= mem + UNIT * UNITS) return false;
-    const size_t i = (size_t)(c - mem) / UNIT, n = (bytes + UNIT - 1) / UNIT;
-    std::fill(used + i, used + i + n, false);
-    return true;
-}
+static void host_unpin(void *p) { (void)hipHostFree(p); }
 
 extern "C" int l2h_ctx_create(int device, l2h_ctx **out) {
     if (!out) return set_err(nullptr, L2H_EINVAL, "l2h_ctx_create: out is NULL");
@@ -171,10 +158,7 @@ extern "C" int l2h_ctx_create(int device, l2h_ctx **out) {
         delete ctx;
         return L2H_ENODEV;
     }
-    if (hipHostMalloc((void **)&ctx->pinned.mem, PinnedArena::UNIT * PinnedArena::UNITS, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->pinned.mem = nullptr;
-    }
+    ctx->pinned.open(host_pin, host_unpin);
     *out = ctx;
     return L2H_OK;
 }
@@ -185,7 +169,7 @@ extern "C" void l2h_ctx_destroy(l2h_ctx *ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipStreamDestroy(ctx->stream);
     }
-    if (ctx->pinned.mem) (void)hipHostFree(ctx->pinned.mem);
+    ctx->pinned.close();
     delete ctx;
 }
 
@@ -303,13 +287,7 @@ static void model_free_state(l2h_model *m) {
     m->allocs.clear();
     for (void *p : m->uc_allocs) uncached_release(p);
     m->uc_allocs.clear();
-    if (m->box.mem && !m->ctx->pinned.give(m->box.mem, m->box.bytes)) {
-        if (m->box.pinned)
-            (void)hipHostFree(m->box.mem);
-        else
-            free(m->box.mem);
-    }
-    m->box = HostBox();
+    m->box.release(m->ctx->pinned);
     m->pf_cap = 0;
     m->pf_wbf = nullptr;
     m->pf_copy_tried = false;
@@ -1061,26 +1039,12 @@ static int loop_buffers(l2h_model *m) {
     if ((rc = dalloc(m, &(p), (n), (z)))) \
         return rc;
     // the control blocks (the second: a layered model's steps hand the first on through it) and the prompt behind them
-    static_assert(sizeof(DecodeCtl) % 16 == 0, "the prompt follows the control blocks");
     const int64_t n = m->c.seq_len;
     DA(m->ctl, 2 + (n * 4 + (int64_t)sizeof(DecodeCtl) - 1) / (int64_t)sizeof(DecodeCtl), true);
     m->prompt_dev = (int32_t *)(m->ctl + 2);
     m->max_out = m->c.seq_len;
     DA(m->out_tokens, m->max_out, true);
-    HostBox &b = m->box;
-    b.bytes = 2 * sizeof(DecodeCtl) + 2 * (size_t)n * 4 + 64;
-    b.mem = m->ctx->pinned.take(b.bytes);
-    if (!b.mem && !(b.pinned = hipHostMalloc(&b.mem, b.bytes, hipHostMallocDefault) == hipSuccess)) {
-        (void)hipGetLastError();  // (then copies wait, as they do from any memory of a program)
-        b.mem = malloc(b.bytes);
-        if (!b.mem) return set_err(m->ctx, L2H_EHIP, "out of host memory");
-    }
-    memset(b.mem, 0, b.bytes);
-    b.ctl = (DecodeCtl *)b.mem;
-    b.prompt = (int32_t *)(b.ctl + 2);
-    b.out = b.prompt + n;
-    b.pick = b.out + n;
-    b.gave_up = (unsigned *)b.pick + 1;
+    if (!m->box.make(m->ctx->pinned, n)) return set_err(m->ctx, L2H_EHIP, "out of host memory");
     DA(m->argmax_partial, std::max(L2H_ARGMAX_BLOCKS, m->ctx->prop.multiProcessorCount), true);
 #undef DA
     return L2H_OK;

@@ -3,22 +3,11 @@
 #pragma once
 
 #include <algorithm>
-#include <mutex>
 #include <string>
 #include <vector>
 
+#include "host_box.h"
 #include "l2h_internal.h"
-
-// Pinned host memory of a context for its models' boxes (HostBox), a few kilobytes each: made once, for pinning takes half a millisecond.  What does not
-// fit is pinned by itself.
-struct PinnedArena {
-    static constexpr size_t UNIT = 4096, UNITS = 64;
-    std::mutex lock;
-    char *mem = nullptr;  // UNIT x UNITS, or none
-    bool used[UNITS] = {};
-    void *take(size_t bytes);
-    bool give(void *p, size_t bytes);  // false: not from here
-};
 
 struct l2h_ctx {
     PinnedArena pinned;
@@ -42,19 +31,6 @@ int set_err(l2h_ctx *ctx, int code, const char *fmt, ...);
 static inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 struct Layered;  // what a layered model adds (layered.cpp)
-
-// What a call hands to the device and gets back, in host memory that stays: pinned, so that a copy is a request among others and the call waits once, at
-// its end (from a call's own stack every copy was a wait).  One call of a model at a time uses it.
-struct HostBox {
-    DecodeCtl *ctl = nullptr;   // [2], and the prompt behind them, as on the device
-    int32_t *prompt = nullptr;  // [seq_len]
-    int32_t *out = nullptr;     // [seq_len] tokens
-    int32_t *pick = nullptr;    // l2h_sample's
-    unsigned *gave_up = nullptr;
-    void *mem = nullptr;
-    size_t bytes = 0;
-    bool pinned = false;  // by itself (or from the context's arena, which knows)
-};
 
 struct l2h_model {
     l2h_ctx *ctx = nullptr;

@@ -6,6 +6,7 @@
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
 #include "../../llama2.jl_amd/csrc/delta_plan.h"
+#include "../../llama2.jl_amd/csrc/host_box.h"
 #include "../../llama2.jl_amd/csrc/rows_plan.h"
 #include "../../llama2.jl_amd/csrc/tiles_plan.h"
 
@@ -254,6 +255,65 @@ static void check_delta_plan() {
            !wide(96, 64, 256, 2048) && !wide(32, 64, 256, 300) && !wide(8, 256, 256, 64) && !wide(32, 256, 128, 300));
 }
 
+// a context's pinned block and its models' boxes, with memory of the program's in place of pinned one: nothing is handed out twice, what does not fit
+// is pinned by itself, what cannot be pinned is ordinary memory, and everything is given back (the sanitizer looks for leaks)
+static int pins = 0;
+static bool may_pin = true;
+static void *test_pin(size_t bytes) {
+    if (!may_pin) return nullptr;
+    pins++;
+    return malloc(bytes);
+}
+static void test_unpin(void *p) {
+    pins--;
+    free(p);
+}
+static void fill(HostBox &b, int64_t n, int with) {
+    b.ctl[0].pos = b.ctl[1].pos = *b.pick = with;
+    *b.gave_up = (unsigned)with;
+    for (int64_t i = 0; i < n; i++) b.prompt[i] = b.out[i] = with;
+}
+static bool holds(const HostBox &b, int64_t n, int with) {
+    bool ok = b.ctl[0].pos == with && b.ctl[1].pos == with && *b.pick == with && *b.gave_up == (unsigned)with;
+    for (int64_t i = 0; i < n; i++) ok = ok && b.prompt[i] == with && b.out[i] == with;
+    return ok;
+}
+static void check_boxes() {
+    for (bool block : {true, false}) {
+        may_pin = block;
+        PinnedArena arena;
+        arena.open(test_pin, test_unpin);
+        EXPECT((arena.mem != nullptr) == block && pins == (int)block);
+        const int64_t n[7] = {1, 500, 512, 4096, 20000, 1000, 40000};  // (the last takes more than the block)
+        for (int round = 0; round < 3; round++) {
+            may_pin = round != 1;
+            std::vector<HostBox> boxes(35);
+            for (size_t i = 0; i < boxes.size(); i++) {
+                EXPECT(boxes[i].make(arena, n[i % 7]));
+                fill(boxes[i], n[i % 7], (int)i + 1);
+                // asked again, a model keeps what it has
+                const void *mem = boxes[i].mem;
+                std::vector<bool> used(arena.used, arena.used + PinnedArena::UNITS);
+                EXPECT(boxes[i].make(arena, n[i % 7]) && boxes[i].mem == mem && std::equal(used.begin(), used.end(), arena.used) && holds(boxes[i], n[i % 7], (int)i + 1));
+                if (i % 7 == 6) EXPECT(boxes[i].pinned == may_pin);
+            }
+            for (size_t i = 0; i < boxes.size(); i++) EXPECT(holds(boxes[i], n[i % 7], (int)i + 1));
+            // places in the middle that come free are used again
+            if (block) {
+                const void *at = boxes[1].mem;
+                EXPECT((const char *)at >= arena.mem && (const char *)at < arena.mem + PinnedArena::UNIT * PinnedArena::UNITS);
+                boxes[1].release(arena);
+                EXPECT(!boxes[1].mem && boxes[1].make(arena, 500) && boxes[1].mem == at);
+            }
+            for (HostBox &b : boxes) b.release(arena);
+            for (bool u : arena.used) EXPECT(!u);
+            EXPECT(pins == (int)block);
+        }
+        arena.close();
+        EXPECT(pins == 0);
+    }
+}
+
 // every tile of a prompt's product is taken exactly once, as a whole or as both of its halves
 static void check_tiles_plan() {
     for (int n_cu : {32, 64, 250, 256}) {
@@ -300,6 +360,7 @@ int main() {
     check_parts_rule();
     check_rows_plan();
     check_delta_plan();
+    check_boxes();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
     check_shape(4096, 14336, 32, 32, 8, 128256, 512, q4, 14, 0, true);    // the headline model
