@@ -164,10 +164,14 @@ static hipError_t few_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
         hipLaunchKernelGGL((few_kernel<PREC, EPI, RN, JM>), dim3(8 * ((n_nt * n_mt + 7) / 8)), dim3(64 * FEW_WAVES), 0, s, a, n_nt, n_mt); \
         return hipGetLastError();                                                                                                         \
     } while (0)
-    // 32 rows and 64 positions at a time where that gives every CU a workgroup: half the reads of the positions
+    // 32 rows and 64 positions at a time where that gives every CU a workgroup: half the reads of the positions (fp32 products of that size go to k_gemm's tiles)
     if (a.M <= 16) GO(1, 1);
-    if (a.M <= 32 || ((cols + 31) / 32) * ((a.M + 63) / 64) < 256) GO(1, 2);
-    GO(2, 4);
+    if constexpr (PREC) {
+        GO(1, 2);
+    } else {
+        if (a.M <= 32 || ((cols + 31) / 32) * ((a.M + 63) / 64) < 256) GO(1, 2);
+        GO(2, 4);
+    }
 #undef GO
 }
 

@@ -124,40 +124,27 @@ struct GemmArgs {
 #define L_IMAGE_TILE 256  // ... and for k_tiles
 hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // The same for few rows or positions (k_few.hip), which k_gemm hands on to where that is the faster way; cols: columns the epilogue
-// covers.  Gains: the time of k_gemm's own tiles over that of k_few, distinct matrices one after the other.
+// covers.  Distinct matrices one after the other:
 //
-// Grouped: up to 48 positions a matrix.  Gains at 12, 32, 48 and 56, 8 to 96 matrices of 512 to 4096 inputs: 2.7 to 12, 1.5 to 9, 1.0 to 8
-// and 0.8 to 5 in fp32; in bf16 2.4 to 8, 1.7 to 8, 1.2 to 7 and 1.0 to 5.  Beyond, in fp32 (bf16 products have images there), while blocks
-// of 128 x 128 would be few for the CUs: up to 224 positions a matrix and, in all, (positions) x (blocks of 128 columns) up to 28 672.
-// Sixty products of 8 to 32 matrices with 256 to 4096 rows, 56 to 240 positions each: 1.2 to 5 at up to half of that, 0.8 to 1.3 there, 0.6 to
-// 0.9 at twice as much (16 matrices of 4096 x 2048, 192 positions each: 0.59).  Within it the blocks are the faster way only near
-// 104 to 136 positions, which just fill one (0.8 to 1.6).
+// bf16, the time of k_gemm's own tiles over that of k_few.  Grouped, up to 48 positions a matrix (beyond, there are images): at 12, 32, 48 and 56, 8 to 96
+// matrices of 512 to 4096 inputs, 2.4 to 8, 1.7 to 8, 1.2 to 7 and 1.0 to 5.  Plain, up to 128 positions (1.5 to 13, 256 to 32 000 rows), otherwise where tiles of
+// 64 x 64 are at most 256 (8192 rows, 128 positions: 1.6 to 2.0).
 //
-// Plain: up to 128 positions in bf16 (1.5 to 13, 256 to 32 000 rows), 32 in fp32 (1.0 to 10).  Otherwise where tiles of 64 x 64 are few:
-// at most 256 in bf16 (8192 rows, 128 positions: 1.6 to 2.0), 384 in fp32 (8192 rows, 128 positions, 256 tiles: 1.06 to 1.22; 160 positions,
-// 384 tiles: 1.15 to 1.3; 448 and 500 tiles: 0.92 to 0.99).
+// fp32, k_few's time over that of the tiles, at 256 to 4096 inputs.  Plain, up to 8 positions (0.3 to 0.97) and up to 2^17 results, 2^18 of up to 16 positions: of 17
+// positions and more 0.5 to 0.95 up to 2^16.5 results, 0.65 to 1.01 at 2^17, 0.95 to 1.34 at 2^17.5, 0.96 to 1.77 at 2^18, 1.2 to 2.1 at 2^20; of 9 to 12 positions 0.82 to
+// 1.08 beyond 2^18, where the tiles, whose sums are nearer to 64 bits, take them all the same; of 16 0.99 to 1.15 at 2^18.  Grouped, up to 64 positions a matrix and 2^18
+// results: 8, 16, 32 and 64 positions each 0.4 to 0.99 up to 2^17, 0.75 to 1.27 at 2^18, 0.93 to 1.66 at 2^19; of 2 and 4 each 0.9 to 1.2; of 100 each 1.13 to 1.6, of 128
+// 1.2 to 1.9, of 512 1.2 to 1.9 up to 2^17.
 #define L_FEW_M 128
-#define L_FEW_M_F32 32
+#define L_FEW_M_F32 8
 #define L_FEW_EACH 48
-#define L_FEW_EACH_F32 224
-#define L_FEW_BLOCKS_F32 28672
+#define L_FEW_EACH_F32 64
 #define L_FEW_TILES 256
-#define L_FEW_TILES_F32 384
+#define L_FEW_RESULTS_F32 131072
 inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
-    if (a.tiles)
-        return a.rows_each <= L_FEW_EACH || (prec && a.rows_each <= L_FEW_EACH_F32 && a.M * ((cols + 127) / 128) <= L_FEW_BLOCKS_F32);
-    return a.M <= (prec ? L_FEW_M_F32 : L_FEW_M) || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (prec ? L_FEW_TILES_F32 : L_FEW_TILES);
-}
-// The fp32 products that go to k_gemm's tiles on the bf16 matrix cores all the same (the gains above are over tiles of the fp32 instructions): not up to 8
-// positions, nor up to 2^17 results in all, 2^18 of up to 16 positions or of several matrices.  k_few's time and theirs at
-// 256 to 4096 inputs, us: 2^17 results (2048 rows, 64 positions; 256 x 509) 4.1 to 20 and 4.7 to 23, 2^18 (4096 x 64; 2048 x 128; 512 x 509)
-// 5.2 to 39 and 4.9 to 30.  16 000 rows, 9 and 16 positions: 11 to 39 and 13 to 41; 13 to 48 and 13 to 41.  128 256 rows of 2048 inputs, 1 position:
-// 118 and 139; 9: 135 and 142.  8 and 16 matrices of 512 rows, 2^17 results in all: 5.6 to 15 and 8.3 to 20; 2^18: 7.6 to 22 and 8.4 to 21; 2048 rows,
-// 32 positions each, 2^19 to 2^20: 13 to 76 and 9.6 to 40.
-#define L_PARTS_M 8
-#define L_PARTS_RESULTS 131072
-inline bool k_parts_pays(const GemmArgs &a, int64_t cols) {
-    return a.M > L_PARTS_M && a.M * cols > (a.tiles || a.M <= 16 ? 2 : 1) * L_PARTS_RESULTS;
+    if (prec) return a.M <= L_FEW_M_F32 || (a.M * cols <= (a.tiles || a.M <= 16 ? 2 : 1) * L_FEW_RESULTS_F32 && (!a.tiles || a.rows_each <= L_FEW_EACH_F32));
+    if (a.tiles) return a.rows_each <= L_FEW_EACH;
+    return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= L_FEW_TILES;
 }
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
 

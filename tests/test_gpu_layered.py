@@ -217,23 +217,24 @@ def test_short_prompts(pkg, precision):
 
 
 def test_fp32_products_on_both_sides_of_their_rule(pkg):
-    """Experts with more than 48 positions each: at 2048 positions (all slots x 4 blocks of columns) is beyond the border between the kernel
-    for few positions and blocks of 128 x 128, at 1700 short of it.  A classifier of 385 tiles of 64 rows: 30 positions and 40."""
-    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16, mlp=lc.moe(40, 4, 390))], width=450, vocab=60)
-    t = lc.settle_routers(c, ref.random_tensors(c, 51), 5)
-    tok = lc.tokens(2048, c["vocab"], 6)
-    want = ref.Sequence(c, t).run(tok)
-    dev = lc.language_model(pkg, c, t, seq_len=2100).device()
-    for n in (1700, 2048):
-        at = np.arange(n - 1, 0, -37)[::-1]
-        assert lc.error(dev.prefill_logits(tok[:n], at), want[at]) <= TOL["float32"], n
-    dev.close()
+    """The kernel for few rows or positions, and the tiles.  40 experts, four a position: 168 positions are 672 x 390 results, just below 2^18; 169 are beyond.  Three
+    experts, one a position: 64 positions each, and 65.  A classifier of 24 601 rows: 8 positions, 10 (below 2^18 results), 11 and 40."""
+    for layer, width, cuts in ((lc.moe(40, 4, 390), 450, (168, 169, 1700, 2048)), (lc.moe(3, 1, 24), 72, (192, 195))):
+        c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16, mlp=layer)], width=width, vocab=60)
+        t = lc.settle_routers(c, ref.random_tensors(c, 51), 5)
+        tok = lc.tokens(max(cuts), c["vocab"], 6)
+        want = ref.Sequence(c, t).run(tok)
+        dev = lc.language_model(pkg, c, t, seq_len=2100).device()
+        for n in cuts:
+            at = np.arange(n - 1, 0, -37)[::-1]
+            assert lc.error(dev.prefill_logits(tok[:n], at), want[at]) <= TOL["float32"], n
+        dev.close()
     c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16)], width=70, vocab=24601)
     t = ref.random_tensors(c, 52)
     tok = lc.tokens(50, c["vocab"], 6)
     want = ref.Sequence(c, t).run(tok)
     dev = lc.language_model(pkg, c, t).device()
-    for n in (30, 40):
+    for n in (8, 10, 11, 30, 40):
         at = np.arange(50 - n, 50)
         assert lc.error(dev.prefill_logits(tok, at), want[at]) <= TOL["float32"], n
     dev.close()
