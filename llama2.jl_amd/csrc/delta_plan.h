@@ -1,9 +1,13 @@
-// How k_delta.hip takes a prompt's chunks: the record of a chunk, and the chunks whose records lie in memory together.
+// How k_delta.hip lays out the ring of convolution inputs and takes a prompt's chunks: the record of a chunk, and the chunks whose records lie in memory together.
 #pragma once
 
 #include <algorithm>
 
 #include "layered.h"
+
+// The ring of convolution inputs has `taps` slots; a token's step writes slot now = pos % taps while other workgroups read those of the j-th token
+// before it (1 <= j; -1: there is none).
+__host__ __device__ inline int delta_ring_slot(int taps, int now, int j) { return j >= taps ? -1 : now - j < 0 ? now - j + taps : now - j; }
 
 #define WK_T 32  // tokens of a chunk
 

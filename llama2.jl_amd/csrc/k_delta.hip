@@ -11,8 +11,8 @@
 // ---------------------------------------------------------------------------------------------------------------
 #define CONV_AHEAD 4  // taps whose inputs are fetched together
 
-// What a channel's convolution reads: its projection, the taps' weights and the ring's slots.  No load is skipped (a slot or weight that is not
-// used is read all the same, and replaced by zero in the sum).
+// What a channel's convolution reads: its projection, the taps' weights and the ring's slots.  No load is skipped: a weight that is not used is read all the same,
+// in place of a slot that there is none for the projection again (not a slot: the token's own is being written), and both are left out of the sum.
 struct DeltaConv {
     float cur, w[CONV_AHEAD], x[CONV_AHEAD];  // (x[0] is not read: it is cur)
 };
@@ -21,9 +21,13 @@ __device__ __forceinline__ void delta_conv_weights(DeltaConv &v, const float *co
 #pragma unroll
     for (int j = 0; j < CONV_AHEAD; j++) v.w[j] = conv[(int64_t)max(taps - 1 - j, 0) * C + ch];
 }
-__device__ __forceinline__ void delta_conv_ring(DeltaConv &v, const float *ring, int C, int taps, int ch, int now) {
+__device__ __forceinline__ void delta_conv_ring(DeltaConv &v, const float *ring, const float *in, int C, int taps, int ch, int now) {
 #pragma unroll
-    for (int j = 1; j < CONV_AHEAD; j++) v.x[j] = ring[(int64_t)(j < taps ? (now - j < 0 ? now - j + taps : now - j) : 0) * C + ch];
+    for (int j = 1; j < CONV_AHEAD; j++) {
+        const int slot = delta_ring_slot(taps, now, j);
+        const float *row = slot < 0 ? in : ring + (int64_t)slot * C;
+        v.x[j] = row[ch];
+    }
 }
 // the channel's convolution at `pos`: cur is its projection, ring slot `now` = pos % taps will hold it
 __device__ __forceinline__ float delta_conv(const DeltaConv &c, const float *conv, const float *ring, int C, int taps, int ch, int pos) {
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(DeltaShape d, DeltaWeig
     const int now = pos % d.taps;
 #pragma unroll
     for (int ii = 0; ii < NC; ii++)
-        if (256 * ii + 64 * wave < n_ch) delta_conv_ring(cv[ii], ring, C, d.taps, ch[ii], now);
+        if (256 * ii + 64 * wave < n_ch) delta_conv_ring(cv[ii], ring, in, C, d.taps, ch[ii], now);
     // the first 128 inputs of the factors' rows
     const int l8 = t & 7, r8 = t >> 3;
     uint4 fa[NR / 4][2], fg[2];

@@ -242,6 +242,17 @@ static void check_delta_plan() {
            !wide(96, 64, 256, 2048) && !wide(32, 64, 256, 300) && !wide(8, 256, 256, 64) && !wide(32, 256, 128, 300));
 }
 
+// no step of the delta rule reads the slot of the ring that it writes
+static void check_delta_ring() {
+    for (int taps = 1; taps <= 64; taps++)
+        for (int pos = 0; pos < 200; pos++)
+            for (int j = 1; j < 70; j++) {
+                const int slot = delta_ring_slot(taps, pos % taps, j);
+                EXPECT(slot != pos % taps && slot < taps && (slot < 0 ? slot == -1 && j >= taps : j < taps));
+                if (slot >= 0 && j <= pos) EXPECT(slot == (pos - j) % taps);
+            }
+}
+
 // a context's pinned block and its models' boxes, with memory of the program's in place of pinned one: nothing is handed out twice, what does not fit
 // is pinned by itself, what cannot be pinned is ordinary memory, and everything is given back (the sanitizer looks for leaks)
 static int pins = 0;
@@ -346,6 +357,7 @@ int main() {
     check_product_rule();
     check_rows_plan();
     check_delta_plan();
+    check_delta_ring();
     check_boxes();
     const int q4[7] = {12, 12, 12, 12, 12, 12, 12}, q5m[7] = {13, 13, 13, 13, 13, 14, 13}, mix[7] = {12, 12, 13, 12, 12, 14, 12},
               f32[7] = {0, 0, 0, 0, 0, 0, 0}, bad[7] = {12, 12, 12, 12, 12, 12, 13};
