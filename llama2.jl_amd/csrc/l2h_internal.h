@@ -231,7 +231,7 @@ inline int flow_form(const FlowArgs &a) {
 // Each returns hipGetLastError() of its launch.
 hipError_t k_repack(hipStream_t s, const DevTensor &t, const void *raw_dev, bool inverse, void *raw_out);
 hipError_t k_embed(hipStream_t s, const DevTensor &emb, const DecodeCtl *ctl, const int32_t *prompt, float *x,
-                   float *rope_cs, int head_size, float theta_scale, float scale = 1.0f, float *x_copy = nullptr);
+                   float *rope_cs, int head_size, float theta_scale);
 hipError_t k_dequant(hipStream_t s, const DevTensor &t, int64_t row0, int64_t nrows, float *y);
 hipError_t k_swiglu(hipStream_t s, float *hb, const float *hb2, int n);
 hipError_t k_matvec(hipStream_t s, PhaseArgs a, int pro, int epi);
