@@ -247,16 +247,20 @@ hipError_t k_window_prepare(hipStream_t s, const WindowShape &w, const float *fr
 // operand for four tiles is one word of 16 bytes of a key's values, and its results are 16 neighbouring columns of one query.
 // What bounds it is the matrix cores' 2 x 32 cycles for every four elements of a head, on the CU whose queries see the most keys, and the loads
 // ahead of them: a tile's values are requested before its scores are formed and the next tile's keys behind them.  8 heads of 128, 509 queries, all before
-// them in the window: 26 us; with a key a lane and the products on the vector units 94.
+// them in the window: 26 us; with a key a lane and the products on the vector units 94.  Where windows are short it is the queries' loads and the
+// outputs' stores, 16 bytes each a lane where sizes allow it, and wavefronts without keys, of which there are none (k_window_rows): 32 heads of 128, 2048 queries, a window of 8
+// 124 us with eight wavefronts a block, 34 with one; words of 4 bytes 155.
 // N: groups of 64 elements of a head (key and value elements up to 64 N); NW: wavefronts
 typedef float wr_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 wr_bf16x4 __attribute__((ext_vector_type(4)));
 #define WR_Q 16
 template <int PREC, int N, int NW>
 __global__ __launch_bounds__(64 * NW) void window_rows_kernel(WindowShape w, const float *qf, const float *raw, int64_t ldr, const float *kc,
                                                               const float *vc, int M, int pos0, void *outa, int64_t lda) {
     constexpr int DT = 4 * N;
-    __shared__ __align__(16) wr_f32x4 s_o[NW / 2][4 * N][64];
-    __shared__ float s_m[NW / 2][64], s_l[NW / 2][64];
+    constexpr int NJ = NW > 1 ? NW / 2 : 1;
+    __shared__ __align__(16) wr_f32x4 s_o[NJ][4 * N][64];
+    __shared__ float s_m[NJ][64], s_l[NJ][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
     // (the blocks that see the most keys first)
     const int h = blockIdx.y, q0 = (int)(gridDim.x - 1 - blockIdx.x) * WR_Q, D = w.D, V = w.V, D4 = w.Dp() / 4, g = h / (w.H / w.G);
@@ -287,14 +291,14 @@ __global__ __launch_bounds__(64 * NW) void window_rows_kernel(WindowShape w, con
     if (k0 <= last) fetch_keys(k0);
     {
         const float *p = qf + ((int64_t)min(q0 + col, M - 1) * w.H + h) * D;
+        const bool d4 = D % 4 == 0;
 #pragma unroll
-        for (int i = 0; i < DT; i++)
+        for (int i = 0; i < DT; i++) {
+            const int e = 16 * i + 4 * quad;
+            q[i] = d4 ? *(const wr_f32x4 *)(p + min(e, D - 4)) : wr_f32x4{p[min(e, D - 1)], p[min(e + 1, D - 1)], p[min(e + 2, D - 1)], p[min(e + 3, D - 1)]};
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int e = 16 * i + 4 * quad + r;
-                const float x = p[min(e, D - 1)];
-                q[i][r] = e < D ? x : 0.0f;
-            }
+            for (int r = 0; r < 4; r++) q[i][r] = e + r < D ? q[i][r] : 0.0f;
+        }
     }
     float mrun = -INFINITY, lrun = 0.0f;  // of query `col`: the same in the four lanes that have it
 #pragma unroll
@@ -377,40 +381,66 @@ __global__ __launch_bounds__(64 * NW) void window_rows_kernel(WindowShape w, con
     if (wave > 0 || m >= M) return;
     float f = 1.0f / lrun;
     if (w.gated) f *= l_sigmoid(raw[(int64_t)m * ldr + w.off_g() + h]);
+    const int64_t at = m * lda + h * V;
 #pragma unroll
     for (int n = 0; n < N; n++)
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
+            const int c = 64 * n + 16 * quad + 4 * r;
+            const wr_f32x4 o = {acc[n][0][r] * f, acc[n][1][r] * f, acc[n][2][r] * f, acc[n][3][r] * f};
+            if (v4) {
+                if (c >= V) continue;
+                if (PREC)
+                    *(wr_f32x4 *)((float *)outa + at + c) = o;
+                else
+                    *(wr_bf16x4 *)((__bf16 *)outa + at + c) = wr_bf16x4{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
+            } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int c = 64 * n + 16 * quad + 4 * r + j;
-                if (c < V) l_store_act<PREC>(outa, m * lda + h * V + c, acc[n][j][r] * f);
+                for (int j = 0; j < 4; j++)
+                    if (c + j < V) l_store_act<PREC>(outa, at + c + j, o[j]);
             }
+        }
     if (h == w.H - 1)
         for (int64_t j = (int64_t)w.H * V + quad; j < lda; j += 4) l_store_act<PREC>(outa, m * lda + j, 0.0f);
+}
+template <int PREC, int N, int NW>
+static hipError_t window_rows_go(hipStream_t s, dim3 grid, const WindowShape &w, const float *qf, const float *raw, int64_t ldr, const float *kc, const float *vc, int M,
+                                 int pos0, void *outa, int64_t lda) {
+    hipLaunchKernelGGL((window_rows_kernel<PREC, N, NW>), grid, dim3(64 * NW), 0, s, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda);
+    return hipGetLastError();
 }
 hipError_t k_window_rows(hipStream_t s, const WindowShape &w, const float *qf, const float *raw, int64_t ldr, const float *kc,
                          const float *vc, int M, int pos0, void *outa, int64_t lda, int prec) {
     if (w.V > 256 || w.D > 256 || pos0 < 0 || M < 1 || pos0 + M > w.seq_len) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((M + WR_Q - 1) / WR_Q), (unsigned)w.H);
+    // Wavefronts a block: as many as have a tile of keys each while the chip has room for them (eight a CU; four of heads above 128 elements, which take a
+    // SIMD's registers alone) or while each has six tiles; two rather than one where there is room.  Heads of 128, 2048 queries, us with one, two, four and eight
+    // wavefronts: 8 heads, a window of 33 14, 15, 20, 32; of 300 51, 42, 48, 55; of 4096 274, 211, 180, 166; 2 heads, of 300 46, 26, 17, 15; 32 heads, of 33 40, 49, 63, 124.
+    // 600 heads, lengths and windows: within 1.27 of the best of the four, and none slower than keys a lane on the vector units.
     const int n = (std::max(w.Dp(), w.V) + 63) / 64;
-#define GO(P, N, NW) hipLaunchKernelGGL((window_rows_kernel<P, N, NW>), grid, dim3(64 * NW), 0, s, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda)
+    const int64_t blocks = (int64_t)grid.x * grid.y, tiles = (std::min<int64_t>((int64_t)w.window + WR_Q - 1, pos0 + M) + 15) / 16, room = n > 2 ? 1024 : 2048;
+    int nw = 2 * blocks <= room ? 2 : 1;
+    for (int c : {2, 4, 8})
+        if (tiles >= c && (blocks * c <= room || tiles >= 6 * c) && (c < 8 || n <= 2)) nw = c;
+#define GO1(N, NW)                                                                                                                      \
+    return prec ? window_rows_go<1, N, NW>(s, grid, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda)                                          \
+                : window_rows_go<0, N, NW>(s, grid, w, qf, raw, ldr, kc, vc, M, pos0, outa, lda)
+#define GO(N)            \
+    if (nw == 1)         \
+        GO1(N, 1);       \
+    else if (nw == 2)    \
+        GO1(N, 2);       \
+    else if (nw == 4)    \
+        GO1(N, 4)
     if (n == 1) {
-        if (prec)
-            GO(1, 1, 8);
-        else
-            GO(0, 1, 8);
+        GO(1);
+        GO1(1, 8);
     } else if (n == 2) {
-        if (prec)
-            GO(1, 2, 8);
-        else
-            GO(0, 2, 8);
-    } else {
-        if (prec)
-            GO(1, 4, 4);
-        else
-            GO(0, 4, 4);
+        GO(2);
+        GO1(2, 8);
     }
+    GO(4);
+#undef GO1
 #undef GO
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
