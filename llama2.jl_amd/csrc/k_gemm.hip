@@ -143,7 +143,10 @@ __device__ __forceinline__ GemmParts gemm_split(float4 a, float4 b) {
 // 4096 x 1024: 41, 20.5; 1024 x 4096: 42, 25; 1608 x 1024: 25, 12.6; 2048 positions, 4096 x 1024: 139, 71; 16 matrices of 2048 x 2048, 64 and 192
 // positions each: 132, 43 and 380, 134.  (Activations stored in parts: 6 bytes an element where 4 do, 19 and 39 us for the first two, but products of
 // few positions were 1.2 to 1.3 times slower.  Two steps of loads under way: the same.)
-template <int EPI, bool GROUPED, int KS, int TM>
+// SHORT (for one or two steps; KS 1, TM 64): a wavefront has a quarter of the results instead, over all inputs.  Operands are read from LDS and split twice, but nothing is
+// exchanged, which took longer than the products; the sums are the same.  us, tiles of 128 x 128 on the fp32 instructions, otherwise and SHORT: 64 inputs, 16 384 rows with an
+// activation, 2048 positions 76, 101, 68; 8192, 300: 10.5, 13.0, 8.6; 128 inputs, 8192 rows, 2048 positions 62, 57, 40; 1024, 300 (3 x 10^5 results) 5.8, 6.7, 6.9.
+template <int EPI, bool GROUPED, int KS, int TM, bool SHORT = false>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, unsigned n_nt) {
     constexpr int T = 64, KSTEP = 64, BUFFER = (2 * T + 4 * TM) * KSTEP, FOLD = 8, JM = TM / 32, XL = TM / 16;
     extern __shared__ __align__(16) unsigned char s_raw[];  // [KS][2][BUFFER], then the wavefronts' sums
@@ -195,14 +198,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
         for (int i = 0; i < XL; i++) f.x[i] = *(const l_u32x4 *)(xrow[i] + k0);
         __builtin_amdgcn_sched_barrier(0);  // (requests stay in the order of the steps: a step's wait leaves the next one's under way)
     };
-    l_f32x16 acc[2][JM], total[2][JM];
-    auto clear = [&](l_f32x16(&v)[2][JM]) {
-#pragma unroll
-        for (int o = 0; o < 2 * JM; o++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) v[o / JM][o % JM][r] = 0.0f;
-    };
-    auto run = [&](Step &f, int step, int buffer) {
+    auto to_lds = [&](const Step &f, int buffer) {
         l_u32x4 *s_w = (l_u32x4 *)(s_raw + (2 * part + buffer) * BUFFER), *s_x = s_w + T * 8;
 #pragma unroll
         for (int i = 0; i < 2; i++) {
@@ -215,72 +211,113 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
             s_x[r * 16 + ((t & 15) ^ (r & 15))] = f.x[i];
         }
         l_lds_barrier();
-        gload(f, step + 1);
-        if (KS > 1 && first + step >= steps) return;
-        // (a wavefront takes a quarter of the step's inputs)
-        const int c = 2 * wave + (lane >> 5);
-        l_bf16x8 A[2];
-        GemmParts B[JM];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int r = 32 * i + (lane & 31);
-            A[i] = __builtin_bit_cast(l_bf16x8, s_w[r * 8 + (c ^ gemm_swz(r))]);
-            if (i < JM) B[i] = gemm_split(__builtin_bit_cast(float4, s_x[r * 16 + ((2 * c) ^ (r & 15))]), __builtin_bit_cast(float4, s_x[r * 16 + ((2 * c + 1) ^ (r & 15))]));
-        }
-#pragma unroll
-        for (int p = 2; p >= 0; p--)  // (the small parts first)
-#pragma unroll
-            for (int o = 0; o < 2 * JM; o++)
-                acc[o / JM][o % JM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[o / JM], B[o % JM].part[p], acc[o / JM][o % JM], 0, 0, 0);
     };
+    // inputs 8 c .. 8 c + 7 of a step, of row r of W and of X
+    auto weights = [&](int buffer, int r, int c) {
+        return __builtin_bit_cast(l_bf16x8, ((const l_u32x4 *)(s_raw + (2 * part + buffer) * BUFFER))[r * 8 + (c ^ gemm_swz(r))]);
+    };
+    auto parts = [&](int buffer, int r, int c) {
+        const l_u32x4 *s_x = (const l_u32x4 *)(s_raw + (2 * part + buffer) * BUFFER) + T * 8;
+        return gemm_split(__builtin_bit_cast(float4, s_x[r * 16 + ((2 * c) ^ (r & 15))]), __builtin_bit_cast(float4, s_x[r * 16 + ((2 * c + 1) ^ (r & 15))]));
+    };
+    l_f32x16 mine[1][1];
+    float *own;
     Step f;
     gload(f, 0);
-    clear(total);
-    clear(acc);
-    auto fold = [&] {
+    if constexpr (SHORT) {
+        l_f32x16 quarter[4];  // (of a step's inputs, as the wavefronts have them otherwise: the same sums)
 #pragma unroll
-        for (int o = 0; o < 2 * JM; o++) total[o / JM][o % JM] += acc[o / JM][o % JM];
-        clear(acc);
-    };
-    const int pairs = share & ~1;
-    for (int u0 = 0; u0 < pairs; u0 += FOLD) {
-        const int u1 = min(u0 + FOLD, pairs);
-        for (int u = u0; u < u1; u += 2) {
-            run(f, u, 0);
-            run(f, u + 1, 1);
+        for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) quarter[kk][r] = 0.0f;
+        for (int u = 0; u < steps; u++) {
+            to_lds(f, u & 1);
+            if (u + 1 < steps) gload(f, u + 1);
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                const int c = 2 * kk + (lane >> 5);
+                const l_bf16x8 A = weights(u & 1, 32 * (wave / JM) + (lane & 31), c);
+                const GemmParts B = parts(u & 1, 32 * (wave % JM) + (lane & 31), c);
+#pragma unroll
+                for (int p = 2; p >= 0; p--) quarter[kk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B.part[p], quarter[kk], 0, 0, 0);
+            }
         }
-        fold();
-    }
-    if (share & 1) {
-        run(f, pairs, 0);
-        fold();
-    }
-    // the four wavefronts' sums of a 32 x 32 tile each
-    l_lds_barrier();
-    float4 *sums = (float4 *)s_raw;
+        mine[0][0] = quarter[0] + quarter[1] + quarter[2] + quarter[3];
+        l_lds_barrier();
+        own = (float *)s_raw + gemm_epilogue_floats(1, 1) * wave;
+    } else {
+        l_f32x16 acc[2][JM], total[2][JM];
+        auto clear = [&](l_f32x16(&v)[2][JM]) {
 #pragma unroll
-    for (int o = 0; o < 2 * JM; o++)
+            for (int o = 0; o < 2 * JM; o++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) v[o / JM][o % JM][r] = 0.0f;
+        };
+        auto run = [&](Step &f, int step, int buffer) {
+            to_lds(f, buffer);
+            gload(f, step + 1);
+            if (KS > 1 && first + step >= steps) return;
+            // (a wavefront takes a quarter of the step's inputs)
+            const int c = 2 * wave + (lane >> 5);
+            l_bf16x8 A[2];
+            GemmParts B[JM];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                A[i] = weights(buffer, 32 * i + (lane & 31), c);
+                if (i < JM) B[i] = parts(buffer, 32 * i + (lane & 31), c);
+            }
+#pragma unroll
+            for (int p = 2; p >= 0; p--)  // (the small parts first)
+#pragma unroll
+                for (int o = 0; o < 2 * JM; o++)
+                    acc[o / JM][o % JM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[o / JM], B[o % JM].part[p], acc[o / JM][o % JM], 0, 0, 0);
+        };
+        clear(total);
+        clear(acc);
+        auto fold = [&] {
+#pragma unroll
+            for (int o = 0; o < 2 * JM; o++) total[o / JM][o % JM] += acc[o / JM][o % JM];
+            clear(acc);
+        };
+        const int pairs = share & ~1;
+        for (int u0 = 0; u0 < pairs; u0 += FOLD) {
+            const int u1 = min(u0 + FOLD, pairs);
+            for (int u = u0; u < u1; u += 2) {
+                run(f, u, 0);
+                run(f, u + 1, 1);
+            }
+            fold();
+        }
+        if (share & 1) {
+            run(f, pairs, 0);
+            fold();
+        }
+        // the four wavefronts' sums of a 32 x 32 tile each
+        l_lds_barrier();
+        float4 *sums = (float4 *)s_raw;
+#pragma unroll
+        for (int o = 0; o < 2 * JM; o++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const l_f32x16 &v = total[o / JM][o % JM];
+                sums[((o * 4 * KS + 4 * part + wave) * 4 + q) * 64 + lane] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+            }
+        l_lds_barrier();
+        if (part || wave >= 2 * JM) return;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const l_f32x16 &v = total[o / JM][o % JM];
-            sums[((o * 4 * KS + 4 * part + wave) * 4 + q) * 64 + lane] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-        }
-    l_lds_barrier();
-    if (part || wave >= 2 * JM) return;
-    l_f32x16 mine[1][1];
+            float4 v = sums[(wave * 4 * KS * 4 + q) * 64 + lane];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        float4 v = sums[(wave * 4 * KS * 4 + q) * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < 4 * KS; w++) {
-            const float4 z = sums[((wave * 4 * KS + w) * 4 + q) * 64 + lane];
-            v = make_float4(v.x + z.x, v.y + z.y, v.z + z.z, v.w + z.w);
+            for (int w = 1; w < 4 * KS; w++) {
+                const float4 z = sums[((wave * 4 * KS + w) * 4 + q) * 64 + lane];
+                v = make_float4(v.x + z.x, v.y + z.y, v.z + z.z, v.w + z.w);
+            }
+            mine[0][0][4 * q] = v.x, mine[0][0][4 * q + 1] = v.y, mine[0][0][4 * q + 2] = v.z, mine[0][0][4 * q + 3] = v.w;
         }
-        mine[0][0][4 * q] = v.x, mine[0][0][4 * q + 1] = v.y, mine[0][0][4 * q + 2] = v.z, mine[0][0][4 * q + 3] = v.w;
+        // (a wavefront's own quarter of s_raw: no other one reads it any more)
+        static_assert(4 * gemm_epilogue_floats(1, 1) <= 16384 * KS, "the epilogue's floats lie among a wavefront's own sums");
+        own = (float *)s_raw + 4096 * KS * wave;
     }
-    // (a wavefront's own quarter of s_raw: no other one reads it any more)
-    static_assert(4 * gemm_epilogue_floats(1, 1) <= 16384 * KS, "the epilogue's floats lie among a wavefront's own sums");
-    float *own = (float *)s_raw + 4096 * KS * wave;
     m0 += 32 * (wave % JM), n0 += 32 * (wave / JM);
     // An infinite activation's parts are itself and NaNs, and an infinite weight times a part that is zero is one: results that are NaN are computed again, on
     // the fp32 instructions (lane l has element l / 32 of two of row l % 32; a half's eight elements of 16 are consecutive).  509 positions through two experts of
@@ -308,16 +345,16 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_parts_kernel(GemmArgs a, uns
     gemm_epilogue<1, EPI, 1, 1>(a, mine, own, mb, m0, mcount, n0, lane);
 }
 
-template <int EPI, bool GROUPED, int KS, int TM>
+template <int EPI, bool GROUPED, int KS, int TM, bool SHORT = false>
 static hipError_t gemm_parts_go(hipStream_t s, const GemmArgs &a, unsigned n_nt) {
-    constexpr unsigned lds = KS * TM * 1024u;  // (the sums; the operands take three quarters of it, or all)
-    static_assert(2 * (128 + 4 * TM) * 64 <= TM * 1024, "two steps' operands lie in it");
+    constexpr unsigned lds = SHORT ? 2 * (128 + 4 * TM) * 64 : KS * TM * 1024u;  // (the sums; the operands take three quarters of it, or all)
+    static_assert(2 * (128 + 4 * TM) * 64 <= TM * 1024 && 4 * 4 * gemm_epilogue_floats(1, 1) <= 2 * (128 + 4 * TM) * 64, "two steps' operands lie in it; SHORT: the epilogue's floats");
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void *)gemm_parts_kernel<EPI, GROUPED, KS, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_parts_kernel<EPI, GROUPED, KS, TM, SHORT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     const dim3 grid = GROUPED ? dim3(8 * (((unsigned)a.max_tiles * n_nt + 7) / 8), L_GEMM_TILE / TM) : dim3((unsigned)((a.M + TM - 1) / TM), n_nt);
-    hipLaunchKernelGGL((gemm_parts_kernel<EPI, GROUPED, KS, TM>), grid, dim3(256 * KS), lds, s, a, n_nt);
+    hipLaunchKernelGGL((gemm_parts_kernel<EPI, GROUPED, KS, TM, SHORT>), grid, dim3(256 * KS), lds, s, a, n_nt);
     return hipGetLastError();
 }
 template <int EPI, bool GROUPED>
@@ -328,6 +365,8 @@ static hipError_t gemm_parts_launch(hipStream_t s, const GemmArgs &a, int64_t co
     // 15.9, 12.9, 12.2; x 256: 7.3, 7.3, 6.7; 100 positions, 8192 x 1024 (256) 15.8, 12.9, 14.0; 509, 3392 x 1024 (424) 20, 23, 21.  (A matrix's last block of
     // a grouped product is half full on average.)
     const int64_t halves = GROUPED ? (a.M + 63) / 64 + a.M / (2 * max(a.rows_each, 1)) : (a.M + 63) / 64, tiles = halves * n_nt;
+    // (of one or two steps, all results: see SHORT)
+    if (a.ld <= 128) return gemm_parts_go<EPI, GROUPED, 1, 64, true>(s, a, n_nt);
     if constexpr (!GROUPED)
         if (tiles <= 128 || (a.ld < 512 && tiles <= 256)) return gemm_parts_go<EPI, false, 2, 32>(s, a, n_nt);
     return a.ld >= 512 && tiles <= 256 ? gemm_parts_go<EPI, GROUPED, 2, 64>(s, a, n_nt) : gemm_parts_go<EPI, GROUPED, 1, 64>(s, a, n_nt);

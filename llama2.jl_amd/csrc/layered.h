@@ -132,7 +132,8 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 //
 // fp32, k_few's time over that of the tiles, at 256 to 4096 inputs.  Plain, up to 8 positions (0.3 to 0.97) and up to 2^17 results, 2^18 of up to 16 positions: of 17
 // positions and more 0.5 to 0.95 up to 2^16.5 results, 0.65 to 1.01 at 2^17, 0.95 to 1.34 at 2^17.5, 0.96 to 1.77 at 2^18, 1.2 to 2.1 at 2^20; of 9 to 12 positions 0.82 to
-// 1.08 beyond 2^18, where the tiles, whose sums are nearer to 64 bits, take them all the same; of 16 0.99 to 1.15 at 2^18.  Grouped, up to 64 positions a matrix and 2^18
+// 1.08 beyond 2^18, where the tiles, whose sums are nearer to 64 bits (of 256 inputs 0.9e-7 against 1.5e-7, of 4096 1.4e-7 and 4.0e-7), take them all the same; of 16 0.99 to
+// 1.15 at 2^18.  (With an activation behind them, from 2^17 to 2^18.3 results: up to 512 inputs 0.7 to 1.0, a microsecond, for the same reason.)  Grouped, up to 64 positions a matrix and 2^18
 // results: 8, 16, 32 and 64 positions each 0.4 to 0.99 up to 2^17, 0.75 to 1.27 at 2^18, 0.93 to 1.66 at 2^19; of 2 and 4 each 0.9 to 1.2; of 100 each 1.13 to 1.6, of 128
 // 1.2 to 1.9, of 512 1.2 to 1.9 up to 2^17.
 #define L_FEW_M 128

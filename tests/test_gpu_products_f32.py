@@ -32,8 +32,17 @@ def test_logits(pkg, width, vocab, n):
     assert lc.error(got, want) <= TOL
 
 
+# one and two steps of inputs (60, 64, 100, 128) with every epilogue that a prompt's products of them have: results, activations, gates and decays; more tiles than CUs, edges
+@pytest.mark.parametrize("width,ff,ranks,n", [(60, 2050, (64, 100), 130), (64, 16500, (1, 128), 97), (100, 2049, (128, 65), 161), (128, 9001, (100, 60), 64)])
+def test_few_inputs(pkg, width, ff, ranks, n):
+    c = lc.config([lc.delta(heads=24, kv_heads=4, dim=100, vdim=90, conv=4, ranks=ranks, mlp=lc.dense(ff))], width=width, vocab=2500)
+    t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 12).items()}
+    got, want = check(pkg, c, t, n)
+    assert lc.error(got, want) <= TOL
+
+
 # (experts, chosen, elements, width, positions): about 60, 65 and 150 positions an expert
-@pytest.mark.parametrize("experts,top,ff,width,n", [(9, 3, 530, 72, 181), (4, 2, 1030, 600, 130), (3, 3, 333, 515, 150)])
+@pytest.mark.parametrize("experts,top,ff,width,n", [(9, 3, 530, 72, 181), (4, 2, 1030, 600, 130), (3, 3, 333, 515, 150), (5, 2, 1100, 110, 200)])
 def test_experts(pkg, experts, top, ff, width, n):
     c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16, mlp=lc.moe(experts, top, ff))], width=width, vocab=50)
     t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 4).items()}
