@@ -566,8 +566,18 @@ hipError_t k_route(hipStream_t s, const float *z, int64_t ldz, const float *bias
 // one workgroup: counts, offsets, slots and the list of tiles.  The order of an expert's slots is whatever the LDS counters
 // give; every slot is computed on its own, so no result depends on it.  What bounds it is latency, so a thread's first GROUP_Q choices are
 // requested together, a choice is counted once (its place among its expert's is what the counter was) and the offsets are a scan: 2048 tokens with four of
-// 32 experts each 8.6 us, against 15.
+// 32 experts each 10 us, against 15; 57 tokens with four of 16 2.8 and 3.4, of 64 2.9 and 8.0; one of 2, whose offsets were no work, 2.7 and 2.5.
 #define GROUP_Q 8
+// sums over the lanes up to and including this one, without LDS: within the rows of sixteen lanes, then the rows before
+template <int SHIFT>
+__device__ __forceinline__ int group_add(int v) {
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x110 + SHIFT, 0xF, 0xF, true);  // row_shr
+}
+__device__ __forceinline__ int group_scan(int v, int lane) {
+    v = group_add<8>(group_add<4>(group_add<2>(group_add<1>(v))));
+    const int a = __builtin_amdgcn_readlane(v, 15), b = __builtin_amdgcn_readlane(v, 31), c = __builtin_amdgcn_readlane(v, 47);
+    return v + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
+}
 __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                                                      float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows) {
     extern __shared__ __align__(16) int s_int[];
@@ -591,27 +601,23 @@ __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, cons
     __syncthreads();
     // rows and tiles of the experts before e (E <= 1024: a thread for each)
     const int rows = t < E ? cnt[t] : 0, nt = (rows + tile_rows - 1) / tile_rows;
-    int sr = rows, st = nt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int r = __shfl_up(sr, d, WAVE), k = __shfl_up(st, d, WAVE);
-        sr += lane >= d ? r : 0;
-        st += lane >= d ? k : 0;
-    }
-    if (lane == 63) {
-        s_wave[0][wave] = sr;
-        s_wave[1][wave] = st;
-    }
-    __syncthreads();
-    for (int w = 0; w < wave; w++) {
-        sr += s_wave[0][w];
-        st += s_wave[1][w];
+    int sr = group_scan(rows, lane), st = group_scan(nt, lane);
+    if (E > 64) {
+        if (lane == 63) {
+            s_wave[0][wave] = sr;
+            s_wave[1][wave] = st;
+        }
+        __syncthreads();
+        for (int w = 0; w < wave; w++) {
+            sr += s_wave[0][w];
+            st += s_wave[1][w];
+        }
     }
     if (t < E) {
         off[t] = sr - rows;
         for (int k = 0; k < nt; k++) tiles[st - nt + k] = GemmTile{t, sr - rows + k * tile_rows, min(tile_rows, rows - k * tile_rows)};
+        if (t == E - 1) n_tiles[0] = st;
     }
-    if (t == 1023) n_tiles[0] = st;
     __syncthreads();
     auto put = [&](int i, int expert, float scale, int place) {
         const int slot = off[expert] + place;
