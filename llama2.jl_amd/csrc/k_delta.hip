@@ -315,14 +315,17 @@ __device__ __forceinline__ float delta_wave_sum16(const float (&v)[16], int lane
     return s + __shfl_xor(s, 32, WAVE);
 }
 
-// NE: key channels per lane (D <= 64 NE)
-template <int PREC, int NE>
+// NE: key channels per lane (D <= 64 NE).  TOGETHER: the inputs of all of them are requested together.  That takes 15 registers each, and pays with two of
+// up to four taps; otherwise the wavefronts that it costs are worth more.  2048 tokens, 8 heads of 256 x 256, 4 and 7 taps: 31 and 65 us (together, and a token's key heads
+// and values before the next token's, 34 and 98); 8 of 128 x 128, 7 and 16 taps: 34 and 98 (44 and 126).
+template <int PREC, int NE, bool TOGETHER>
 __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaShape d, const float *conv, const float *raw, int64_t ldr,
                                                             const float *ring, int M, int pos0, float *qkv, float *kq, float *beta,
                                                             void *fa, int64_t lfa, void *fg, int64_t lfg) {
     const int lane = threadIdx.x & 63, nv = (d.V + 63) / 64;
-    const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = blockIdx.y * PREP_T, n = min(PREP_T, M - m0);
+    // (the key heads of all tokens first: they take longest)
+    const int unit = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = blockIdx.x * PREP_T, n = min(PREP_T, M - m0);
     const int C = d.channels(), GD = d.G * d.D, taps = d.taps;
     PrepRows rows;
 #pragma unroll
@@ -365,23 +368,22 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaShape d, const 
     }
     // a key head's q and k
     float q[NE][PREP_T], k[NE][PREP_T];
-    {
-        PrepIn iq[NE], ik[NE];
+    auto channel = [&](int i) { return unit * d.D + min(lane + 64 * i, d.D - 1); };
+    PrepIn in[TOGETHER ? 2 * NE : 1];
+    if (TOGETHER)
 #pragma unroll
-        for (int i = 0; i < NE; i++) {
-            const int ch = unit * d.D + min(lane + 64 * i, d.D - 1);
-            delta_conv_request(iq[i], rows, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0);
-            delta_conv_request(ik[i], rows, conv, raw, ldr, ring, C, taps, GD + ch, m0, M, pos0);
-        }
+        for (int i = 0; i < 2 * NE; i++) delta_conv_request(in[i], rows, conv, raw, ldr, ring, C, taps, (i & 1 ? GD : 0) + channel(i >> 1), m0, M, pos0);
 #pragma unroll
-        for (int i = 0; i < NE; i++) {
-            const int e = lane + 64 * i, ch = unit * d.D + min(e, d.D - 1);
-            delta_conv_rows(iq[i], conv, raw, ldr, ring, C, taps, ch, m0, M, pos0, q[i]);
-            delta_conv_rows(ik[i], conv, raw, ldr, ring, C, taps, GD + ch, m0, M, pos0, k[i]);
-            if (e >= d.D)
+    for (int i = 0; i < 2 * NE; i++) {
+        PrepIn &x = in[TOGETHER ? i : 0];
+        const int ch = (i & 1 ? GD : 0) + channel(i >> 1);
+        if (!TOGETHER) delta_conv_request(x, rows, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0);
+        float(&y)[PREP_T] = i & 1 ? k[i >> 1] : q[i >> 1];
+        delta_conv_rows(x, conv, raw, ldr, ring, C, taps, ch, m0, M, pos0, y);
+        if (lane + 64 * (i >> 1) >= d.D)
 #pragma unroll
-                for (int j = 0; j < PREP_T; j++) q[i][j] = k[i][j] = 0.0f;
-        }
+            for (int j = 0; j < PREP_T; j++) y[j] = 0.0f;
+        if (!TOGETHER) __builtin_amdgcn_sched_barrier(0);
     }
     // lane l: what makes a unit vector of token l % 8's q, or of its k (l % 16 >= 8)
     float v[2 * PREP_T], f;
@@ -427,22 +429,26 @@ hipError_t k_delta_prepare(hipStream_t s, const DeltaShape &d, const float *conv
                            int M, int pos0, float *qkv, float *kq, float *beta, void *fa, int64_t lfa, void *fg, int64_t lfg,
                            int prec) {
     if (d.D > 256 || M < 1) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((d.G + d.H * ((d.V + 63) / 64) + 1 + 3) / 4), (unsigned)((M + PREP_T - 1) / PREP_T));
-#define GO(N)                                                                                                                            \
-    do {                                                                                                                                 \
-        if (prec)                                                                                                                        \
-            hipLaunchKernelGGL((delta_prepare_kernel<1, N>), grid, dim3(256), 0, s, d, conv, raw, ldr, ring, M, pos0, qkv, kq, beta, fa, \
-                               lfa, fg, lfg);                                                                                            \
-        else                                                                                                                             \
-            hipLaunchKernelGGL((delta_prepare_kernel<0, N>), grid, dim3(256), 0, s, d, conv, raw, ldr, ring, M, pos0, qkv, kq, beta, fa, \
-                               lfa, fg, lfg);                                                                                            \
+    const dim3 grid((unsigned)((M + PREP_T - 1) / PREP_T), (unsigned)((d.G + d.H * ((d.V + 63) / 64) + 1 + 3) / 4));
+#define GO(N, TOGETHER)                                                                                                                            \
+    do {                                                                                                                                           \
+        if (prec)                                                                                                                                  \
+            hipLaunchKernelGGL((delta_prepare_kernel<1, N, TOGETHER>), grid, dim3(256), 0, s, d, conv, raw, ldr, ring, M, pos0, qkv, kq, beta, fa, \
+                               lfa, fg, lfg);                                                                                                      \
+        else                                                                                                                                       \
+            hipLaunchKernelGGL((delta_prepare_kernel<0, N, TOGETHER>), grid, dim3(256), 0, s, d, conv, raw, ldr, ring, M, pos0, qkv, kq, beta, fa, \
+                               lfa, fg, lfg);                                                                                                      \
     } while (0)
-    switch ((d.D + 63) / 64) {
-    case 1: GO(1); break;
-    case 2: GO(2); break;
-    case 3: GO(3); break;
-    default: GO(4); break;
-    }
+    if (d.D <= 64)
+        GO(1, true);
+    else if (d.D <= 128 && d.taps <= CONV_AHEAD)
+        GO(2, true);
+    else if (d.D <= 128)
+        GO(2, false);
+    else if (d.D <= 192)
+        GO(3, false);
+    else
+        GO(4, false);
 #undef GO
     return hipGetLastError();
 }
