@@ -389,10 +389,12 @@ static hipError_t gemm_launch(hipStream_t s, const GemmArgs &a) {
         return hipGetLastError();
     }
     if (PREC) return gemm_parts_launch<EPI, false>(s, a, cols);
-    // (up to two steps of 64 inputs, a tile is its loads' latency and its epilogue: four small ones a CU wait for each other less.  2048 positions x 2048
-    // rows of 128 inputs, softplus or sigmoid behind them: 11 and 10 us, in tiles of 128 x 128 16 and 14)
+    // (up to two steps of 64 inputs, a tile is its loads' latency and its epilogue: four small ones a CU wait for each other less, unless there is little
+    // behind the products and tiles enough.  128 inputs, us, tiles of 64 x 64 and 128 x 128: 2048 positions x 2048 rows, softplus 10.1 and 14.4, an activation 8.5 and 16.3, stored
+    // 7.7 and 8.4; x 8192 rows 26 and 29, 20 and 32, 19.7 and 20.2; x 16 384 57 and 55, 37 and 54, 43 and 40; 300 x 32 000, stored 16.7 and 14.4)
+    constexpr int64_t enough = EPI == GE_STORE || EPI == GE_RESID ? 640 : EPI == GE_DECAY || EPI == GE_SIGMOID ? 2048 : (int64_t)1 << 62;
     const int64_t big = ((cols + 127) / 128) * ((a.M + 127) / 128);
-    if (big >= 256 && a.ld > 128)
+    if (big >= (a.ld > 128 ? 256 : enough))
         hipLaunchKernelGGL((gemm_kernel<EPI, 128, 128, false>), dim3((unsigned)((a.M + 127) / 128), (unsigned)((cols + 127) / 128)), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((gemm_kernel<EPI, 64, 64, false>), dim3((unsigned)((a.M + 63) / 64), (unsigned)((cols + 63) / 64)), dim3(256), 0, s, a);

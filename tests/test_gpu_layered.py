@@ -240,6 +240,19 @@ def test_fp32_products_on_both_sides_of_their_rule(pkg):
     dev.close()
 
 
+@pytest.mark.parametrize("width,vocab,n", [(64, 27300, 300), (128, 27301, 299), (100, 27200, 300)])
+def test_many_rows_of_few_inputs(pkg, width, vocab, n):
+    """bf16 logits of one or two steps of inputs through this library's own tiles: 642, 642 and 639 of 128 x 128, beside which lies their rule"""
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16)], width=width, vocab=vocab)
+    t = {k: ref.bf16(np.array(v)) for k, v in ref.random_tensors(c, 53).items()}
+    tok = lc.tokens(n, c["vocab"], 6)
+    want = ref.Sequence(c, t).run(tok)
+    dev = lc.language_model(pkg, c, t, precision="bfloat16").device()
+    dev.set_prefill_library(False)
+    assert lc.error(dev.prefill_logits(tok, np.arange(n)), want) <= TOL["bfloat16"]
+    dev.close()
+
+
 @pytest.mark.parametrize("stage", ["0", "100", "4000", "70001"])
 def test_upload_through_any_staging_block(pkg, monkeypatch, stage):
     """Matrices go up the same through a block of any size: one that holds no row of theirs or cannot be had (0), some rows, whole matrices"""
