@@ -247,7 +247,7 @@ hipError_t k_window_prepare(hipStream_t s, const WindowShape &w, const float *fr
 // operand for four tiles is one word of 16 bytes of a key's values, and its results are 16 neighbouring columns of one query.
 // What bounds it is the matrix cores' 2 x 32 cycles for every four elements of a head, on the CU whose queries see the most keys, and the loads
 // ahead of them: a tile's values are requested before its scores are formed and the next tile's keys behind them.  8 heads of 128, 509 queries, all before
-// them in the window: 26 us; with a key a lane and the products on the vector units 94.  Where windows are short it is the queries' loads and the
+// them in the window: 21 us; with a key a lane and the products on the vector units 94.  Where windows are short it is the queries' loads and the
 // outputs' stores, 16 bytes each a lane where sizes allow it, and wavefronts without keys, of which there are none (k_window_rows): 32 heads of 128, 2048 queries, a window of 8
 // 124 us with eight wavefronts a block, 34 with one; words of 4 bytes 155.
 // N: groups of 64 elements of a head (key and value elements up to 64 N); NW: wavefronts

@@ -1,5 +1,5 @@
-"""The delta rule's prompt pass in chunks of 32 tokens: lengths around a tile of 16 tokens, a chunk and three of them (the operands under way), from an
-empty state and going on from one, heads at the edges of what a wavefront takes."""
+"""The delta rule's prompt pass from an empty state and going on from one, heads at the edges of what a wavefront takes.  From 48 tokens on lengths around
+chunks (of 32; of 16 where a head has more than 128 value elements) and three of them, the operands under way; below that it goes token by token."""
 import numpy as np
 import pytest
 

@@ -41,7 +41,7 @@ def test_few_inputs(pkg, width, ff, ranks, n):
     assert lc.error(got, want) <= TOL
 
 
-# (experts, chosen, elements, width, positions): about 60, 65 and 150 positions an expert
+# (experts, chosen, elements, width, positions): about 60, 65, 150 and 80 positions an expert
 @pytest.mark.parametrize("experts,top,ff,width,n", [(9, 3, 530, 72, 181), (4, 2, 1030, 600, 130), (3, 3, 333, 515, 150), (5, 2, 1100, 110, 200)])
 def test_experts(pkg, experts, top, ff, width, n):
     c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, size=8, rot=16, mlp=lc.moe(experts, top, ff))], width=width, vocab=50)
