@@ -26,6 +26,26 @@ __device__ __forceinline__ float wave_max_f32(float v) {
     return v;
 }
 
+// the largest of the wavefront's, in every lane: sixteen lanes by DPP, the four of those on the scalar path
+template <int CTRL>
+__device__ __forceinline__ unsigned long long dpp_max_u64(unsigned long long v) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, 0xF, 0xF, true);
+    const unsigned long long o = (unsigned long long)hi << 32 | lo;
+    return o > v ? o : v;
+}
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+    v = dpp_max_u64<0x121>(dpp_max_u64<0x122>(dpp_max_u64<0x124>(dpp_max_u64<0x128>(v))));  // row_ror: 8, 4, 2, 1
+    unsigned long long m = 0;
+#pragma unroll
+    for (int i = 0; i < 64; i += 16) {
+        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, i), hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), i);
+        const unsigned long long o = (unsigned long long)hi << 32 | lo;
+        m = o > m ? o : m;
+    }
+    return m;
+}
+
 // Sum of one double per thread over a workgroup of up to 1024 threads; every thread gets
 // the total.  `red` is LDS scratch of at least 16 doubles.  The order of the fp64
 // additions is fixed by the thread layout.

@@ -51,11 +51,7 @@ __device__ __forceinline__ float delta_fma8(uint4 p, const float *x, float acc) 
     acc = fmaf(l_bf16_lo(p.w), b.z, acc);
     return fmaf(l_bf16_hi(p.w), b.w, acc);
 }
-__device__ __forceinline__ float delta_sum8(float acc) {
-#pragma unroll
-    for (int m = 4; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, WAVE);
-    return acc;
-}
+__device__ __forceinline__ float delta_sum8(float acc) { return l_dpp_add<0x141>(l_dpp_add<0x4E>(l_dpp_add<0xB1>(acc))); }  // lanes l ^ 1, l ^ 2, 7 - l
 
 // one of 16 sums over the 16 lanes of a row: lane l gets that of v[l].  Every step halves the sums: lanes l and 15 - l, l and 7 - l, l and l ^ 2, l and l ^ 1
 template <int CTRL>
@@ -71,13 +67,6 @@ __device__ __forceinline__ float delta_sum16(const float (&v)[16], int l) {
 #pragma unroll
     for (int i = 0; i < 2; i++) c[i] = delta_swap_add<0x4E>(l & 2, b[i], b[i + 2]);
     return delta_swap_add<0xB1>(l & 1, c[0], c[1]);
-}
-
-// sum over the wavefront, in every lane: the rows of sixteen lanes without LDS
-__device__ __forceinline__ float delta_wave_sum(float v) {
-    v = l_dpp_add<0x121>(l_dpp_add<0x122>(l_dpp_add<0x124>(l_dpp_add<0x128>(v))));  // row_ror: 8, 4, 2, 1
-    v += __shfl_xor(v, 16, WAVE);
-    return v + __shfl_xor(v, 32, WAVE);
 }
 
 // What bounds this is latency: 56 KB a workgroup (1.2 us of HBM in all) in front of a chain of three sums.  So everything is
@@ -164,7 +153,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(DeltaShape d, DeltaWeig
         const float *x = wave == 0 ? s_q : s_k, *y = wave == 1 ? s_k : s_q;
         float ss = 0.0f;
         for (int e = lane; e < D; e += 64) ss = fmaf(x[e], y[e], ss);
-        ss = delta_wave_sum(ss);
+        ss = l_wave_sum(ss);
         if (wave < 2) ss = 1.0f / sqrtf(ss + 1e-6f);
         if (wave == 0) ss *= 1.0f / sqrtf((float)D);
         if (lane == 0) s_unit[wave] = ss;

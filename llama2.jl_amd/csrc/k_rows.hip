@@ -82,7 +82,7 @@ static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu, const Ro
     if constexpr (PRO == RP_PLAIN || PRO == RP_DOWN) {
         return rows_split<PRO, EPI, 8, false>(s, a, n_cu, m, keys);
     } else if constexpr (PRO == RP_HEADNORM) {
-        return rows_split<PRO, EPI, 4, false>(s, a, n_cu, m, keys);
+        return a.K <= 2 * 4 * ROWS_THREADS ? rows_split<PRO, EPI, 2, false>(s, a, n_cu, m, keys) : rows_split<PRO, EPI, 4, false>(s, a, n_cu, m, keys);
     } else {
         const bool few = a.K <= 2 * 4 * ROWS_THREADS;
         if constexpr (PRO == RP_NORM && (EPI == RE_STORE || EPI == RE_STORE_GLU || EPI == RE_STORE_KEY)) {
@@ -94,9 +94,10 @@ static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu, const Ro
 }
 
 hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, const RowsMore &more) {
-    if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.ld % 64 != 0 || a.K > a.ld || a.K < 1) return hipErrorInvalidValue;
+    if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.n_rows > 0x7FFFFFFF || a.ld % 64 != 0 || a.K > a.ld || a.K < 1) return hipErrorInvalidValue;
     if ((pro == RP_UP || pro == RP_DOWN) &&
-        (!a.z || a.n_experts < 1 || a.n_experts > ROWS_MAX_EXPERTS || a.top < 1 || a.top > ROWS_MAX_TOP || a.top > a.n_experts))
+        (!a.z || a.n_experts < 1 || a.n_experts > ROWS_MAX_EXPERTS || a.top < 1 || a.top > ROWS_MAX_TOP || a.top > a.n_experts ||
+                                           a.n_experts * a.rows_each > 0x7FFFFFFF))
         return hipErrorInvalidValue;
     if ((epi == RE_GLU && a.n_rows % 2 != 0) || (epi == RE_STORE_GLU && (a.n_rows % 2 != 0 || a.glu_from % 2 != 0 || !a.out2)))
         return hipErrorInvalidValue;
@@ -127,6 +128,6 @@ hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, 
 }
 
 hipError_t k_rows_keys(hipStream_t s, const RowsArgs &a, int n_cu, const RowsKeys &keys) {
-    if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.ld % 64 != 0 || a.K > a.ld || a.K < 1 || !keys.keys || !keys.ctl || !keys.next) return hipErrorInvalidValue;
+    if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.n_rows > 0x7FFFFFFF || a.ld % 64 != 0 || a.K > a.ld || a.K < 1 || !keys.keys || !keys.ctl || !keys.next) return hipErrorInvalidValue;
     return rows_pick<RP_NORM, RE_STORE_KEY>(s, a, n_cu, RowsMore(), keys);
 }

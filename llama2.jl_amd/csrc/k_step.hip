@@ -103,7 +103,7 @@ __device__ __forceinline__ void step_query_body(const LatentStep &a, int h, Step
             for (int i = w.R + lane; i < Rp; i += 64) row[Cp + i] = 0.0f;
         }
         const float v = t < C ? kv[t] : 0.0f, g = t < C ? a.kvnorm[t] : 0.0f;
-        const float r = 1.0f / sqrtf(l_block_sum_lds(v * v, s.red) / (float)C + w.eps);
+        const float r = l_rsqrt(l_block_sum_lds(v * v, s.red) / (float)C + w.eps);
         if (t < Cp) row[t] = v * r * g;  // (zero from C on)
     }
     float acc[8];

@@ -260,8 +260,14 @@ hipError_t k_softmax(hipStream_t s, float *x, int64_t n);
 hipError_t k_argmax(hipStream_t s, const float *x, int64_t n, int64_t *partial, DecodeCtl *ctl, int32_t *out_tokens,
                     int max_out, bool step);
 hipError_t k_argmax_keys(hipStream_t s, const unsigned long long *keys, int n, DecodeCtl *ctl, int32_t *out_tokens, int max_out);
+// what a step's first launch copies for the per-token inputs of the layers: a row of n elements for every token, and the token's own
+struct StepSide {
+    const uint16_t *table = nullptr;
+    uint16_t *row = nullptr;
+    int64_t n = 0;
+};
 hipError_t k_step_begin(hipStream_t s, const DevTensor &emb, const DecodeCtl *prev, DecodeCtl *ctl, const unsigned long long *keys, int n_keys,
-                        const int32_t *prompt, int32_t *out_tokens, int max_out, float *x, float scale, float *x_copy);
+                        const int32_t *prompt, int32_t *out_tokens, int max_out, float *x, float scale, float *x_copy, const StepSide &side);
 // argmax without allocations: k_noalloc_init once per device (that device current), then k_argmax_noalloc
 hipError_t k_noalloc_init(int device);
 hipError_t k_argmax_noalloc(hipStream_t s, int device, const float *x_dev, int64_t n, int32_t *out_dev);

@@ -45,7 +45,7 @@ struct Layered {
     std::vector<LayerRun> run;
     LMat head;
     float *loop_step = nullptr;
-    uint16_t *side_emb = nullptr;
+    uint16_t *side_emb = nullptr, *side_row = nullptr;  // (the row of the step's token)
     float *final_norm = nullptr;
     uint64_t have = 0;
     int pos = 0;  // positions the state has taken in
@@ -54,6 +54,7 @@ struct Layered {
     // one token
     float *x_alt = nullptr, *in = nullptr, *mix = nullptr, *ssq = nullptr, *gate = nullptr, *hid = nullptr, *z = nullptr,
           *se = nullptr, *y = nullptr, *part = nullptr, *x0 = nullptr, *lq = nullptr, *qa = nullptr;
+    int32_t *sel = nullptr;  // the experts that a step's last choice has left
     unsigned *count = nullptr;  // k_step_latent's, zero between launches
     unsigned long long *keys = nullptr;  // the classifier's, a key for each of its workgroups
     int n_keys = 0;
@@ -605,7 +606,7 @@ int layered_finalize(l2h_model *m) {
     l2h_ctx *ctx = m->ctx;
     Layered *l = m->lay;
     const l2h_layered_config &c = l->c;
-    int n_in = 1, hv = 1, hid = 1, ne = 1, ssq = 1;
+    int n_in = 1, hv = 1, hid = 1, ne = 1, ssq = 1, top = 1;
     int64_t part = 1, lq = 0, qa = 0;
     int heads = 0;
     auto missing = [&](uint64_t have, int role, int layer) -> int {
@@ -663,7 +664,7 @@ int layered_finalize(l2h_model *m) {
         n_in = std::max(n_in, L.n_plain);
         hv = std::max(hv, std::max(d.n_heads * d.vdim, L.joined ? L.o.ld : 0));
         if (d.ff != L2H_FF_NONE) hid = std::max(hid, d.ff_dim * (d.ff == L2H_FF_EXPERTS ? d.top : 1));
-        if (d.ff == L2H_FF_EXPERTS) ne = std::max(ne, d.n_experts);
+        if (d.ff == L2H_FF_EXPERTS) ne = std::max(ne, d.n_experts), top = std::max(top, d.top);
     }
     for (LayerRun &r : l->run) {
         const LayerDev &L = l->layer[(size_t)r.layer];
@@ -687,6 +688,8 @@ int layered_finalize(l2h_model *m) {
     DA(l->hid, hid, true);
     DA(l->z, ne, true);
     DA(l->se, std::max(1, c.side_dim), true);
+    DA(l->side_row, std::max<int64_t>(1, (int64_t)c.n_layers * c.side_dim), true);
+    DA(l->sel, top, true);
     DA(l->y, c.width, true);
     RowsArgs head = rows_of(l->head, m->x, m->logits);
     head.y = c.side_dim ? l->y : nullptr;  // (what the last layer leaves pending)
@@ -802,12 +805,13 @@ struct LatentLayerStep {
     int up_pro, down_pro;
     int64_t stride = 0;  // from row to row of `down` and `o` (0: their ld)
 };
-static void set_router(RowsArgs &a, const LayerDev &L, const float *z) {
+static void set_router(RowsArgs &a, const LayerDev &L, const float *z, int32_t *sel) {
     a.z = z;
     a.z_bias = L.router_bias;
     a.n_experts = L.d.n_experts;
     a.top = L.d.top;
     a.route = L.d.route;
+    a.sel = sel;
 }
 static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int cu, LatentLayerStep &a) {
     const l2h_layer &d = L.d;
@@ -835,8 +839,8 @@ static bool shares_launches(const Layered *l, const LayerDev &L, float *x, int c
     a.up_pro = dense ? RP_NORM : RP_UP;
     a.down_pro = dense ? RP_PLAIN : RP_DOWN;
     if (!dense) {
-        set_router(a.up, L, l->in + L.off_z);
-        set_router(a.down, L, l->in + L.off_z);
+        set_router(a.up, L, l->in + L.off_z, l->sel);
+        set_router(a.down, L, l->in + L.off_z, l->sel);
         a.up.rows_each = L.up_rows();
         a.up.n_rows = (int64_t)d.top * L.up_rows();
         a.down.rows_each = a.down.n_rows = l->c.width;
@@ -908,7 +912,7 @@ static hipError_t separate_launches(l2h_model *m, LayerDev &L, const LayerRun &r
             r.normw = up.normw;
             r.eps = c.norm_eps;
             if (!early) CK(k_rows(s, r, RP_NORM, RE_STORE, cu));
-            for (RowsArgs *a : {&up, &down}) set_router(*a, L, early ? l->in + L.off_z : l->z);
+            for (RowsArgs *a : {&up, &down}) set_router(*a, L, early ? l->in + L.off_z : l->z, l->sel);
             up.rows_each = L.up_rows();
             up.n_rows = (int64_t)d.top * L.up_rows();
             down.rows_each = c.width;
@@ -928,7 +932,8 @@ hipError_t layered_enqueue_token(l2h_model *m) {
     const l2h_layered_config &c = l->c;
     hipError_t e;
     Stream st(m);
-    CK(k_step_begin(s, m->glob[L2H_TOK_EMB], m->ctl + 1, m->ctl, l->keys, l->n_keys, m->prompt_dev, m->out_tokens, m->max_out, st.x, c.embed_scale, l->x0));
+    CK(k_step_begin(s, m->glob[L2H_TOK_EMB], m->ctl + 1, m->ctl, l->keys, l->n_keys, m->prompt_dev, m->out_tokens, m->max_out, st.x, c.embed_scale, l->x0,
+                    StepSide{l->side_emb, l->side_row, (int64_t)c.n_layers * c.side_dim}));
     // What a pass of a loop begins with, x += [x0] + step, is added by the launch that completes the stream before it (a launch of its own: 4.5 us of
     // a 280 us token twice) unless that is the embedding's or a pending update comes in between.
     bool added = false;
@@ -965,10 +970,7 @@ hipError_t layered_enqueue_token(l2h_model *m) {
         if (c.side_dim) {
             RowsArgs g = rows_of(L.side_gate, x, l->se);
             g.act = LACT_GELU_TANH;
-            g.emb = l->side_emb + (int64_t)run.layer * c.side_dim;
-            g.emb_ld = (int64_t)c.n_layers * c.side_dim;
-            g.ctl = m->ctl;
-            g.prompt = m->prompt_dev;
+            g.emb = l->side_row + (int64_t)run.layer * c.side_dim;
             CK(k_rows(s, g, RP_PLAIN, RE_EMBED, cu));
             CK(k_rows(s, rows_of(L.side_proj, l->se, l->y), RP_PLAIN, RE_STORE, cu));
             st.yw = L.side_norm;

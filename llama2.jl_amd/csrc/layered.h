@@ -31,7 +31,7 @@ enum { LROUTE_SIGMOID_IN = 0, LROUTE_SOFTMAX_OUT = 1 };
 //   RP_HEADNORM x[h * hv + j] * rms over the head's hv elements (from partial sums of squares) * normw[j] * gate[...]
 enum { RP_PLAIN = 0, RP_NORM = 1, RP_UP = 2, RP_DOWN = 3, RP_HEADNORM = 4 };
 // epilogues: RE_STORE v; RE_RESID resid + mult * v; RE_ACT act(v); RE_UP act(score * v) or score * act(v) with the expert's score;
-// RE_EMBED act(v) * the token's row of an embedding table; RE_GLU rows 2 i and 2 i + 1 give out[i] = act(v) * v', with the
+// RE_EMBED act(v) * emb[row]; RE_GLU rows 2 i and 2 i + 1 give out[i] = act(v) * v', with the
 // expert's score behind RP_UP; RE_STORE_GLU stores rows below glu_from and treats the others so, into out2; RE_STORE_AGENT v, past the
 // caches of the storing workgroup; RE_RESID_MORE as RE_RESID, with a RowsMore (k_rows takes it where one of its fields is set); RE_STORE_KEY v, and a
 // workgroup's largest (k_rows_keys)
@@ -55,10 +55,8 @@ struct RowsArgs {
     int64_t rows_each = 0;
     const float *ssq = nullptr, *gate = nullptr;  // RP_HEADNORM
     int hv = 0, n_split = 0;
-    const uint16_t *emb = nullptr;  // RE_EMBED: element emb[token * emb_ld + row]
-    int64_t emb_ld = 0;
-    const DecodeCtl *ctl = nullptr;
-    const int32_t *prompt = nullptr;
+    const uint16_t *emb = nullptr;  // RE_EMBED
+    int32_t *sel = nullptr;         // RP_UP leaves the chosen experts there, RP_DOWN finds them (or chooses for itself)
 };
 // What few products of a residual have.  Apart, for the sake of the others: with these fields and their branches in every launch a token of Vudelix took 1 % longer
 // (width 768, 4 layers: 170.6 us against 169.2).

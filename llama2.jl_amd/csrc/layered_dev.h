@@ -58,32 +58,26 @@ __device__ __forceinline__ float l_act_rounded(int act, float z) {
     return l_act(act, z);
 }
 
-__device__ __forceinline__ float l_wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, WAVE);
-    return v;
+// 1 / sqrt(x) within a unit in the last place: the hardware's with a step of Newton's method.  (1 / sqrtf(x), with its exact root and quotient, is forty
+// instructions in a row, which a launch of a decode step also has to fetch: 0.1 us of 3.)
+__device__ __forceinline__ float l_rsqrt(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), e = fmaf(-x * y, y, 1.0f), z = fmaf(0.5f * y, e, y);
+    return e == e ? z : y;  // (0 and infinity as they are)
 }
+
 // v plus its value in another lane of the same sixteen
 template <int CTRL>
 __device__ __forceinline__ float l_dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-template <int CTRL>
-__device__ __forceinline__ unsigned long long l_dpp_max(unsigned long long v) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, 0xF, 0xF, true);
-    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, 0xF, 0xF, true);
-    const unsigned long long o = (unsigned long long)hi << 32 | lo;
-    return o > v ? o : v;
-}
-// the largest of the wavefront's, in every lane
-__device__ __forceinline__ unsigned long long l_wave_max(unsigned long long v) {
-    v = l_dpp_max<0x121>(l_dpp_max<0x122>(l_dpp_max<0x124>(l_dpp_max<0x128>(v))));  // row_ror: 8, 4, 2, 1
-#pragma unroll
-    for (int m = 16; m <= 32; m <<= 1) {
-        const unsigned long long o = __shfl_xor(v, m, WAVE);
-        v = o > v ? o : v;
-    }
-    return v;
+// Sum over the wavefront, in every lane: sixteen lanes by DPP, the four sums of those on the scalar path (no LDS: six exchanges through it take 0.2 us,
+// and a launch of a decode step has two to four such sums one after the other).
+__device__ __forceinline__ float l_wave_sum(float v) {
+    v = l_dpp_add<0x121>(l_dpp_add<0x122>(l_dpp_add<0x124>(l_dpp_add<0x128>(v))));  // row_ror: 8, 4, 2, 1
+    const int i = __float_as_int(v);
+    const float a = __int_as_float(__builtin_amdgcn_readlane(i, 0)), b = __int_as_float(__builtin_amdgcn_readlane(i, 16)),
+                c = __int_as_float(__builtin_amdgcn_readlane(i, 32)), d = __int_as_float(__builtin_amdgcn_readlane(i, 48));
+    return (a + b) + (c + d);
 }
 // sum over the workgroup; `red` holds one float per wavefront; every thread gets the total
 __device__ __forceinline__ float l_block_sum(float v, float *red) {
@@ -119,11 +113,6 @@ __device__ __forceinline__ void l_store_act(void *p, int64_t i, float v) {
         ((__bf16 *)p)[i] = (__bf16)v;
 }
 
-// the token of the current decode step (as embed_kernel picks it)
-__device__ __forceinline__ int l_step_token(const DecodeCtl *ctl, const int32_t *prompt) {
-    return ctl->step < ctl->n_prompt ? prompt[ctl->step] : ctl->last_argmax;
-}
-
 // Rotation of the pairs (2 i, 2 i + 1), or with `half` (i, i + rot / 2), i < rot / 2, of one head at `pos` and division by the
 // head's root mean square, by one wavefront.  src and dst hold D elements.
 __device__ __forceinline__ void l_rotate_norm(const float *src, float *dst, int D, int rot, int half, const float *freq, int pos,
@@ -145,7 +134,7 @@ __device__ __forceinline__ void l_rotate_norm(const float *src, float *dst, int 
         if (ib < D) dst[ib] = b;
     }
     if (!norm) return;
-    const float r = 1.0f / sqrtf(l_wave_sum(ss) / (float)D + eps);
+    const float r = l_rsqrt(l_wave_sum(ss) / (float)D + eps);
     for (int p = lane; 2 * p < D; p += 64) {
         const bool apart = half && 2 * p < rot;
         const int ia = apart ? p : 2 * p, ib = apart ? p + rot / 2 : 2 * p + 1;

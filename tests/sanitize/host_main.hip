@@ -194,6 +194,16 @@ static void check_rows_plan() {
                     }
 }
 
+// quotients without a division, where rounding could show: around multiples, over all of the range
+static void check_rows_div() {
+    for (unsigned d = 1; d < 70000; d += d < 3000 ? 1 : 61) {
+        const RowsDiv v = rows_div(d);
+        for (unsigned long long k = 0; k * d < 0x80000000ull; k += 1 + k / 7)
+            for (long long n : {(long long)(k * d) - 1, (long long)(k * d), (long long)(k * d + d / 2), 0x7FFFFFFFll})
+                if (n >= 0 && n < 0x80000000ll) EXPECT(rows_quot((unsigned)n, v) == (unsigned)n / d);
+    }
+}
+
 // the delta rule's scratch holds what every prompt of up to its length takes of it, and is not more than the outputs and records of chunks of 16 tokens
 // by what the rule says; with less memory, fewer chunks a pass
 static void check_delta_plan() {
@@ -356,6 +366,7 @@ int main() {
     check_small_plan();
     check_product_rule();
     check_rows_plan();
+    check_rows_div();
     check_delta_plan();
     check_delta_ring();
     check_boxes();
