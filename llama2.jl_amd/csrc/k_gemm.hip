@@ -580,10 +580,18 @@ __device__ __forceinline__ int group_scan(int v, int lane) {
     const int a = __builtin_amdgcn_readlane(v, 15), b = __builtin_amdgcn_readlane(v, 31), c = __builtin_amdgcn_readlane(v, 47);
     return v + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
 }
+// What the lists of blocks are made of: blocks of tile_rows (IMAGES: of tiles_plan.h's units, with a bound for each of two products)
+struct GroupLists {
+    GemmTile *tiles[2];
+    int tile_rows;
+    unsigned bound[2];
+};
+template <bool IMAGES>
 __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
-                                                     float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows) {
+                                                     float *slot_scale, int32_t *slot_of, int32_t *n_tiles, GroupLists lists) {
+    constexpr int NP = IMAGES ? 2 : 1;
     extern __shared__ __align__(16) int s_int[];
-    __shared__ int s_wave[2][16];
+    __shared__ int s_wave[1 + NP][16];
     int *cnt = s_int, *off = s_int + E;
     const int n = M * top, t = threadIdx.x, lane = t & 63, wave = t >> 6;
     int c[GROUP_Q], rank[GROUP_Q];
@@ -601,24 +609,45 @@ __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, cons
         if (t + 1024 * u < n) rank[u] = atomicAdd(&cnt[c[u]], 1);
     for (int i = t + 1024 * GROUP_Q; i < n; i += 1024) slot_of[i] = atomicAdd(&cnt[choice[i]], 1);
     __syncthreads();
-    // rows and tiles of the experts before e (E <= 1024: a thread for each)
-    const int rows = t < E ? cnt[t] : 0, nt = (rows + tile_rows - 1) / tile_rows;
-    int sr = group_scan(rows, lane), st = group_scan(nt, lane);
+    // rows and blocks of the experts before e (E <= 1024: a thread for each)
+    const int rows = t < E ? cnt[t] : 0;
+    const unsigned units = (unsigned)(rows + TILES_UNIT - 1) / TILES_UNIT;
+    int nt[NP];
+    if constexpr (IMAGES) {
+#pragma unroll
+        for (int p = 0; p < NP; p++) nt[p] = (int)tiles_blocks(units, lists.bound[p]);
+    } else {
+        nt[0] = (rows + lists.tile_rows - 1) / lists.tile_rows;
+    }
+    int sr = group_scan(rows, lane), st[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) st[p] = group_scan(nt[p], lane);
     if (E > 64) {
         if (lane == 63) {
             s_wave[0][wave] = sr;
-            s_wave[1][wave] = st;
+#pragma unroll
+            for (int p = 0; p < NP; p++) s_wave[1 + p][wave] = st[p];
         }
         __syncthreads();
         for (int w = 0; w < wave; w++) {
             sr += s_wave[0][w];
-            st += s_wave[1][w];
+#pragma unroll
+            for (int p = 0; p < NP; p++) st[p] += s_wave[1 + p][w];
         }
     }
     if (t < E) {
         off[t] = sr - rows;
-        for (int k = 0; k < nt; k++) tiles[st - nt + k] = GemmTile{t, sr - rows + k * tile_rows, min(tile_rows, rows - k * tile_rows)};
-        if (t == E - 1) n_tiles[0] = st;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            GemmTile *tiles = lists.tiles[p] + (st[p] - nt[p]);
+            const TilesShares share(IMAGES ? units : 0, IMAGES ? (unsigned)nt[p] : 0);
+            for (int k = 0, r0 = 0; k < nt[p]; k++) {
+                const int r1 = IMAGES ? TILES_UNIT * (int)share.at((unsigned)k + 1) : r0 + lists.tile_rows;
+                tiles[k] = GemmTile{t, sr - rows + r0, min(r1, rows) - r0};
+                r0 = r1;
+            }
+            if (t == E - 1) n_tiles[p] = st[p];
+        }
     }
     __syncthreads();
     auto put = [&](int i, int expert, float scale, int place) {
@@ -634,9 +663,18 @@ __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, cons
 }
 hipError_t k_group(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                    float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows) {
-    if (E < 1 || E > 1024 || M < 1 || top < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 2 * E * sizeof(int), s, choice, score, M, E, top, slot_row, slot_scale, slot_of,
-                       tiles, n_tiles, tile_rows);
+    if (E < 1 || E > 1024 || M < 1 || top < 1 || tile_rows < 1) return hipErrorInvalidValue;
+    GroupLists l = {};
+    l.tiles[0] = tiles;
+    l.tile_rows = tile_rows;
+    hipLaunchKernelGGL(group_kernel<false>, dim3(1), dim3(1024), 2 * E * sizeof(int), s, choice, score, M, E, top, slot_row, slot_scale, slot_of, n_tiles, l);
+    return hipGetLastError();
+}
+hipError_t k_group_images(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row, float *slot_scale,
+                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const unsigned bound[2]) {
+    if (E < 1 || E > 1024 || M < 1 || top < 1 || bound[0] < 1 || bound[0] > TILES_MAX_UNITS || bound[1] < 1 || bound[1] > TILES_MAX_UNITS) return hipErrorInvalidValue;
+    const GroupLists l = {{tiles[0], tiles[1]}, 0, {bound[0], bound[1]}};
+    hipLaunchKernelGGL(group_kernel<true>, dim3(1), dim3(1024), 2 * E * sizeof(int), s, choice, score, M, E, top, slot_row, slot_scale, slot_of, n_tiles, l);
     return hipGetLastError();
 }
 

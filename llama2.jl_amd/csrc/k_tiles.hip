@@ -78,20 +78,28 @@ __global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, u
         nt = item / n_mt;
         m0 = (int)(item % n_mt) * 64 * JT;
     }
-    // (A block of a grouped product that has at most 128 rows takes half the positions, in three stages: its steps last as long as their loads.
-    // 16 experts of about 84 rows, 2048 x 4096 and 4096 x 2048: 99 and 66 us in two stages, 84 and 58 in three; 32 of about 256, half
-    // of them with a few rows more, 392 and 211 against 378 and 202.)
-    if (GROUPED && JT == 4 && mcount <= 128)
-        tiles_item<EPI, 2, pf_tile_stages(2)>(a, w, nt, mb, m0, mcount, s_all);
-    else
+    if constexpr (GROUPED) {
+        const int units = (mcount + 63) >> 6;
+        if (units == 5)
+            tiles_item<EPI, 5, pf_tile_stages(5)>(a, w, nt, mb, m0, mcount, s_all);
+        else if (units == 4)
+            tiles_item<EPI, 4, pf_tile_stages(4)>(a, w, nt, mb, m0, mcount, s_all);
+        else if (units == 3)
+            tiles_item<EPI, 3, pf_tile_stages(3)>(a, w, nt, mb, m0, mcount, s_all);
+        else if (units == 2)
+            tiles_item<EPI, 2, pf_tile_stages(2)>(a, w, nt, mb, m0, mcount, s_all);
+        else
+            tiles_item<EPI, 1, pf_tile_stages(1)>(a, w, nt, mb, m0, mcount, s_all);
+    } else {
         tiles_item<EPI, JT, pf_tile_stages(JT)>(a, w, nt, mb, m0, mcount, s_all);
+    }
 }
 
 #define TILES_MAX_DEVICES 64
 
 template <int EPI, int JT, bool GROUPED>
 static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, unsigned n_mt, int n_cu) {
-    constexpr int lds = pf_tile_lds(2) > pf_tile_lds(JT) ? pf_tile_lds(2) : pf_tile_lds(JT);  // (halves and small blocks among them)
+    constexpr int lds = std::max(pf_tile_lds(2), pf_tile_lds(GROUPED ? 5 : JT));  // (halves and smaller blocks among them)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;

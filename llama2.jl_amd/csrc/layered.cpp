@@ -62,7 +62,7 @@ struct Layered {
     int cap = 0;
     int64_t rec_floats = 0;
     int32_t *tok = nullptr, *choice = nullptr, *slot_row = nullptr, *slot_of = nullptr, *n_tiles = nullptr, *want = nullptr;
-    GemmTile *tiles = nullptr;
+    GemmTile *tiles = nullptr, *tiles2 = nullptr;  // blocks of the experts' up and down products
     float *X = nullptr, *raw = nullptr, *qkv = nullptr, *kq = nullptr, *beta = nullptr, *lg = nullptr, *gt = nullptr, *ob = nullptr,
           *zb = nullptr, *score = nullptr, *slot_scale = nullptr, *yb = nullptr, *Y = nullptr, *wl = nullptr, *rec = nullptr, *X0 = nullptr, *lat_qa = nullptr,
           *lat_part = nullptr, *kvx = nullptr;
@@ -1114,7 +1114,7 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
             ne = std::max<int64_t>(ne, d.n_experts);
             slots = std::max<int64_t>(slots, d.top);
             up_slots = std::max<int64_t>(up_slots, (int64_t)d.top * L.down.ld);
-            tiles = std::max<int64_t>(tiles, ((int64_t)cap * d.top + L_GEMM_TILE - 1) / L_GEMM_TILE + d.n_experts);
+            tiles = std::max<int64_t>(tiles, tiles_most((int64_t)cap * d.top, d.n_experts, 1));  // (of any blocks)
         }
     }
     if (kvt) DA(l->kvt, kvt);
@@ -1152,7 +1152,8 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
         DA(l->slot_scale, cap * slots);
         DA(l->slot_of, cap * slots);
         DA(l->tiles, tiles);
-        DA(l->n_tiles, 1);
+        DA(l->tiles2, tiles);
+        DA(l->n_tiles, 2);
         DA(l->yb, cap * slots * c.width);
     }
     if (c.side_dim) {
@@ -1326,18 +1327,26 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     CK(k_route(s, d.parallel ? l->raw + L.off_z : l->zb, d.parallel ? L.n_plain : d.n_experts, L.router_bias, M, d.n_experts, d.top, d.route,
                l->choice, l->score));
     const bool image = image_takes(L.up, M) && image_takes(L.down, M);
-    const int rows = image ? L_IMAGE_TILE : L_GEMM_TILE;
-    CK(k_group(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, l->tiles, l->n_tiles, rows));
-    const int slots = M * d.top, max_tiles = (slots + rows - 1) / rows + d.n_experts;
+    const int slots = M * d.top, cu = m->ctx->prop.multiProcessorCount;
     GemmArgs up = gemm_of(L.up, l->xn, slots), down = gemm_of(L.down, l->hb, slots);
-    for (GemmArgs *a : {&up, &down}) {
-        a->tiles = l->tiles;
-        a->n_tiles = l->n_tiles;
-        a->max_tiles = max_tiles;
-        a->rows_each = slots / d.n_experts;
-    }
-    const int epi = d.ff_gated ? GE_GLU : GE_UP;
     up.n_rows = L.up_rows();
+    down.n_rows = l->W();
+    GemmTile *const lists[2] = {l->tiles, l->tiles2};
+    GemmArgs *const products[2] = {&up, &down};
+    unsigned bound[2];
+    for (int p = 0; p < 2; p++) {
+        GemmArgs &a = *products[p];
+        a.tiles = image ? lists[p] : l->tiles;
+        a.n_tiles = image ? l->n_tiles + p : l->n_tiles;
+        a.rows_each = slots / d.n_experts;
+        bound[p] = tiles_bound(slots, d.n_experts, (unsigned)((a.n_rows + 255) / 256), (unsigned)a.ld >> 6, (unsigned)cu);
+        a.max_tiles = image ? (int)tiles_most(slots, d.n_experts, bound[p]) : (slots + L_GEMM_TILE - 1) / L_GEMM_TILE + d.n_experts;
+    }
+    if (image)
+        CK(k_group_images(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, lists, l->n_tiles, bound));
+    else
+        CK(k_group(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, l->tiles, l->n_tiles, L_GEMM_TILE));
+    const int epi = d.ff_gated ? GE_GLU : GE_UP;
     up.expert_stride = (int64_t)L.up_rows() * L.up.ld;
     up.gather = l->slot_row;
     up.row_scale = l->slot_scale;
@@ -1348,18 +1357,17 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     if (image) {
         up.w = L.up.image;
         up.expert_stride = L.up.image_stride;
-        CK(k_tiles(s, up, epi, m->ctx->prop.multiProcessorCount));
+        CK(k_tiles(s, up, epi, cu));
     } else {
         CK(k_gemm(s, up, prec, epi));
     }
-    down.n_rows = l->W();
     down.expert_stride = (int64_t)l->W() * L.down.ld;
     down.outf = l->yb;
     down.ldo = l->W();
     if (image) {
         down.w = L.down.image;
         down.expert_stride = L.down.image_stride;
-        CK(k_tiles(s, down, GE_STORE, m->ctx->prop.multiProcessorCount));
+        CK(k_tiles(s, down, GE_STORE, cu));
     } else {
         CK(k_gemm(s, down, prec, GE_STORE));
     }

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "l2h_internal.h"
+#include "tiles_plan.h"
 
 struct LMat {
     uint16_t *w = nullptr;
@@ -118,8 +119,7 @@ struct GemmArgs {
     int rows_each = 0;  // rows of a matrix on average
     const int32_t *gather = nullptr;  // row of x for each row of the product
 };
-#define L_GEMM_TILE 128   // rows of a block for k_gemm ...
-#define L_IMAGE_TILE 256  // ... and for k_tiles
+#define L_GEMM_TILE 128  // rows of a block for k_gemm
 hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // The same for few rows or positions (k_few.hip), which k_gemm hands on to where that is the faster way; cols: columns the epilogue
 // covers.  Distinct matrices one after the other:
@@ -167,6 +167,9 @@ hipError_t k_route(hipStream_t s, const float *z, int64_t ldz, const float *bias
                    float *score);
 hipError_t k_group(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                    float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows);
+// with a list of blocks for each of two products from tile images, of at most bound[p] units (tiles_plan.h): tiles[p], n_tiles[p]
+hipError_t k_group_images(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row, float *slot_scale,
+                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const unsigned bound[2]);
 // x[m] += mult * sum_k y[slot_of[m][k]]
 hipError_t k_gather_add(hipStream_t s, float *x, const float *y, const int32_t *slot_of, int M, int top, int K, float mult);
 // x[m] += a[m] + b, a or not

@@ -26,19 +26,19 @@ __host__ __device__ __forceinline__ int pf_swz(int r) { return (r >> 1) & 7; }
 
 // Product of bf16 tiles prepared beforehand (32 KB images of 256 weight rows x 64 inputs, 16-byte chunk c of row r at chunk
 // index 8 r + (c ^ pf_swz(r))): no arithmetic on the operands.  A workgroup's tile is 256 weight rows
-// x 64 JT positions (JT = 4: 256 positions, 64 KB fetched per 64 inputs, half the bytes per product of a 128 x 128 tile; JT = 2: 128 positions, for matrices with too few rows to give
-// every CU a 256 x 256 tile), worked on by 8 wavefronts, 4 row groups x 2 position groups, each 64 rows x
+// x 64 JT positions (JT = 4: 256 positions, 64 KB fetched per 64 inputs, half the bytes per product of a 128 x 128 tile; fewer for matrices with too few rows to give
+// every CU a 256 x 256 tile, and for blocks of a grouped product), worked on by 8 wavefronts, 4 row groups x 2 position groups, each 64 rows x
 // 32 JT positions.  Both operand tiles of a K step travel from global memory
 // straight into LDS (16 bytes per lane and load, a wavefront's load filling 1 KB in lane order): the weight
 // tile is a linear copy of its 32 KB image, the position tile gets the c ^ pf_swz(r) placement by the choice
 // of the address each lane reads.  The loads of step kt + 1 are in flight during the products of step kt, one barrier
-// per step, with two LDS stages of 64 KB; of the 48 KB stages of JT = 2 three fit, and the loads of step kt + 2 are in
+// per step, with two LDS stages of up to 72 KB; of the 48 KB stages of JT = 2 three fit, and the loads of step kt + 2 are in
 // flight too: where such tiles do not fill the chip a step takes as long as its loads (333 positions x 14 336 rows x 4096
 // inputs: 98 us with two stages, 88 with three).
 typedef uint32_t pf_u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int pf_tile_stage(int jt) { return 32768 + 64 * jt * 128; }  // bytes: weight tile, then position tile
-constexpr int pf_tile_stages(int jt) { return jt == 2 ? 3 : 2; }
+constexpr int pf_tile_stages(int jt) { return jt <= 2 ? 3 : 2; }
 constexpr int pf_tile_lds(int jt) { return pf_tile_stages(jt) * pf_tile_stage(jt); }
 
 // wtiles: the row group's tiles, K / 64 of them in a row; act: bf16 rows of K elements; s_all: STAGES * pf_tile_stage(JT) bytes of LDS.  row(r) is the
@@ -60,21 +60,14 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
         const int r = 8 * (JT * wave + i) + (lane >> 3);
         gx[i] = (const unsigned char *)(act + row(r) * K + 8 * ((lane & 7) ^ pf_swz(r)));
     }
-    // LDS byte offsets of this lane's operands inside a stage: slice kk holds chunk 2 kk + lane / 32 of its rows
-    unsigned aw[2][4], ax[JT][4];
+    // LDS byte offsets of this lane's operands inside a stage: slice kk holds chunk 2 kk + lane / 32 of its rows, and 32 rows further on (4096 bytes, an
+    // offset of the read itself) lies the same chunk at the same place of its row
+    unsigned aw[4], ax[4];
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) {
-        const int c = 2 * kk + (lane >> 5);
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int ra = 64 * wn + 32 * i + (lane & 31);
-            aw[i][kk] = 16u * (unsigned)(ra * 8 + (c ^ pf_swz(ra)));
-        }
-#pragma unroll
-        for (int j = 0; j < JT; j++) {
-            const int rb = 32 * JT * wm + 32 * j + (lane & 31);
-            ax[j][kk] = 32768u + 16u * (unsigned)(rb * 8 + (c ^ pf_swz(rb)));
-        }
+        const unsigned at = 128u * (unsigned)(lane & 31) + 16u * (unsigned)((2 * kk + (lane >> 5)) ^ pf_swz(lane & 31));
+        aw[kk] = at + 8192u * (unsigned)wn;
+        ax[kk] = at + 32768u + 4096u * (unsigned)(JT * wm);
     }
     const unsigned lds0 = (unsigned)(size_t)s_all;
 
@@ -109,37 +102,52 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
     // products after the wait (LDS reads complete in order, so lgkmcnt(2 + JT) retires all but the newest set;
     // the build's asm check walks the generated code for any other touch of such a register).
     pf_u32x4 F0[2 + JT], F1[2 + JT];
-#define PF_READ(F, KK)                                                                                            \
-    do {                                                                                                          \
-        if constexpr (JT == 2)                                                                                    \
-            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7"  \
-                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3])                                     \
-                         : "v"(sb + aw[0][KK]), "v"(sb + aw[1][KK]), "v"(sb + ax[0][KK]), "v"(sb + ax[1][KK])     \
-                         : "memory");                                                                             \
-        else                                                                                                      \
-            asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %8\n\tds_read_b128 %3, %9"  \
-                         "\n\tds_read_b128 %4, %10\n\tds_read_b128 %5, %11"                                       \
-                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4]), "=&v"(F[5])           \
-                         : "v"(sb + aw[0][KK]), "v"(sb + aw[1][KK]), "v"(sb + ax[0][KK]), "v"(sb + ax[1][KK]),    \
-                           "v"(sb + ax[JT - 2][KK]), "v"(sb + ax[JT - 1][KK])                                     \
-                         : "memory");                                                                             \
+#define PF_READ(F, KK)                                                                                                                                \
+    do {                                                                                                                                              \
+        if constexpr (JT == 1)                                                                                                                        \
+            asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:4096\n\t"                                                                 \
+                         "ds_read_b128 %2, %4"                                                                                                        \
+                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2])                                                                                      \
+                         : "v"(sb + aw[KK]), "v"(sb + ax[KK])                                                                                         \
+                         : "memory");                                                                                                                 \
+        else if constexpr (JT == 2)                                                                                                                   \
+            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:4096\n\t"                                                                 \
+                         "ds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:4096"                                                                     \
+                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3])                                                                         \
+                         : "v"(sb + aw[KK]), "v"(sb + ax[KK])                                                                                         \
+                         : "memory");                                                                                                                 \
+        else if constexpr (JT == 3)                                                                                                                   \
+            asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %5 offset:4096\n\tds_read_b128 %2, %6\n\t"                                          \
+                         "ds_read_b128 %3, %6 offset:4096\n\tds_read_b128 %4, %6 offset:8192"                                                         \
+                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4])                                                            \
+                         : "v"(sb + aw[KK]), "v"(sb + ax[KK])                                                                                         \
+                         : "memory");                                                                                                                 \
+        else if constexpr (JT == 4)                                                                                                                   \
+            asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:4096\n\tds_read_b128 %2, %7\n\t"                                          \
+                         "ds_read_b128 %3, %7 offset:4096\n\tds_read_b128 %4, %7 offset:8192\n\tds_read_b128 %5, %7 offset:12288"                     \
+                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4]), "=&v"(F[5])                                               \
+                         : "v"(sb + aw[KK]), "v"(sb + ax[KK])                                                                                         \
+                         : "memory");                                                                                                                 \
+        else if constexpr (JT == 5)                                                                                                                   \
+            asm volatile("ds_read_b128 %0, %7\n\tds_read_b128 %1, %7 offset:4096\n\tds_read_b128 %2, %8\n\tds_read_b128 %3, %8 offset:4096\n\t"       \
+                         "ds_read_b128 %4, %8 offset:8192\n\tds_read_b128 %5, %8 offset:12288\n\tds_read_b128 %6, %8 offset:16384"                    \
+                         : "=&v"(F[0]), "=&v"(F[1]), "=&v"(F[2]), "=&v"(F[3]), "=&v"(F[4]), "=&v"(F[5]), "=&v"(F[6])                                  \
+                         : "v"(sb + aw[KK]), "v"(sb + ax[KK])                                                                                         \
+                         : "memory");                                                                                                                 \
     } while (0)
     // LAST: nothing newer is in flight
-#define PF_WAIT(F, LAST)                                                                                          \
-    do {                                                                                                          \
-        if constexpr (JT == 2) {                                                                                  \
-            if (LAST)                                                                                             \
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3])::"memory");  \
-            else                                                                                                  \
-                asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3])::"memory");  \
-        } else {                                                                                                  \
-            if (LAST)                                                                                             \
-                asm volatile("s_waitcnt lgkmcnt(0)"                                                               \
-                             : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[JT]), "+v"(F[JT + 1])::"memory"); \
-            else                                                                                                  \
-                asm volatile("s_waitcnt lgkmcnt(6)"                                                               \
-                             : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[JT]), "+v"(F[JT + 1])::"memory"); \
-        }                                                                                                         \
+#define PF_WAIT(F, LAST)                                                                                                                              \
+    do {                                                                                                                                              \
+        if constexpr (JT == 1)                                                                                                                        \
+            asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]) : "n"((LAST) ? 0 : 2 + JT) : "memory");                         \
+        else if constexpr (JT == 2)                                                                                                                   \
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]) : "n"((LAST) ? 0 : 2 + JT) : "memory");             \
+        else if constexpr (JT == 3)                                                                                                                   \
+            asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]) : "n"((LAST) ? 0 : 2 + JT) : "memory"); \
+        else if constexpr (JT == 4)                                                                                                                   \
+            asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]), "+v"(F[5]) : "n"((LAST) ? 0 : 2 + JT) : "memory");\
+        else if constexpr (JT == 5)                                                                                                                   \
+            asm volatile("s_waitcnt lgkmcnt(%7)" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]), "+v"(F[5]), "+v"(F[6]) : "n"((LAST) ? 0 : 2 + JT) : "memory");\
     } while (0)
 #define PF_PRODUCTS(F)                                                                                            \
     do {                                                                                                          \
@@ -159,21 +167,24 @@ __device__ __forceinline__ void pf_tile_product(const uint16_t *wtiles, const ui
     // barrier between the slices of two stages, 439 like this.)
     constexpr int AHEAD = STAGES - 1;  // stages under way
     // this wavefront's loads of the oldest stage under way have landed (NEWER: those of another one may be under way)
-#define PF_LANDED(NEWER)                                       \
-    do {                                                       \
-        if (NEWER)                                             \
-            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");   \
-        else                                                   \
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   \
-        __builtin_amdgcn_s_barrier();                          \
+#define PF_LANDED(NEWER)                                                                  \
+    do {                                                                                  \
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NEWER) ? 4 + JT : 0) : "memory");       \
+        __builtin_amdgcn_s_barrier();                                                     \
     } while (0)
     // (the products of F are not to move in front of what stands before this)
-#define PF_HERE(F)                                                                                                       \
-    do {                                                                                                                 \
-        if constexpr (JT == 2)                                                                                           \
-            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]));                                           \
-        else                                                                                                             \
-            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[JT]), "+v"(F[JT + 1]));             \
+#define PF_HERE(F)                                                                                                                \
+    do {                                                                                                                          \
+        if constexpr (JT == 1)                                                                                                    \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]));                                                                \
+        else if constexpr (JT == 2)                                                                                               \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]));                                                    \
+        else if constexpr (JT == 3)                                                                                               \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]));                                        \
+        else if constexpr (JT == 4)                                                                                               \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]), "+v"(F[5]));                            \
+        else if constexpr (JT == 5)                                                                                               \
+            asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]), "+v"(F[5]), "+v"(F[6]));                \
     } while (0)
     int stage = 0;
     unsigned sb = lds0;

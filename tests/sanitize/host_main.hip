@@ -349,6 +349,36 @@ static void check_tiles_plan() {
             }
         EXPECT(n_cu != 256 || split == 7 * 128);
     }
+    // an expert's blocks have all of its units once, in shares that differ by one at most and are within the bound; all blocks fit the lists and grids
+    for (unsigned b = 1; b <= TILES_MAX_UNITS; b++) {
+        for (unsigned units = 0; units <= 400; units++) {
+            const TilesSplit v = tiles_split(units, b);
+            EXPECT(v.blocks == (units + b - 1) / b && v.largest <= b);
+            unsigned at = 0, weight = 0;
+            const TilesShares share(units, v.blocks);
+            for (unsigned k = 0; k < v.blocks; k++) {
+                const unsigned u = share.at(k + 1) - at;
+                EXPECT(share.at(k) == at && u >= 1 && u <= v.largest && u + 1 >= v.largest);
+                at += u;
+                weight += tiles_weight(u);
+            }
+            EXPECT(at == units && weight == v.weight);
+        }
+        unsigned seed = 7 * b;
+        for (int experts : {1, 2, 7, 64, 300}) {
+            int64_t rows = 0, blocks = 0;
+            for (int e = 0; e < experts; e++) {
+                seed = seed * 1664525u + 1013904223u;
+                const int64_t n = e % 3 == 0 ? 1 : (seed >> 20) % 700;
+                rows += n;
+                blocks += tiles_split((unsigned)((n + TILES_UNIT - 1) / TILES_UNIT), b).blocks;
+            }
+            EXPECT(blocks <= tiles_most(rows, experts, b) && tiles_most(rows, experts, b) <= tiles_most(rows, experts, 1));
+        }
+    }
+    // what the rule was made from: the bound of the least time at each (rows, experts, row groups, steps)
+    EXPECT(tiles_bound(8192, 32, 4, 32, 256) == 3 && tiles_bound(8192, 32, 8, 16, 256) == 5 && tiles_bound(8192, 32, 16, 64, 256) == 5);
+    EXPECT(tiles_bound(1332, 16, 8, 64, 256) == 1 && tiles_bound(1332, 16, 16, 32, 256) == 2 && tiles_bound(8000, 16, 8, 32, 256) == 5);
     // a grouped product's grid is made for the most tiles there can be, and dealt out by how many there are
     for (unsigned most = 1; most <= 300; most++)
         for (unsigned n = 1; n <= most; n++) {
