@@ -7,6 +7,7 @@
 // in the KV cache and the last position's logits, to bf16 accuracy.
 #include "matvec_dev.h"
 #include "pf_tile.h"
+#include "tiles_plan.h"
 
 
 // ------------------------------------------------------------------------------------------
@@ -498,11 +499,10 @@ __global__ __launch_bounds__(256) void pf_gemm_kernel(PfGemmArgs a) {
 // the 8 XCDs in turn, so workgroup w takes tile (w % 8) * per + w / 8: each XCD works through a contiguous run of tiles,
 // positions fastest, and the workgroups that share a weight tile share an L2.
 
-// the tile (row group nt, position block mt) of one workgroup
+// the tile (row group nt, 64 JT positions from m0) of one workgroup
 template <int EPI, int JT>
-__device__ __forceinline__ void pf_gemm_bf16_tile(const PfGemmArgs &a, unsigned nt, unsigned mt, uint4 *s_all) {
+__device__ __forceinline__ void pf_gemm_bf16_tile(const PfGemmArgs &a, unsigned nt, int m0, uint4 *s_all) {
     const int64_t n0 = (int64_t)nt * 256;
-    const int m0 = (int)mt * 64 * JT;
     pf_tile_product<JT>(
         a.wbf + (int64_t)nt * (a.K >> 6) * 16384, a.act, a.K, s_all,
         [&](int r) { return (int64_t)min(m0 + r, a.M - 1); },  // rows past the end repeat the last one; their results are not stored
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(512) void pf_gemm_bf16_kernel(PfGemmArgs a, unsigne
     extern __shared__ uint4 s_all[];
     const unsigned tile = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
     if (tile >= n_tiles) return;
-    pf_gemm_bf16_tile<EPI, JT>(a, nt0 + tile / n_mt, tile % n_mt, s_all);
+    pf_gemm_bf16_tile<EPI, JT>(a, nt0 + tile / n_mt, (int)(tile % n_mt) * 64 * JT, s_all);
 }
 
 // One round of the CUs over a matrix that would need between one and two rounds of 256 x 128 tiles: the
@@ -532,12 +532,31 @@ __global__ __launch_bounds__(512) void pf_gemm_bf16_mixed_kernel(PfGemmArgs a, u
     if (k < per4) {
         const unsigned tile = xcd * per4 + k;
         if (tile >= n_tiles4) return;
-        pf_gemm_bf16_tile<EPI, 4>(a, tile / n_mt4, tile % n_mt4, s_all);
+        pf_gemm_bf16_tile<EPI, 4>(a, tile / n_mt4, (int)(tile % n_mt4) * 256, s_all);
     } else {
         const unsigned tile = xcd * per2 + (k - per4);
         if (tile >= n_tiles2) return;
-        pf_gemm_bf16_tile<EPI, 2>(a, nt4 + tile / n_mt2, tile % n_mt2, s_all);
+        pf_gemm_bf16_tile<EPI, 2>(a, nt4 + tile / n_mt2, (int)(tile % n_mt2) * 128, s_all);
     }
+}
+
+// The positions in equal shares of one to five units of 64 (tiles_plan.h): between the sizes that whole rounds of 256 x 256 tiles fit.
+template <int EPI>
+__global__ __launch_bounds__(512) void pf_gemm_bf16_shares_kernel(PfGemmArgs a, unsigned blocks, unsigned n_items) {
+    extern __shared__ uint4 s_all[];
+    const TilesBlock k = tiles_block((unsigned)(a.M + TILES_UNIT - 1) / TILES_UNIT, blocks, n_items, blockIdx.x);
+    if (!k.any) return;
+    const int m0 = (int)k.at * TILES_UNIT;
+    if (k.units == 5)
+        pf_gemm_bf16_tile<EPI, 5>(a, k.nt, m0, s_all);
+    else if (k.units == 4)
+        pf_gemm_bf16_tile<EPI, 4>(a, k.nt, m0, s_all);
+    else if (k.units == 3)
+        pf_gemm_bf16_tile<EPI, 3>(a, k.nt, m0, s_all);
+    else if (k.units == 2)
+        pf_gemm_bf16_tile<EPI, 2>(a, k.nt, m0, s_all);
+    else
+        pf_gemm_bf16_tile<EPI, 1>(a, k.nt, m0, s_all);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1022,35 +1041,63 @@ hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave
 #undef GO
             return hipGetLastError();
         };
-        const unsigned n_mt2 = (unsigned)((M + 127) / 128);
-        if (nt4 == 0 && n_nt * n_mt2 > 256 && n_mt2 > n_mt4) {
+        const unsigned n_mt2 = (unsigned)((M + 127) / 128), units = (unsigned)((M + TILES_UNIT - 1) / TILES_UNIT), steps = (unsigned)(K >> 6);
+        const bool between = nt4 == 0 && n_nt * n_mt2 > 256 && n_mt2 > n_mt4;
+        const unsigned na = between ? (n_nt * n_mt2 - 256 + (n_mt2 - n_mt4) - 1) / (n_mt2 - n_mt4) : 0;
+        const bool mixed = between && na <= n_nt;
+        // The estimated time of that, or of one round of both, against all positions in equal shares.  us, that and shares, 64 / 333 / 640 / 1000 / 1500 / 2048 positions: 28 672
+        // rows x 4096 inputs 49 / 101 / 157 / 218 / 314 / 374 and 38 / 76 / 119 / 200 / 300 / 391; 16 384 x 3072 38 / 44 / 79 / 83 / 163 / 164 and 26 / 46 / 62 / 83 / 123 / 164;
+        // 2752 x 512 13 / 15 / 15 / 16 / 16 / 16 and 9 / 10 / 10 / 10 / 16 / 17.
+        const unsigned bound = tiles_dense_bound(units, n_nt, steps, 256), rest = (n_nt - nt4) * n_mt2;
+        const float time = mixed ? tiles_cost(4, steps) : (float)((nt4 * n_mt4 + 255) / 256) * tiles_cost(4, steps) + (float)((rest + 255) / 256) * tiles_cost(2, steps);
+        if (tiles_dense_time(units, bound, n_nt, steps, 256) < time) {
+            const unsigned blocks = tiles_blocks(units, bound), n_items = n_nt * blocks;
+            const size_t lds = (size_t)std::max(pf_tile_lds(2), pf_tile_lds(5));
+#define GO(E)                                                                                                       \
+    do {                                                                                                            \
+        static bool attr_set[PF_MAX_DEVICES] = {};                                                                  \
+        if (!attr_set[dev]) {                                                                                       \
+            const hipError_t e = hipFuncSetAttribute((const void *)pf_gemm_bf16_shares_kernel<E>,                   \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
+            if (e != hipSuccess) return e;                                                                          \
+            attr_set[dev] = true;                                                                                   \
+        }                                                                                                           \
+        hipLaunchKernelGGL((pf_gemm_bf16_shares_kernel<E>), dim3(tiles_workgroups(n_items)), dim3(512), lds, s, a, blocks, n_items); \
+    } while (0)
+            switch (epi) {
+            case PF_STORE: GO(PF_STORE); break;
+            case PF_RESID: GO(PF_RESID); break;
+            case PF_SWIGLU: GO(PF_SWIGLU); break;
+            default: return hipErrorInvalidValue;
+            }
+#undef GO
+            return hipGetLastError();
+        }
+        if (mixed) {
             // more than one round of 256 x 128 tiles, less than one of 256 x 256: mix the two so that the work
             // fits one round, na row groups in large tiles
-            const unsigned na = (n_nt * n_mt2 - 256 + (n_mt2 - n_mt4) - 1) / (n_mt2 - n_mt4);
-            if (na <= n_nt) {
-                const unsigned t4 = na * n_mt4, t2 = (n_nt - na) * n_mt2, per4 = (t4 + 7) / 8, per2 = (t2 + 7) / 8;
-                const dim3 grid(8 * (per4 + per2));
-                const size_t lds = (size_t)std::max(pf_tile_lds(4), pf_tile_lds(2));
+            const unsigned t4 = na * n_mt4, t2 = (n_nt - na) * n_mt2, per4 = (t4 + 7) / 8, per2 = (t2 + 7) / 8;
+            const dim3 grid(8 * (per4 + per2));
+            const size_t lds = (size_t)std::max(pf_tile_lds(4), pf_tile_lds(2));
 #define GO(E)                                                                                                       \
     do {                                                                                                            \
         static bool attr_set[PF_MAX_DEVICES] = {};                                                                  \
         if (!attr_set[dev]) {                                                                                       \
             const hipError_t e = hipFuncSetAttribute((const void *)pf_gemm_bf16_mixed_kernel<E>,                    \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
             if (e != hipSuccess) return e;                                                                          \
             attr_set[dev] = true;                                                                                   \
         }                                                                                                           \
         hipLaunchKernelGGL((pf_gemm_bf16_mixed_kernel<E>), grid, dim3(512), lds, s, a, na, n_mt4, n_mt2, t4, t2, per4, per2); \
     } while (0)
-                switch (epi) {
-                case PF_STORE: GO(PF_STORE); break;
-                case PF_RESID: GO(PF_RESID); break;
-                case PF_SWIGLU: GO(PF_SWIGLU); break;
-                default: return hipErrorInvalidValue;
-                }
-#undef GO
-                return hipGetLastError();
+            switch (epi) {
+            case PF_STORE: GO(PF_STORE); break;
+            case PF_RESID: GO(PF_RESID); break;
+            case PF_SWIGLU: GO(PF_SWIGLU); break;
+            default: return hipErrorInvalidValue;
             }
+#undef GO
+            return hipGetLastError();
         }
         if (nt4 > 0) {
             const hipError_t e = launch(4, 0, nt4);

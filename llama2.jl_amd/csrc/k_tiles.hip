@@ -43,76 +43,79 @@ __device__ __forceinline__ void tiles_item(const GemmArgs &a, const uint16_t *w,
         });
 }
 
-// Items (row group of 256, block of 64 JT positions) are dealt to the 8 XCDs as contiguous runs: positions fastest in a single
+// a block of up to five units of 64 positions
+template <int EPI>
+__device__ __forceinline__ void tiles_units(const GemmArgs &a, const uint16_t *w, unsigned nt, int64_t mb, int m0, int mcount, unsigned units, uint4 *s_all) {
+    if (units == 5)
+        tiles_item<EPI, 5, pf_tile_stages(5)>(a, w, nt, mb, m0, mcount, s_all);
+    else if (units == 4)
+        tiles_item<EPI, 4, pf_tile_stages(4)>(a, w, nt, mb, m0, mcount, s_all);
+    else if (units == 3)
+        tiles_item<EPI, 3, pf_tile_stages(3)>(a, w, nt, mb, m0, mcount, s_all);
+    else if (units == 2)
+        tiles_item<EPI, 2, pf_tile_stages(2)>(a, w, nt, mb, m0, mcount, s_all);
+    else
+        tiles_item<EPI, 1, pf_tile_stages(1)>(a, w, nt, mb, m0, mcount, s_all);
+}
+
+// Items (row group of 256, block of positions) are dealt to the 8 XCDs as contiguous runs: positions fastest in a single
 // product, so that workgroups on one weight tile share an L2; row groups fastest in a grouped one, where a block of positions
-// is used with one expert's matrix only.  Of a single product of JT = 4 the last items may go as halves (tiles_plan).
-template <int EPI, int JT, bool GROUPED>
+// is used with one expert's matrix only.
+// WHOLE: blocks of 256 positions of a single product, the last items as halves where that pays (tiles_plan); SHARES: its positions in equal shares of up to
+// five units; GROUPED: the blocks that a.tiles lists.
+enum { TILES_WHOLE = 0, TILES_SHARES = 1, TILES_GROUPED = 2 };
+template <int EPI, int MODE>
 __global__ __launch_bounds__(512) void tiles_kernel(GemmArgs a, unsigned n_nt, unsigned n_mt, TilesPlan plan) {
     extern __shared__ uint4 s_all[];
-    unsigned item;
-    if (!GROUPED && JT == 4) {
+    if constexpr (MODE == TILES_WHOLE) {
         const TilesWork work = tiles_work(plan, blockIdx.x);
         if (!work.any) return;
-        if (work.half >= 0) {
-            const int m0 = (int)(work.item % n_mt) * 256 + 128 * work.half;
-            if (m0 < a.M) tiles_item<EPI, 2, pf_tile_stages(2)>(a, a.w, work.item / n_mt, 0, m0, a.M, s_all);
-            return;
-        }
-        item = work.item;
+        const int m0 = (int)(work.item % n_mt) * 256;
+        if (work.half < 0)
+            tiles_item<EPI, 4, pf_tile_stages(4)>(a, a.w, work.item / n_mt, 0, m0, a.M, s_all);
+        else if (m0 + 128 * work.half < a.M)
+            tiles_item<EPI, 2, pf_tile_stages(2)>(a, a.w, work.item / n_mt, 0, m0 + 128 * work.half, a.M, s_all);
+    } else if constexpr (MODE == TILES_SHARES) {
+        const TilesBlock k = tiles_block((unsigned)(a.M + TILES_UNIT - 1) / TILES_UNIT, n_mt, plan.n, blockIdx.x);
+        if (k.any) tiles_units<EPI>(a, a.w, k.nt, 0, (int)k.at * TILES_UNIT, a.M, k.units, s_all);
     } else {
-        const unsigned n_items = GROUPED ? (unsigned)a.n_tiles[0] * n_nt : plan.n;
-        item = tiles_deal(n_items, blockIdx.x);
+        const unsigned n_items = (unsigned)a.n_tiles[0] * n_nt, item = tiles_deal(n_items, blockIdx.x);
         if (item >= n_items) return;
-    }
-    unsigned nt;
-    int64_t mb = 0;
-    int m0 = 0, mcount = a.M;
-    const uint16_t *w = a.w;
-    if (GROUPED) {
         const GemmTile g = a.tiles[item / n_nt];
-        nt = item % n_nt;
-        w += g.expert * a.expert_stride;
-        mb = g.row0;
-        mcount = g.n;
-    } else {
-        nt = item / n_mt;
-        m0 = (int)(item % n_mt) * 64 * JT;
-    }
-    if constexpr (GROUPED) {
-        const int units = (mcount + 63) >> 6;
-        if (units == 5)
-            tiles_item<EPI, 5, pf_tile_stages(5)>(a, w, nt, mb, m0, mcount, s_all);
-        else if (units == 4)
-            tiles_item<EPI, 4, pf_tile_stages(4)>(a, w, nt, mb, m0, mcount, s_all);
-        else if (units == 3)
-            tiles_item<EPI, 3, pf_tile_stages(3)>(a, w, nt, mb, m0, mcount, s_all);
-        else if (units == 2)
-            tiles_item<EPI, 2, pf_tile_stages(2)>(a, w, nt, mb, m0, mcount, s_all);
-        else
-            tiles_item<EPI, 1, pf_tile_stages(1)>(a, w, nt, mb, m0, mcount, s_all);
-    } else {
-        tiles_item<EPI, JT, pf_tile_stages(JT)>(a, w, nt, mb, m0, mcount, s_all);
+        tiles_units<EPI>(a, a.w + g.expert * a.expert_stride, item % n_nt, g.row0, 0, g.n, (unsigned)(g.n + TILES_UNIT - 1) / TILES_UNIT, s_all);
     }
 }
 
 #define TILES_MAX_DEVICES 64
 
-template <int EPI, int JT, bool GROUPED>
-static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, unsigned n_mt, int n_cu) {
-    constexpr int lds = std::max(pf_tile_lds(2), pf_tile_lds(GROUPED ? 5 : JT));  // (halves and smaller blocks among them)
+// n: tiles or items, n_mt: blocks of positions to a row group
+template <int EPI, int MODE>
+static hipError_t tiles_launch(hipStream_t s, const GemmArgs &a, unsigned n_nt, unsigned n_mt, const TilesPlan &plan) {
+    constexpr int lds = std::max(pf_tile_lds(2), pf_tile_lds(MODE == TILES_WHOLE ? 4 : TILES_MAX_UNITS));  // (halves and smaller blocks among them)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= TILES_MAX_DEVICES) return hipErrorInvalidDevice;
     static bool attr_set[TILES_MAX_DEVICES] = {};
     if (!attr_set[dev]) {
-        e = hipFuncSetAttribute((const void *)tiles_kernel<EPI, JT, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        e = hipFuncSetAttribute((const void *)tiles_kernel<EPI, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
         attr_set[dev] = true;
     }
-    const TilesPlan plan = tiles_plan(GROUPED ? (unsigned)a.max_tiles * n_nt : n_nt * n_mt, !GROUPED && JT == 4, n_cu);
-    hipLaunchKernelGGL((tiles_kernel<EPI, JT, GROUPED>), dim3(tiles_grid(plan)), dim3(512), lds, s, a, n_nt, n_mt, plan);
+    hipLaunchKernelGGL((tiles_kernel<EPI, MODE>), dim3(tiles_grid(plan)), dim3(512), lds, s, a, n_nt, n_mt, plan);
     return hipGetLastError();
+}
+// A single product: whole tiles and halves, or shares, whichever are likely through first.  us, whole tiles (of 128 positions where those are fewer than the compute
+// units) and shares, 130 / 333 / 640 / 1300 / 2048 positions: 8192 rows x 2048 inputs 36 / 37 / 40 / 76 / 81 and 22 / 24 / 40 / 58 / 81; gated 28 672 x 4096 73 / 118 / 176 /
+// 336 / 427 and 73 / 88 / 141 / 322 / 450; 4096 x 1024 25 / 25 / 26 / 28 / 31 and 15 / 16 / 17 / 28 / 31.
+template <int EPI>
+static hipError_t tiles_single(hipStream_t s, const GemmArgs &a, unsigned n_nt, int n_cu) {
+    const unsigned n_mt = (unsigned)((a.M + 255) / 256), units = (unsigned)((a.M + TILES_UNIT - 1) / TILES_UNIT), steps = (unsigned)a.ld >> 6, cu = (unsigned)n_cu;
+    const TilesPlan plan = tiles_plan(n_nt * n_mt, true, n_cu);
+    const unsigned b = tiles_dense_bound(units, n_nt, steps, cu);
+    if (tiles_whole_time(plan, steps, cu) <= tiles_dense_time(units, b, n_nt, steps, cu)) return tiles_launch<EPI, TILES_WHOLE>(s, a, n_nt, n_mt, plan);
+    const unsigned blocks = tiles_blocks(units, b);
+    return tiles_launch<EPI, TILES_SHARES>(s, a, n_nt, blocks, tiles_plan(n_nt * blocks, false, n_cu));
 }
 
 // a.w: the image; otherwise as k_gemm with bf16 activations (ldx == ld)
@@ -126,15 +129,13 @@ hipError_t k_tiles(hipStream_t s, const GemmArgs &args, int epi, int n_cu) {
     const bool covered = a.outa && a.acols >= a.n_rows && a.acols <= 256 * (int64_t)n_nt;
     const bool pairs = a.outa && a.n_rows % 2 == 0 && 2 * a.acols >= a.n_rows && 2 * a.acols <= 256 * (int64_t)n_nt;
     if (a.tiles) {
-        if (epi == GE_UP && covered) return tiles_launch<GE_UP, 4, true>(s, a, n_nt, 0, n_cu);
-        if (epi == GE_GLU && pairs) return tiles_launch<GE_GLU, 4, true>(s, a, n_nt, 0, n_cu);
-        if (epi == GE_STORE && a.outf && a.ldo >= a.n_rows) return tiles_launch<GE_STORE, 4, true>(s, a, n_nt, 0, n_cu);
+        const TilesPlan plan = tiles_plan((unsigned)a.max_tiles * n_nt, false, n_cu);
+        if (epi == GE_UP && covered) return tiles_launch<GE_UP, TILES_GROUPED>(s, a, n_nt, 0, plan);
+        if (epi == GE_GLU && pairs) return tiles_launch<GE_GLU, TILES_GROUPED>(s, a, n_nt, 0, plan);
+        if (epi == GE_STORE && a.outf && a.ldo >= a.n_rows) return tiles_launch<GE_STORE, TILES_GROUPED>(s, a, n_nt, 0, plan);
         return hipErrorInvalidValue;
     }
-    if (!(epi == GE_ACT && covered) && !(epi == GE_GLU && pairs)) return hipErrorInvalidValue;
-    const unsigned n_mt4 = (unsigned)((a.M + 255) / 256), n_mt2 = (unsigned)((a.M + 127) / 128);
-    if (epi == GE_GLU)
-        return n_nt * n_mt4 >= 256 ? tiles_launch<GE_GLU, 4, false>(s, a, n_nt, n_mt4, n_cu) : tiles_launch<GE_GLU, 2, false>(s, a, n_nt, n_mt2, n_cu);
-    if (n_nt * n_mt4 >= 256) return tiles_launch<GE_ACT, 4, false>(s, a, n_nt, n_mt4, n_cu);
-    return tiles_launch<GE_ACT, 2, false>(s, a, n_nt, n_mt2, n_cu);
+    if (epi == GE_ACT && covered) return tiles_single<GE_ACT>(s, a, n_nt, n_cu);
+    if (epi == GE_GLU && pairs) return tiles_single<GE_GLU>(s, a, n_nt, n_cu);
+    return hipErrorInvalidValue;
 }

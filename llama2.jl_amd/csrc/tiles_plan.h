@@ -105,3 +105,33 @@ inline unsigned tiles_bound(int64_t rows, int experts, unsigned n_nt, unsigned s
 inline int64_t tiles_most(int64_t rows, int experts, unsigned b) {
     return ((rows + TILES_UNIT - 1) / TILES_UNIT + experts) / b + experts;
 }
+
+// A single product's positions in the same kind of blocks, every row group's alike: the bound for them and what they may take
+inline float tiles_cost(unsigned units, unsigned steps) { return 180.0f + (float)(steps * tiles_weight(units)); }
+// (whole tiles of 256 positions, and their rest as halves)
+inline float tiles_whole_time(const TilesPlan &p, unsigned steps, unsigned n_cu) {
+    return (float)((p.whole + n_cu - 1) / n_cu) * tiles_cost(4, steps) + (p.whole < p.n ? tiles_cost(2, steps) : 0.0f);
+}
+inline float tiles_dense_time(unsigned units, unsigned b, unsigned n_nt, unsigned steps, unsigned n_cu) {
+    const TilesSplit v = tiles_split(units, b);
+    const float rounds = (float)((v.blocks * n_nt + n_cu - 1) / n_cu), sum = rounds * (180.0f + (float)steps * (float)v.weight / (float)v.blocks);
+    return std::max(sum, tiles_cost(v.largest, steps));
+}
+inline unsigned tiles_dense_bound(unsigned units, unsigned n_nt, unsigned steps, unsigned n_cu) {
+    unsigned best = 1;
+    for (unsigned b = 2; b <= TILES_MAX_UNITS; b++)
+        if (tiles_dense_time(units, b, n_nt, steps, n_cu) <= tiles_dense_time(units, best, n_nt, steps, n_cu)) best = b;
+    return best;
+}
+// block k of `blocks` of a row group's units, item = row group * blocks + k of a grid of tiles_workgroups(items)
+struct TilesBlock {
+    bool any;
+    unsigned nt, at, units;  // at: in units
+};
+__host__ __device__ inline TilesBlock tiles_block(unsigned units, unsigned blocks, unsigned items, unsigned workgroup) {
+    const unsigned item = tiles_deal(items, workgroup);
+    if (item >= items) return {false, 0, 0, 0};
+    const unsigned nt = item / blocks, k = item - nt * blocks;
+    const TilesShares s(units, blocks);
+    return {true, nt, s.at(k), s.at(k + 1) - s.at(k)};
+}
