@@ -241,6 +241,26 @@ class BoxGuard {
     bool waited = false;
 };
 
+// Words between the device and the model's box: one launch for all runs where kernels see the box, a copy each otherwise.  (A drawn token of the smallest model, its
+// step and the draw, 117 us with copies and a launch for the pick, 105 like this; of a layered one of width 768 162 and 147, a third of that the step's own.)
+static hipError_t hand_over(l2h_model *m, const WordCopies &c) {
+    if (m->box.seen) return k_words(m->ctx->stream, c);
+    for (const WordCopy &w : c.run)
+        if (w.n > 0) {
+            const hipError_t e = hipMemcpyAsync(w.to, w.from, (size_t)w.n * 4, hipMemcpyDefault, m->ctx->stream);
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
+}
+static WordCopy words(const void *from, void *to, int64_t n) {
+    WordCopy w;
+    w.from = (const uint32_t *)from;
+    w.to = (uint32_t *)to;
+    w.n = n;
+    return w;
+}
+#define CTL_WORDS ((int64_t)(sizeof(DecodeCtl) / 4))
+
 static int q8_alloc(l2h_ctx *ctx, int64_t n, Q8Dev *q, std::vector<void *> *track) {
     void *p = nullptr;
     const int64_t o_bs = align256(n), o_d = o_bs + align256(n / 8 + 16);
@@ -1195,11 +1215,10 @@ static int last_token(l2h_model *m, int n) {
 }
 
 // after the stream has drained: did a workgroup of the persistent kernel give up at a barrier?
-// (mega_ask is requested behind the launches, mega_check reads the answer once the stream has drained)
-static int mega_ask(l2h_model *m) {
+// (mega_flag is handed over behind the launches, mega_check reads the answer once the stream has drained)
+static WordCopy mega_flag(l2h_model *m) {
     const void *flag = m->flow ? (const void *)m->flow_args.abort_flag : m->mega ? (const void *)&m->bar->abort : nullptr;
-    if (flag) HIPCHK(m->ctx, hipMemcpyAsync(m->box.gave_up, flag, 4, hipMemcpyDeviceToHost, m->ctx->stream));
-    return L2H_OK;
+    return words(flag, m->box.gave_up, flag ? 1 : 0);
 }
 static int mega_check(l2h_model *m) {
     if (m->flow) {
@@ -1311,7 +1330,7 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     BoxGuard guard(m);
     m->box.ctl[0] = m->box.ctl[1] = h;
     memcpy(m->box.prompt, prompt, (size_t)n_prompt * 4);
-    HIPCHK(ctx, hipMemcpyAsync(m->ctl, m->box.ctl, 2 * sizeof h + (size_t)n_prompt * 4, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(ctx, hand_over(m, {{words(m->box.ctl, m->ctl, 2 * CTL_WORDS + n_prompt)}}));
     if (m->lay && total > 0) layered_advance(m, pos0 + total);
     DeviceTurn turn(m);
     if (decode_ms) {
@@ -1333,8 +1352,7 @@ static int generate_once(l2h_model *m, const int32_t *prompt, int n_prompt, int 
     } else {
         if ((rc = run_steps(m, total)) || (rc = last_token(m, total))) return rc;
     }
-    if (n_new > 0) HIPCHK(ctx, hipMemcpyAsync(m->box.out, m->out_tokens, (size_t)n_new * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if ((rc = mega_ask(m))) return rc;
+    HIPCHK(ctx, hand_over(m, {{words(m->out_tokens, m->box.out, n_new), mega_flag(m)}}));
     if (last_logits)
         HIPCHK(ctx, hipMemcpyAsync(last_logits, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost,
                                    ctx->stream));
@@ -1557,7 +1575,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
         float *wl = want_logits ? want_logits + (int64_t)w0 * m->c.vocab_size : nullptr;
         w0 += (int)rows.size();
         if (m->lay) {
-            HIPCHK(ctx, hipMemcpyAsync(layered_token_buffer(m), m->box.prompt + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
+            HIPCHK(ctx, hand_over(m, {{words(m->box.prompt + c0, layered_token_buffer(m), M)}}));
             const hipError_t e = layered_prefill_chunk(m, M, pos0 + c0);
             if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "prompt pass launch failed: %s", hipGetErrorString(e));
             layered_advance(m, pos0 + c0 + M);
@@ -1583,7 +1601,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
                 if ((rc = prefill_expand(m, false))) return rc;
             }
         }
-        HIPCHK(ctx, hipMemcpyAsync(m->pf_tok, m->box.prompt + c0, (size_t)M * 4, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(ctx, hand_over(m, {{words(m->box.prompt + c0, m->pf_tok, M)}}));
         hipError_t e = prefill_chunk(m, M, pos0 + c0);
         if (e != hipSuccess)
             return set_err(ctx, L2H_EHIP, "prompt pass launch failed: %s%s%s", hipGetErrorString(e),
@@ -1602,20 +1620,19 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
     }
     // last position: its hidden state becomes the decode state; classifier and argmax as in a decode step
     m->flow_holds_state = false;
-    if (!m->lay)
-        HIPCHK(ctx, hipMemcpyAsync(m->x, m->pf_x + (int64_t)(M - 1) * m->c.dim, (size_t)m->c.dim * 4,
-                                   hipMemcpyDeviceToDevice, ctx->stream));
     DecodeCtl h{};
     h.token = tokens[n - 1];
     h.pos = pos0 + n - 1;
     h.n_prompt = 1;
     m->box.ctl[0] = h;
-    HIPCHK(ctx, hipMemcpyAsync(m->ctl, m->box.ctl, sizeof h, hipMemcpyHostToDevice, ctx->stream));
+    WordCopy x;
+    if (!m->lay) x = words(m->pf_x + (int64_t)(M - 1) * m->c.dim, m->x, m->c.dim);
+    HIPCHK(ctx, hand_over(m, {{words(m->box.ctl, m->ctl, CTL_WORDS), x}}));
     hipError_t e = m->lay ? layered_output(m) : launch_output(m);
     if (e == hipSuccess)
         e = k_argmax(ctx->stream, m->logits, m->c.vocab_size, m->argmax_partial, m->ctl, m->out_tokens, m->max_out, false);
     if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "classifier launch failed: %s", hipGetErrorString(e));
-    if (next_token) HIPCHK(ctx, hipMemcpyAsync(m->box.out, m->out_tokens, 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (next_token) HIPCHK(ctx, hand_over(m, {{words(m->out_tokens, m->box.out, 1)}}));
     if (last_logits)
         HIPCHK(ctx, hipMemcpyAsync(last_logits, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost,
                                    ctx->stream));
@@ -1663,13 +1680,14 @@ extern "C" int l2h_sample(l2h_model *m, float temperature, float u, int32_t *tok
     if (!m->sample_p) {
         int rc;
         if (!m->sample_part && (rc = dalloc(m, &m->sample_part, L_SAMPLE_PART_DOUBLES, false))) return rc;
-        if (!m->sample_out && (rc = dalloc(m, &m->sample_out, 1, true))) return rc;
+        if (!m->sample_out && (rc = dalloc(m, &m->sample_out, 2, true))) return rc;
         if ((rc = dalloc(m, &m->sample_p, m->c.vocab_size, false))) return rc;
     }
-    HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_part, m->sample_out));
+    HIPCHK(ctx, k_sample(ctx->stream, m->logits, m->c.vocab_size, temperature, u, m->sample_p, m->sample_part, (unsigned *)m->sample_out + 1,
+                         m->box.seen ? m->box.pick : m->sample_out));
     if (probs)
         HIPCHK(ctx, hipMemcpyAsync(probs, m->sample_p, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(m->box.pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (!m->box.seen) HIPCHK(ctx, hipMemcpyAsync(m->box.pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     const int32_t pick = *m->box.pick;
     if (pick < 0) return set_err(ctx, L2H_EINVAL, "nothing to draw from: the logits divided by %g are not all finite", (double)temperature);

@@ -48,7 +48,7 @@ struct PinnedArena {
     }
 };
 
-// What a call hands to the device and gets back, in host memory that stays: pinned, so that a copy is a request among others and the call waits once, at
+// What a call hands to the device and gets back, in host memory that stays: pinned, so that kernels fetch and leave it themselves and the call waits once, at
 // its end (from a call's own stack every copy was a wait).  One call of a model at a time uses it.
 struct HostBox {
     DecodeCtl *ctl = nullptr;   // [2], and the prompt behind them, as on the device
@@ -59,6 +59,7 @@ struct HostBox {
     void *mem = nullptr;
     size_t bytes = 0;
     bool pinned = false;  // by itself (or from the context's arena, which knows)
+    bool seen = false;    // kernels read and write it: it is pinned either way
     // for sequences of n tokens; a box that is there stays (a model is asked to finalize again after it failed).  false: no memory
     bool make(PinnedArena &arena, int64_t n) {
         if (mem) return true;
@@ -69,6 +70,7 @@ struct HostBox {
             mem = arena.pin(bytes);
             pinned = mem != nullptr;
         }
+        seen = mem != nullptr;
         if (!mem) mem = malloc(bytes);  // (then copies wait, as they do from any memory of a program)
         if (!mem) return false;
         memset(mem, 0, bytes);

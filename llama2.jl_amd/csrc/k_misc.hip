@@ -469,9 +469,10 @@ hipError_t k_f32_to_f64(hipStream_t s, const float *x, double *y, int64_t n) {
 // index whose cumulative weight reaches u * sum(weights).  exp in fp64 rounded to fp32 and the sums
 // in fp64 (as everywhere in this library).
 // ------------------------------------------------------------------------------------------
-// In four launches over SAMPLE_PARTS workgroups at most, each a run of the logits: one workgroup alone took 558 us for 128 256 of
-// them (125 exponentials in fp64 a thread, and 1024 running sums added by one thread), the four take 18 us, which is what four
-// dependent launches take.  part: the runs' largest values, sums of exponentials, sums of probabilities.
+// In three launches over SAMPLE_PARTS workgroups at most, each a run of the logits, because a run's exponentials need the largest of all and its probabilities the
+// sum of all; the workgroup that is through last picks, so that nobody waits.  (One workgroup alone: 558 us for 128 256 of them, 125 exponentials in fp64 a
+// thread; a fourth launch for the pick: 5 us more.)  Up to SAMPLE_ONE logits one workgroup does it all, whose elements stay in registers.
+// part: the runs' largest values, sums of exponentials, sums of probabilities.
 #define SAMPLE_THREADS 256
 #define SAMPLE_PARTS 256
 struct SampleRun {
@@ -506,64 +507,78 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_exp_kernel(int n, int p
     sum = block_sum_f64(sum, red);
     if (threadIdx.x == 0) part[SAMPLE_PARTS + blockIdx.x] = sum;
 }
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int per, int parts, float *p, double *part) {
-    __shared__ double red[SAMPLE_THREADS / 64];
-    const SampleRun r = sample_run(n, per, blockIdx.x);
-    const float sf = (float)block_sum_f64((int)threadIdx.x < parts ? part[SAMPLE_PARTS + threadIdx.x] : 0.0, red);
-    double sum = 0.0;
-    for (int i = r.lo + threadIdx.x; i < r.hi; i += SAMPLE_THREADS) {
-        const float pr = p[i] / sf;
-        p[i] = pr;
-        sum += (double)pr;
+// Sums over the workgroup's values: of the threads before this one; `all`: of all of them.  red: a double a wavefront
+__device__ __forceinline__ double sample_before(double v, double *red, double *all) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+        const double o = __shfl_up(x, d, WAVE);
+        x += lane >= d ? o : 0.0;
     }
     __syncthreads();
-    sum = block_sum_f64(sum, red);
-    if (threadIdx.x == 0) part[2 * SAMPLE_PARTS + blockIdx.x] = sum;
+    if (lane == 63) red[wave] = x;
+    __syncthreads();
+    double before = 0.0, sum = 0.0;
+    for (int w = 0; w < nw; w++) {
+        before += w < wave ? red[w] : 0.0;
+        sum += red[w];
+    }
+    *all = sum;
+    return before + (x - v);
 }
-// running sums over the workgroup's values: cum[t + 1] = v of threads 0 .. t, cum[0] = 0
-__device__ void sample_scan(double v, double *cum) {
+__device__ __forceinline__ float sample_load(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// Probabilities and their sums; then, by the workgroup that is through last (count: zero between launches), the pick: the first index at which the running
+// sum reaches u times the whole (the last one of its run if rounding leaves the target just above the total).
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int per, int parts, float u, float *p, double *part, unsigned *count, int32_t *out) {
+    __shared__ double red[SAMPLE_THREADS / 64], s_before;
+    __shared__ int s_last, s_at, s_pick;
     const int t = threadIdx.x;
-    if (t == 0) cum[0] = 0.0;
-    cum[t + 1] = v;
-    for (int d = 1; d < SAMPLE_THREADS; d *= 2) {
+    {
+        const SampleRun r = sample_run(n, per, blockIdx.x);
+        const float sf = (float)block_sum_f64(t < parts ? part[SAMPLE_PARTS + t] : 0.0, red);
+        double sum = 0.0;
+        for (int i = r.lo + t; i < r.hi; i += SAMPLE_THREADS) {
+            const float pr = p[i] / sf;
+            __hip_atomic_store(p + i, pr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (read by another workgroup)
+            sum += (double)pr;
+        }
         __syncthreads();
-        const double w = t + 1 > d ? cum[t + 1 - d] : 0.0;
-        __syncthreads();
-        cum[t + 1] += w;
+        sum = block_sum_f64(sum, red);
+        if (t == 0) __hip_atomic_store(part + 2 * SAMPLE_PARTS + blockIdx.x, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (they are in memory before the count says so)
+    __syncthreads();
+    if (t == 0) {
+        s_last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)parts - 1u;
+        if (s_last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_at = s_pick = 0x7FFFFFFF;
     }
     __syncthreads();
-}
-// the first index at which the running sum reaches u times the whole (the last one of its run if rounding leaves the target just
-// above the total)
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(int n, int per, int parts, float u, const float *p, const double *part, int32_t *out) {
-    __shared__ double cum[SAMPLE_THREADS + 1];
-    __shared__ int s_at, s_pick;
-    const int t = threadIdx.x;
-    sample_scan(t < parts ? part[2 * SAMPLE_PARTS + t] : 0.0, cum);
-    const double target = (double)u * cum[parts];
-    if (t == 0) s_at = s_pick = 0x7FFFFFFF;
-    __syncthreads();
+    if (!s_last) return;
+    const double v = t < parts ? __hip_atomic_load(part + 2 * SAMPLE_PARTS + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+    double all;
+    const double before = sample_before(v, red, &all), target = (double)u * all;
     // (runs are not empty)
-    if (t < parts && ((cum[t] < target && (target <= cum[t + 1] || t == parts - 1)) || (t == 0 && target <= 0.0)))
+    if (t < parts && ((before < target && (target <= before + v || t == parts - 1)) || (t == 0 && target <= 0.0)))
         atomicMin(&s_at, t);  // (rounding may leave a running sum a last bit below the one before it)
     __syncthreads();
     if (s_at == 0x7FFFFFFF) {  // (the probabilities are not numbers: one of the logits was none, or was not finite once divided)
         if (t == 0) *out = -1;
         return;
     }
+    if (t == s_at) s_before = before;
     const SampleRun r = sample_run(n, per, s_at);
-    const double before = cum[s_at];
     const int each = (per + SAMPLE_THREADS - 1) / SAMPLE_THREADS, lo = min(r.hi, r.lo + t * each), hi = min(r.hi, lo + each);
     double mine = 0.0;
-    for (int i = lo; i < hi; i++) mine += (double)p[i];
-    __syncthreads();
-    sample_scan(mine, cum);
+    for (int i = lo; i < hi; i++) mine += (double)sample_load(p + i);
+    const double ahead = sample_before(mine, red, &all) + s_before;  // (behind its barriers)
     const bool last = hi == r.hi && lo < hi;
-    if (lo < hi && (before + cum[t] < target || t == 0) && (target <= before + cum[t + 1] || last)) {
-        double cw = before + cum[t];
+    if (lo < hi && (ahead < target || t == 0) && (target <= ahead + mine || last)) {
+        double cw = ahead;
         int pick = hi - 1;
         for (int i = lo; i < hi; i++) {
-            cw += (double)p[i];
+            cw += (double)sample_load(p + i);
             if (cw >= target) {
                 pick = i;
                 break;
@@ -575,11 +590,88 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(int n, int 
     if (t == 0) *out = s_pick;
 }
 
-hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, int32_t *out) {
+// the same for up to SAMPLE_ONE logits, four a thread
+#define SAMPLE_ONE 4096
+__global__ __launch_bounds__(1024) void sample_one_kernel(const float *logits, int n, float temperature, float u, float *p, int32_t *out) {
+    __shared__ float redf[16];
+    __shared__ double red[16];
+    __shared__ int s_pick;
+    const int t = threadIdx.x, i0 = 4 * t;
+    float v[4], mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v[k] = i0 + k < n ? logits[i0 + k] / temperature : -INFINITY;
+        mx = fmaxf(mx, v[k]);
+    }
+    mx = block_max_f32(mx, redf);
+    double sum = 0.0;
+#pragma nounroll
+    for (int k = 0; k < 4; k++) {  // (one exponential's code)
+        const float x = k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+        const float e = i0 + k < n ? (float)exp((double)(x - mx)) : 0.0f;
+        if (k == 0) v[0] = e;
+        if (k == 1) v[1] = e;
+        if (k == 2) v[2] = e;
+        if (k == 3) v[3] = e;
+        sum += (double)e;
+    }
+    const float sf = (float)block_sum_f64(sum, red);
+    double own = 0.0, all;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v[k] /= sf;
+        if (i0 + k >= n) break;
+        p[i0 + k] = v[k];
+        own += (double)v[k];
+    }
+    if (t == 0) s_pick = 0x7FFFFFFF;
+    const double before = sample_before(own, red, &all), target = (double)u * all;
+    if (!(target <= all)) {  // (not numbers)
+        if (t == 0) *out = -1;
+        return;
+    }
+    if (i0 < n && (before < target || t == 0) && (target <= before + own || i0 + 4 >= n)) {
+        double cw = before;
+        int pick = min(i0 + 3, n - 1);
+        bool there = false;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            cw += i0 + k < n ? (double)v[k] : 0.0;
+            if (!there && i0 + k < n && cw >= target) {
+                pick = i0 + k;
+                there = true;
+            }
+        }
+        atomicMin(&s_pick, pick);
+    }
+    __syncthreads();
+    if (t == 0) *out = s_pick;
+}
+
+hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, unsigned *count, int32_t *out) {
+    if (n <= SAMPLE_ONE) {
+        hipLaunchKernelGGL(sample_one_kernel, dim3(1), dim3(1024), 0, s, logits, n, temperature, u, p, out);
+        return hipGetLastError();
+    }
     const int per = std::max(1024, (int)(((int64_t)n + SAMPLE_PARTS - 1) / SAMPLE_PARTS)), parts = (int)(((int64_t)n + per - 1) / per);
     hipLaunchKernelGGL(sample_max_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, logits, n, per, temperature, p, part);
     hipLaunchKernelGGL(sample_exp_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, n, per, parts, p, part);
-    hipLaunchKernelGGL(sample_prob_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, n, per, parts, p, part);
-    hipLaunchKernelGGL(sample_pick_kernel, dim3(1), dim3(SAMPLE_THREADS), 0, s, n, per, parts, u, p, part, out);
+    hipLaunchKernelGGL(sample_prob_kernel, dim3(parts), dim3(SAMPLE_THREADS), 0, s, n, per, parts, u, p, part, count, out);
+    return hipGetLastError();
+}
+
+// Up to WORD_COPIES runs of 4-byte words from and to anywhere the device sees: what a call hands over and gets back, in one launch of 2 us where a copy of each is one of
+// 4 to 5 and twice the work for the host.
+__global__ __launch_bounds__(1024) void words_kernel(WordCopies c) {
+    const WordCopy w = c.run[blockIdx.x];
+    for (int64_t i = threadIdx.x; i < w.n; i += 1024) w.to[i] = w.from[i];
+}
+hipError_t k_words(hipStream_t s, const WordCopies &c) {
+    int n = 0;
+    WordCopies d;
+    for (const WordCopy &w : c.run)
+        if (w.n > 0) d.run[n++] = w;
+    if (!n) return hipSuccess;
+    hipLaunchKernelGGL(words_kernel, dim3((unsigned)n), dim3(1024), 0, s, d);
     return hipGetLastError();
 }

@@ -272,7 +272,18 @@ hipError_t k_step_begin(hipStream_t s, const DevTensor &emb, const DecodeCtl *pr
 hipError_t k_noalloc_init(int device);
 hipError_t k_argmax_noalloc(hipStream_t s, int device, const float *x_dev, int64_t n, int32_t *out_dev);
 #define L_SAMPLE_PART_DOUBLES (3 * 256)
-hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, int32_t *out);
+// count: zero between calls; out: on the device, or pinned host memory
+hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, unsigned *count, int32_t *out);
+#define WORD_COPIES 3
+struct WordCopy {
+    const uint32_t *from = nullptr;
+    uint32_t *to = nullptr;
+    int64_t n = 0;
+};
+struct WordCopies {
+    WordCopy run[WORD_COPIES];
+};
+hipError_t k_words(hipStream_t s, const WordCopies &c);
 hipError_t k_kv_layout(hipStream_t s, float *kc, float *vc, float *k_lin, float *v_lin, int pos0, int n, int head_size,
                        int n_kv_heads, int seq_len, bool to_cache, int kv16);
 hipError_t k_stream_read(hipStream_t s, const uint4 *p, int64_t n16, uint32_t *sink);

@@ -1442,7 +1442,11 @@ hipError_t layered_prefill_chunk(l2h_model *m, int M, int pos0) {
     CK(keep((int)l->run.size() - 1));
     l->kept_n = M;
     // the last position becomes the decode state's residual stream
-    return hipMemcpyAsync(m->x, l->X + (int64_t)(M - 1) * W, (size_t)W * 4, hipMemcpyDeviceToDevice, s);
+    WordCopies last;
+    last.run[0].from = (const uint32_t *)(l->X + (int64_t)(M - 1) * W);
+    last.run[0].to = (uint32_t *)m->x;
+    last.run[0].n = W;
+    return k_words(s, last);
 }
 
 // logits of n rows of the chunk just computed; rows[] (host) index the chunk's positions

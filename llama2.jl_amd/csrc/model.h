@@ -71,7 +71,7 @@ struct l2h_model {
 #endif
     float *sample_p = nullptr;  // probabilities of the last l2h_sample call
     double *sample_part = nullptr;
-    int32_t *sample_out = nullptr;
+    int32_t *sample_out = nullptr;  // [2]: the pick, unless it goes to the box, and the draw's count of workgroups
     // streaming decode kernel
     bool flow = false;
     bool wait_limit_set = false;  // l2h_model_set_wait_limit: the caller is told where a wait gave up

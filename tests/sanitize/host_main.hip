@@ -304,6 +304,7 @@ static void check_boxes() {
                 std::vector<bool> used(arena.used, arena.used + PinnedArena::UNITS);
                 EXPECT(boxes[i].make(arena, n[i % 7]) && boxes[i].mem == mem && std::equal(used.begin(), used.end(), arena.used) && holds(boxes[i], n[i % 7], (int)i + 1));
                 if (i % 7 == 6) EXPECT(boxes[i].pinned == may_pin);
+                EXPECT(boxes[i].seen == (boxes[i].pinned || (block && i % 7 != 6 && (const char *)boxes[i].mem >= arena.mem && (const char *)boxes[i].mem < arena.mem + PinnedArena::UNIT * PinnedArena::UNITS)));
             }
             for (size_t i = 0; i < boxes.size(); i++) EXPECT(holds(boxes[i], n[i % 7], (int)i + 1));
             // places in the middle that come free are used again
