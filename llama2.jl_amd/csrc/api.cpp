@@ -1531,6 +1531,62 @@ static hipError_t prefill_chunk(l2h_model *m, int M, int pos0) {
     return hipSuccess;
 }
 
+// Workspace for the logits of wanted positions, laid out at the first call that wants several: up to 64 MiB of them stay on the
+// device, so that the copies to the host (27 us a row of 128256 into memory that the caller has not touched yet, the longer
+// half of such a call) come after their passes and not between them: 64 positions of that vocabulary 13.1 -> 4.6 ms with the
+// prompt of 1024, 3 layers of width 4096.  Where the workspace does not fit, or the classifier's inputs are too long for the
+// kernel, the positions go one at a time.
+static void score_buffers(l2h_model *m) {
+    if (m->score_tried) return;
+    m->score_tried = true;
+    const DevTensor &w = m->glob[L2H_OUTPUT];
+    const int64_t V = m->c.vocab_size;
+    if (w.ne1 != V || k_score_positions(w) == 0) return;
+    const int cap = (int)std::min<int64_t>(m->c.seq_len, std::max<int64_t>(1, ((int64_t)64 << 20) / (4 * V)));
+    if (dalloc(m, &m->score_images, k_score_image_bytes(w), false) || dalloc(m, &m->score_y, cap * V, false)) {
+        (void)hipGetLastError();
+        return;
+    }
+    m->score_cap = cap;
+}
+
+// logits of rows `rows` of the pass's residual stream, to `logits` on the host; the last of them stays the model's hidden state
+// and logits
+static int score_rows(l2h_model *m, const std::vector<int32_t> &rows, float *logits) {
+    l2h_ctx *ctx = m->ctx;
+    const int64_t V = m->c.vocab_size, dim = m->c.dim;
+    const int n = (int)rows.size();
+    if (n > 1) score_buffers(m);
+    if (n == 1 || !m->score_cap) {
+        for (int i = 0; i < n; i++) {
+            HIPCHK(ctx, hand_over(m, {{words(m->pf_x + rows[i] * dim, m->x, dim)}}));
+            const hipError_t e = launch_output(m);
+            if (e != hipSuccess) return set_err(ctx, L2H_EHIP, "classifier launch failed: %s", hipGetErrorString(e));
+            HIPCHK(ctx, hipMemcpyAsync(logits + i * V, m->logits, (size_t)V * 4, hipMemcpyDeviceToHost, ctx->stream));
+        }
+        return L2H_OK;
+    }
+    const DevTensor &w = m->glob[L2H_OUTPUT];
+    // (copies of 1 MiB and more to memory that is not pinned are no faster than pieces below that: 5.1 and 4.9 ms)
+    const int most = k_score_positions(w), piece = (int)std::max<int64_t>(1, ((1 << 20) - 1) / (4 * V));
+    for (int i0 = 0; i0 < n; i0 += m->score_cap) {
+        const int k = std::min(m->score_cap, n - i0);
+        for (int i = 0; i < k; i += most) {
+            ScoreRows r{};
+            const int take = std::min(most, k - i);
+            for (int p = 0; p < take; p++) r.row[p] = rows[i0 + i + p];
+            HIPCHK(ctx, k_score(ctx->stream, w, m->pf_x, r, take, m->glob[L2H_RMS_FINAL].f32, m->score_images, m->score_y + i * V));
+        }
+        if (i0 + k == n) {
+            HIPCHK(ctx, hipMemcpyAsync(m->x, m->pf_x + rows[n - 1] * dim, (size_t)dim * 4, hipMemcpyDeviceToDevice, ctx->stream));
+            HIPCHK(ctx, hipMemcpyAsync(m->logits, m->score_y + (k - 1) * V, (size_t)V * 4, hipMemcpyDeviceToDevice, ctx->stream));
+        }
+        for (int i = 0; i < k; i += piece)
+            HIPCHK(ctx, hipMemcpyAsync(logits + (i0 + i) * V, m->score_y + i * V, (size_t)std::min(piece, k - i) * V * 4, hipMemcpyDeviceToHost, ctx->stream));
+    }
+    return L2H_OK;
+}
+
 // want[0..n_want): positions (indexes into tokens) whose logits go to want_logits
 static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, const int32_t *want, int n_want, float *want_logits,
                         float *last_logits, int32_t *next_token) {
@@ -1606,12 +1662,7 @@ static int prefill_impl(l2h_model *m, const int32_t *tokens, int n, int pos0, co
         if (e != hipSuccess)
             return set_err(ctx, L2H_EHIP, "prompt pass launch failed: %s%s%s", hipGetErrorString(e),
                            m->pf_lt_err.empty() ? "" : "; ", m->pf_lt_err.c_str());
-        for (size_t i = 0; i < rows.size(); i++) {
-            HIPCHK(ctx, hipMemcpyAsync(m->x, m->pf_x + (int64_t)rows[i] * m->c.dim, (size_t)m->c.dim * 4, hipMemcpyDeviceToDevice, ctx->stream));
-            const hipError_t el = launch_output(m);
-            if (el != hipSuccess) return set_err(ctx, L2H_EHIP, "classifier launch failed: %s", hipGetErrorString(el));
-            HIPCHK(ctx, hipMemcpyAsync(wl + (int64_t)i * m->c.vocab_size, m->logits, (size_t)m->c.vocab_size * 4, hipMemcpyDeviceToHost, ctx->stream));
-        }
+        if (!rows.empty() && (rc = score_rows(m, rows, wl))) return rc;
     }
     if (!last_logits && !next_token) {
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));

@@ -245,6 +245,14 @@ hipError_t k_mega_bind(hipStream_t s, const PhaseArgs *ph);
 hipError_t k_mega_launch(hipStream_t s, const MegaArgs &g, int t_qkv, int t_wo, int t_w13, int t_w2, int t_out, int grid,
                          size_t lds);
 hipError_t k_stage_dump(hipStream_t s, const float *x, const float *normw, int64_t n, int pro, Q8Dev q8_out, float *f32_out);
+// logits y[n][w.ne1] of n positions, rows rows.row[] of x [..][w.ne0]: final rmsnorm and classifier, one pass over the weights
+constexpr int SCORE_POSITIONS = 8;
+struct ScoreRows {
+    int32_t row[SCORE_POSITIONS];
+};
+int k_score_positions(const DevTensor &w);        // positions of one pass: 8, 4, or 0 where the kernel does not take the matrix
+int64_t k_score_image_bytes(const DevTensor &w);  // bytes of `images`
+hipError_t k_score(hipStream_t s, const DevTensor &w, const float *x, const ScoreRows &rows, int n, const float *normw, char *images, float *y);
 // the same quantization in the streaming decode kernel's form (four blocks per wavefront)
 hipError_t k_quantize_rows16(hipStream_t s, const float *x, int64_t n, Q8Dev q8_out);
 hipError_t k_rope_only(hipStream_t s, float *x, int head_size, int n_heads, int pos, float theta_scale, int neox);

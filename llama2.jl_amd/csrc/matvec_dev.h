@@ -176,32 +176,37 @@ __device__ __forceinline__ SegPtrs seg_ptrs(const PhaseArgs &a, int seg, int lay
     return p;
 }
 
-template <int TYPE>
-__device__ __forceinline__ void load_chunk(Chunk<TYPE> &c, const SegPtrs &t, int64_t row, int g);
-
-template <>
-__device__ __forceinline__ void load_chunk<L2H_TYPE_Q4_K>(Chunk<L2H_TYPE_Q4_K> &c, const SegPtrs &t, int64_t row,
-                                                          int g) {
-    c.w = ldg_nt(t.qs + row * t.nb * 8 + g);
-    c.hdr = ldg_nt(t.hdr + row * t.nb + (g >> 3));
+// NT: past the caches, for weights that one workgroup reads once in whole lines.  Off where a line's pieces are read by several
+// instructions with other rows' in between (the classifier for several positions).
+template <bool NT, class T>
+__device__ __forceinline__ T ld_weight(const T *p) {
+    if constexpr (!NT)
+        return *p;
+    else if constexpr (sizeof(T) == 16)
+        return ldg_nt(p);
+    else
+        return __builtin_nontemporal_load(p);
 }
-template <>
-__device__ __forceinline__ void load_chunk<L2H_TYPE_Q5_K>(Chunk<L2H_TYPE_Q5_K> &c, const SegPtrs &t, int64_t row,
-                                                          int g) {
-    c.w = ldg_nt(t.qs + row * t.nb * 8 + g);
-    c.qh = ldg_nt(t.qh + (row * t.nb + (g >> 3)) * 2 + (g & 1));
-    c.hdr = ldg_nt(t.hdr + row * t.nb + (g >> 3));
+template <bool NT = true>
+__device__ __forceinline__ void load_chunk(Chunk<L2H_TYPE_Q4_K> &c, const SegPtrs &t, int64_t row, int g) {
+    c.w = ld_weight<NT>(t.qs + row * t.nb * 8 + g);
+    c.hdr = ld_weight<NT>(t.hdr + row * t.nb + (g >> 3));
 }
-template <>
-__device__ __forceinline__ void load_chunk<L2H_TYPE_Q6_K>(Chunk<L2H_TYPE_Q6_K> &c, const SegPtrs &t, int64_t row,
-                                                          int g) {
+template <bool NT = true>
+__device__ __forceinline__ void load_chunk(Chunk<L2H_TYPE_Q5_K> &c, const SegPtrs &t, int64_t row, int g) {
+    c.w = ld_weight<NT>(t.qs + row * t.nb * 8 + g);
+    c.qh = ld_weight<NT>(t.qh + (row * t.nb + (g >> 3)) * 2 + (g & 1));
+    c.hdr = ld_weight<NT>(t.hdr + row * t.nb + (g >> 3));
+}
+template <bool NT = true>
+__device__ __forceinline__ void load_chunk(Chunk<L2H_TYPE_Q6_K> &c, const SegPtrs &t, int64_t row, int g) {
     const int64_t blk = row * t.nb + (g >> 2);
     const int n = (g >> 1) & 1, h = g & 1;
-    c.la = ldg_nt(t.qs + blk * 8 + 4 * n + h);
-    c.lb = ldg_nt(t.qs + blk * 8 + 4 * n + 2 + h);
-    c.qh = ldg_nt(t.qh + blk * 4 + 2 * n + h);
-    c.sc = __builtin_nontemporal_load(t.sc6 + blk * 4 + 2 * n + h);
-    c.d = (uint32_t)__builtin_nontemporal_load(t.d6 + blk);
+    c.la = ld_weight<NT>(t.qs + blk * 8 + 4 * n + h);
+    c.lb = ld_weight<NT>(t.qs + blk * 8 + 4 * n + 2 + h);
+    c.qh = ld_weight<NT>(t.qh + blk * 4 + 2 * n + h);
+    c.sc = ld_weight<NT>(t.sc6 + blk * 4 + 2 * n + h);
+    c.d = (uint32_t)ld_weight<NT>(t.d6 + blk);
 }
 
 // ---- this lane's fp64 share of one chunk; DEBUG also stores the per-block integer sums ----------
@@ -742,7 +747,7 @@ __device__ __forceinline__ void matvec_phase(const PhaseArgs &a, int layer, int 
             const int ci = lane + WAVE * step;
             if (ro < rt && lr < n_local && step < nsteps && ci < nchunks) {
                 const RowRef rr = uniform_row(logical_row<EPI>(a, L_lo + lr));
-                if (rr.seg >= 0) load_chunk<TYPE>(t.c[k], seg_ptrs(a, rr.seg, layer), rr.row, ci);
+                if (rr.seg >= 0) load_chunk(t.c[k], seg_ptrs(a, rr.seg, layer), rr.row, ci);
             }
         }
     };
@@ -843,7 +848,7 @@ __device__ __forceinline__ void matvec_prefetch(const PhaseArgs &a, int layer, i
         const int ci = lane + WAVE * step;
         if (ro < rt && lr < n_local && step < nsteps && ci < nchunks) {
             const RowRef rr = uniform_row(logical_row<EPI>(a, L_lo + lr));
-            if (rr.seg >= 0) load_chunk<TYPE>(t.c[k], seg_ptrs(a, rr.seg, layer), rr.row, ci);
+            if (rr.seg >= 0) load_chunk(t.c[k], seg_ptrs(a, rr.seg, layer), rr.row, ci);
         }
     }
 }

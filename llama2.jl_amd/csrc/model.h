@@ -88,6 +88,11 @@ struct l2h_model {
     int32_t *pf_tok = nullptr;
     unsigned char *pf_kvt = nullptr;  // one layer's K / V^T as bf16 tiles of 32 keys (k_pf_kv_tiles)
     int pf_kvt_tiles = 0;             // tiles per KV head
+    // logits of wanted positions: up to score_cap rows of the vocabulary and a pass's quantized inputs (score_buffers)
+    int score_cap = 0;
+    bool score_tried = false;
+    float *score_y = nullptr;
+    char *score_images = nullptr;
     // bf16 copy of the layer matrices for the prompt pass: per layer q|k|v rows, wo, w1/w3 rows in turn, w2
     int pf_copy_mode = 1;          // 0 never, 1 when it fits
     bool pf_copy_tried = false;
