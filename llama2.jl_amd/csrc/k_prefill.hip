@@ -151,7 +151,8 @@ struct PfGemmArgs {
     int interleave;  // logical row L = (segment L & 1, row L >> 1): w1/w3 pairs for SwiGLU
     int64_t n_rows;  // logical rows
     int64_t K;
-    const uint16_t *act;  // bf16 [M][K]
+    int64_t ld;           // elements from one row of act (pf_expand_kernel: one expanded row) to the next, at least K
+    const uint16_t *act;  // bf16 [M][ld]
     int M;
     float *out;  // STORE: fp32 [M][ldo] at column out_col0 + L; RESID: out[m][L] += C
     int64_t ldo, out_col0;
@@ -328,12 +329,13 @@ __device__ __forceinline__ void pf_row_ptr(const PfGemmArgs &a, int64_t L, PfRow
 // product kernel uses on them.  The destination is a sequence of 32 KB tiles, tile (nt, kt) = weight
 // rows 256 nt.. x inputs 64 kt.. at ((nt K/64) + kt) * 16384 elements, and inside a tile the image the
 // product kernel keeps in LDS: the 16-byte chunk c of row r at chunk index 8 r + (c ^ pf_swz(r)).  Logical
-// row L goes to row dst_row0 + L; rows from n_rows up to rows_end (padding of the last tile) are zero.
-// plain: row R is K values in a row at dst + R K instead (the layout a library product takes).
+// row L goes to row dst_row0 + L; rows from n_rows up to rows_end (padding of the last tile) are zero, and so are the inputs from K
+// up to ld, a multiple of 64.
+// plain: row R is ld values in a row at dst + R ld instead (the layout a library product takes).
 template <int TYPE>
 __global__ __launch_bounds__(256) void pf_expand_kernel(PfGemmArgs a, uint16_t *dst, int64_t dst_row0, int64_t rows_end,
                                                         int plain) {
-    const int64_t groups = a.K >> 5, nk = a.K >> 6;
+    const int64_t groups = a.ld >> 5, nk = a.ld >> 6;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= rows_end * groups) return;
     const int64_t L = idx / groups, g = idx - L * groups, k0 = 32 * g;
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(256) void pf_expand_kernel(PfGemmArgs a, uint16_t *
     pf_convert<TYPE>(raw, rp, lr.row, k0, a.K, wv);
     const int64_t R = dst_row0 + L, nt = R >> 8, kt = g >> 1;
     if (plain) {
-        uint4 *row = (uint4 *)(dst + R * a.K + k0);
+        uint4 *row = (uint4 *)(dst + R * a.ld + k0);
 #pragma unroll
         for (int cc = 0; cc < 4; cc++) row[cc] = wv[cc];
         return;
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(256) void pf_gemm_kernel(PfGemmArgs a) {
     for (int i = 0; i < XL; i++) {
         const int m = m0 + (t >> 3) + 32 * i;
         xvalid[i] = m < a.M;
-        xrow[i] = a.act + (int64_t)(xvalid[i] ? m : 0) * K + 8 * xc;
+        xrow[i] = a.act + (int64_t)(xvalid[i] ? m : 0) * a.ld + 8 * xc;
     }
 
     f32x16 acc[2][JT];
@@ -975,7 +977,7 @@ static hipError_t pf_weight_args(PfGemmArgs &a, const DevTensor *w, int nseg, in
 // k_pf_expand; see PfGemmArgs for the outputs
 hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave, const uint16_t *wbf, int64_t n_rows_bf,
                      const uint16_t *act, int M, int64_t K, int epi, float *out, int64_t ldo, int64_t out_col0,
-                     uint16_t *out_bf, int64_t ldb) {
+                     uint16_t *out_bf, int64_t ldb, int64_t lda) {
     PfGemmArgs a{};
     if (wbf) {
         if (K % 64 != 0) return hipErrorInvalidValue;
@@ -987,7 +989,10 @@ hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave
         if (e != hipSuccess) return e;
     }
     if (K % 8 != 0 || M < 1) return hipErrorInvalidValue;
+    if (lda == 0) lda = K;
+    if (lda < K || lda % 8 != 0 || (wbf && lda != K)) return hipErrorInvalidValue;
     const int64_t rows = a.n_rows;
+    a.ld = lda;
     a.act = act;
     a.M = M;
     a.out = out;
@@ -1117,16 +1122,17 @@ hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave
 
 // Expands the rows of the nseg tensors (one after another, or w1/w3 rows in turn when interleave is set) to
 // bf16 into the tiled matrix dst (see pf_expand_kernel) from row dst_row0 on; with pad the rows up to the
-// next multiple of 256 are zeroed.  K a multiple of 64.
-hipError_t k_pf_expand(hipStream_t s, const DevTensor *w, int nseg, int interleave, int64_t K, uint16_t *dst,
+// next multiple of 256 are zeroed.  Rows of ld inputs, a multiple of 64; of fp32 weights K may be less.
+hipError_t k_pf_expand(hipStream_t s, const DevTensor *w, int nseg, int interleave, int64_t K, int64_t ld, uint16_t *dst,
                        int64_t dst_row0, int pad, int plain) {
     PfGemmArgs a{};
     const hipError_t e = pf_weight_args(a, w, nseg, interleave, K);
     if (e != hipSuccess) return e;
-    if (K % 64 != 0) return hipErrorInvalidValue;
+    if (ld % 64 != 0 || ld < K || (ld != K && w[0].type != L2H_TYPE_F32)) return hipErrorInvalidValue;
+    a.ld = ld;
     int64_t rows_end = a.n_rows;
     if (pad) rows_end = (dst_row0 + a.n_rows + 255) / 256 * 256 - dst_row0;
-    const int64_t n = rows_end * (K >> 5);
+    const int64_t n = rows_end * (ld >> 5);
     const dim3 grid((unsigned)((n + 255) / 256));
 #define GO(T) hipLaunchKernelGGL((pf_expand_kernel<T>), grid, dim3(256), 0, s, a, dst, dst_row0, rows_end, plain)
     switch (w[0].type) {

@@ -306,11 +306,11 @@ hipError_t k_pf_rope_scatter(hipStream_t s, const float *raw, const float *cs, u
                              int pos0, int dim, int kv_dim, int hs, int seq_len, int neox);
 hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave, const uint16_t *wbf, int64_t n_rows_bf,
                      const uint16_t *act, int M, int64_t K, int epi, float *out, int64_t ldo, int64_t out_col0,
-                     uint16_t *out_bf, int64_t ldb);
+                     uint16_t *out_bf, int64_t ldb, int64_t lda = 0);  // lda: elements between rows of act, 0 = K
 bool k_pf_few_pays(int64_t rows, int M);
 hipError_t k_pf_few(hipStream_t s, const uint16_t *wbf, int64_t rows, const uint16_t *act, int M, int64_t K, uint16_t *hb, int64_t ldb);
-// plain: rows of K bf16 values one after the other (what pf_lt_gemm multiplies from) instead of the product kernels' tiles
-hipError_t k_pf_expand(hipStream_t s, const DevTensor *w, int nseg, int interleave, int64_t K, uint16_t *dst,
+// plain: rows of ld bf16 values one after the other (what pf_lt_gemm multiplies from) instead of the product kernels' tiles
+hipError_t k_pf_expand(hipStream_t s, const DevTensor *w, int nseg, int interleave, int64_t K, int64_t ld, uint16_t *dst,
                        int64_t dst_row0, int pad, int plain);
 // hipBLASLt for the plain products of the prompt pass (pf_lt.cpp): D[M][0..N) (fp32, row stride ldd) = alpha X[M][K] W[N][K]^T
 // (+ D if accumulate), bf16 operands, fp32 sums.  pf_lt_open returns nullptr, and says why, where the library cannot be used.
