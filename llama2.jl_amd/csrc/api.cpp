@@ -1506,9 +1506,7 @@ static hipError_t prefill_chunk(l2h_model *m, int M, int pos0) {
                 i = j;
             }
         }
-        CK(k_pf_rope_scatter(s, m->pf_raw, m->pf_cs, m->pf_q, kc, vc, M, pos0, dim, kvd, m->hs, c.seq_len,
-                             c.rope_is_neox));
-        CK(k_pf_kv_tiles(s, kc, vc, m->pf_kvt, (pos0 + M + 31) / 32, m->pf_kvt_tiles, m->hs, c.n_kv_heads, c.seq_len));
+        CK(k_pf_rope_tiles(s, m->pf_raw, m->pf_cs, m->pf_q, kc, vc, m->pf_kvt, m->pf_kvt_tiles, M, pos0, dim, kvd, m->hs, c.seq_len, c.rope_is_neox));
         CK(k_pf_attention(s, m->pf_q, m->pf_att, m->pf_kvt, m->pf_kvt_tiles, M, pos0, m->hs, c.n_heads, c.n_kv_heads, dim));
         const DevTensor wo = m->L(l, L2H_WO);
         if (lib)

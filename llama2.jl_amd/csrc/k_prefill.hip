@@ -96,52 +96,6 @@ __global__ __launch_bounds__(256) void pf_rmsnorm_kernel(const float *X, const f
     for (int64_t i = threadIdx.x; i < K; i += blockDim.x) o[i] = (__bf16)(w[i] * (ss * x[i]));
 }
 
-__global__ __launch_bounds__(256) void pf_rope_scatter_kernel(const float *raw, const float *cs, uint16_t *Qb,
-                                                              float *kc, float *vc, int M, int pos0, int dim,
-                                                              int kv_dim, int hs, int seq_len, int neox) {
-    const int m = blockIdx.x;
-    if (m >= M) return;
-    const float *r = raw + (int64_t)m * (dim + 2 * kv_dim);
-    const int half = hs >> 1, pos = pos0 + m;
-    // a thread turns 4 consecutive pairs of one head: rotation indices i0 .. i0+3, whose 8 elements are two
-    // runs of 4 (interleaved pairs: 2 i0 .. and 2 i0 + 4 ..; half-split pairs: i0 .. and i0 + half ..)
-    const int qpH = half >> 2, nquads = ((dim + kv_dim) / hs) * qpH;
-    for (int p = threadIdx.x; p < nquads; p += blockDim.x) {
-        const int hh = p / qpH, i0 = 4 * (p % qpH);
-        const bool is_q = hh < dim / hs;
-        const int h = is_q ? hh : hh - dim / hs;
-        const float *src = r + (is_q ? 0 : dim) + h * hs;
-        const int ea = neox ? i0 : 2 * i0, eb = neox ? i0 + half : 2 * i0 + 4;
-        const float4 a = *(const float4 *)(src + ea), b = *(const float4 *)(src + eb);
-        const float4 c0 = *(const float4 *)(cs + ((int64_t)m * half + i0) * 2);      // cos, sin of i0, i0+1
-        const float4 c1 = *(const float4 *)(cs + ((int64_t)m * half + i0 + 2) * 2);  // ... of i0+2, i0+3
-        float4 oa, ob;
-        if (neox) {  // pair k = (a[k], b[k])
-            oa.x = (a.x * c0.x) - (b.x * c0.y), ob.x = (a.x * c0.y) + (b.x * c0.x);
-            oa.y = (a.y * c0.z) - (b.y * c0.w), ob.y = (a.y * c0.w) + (b.y * c0.z);
-            oa.z = (a.z * c1.x) - (b.z * c1.y), ob.z = (a.z * c1.y) + (b.z * c1.x);
-            oa.w = (a.w * c1.z) - (b.w * c1.w), ob.w = (a.w * c1.w) + (b.w * c1.z);
-        } else {  // pairs (a.x, a.y), (a.z, a.w), (b.x, b.y), (b.z, b.w)
-            oa.x = (a.x * c0.x) - (a.y * c0.y), oa.y = (a.x * c0.y) + (a.y * c0.x);
-            oa.z = (a.z * c0.z) - (a.w * c0.w), oa.w = (a.z * c0.w) + (a.w * c0.z);
-            ob.x = (b.x * c1.x) - (b.y * c1.y), ob.y = (b.x * c1.y) + (b.y * c1.x);
-            ob.z = (b.z * c1.z) - (b.w * c1.w), ob.w = (b.z * c1.w) + (b.w * c1.z);
-        }
-        if (is_q) {
-            uint16_t *q = Qb + (int64_t)m * dim + h * hs;
-            *(uint2 *)(q + ea) = make_uint2(pack_bf16(oa.x, oa.y), pack_bf16(oa.z, oa.w));
-            *(uint2 *)(q + eb) = make_uint2(pack_bf16(ob.x, ob.y), pack_bf16(ob.z, ob.w));
-        } else {  // kv.key_cache[:, :, pos] = k (src/inference.jl:259), elements in groups of 4 per timestep
-            *(float4 *)(kc + (((int64_t)h * (hs >> 2) + (ea >> 2)) * seq_len + pos) * 4) = oa;
-            *(float4 *)(kc + (((int64_t)h * (hs >> 2) + (eb >> 2)) * seq_len + pos) * 4) = ob;
-        }
-    }
-    for (int e = 4 * threadIdx.x; e < kv_dim; e += 4 * blockDim.x) {  // kv.value_cache[pos, :, :] = v (:260)
-        const int h = e / hs, d = e % hs;
-        *(float4 *)(vc + ((int64_t)h * seq_len + pos) * hs + d) = *(const float4 *)(r + dim + kv_dim + e);
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // dense product  C[m][L] = sum_k act[m][k] * W[L][k]   over logical weight rows L
 // ------------------------------------------------------------------------------------------
@@ -605,6 +559,18 @@ struct PfKvTile {
     static constexpr int BYTES = (K_BYTES + V_BYTES + 1023) / 1024 * 1024;  // copied 1 KB at a time
 };
 
+// elements 4 d4 .. of a key's value row into V^T (keys permuted: 16 s + 8 a + 4 g + b -> slot 16 s + 8 g + 4 a + b)
+template <class T>
+__device__ __forceinline__ void pf_v_transposed(unsigned char *s_v, int key, int d4, const float4 &v) {
+    const int rem = key & 15;
+    const int slot = (key & 16) + 8 * ((rem >> 2) & 1) + 4 * (rem >> 3) + (rem & 3);
+    __bf16 *dst = (__bf16 *)(s_v + (4 * d4) * T::VROW) + slot;
+    dst[0] = (__bf16)v.x;
+    dst[T::VROW / 2] = (__bf16)v.y;
+    dst[T::VROW] = (__bf16)v.z;
+    dst[3 * T::VROW / 2] = (__bf16)v.w;
+}
+
 template <int HS>
 __global__ __launch_bounds__(256) void pf_kv_tiles_kernel(const float *kc, const float *vc, unsigned char *tiles,
                                                           int seq_len, int n_tiles_max, int tile0, int kq, int vd) {
@@ -637,17 +603,100 @@ __global__ __launch_bounds__(256) void pf_kv_tiles_kernel(const float *kc, const
                 v.w = 4 * d4 + 3 < vd ? src[3] : 0.f;
             }
         }
-        // key = 16 s + 8 a + 4 g + b  ->  slot 16 s + 8 g + 4 a + b
-        const int rem = key & 15;
-        const int slot = (key & 16) + 8 * ((rem >> 2) & 1) + 4 * (rem >> 3) + (rem & 3);
-        __bf16 *dst = (__bf16 *)(s_v + (4 * d4) * T::VROW) + slot;
-        dst[0] = (__bf16)v.x;
-        dst[T::VROW / 2] = (__bf16)v.y;
-        dst[T::VROW] = (__bf16)v.z;
-        dst[3 * T::VROW / 2] = (__bf16)v.w;
+        pf_v_transposed<T>(s_v, key, d4, v);
     }
     __syncthreads();
     uint4 *dst = (uint4 *)(tiles + ((int64_t)kvh * n_tiles_max + kt) * T::BYTES);
+    for (int c = t; c < T::BYTES / 16; c += 256) dst[c] = ((const uint4 *)s_img)[c];
+}
+
+// What lies between the projections and the attention of a prompt, in one launch: rope! of the queries (to bf16) and keys
+// (src/inference.jl:112-157), the new positions' rows of the fp32 caches (:259-260) and all bf16 tiles.  The first
+// n_tiles * n_kv workgroups make a tile each, of new positions from the projections and of earlier ones from the caches; the
+// others turn a position's query heads each.  A lane of a tile's keys takes a position and pairs, so that the caches' groups of
+// four elements are written 512 bytes at a time.  (As two launches, the second reading the rows back: 19.8 + 7.8 us at 2048
+// positions of 32 and 8 heads of 128, 3.5 + 3.5 at 40 of 8 and 2 of 64; 17.9 and 4.4 like this.)
+struct PfRope {
+    const float *raw, *cs;  // projections [M][dim + 2 kv_dim]; cos, sin [M][hs / 2][2]
+    uint16_t *q;            // [M][dim]
+    float *kc, *vc;
+    unsigned char *tiles;
+    int n_tiles, n_tiles_max, n_kv, M, pos0, dim, kv_dim, seq_len, neox;
+};
+// pairs i0 .. i0 + 3 of one head at src: elements ea .. ea + 3 and eb .. eb + 3 turned (interleaved pairs: 2 i0 .. and 2 i0 + 4 ..;
+// half-split pairs: i0 .. and i0 + half ..)
+__device__ __forceinline__ void pf_turn(const float *src, const float *cs, int i0, int half, int neox, int &ea, int &eb, float4 &oa, float4 &ob) {
+    ea = neox ? i0 : 2 * i0, eb = neox ? i0 + half : 2 * i0 + 4;
+    const float4 a = *(const float4 *)(src + ea), b = *(const float4 *)(src + eb);
+    const float4 c0 = *(const float4 *)(cs + i0 * 2);      // cos, sin of i0, i0+1
+    const float4 c1 = *(const float4 *)(cs + i0 * 2 + 4);  // ... of i0+2, i0+3
+    if (neox) {  // pair k = (a[k], b[k])
+        oa.x = (a.x * c0.x) - (b.x * c0.y), ob.x = (a.x * c0.y) + (b.x * c0.x);
+        oa.y = (a.y * c0.z) - (b.y * c0.w), ob.y = (a.y * c0.w) + (b.y * c0.z);
+        oa.z = (a.z * c1.x) - (b.z * c1.y), ob.z = (a.z * c1.y) + (b.z * c1.x);
+        oa.w = (a.w * c1.z) - (b.w * c1.w), ob.w = (a.w * c1.w) + (b.w * c1.z);
+    } else {  // pairs (a.x, a.y), (a.z, a.w), (b.x, b.y), (b.z, b.w)
+        oa.x = (a.x * c0.x) - (a.y * c0.y), oa.y = (a.x * c0.y) + (a.y * c0.x);
+        oa.z = (a.z * c0.z) - (a.w * c0.w), oa.w = (a.z * c0.w) + (a.w * c0.z);
+        ob.x = (b.x * c1.x) - (b.y * c1.y), ob.y = (b.x * c1.y) + (b.y * c1.x);
+        ob.z = (b.z * c1.z) - (b.w * c1.w), ob.w = (b.z * c1.w) + (b.w * c1.z);
+    }
+}
+template <int HS>
+__global__ __launch_bounds__(256) void pf_rope_tiles_kernel(PfRope a) {
+    typedef PfKvTile<HS> T;
+    __shared__ __align__(16) unsigned char s_img[T::BYTES];
+    constexpr int HALF = HS / 2;
+    const int t = threadIdx.x, ld = a.dim + 2 * a.kv_dim;
+    if ((int)blockIdx.x >= a.n_tiles * a.n_kv) {
+        const int m = (int)blockIdx.x - a.n_tiles * a.n_kv;
+        for (int p = t; p < a.dim / 8; p += 256) {
+            const int h = p / (HALF / 4), i0 = 4 * (p % (HALF / 4));
+            int ea, eb;
+            float4 oa, ob;
+            pf_turn(a.raw + (int64_t)m * ld + h * HS, a.cs + (int64_t)m * HS, i0, HALF, a.neox, ea, eb, oa, ob);
+            uint16_t *q = a.q + (int64_t)m * a.dim + h * HS;
+            *(uint2 *)(q + ea) = make_uint2(pack_bf16(oa.x, oa.y), pack_bf16(oa.z, oa.w));
+            *(uint2 *)(q + eb) = make_uint2(pack_bf16(ob.x, ob.y), pack_bf16(ob.z, ob.w));
+        }
+        return;
+    }
+    unsigned char *s_k = s_img, *s_v = s_img + T::K_BYTES;
+    const int kt = (int)blockIdx.x % a.n_tiles, kvh = (int)blockIdx.x / a.n_tiles, key0 = 32 * kt, end = a.pos0 + a.M;
+    // (the padding behind the rows and the tile is copied with it)
+    for (int c = t; c < T::BYTES / 16; c += 256) ((uint4 *)s_img)[c] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    for (int idx = t; idx < 32 * (HS / 8); idx += 256) {
+        const int key = idx & 31, i0 = 4 * (idx >> 5), pos = key0 + key;
+        int ea = a.neox ? i0 : 2 * i0, eb = a.neox ? i0 + HALF : 2 * i0 + 4;
+        float4 oa = make_float4(0.f, 0.f, 0.f, 0.f), ob = oa;
+        float *ca = a.kc + (((int64_t)kvh * (HS / 4) + (ea >> 2)) * a.seq_len + pos) * 4, *cb = a.kc + (((int64_t)kvh * (HS / 4) + (eb >> 2)) * a.seq_len + pos) * 4;
+        if (pos < a.pos0) {
+            oa = *(const float4 *)ca;
+            ob = *(const float4 *)cb;
+        } else if (pos < end) {
+            const int m = pos - a.pos0;
+            pf_turn(a.raw + (int64_t)m * ld + a.dim + kvh * HS, a.cs + (int64_t)m * HS, i0, HALF, a.neox, ea, eb, oa, ob);
+            *(float4 *)ca = oa;  // kv.key_cache[:, :, pos] = k, elements in groups of 4 per timestep
+            *(float4 *)cb = ob;
+        }
+        *(uint2 *)(s_k + key * T::KROW + ea * 2) = make_uint2(pack_bf16(oa.x, oa.y), pack_bf16(oa.z, oa.w));
+        *(uint2 *)(s_k + key * T::KROW + eb * 2) = make_uint2(pack_bf16(ob.x, ob.y), pack_bf16(ob.z, ob.w));
+    }
+    for (int idx = t; idx < 32 * (HS / 4); idx += 256) {
+        const int d4 = idx % (HS / 4), key = idx / (HS / 4), pos = key0 + key;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        float *cv = a.vc + ((int64_t)kvh * a.seq_len + pos) * HS + 4 * d4;
+        if (pos < a.pos0) {
+            v = *(const float4 *)cv;
+        } else if (pos < end) {
+            v = *(const float4 *)(a.raw + (int64_t)(pos - a.pos0) * ld + a.dim + a.kv_dim + kvh * HS + 4 * d4);
+            *(float4 *)cv = v;  // kv.value_cache[pos, :, :] = v
+        }
+        pf_v_transposed<T>(s_v, key, d4, v);
+    }
+    __syncthreads();
+    uint4 *dst = (uint4 *)(a.tiles + ((int64_t)kvh * a.n_tiles_max + kt) * T::BYTES);
     for (int c = t; c < T::BYTES / 16; c += 256) dst[c] = ((const uint4 *)s_img)[c];
 }
 
@@ -955,13 +1004,6 @@ hipError_t k_pf_rmsnorm(hipStream_t s, const float *X, const float *w, uint16_t 
     hipLaunchKernelGGL(pf_rmsnorm_kernel, dim3((unsigned)M), dim3(256), 0, s, X, w, out, K);
     return hipGetLastError();
 }
-hipError_t k_pf_rope_scatter(hipStream_t s, const float *raw, const float *cs, uint16_t *Qb, float *kc, float *vc, int M,
-                             int pos0, int dim, int kv_dim, int hs, int seq_len, int neox) {
-    hipLaunchKernelGGL(pf_rope_scatter_kernel, dim3((unsigned)M), dim3(256), 0, s, raw, cs, Qb, kc, vc, M, pos0, dim,
-                       kv_dim, hs, seq_len, neox);
-    return hipGetLastError();
-}
-
 // JT tiles of 32 positions per wavefront column: 64 JT positions per workgroup
 template <int TYPE, int JT>
 static hipError_t pf_gemm_type(hipStream_t s, const PfGemmArgs &a, int epi, int64_t rows) {
@@ -1188,6 +1230,25 @@ hipError_t k_pf_kv_tiles(hipStream_t s, const float *kc, const float *vc, unsign
     if (n_tiles < 1 || n_tiles > n_tiles_max) return hipErrorInvalidValue;
     const dim3 grid((unsigned)n_tiles, (unsigned)n_kv);
 #define GO(HS) hipLaunchKernelGGL((pf_kv_tiles_kernel<HS>), grid, dim3(256), 0, s, kc, vc, tiles, seq_len, n_tiles_max, tile0, kq, vdim)
+    switch (hs) {
+    case 32: GO(32); break;
+    case 64: GO(64); break;
+    case 96: GO(96); break;
+    case 128: GO(128); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef GO
+    return hipGetLastError();
+}
+
+// the tiles of keys 0 .. pos0 + M - 1 and what leads to them (pf_rope_tiles_kernel); head sizes as for the attention
+hipError_t k_pf_rope_tiles(hipStream_t s, const float *raw, const float *cs, uint16_t *q, float *kc, float *vc, unsigned char *tiles,
+                           int n_tiles_max, int M, int pos0, int dim, int kv_dim, int hs, int seq_len, int neox) {
+    const int n_tiles = (pos0 + M + 31) / 32;
+    if (M < 1 || pos0 < 0 || pos0 + M > seq_len || n_tiles > n_tiles_max || dim % hs != 0 || kv_dim % hs != 0) return hipErrorInvalidValue;
+    const PfRope a{raw, cs, q, kc, vc, tiles, n_tiles, n_tiles_max, kv_dim / hs, M, pos0, dim, kv_dim, seq_len, neox};
+    const dim3 grid((unsigned)(n_tiles * a.n_kv + M));
+#define GO(HS) hipLaunchKernelGGL((pf_rope_tiles_kernel<HS>), grid, dim3(256), 0, s, a)
     switch (hs) {
     case 32: GO(32); break;
     case 64: GO(64); break;

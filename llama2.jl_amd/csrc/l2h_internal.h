@@ -302,8 +302,8 @@ enum { PF_STORE = 0, PF_RESID = 1, PF_SWIGLU = 2 };
 hipError_t k_pf_embed(hipStream_t s, const DevTensor &emb, const int32_t *tokens, float *X, int M, float scale = 1.0f, float *X_copy = nullptr);
 hipError_t k_pf_rope_table(hipStream_t s, float *cs, int pos0, int M, int half, float theta_scale);
 hipError_t k_pf_rmsnorm(hipStream_t s, const float *X, const float *w, uint16_t *out, int M, int64_t K);
-hipError_t k_pf_rope_scatter(hipStream_t s, const float *raw, const float *cs, uint16_t *Qb, float *kc, float *vc, int M,
-                             int pos0, int dim, int kv_dim, int hs, int seq_len, int neox);
+hipError_t k_pf_rope_tiles(hipStream_t s, const float *raw, const float *cs, uint16_t *q, float *kc, float *vc, unsigned char *tiles,
+                           int n_tiles_max, int M, int pos0, int dim, int kv_dim, int hs, int seq_len, int neox);
 hipError_t k_pf_gemm(hipStream_t s, const DevTensor *w, int nseg, int interleave, const uint16_t *wbf, int64_t n_rows_bf,
                      const uint16_t *act, int M, int64_t K, int epi, float *out, int64_t ldo, int64_t out_col0,
                      uint16_t *out_bf, int64_t ldb, int64_t lda = 0);  // lda: elements between rows of act, 0 = K
