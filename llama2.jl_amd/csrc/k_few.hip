@@ -1,13 +1,17 @@
 // The products of k_gemm.hip for few positions, few rows, or both: C[m][n] = sum_k X[m][k] W[n][k] where tiles of 64 x 64 results
 // would leave most of the chip without one.
 //
-// What bounds such a product is reading the matrix once, so as many wavefronts as possible have a share of it under way: a
-// workgroup takes 16 or 32 rows and 16 to 64 positions, its eight wavefronts an eighth of the inputs each, and their sums are
-// added in LDS, in order.  Operands go from memory straight to the registers that the matrix instructions take (a lane holds 8
-// consecutive inputs of one row), the next step's under way during this one's; a position's inputs come from the L2.  Measured,
-// tiles of 64 x 64 and this, microseconds: 57 positions, 2048 x 10240 bf16: 237, 29; 57 x 32768 x 2048: 55, 29; a router's 16
-// experts, 333 positions x 4096 inputs: 93, 13; 16 gated experts of 2048 x 2048 with 14 positions each: 94, 42.  (Three steps
-// under way instead of one: no faster; what is left is the addresses, 16 rows a load, which lie a multiple of 4 KB apart.)
+// What bounds such a product is reading the matrix once, so as many wavefronts as possible have a share of it under way.
+//
+// few_kernel (fp32, and bf16 of up to 16 positions): a workgroup takes 16 rows and 16 or 32 positions, its eight wavefronts an eighth of the inputs each, and
+// their sums are added in LDS, in order.  Operands go from memory straight to the registers that the matrix instructions take (a lane holds 8 consecutive
+// inputs of one row), the next step's under way during this one's; a position's inputs come from the L2.  A load's 16 rows lie a multiple of 4 KB apart, which
+// is what bounds it from 17 positions on.
+//
+// few_ring_kernel (bf16, few_ring.h): whole lines, through LDS.  Microseconds before (few_kernel with up to 32 rows and 64 positions) and now, a matrix of its
+// own in each launch: 64 positions, 16 384 rows x 2048 inputs 30.6, 17.1; 28 672 x 4096 106, 49.9; 4096 x 14 336 81.7, 30.4; 2048 x 8192 24.7, 13.5; 3072 x 2048 14.3,
+// 8.2; a router's 32 rows x 4096, 12.6, 5.3; 16 experts of 2048 x 2048, 14 and 64 positions each: 43, 28.6 and 124, 47.8.
+#include "few_ring.h"
 #include "layered_gemm.h"
 
 typedef __bf16 few_bf16x8 __attribute__((ext_vector_type(8)));
@@ -118,6 +122,95 @@ __device__ __forceinline__ void few_item(const GemmArgs &a, const uint16_t *W, i
     }
 }
 
+// bf16, rows n0 .. n0 + TN - 1 of W x positions m0 .. m0 + TM - 1; store(quads of the tile, sum) takes the sums of steps k0 .. k1 of 64 inputs
+template <int TN, int TM, class Store>
+__device__ __forceinline__ void few_ring_sums(const GemmArgs &a, const uint16_t *W, int64_t n0, int64_t mb, int m0, int mcount, int k0, int k1, unsigned char *s,
+                                              Store store) {
+    constexpr int LA = TN / 8, LX = TM / 8;
+    const int t = threadIdx.x, lane = t & 63;
+    const uint16_t *wp[LA], *xp[LX];
+#pragma unroll
+    for (int i = 0; i < LA; i++) wp[i] = W + min(n0 + few_ring_row(i, lane), a.n_rows - 1) * a.ld + 64 * k0 + 8 * few_ring_chunk(i, lane);
+#pragma unroll
+    for (int i = 0; i < LX; i++) {
+        int64_t row = mb + min(m0 + few_ring_row(i, lane), mcount - 1);  // (rows past the end repeat the last one; not stored)
+        if (a.gather) row = a.gather[row];
+        xp[i] = (const uint16_t *)a.x + row * a.ldx + 64 * k0 + 8 * few_ring_chunk(i, lane);
+    }
+    few_ring<TN, TM>(k1 - k0, blockIdx.x >> 3, s, [&](int i, int k) { return wp[i] + 64 * k; }, [&](int i, int k) { return xp[i] + 64 * k; });
+    for (int o = t; o < TM * TN / 4; o += 256) store(o, few_ring_sum<TN, TM>(s, o / (TN / 4), o % (TN / 4)));
+}
+template <int EPI, int TN>
+__device__ __forceinline__ void few_ring_store(const GemmArgs &a, int64_t n0, int64_t mb, int m0, int mcount, int o, float4 v) {
+    const int p = o / (TN / 4);
+    const int64_t n = n0 + 4 * (o % (TN / 4));
+    if (m0 + p < mcount) gemm_store4<0, EPI>(a, mb + m0 + p, n, gemm_row<EPI>(a, mb + m0 + p), gemm_col<EPI>(a, n), v.x, v.y, v.z, v.w);
+}
+// `splits` workgroups share an item's inputs.  Each leaves its sums in a.part; the one that is through last (a.arrived: zero between launches) adds all of them,
+// in order, so that nobody waits.
+template <int EPI, int TN, int TM>
+__global__ __launch_bounds__(256) void few_ring_kernel(GemmArgs a, unsigned n_nt, unsigned n_mt, unsigned splits) {
+    extern __shared__ __align__(16) unsigned char s_ring[];
+    __shared__ unsigned s_before;
+    const unsigned n_items = n_nt * n_mt * splits, per = (n_items + 7) / 8, k = blockIdx.x >> 3, id = (blockIdx.x & 7u) * per + k;
+    if (k >= per || id >= n_items) return;
+    const unsigned item = id / splits, part = id % splits;
+    const int64_t n0 = (int64_t)(item / n_mt) * TN;
+    const int m0 = (int)(item % n_mt) * TM, nk = a.ld >> 6, t = threadIdx.x;
+    if (splits == 1) {
+        few_ring_sums<TN, TM>(a, a.w, n0, 0, m0, a.M, 0, nk, s_ring, [&](int o, float4 v) { few_ring_store<EPI, TN>(a, n0, 0, m0, a.M, o, v); });
+        return;
+    }
+    typedef unsigned long long u64;
+    constexpr int QUADS = TM * TN / 4;
+    u64 *mine = (u64 *)(a.part + (int64_t)id * 4 * QUADS);
+    few_ring_sums<TN, TM>(a, a.w, n0, 0, m0, a.M, (int)(nk * part / splits), (int)(nk * (part + 1) / splits), s_ring, [&](int o, float4 v) {
+        // (halves of a quad apart, so that lanes store consecutive words)
+        __hip_atomic_store(mine + o, (u64)__float_as_uint(v.x) | (u64)__float_as_uint(v.y) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(mine + QUADS + o, (u64)__float_as_uint(v.z) | (u64)__float_as_uint(v.w) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the sums have been written where everyone reads them
+    __syncthreads();
+    if (t == 0) {
+        s_before = __hip_atomic_fetch_add(a.arrived + item, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (s_before == splits - 1) __hip_atomic_store(a.arrived + item, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (s_before != splits - 1) return;
+    const u64 *all = (const u64 *)(a.part + (int64_t)item * splits * 4 * QUADS);
+    for (int o = t; o < QUADS; o += 256) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (unsigned p = 0; p < splits; p++) {
+            const u64 lo = __hip_atomic_load(all + 2 * QUADS * p + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const u64 hi = __hip_atomic_load(all + 2 * QUADS * p + QUADS + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v.x += __uint_as_float((unsigned)lo);
+            v.y += __uint_as_float((unsigned)(lo >> 32));
+            v.z += __uint_as_float((unsigned)hi);
+            v.w += __uint_as_float((unsigned)(hi >> 32));
+        }
+        few_ring_store<EPI, TN>(a, n0, 0, m0, a.M, o, v);
+    }
+}
+// an expert's rows, 64 positions at a time or what is left
+template <int EPI, int TN>
+__global__ __launch_bounds__(256) void few_ring_grouped_kernel(GemmArgs a, unsigned n_nt) {
+    extern __shared__ __align__(16) unsigned char s_ring[];
+    const unsigned n_items = (unsigned)a.n_tiles[0] * n_nt, per = (n_items + 7) / 8, k = blockIdx.x >> 3, item = (blockIdx.x & 7u) * per + k;
+    if (k >= per || item >= n_items) return;
+    const GemmTile g = a.tiles[item / n_nt];
+    const uint16_t *w = a.w + g.expert * a.expert_stride;
+    const int64_t n0 = (int64_t)(item % n_nt) * TN;
+    for (int m0 = 0; m0 < g.n; m0 += 64) {
+        if (m0) __syncthreads();
+        auto store = [&](int o, float4 v) { few_ring_store<EPI, TN>(a, n0, g.row0, m0, g.n, o, v); };
+        if (g.n - m0 <= 32)
+            few_ring_sums<TN, 32>(a, w, n0, g.row0, m0, g.n, 0, a.ld >> 6, s_ring, store);
+        else
+            few_ring_sums<TN, 64>(a, w, n0, g.row0, m0, g.n, 0, a.ld >> 6, s_ring, store);
+    }
+}
+
 // Items (rows, positions) are dealt to the 8 XCDs as contiguous runs, positions fastest: workgroups on the same rows share an L2.
 template <int PREC, int EPI, int RN, int JM>
 __global__ __launch_bounds__(64 * FEW_WAVES) void few_kernel(GemmArgs a, unsigned n_nt, unsigned n_mt) {
@@ -148,15 +241,87 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void few_grouped_kernel(GemmArgs a,
     }
 }
 
+// ---- which kernel, for bf16 ----
+// us, few_kernel, then tiles of 32 x 32, 64 x 32, 32 x 64 and 64 x 64 results (rows x positions); S: workgroups that share a tile's inputs
+//   3072 x 2048,  24 positions:  7.7 |  7.4,  9.5,  8.7, 12.1      16 384 x 2048, 32: 26.8 | 17.0, 15.0, 18.0, 15.6
+//                 64:           14.3 |  8.2,  9.8,  9.4, 13.0                     64: 30.6 | 27.1, 21.8, 20.7, 17.1
+//                128:           19.6 | 12.6, 10.4,  9.9, 12.8      28 672 x 4096, 32: 85.2 | 50.2, 42.8, 54.1, 44.5
+//                192:           26.1 | 15.5, 13.5, 15.4, 11.9                     64: 106  | 76.7, 64.8, 61.9, 49.9
+//   2048 x 8192,  32: 24.7 | 20.3 S1, 11.1 S4; 64: 24.7 | 16.0 S2 in 32 x 32, 25.5 S1, 13.5 S4 in 32 x 64
+//   4096 x 14 336, 32: 42.2 | 38.1 S1, 26.3 S2; 64: 81.7 | 32.7 S2 in 32 x 64, 30.4 S4 in 64 x 64
+//   32 x 4096, 64: 12.6 | 6.9 S1, 5.3 S4; 2048 x 2048, 24: 7.6 | 7.0 S1, 7.3 S2 (a share costs 1.7 us, and a step of 64 inputs 0.05 to 0.1)
+// So: the smallest tiles that come to at most one a compute unit (of many inputs, where they can be shared out, all positions up to 64 in one tile), and the
+// largest beyond.  Up to 16 positions few_kernel's 16 x 16 results have more workgroups: 2 to 16 positions of 2048 x 2048 5.5 to 6.5 | 6.0 to 6.6, 4096 x 4096 9.2 to
+// 10.3 | 10.4 to 10.6, but 2048 x 8192 13.8 to 17.1 | 10.5 to 10.8 S4, 4096 x 14 336 24.6 to 28.8 | 23.9 to 24.2 S2, 8 of 16 384 x 2048 15.3 | 14.4.
+struct FewPlan {
+    int rows = 0, positions = 0;  // of a tile (0: few_kernel)
+    unsigned splits = 1;
+};
+static FewPlan few_plan(const GemmArgs &a, int64_t cols) {
+    FewPlan p;
+    const int nk = a.ld / 64;
+    if (nk < 4) return p;  // (wavefronts without a step; 4096 x 128, 120 positions: 3.3 | 3.4, with a decay behind it 4.0 | 4.3)
+    auto tiles = [&](int rows, int positions) { return (cols + rows - 1) / rows * ((a.M + positions - 1) / positions); };
+    if (tiles(32, 32) <= FEW_PART_ITEMS && (a.M <= 32 || nk < 64))
+        p.rows = p.positions = 32;
+    else if (a.M > 32 && tiles(32, 64) <= FEW_PART_ITEMS)
+        p.rows = 32, p.positions = 64;
+    else
+        p.rows = 64, p.positions = a.M <= 32 ? 32 : 64;
+    if (nk >= 64 && a.part && a.arrived)
+        p.splits = (unsigned)max((int64_t)1, min((int64_t)min(8, nk / 16), FEW_PART_ITEMS / tiles(p.rows, p.positions)));
+    if (a.M <= 16 && !(p.splits >= 4 || (p.splits >= 2 && nk >= 128) || (a.M > 4 && tiles(64, 32) >= FEW_PART_ITEMS))) p.rows = 0;
+    return p;
+}
+#define FEW_MAX_DEVICES 64
+template <class... P, class... V>
+static hipError_t few_ring_go(hipStream_t s, void (*kernel)(P...), bool (&set)[FEW_MAX_DEVICES], int lds, int64_t workgroups, V... v) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= FEW_MAX_DEVICES) return hipErrorInvalidDevice;
+    if (!set[dev]) {
+        e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+        set[dev] = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((workgroups + 7) / 8))), dim3(256), lds, s, v...);
+    return hipGetLastError();
+}
+template <int EPI, int TN, int TM>
+static hipError_t few_ring_plain(hipStream_t s, const GemmArgs &a, int64_t cols, unsigned splits) {
+    static bool set[FEW_MAX_DEVICES] = {};
+    const unsigned n_nt = (unsigned)((cols + TN - 1) / TN), n_mt = (unsigned)((a.M + TM - 1) / TM);
+    return few_ring_go(s, few_ring_kernel<EPI, TN, TM>, set, few_ring_lds(TN, TM), (int64_t)n_nt * n_mt * splits, a, n_nt, n_mt, splits);
+}
+template <int EPI, int TN>
+static hipError_t few_ring_grouped(hipStream_t s, const GemmArgs &a, int64_t cols) {
+    static bool set[FEW_MAX_DEVICES] = {};
+    const unsigned n_nt = (unsigned)((cols + TN - 1) / TN);
+    return few_ring_go(s, few_ring_grouped_kernel<EPI, TN>, set, max(few_ring_lds(TN, 32), few_ring_lds(TN, 64)), (int64_t)a.max_tiles * n_nt, a, n_nt);
+}
 template <int PREC, int EPI>
 static hipError_t few_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
     if (a.tiles) {
         if constexpr (EPI == GE_STORE || EPI == GE_UP || EPI == GE_GLU) {
+            if constexpr (PREC == 0) {
+                // us, few_grouped_kernel and tiles of 32 and 64 rows; 8 matrices of 512 x 512 (64 tiles of 64 rows), 8, 16 and 48 positions each: 3.6, 4.0, 6.5;
+                // 3.9, 4.0, 6.1; 4.6, 4.8, 7.9; of 2048 x 1024 (256): 11.0, 13.8, 30.4; 11.1, 11.6, 17.8; 9.5, 9.9, 15.0; 16 of 2048 x 2048, 2, 16 and 64 each:
+                // 29.2, 42.9, 124; 27.6, 29.9, 53.9; 27.8, 28.6, 47.8
+                const int64_t wide = a.M / max(a.rows_each, 1) * ((cols + 63) / 64);
+                if (wide >= 192) return few_ring_grouped<EPI, 64>(s, a, cols);
+                if (a.rows_each > 8) return few_ring_grouped<EPI, 32>(s, a, cols);
+            }
             const unsigned n_nt = (unsigned)((cols + 15) / 16), most = (unsigned)a.max_tiles * n_nt;
             hipLaunchKernelGGL((few_grouped_kernel<PREC, EPI>), dim3(8 * ((most + 7) / 8)), dim3(64 * FEW_WAVES), 0, s, a, n_nt);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;
+    }
+    if constexpr (PREC == 0) {
+        const FewPlan p = few_plan(a, cols);
+        if (p.rows == 32) return p.positions == 32 ? few_ring_plain<EPI, 32, 32>(s, a, cols, p.splits) : few_ring_plain<EPI, 32, 64>(s, a, cols, p.splits);
+        if (p.rows == 64) return p.positions == 32 ? few_ring_plain<EPI, 64, 32>(s, a, cols, p.splits) : few_ring_plain<EPI, 64, 64>(s, a, cols, p.splits);
     }
 #define GO(RN, JM)                                                                                                                        \
     do {                                                                                                                                  \
@@ -164,14 +329,8 @@ static hipError_t few_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
         hipLaunchKernelGGL((few_kernel<PREC, EPI, RN, JM>), dim3(8 * ((n_nt * n_mt + 7) / 8)), dim3(64 * FEW_WAVES), 0, s, a, n_nt, n_mt); \
         return hipGetLastError();                                                                                                         \
     } while (0)
-    // 32 rows and 64 positions at a time where that gives every CU a workgroup: half the reads of the positions (fp32 products of that size go to k_gemm's tiles)
     if (a.M <= 16) GO(1, 1);
-    if constexpr (PREC) {
-        GO(1, 2);
-    } else {
-        if (a.M <= 32 || ((cols + 31) / 32) * ((a.M + 63) / 64) < 256) GO(1, 2);
-        GO(2, 4);
-    }
+    GO(1, 2);
 #undef GO
 }
 

@@ -66,6 +66,9 @@ struct Layered {
     float *X = nullptr, *raw = nullptr, *qkv = nullptr, *kq = nullptr, *beta = nullptr, *lg = nullptr, *gt = nullptr, *ob = nullptr,
           *zb = nullptr, *score = nullptr, *slot_scale = nullptr, *yb = nullptr, *Y = nullptr, *wl = nullptr, *rec = nullptr, *X0 = nullptr, *lat_qa = nullptr,
           *lat_part = nullptr, *kvx = nullptr;
+    float *few_part = nullptr;  // sums of the products of few positions that workgroups share (4 MB)
+    unsigned *few_arrived = nullptr;
+    bool few_tried = false;
     uint16_t *qb = nullptr, *xc = nullptr;
     int kvx_cap = 0;
     void *cq = nullptr;
@@ -1059,6 +1062,14 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
         DA(l->wl, (int64_t)((n_want + 255) / 256 * 256) * c.vocab_size);
         l->want_cap = n_want;
     }
+    if (!l->few_tried && !c.precision) {
+        l->few_tried = true;
+        if (dalloc(m, &l->few_part, FEW_PART_FLOATS, false) || dalloc(m, &l->few_arrived, FEW_PART_ITEMS, true)) {  // (products go without)
+            l->few_part = nullptr;
+            l->few_arrived = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     if (l->keep && l->kept_cap < cap) {
         DA(l->kept, (int64_t)l->run.size() * cap * c.width);
         l->kept_cap = cap;
@@ -1212,6 +1223,8 @@ static hipError_t product(l2h_model *m, GemmArgs a, int epi, float *out, int64_t
     a.outf = out;
     a.ldo = ldo;
     a.mult = mult;
+    a.part = m->lay->few_part;
+    a.arrived = m->lay->few_arrived;
     return k_gemm(m->ctx->stream, a, m->lay->c.precision, epi);
 }
 static bool image_takes(const LMat &w, int M) { return w.image && M >= L_BIG_MIN_M; }
@@ -1223,6 +1236,8 @@ static hipError_t to_acts(l2h_model *m, GemmArgs a, int epi, void *out, int64_t 
         a.w = w->image;
         return k_tiles(m->ctx->stream, a, epi, m->ctx->prop.multiProcessorCount);
     }
+    a.part = m->lay->few_part;
+    a.arrived = m->lay->few_arrived;
     return k_gemm(m->ctx->stream, a, m->lay->c.precision, epi);
 }
 

@@ -118,15 +118,19 @@ struct GemmArgs {
     int64_t expert_stride = 0;
     int rows_each = 0;  // rows of a matrix on average
     const int32_t *gather = nullptr;  // row of x for each row of the product
+    // where workgroups that share a block of results leave their sums (FEW_PART_FLOATS), and how many are through with each (FEW_PART_ITEMS, zero between
+    // launches); without, nothing is shared out
+    float *part = nullptr;
+    unsigned *arrived = nullptr;
 };
 #define L_GEMM_TILE 128  // rows of a block for k_gemm
 hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // The same for few rows or positions (k_few.hip), which k_gemm hands on to where that is the faster way; cols: columns the epilogue
 // covers.  Distinct matrices one after the other:
 //
-// bf16, the time of k_gemm's own tiles over that of k_few.  Grouped, up to 48 positions a matrix (beyond, there are images): at 12, 32, 48 and 56, 8 to 96
-// matrices of 512 to 4096 inputs, 2.4 to 8, 1.7 to 8, 1.2 to 7 and 1.0 to 5.  Plain, up to 128 positions (1.5 to 13, 256 to 32 000 rows), otherwise where tiles of
-// 64 x 64 are at most 256 (8192 rows, 128 positions: 1.6 to 2.0).
+// bf16, the time of k_gemm's own tiles over that of k_few.  Grouped, up to 60 positions a matrix: 8 and 16 matrices of 256 to 2048 inputs, at 8, 32 and 64 positions 1.8
+// to 2.6, 1.7 to 2.3 and 1.4 to 1.8, at 96 0.9 to 1.5.  Plain, up to 128 positions (1.0 to 2.0, 256 to 2048 inputs, up to 32 000 rows), otherwise where tiles of
+// 64 x 64 are at most 256 (1.0 to 1.9), or 768 of at least 2048 inputs: 288 tiles 1.6, 512 1.3, 768 1.1, 1500 0.9; of 512 inputs 512 tiles 0.8.
 //
 // fp32, k_few's time over that of the tiles, at 256 to 4096 inputs.  Plain, up to 8 positions (0.3 to 0.97) and up to 2^17 results, 2^18 of up to 16 positions: of 17
 // positions and more 0.5 to 0.95 up to 2^16.5 results, 0.65 to 1.01 at 2^17, 0.95 to 1.34 at 2^17.5, 0.96 to 1.77 at 2^18, 1.2 to 2.1 at 2^20; of 9 to 12 positions 0.82 to
@@ -134,16 +138,19 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // 1.15 at 2^18.  (With an activation behind them, from 2^17 to 2^18.3 results: up to 512 inputs 0.7 to 1.0, a microsecond, for the same reason.)  Grouped, up to 64 positions a matrix and 2^18
 // results: 8, 16, 32 and 64 positions each 0.4 to 0.99 up to 2^17, 0.75 to 1.27 at 2^18, 0.93 to 1.66 at 2^19; of 2 and 4 each 0.9 to 1.2; of 100 each 1.13 to 1.6, of 128
 // 1.2 to 1.9, of 512 1.2 to 1.9 up to 2^17.
+// tiles of a product that workgroups share out, at most, and their sums
+#define FEW_PART_ITEMS 256
+#define FEW_PART_FLOATS (FEW_PART_ITEMS * 64 * 64)
 #define L_FEW_M 128
 #define L_FEW_M_F32 8
-#define L_FEW_EACH 48
+#define L_FEW_EACH 60
 #define L_FEW_EACH_F32 64
 #define L_FEW_TILES 256
 #define L_FEW_RESULTS_F32 131072
 inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
     if (prec) return a.M <= L_FEW_M_F32 || (a.M * cols <= (a.tiles || a.M <= 16 ? 2 : 1) * L_FEW_RESULTS_F32 && (!a.tiles || a.rows_each <= L_FEW_EACH_F32));
     if (a.tiles) return a.rows_each <= L_FEW_EACH;
-    return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= L_FEW_TILES;
+    return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (a.ld >= 2048 ? 3 : 1) * L_FEW_TILES;
 }
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
 

@@ -1,0 +1,47 @@
+"""bf16 products of 17 to 200 positions (and fewer, of many inputs): tiles of 32 and 64 rows x 32 and 64 positions, workgroups that share a tile's inputs,
+experts' rows a tile at a time, inputs that do not go round four wavefronts, row counts that are no multiple of anything.  Against the restatement, and every
+call again: the same bits, whoever was through last."""
+import numpy as np
+import pytest
+
+import layered_cases as lc
+from oracle import layered_np as ref
+
+pytestmark = pytest.mark.gpu
+
+TOL = 3e-2  # bf16 activations against 64 bits, as for the other prompts
+
+
+def _check(pkg, c, sizes, seed):
+    t = lc.settle_routers(c, ref.random_tensors(c, seed), seed)
+    tok = lc.tokens(max(sizes), c["vocab"], 4)
+    want = ref.Sequence(c, t).run(tok)
+    dev = lc.language_model(pkg, c, t, precision="bfloat16").device()
+    dev.set_prefill_library(False)
+    for n in sizes:
+        at = np.arange(max(0, n - 70), n)
+        got = dev.prefill_logits(tok[:n], at)
+        assert lc.error(got, want[at]) <= TOL, n
+        assert np.array_equal(got, dev.prefill_logits(tok[:n], at)), n
+    dev.close()
+
+
+# inputs of the down product: 65, 64 and 130 steps of 64, shared by 4, 4 and 8 workgroups a tile; of 1300 rows by 2 from 129 positions on
+@pytest.mark.parametrize("width,ff,sizes", [(334, 4150, (3, 16, 17, 32, 33, 64, 65, 130)), (66, 8310, (9, 40, 96)), (1300, 4096, (24, 60, 129, 190))])
+def test_shared_inputs(pkg, width, ff, sizes):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=32, vdim=32, rot=32, mlp=lc.dense(ff))], width=width, vocab=120)
+    _check(pkg, c, sizes, 61)
+
+
+# logits of up to 70 positions: 32 x 32, 64 x 32 and 64 x 64 of 8210 rows, 32 x 64 of 4120; 5 and 6 steps of inputs
+@pytest.mark.parametrize("vocab,width", [(8210, 334), (4120, 300), (16390, 257)])
+def test_many_rows(pkg, vocab, width):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, rot=16, mlp=lc.dense(515))], width=width, vocab=vocab)
+    _check(pkg, c, (5, 8, 17, 32, 33, 64, 65, 70), 62)
+
+
+# (experts, chosen, rows of the up product): few rows, up to 8 positions an expert on average and more; many rows; an expert with more than 64
+@pytest.mark.parametrize("experts,top,rows", [(8, 2, 70), (8, 4, 2100), (3, 1, 520)])
+def test_experts(pkg, experts, top, rows):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, rot=16, mlp=lc.moe(experts, top, rows))], width=330, vocab=60)
+    _check(pkg, c, (6, 17, 33, 70, 110, 127), 63)
