@@ -16,21 +16,47 @@ constexpr int FEW_RING_SUMS = 8 * 33;  // 16-byte words of 32 rows x 32 position
 __device__ __forceinline__ int few_ring_row(int i, int lane) { return 8 * i + (lane >> 3); }
 __device__ __forceinline__ int few_ring_chunk(int i, int lane) { return (lane & 7) ^ pf_swz(few_ring_row(i, lane)); }
 
-// a(i, k): address of the 16 bytes that load i of this lane brings of the rows' step k; x(i, k): of the positions'.  nk: steps.  first: where among its steps a
-// wavefront begins (modulo their number): rows lie a multiple of 4 KB apart, so workgroups in step would all ask the same channels.  (16 384 rows x 2048 inputs, 8 to 32
-// positions: 19.4 us without, 15.9 with it.)  s: few_ring_lds() bytes.  Behind the call s holds wavefront w's sums in words
+// Which steps a wavefront takes, and in which order: every fourth one, from `first` on among its own (modulo their number): rows lie a multiple of 4 KB apart, so
+// workgroups in step would all ask the same channels.  (16 384 rows x 2048 inputs, 8 to 32 positions: 19.4 us without, 15.9 with it.)
+struct FewQuarters {
+    int n, from, wave;
+    __device__ __forceinline__ FewQuarters(int nk, unsigned first, int wave) : n(nk > wave ? (nk - wave + 3) >> 2 : 0), from(0), wave(wave) {
+        if (n) from = (int)(first % (unsigned)n);
+    }
+    __device__ __forceinline__ int step(int i) const {
+        const int j = i + from;
+        return wave + 4 * (j < n ? j : j - n);
+    }
+    __device__ __forceinline__ int cut() const { return -1; }
+};
+// Or two eighths of the inputs, w and w + 4, each summed by itself in order: the same sums whichever comes first.
+struct FewEighths {
+    int n, at[2], before;
+    __device__ __forceinline__ FewEighths(int nk, unsigned first, int wave) {
+        const int lo = nk * wave / 8, n_lo = nk * (wave + 1) / 8 - lo, hi = nk * (wave + 4) / 8, n_hi = nk * (wave + 5) / 8 - hi;
+        const bool turned = first & 1u;
+        before = turned ? n_hi : n_lo;
+        at[0] = turned ? hi : lo;
+        at[1] = (turned ? lo : hi) - before;
+        n = n_lo + n_hi;
+    }
+    __device__ __forceinline__ int step(int i) const { return i + at[i >= before]; }
+    __device__ __forceinline__ int cut() const { return before; }
+};
+
+// a(i, k): address of the 16 bytes that load i of this lane brings of the rows' step k; x(i, k): of the positions'.  nk: steps.  s: few_ring_lds() bytes.  Behind the call s holds wavefront w's sums in words
 // [w][rows / 32][positions / 32][FEW_RING_SUMS], and all wavefronts have met.
-template <int TN, int TM, class A, class X>
+template <int TN, int TM, class Order, class A, class X>
 __device__ __forceinline__ void few_ring(int nk, unsigned first, unsigned char *s, A a, X x) {
     constexpr int BLOCK = few_ring_block(TN, TM), DEPTH = few_ring_depth(TN, TM), IT = TN / 32, JT = TM / 32, LA = TN / 8, LX = TM / 8, LOADS = LA + LX;
     static_assert(DEPTH >= 2 && DEPTH <= 4 && 3 * LOADS < 64, "counts of loads under way");
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     unsigned char *ring = s + wave * (DEPTH * BLOCK);
-    const int n = nk > wave ? (nk - wave + 3) >> 2 : 0;  // this wavefront's steps
-    const int from = n ? (int)(first % (unsigned)n) : 0;
+    const Order order(nk, first, wave);
+    const int n = order.n;  // this wavefront's steps
     auto issue = [&](int i, int slot) {
         unsigned char *to = ring + slot * BLOCK;
-        const int j = i + from, k = wave + 4 * (j < n ? j : j - n);
+        const int k = order.step(i);
 #pragma unroll
         for (int l = 0; l < LA; l++) __builtin_amdgcn_global_load_lds((const PF_AS1 void *)a(l, k), (PF_AS3 void *)(to + 1024 * l), 16, 0, 0);
 #pragma unroll
@@ -39,13 +65,18 @@ __device__ __forceinline__ void few_ring(int nk, unsigned first, unsigned char *
     unsigned at[4];
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) at[kk] = 128u * (unsigned)(lane & 31) + 16u * (unsigned)((2 * kk + (lane >> 5)) ^ pf_swz(lane & 31));
-    f32x16 acc[IT][JT];
+    f32x16 acc[IT][JT], other[IT][JT];  // (other: the sums before the cut)
+    auto clear = [&](f32x16(&c)[IT][JT]) {
 #pragma unroll
-    for (int i = 0; i < IT; i++)
+        for (int i = 0; i < IT; i++)
 #pragma unroll
-        for (int j = 0; j < JT; j++)
+            for (int j = 0; j < JT; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+                for (int r = 0; r < 16; r++) c[i][j][r] = 0.0f;
+    };
+    constexpr bool CUT = __is_same(Order, FewEighths);
+    clear(acc);
+    if constexpr (CUT) clear(other);
     // A step's operands come into registers at once, and the next step of its slot is requested before they are multiplied.  (Reads and their wait in one statement:
     // the compiler would make reads of its own wait for every load under way.)
     pf_u32x4 F[4][IT + JT];
@@ -75,7 +106,15 @@ __device__ __forceinline__ void few_ring(int nk, unsigned first, unsigned char *
                              : "memory");
         }
     };
-    auto multiply = [&] {
+    auto multiply = [&](int i_step) {
+        if constexpr (CUT)
+            if (i_step == order.cut()) {
+#pragma unroll
+                for (int i = 0; i < IT; i++)
+#pragma unroll
+                    for (int j = 0; j < JT; j++) other[i][j] = acc[i][j];
+                clear(acc);
+            }
 #pragma unroll
         for (int kk = 0; kk < 4; kk++)
 #pragma unroll
@@ -90,7 +129,7 @@ __device__ __forceinline__ void few_ring(int nk, unsigned first, unsigned char *
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * LOADS) : "memory");
         read(slot);
         issue(i + DEPTH, slot);
-        multiply();
+        multiply(i);
         slot = slot == DEPTH - 1 ? 0 : slot + 1;
     }
     for (; i < n; i++) {
@@ -103,9 +142,14 @@ __device__ __forceinline__ void few_ring(int nk, unsigned first, unsigned char *
         else
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         read(slot);
-        multiply();
+        multiply(i);
         slot = slot == DEPTH - 1 ? 0 : slot + 1;
     }
+    if constexpr (CUT)
+#pragma unroll
+        for (int i = 0; i < IT; i++)
+#pragma unroll
+            for (int j = 0; j < JT; j++) acc[i][j] += other[i][j];
     __syncthreads();  // (the sums' places are another wavefront's ring)
 #pragma unroll
     for (int i = 0; i < IT; i++)
@@ -127,4 +171,20 @@ __device__ __forceinline__ float4 few_ring_sum(const unsigned char *s, int p, in
     for (int w = 0; w < 4; w++) v[w] = *(const float4 *)(s + 16 * (((w * IT + (q >> 3)) * JT + (p >> 5)) * FEW_RING_SUMS + 33 * (q & 7) + (p & 31)));
     return make_float4((v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y), (v[0].z + v[1].z) + (v[2].z + v[3].z),
                        (v[0].w + v[1].w) + (v[2].w + v[3].w));
+}
+// launches one of the kernels above: workgroups a multiple of 8, LDS beyond 64 KB allowed once a device
+#define FEW_RING_DEVICES 64
+template <class... P, class... V>
+static hipError_t few_ring_go(hipStream_t s, void (*kernel)(P...), bool (&set)[FEW_RING_DEVICES], int lds, int64_t workgroups, V... v) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= FEW_RING_DEVICES) return hipErrorInvalidDevice;
+    if (!set[dev]) {
+        e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+        set[dev] = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((workgroups + 7) / 8))), dim3(256), lds, s, v...);
+    return hipGetLastError();
 }

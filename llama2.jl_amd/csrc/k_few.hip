@@ -137,7 +137,7 @@ __device__ __forceinline__ void few_ring_sums(const GemmArgs &a, const uint16_t 
         if (a.gather) row = a.gather[row];
         xp[i] = (const uint16_t *)a.x + row * a.ldx + 64 * k0 + 8 * few_ring_chunk(i, lane);
     }
-    few_ring<TN, TM>(k1 - k0, blockIdx.x >> 3, s, [&](int i, int k) { return wp[i] + 64 * k; }, [&](int i, int k) { return xp[i] + 64 * k; });
+    few_ring<TN, TM, FewQuarters>(k1 - k0, blockIdx.x >> 3, s, [&](int i, int k) { return wp[i] + 64 * k; }, [&](int i, int k) { return xp[i] + 64 * k; });
     for (int o = t; o < TM * TN / 4; o += 256) store(o, few_ring_sum<TN, TM>(s, o / (TN / 4), o % (TN / 4)));
 }
 template <int EPI, int TN>
@@ -264,7 +264,7 @@ static FewPlan few_plan(const GemmArgs &a, int64_t cols) {
     auto tiles = [&](int rows, int positions) { return (cols + rows - 1) / rows * ((a.M + positions - 1) / positions); };
     if (tiles(32, 32) <= FEW_PART_ITEMS && (a.M <= 32 || nk < 64))
         p.rows = p.positions = 32;
-    else if (a.M > 32 && tiles(32, 64) <= FEW_PART_ITEMS)
+    else if (a.M > 32 && tiles(32, 64) <= FEW_PART_ITEMS && !(nk >= 128 && a.M <= 64 && tiles(32, 64) > 64))
         p.rows = 32, p.positions = 64;
     else
         p.rows = 64, p.positions = a.M <= 32 ? 32 : 64;
@@ -273,30 +273,15 @@ static FewPlan few_plan(const GemmArgs &a, int64_t cols) {
     if (a.M <= 16 && !(p.splits >= 4 || (p.splits >= 2 && nk >= 128) || (a.M > 4 && tiles(64, 32) >= FEW_PART_ITEMS))) p.rows = 0;
     return p;
 }
-#define FEW_MAX_DEVICES 64
-template <class... P, class... V>
-static hipError_t few_ring_go(hipStream_t s, void (*kernel)(P...), bool (&set)[FEW_MAX_DEVICES], int lds, int64_t workgroups, V... v) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= FEW_MAX_DEVICES) return hipErrorInvalidDevice;
-    if (!set[dev]) {
-        e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-        set[dev] = true;
-    }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((workgroups + 7) / 8))), dim3(256), lds, s, v...);
-    return hipGetLastError();
-}
 template <int EPI, int TN, int TM>
 static hipError_t few_ring_plain(hipStream_t s, const GemmArgs &a, int64_t cols, unsigned splits) {
-    static bool set[FEW_MAX_DEVICES] = {};
+    static bool set[FEW_RING_DEVICES] = {};
     const unsigned n_nt = (unsigned)((cols + TN - 1) / TN), n_mt = (unsigned)((a.M + TM - 1) / TM);
     return few_ring_go(s, few_ring_kernel<EPI, TN, TM>, set, few_ring_lds(TN, TM), (int64_t)n_nt * n_mt * splits, a, n_nt, n_mt, splits);
 }
 template <int EPI, int TN>
 static hipError_t few_ring_grouped(hipStream_t s, const GemmArgs &a, int64_t cols) {
-    static bool set[FEW_MAX_DEVICES] = {};
+    static bool set[FEW_RING_DEVICES] = {};
     const unsigned n_nt = (unsigned)((cols + TN - 1) / TN);
     return few_ring_go(s, few_ring_grouped_kernel<EPI, TN>, set, max(few_ring_lds(TN, 32), few_ring_lds(TN, 64)), (int64_t)a.max_tiles * n_nt, a, n_nt);
 }

@@ -45,3 +45,24 @@ def test_many_rows(pkg, vocab, width):
 def test_experts(pkg, experts, top, rows):
     c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, rot=16, mlp=lc.moe(experts, top, rows))], width=330, vocab=60)
     _check(pkg, c, (6, 17, 33, 70, 110, 127), 63)
+
+
+# w1 | w3 in tiles of 32 x 32, 32 x 64, 64 x 32 and 64 x 64; eighths of 1, 2, 3 and 21 steps of inputs, of which some are empty or longer
+@pytest.mark.parametrize("dim,hidden,lengths", [(128, 2048, (33, 65, 128, 130)), (192, 8192, (1, 8, 17, 40, 64)), (1344, 4160, (24, 64, 70, 128))])
+def test_llama(pkg, dim, hidden, lengths):
+    """Against the products that sum their inputs in one part: one more rounding to bf16 the other way for the odd element, as for other prompts with
+    and without the library's products"""
+    from llama2_jl_amd import synth
+    cfg = pkg.ModelConfig(dim=dim, hidden_dim=hidden, n_layers=2, n_heads=dim // 32, n_kv_heads=1, vocab_size=256, seq_len=max(lengths), rope_freq_base=10000.0,
+                          rope_is_neox=False)
+    dev = synth.synthetic_model(cfg, synth.PLAN_F32, seed=3).device()
+    for n in lengths:
+        prompt, got = synth.seeded_prompt(n, n, 256), []
+        for library in (True, False, True):
+            dev.set_prefill_library(library)
+            dev.reset()
+            got.append(dev.prefill_logits(prompt, np.arange(n)))
+            assert dev.prefill_library == library
+        assert np.array_equal(got[0], got[2]), n
+        assert np.linalg.norm(got[0] - got[1]) <= 1.5e-2 * np.linalg.norm(got[1]), n
+    dev.close()
