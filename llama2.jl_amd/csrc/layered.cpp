@@ -1208,7 +1208,7 @@ static GemmArgs gemm_of(const LMat &w, const void *x, int M) {
 // that few different shapes occur: the rows beyond M are computed from whatever the buffers hold, and never read
 static bool library_takes(const l2h_model *m, const GemmArgs &a) {
     return m->lay->c.precision == 0 && m->pf_lt && m->pf_library_mode && a.M >= L_BIG_MIN_M &&
-           (double)a.M * (double)a.n_rows * (double)a.ld >= (double)(1 << 26);
+           (double)a.M * (double)a.n_rows * (double)a.ld >= (double)(1 << 26) && !k_few_plain_pays(a);
 }
 static hipError_t product(l2h_model *m, GemmArgs a, int epi, float *out, int64_t ldo, float mult) {
     if ((epi == GE_STORE || epi == GE_RESID) && library_takes(m, a)) {
@@ -1349,12 +1349,15 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     GemmTile *const lists[2] = {l->tiles, l->tiles2};
     GemmArgs *const products[2] = {&up, &down};
     unsigned bound[2];
+    bool few[2];
     for (int p = 0; p < 2; p++) {
         GemmArgs &a = *products[p];
         a.tiles = image ? lists[p] : l->tiles;
         a.n_tiles = image ? l->n_tiles + p : l->n_tiles;
         a.rows_each = slots / d.n_experts;
-        bound[p] = tiles_bound(slots, d.n_experts, (unsigned)((a.n_rows + 255) / 256), (unsigned)a.ld >> 6, (unsigned)cu);
+        few[p] = image && k_few_experts_pays(d.n_experts, a.n_rows, a.ld, a.rows_each);
+        a.few = few[p];
+        bound[p] = few[p] ? 1 : tiles_bound(slots, d.n_experts, (unsigned)((a.n_rows + 255) / 256), (unsigned)a.ld >> 6, (unsigned)cu);
         a.max_tiles = image ? (int)tiles_most(slots, d.n_experts, bound[p]) : (slots + L_GEMM_TILE - 1) / L_GEMM_TILE + d.n_experts;
     }
     if (image)
@@ -1369,7 +1372,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     up.act = d.ff_act;
     up.outa = l->hb;
     up.lda = L.down.ld;
-    if (image) {
+    if (image && !few[0]) {
         up.w = L.up.image;
         up.expert_stride = L.up.image_stride;
         CK(k_tiles(s, up, epi, cu));
@@ -1379,7 +1382,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     down.expert_stride = (int64_t)l->W() * L.down.ld;
     down.outf = l->yb;
     down.ldo = l->W();
-    if (image) {
+    if (image && !few[1]) {
         down.w = L.down.image;
         down.expert_stride = L.down.image_stride;
         CK(k_tiles(s, down, GE_STORE, cu));

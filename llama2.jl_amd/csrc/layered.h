@@ -117,6 +117,7 @@ struct GemmArgs {
     int max_tiles = 0;
     int64_t expert_stride = 0;
     int rows_each = 0;  // rows of a matrix on average
+    bool few = false;   // to k_few, whatever k_few_pays says
     const int32_t *gather = nullptr;  // row of x for each row of the product
     // where workgroups that share a block of results leave their sums (FEW_PART_FLOATS), and how many are through with each (FEW_PART_ITEMS, zero between
     // launches); without, nothing is shared out
@@ -149,10 +150,26 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 #define L_FEW_RESULTS_F32 131072
 inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
     if (prec) return a.M <= L_FEW_M_F32 || (a.M * cols <= (a.tiles || a.M <= 16 ? 2 : 1) * L_FEW_RESULTS_F32 && (!a.tiles || a.rows_each <= L_FEW_EACH_F32));
+    if (a.few) return true;
     if (a.tiles) return a.rows_each <= L_FEW_EACH;
     return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (a.ld >= 2048 ? 3 : 1) * L_FEW_TILES;
 }
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
+// Experts' products of a bf16 prompt that have a tile image: k_few from the plain rows where the image's row groups of 256 are too few for the compute units.  us, k_tiles
+// and k_few, 16, 48 and 83 positions an expert: 8 of 512 x 512 (16 groups) 7.2, 9.9, 11.0 and 4.0, 6.1, 7.3; 32 of 512 x 1024 (64) 16.6, 19.7, 21.6 and 9.5, 14.2, 16.6; 8 of
+// 1792 x 3584 (56) 42, 51, 54 and 21, 36, 38; 128 each 1.3 to 1.5 times; 16 of 2048 x 4096 (128) 56, 64, 72 and 48, 64, 85; 32 of 1024 x 2048 (128) 31, 35, 38 and 28, 36, 47; 16 of
+// 2048 x 1024 (128) 17.5, 20.6, 23.3 and 17.2, 23.0, 29.4; 16 of 4096 x 2048 (256) 49, 52, 57 and 51, 70, 95.
+inline bool k_few_experts_pays(int experts, int64_t rows, int ld, int rows_each) {
+    const int64_t groups = experts * ((rows + 255) / 256);
+    return (groups <= 64 && rows_each <= 128) || (groups <= 128 && rows_each <= 32 && ld >= 2048);
+}
+// A plain product (GE_STORE, GE_RESID) that the library would take: k_few where tiles of 64 x 64 are at most one a compute unit and its inputs few enough.  us, the library
+// with positions in whole groups of 128 and k_few, 130, 256, 333 and 500 positions: 1024 x 1024 5.5, 5.4, 6.5, 6.5 and 4.5, 4.6, 5.7, 5.8; 2048 x 2048 10.1, 10.1, 12.6, 12.8 and 8.1, 9.1,
+// 10.3, 11.5; 1024 x 4096 12.0, 12.0, 15.1, 15.7 and 10.3, 11.2, 12.0, 15.1; 4096 x 4096 22.9, 22.8 and 18.3, 23.0, but 333 (384 tiles) 24.9 and 32.5; 2048 x 6144 23.2, 23.2, 27.5, 27.3 and
+// 17.7, 21.1, 29.0, 31.7; 6144 x 2048, 130 (288) 16.0 and 20.5.  More than 512 positions only of a router: 2048 of 32 x 2048 6.8 and 5.4, but of 256 x 2048 8.8 and 13.0
+inline bool k_few_plain_pays(const GemmArgs &a) {
+    return (a.M <= 512 || a.n_rows <= 32) && (a.n_rows + 63) / 64 * ((a.M + 63) / 64) <= L_FEW_TILES && (a.ld <= 4096 || a.M <= 256);
+}
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations
 hipError_t k_tiles(hipStream_t s, const GemmArgs &a, int epi, int n_cu);

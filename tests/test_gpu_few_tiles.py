@@ -66,3 +66,21 @@ def test_llama(pkg, dim, hidden, lengths):
         assert np.array_equal(got[0], got[2]), n
         assert np.linalg.norm(got[0] - got[1]) <= 1.5e-2 * np.linalg.norm(got[1]), n
     dev.close()
+
+
+# prompts that have tile images: both, one and none of the experts' products from the plain rows; an expert's last block with a single row
+@pytest.mark.parametrize("experts,top,rows,sizes", [(8, 2, 300, (130, 257, 500, 516)), (5, 1, 4100, (129, 400)), (70, 2, 260, (140,))])
+def test_experts_with_images(pkg, experts, top, rows, sizes):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, rot=16, mlp=lc.moe(experts, top, rows))], width=330, vocab=60)
+    t = lc.settle_routers(c, ref.random_tensors(c, 64), 64)
+    tok = lc.tokens(max(sizes), c["vocab"], 4)
+    want = ref.Sequence(c, t).run(tok)
+    for images in (True, False):
+        dev = lc.language_model(pkg, c, t, seq_len=520, precision="bfloat16").device()
+        dev.set_prefill_copy(images)
+        for n in sizes:
+            got = dev.prefill_logits(tok[:n], np.arange(n))
+            assert dev.chosen("tile_images") == (2 if images else 0)
+            for lo in range(0, n, 64):
+                assert lc.error(got[lo:lo + 64], want[lo:min(lo + 64, n)]) <= TOL, (n, lo)
+        dev.close()
