@@ -1062,14 +1062,6 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
         DA(l->wl, (int64_t)((n_want + 255) / 256 * 256) * c.vocab_size);
         l->want_cap = n_want;
     }
-    if (!l->few_tried && !c.precision) {
-        l->few_tried = true;
-        if (dalloc(m, &l->few_part, FEW_PART_FLOATS, false) || dalloc(m, &l->few_arrived, FEW_PART_ITEMS, true)) {  // (products go without)
-            l->few_part = nullptr;
-            l->few_arrived = nullptr;
-            (void)hipGetLastError();
-        }
-    }
     if (l->keep && l->kept_cap < cap) {
         DA(l->kept, (int64_t)l->run.size() * cap * c.width);
         l->kept_cap = cap;
@@ -1183,6 +1175,15 @@ int layered_prefill_buffers(l2h_model *m, int cap, int n_want) {
     }
 #undef DB
 #undef DA
+    // (behind everything that a pass cannot do without)
+    if (!l->few_tried && !c.precision) {
+        l->few_tried = true;
+        if (dalloc(m, &l->few_part, FEW_PART_FLOATS, false) || dalloc(m, &l->few_arrived, FEW_PART_ITEMS, true)) {  // (products go without)
+            l->few_part = nullptr;
+            l->few_arrived = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     l->cap = cap;
     return L2H_OK;
 }
