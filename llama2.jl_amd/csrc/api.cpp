@@ -1743,7 +1743,7 @@ extern "C" int l2h_sample(l2h_model *m, float temperature, float u, int32_t *tok
     if (!m->box.seen) HIPCHK(ctx, hipMemcpyAsync(m->box.pick, m->sample_out, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     const int32_t pick = *m->box.pick;
-    if (pick < 0) return set_err(ctx, L2H_EINVAL, "nothing to draw from: the logits divided by %g are not all finite", (double)temperature);
+    if (pick < 0 || pick >= m->c.vocab_size) return set_err(ctx, L2H_EINVAL, "nothing to draw from: the logits divided by %g are not all finite", (double)temperature);
     *token = pick;
     return L2H_OK;
 }

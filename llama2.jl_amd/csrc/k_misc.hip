@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "dev_common.h"
+#include "draw.h"
 
 // ------------------------------------------------------------------------------------------
 // Repack GGUF super-blocks <-> field streams (see DevTensor).  One thread per 16-bit word
@@ -507,8 +508,12 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_exp_kernel(int n, int p
     sum = block_sum_f64(sum, red);
     if (threadIdx.x == 0) part[SAMPLE_PARTS + blockIdx.x] = sum;
 }
-// Sums over the workgroup's values: of the threads before this one; `all`: of all of them.  red: a double a wavefront
-__device__ __forceinline__ double sample_before(double v, double *red, double *all) {
+// Running sums over the workgroup's values: in front of this thread's and behind it (draw.h: a thread's end is the next one's lower, bit for bit); all: behind
+// the last.  red: a double a wavefront
+struct SampleEnds {
+    double lower, end, all;
+};
+__device__ __forceinline__ SampleEnds sample_ends(double v, double *red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     double x = v;
 #pragma unroll
@@ -516,23 +521,36 @@ __device__ __forceinline__ double sample_before(double v, double *red, double *a
         const double o = __shfl_up(x, d, WAVE);
         x += lane >= d ? o : 0.0;
     }
+    const double up = __shfl_up(x, 1, WAVE);
     __syncthreads();
     if (lane == 63) red[wave] = x;
     __syncthreads();
-    double before = 0.0, sum = 0.0;
+    double base = 0.0, all = 0.0;
     for (int w = 0; w < nw; w++) {
-        before += w < wave ? red[w] : 0.0;
-        sum += red[w];
+        if (w == wave) base = all;
+        all += red[w];
     }
-    *all = sum;
-    return before + (x - v);
+    return {base + (lane ? up : 0.0), base + x, all};
+}
+// the thread that takes a draw of such sums; s_own: two words of LDS that nobody else uses
+__device__ __forceinline__ void sample_owner_clear(int *s_own) {  // (by one thread, a barrier before sample_owner)
+    s_own[0] = 0x7FFFFFFF;
+    s_own[1] = -1;
+}
+__device__ __forceinline__ int sample_owner(double own, double end, double target, int *s_own) {
+    const int wave0 = threadIdx.x & ~63;
+    const unsigned long long weight = __ballot(own > 0.0), reach = __ballot(draw_reaches(own, end, target));
+    if ((threadIdx.x & 63) == 0 && reach) atomicMin(s_own, wave0 + __ffsll(reach) - 1);
+    if ((threadIdx.x & 63) == 0 && weight) atomicMax(s_own + 1, wave0 + 63 - __clzll((long long)weight));
+    __syncthreads();
+    return s_own[0] == 0x7FFFFFFF ? s_own[1] : s_own[0];
 }
 __device__ __forceinline__ float sample_load(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// Probabilities and their sums; then, by the workgroup that is through last (count: zero between launches), the pick: the first index at which the running
-// sum reaches u times the whole (the last one of its run if rounding leaves the target just above the total).
+// Probabilities and their sums; then, by the workgroup that is through last (count: zero between launches), the pick: the run that the target, u times the
+// whole, lies in, then the element.
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int per, int parts, float u, float *p, double *part, unsigned *count, int32_t *out) {
-    __shared__ double red[SAMPLE_THREADS / 64], s_before;
-    __shared__ int s_last, s_at, s_pick;
+    __shared__ double red[SAMPLE_THREADS / 64], s_lower;
+    __shared__ int s_last, s_run[2], s_own[2];
     const int t = threadIdx.x;
     {
         const SampleRun r = sample_run(n, per, blockIdx.x);
@@ -552,42 +570,29 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int 
     if (t == 0) {
         s_last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)parts - 1u;
         if (s_last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_at = s_pick = 0x7FFFFFFF;
+        sample_owner_clear(s_run);
+        sample_owner_clear(s_own);
     }
     __syncthreads();
     if (!s_last) return;
     const double v = t < parts ? __hip_atomic_load(part + 2 * SAMPLE_PARTS + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-    double all;
-    const double before = sample_before(v, red, &all), target = (double)u * all;
-    // (runs are not empty)
-    if (t < parts && ((before < target && (target <= before + v || t == parts - 1)) || (t == 0 && target <= 0.0)))
-        atomicMin(&s_at, t);  // (rounding may leave a running sum a last bit below the one before it)
-    __syncthreads();
-    if (s_at == 0x7FFFFFFF) {  // (the probabilities are not numbers: one of the logits was none, or was not finite once divided)
+    const SampleEnds runs = sample_ends(v, red);
+    const double target = (double)u * runs.all;
+    if (!(runs.all > 0.0)) {  // (the probabilities are not numbers: one of the logits was none, or was not finite once divided)
         if (t == 0) *out = -1;
         return;
     }
-    if (t == s_at) s_before = before;
-    const SampleRun r = sample_run(n, per, s_at);
+    const int at = sample_owner(v, runs.end, target, s_run);
+    if (t == at) s_lower = runs.lower;
+    const SampleRun r = sample_run(n, per, at);
     const int each = (per + SAMPLE_THREADS - 1) / SAMPLE_THREADS, lo = min(r.hi, r.lo + t * each), hi = min(r.hi, lo + each);
     double mine = 0.0;
     for (int i = lo; i < hi; i++) mine += (double)sample_load(p + i);
-    const double ahead = sample_before(mine, red, &all) + s_before;  // (behind its barriers)
-    const bool last = hi == r.hi && lo < hi;
-    if (lo < hi && (ahead < target || t == 0) && (target <= ahead + mine || last)) {
-        double cw = ahead;
-        int pick = hi - 1;
-        for (int i = lo; i < hi; i++) {
-            cw += (double)sample_load(p + i);
-            if (cw >= target) {
-                pick = i;
-                break;
-            }
-        }
-        atomicMin(&s_pick, pick);
-    }
-    __syncthreads();
-    if (t == 0) *out = s_pick;
+    const SampleEnds own = sample_ends(mine, red);  // (s_lower is behind its barriers)
+    if (t != sample_owner(mine, s_lower + own.end, target, s_own)) return;
+    DrawWalk walk(s_lower + own.lower, target);
+    for (int i = lo; i < hi; i++) walk.next(i, sample_load(p + i));
+    *out = target > 0.0 ? walk.pick : 0;  // (u = 0 is reached by the first of all)
 }
 
 // the same for up to SAMPLE_ONE logits, four a thread
@@ -595,7 +600,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_prob_kernel(int n, int 
 __global__ __launch_bounds__(1024) void sample_one_kernel(const float *logits, int n, float temperature, float u, float *p, int32_t *out) {
     __shared__ float redf[16];
     __shared__ double red[16];
-    __shared__ int s_pick;
+    __shared__ int s_own[2];
     const int t = threadIdx.x, i0 = 4 * t;
     float v[4], mx = -INFINITY;
 #pragma unroll
@@ -616,7 +621,7 @@ __global__ __launch_bounds__(1024) void sample_one_kernel(const float *logits, i
         sum += (double)e;
     }
     const float sf = (float)block_sum_f64(sum, red);
-    double own = 0.0, all;
+    double own = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         v[k] /= sf;
@@ -624,28 +629,19 @@ __global__ __launch_bounds__(1024) void sample_one_kernel(const float *logits, i
         p[i0 + k] = v[k];
         own += (double)v[k];
     }
-    if (t == 0) s_pick = 0x7FFFFFFF;
-    const double before = sample_before(own, red, &all), target = (double)u * all;
-    if (!(target <= all)) {  // (not numbers)
+    if (t == 0) sample_owner_clear(s_own);
+    const SampleEnds ends = sample_ends(own, red);
+    const double target = (double)u * ends.all;
+    if (!(ends.all > 0.0)) {  // (not numbers)
         if (t == 0) *out = -1;
         return;
     }
-    if (i0 < n && (before < target || t == 0) && (target <= before + own || i0 + 4 >= n)) {
-        double cw = before;
-        int pick = min(i0 + 3, n - 1);
-        bool there = false;
+    if (t != sample_owner(own, ends.end, target, s_own)) return;
+    DrawWalk walk(ends.lower, target);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            cw += i0 + k < n ? (double)v[k] : 0.0;
-            if (!there && i0 + k < n && cw >= target) {
-                pick = i0 + k;
-                there = true;
-            }
-        }
-        atomicMin(&s_pick, pick);
-    }
-    __syncthreads();
-    if (t == 0) *out = s_pick;
+    for (int k = 0; k < 4; k++)
+        if (i0 + k < n) walk.next(i0 + k, v[k]);
+    *out = target > 0.0 ? walk.pick : 0;
 }
 
 hipError_t k_sample(hipStream_t s, const float *logits, int n, float temperature, float u, float *p, double *part, unsigned *count, int32_t *out) {

@@ -6,6 +6,7 @@
 #include "../../llama2.jl_amd/csrc/k_flow.hip"
 #include "../../llama2.jl_amd/csrc/synth.cpp"
 #include "../../llama2.jl_amd/csrc/delta_plan.h"
+#include "../../llama2.jl_amd/csrc/draw.h"
 #include "../../llama2.jl_amd/csrc/host_box.h"
 #include "../../llama2.jl_amd/csrc/rows_plan.h"
 #include "../../llama2.jl_amd/csrc/tiles_plan.h"
@@ -392,7 +393,85 @@ static void check_tiles_plan() {
         }
 }
 
+// a draw's running sums as a workgroup of the draw kernels forms them: in wavefronts by doubling distances, then wavefront by wavefront
+struct DrawSums {
+    std::vector<double> own, lower, end;
+    double all = 0.0;
+    explicit DrawSums(const std::vector<double> &v) : own(v), lower(v.size()), end(v.size()) {
+        for (size_t w0 = 0; w0 < v.size(); w0 += 64) {
+            double x[64], y[64];
+            for (int l = 0; l < 64; l++) x[l] = v[w0 + l];
+            for (int d = 1; d < 64; d *= 2) {
+                for (int l = 0; l < 64; l++) y[l] = x[l] + (l >= d ? x[l - d] : 0.0);
+                for (int l = 0; l < 64; l++) x[l] = y[l];
+            }
+            for (int l = 0; l < 64; l++) {
+                lower[w0 + l] = all + (l ? x[l - 1] : 0.0);
+                end[w0 + l] = all + x[l];
+            }
+            all += x[63];
+        }
+    }
+    int owner(double target) const {
+        int first = -1, last = -1;
+        for (int t = 0; t < (int)own.size(); t++) {
+            if (own[t] > 0.0) last = t;
+            if (first < 0 && draw_reaches(own[t], end[t], target)) first = t;
+        }
+        return first < 0 ? last : first;
+    }
+};
+// Every target has an owner and a pick that has weight: at every border between two threads and the numbers beside it, with probabilities of the same size,
+// of very different sizes and many of zero.  The pick is where the running sum in order reaches the target, within what two orders of the sum can differ by.
+static void check_draw() {
+    unsigned long long seed = 12345;
+    auto uniform = [&] { return (double)((seed = seed * 6364136223846793005ull + 1442695040888963407ull) >> 40) / 16777216.0; };
+    for (int round = 0; round < 24; round++) {
+        const int n = round % 3 == 0 ? 4096 : round % 3 == 1 ? 8 : 1000 + (int)(3000 * uniform());
+        std::vector<float> p(n);
+        double sum = 0.0;
+        for (float &v : p) {
+            const double z = round % 4 == 0 ? 6 * uniform() : round % 4 == 1 ? 60 * uniform() : uniform() < 0.6 ? 200.0 : 20 * uniform();
+            v = (float)exp(-z);
+            sum += (double)v;
+        }
+        if (round == 1) {  // logits -37.82 four times, 0, -200 three times
+            for (int i = 0; i < 8; i++) p[i] = i < 4 ? (float)exp(-37.82) : i == 4 ? 1.0f : 0.0f;
+            sum = 1.0;
+        }
+        for (float &v : p) v /= (float)sum;
+        std::vector<double> own(1024, 0.0), cum(n + 1, 0.0);
+        for (int i = 0; i < n; i++) {
+            own[i / 4] += (double)p[i];
+            cum[i + 1] = cum[i] + (double)p[i];
+        }
+        const DrawSums s(own);
+        for (int t = 0; t + 1 < 1024; t++) EXPECT(s.end[t] == s.lower[t + 1]);
+        const double slack = 1024 * 2.3e-16 * s.all;
+        for (int t = 0; 4 * t < n; t++)
+            for (int k = 0; k < 8; k++) {
+                // (below and above the thread's two ends, what the difference of its end and its own sum comes to, and a number inside)
+                const double at = k < 3 ? s.end[t] : k < 6 ? s.end[t] - own[t] : s.lower[t] + uniform() * own[t];
+                const double target = k % 3 == 1 ? nextafter(at, 0.0) : k % 3 == 2 ? nextafter(at, 2.0) : at;
+                if (!(target > 0.0 && target <= s.all)) continue;
+                const int owner = s.owner(target);
+                EXPECT(owner >= 0 && 4 * owner < n);
+                if (owner < 0 || 4 * owner >= n) return;
+                DrawWalk walk(s.lower[owner], target);
+                for (int i = 4 * owner; i < std::min(n, 4 * owner + 4); i++) walk.next(i, p[i]);
+                EXPECT(p[walk.pick] > 0.0f && cum[walk.pick] <= target + slack && cum[walk.pick + 1] >= target - slack);
+            }
+    }
+    // the example: the target lies above the end of the first four and far below the rest
+    std::vector<double> v(1024, 0.0);
+    for (int i = 0; i < 4; i++) v[0] += (double)(float)exp(-37.82);
+    v[1] = 1.0;
+    const DrawSums s(v);
+    EXPECT(s.owner((double)2e-16f * s.all) == 1 && s.owner(1.5e-16) == 0);
+}
+
 int main() {
+    check_draw();
     check_tiles_plan();
     check_small_plan();
     check_product_rule();
