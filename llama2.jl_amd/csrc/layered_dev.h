@@ -59,10 +59,13 @@ __device__ __forceinline__ float l_act_rounded(int act, float z) {
 }
 
 // 1 / sqrt(x) within a unit in the last place: the hardware's with a step of Newton's method.  (1 / sqrtf(x), with its exact root and quotient, is forty
-// instructions in a row, which a launch of a decode step also has to fetch: 0.1 us of 3.)
+// instructions in a row, which a launch of a decode step also has to fetch: 0.1 us of 3.)  The hardware takes numbers below 2^-126 for zero: small ones go in
+// 2^32 times as large, which is exact.
 __device__ __forceinline__ float l_rsqrt(float x) {
-    const float y = __builtin_amdgcn_rsqf(x), e = fmaf(-x * y, y, 1.0f), z = fmaf(0.5f * y, e, y);
-    return e == e ? z : y;  // (0 and infinity as they are)
+    const bool small = x < 0x1p-100f;
+    const float v = small ? x * 0x1p32f : x;
+    const float y = __builtin_amdgcn_rsqf(v), e = fmaf(-v * y, y, 1.0f), z = fmaf(0.5f * y, e, y), r = e == e ? z : y;  // (0 and infinity as they are)
+    return small ? r * 0x1p16f : r;
 }
 
 // v plus its value in another lane of the same sixteen

@@ -40,3 +40,28 @@ def test_head_norm(pkg, heads, vdim):
     c = lc.config([lc.delta(heads=heads, kv_heads=1, dim=20, vdim=vdim, conv=2, ranks=(8, 8))])
     t = layered_np.random_tensors(c, 4)
     _steps(lc.language_model(pkg, c, t).device(), layered_np, c, t)
+
+
+@pytest.mark.parametrize("design,tiny", [
+    ("vudelix", "embed"),         # the norm in front of a layer's first product
+    ("vudelix", "l0.mix.q"),      # a query's norm
+    ("vudelix", "l0.side.proj"),  # a pending update's norm
+    ("lezepel", "embed"),
+    ("lezepel", "l0.mix.dq"),     # norms inside latent attention
+    ("lezepel", "l0.mix.dkv"),
+])
+def test_norms_of_vectors_whose_squares_are_denormal(pkg, design, tiny):
+    """norm_eps 0 and vectors of 2^-66: their mean squares are fp32 numbers below 2^-126, of 17 bits, each rounded by 2^-18 at most, so that the root of
+    their mean is off by far less than the tolerance.  (Not of a delta rule's heads, whose outputs differ by more than that range.)"""
+    if design == "vudelix":
+        c = lc.config([lc.attention()], eps=0.0, side=40 if "side" in tiny else 0)
+        cases, ref = lc, layered_np
+    else:
+        c = zc.config([zc.layer()], eps=0.0, scale=1.0)
+        cases, ref = zc, lezepel_np
+    t = {k: np.array(v) for k, v in ref.random_tensors(c, 6).items()}
+    t[tiny] = t[tiny] * 2.0 ** -66
+    if tiny == "l0.mix.dkv":  # (only the compressed keys and values: the rotated part's scale is in the scores)
+        rank = t["l0.mix.dkv.norm"].size
+        t[tiny][rank:] *= 2.0 ** 66
+    _steps(cases.language_model(pkg, c, t).device(), ref, c, t)
