@@ -95,9 +95,8 @@ static hipError_t rows_pick(hipStream_t s, const RowsArgs &a, int n_cu, const Ro
 
 hipError_t k_rows(hipStream_t s, const RowsArgs &a, int pro, int epi, int n_cu, const RowsMore &more) {
     if (!a.w || !a.x || !a.out || a.n_rows < 1 || a.n_rows > 0x7FFFFFFF || a.ld % 64 != 0 || a.K > a.ld || a.K < 1) return hipErrorInvalidValue;
-    if ((pro == RP_UP || pro == RP_DOWN) &&
-        (!a.z || a.n_experts < 1 || a.n_experts > ROWS_MAX_EXPERTS || a.top < 1 || a.top > ROWS_MAX_TOP || a.top > a.n_experts ||
-                                           a.n_experts * a.rows_each > 0x7FFFFFFF))
+    if ((pro == RP_UP || pro == RP_DOWN) && (!a.z || !a.sel || a.n_experts < 1 || a.n_experts > ROWS_MAX_EXPERTS || a.top < 1 || a.top > ROWS_MAX_TOP ||
+                                             a.top > a.n_experts || a.n_experts * a.rows_each > 0x7FFFFFFF))
         return hipErrorInvalidValue;
     if ((epi == RE_GLU && a.n_rows % 2 != 0) || (epi == RE_STORE_GLU && (a.n_rows % 2 != 0 || a.glu_from % 2 != 0 || !a.out2)))
         return hipErrorInvalidValue;

@@ -378,7 +378,7 @@ hipError_t k_step_pair(hipStream_t s, const LatentStep &a, const RowsArgs &uq, c
     const int64_t n = step_grid(up, pro, n_cu, u, n_first);
     const RowsPlan pl = rows_plan(up, pro, u, n);
     const size_t lds = std::max(sizeof(StepLds), std::max(rows_lds(uq, RP_NORM, plq.pairs + 1), rows_lds(up, pro, pl.pairs + 1)));
-    if (lds > 64 * 1024 || up.n_rows % 2 != 0) return hipErrorInvalidValue;
+    if (lds > 64 * 1024 || up.n_rows % 2 != 0 || (pro == RP_UP && !up.sel)) return hipErrorInvalidValue;
 #define GO(P, U_)                                                                                                                               \
     if (pro == P && u == U_) {                                                                                                                  \
         hipLaunchKernelGGL((step_pair_kernel<P, U_>), dim3((unsigned)(n_first + n)), dim3(ROWS_THREADS), lds, s, a, uq, plq, each, up, pl, n_first);\
@@ -400,7 +400,7 @@ hipError_t k_step_latent(hipStream_t s, const LatentStep &a, const RowsArgs &dow
     RowsMore m;
     m.stride = stride ? stride : down.ld;
     const size_t lds = std::max(sizeof(StepLds), rows_lds(down, pro, pl.pairs + 1));
-    if (lds > 64 * 1024) return hipErrorInvalidValue;
+    if (lds > 64 * 1024 || (pro == RP_DOWN && !down.sel)) return hipErrorInvalidValue;
 #define GO(P, U_)                                                                                                                        \
     if (pro == P && u == U_) {                                                                                                           \
         hipLaunchKernelGGL((step_latent_kernel<P, U_>), dim3((unsigned)(n_first + n)), dim3(ROWS_THREADS), lds, s, a, down, pl, m, n_first); \

@@ -57,7 +57,7 @@ struct RowsArgs {
     const float *ssq = nullptr, *gate = nullptr;  // RP_HEADNORM
     int hv = 0, n_split = 0;
     const uint16_t *emb = nullptr;  // RE_EMBED
-    int32_t *sel = nullptr;         // RP_UP leaves the chosen experts there, RP_DOWN finds them (or chooses for itself)
+    int32_t *sel = nullptr;         // RP_UP leaves the chosen experts there, RP_DOWN finds them
 };
 // What few products of a residual have.  Apart, for the sake of the others: with these fields and their branches in every launch a token of Vudelix took 1 % longer
 // (width 768, 4 layers: 170.6 us against 169.2).

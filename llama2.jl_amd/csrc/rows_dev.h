@@ -108,7 +108,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     __shared__ float s_red[2][ROWS_WAVES];
     __shared__ float s_part[ROWS_WAVES][2];
     __shared__ int s_head[ROWS_WAVES];  // the pair that s_part belongs to
-    __shared__ int s_sel[ROWS_WAVES][ROWS_MAX_TOP];  // (a choice by the wavefronts, each for itself, has a row for each)
+    __shared__ int s_sel[PRO == RP_UP ? ROWS_WAVES : 1][ROWS_MAX_TOP];  // (a choice by the wavefronts, each for itself, has a row for each)
     __shared__ float s_score[ROWS_MAX_TOP];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int K = a.K, ld = a.ld, plane = pl.plane;
@@ -128,8 +128,8 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     DecodeCtl ctl;
     if (EPI == RE_STORE_KEY && b == 0) ctl = *keys.ctl;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    constexpr bool choice = PRO == RP_UP || PRO == RP_DOWN;
-    const bool chosen = PRO == RP_DOWN && a.sel, by_wave = choice && !chosen && a.n_experts <= 64;
+    constexpr bool choice = PRO == RP_UP, chosen = PRO == RP_DOWN;  // (of experts: made here, or handed on in a.sel)
+    const bool by_wave = choice && a.n_experts <= 64;
     float z = -INFINITY, zb = 0.0f;  // an expert a lane
     int rank = 0;
     if (by_wave && lane < a.n_experts) {
@@ -231,8 +231,8 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     fetch(cur, k);
     asm volatile("" ::: "memory");
     if (chosen) sel = s_sel[0];
-    if (by_wave && PRO == RP_UP && wave == 0) rows_scores(z, rank, a.top, a.route, s_score, lane);
-    if (PRO == RP_UP && a.sel && b == 0 && t < a.top) a.sel[t] = s_sel[0][t];  // (the first wavefront's own choice, or behind a barrier)
+    if (by_wave && wave == 0) rows_scores(z, rank, a.top, a.route, s_score, lane);
+    if (choice && b == 0 && t < a.top) a.sel[t] = s_sel[0][t];  // (the first wavefront's own choice, or behind a barrier)
     if (lane == 0) s_head[wave] = -1;
 
     // ---- the vector -------------------------------------------------------------------------------------------

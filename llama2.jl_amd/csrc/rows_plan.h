@@ -14,7 +14,7 @@ inline int rows_vectors(const RowsArgs &a, int pro) { return pro == RP_DOWN ? a.
 
 // LDS of a workgroup of `pairs` row pairs: the vectors, then the results, where the choice of experts has its logits before
 inline size_t rows_lds(const RowsArgs &a, int pro, int64_t pairs) {
-    return ((size_t)rows_vectors(a, pro) * a.ld + std::max<size_t>(2 * (size_t)pairs, pro == RP_UP || pro == RP_DOWN ? a.n_experts : 0)) * sizeof(float);
+    return ((size_t)rows_vectors(a, pro) * a.ld + std::max<size_t>(2 * (size_t)pairs, pro == RP_UP ? a.n_experts : 0)) * sizeof(float);
 }
 
 // steps of 512 u inputs (rows_kernel) in all
