@@ -22,10 +22,14 @@ inline int64_t rows_steps(const RowsArgs &a, int pro, int u) {
     return (a.n_rows + 1) / 2 * rows_vectors(a, pro) * ((a.ld + 512 * u - 1) / (512 * u));
 }
 
+// LDS of a workgroup beside rows_lds(), rounded up: sums, and behind a choice of experts each wavefront's own (2464 bytes; 352 and fewer otherwise)
+inline size_t rows_fixed_lds(int pro) { return (pro == RP_UP ? 3 : 2) * 1024; }
+
 // two workgroups per CU where LDS holds their vectors and results
 inline int64_t rows_most(const RowsArgs &a, int pro, int n_cu) {
     const int64_t pairs = (a.n_rows + 1) / 2;
-    return (rows_lds(a, pro, std::min<int64_t>(ROWS_MAX_PAIRS, pairs / (2 * n_cu) + 1)) > 78 * 1024 ? 1 : 2) * (int64_t)n_cu;
+    const size_t lds = rows_lds(a, pro, std::min<int64_t>(ROWS_MAX_PAIRS, pairs / (2 * n_cu) + 1)) + rows_fixed_lds(pro);
+    return (lds > 80 * 1024 ? 1 : 2) * (int64_t)n_cu;
 }
 
 // workgroups: no more than that while there is a step for every wavefront and, beside the vectors, LDS for the results

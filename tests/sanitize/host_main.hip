@@ -193,6 +193,16 @@ static void check_rows_plan() {
                             EXPECT(n >= 1 && n <= pairs && rows_lds(a, pro, pairs / n + 1) <= ROWS_LDS);
                         }
                     }
+    // a grid made for two workgroups a CU has two there: the kernels' own LDS, as the compiler lays it out (96 bytes, 352 with a choice that is handed on, 2464
+    // with one made), comes on top of the vectors and results, in whole units of 1280 bytes
+    for (int pro : {RP_PLAIN, RP_NORM, RP_UP, RP_DOWN})
+        for (int K = 18432; K <= 20480; K += 64)
+            for (int64_t rows : {(int64_t)1024, (int64_t)40000, (int64_t)262144}) {
+                RowsArgs a;
+                a.K = a.ld = K, a.n_rows = rows, a.top = 1, a.n_experts = 8;
+                const size_t own = pro == RP_UP ? 2464 : pro == RP_DOWN ? 352 : 224, lds = rows_lds(a, pro, (rows + 1) / 2 / 512 + 1) + own;
+                if (rows_most(a, pro, 256) == 512) EXPECT(2 * ((lds + 1279) / 1280) * 1280 <= 160 * 1024);
+            }
 }
 
 // quotients without a division, where rounding could show: around multiples, over all of the range
