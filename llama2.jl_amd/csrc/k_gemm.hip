@@ -580,11 +580,11 @@ __device__ __forceinline__ int group_scan(int v, int lane) {
     const int a = __builtin_amdgcn_readlane(v, 15), b = __builtin_amdgcn_readlane(v, 31), c = __builtin_amdgcn_readlane(v, 47);
     return v + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
 }
-// What the lists of blocks are made of: blocks of tile_rows (IMAGES: of tiles_plan.h's units, with a bound for each of two products)
+// What the lists of blocks are made of: blocks of tile_rows (IMAGES: of tiles_plan.h's units, with a rule for each of two products)
 struct GroupLists {
     GemmTile *tiles[2];
     int tile_rows;
-    unsigned bound[2];
+    TilesRule rule[2];
 };
 template <bool IMAGES>
 __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
@@ -609,13 +609,37 @@ __global__ __launch_bounds__(1024) void group_kernel(const int32_t *choice, cons
         if (t + 1024 * u < n) rank[u] = atomicAdd(&cnt[c[u]], 1);
     for (int i = t + 1024 * GROUP_Q; i < n; i += 1024) slot_of[i] = atomicAdd(&cnt[choice[i]], 1);
     __syncthreads();
+    // each product's bound, or whole tiles: four wavefronts add up one product's blocks of one kind each
+    unsigned bound[NP];
+    if constexpr (IMAGES) {
+        __shared__ float s_time[4];
+        const bool ask = lists.rule[0].n_cu | lists.rule[1].n_cu;
+        if (ask) {
+            const int w = __builtin_amdgcn_readfirstlane(wave);
+            if (w < 4) {
+                const TilesRule r = lists.rule[w & 1];
+                int blocks = 0, weight = 0;
+                for (int e = lane; e < E; e += 64) {
+                    const TilesSplit v = tiles_split((unsigned)(cnt[e] + TILES_UNIT - 1) / TILES_UNIT, w < 2 ? r.bound : TILES_WHOLE_UNITS);
+                    blocks += (int)v.blocks;
+                    weight += (int)v.weight;
+                }
+                blocks = group_scan(blocks, lane);
+                weight = group_scan(weight, lane);
+                if (lane == 63) s_time[w] = r.n_cu ? tiles_rounds(r, (unsigned)blocks, (unsigned)weight) : 0.0f;
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int p = 0; p < NP; p++) bound[p] = ask && s_time[2 + p] < s_time[p] ? TILES_WHOLE_UNITS : lists.rule[p].bound;
+    }
     // rows and blocks of the experts before e (E <= 1024: a thread for each)
     const int rows = t < E ? cnt[t] : 0;
     const unsigned units = (unsigned)(rows + TILES_UNIT - 1) / TILES_UNIT;
     int nt[NP];
     if constexpr (IMAGES) {
 #pragma unroll
-        for (int p = 0; p < NP; p++) nt[p] = (int)tiles_blocks(units, lists.bound[p]);
+        for (int p = 0; p < NP; p++) nt[p] = (int)tiles_blocks(units, bound[p]);
     } else {
         nt[0] = (rows + lists.tile_rows - 1) / lists.tile_rows;
     }
@@ -671,9 +695,9 @@ hipError_t k_group(hipStream_t s, const int32_t *choice, const float *score, int
     return hipGetLastError();
 }
 hipError_t k_group_images(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row, float *slot_scale,
-                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const unsigned bound[2]) {
-    if (E < 1 || E > 1024 || M < 1 || top < 1 || bound[0] < 1 || bound[0] > TILES_MAX_UNITS || bound[1] < 1 || bound[1] > TILES_MAX_UNITS) return hipErrorInvalidValue;
-    const GroupLists l = {{tiles[0], tiles[1]}, 0, {bound[0], bound[1]}};
+                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const TilesRule rule[2]) {
+    if (E < 1 || E > 1024 || M < 1 || top < 1 || rule[0].bound < 1 || rule[0].bound > TILES_MAX_UNITS || rule[1].bound < 1 || rule[1].bound > TILES_MAX_UNITS) return hipErrorInvalidValue;
+    const GroupLists l = {{tiles[0], tiles[1]}, 0, {rule[0], rule[1]}};
     hipLaunchKernelGGL(group_kernel<true>, dim3(1), dim3(1024), 2 * E * sizeof(int), s, choice, score, M, E, top, slot_row, slot_scale, slot_of, n_tiles, l);
     return hipGetLastError();
 }

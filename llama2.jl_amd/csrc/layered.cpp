@@ -1349,7 +1349,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
     down.n_rows = l->W();
     GemmTile *const lists[2] = {l->tiles, l->tiles2};
     GemmArgs *const products[2] = {&up, &down};
-    unsigned bound[2];
+    TilesRule rule[2];
     bool few[2];
     for (int p = 0; p < 2; p++) {
         GemmArgs &a = *products[p];
@@ -1358,11 +1358,11 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
         a.rows_each = slots / d.n_experts;
         few[p] = image && k_few_experts_pays(d.n_experts, a.n_rows, a.ld, a.rows_each);
         a.few = few[p];
-        bound[p] = few[p] ? 1 : tiles_bound(slots, d.n_experts, (unsigned)((a.n_rows + 255) / 256), (unsigned)a.ld >> 6, (unsigned)cu);
-        a.max_tiles = image ? (int)tiles_most(slots, d.n_experts, bound[p]) : (slots + L_GEMM_TILE - 1) / L_GEMM_TILE + d.n_experts;
+        rule[p] = few[p] ? TilesRule{1, 0, 0, 0} : tiles_rule(slots, d.n_experts, (unsigned)((a.n_rows + 255) / 256), (unsigned)a.ld >> 6, (unsigned)cu);
+        a.max_tiles = image ? (int)tiles_most(slots, d.n_experts, rule[p]) : (slots + L_GEMM_TILE - 1) / L_GEMM_TILE + d.n_experts;
     }
     if (image)
-        CK(k_group_images(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, lists, l->n_tiles, bound));
+        CK(k_group_images(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, lists, l->n_tiles, rule));
     else
         CK(k_group(s, l->choice, l->score, M, d.n_experts, d.top, l->slot_row, l->slot_scale, l->slot_of, l->tiles, l->n_tiles, L_GEMM_TILE));
     const int epi = d.ff_gated ? GE_GLU : GE_UP;

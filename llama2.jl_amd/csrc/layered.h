@@ -191,9 +191,9 @@ hipError_t k_route(hipStream_t s, const float *z, int64_t ldz, const float *bias
                    float *score);
 hipError_t k_group(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row,
                    float *slot_scale, int32_t *slot_of, GemmTile *tiles, int32_t *n_tiles, int tile_rows);
-// with a list of blocks for each of two products from tile images, of at most bound[p] units (tiles_plan.h): tiles[p], n_tiles[p]
+// with a list of blocks for each of two products from tile images, by rule[p] (tiles_plan.h): tiles[p], n_tiles[p]
 hipError_t k_group_images(hipStream_t s, const int32_t *choice, const float *score, int M, int E, int top, int32_t *slot_row, float *slot_scale,
-                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const unsigned bound[2]);
+                          int32_t *slot_of, GemmTile *const tiles[2], int32_t *n_tiles, const TilesRule rule[2]);
 // x[m] += mult * sum_k y[slot_of[m][k]]
 hipError_t k_gather_add(hipStream_t s, float *x, const float *y, const int32_t *slot_of, int M, int top, int K, float mult);
 // x[m] += a[m] + b, a or not

@@ -101,9 +101,32 @@ inline unsigned tiles_bound(int64_t rows, int experts, unsigned n_nt, unsigned s
         if (tiles_time((double)rows, experts, b, n_nt, steps, n_cu) < tiles_time((double)rows, experts, best, n_nt, steps, n_cu)) best = b;
     return best;
 }
+// The bound is made for experts that have about as many rows each.  Where it is more than one, the launch that counts the rows compares it with blocks of whole tiles,
+// by the blocks that there really are: few experts may take most.  us, that bound, with this, and blocks of 256 as they come; 16 experts of which two take every one of
+// 500 positions, 3584 x 3584 134, 108, 108; four every one of 2000, 2048 x 2048 73, 62, 65, 3584 x 3584 208, 175, 181, 4096 x 4096 232, 195, 203; one of them, 4096 x
+// 4096 325, 292, 303; the counting launch 3.4 and 8.7 to 4.1 and 9.4.  (Over 7 shapes, 130 to 2000 positions and 1 to 4 such experts 2 % above blocks of 256 at most, 0.64 to
+// 0.79 of their time in the mean; a bound of one is never the slower of those.)
+#define TILES_WHOLE_UNITS 4
+struct TilesRule {
+    unsigned bound, n_nt, steps, n_cu;  // n_cu 0: the bound, whatever the blocks
+};
+// rounds of the blocks, each of the time of the mean block
+__host__ __device__ inline float tiles_rounds(const TilesRule &r, unsigned blocks, unsigned weight) {
+    return (float)tiles_quot(blocks * r.n_nt + r.n_cu - 1, r.n_cu) * (180.0f + (float)(r.steps * weight) / (float)blocks);
+}
+
 // and the most blocks that there can be
 inline int64_t tiles_most(int64_t rows, int experts, unsigned b) {
     return ((rows + TILES_UNIT - 1) / TILES_UNIT + experts) / b + experts;
+}
+
+// of a rule that may come to either
+inline int64_t tiles_most(int64_t rows, int experts, const TilesRule &r) { return tiles_most(rows, experts, r.n_cu ? std::min(r.bound, (unsigned)TILES_WHOLE_UNITS) : r.bound); }
+inline TilesRule tiles_rule(int64_t rows, int experts, unsigned n_nt, unsigned steps, unsigned n_cu) {
+    TilesRule r = {tiles_bound(rows, experts, n_nt, steps, n_cu), n_nt, steps, n_cu};
+    const int64_t most = tiles_most(rows, experts, 1);
+    if (r.bound == 1 || r.bound == TILES_WHOLE_UNITS || most * n_nt + n_cu >= (1 << 21) || most * 25 * steps >= ((int64_t)1 << 31)) r.n_cu = 0;
+    return r;
 }
 
 // A single product's positions in the same kind of blocks, every row group's alike: the bound for them and what they may take

@@ -41,3 +41,30 @@ def test_blocks(pkg, kind, n, experts, top, rows):
     for lo in range(0, n, 64):  # (every part by itself: a block left out is not to hide in the mean)
         assert lc.error(got[True][lo:lo + 64], want[lo:lo + 64]) <= TOL, lo
         assert lc.error(got[True][lo:lo + 64], got[False][lo:lo + 64]) <= SAME, lo
+
+
+# (positions, experts, chosen, rows of an expert's up product): the same few experts take every position, so that blocks of whole tiles are chosen where the
+# experts' mean asks for blocks of 128, with a thread an expert in one wavefront or in two
+@pytest.mark.parametrize("n,experts,top,rows", [(700, 24, 3, 4096), (700, 65, 8, 2048)])
+def test_few_experts_take_all(pkg, n, experts, top, rows):
+    c = zc.config([zc.layer(heads=2, dim=12, rot_dim=4, vdim=16, kv_rank=20, q_rank=24, mlp=zc.moe(experts, top, rows // 2))], width=200, vocab=50, scale=1.0)
+    t = zc.settle_routers(c, lezepel_np.random_tensors(c, 8), 8)
+    bias = t["l0.mlp.router.b"]
+    bias[:] = np.where(np.arange(experts) % (experts // top) == 1, 60.0, 0.0)
+    bias[np.flatnonzero(bias)[top:]] = 0.0
+    bias[bias > 0] += np.arange(top)
+    t["l0.mlp.router.b"] = lezepel_np.bf16(bias)
+    tok = lc.tokens(n, 50, 2)
+    want = lezepel_np.Sequence(c, t).run(tok)
+    got = {}
+    lm = zc.language_model(pkg, c, t, n, "bfloat16")
+    for images in (True, False):
+        lm._device = None
+        dev = lm.device()
+        dev.set_prefill_copy(images)
+        got[images] = dev.prefill_logits(tok, np.arange(n))
+        assert dev.chosen("tile_images") == (2 if images else 0)
+        dev.close()
+    for lo in range(0, n, 64):
+        assert lc.error(got[True][lo:lo + 64], want[lo:lo + 64]) <= TOL, lo
+        assert lc.error(got[True][lo:lo + 64], got[False][lo:lo + 64]) <= SAME, lo
