@@ -3,13 +3,12 @@
 //
 // What bounds such a product is reading the matrix once, so as many wavefronts as possible have a share of it under way.
 //
-// few_kernel (fp32, and bf16 of up to 16 positions): a workgroup takes 16 rows and 16 or 32 positions, its eight wavefronts an eighth of the inputs each, and
+// few_kernel (fp32, and bf16 of up to 16 positions or few inputs): a workgroup takes 16 or 32 rows and 16 to 64 positions, its eight wavefronts an eighth of the inputs each, and
 // their sums are added in LDS, in order.  Operands go from memory straight to the registers that the matrix instructions take (a lane holds 8 consecutive
 // inputs of one row), the next step's under way during this one's; a position's inputs come from the L2.  A load's 16 rows lie a multiple of 4 KB apart, which
 // is what bounds it from 17 positions on.
 //
-// few_ring_kernel (bf16, few_ring.h): whole lines, through LDS.  Microseconds before (few_kernel with up to 32 rows and 64 positions) and now, a matrix of its
-// own in each launch: 64 positions, 16 384 rows x 2048 inputs 30.6, 17.1; 28 672 x 4096 106, 49.9; 4096 x 14 336 81.7, 30.4; 2048 x 8192 24.7, 13.5; 3072 x 2048 14.3,
+// few_ring_kernel (bf16, few_ring.h): whole lines, through LDS.  Microseconds of few_kernel and of this, a matrix of its own in each launch: 64 positions, 16 384 rows x 2048 inputs 30.6, 17.1; 28 672 x 4096 106, 49.9; 4096 x 14 336 81.7, 30.4; 2048 x 8192 24.7, 13.5; 3072 x 2048 14.3,
 // 8.2; a router's 32 rows x 4096, 12.6, 5.3; 16 experts of 2048 x 2048, 14 and 64 positions each: 43, 28.6 and 124, 47.8.
 #include "few_ring.h"
 #include "layered_gemm.h"
@@ -253,6 +252,16 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void few_grouped_kernel(GemmArgs a,
 // So: the smallest tiles that come to at most one a compute unit (of many inputs, where they can be shared out, all positions up to 64 in one tile), and the
 // largest beyond.  Up to 16 positions few_kernel's 16 x 16 results have more workgroups: 2 to 16 positions of 2048 x 2048 5.5 to 6.5 | 6.0 to 6.6, 4096 x 4096 9.2 to
 // 10.3 | 10.4 to 10.6, but 2048 x 8192 13.8 to 17.1 | 10.5 to 10.8 S4, 4096 x 14 336 24.6 to 28.8 | 23.9 to 24.2 S2, 8 of 16 384 x 2048 15.3 | 14.4.
+//
+// All of that is of many inputs.  A tile of the ring costs the fill of its LDS and its epilogue, which nothing hides (one workgroup a compute unit), so with fewer inputs, in steps of 64,
+// it has to be one of a full round.  The ring's time over few_kernel's, worst of four epilogues:
+//   one round: 8 steps and more 0.5 to 1.04.  4 (256 inputs): 2048 rows, 24 to 128 positions 0.85 to 1.02; 4096, 17 and 64 1.06 and 0.86; 8192, 17 and 64 (tiles of 64 rows) 0.98 and
+//     1.00; 8192 and 16 384, 128 and 33 1.10 and 1.16.  6: 4096, 17 1.03, 64 0.81; 8192, 128 0.97; 16 384, 33 1.05.  Below 4, 17 to 128 positions 0.9 to 1.8.
+//   more: 4 to 7 steps 1.0 to 1.4 (32 000 rows, 32 positions 0.96 to 1.04).  8: 16 384 rows, 32 positions 0.90; 20 480 1.14, 28 672 0.97; 33 of 28 672 1.05, 64 0.99.  12: 18 432, 17, 32 and 64
+//     1.19, 1.01 and 0.99; 28 672, 17 0.94.  16: 18 432, 17 and 24 1.10 and 0.98; 24 576, 17 0.97.  24: 18 432, 17 0.99.  From 65 positions on of 12 and more 0.6 to 1.02.
+//   up to 16 positions: 12: 16 384, 5 and 16 1.06 and 0.93.  32: 16 384 rows, 5, 8 and 16 positions 1.01, 0.95 and 0.78; 20 480 1.25, 1.13 and 0.99; 28 672 1.07, 0.97 and 0.82.  64: 1.0, 0.9 and 0.7; 1.12,
+//     1.0 and 0.87; 0.95, 0.85 and 0.70.
+// Steps times the results' share of the rounds' room, against 6.5, is the line that those lie on two sides of.
 struct FewPlan {
     int rows = 0, positions = 0;  // of a tile (0: few_kernel)
     unsigned splits = 1;
@@ -260,7 +269,7 @@ struct FewPlan {
 static FewPlan few_plan(const GemmArgs &a, int64_t cols) {
     FewPlan p;
     const int nk = a.ld / 64;
-    if (nk < 4) return p;  // (wavefronts without a step; 4096 x 128, 120 positions: 3.3 | 3.4, with a decay behind it 4.0 | 4.3)
+    if (nk < 4) return p;
     auto tiles = [&](int rows, int positions) { return (cols + rows - 1) / rows * ((a.M + positions - 1) / positions); };
     if (tiles(32, 32) <= FEW_PART_ITEMS && (a.M <= 32 || nk < 64))
         p.rows = p.positions = 32;
@@ -268,9 +277,17 @@ static FewPlan few_plan(const GemmArgs &a, int64_t cols) {
         p.rows = 32, p.positions = 64;
     else
         p.rows = 64, p.positions = a.M <= 32 ? 32 : 64;
-    if (nk >= 64 && a.part && a.arrived)
-        p.splits = (unsigned)max((int64_t)1, min((int64_t)min(8, nk / 16), FEW_PART_ITEMS / tiles(p.rows, p.positions)));
-    if (a.M <= 16 && !(p.splits >= 4 || (p.splits >= 2 && nk >= 128) || (a.M > 4 && tiles(64, 32) >= FEW_PART_ITEMS))) p.rows = 0;
+    const int64_t n = tiles(p.rows, p.positions), rounds = (n + FEW_PART_ITEMS - 1) / FEW_PART_ITEMS;
+    if (nk >= 64 && a.part && a.arrived) p.splits = (unsigned)max((int64_t)1, min((int64_t)min(8, nk / 16), FEW_PART_ITEMS / n));
+    const bool filled = 2 * nk * cols * a.M >= 13 * rounds * FEW_PART_ITEMS * p.rows * p.positions;
+    bool ring;
+    if (a.M <= 16)
+        ring = p.splits >= 4 || (p.splits >= 2 && nk >= 128) || (n >= FEW_PART_ITEMS && filled);
+    else if (rounds == 1)
+        ring = nk >= 8 || (!(nk < 6 && p.rows == 64) && (a.M > 32 || n > FEW_PART_ITEMS / 2));
+    else
+        ring = nk >= 8 && (filled || a.M > 64);
+    if (!ring) p.rows = 0;
     return p;
 }
 template <int EPI, int TN, int TM>
@@ -292,10 +309,19 @@ static hipError_t few_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
             if constexpr (PREC == 0) {
                 // us, few_grouped_kernel and tiles of 32 and 64 rows; 8 matrices of 512 x 512 (64 tiles of 64 rows), 8, 16 and 48 positions each: 3.6, 4.0, 6.5;
                 // 3.9, 4.0, 6.1; 4.6, 4.8, 7.9; of 2048 x 1024 (256): 11.0, 13.8, 30.4; 11.1, 11.6, 17.8; 9.5, 9.9, 15.0; 16 of 2048 x 2048, 2, 16 and 64 each:
-                // 29.2, 42.9, 124; 27.6, 29.9, 53.9; 27.8, 28.6, 47.8
-                const int64_t wide = a.M / max(a.rows_each, 1) * ((cols + 63) / 64);
-                if (wide >= 192) return few_ring_grouped<EPI, 64>(s, a, cols);
-                if (a.rows_each > 8) return few_ring_grouped<EPI, 32>(s, a, cols);
+                // 29.2, 42.9, 124; 27.6, 29.9, 53.9; 27.8, 28.6, 47.8.
+                // So: 64 rows where that gives most compute units a tile, and as many to each (250 tiles 0.8 to 1.02 of few_grouped_kernel's time, 280 to 340 1.0 to 1.3; of 64 to 192 inputs and
+                // 48 positions each 1.0 to 1.2 with a gate), otherwise 32 rows where the loop is long enough for the fill of the ring and its epilogue.  Their time over
+                // few_grouped_kernel's, 32 to 128 tiles of 64 rows, 9, 16, 32 and 48 positions each, stored: 256 inputs 1.1, 1.05, 1.0 to 1.1, 0.9 to 1.0; 512 1.05, 0.95, 0.8 to 1.0, 0.7
+                // to 0.9; 2048 1.0 to 1.1, 0.75 to 1.0, 0.6 to 0.9, 0.5 to 0.8; with a gate: 512 1.04 to 1.14, 1.0 to 1.1, 1.02 to 1.3, 0.94 to 1.2; 2048 1.1, 0.95 to 1.1, 0.9 to 1.2, 0.7 to 1.06,
+                // the smaller figures at 128 tiles.
+                const int64_t nk = a.ld / 64, each = a.rows_each, wide = few_blocks(a, cols), rounds = (wide + FEW_PART_ITEMS - 1) / FEW_PART_ITEMS;
+                constexpr bool stored = EPI == GE_STORE;
+                if (3 * wide >= 2 * FEW_PART_ITEMS * rounds) {
+                    if (nk >= 4 || each <= 32 || (stored && nk >= 2)) return few_ring_grouped<EPI, 64>(s, a, cols);
+                } else if (stored ? nk >= 6 && nk * each >= 160 : (wide >= 80 && nk * each >= 384) || nk * each >= 1600) {
+                    return few_ring_grouped<EPI, 32>(s, a, cols);
+                }
             }
             const unsigned n_nt = (unsigned)((cols + 15) / 16), most = (unsigned)a.max_tiles * n_nt;
             hipLaunchKernelGGL((few_grouped_kernel<PREC, EPI>), dim3(8 * ((most + 7) / 8)), dim3(64 * FEW_WAVES), 0, s, a, n_nt);
@@ -315,6 +341,9 @@ static hipError_t few_launch(hipStream_t s, const GemmArgs &a, int64_t cols) {
         return hipGetLastError();                                                                                                         \
     } while (0)
     if (a.M <= 16) GO(1, 1);
+    // 32 rows and 64 positions at a time where that gives every CU a workgroup: half the reads of the positions (fp32 products of that size go to k_gemm's tiles)
+    if constexpr (PREC == 0)
+        if (a.M > 32 && ((cols + 31) / 32) * ((a.M + 63) / 64) >= 256) GO(2, 4);
     GO(1, 2);
 #undef GO
 }

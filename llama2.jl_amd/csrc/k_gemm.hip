@@ -405,7 +405,7 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &args, int prec, int epi) {
     GemmArgs a = args;
     if (!a.acols) a.acols = a.lda;
     if (!a.w || !a.x || a.n_rows < 1 || a.M < 1 || a.ld % 64 != 0 || a.ldx < a.ld || a.lda % 64 != 0 || a.acols % 64 != 0 ||
-        a.acols > a.lda)
+        a.acols > a.lda || (a.tiles && a.matrices < 1))
         return hipErrorInvalidValue;
     const bool acts = epi == GE_ACT || epi == GE_UP || epi == GE_EMBED;
     if (epi == GE_GLU ? (!a.outa || a.n_rows % 2 != 0 || 2 * a.acols < a.n_rows)

@@ -1355,6 +1355,7 @@ static hipError_t prompt_experts(l2h_model *m, LayerDev &L, int M) {
         GemmArgs &a = *products[p];
         a.tiles = image ? lists[p] : l->tiles;
         a.n_tiles = image ? l->n_tiles + p : l->n_tiles;
+        a.matrices = d.n_experts;
         a.rows_each = slots / d.n_experts;
         few[p] = image && k_few_experts_pays(d.n_experts, a.n_rows, a.ld, a.rows_each);
         a.few = few[p];

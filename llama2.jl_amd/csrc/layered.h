@@ -116,7 +116,7 @@ struct GemmArgs {
     const int32_t *n_tiles = nullptr;
     int max_tiles = 0;
     int64_t expert_stride = 0;
-    int rows_each = 0;  // rows of a matrix on average
+    int matrices = 0, rows_each = 0;  // how many there are; rows of one on average
     bool few = false;   // to k_few, whatever k_few_pays says
     const int32_t *gather = nullptr;  // row of x for each row of the product
     // where workgroups that share a block of results leave their sums (FEW_PART_FLOATS), and how many are through with each (FEW_PART_ITEMS, zero between
@@ -129,9 +129,11 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 // The same for few rows or positions (k_few.hip), which k_gemm hands on to where that is the faster way; cols: columns the epilogue
 // covers.  Distinct matrices one after the other:
 //
-// bf16, the time of k_gemm's own tiles over that of k_few.  Grouped, up to 60 positions a matrix: 8 and 16 matrices of 256 to 2048 inputs, at 8, 32 and 64 positions 1.8
-// to 2.6, 1.7 to 2.3 and 1.4 to 1.8, at 96 0.9 to 1.5.  Plain, up to 128 positions (1.0 to 2.0, 256 to 2048 inputs, up to 32 000 rows), otherwise where tiles of
-// 64 x 64 are at most 256 (1.0 to 1.9), or 768 of at least 2048 inputs: 288 tiles 1.6, 512 1.3, 768 1.1, 1500 0.9; of 512 inputs 512 tiles 0.8.
+// bf16, the time of k_gemm's own tiles over that of k_few.  Grouped, up to 48 positions a matrix (8 and 16 matrices of 256 to 2048 inputs, at 8 and 32 1.8 to 2.6 and 1.7 to
+// 2.3), and up to 60 where there are few blocks of 64 rows, for longer loops more: 60 positions each of 64, 256, 512, 1024 and 2048 inputs, 128 blocks 1.0 to 1.1, 1.3, 1.6, 2.0 and 2.4, 256
+// 0.85 to 0.9, 1.1, 1.2, 1.4 to 1.5 and 1.6, 512 0.6, 0.8, 0.8 to 1.0, 0.9 to 1.1 and 1.0 to 1.2, 1024 0.4, 0.5, 0.6 to 0.7, 0.7 to 0.8 and 0.9 to 1.1.  Plain, up to 64 positions, up to 128 of at
+// least 768 inputs (1.0 to 2.0, up to 32 000 rows; 65 to 128 of fewer inputs in more than 256 tiles of 64 x 64 0.6 to 0.9), otherwise where such tiles are at most 256
+// (1.0 to 1.9), or 768 of at least 2048 inputs: 288 tiles 1.6, 512 1.3, 768 1.1, 1500 0.9; of 512 inputs 512 tiles 0.8.
 //
 // fp32, k_few's time over that of the tiles, at 256 to 4096 inputs.  Plain, up to 8 positions (0.3 to 0.97) and up to 2^17 results, 2^18 of up to 16 positions: of 17
 // positions and more 0.5 to 0.95 up to 2^16.5 results, 0.65 to 1.01 at 2^17, 0.95 to 1.34 at 2^17.5, 0.96 to 1.77 at 2^18, 1.2 to 2.1 at 2^20; of 9 to 12 positions 0.82 to
@@ -144,31 +146,39 @@ hipError_t k_gemm(hipStream_t s, const GemmArgs &a, int prec, int epi);
 #define FEW_PART_FLOATS (FEW_PART_ITEMS * 64 * 64)
 #define L_FEW_M 128
 #define L_FEW_M_F32 8
-#define L_FEW_EACH 60
+#define L_FEW_EACH 48
+#define L_FEW_EACH_MOST 60
 #define L_FEW_EACH_F32 64
 #define L_FEW_TILES 256
 #define L_FEW_RESULTS_F32 131072
+inline int64_t few_blocks(const GemmArgs &a, int64_t cols) { return a.matrices * ((cols + 63) / 64); }  // of 64 rows
 inline bool k_few_pays(const GemmArgs &a, int prec, int64_t cols) {
     if (prec) return a.M <= L_FEW_M_F32 || (a.M * cols <= (a.tiles || a.M <= 16 ? 2 : 1) * L_FEW_RESULTS_F32 && (!a.tiles || a.rows_each <= L_FEW_EACH_F32));
     if (a.few) return true;
-    if (a.tiles) return a.rows_each <= L_FEW_EACH;
-    return a.M <= L_FEW_M || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (a.ld >= 2048 ? 3 : 1) * L_FEW_TILES;
+    if (a.tiles) return a.rows_each <= L_FEW_EACH || (a.rows_each <= L_FEW_EACH_MOST && few_blocks(a, cols) <= (a.ld >= 2048 ? 2 * L_FEW_TILES : a.ld >= 256 ? L_FEW_TILES : L_FEW_TILES / 2));
+    return a.M <= (a.ld >= 768 ? L_FEW_M : L_FEW_M / 2) || ((cols + 63) / 64) * ((a.M + 63) / 64) <= (a.ld >= 2048 ? 3 : 1) * L_FEW_TILES;
 }
 hipError_t k_few(hipStream_t s, const GemmArgs &a, int prec, int epi, int64_t cols);
-// Experts' products of a bf16 prompt that have a tile image: k_few from the plain rows where the image's row groups of 256 are too few for the compute units.  us, k_tiles
+// Experts' products of a bf16 prompt that have a tile image: k_few from the plain rows where the image's row groups of 256 are too few for the compute units, and the inputs or positions not so few
+// that a tile is all prologue and epilogue (60 and 128 positions each, 64 groups of 64 inputs 5.4, 6.2 and 7.6, 11.8, of 256 7.7, 8.2 and 9.9, 13.3; 16 groups 4.4, 5.3 and 3.9, 5.0).  us, k_tiles
 // and k_few, 16, 48 and 83 positions an expert: 8 of 512 x 512 (16 groups) 7.2, 9.9, 11.0 and 4.0, 6.1, 7.3; 32 of 512 x 1024 (64) 16.6, 19.7, 21.6 and 9.5, 14.2, 16.6; 8 of
 // 1792 x 3584 (56) 42, 51, 54 and 21, 36, 38; 128 each 1.3 to 1.5 times; 16 of 2048 x 4096 (128) 56, 64, 72 and 48, 64, 85; 32 of 1024 x 2048 (128) 31, 35, 38 and 28, 36, 47; 16 of
 // 2048 x 1024 (128) 17.5, 20.6, 23.3 and 17.2, 23.0, 29.4; 16 of 4096 x 2048 (256) 49, 52, 57 and 51, 70, 95.
 inline bool k_few_experts_pays(int experts, int64_t rows, int ld, int rows_each) {
     const int64_t groups = experts * ((rows + 255) / 256);
-    return (groups <= 64 && rows_each <= 128) || (groups <= 128 && rows_each <= 32 && ld >= 2048);
+    return (groups <= 64 && rows_each <= 128 && (groups <= 16 || rows_each <= 40 || ld >= 512)) || (groups <= 128 && rows_each <= 32 && ld >= 2048);
 }
 // A plain product (GE_STORE, GE_RESID) that the library would take: k_few where tiles of 64 x 64 are at most one a compute unit and its inputs few enough.  us, the library
 // with positions in whole groups of 128 and k_few, 130, 256, 333 and 500 positions: 1024 x 1024 5.5, 5.4, 6.5, 6.5 and 4.5, 4.6, 5.7, 5.8; 2048 x 2048 10.1, 10.1, 12.6, 12.8 and 8.1, 9.1,
 // 10.3, 11.5; 1024 x 4096 12.0, 12.0, 15.1, 15.7 and 10.3, 11.2, 12.0, 15.1; 4096 x 4096 22.9, 22.8 and 18.3, 23.0, but 333 (384 tiles) 24.9 and 32.5; 2048 x 6144 23.2, 23.2, 27.5, 27.3 and
-// 17.7, 21.1, 29.0, 31.7; 6144 x 2048, 130 (288) 16.0 and 20.5.  More than 512 positions only of a router: 2048 of 32 x 2048 6.8 and 5.4, but of 256 x 2048 8.8 and 13.0
+// 17.7, 21.1, 29.0, 31.7; 6144 x 2048, 130 (288) 16.0 and 20.5.  More than 512 positions only of a router: 2048 of 32 x 2048 6.8 and 5.4, but of 256 x 2048 8.8 and 13.0.
+// Few rows of many inputs go better in more shares than eight: 128 x 3072, 256 6.0 and 6.8, 128 x 4096 6.6 and 7.8, 512 x 4096, 256 and 512 8.1, 10.0 and 8.6, 11.2, but 128 x 2048 5.4 and 5.4, 512 x 3072
+// 7.2, 8.4 and 6.6, 7.0, 768 x 4096 11.9, 14.9 and 10.3, 14.1.  Of 256 inputs, 130, 256 and 512, 1344 rows 4.5 (256), 5.2 (512) and 4.0, 5.9; 2048 4.6, 4.7, 5.3 and 4.1, 4.2, 6.2; 4096 5.3, 5.3 and 5.8, 6.2 (tiles of
+// 32 rows up to 256, where few_plan takes them)
 inline bool k_few_plain_pays(const GemmArgs &a) {
-    return (a.M <= 512 || a.n_rows <= 32) && (a.n_rows + 63) / 64 * ((a.M + 63) / 64) <= L_FEW_TILES && (a.ld <= 4096 || a.M <= 256);
+    const int64_t positions = (a.M + 63) / 64, small = (a.n_rows + 31) / 32 * positions;
+    return (a.M <= 512 || a.n_rows <= 32) && (a.n_rows + 63) / 64 * positions <= L_FEW_TILES && (a.ld <= 4096 || a.M <= 256) &&
+           (a.ld <= 2048 || a.n_rows <= 32 || 6 * a.n_rows >= a.ld) && (a.ld < 256 || a.ld >= 384 || small <= L_FEW_TILES);
 }
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations

@@ -156,10 +156,12 @@ static void check_small_plan() {
 }
 
 // which kernel takes a product of a layered model: `each` positions for each of `experts` matrices (0: one matrix, `each` positions)
-static bool few(int prec, int experts, int64_t cols, int each) {
+static bool few(int prec, int experts, int64_t cols, int each, int ld = 1024) {
     GemmTile tile{};
     GemmArgs a;
     a.n_rows = cols;
+    a.ld = ld;
+    a.matrices = experts;
     a.M = experts ? experts * each : each;
     a.rows_each = each;
     a.tiles = experts ? &tile : nullptr;
@@ -168,6 +170,9 @@ static bool few(int prec, int experts, int64_t cols, int each) {
 static void check_product_rule() {
     // bf16, sizes at which the one or the other takes at least 1.15 times as long (measured), and where the smaller kernel is up to 8 % behind
     EXPECT(few(0, 96, 4096, 48) && !few(0, 8, 512, 64) && few(0, 0, 32000, 128) && !few(0, 0, 32000, 160));
+    // ... by the number of inputs, where the other takes 1.1 to 3.3 times as long
+    EXPECT(!few(0, 0, 32000, 128, 512) && !few(0, 0, 16384, 128, 256) && few(0, 0, 8192, 128, 256) && few(0, 0, 32000, 64, 192));
+    EXPECT(!few(0, 64, 4096, 60, 64) && !few(0, 16, 4096, 60, 256) && !few(0, 64, 1024, 60, 1024) && few(0, 16, 512, 60, 64) && few(0, 32, 512, 60, 512) && few(0, 32, 1024, 60, 2048));
     // fp32, 1.1 times: one matrix ...
     EXPECT(!few(1, 0, 1024, 509) && !few(1, 0, 4096, 64) && !few(1, 0, 512, 509) && !few(1, 0, 32000, 24) && !few(1, 0, 32000, 2048) && !few(1, 0, 8192, 160));
     EXPECT(!few(1, 0, 9216, 128) && !few(1, 0, 14336, 96) && !few(1, 0, 32000, 64) && !few(1, 0, 32000, 256));

@@ -40,6 +40,13 @@ def test_many_rows(pkg, vocab, width):
     _check(pkg, c, (5, 8, 17, 32, 33, 64, 65, 70), 62)
 
 
+# few inputs, 2, 3, 4 and 6 steps: the other kernel's tiles of 16 x 32 and 32 x 64, k_gemm's from 65 positions on of many rows, the ring's where it has one round
+@pytest.mark.parametrize("width,vocab", [(66, 8210), (130, 16400), (200, 4120), (250, 16390), (330, 12300)])
+def test_few_inputs(pkg, width, vocab):
+    c = lc.config([lc.attention(heads=2, kv_heads=1, dim=16, vdim=16, rot=16, mlp=lc.dense(515))], width=width, vocab=vocab)
+    _check(pkg, c, (17, 33, 64, 65), 65)
+
+
 # (experts, chosen, rows of the up product): few rows, up to 8 positions an expert on average and more; many rows; an expert with more than 64
 @pytest.mark.parametrize("experts,top,rows", [(8, 2, 70), (8, 4, 2100), (3, 1, 520)])
 def test_experts(pkg, experts, top, rows):
