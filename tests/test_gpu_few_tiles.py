@@ -54,8 +54,10 @@ def test_experts(pkg, experts, top, rows):
     _check(pkg, c, (6, 17, 33, 70, 110, 127), 63)
 
 
-# w1 | w3 in tiles of 32 x 32, 32 x 64, 64 x 32 and 64 x 64; eighths of 1, 2, 3 and 21 steps of inputs, of which some are empty or longer
-@pytest.mark.parametrize("dim,hidden,lengths", [(128, 2048, (33, 65, 128, 130)), (192, 8192, (1, 8, 17, 40, 64)), (1344, 4160, (24, 64, 70, 128))])
+# w1 | w3 in tiles of 32 x 32, 32 x 64, 64 x 32 and 64 x 64; eighths of 7, 9 and 21 steps of inputs, of which one is empty or some are longer; of 2, 3 and 6
+# steps, and up to 16 positions of 2048 rows, straight to registers, in tiles of 32 x 32 and 64 x 64
+@pytest.mark.parametrize("dim,hidden,lengths", [(128, 2048, (33, 65, 128, 130)), (192, 8192, (1, 8, 17, 40, 64)), (1344, 4160, (24, 64, 70, 128)),
+                                                (384, 1088, (64, 300)), (448, 4096, (33, 65, 128)), (576, 1024, (1, 16, 17))])
 def test_llama(pkg, dim, hidden, lengths):
     """Against the products that sum their inputs in one part: one more rounding to bf16 the other way for the odd element, as for other prompts with
     and without the library's products"""
