@@ -7,6 +7,7 @@
 
 #define ROWS_MAX_EXPERTS 1024
 #define ROWS_MAX_TOP 64
+#define ROWS_CHOOSE 40
 
 // element e of the staged vector: the two halves of every group of 8 lie in separate planes, so that the lanes of a
 // wavefront, each reading 8 consecutive elements as two 16-byte words, touch consecutive words
@@ -53,8 +54,9 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
     acc1 = k < ld ? b : acc1;
 }
 
-// Choice of up to 64 experts by every wavefront for itself, an expert a lane, as l_route chooses: no barrier, no wait of one wavefront for another
-// before the chosen rows can be requested.  sel: of this wavefront's own; the place of the lane's expert is returned.
+// Choice of up to 40 experts by every wavefront for itself, an expert a lane, as l_route chooses: no barrier, no wait of one wavefront for another
+// before the chosen rows can be requested.  (An expert is eight instructions.  Products behind it against those behind a choice that the workgroup makes with two barriers more, in front of the other changes
+// named below: up to 8 experts 0.82 of the time, 16 to 24 0.88, 32 to 40 0.97, 40 to 48 1.01, 56 to 64 1.05, up to 1.13; the workgroup's choice with those changes, 65 to 130 experts, 0.93.)  sel: of this wavefront's own; the place of the lane's expert is returned.
 __device__ __forceinline__ int rows_choose(float v, int E, int top, int *sel, int lane) {
     int rank = 0;
     for (int o = 0; o < E; o += 8) {
@@ -129,7 +131,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &a, const RowsPlan &pl,
     if (EPI == RE_STORE_KEY && b == 0) ctl = *keys.ctl;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     constexpr bool choice = PRO == RP_UP, chosen = PRO == RP_DOWN;  // (of experts: made here, or handed on in a.sel)
-    const bool by_wave = choice && a.n_experts <= 64;
+    const bool by_wave = choice && a.n_experts <= ROWS_CHOOSE;
     float z = -INFINITY, zb = 0.0f;  // an expert a lane
     int rank = 0;
     if (by_wave && lane < a.n_experts) {

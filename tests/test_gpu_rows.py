@@ -1,4 +1,4 @@
-"""Decode steps where their products' prologues change form: the choice of experts by every wavefront for itself (up to 64) or by the workgroup, sigmoid and
+"""Decode steps where their products' prologues change form: the choice of experts by every wavefront for itself (up to 40) or by the workgroup, sigmoid and
 softmax; the head norm whose factors are requested ahead (four partial sums a head, up to 4096 elements) or formed one by one.  Against the fp64
 restatements."""
 import numpy as np
@@ -23,7 +23,7 @@ def _steps(dev, ref, c, t, n=5):
 
 
 @pytest.mark.parametrize("design", ["sigmoid", "softmax"])
-@pytest.mark.parametrize("experts,top", [(1, 1), (7, 7), (8, 3), (63, 5), (64, 64), (65, 5), (65, 64)])
+@pytest.mark.parametrize("experts,top", [(1, 1), (7, 7), (8, 3), (39, 5), (40, 40), (41, 5), (63, 5), (64, 64), (65, 5), (65, 64)])
 def test_choice_of_experts(pkg, design, experts, top):
     if design == "sigmoid":
         c = lc.config([lc.attention(mlp=lc.moe(experts, top, 17)), lc.attention(mlp=lc.moe(experts, top, 40))], width=136)
