@@ -491,10 +491,11 @@ def test_temperature_sampling_on_device(pkg, rng):
         dev.sample_token(1.0, 1.0)
 
 
-@pytest.mark.parametrize("vocab", [3, 1023, 1025, 4096, 262145, 300001])
+@pytest.mark.parametrize("vocab", [3, 1023, 1025, 4096, 4097, 5121, 32000, 128256, 262145, 300001])
 def test_sampling_over_any_number_of_logits(pkg, vocab):
-    """The draw is split into runs of 1024 logits, or of vocab / 256 from 262 144 on: its probabilities and picks against numpy at
-    the borders, on logits of which some are far below the rest."""
+    """Up to 4096 logits one workgroup draws (sample_one_kernel); beyond, runs of 1024 logits do, or of vocab / 256 from 262 144 on
+    (sample_max_kernel, sample_exp_kernel, sample_prob_kernel): probabilities and picks against numpy at the borders, on logits of which
+    some are far below the rest."""
     plan, kw = CASES["f32"]
     dev = _model(pkg, plan, **dict(kw, vocab_size=vocab, n_layers=1)).device()
     logits, _ = dev.forward(2, 0)
@@ -512,7 +513,7 @@ def test_sampling_over_any_number_of_logits(pkg, vocab):
     dev.close()
 
 
-@pytest.mark.parametrize("vocab", [5, 2500])
+@pytest.mark.parametrize("vocab", [5, 2500, 4097, 32000])
 def test_a_draw_from_what_is_not_a_number_is_an_error(pkg, vocab):
     """A temperature at which the division overflows leaves no probabilities: an error, not the token of the draw before."""
     plan, kw = CASES["f32"]

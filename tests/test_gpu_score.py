@@ -36,3 +36,20 @@ def test_wanted_positions(pkg, plan, dim, vocab):
         assert np.all(np.abs(got - alone[want]) <= ulp), want
         assert np.mean(got != alone[want]) <= 1e-3, want
         assert np.array_equal(dev.state("logits"), got[-1])  # the last of them is the model's state
+
+
+def test_more_wanted_positions_than_the_workspace_has_rows(pkg):
+    """The logits' workspace is 64 MiB, 130 rows of a vocabulary of 128 256: positions on both sides of its border, in one call of 140."""
+    from llama2_jl_amd import synth
+    vocab, n = 128256, 150
+    lm = _model(pkg, synth.PLAN_Q4_K_S, dim=256, hidden_dim=256, n_layers=1, vocab_size=vocab, seq_len=160, rope_freq_base=10000.0, rope_is_neox=False,
+                n_heads=4, n_kv_heads=4)
+    dev = lm.device()
+    tok = synth.seeded_prompt(5, n, vocab)
+    want = np.arange(7, 147)
+    got = dev.prefill_logits(tok, want)
+    assert np.array_equal(dev.state("logits"), got[-1])
+    for i in (0, 1, 121, 127, 128, 129, 130, 131, 137, 138, 139):
+        alone = dev.prefill_logits(tok, [want[i]])[0]
+        assert np.all(np.abs(got[i] - alone) <= np.spacing(np.abs(alone))), i
+        assert np.mean(got[i] != alone) <= 1e-3, i
