@@ -174,11 +174,13 @@ inline bool k_few_experts_pays(int experts, int64_t rows, int ld, int rows_each)
 // 17.7, 21.1, 29.0, 31.7; 6144 x 2048, 130 (288) 16.0 and 20.5.  More than 512 positions only of a router: 2048 of 32 x 2048 6.8 and 5.4, but of 256 x 2048 8.8 and 13.0.
 // Few rows of many inputs go better in more shares than eight: 128 x 3072, 256 6.0 and 6.8, 128 x 4096 6.6 and 7.8, 512 x 4096, 256 and 512 8.1, 10.0 and 8.6, 11.2, but 128 x 2048 5.4 and 5.4, 512 x 3072
 // 7.2, 8.4 and 6.6, 7.0, 768 x 4096 11.9, 14.9 and 10.3, 14.1.  Of 256 inputs, 130, 256 and 512, 1344 rows 4.5 (256), 5.2 (512) and 4.0, 5.9; 2048 4.6, 4.7, 5.3 and 4.1, 4.2, 6.2; 4096 5.3, 5.3 and 5.8, 6.2 (tiles of
-// 32 rows up to 256, where few_plan takes them)
+// 32 rows up to 256, where few_plan takes them).  Not so where embedding rows come behind (a.emb), another launch after the library's: 256 x 4096, 333 positions 11.4 + 5.0
+// and 13.3.
 inline bool k_few_plain_pays(const GemmArgs &a) {
     const int64_t positions = (a.M + 63) / 64, small = (a.n_rows + 31) / 32 * positions;
-    return (a.M <= 512 || a.n_rows <= 32) && (a.n_rows + 63) / 64 * positions <= L_FEW_TILES && (a.ld <= 4096 || a.M <= 256) &&
-           (a.ld <= 2048 || a.n_rows <= 32 || 6 * a.n_rows >= a.ld) && (a.ld < 256 || a.ld >= 384 || small <= L_FEW_TILES);
+    const bool tiles = (a.M <= 512 || a.n_rows <= 32) && (a.n_rows + 63) / 64 * positions <= L_FEW_TILES && (a.ld <= 4096 || a.M <= 256);
+    if (a.emb) return tiles;
+    return tiles && (a.ld <= 2048 || a.n_rows <= 32 || 6 * a.n_rows >= a.ld) && (a.ld < 256 || a.ld >= 384 || small <= L_FEW_TILES);
 }
 
 // the same from a tile image (k_tiles.hip): GE_ACT, GE_GLU, and GE_UP / GE_GLU / GE_STORE in the grouped form; bf16 activations

@@ -173,6 +173,20 @@ static void check_product_rule() {
     // ... by the number of inputs, where the other takes 1.1 to 3.3 times as long
     EXPECT(!few(0, 0, 32000, 128, 512) && !few(0, 0, 16384, 128, 256) && few(0, 0, 8192, 128, 256) && few(0, 0, 32000, 64, 192));
     EXPECT(!few(0, 64, 4096, 60, 64) && !few(0, 16, 4096, 60, 256) && !few(0, 64, 1024, 60, 1024) && few(0, 16, 512, 60, 64) && few(0, 32, 512, 60, 512) && few(0, 32, 1024, 60, 2048));
+    // plain ones against the library's, alone and with another launch behind it
+    const uint16_t rows[1] = {};
+    for (const uint16_t *emb : {(const uint16_t *)nullptr, rows}) {
+        GemmArgs a;
+        a.emb = emb;
+        a.M = 333, a.n_rows = 256, a.ld = 4096;
+        EXPECT(k_few_plain_pays(a) == (emb != nullptr));
+        a.ld = 2048;
+        EXPECT(k_few_plain_pays(a));
+        a.M = 512, a.n_rows = 2048, a.ld = 256;
+        EXPECT(k_few_plain_pays(a) == (emb != nullptr));
+        a.n_rows = 4096;
+        EXPECT(!k_few_plain_pays(a));
+    }
     // fp32, 1.1 times: one matrix ...
     EXPECT(!few(1, 0, 1024, 509) && !few(1, 0, 4096, 64) && !few(1, 0, 512, 509) && !few(1, 0, 32000, 24) && !few(1, 0, 32000, 2048) && !few(1, 0, 8192, 160));
     EXPECT(!few(1, 0, 9216, 128) && !few(1, 0, 14336, 96) && !few(1, 0, 32000, 64) && !few(1, 0, 32000, 256));
