@@ -8,8 +8,8 @@
 // inputs of one row), the next step's under way during this one's; a position's inputs come from the L2.  A load's 16 rows lie a multiple of 4 KB apart, which
 // is what bounds it from 17 positions on.
 //
-// few_ring_kernel (bf16, few_ring.h): whole lines, through LDS.  Microseconds of few_kernel and of this, a matrix of its own in each launch: 64 positions, 16 384 rows x 2048 inputs 30.6, 17.1; 28 672 x 4096 106, 49.9; 4096 x 14 336 81.7, 30.4; 2048 x 8192 24.7, 13.5; 3072 x 2048 14.3,
-// 8.2; a router's 32 rows x 4096, 12.6, 5.3; 16 experts of 2048 x 2048, 14 and 64 positions each: 43, 28.6 and 124, 47.8.
+// few_ring_kernel (bf16, few_ring.h): whole lines, through LDS.  Microseconds of few_kernel and of this, a matrix of its own in each launch: 64 positions,
+// 16 384 rows x 2048 inputs 30.6, 17.1; 28 672 x 4096 106, 49.9; 4096 x 14 336 81.7, 30.4; 2048 x 8192 24.7, 13.5; 3072 x 2048 14.3, 8.2; a router's 32 rows x 4096, 12.6, 5.3; 16 experts of 2048 x 2048, 14 and 64 positions each: 43, 28.6 and 124, 47.8.
 #include "few_ring.h"
 #include "layered_gemm.h"
 

@@ -55,8 +55,9 @@ __device__ __forceinline__ void rows_fma(const RowsChunk &c, const float *xv, in
 }
 
 // Choice of up to 40 experts by every wavefront for itself, an expert a lane, as l_route chooses: no barrier, no wait of one wavefront for another
-// before the chosen rows can be requested.  (An expert is eight instructions.  Products behind it against those behind a choice that the workgroup makes with two barriers more, in front of the other changes
-// named below: up to 8 experts 0.82 of the time, 16 to 24 0.88, 32 to 40 0.97, 40 to 48 1.01, 56 to 64 1.05, up to 1.13; the workgroup's choice with those changes, 65 to 130 experts, 0.93.)  sel: of this wavefront's own; the place of the lane's expert is returned.
+// before the chosen rows can be requested.  (An expert is eight instructions.  Products behind it over those behind the workgroup's choice with two barriers
+// more: up to 8 experts 0.82 of the time, 16 to 24 0.88, 32 to 40 0.97, 40 to 48 1.01, 56 to 64 1.05, 1.13 at most.)  sel: of this wavefront's own; the place
+// of the lane's expert is returned.
 __device__ __forceinline__ int rows_choose(float v, int E, int top, int *sel, int lane) {
     int rank = 0;
     for (int o = 0; o < E; o += 8) {
